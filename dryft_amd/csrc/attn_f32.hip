@@ -1,0 +1,257 @@
+// Causal grouped-query attention over the paged cache for the float32 path, on the matrix cores' full-precision
+// instruction (v_mfma_f32_16x16x4_f32), keys and values of one width, a multiple of 16 up to 256:
+//
+//   s[j] = (q . k[j]) * scale  for  lo <= j <= pos,   p = softmax(s),   o = sum_j p[j] v[j]
+//
+// (reference: engine/dryft_qwen3/model.py:172-177, 254-257), lo = 0 or pos - window + 1; query head h reads kv head
+// h / group. A workgroup takes 16 query columns of one kv head: the heads of one row's group (decoding: a workgroup per row,
+// kv head and 16 heads of its group), or 16 rows of a sequence for one head (prompts: a workgroup per tile of 16 rows and
+// head). Its waves take half pages (32 keys) in turn, each with a running maximum and sum of its own, and meet in LDS.
+//
+// Scores of 16 keys are C[key, column] = K . q^T: lane (c, g) holds keys 4g .. 4g + 3 of column c, which is what the second
+// product, O^T[feature, column] += V^T . P, takes as its operand, one entry an instruction; a page of values keeps the
+// positions of a half page in the order that gives a lane its eight of both tiles of 16 keys as 32 contiguous bytes
+// (value_column). So scores never leave registers, and every line of a page is read once by one wave for all columns, where
+// the kernel of one workgroup a (row, head) (attn_rows.hip) read every key with 16 bytes a line and request, once per head
+// of the group. Qwen3-0.6B, 4 sequences, us in the step: decoding at
+// 10 to 280 keys 14.9 against that kernel's 18.6 (what is left are four trips to memory one after the other and 13 of 16
+// columns unused), 525 prompt rows 29.5 against 123.
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+struct AttnF32 {
+  const float* q;                 // [rows, n_heads, D]
+  const float* k_pages;
+  const float* v_pages;
+  const int* page_table;
+  int max_pages;
+  const int* row_slot;            // decoding
+  const int* row_pos;
+  const int* seq_slot;            // prompts
+  const int* cu_rows;
+  const int* tile_cu;
+  const int* seq_start;
+  int n_seqs;
+  float* out;                     // [rows, n_heads, D]
+  int n_heads, n_kv, head_dim;
+  float scale;
+  int window;
+};
+
+template <int DT, int WAVES, bool TILES>
+__global__ __launch_bounds__(WAVES * WAVE) void attn_f32_kernel(AttnF32 a) {
+  extern __shared__ __align__(16) float attn_f32_lds[];
+  constexpr int D = 16 * DT, OS = D + 1;
+  float* merge_o = attn_f32_lds;                           // [WAVES][16][OS]
+  float* merge_m = merge_o + WAVES * 16 * OS;              // [WAVES][16]
+  float* merge_l = merge_m + WAVES * 16;
+  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, c = lane % 16, g = lane / 16;
+  const int group = a.n_heads / a.n_kv;
+  int slot, kvh, columns, pos, first_pos, last_pos;        // pos: this lane's column's; of the first and the last column
+  int64_t q_at;                                            // this lane's column of q and out
+  if (TILES) {
+    const int tile = blockIdx.x, head = blockIdx.y;
+    if (tile >= a.tile_cu[a.n_seqs]) return;
+    int lo = 0, hi = a.n_seqs - 1;                         // the sequence whose tiles hold this one
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) / 2;
+      if (a.tile_cu[mid] <= tile) lo = mid;
+      else hi = mid - 1;
+    }
+    const int r0 = 16 * (tile - a.tile_cu[lo]);
+    slot = a.seq_slot[lo];
+    kvh = head / group;
+    columns = min(16, a.cu_rows[lo + 1] - a.cu_rows[lo] - r0);
+    first_pos = a.seq_start[lo] + r0;
+    last_pos = first_pos + columns - 1;
+    pos = first_pos + min(c, columns - 1);
+    q_at = ((int64_t)(a.cu_rows[lo] + r0 + min(c, columns - 1)) * a.n_heads + head) * D;
+  } else {
+    const int blocks = (group + 15) / 16;
+    const int64_t row = blockIdx.x;
+    kvh = blockIdx.y / blocks;
+    const int h0 = (blockIdx.y % blocks) * 16;
+    slot = a.row_slot[row];
+    columns = min(16, group - h0);
+    first_pos = last_pos = pos = a.row_pos[row];
+    q_at = (row * a.n_heads + kvh * group + h0 + min(c, columns - 1)) * D;
+    if (slot < 0) {                                        // a row that sits out: zeros
+      const int64_t at = (row * a.n_heads + kvh * group + h0) * D;
+      for (int i = threadIdx.x; i < columns * D; i += blockDim.x) a.out[at + i] = 0.f;
+      return;
+    }
+  }
+  if (slot < 0) return;                                    // no tile belongs to a sequence that sits out
+  const int lo_col = a.window > 0 ? max(0, pos - a.window + 1) : 0;
+  const int lo_all = a.window > 0 ? max(0, first_pos - a.window + 1) : 0;
+  const int* table = a.page_table + (int64_t)slot * a.max_pages;
+  f32x4 qv[DT];
+#pragma unroll
+  for (int t = 0; t < DT; ++t) qv[t] = *(const f32x4*)(a.q + q_at + 16 * t + 4 * g);
+  f32x4 o[DT];
+#pragma unroll
+  for (int t = 0; t < DT; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;                            // l: over the keys of this lane alone
+  constexpr bool V_EARLY = DT <= 8;                        // wider heads have no registers for the values that soon
+  int u = lo_all / 32 + wave;
+  int page = 32 * u <= last_pos ? table[u / 2] : -1;
+  for (; 32 * u <= last_pos; u += WAVES) {
+    const int here = page;
+    page = 32 * (u + WAVES) <= last_pos ? table[(u + WAVES) / 2] : -1;
+    if (here < 0) continue;
+    const int64_t base = ((int64_t)here * a.n_kv + kvh) * PAGE_TOKENS * D;
+    const float* kp = a.k_pages + base + (int64_t)(32 * (u & 1) + c) * D + 4 * g;
+    const float* vp = a.v_pages + base + (int64_t)c * PAGE_TOKENS + 32 * (u & 1) + 8 * g;
+    // everything the half page needs is asked for at once: one trip to memory, not one for the keys and one for the values
+    f32x4 kv[2][DT], vv[DT][2];
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int t = 0; t < DT; ++t) kv[half][t] = *(const f32x4*)(kp + 16 * half * D + 16 * t);
+    if (V_EARLY) {
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int half = 0; half < 2; ++half) vv[t][half] = *(const f32x4*)(vp + (int64_t)16 * t * PAGE_TOKENS + 4 * half);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // four sums side by side: an instruction need not wait for the one before it
+    f32x4 s[2], odd[2];
+#pragma unroll
+    for (int half = 0; half < 2; ++half) s[half] = odd[half] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; i += 2)
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          s[half] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[half][t][i], qv[t][i], s[half], 0, 0, 0);
+          odd[half] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[half][t][i + 1], qv[t][i + 1], odd[half], 0, 0, 0);
+        }
+#pragma unroll
+    for (int half = 0; half < 2; ++half) s[half] += odd[half];
+    float top = -INFINITY;
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int j = 32 * u + 16 * half + 4 * g + i;
+        s[half][i] = j >= lo_col && j <= pos ? s[half][i] * a.scale : -INFINITY;
+        top = fmaxf(top, s[half][i]);
+      }
+    top = fmaxf(top, __shfl_xor(top, 16, WAVE));
+    top = fmaxf(top, __shfl_xor(top, 32, WAVE));
+    const float m_new = fmaxf(m, top);
+    // a column that has seen no key yet has m_new = -inf: its weights are zeros
+    const float keep = m_new == -INFINITY ? 0.f : expf(m - m_new);
+    f32x4 p[2];
+    float added = 0.f;
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        p[half][i] = s[half][i] == -INFINITY ? 0.f : expf(s[half][i] - m_new);
+        added += p[half][i];
+      }
+    l = l * keep + added;
+    m = m_new;
+#pragma unroll
+    for (int t = 0; t < DT; ++t) {
+      o[t] *= keep;
+      if (!V_EARLY) {
+#pragma unroll
+        for (int half = 0; half < 2; ++half) vv[t][half] = *(const f32x4*)(vp + (int64_t)16 * t * PAGE_TOKENS + 4 * half);
+      }
+    }
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int t = 0; t < DT; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[t][half][i], p[half][i], o[t], 0, 0, 0);
+  }
+  l += __shfl_xor(l, 16, WAVE);
+  l += __shfl_xor(l, 32, WAVE);
+  // o[t][i] is feature 16 t + 4g + i of column c
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) merge_o[(wave * 16 + c) * OS + 16 * t + 4 * g + i] = o[t][i];
+  if (g == 0) {
+    merge_m[wave * 16 + c] = m;
+    merge_l[wave * 16 + c] = l;
+  }
+  __syncthreads();
+  const int64_t out_step = TILES ? (int64_t)a.n_heads * D : D;           // from one column to the next
+  const int64_t out_at = q_at - (int64_t)min(c, columns - 1) * out_step;  // of the first
+  for (int idx = threadIdx.x; idx < columns * D; idx += blockDim.x) {
+    const int col = idx / D, d = idx % D;
+    float top = -INFINITY;
+#pragma unroll
+    for (int v = 0; v < WAVES; ++v) top = fmaxf(top, merge_m[v * 16 + col]);
+    float sum = 0.f, total = 0.f;
+#pragma unroll
+    for (int v = 0; v < WAVES; ++v) {
+      const float mv = merge_m[v * 16 + col];
+      const float wgt = mv == -INFINITY ? 0.f : expf(mv - top);
+      total += wgt * merge_l[v * 16 + col];
+      sum += wgt * merge_o[(v * 16 + col) * OS + d];
+    }
+    a.out[out_at + col * out_step + d] = total > 0.f ? sum / total : 0.f;
+  }
+}
+
+template <int DT, int WAVES, bool TILES>
+static int launch_attn_f32(const AttnF32& a, dim3 grid, hipStream_t stream) {
+  constexpr int lds = WAVES * 16 * (16 * DT + 1 + 2) * 4;
+  static_assert(lds <= 160 * 1024, "the merge must fit a compute unit's LDS");
+  auto kernel = attn_f32_kernel<DT, WAVES, TILES>;
+  static bool raised = false;                              // more dynamic LDS than the default limit allows
+  if (lds > 64 * 1024 && !raised) {
+    if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return -2;
+    raised = true;
+  }
+  hipLaunchKernelGGL(kernel, grid, dim3(WAVES * WAVE), lds, stream, a);
+  return DRYFT_LAUNCH_CHECK();
+}
+
+template <bool TILES>
+static int dispatch_attn_f32(const AttnF32& a, dim3 grid, hipStream_t stream) {
+  if (a.n_kv <= 0 || a.n_heads % a.n_kv || a.head_dim <= 0 || a.head_dim % 16 || a.head_dim > 256 || grid.y > 65535 ||
+      (((uintptr_t)a.q | (uintptr_t)a.k_pages | (uintptr_t)a.v_pages) & 15))
+    return -1;
+#define ATTN_F32(DTV, WV) case DTV: return launch_attn_f32<DTV, WV, TILES>(a, grid, stream)
+  switch (a.head_dim / 16) {                               // eight waves where the merge of a decoding row fits twice a unit
+    ATTN_F32(1, 4); ATTN_F32(2, 4); ATTN_F32(3, 4); ATTN_F32(4, 4);
+    ATTN_F32(5, 4); ATTN_F32(6, 4); ATTN_F32(7, 4); ATTN_F32(8, (TILES ? 4 : 8));
+    ATTN_F32(9, 4); ATTN_F32(10, 4); ATTN_F32(11, 4); ATTN_F32(12, 4);
+    ATTN_F32(13, 4); ATTN_F32(14, 4); ATTN_F32(15, 4); ATTN_F32(16, 4);
+  }
+#undef ATTN_F32
+  return -1;
+}
+
+// One row per sequence or any rows: each on its own, by its slot and position.
+DRYFT_API int dryft_attn_f32_rows(const void* q, const void* k_pages, const void* v_pages, const int* page_table,
+                                  int max_pages, const int* row_slot, const int* row_pos, void* out, int n_rows, int n_heads,
+                                  int n_kv, int head_dim, float scale, int window, hipStream_t stream) {
+  if (n_rows <= 0) return 0;
+  if (n_kv <= 0) return -1;
+  AttnF32 a = {(const float*)q, (const float*)k_pages, (const float*)v_pages, page_table, max_pages, row_slot, row_pos,
+               nullptr, nullptr, nullptr, nullptr, 0, (float*)out, n_heads, n_kv, head_dim, scale, window};
+  const int blocks = (n_heads / n_kv + 15) / 16;
+  return dispatch_attn_f32<false>(a, dim3(n_rows, n_kv * blocks), stream);
+}
+
+// Rows in tiles of 16 of one sequence (tile_cu: their prefix sums over the sequences; max_tiles bounds their number).
+// Rows of sequences that sit out are not visited.
+DRYFT_API int dryft_attn_f32_tiles(const void* q, const void* k_pages, const void* v_pages, const int* page_table,
+                                   int max_pages, const int* seq_slot, const int* cu_rows, const int* tile_cu,
+                                   const int* seq_start, int n_seqs, int max_tiles, void* out, int n_heads, int n_kv,
+                                   int head_dim, float scale, int window, hipStream_t stream) {
+  if (n_seqs <= 0 || max_tiles <= 0) return 0;
+  AttnF32 a = {(const float*)q, (const float*)k_pages, (const float*)v_pages, page_table, max_pages, nullptr, nullptr,
+               seq_slot, cu_rows, tile_cu, seq_start, n_seqs, (float*)out, n_heads, n_kv, head_dim, scale, window};
+  return dispatch_attn_f32<true>(a, dim3(max_tiles, n_heads), stream);
+}

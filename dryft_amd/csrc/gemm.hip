@@ -1476,91 +1476,6 @@ DRYFT_API int dryft_gemm_narrow_bf16(const void* x, int64_t x_stride, const void
   return DRYFT_LAUNCH_CHECK();
 }
 
-// ------------------------------------------------------------------------------------------- rows of 32-bit values
-// At most 16 rows of 32-bit values (decoding in the float32 path): bound by reading W once. A workgroup owns 8
-// weight rows, two per wave, and walks K in chunks of 256: the rows of x for a chunk are staged in LDS once for all
-// four waves (double-buffered, one barrier per chunk), a lane takes four consecutive values of each of its weight
-// rows (16-byte loads, a wave reads 1 KB of a row per instruction; the next chunk's are in flight while this one is
-// multiplied) and the matching four of every row of x, and multiplies with plain fused multiply-adds. At the end
-// the 64 lanes' sums are added. K must be a multiple of 4; rows beyond N are read from a clamped row, never stored.
-#define ROWS_CHUNK 256
-template <int MR>
-__global__ __launch_bounds__(256) void gemm_rows_f32_kernel(const float* __restrict__ x, int64_t x_stride,
-                                                            const float* __restrict__ w, float* __restrict__ y, int M,
-                                                            int N, int K) {
-  __shared__ __align__(16) float xs[2][MR][ROWS_CHUNK + 4];
-  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-  const int n0 = blockIdx.x * 8 + 2 * wave;
-  const float* w_row[2] = {w + (int64_t)min(n0, N - 1) * K, w + (int64_t)min(n0 + 1, N - 1) * K};
-  float acc[2][MR];
-#pragma unroll
-  for (int r = 0; r < 2; ++r)
-#pragma unroll
-    for (int m = 0; m < MR; ++m) acc[r][m] = 0.f;
-  float xr[MR];                                            // thread t brings value k0 + t of every row of x
-  auto fetch_x = [&](int k0) {                             // beyond K or M: a valid address, stored as zero
-    const int k = min(k0 + (int)threadIdx.x, K - 1);
-#pragma unroll
-    for (int m = 0; m < MR; ++m) xr[m] = x[(int64_t)min(m, M - 1) * x_stride + k];
-  };
-  auto store_x = [&](int buf, int k0) {
-    const bool in = k0 + (int)threadIdx.x < K;
-#pragma unroll
-    for (int m = 0; m < MR; ++m) xs[buf][m][threadIdx.x] = (in && m < M) ? xr[m] : 0.f;
-  };
-  f32x4 wv[2], wn[2];
-  auto fetch = [&](f32x4 (&v)[2], int k0) {                // beyond K: the row's last four values, multiplied by zeros
-    const int kk = min(k0 + 4 * lane, K - 4);
-    v[0] = *(const f32x4*)(w_row[0] + kk);
-    v[1] = *(const f32x4*)(w_row[1] + kk);
-  };
-  fetch_x(0);
-  fetch(wv, 0);
-  store_x(0, 0);
-  int buf = 0;
-  for (int k0 = 0; k0 < K; k0 += ROWS_CHUNK, buf ^= 1) {
-    __syncthreads();                                       // the chunk is staged; the other buffer is free again
-    fetch_x(k0 + ROWS_CHUNK);                              // the next chunk's loads are in flight during the products
-    fetch(wn, k0 + ROWS_CHUNK);
-#pragma unroll
-    for (int m = 0; m < MR; ++m) {
-      const f32x4 xv = *(const f32x4*)&xs[buf][m][4 * lane];   // zeros beyond K
-#pragma unroll
-      for (int r = 0; r < 2; ++r)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[r][m] = fmaf(wv[r][i], xv[i], acc[r][m]);
-    }
-    store_x(buf ^ 1, k0 + ROWS_CHUNK);
-    wv[0] = wn[0];
-    wv[1] = wn[1];
-  }
-#pragma unroll
-  for (int r = 0; r < 2; ++r)
-#pragma unroll
-    for (int m = 0; m < MR; ++m) {
-      const float s = wave_sum(acc[r][m]);
-      if (lane == 0 && m < M && n0 + r < N) y[(int64_t)m * N + n0 + r] = s;
-    }
-}
-
-// M <= 16, K % 4 == 0
-DRYFT_API int dryft_gemm_rows_f32(const void* x, int64_t x_stride, const void* w, void* y, int M, int N, int K,
-                                  hipStream_t stream) {
-  if (M <= 0 || N <= 0) return 0;
-  if (M > 16 || K <= 0 || K % 4) return -1;
-  dim3 grid((N + 7) / 8), block(256);
-#define RW(MRV)                                                                                                \
-  hipLaunchKernelGGL(gemm_rows_f32_kernel<MRV>, grid, block, 0, stream, (const float*)x, x_stride, (const float*)w, \
-                     (float*)y, M, N, K)
-  if (M <= 1) RW(1);
-  else if (M <= 2) RW(2);
-  else if (M <= 4) RW(4);
-  else if (M <= 8) RW(8);
-  else RW(16);
-#undef RW
-  return DRYFT_LAUNCH_CHECK();
-}
-
 // y = T(sum_s partials[s]) in the order s = 0, 1, ...
 template <typename O>
 __global__ void sum_partials_kernel(const float* __restrict__ partials, O* __restrict__ y, int64_t n, int splits) {

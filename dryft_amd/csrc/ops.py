@@ -74,6 +74,13 @@ _SIGNATURES = {
                                             _F, _P, _I, _P, _I, _P],
                   "dryft_attn_decode_fused_bf16": [_P, _L, _I, _L, _P, _P, _I, _I, _F, _P, _P, _I, _I, _P, _P, _P, _I, _P, _P,
                                                    _P, _I, _P, _P, _I, _P, _I, _I, _I, _F, _I, _P]},
+    "attn_f32": {"dryft_attn_f32_rows": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _F, _I, _P],
+                 "dryft_attn_f32_tiles": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _P, _I, _I, _I, _F, _I, _P]},
+    "gemm_f32": {"dryft_gemm_stream_f32": [_P, _L, _P, _P, _I, _I, _I, _P],
+                 "dryft_gemm_rows_f32": [_P, _L, _P, _P, _I, _I, _I, _I, _P],
+                 "dryft_gemm_rows_swiglu_f32": [_P, _L, _P, _P, _I, _I, _I, _P],
+                 "dryft_gemm_direct_f32_shape": [_I, _I],
+                 "dryft_gemm_direct_f32": [_P, _L, _P, _P, _I, _I, _I, _I, _P]},
     "gemm": {"dryft_gemm_tiled": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _P],
              "dryft_gemm_stream_bf16": [_P, _L, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
              "dryft_gemm_stream_swiglu_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _P],
@@ -87,7 +94,6 @@ _SIGNATURES = {
              "dryft_gemm_mid_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _P],
              "dryft_gemm_block_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _I, _P],
              "dryft_gemm_block_f32": [_P, _L, _P, _P, _I, _I, _I, _I, _P],
-             "dryft_gemm_rows_f32": [_P, _L, _P, _P, _I, _I, _I, _P],
              "dryft_gemm_wide_swiglu_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _P],
              "dryft_gemm_narrow_bf16": [_P, _L, _P, _P, _I, _I, _I, _P],
              "dryft_sum_partials": [_P, _P, _L, _I, _I, _P]},
@@ -639,6 +645,53 @@ def attn_rows(q, k_pages, v_pages, page_table, row_slot, row_pos, out, n_heads: 
         _stream()), "attn_rows")
 
 
+ATTN_F32_TILE = 16       # rows of a sequence that a workgroup of attn_f32 takes in steps of many rows
+
+
+def attn_f32_takes(q, k_pages, v_pages, head_dim: int) -> bool:
+    """Does the float32 attention on the matrix cores take these heads (keys and values of one width, a multiple of 16 up
+    to 256) at these addresses?"""
+    return q.dtype == torch.float32 and head_dim % 16 == 0 and 0 < head_dim <= 256 and \
+        all(t.data_ptr() % 16 == 0 for t in (q, k_pages, v_pages))
+
+
+def attn_f32(q, k_pages, v_pages, page_table, out, n_heads: int, n_kv: int, head_dim: int, scale: float, window: int, *,
+             row_slot=None, row_pos=None, tiles=None) -> None:
+    """Causal attention of float32 rows on the matrix cores' full-precision instruction. Either every row on its own
+    (``row_slot``, ``row_pos``: int32, one per row; rows with slot -1 become zeros), or in tiles of ``ATTN_F32_TILE`` rows of
+    a sequence: ``tiles = (seq_slot, cu_rows, tile_cu, seq_start, n_seqs, max_tiles)``, where the rows of sequences that sit
+    out are not written."""
+    _gpu(q, "q", torch.float32)
+    _gpu(out, "out", torch.float32)
+    rows = q.numel() // (n_heads * head_dim)
+    if not (q.is_contiguous() and q.numel() == rows * n_heads * head_dim and out.is_contiguous() and out.numel() == q.numel()):
+        raise KernelError("attn_f32: q and out must be [rows, heads, head_dim]")
+    if not attn_f32_takes(q, k_pages, v_pages, head_dim):
+        raise KernelError(f"attn_f32: head sizes that are multiples of 16 up to 256 at 16-byte addresses, got {head_dim}")
+    if not (n_heads <= 65535):
+        raise KernelError("attn_f32: too many heads")
+    _check_pages(k_pages, v_pages, page_table, n_kv, head_dim, torch.float32)
+    if tiles is None:
+        for name, t in (("row_slot", row_slot), ("row_pos", row_pos)):
+            _gpu(t, name, torch.int32)
+            if not (t.numel() >= rows):
+                raise KernelError(f"{name}: needs {rows} entries")
+        _check(_fn("attn_f32", "dryft_attn_f32_rows")(
+            _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(page_table), page_table.shape[1], _ptr(row_slot), _ptr(row_pos),
+            _ptr(out), rows, n_heads, n_kv, head_dim, float(scale), int(window), _stream()), "attn_f32_rows")
+        return
+    seq_slot, cu_rows, tile_cu, seq_start, n_seqs, max_tiles = tiles
+    for name, t, n in (("seq_slot", seq_slot, n_seqs), ("cu_rows", cu_rows, n_seqs + 1), ("tile_cu", tile_cu, n_seqs + 1),
+                       ("seq_start", seq_start, n_seqs)):
+        _gpu(t, name, torch.int32)
+        if not (t.numel() >= n):
+            raise KernelError(f"{name}: needs {n} entries")
+    _check(_fn("attn_f32", "dryft_attn_f32_tiles")(
+        _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(page_table), page_table.shape[1], _ptr(seq_slot), _ptr(cu_rows),
+        _ptr(tile_cu), _ptr(seq_start), n_seqs, int(max_tiles), _ptr(out), n_heads, n_kv, head_dim, float(scale), int(window),
+        _stream()), "attn_f32_tiles")
+
+
 def _check_rel(rel, n_heads: int) -> None:
     if rel is not None:
         _gpu(rel, "rel", torch.float32)
@@ -1167,9 +1220,16 @@ def gemm_block_f32(x, w, out, shape: int | None = None) -> torch.Tensor:
     return out
 
 
-def gemm_rows_f32(x, w, out) -> torch.Tensor:
-    """``x [M<=16, K] @ w[N, K].T`` on float32 values by plain multiply-adds, every weight read once; ``K`` a
-    multiple of 4 and ``w`` 16-byte aligned."""
+def rows_f32_ok(x, w) -> bool:
+    """Can the products of the float32 path that take 16 bytes of a row at a time read these operands?"""
+    return x.shape[1] % 4 == 0 and x.stride(1) == 1 and x.stride(0) % 4 == 0 and x.data_ptr() % 16 == 0 and \
+        w.data_ptr() % 16 == 0
+
+
+def gemm_rows_f32(x, w, out, splits: int = 1) -> torch.Tensor:
+    """``x [M<=16, K] @ w[N, K].T`` on float32 values with the matrix cores' full-precision instruction, every weight
+    read once; ``K`` a multiple of 4 and ``w`` 16-byte aligned. ``splits`` > 1: ``out`` is ``[splits, M, N]`` and receives
+    sums over as many runs of K. Rows of ``x`` that do not start at 16-byte addresses go to ``gemm_stream_f32``."""
     _gpu(x, "x", torch.float32)
     _gpu(w, "w", torch.float32)
     _gpu(out, "out", torch.float32)
@@ -1179,9 +1239,80 @@ def gemm_rows_f32(x, w, out) -> torch.Tensor:
         raise KernelError("gemm_rows_f32: x [M,K] row-major, w [N,K] contiguous")
     if not (m <= 16 and k % 4 == 0 and w.data_ptr() % 16 == 0):
         raise KernelError(f"gemm_rows_f32: needs M <= 16, K % 4 == 0, aligned w; got M={m} K={k}")
+    if not (1 <= splits <= 64 and out.shape == ((m, n) if splits == 1 else (splits, m, n)) and out.is_contiguous()):
+        raise KernelError(f"gemm_rows_f32: 1 to 64 splits, out contiguous [{m},{n}], or [splits,{m},{n}]")
+    if not rows_f32_ok(x, w):
+        if splits > 1:
+            raise KernelError("gemm_rows_f32: splits need rows of x at 16-byte addresses")
+        return gemm_stream_f32(x, w, out)
+    _check(_fn("gemm_f32", "dryft_gemm_rows_f32")(_ptr(x), x.stride(0), _ptr(w), _ptr(out), m, n, k, int(splits), _stream()),
+           "gemm_rows_f32")
+    return out
+
+
+def gemm_stream_f32(x, w, out) -> torch.Tensor:
+    """``x [M<=16, K] @ w[N, K].T`` on float32 values by plain multiply-adds that read every weight once, whole lines at a
+    time; ``K`` a multiple of 4 and ``w`` 16-byte aligned."""
+    _gpu(x, "x", torch.float32)
+    _gpu(w, "w", torch.float32)
+    _gpu(out, "out", torch.float32)
+    m, k = x.shape
+    n = w.shape[0]
+    if not (w.shape == (n, k) and w.is_contiguous() and x.stride(1) == 1):
+        raise KernelError("gemm_stream_f32: x [M,K] row-major, w [N,K] contiguous")
+    if not (m <= 16 and k % 4 == 0 and w.data_ptr() % 16 == 0):
+        raise KernelError(f"gemm_stream_f32: needs M <= 16, K % 4 == 0, aligned w; got M={m} K={k}")
     if not (out.shape == (m, n) and out.is_contiguous()):
-        raise KernelError(f"gemm_rows_f32: out must be contiguous [{m},{n}]")
-    _check(_fn("gemm", "dryft_gemm_rows_f32")(_ptr(x), x.stride(0), _ptr(w), _ptr(out), m, n, k, _stream()), "gemm_rows_f32")
+        raise KernelError(f"gemm_stream_f32: out must be contiguous [{m},{n}]")
+    _check(_fn("gemm_f32", "dryft_gemm_stream_f32")(_ptr(x), x.stride(0), _ptr(w), _ptr(out), m, n, k, _stream()),
+           "gemm_stream_f32")
+    return out
+
+
+def gemm_rows_swiglu_f32(x, w_gate_up, out) -> torch.Tensor:
+    """``silu(x @ Wg.T) * (x @ Wu.T)`` for ``w_gate_up = [Wg; Wu]`` and at most 16 rows of float32 values, in one kernel;
+    operands as ``rows_f32_ok`` wants them."""
+    _gpu(x, "x", torch.float32)
+    _gpu(w_gate_up, "w_gate_up", torch.float32)
+    _gpu(out, "out", torch.float32)
+    m, k = x.shape
+    two_n = w_gate_up.shape[0]
+    if not (two_n % 2 == 0 and w_gate_up.shape == (two_n, k) and w_gate_up.is_contiguous()):
+        raise KernelError("gemm_rows_swiglu_f32: x [M,K], w [2N,K] contiguous")
+    if not (m <= 16 and rows_f32_ok(x, w_gate_up)):
+        raise KernelError(f"gemm_rows_swiglu_f32: needs M <= 16, K % 4 == 0 and 16-byte aligned rows, got M={m} K={k}")
+    if not (out.shape == (m, two_n // 2) and out.is_contiguous()):
+        raise KernelError(f"gemm_rows_swiglu_f32: out must be contiguous [{m},{two_n // 2}]")
+    _check(_fn("gemm_f32", "dryft_gemm_rows_swiglu_f32")(_ptr(x), x.stride(0), _ptr(w_gate_up), _ptr(out), m, two_n // 2, k,
+                                                         _stream()), "gemm_rows_swiglu_f32")
+    return out
+
+
+DIRECT_F32_STEP = 32     # values of K that gemm_direct_f32 moves at a time; K must be a multiple of it
+
+
+def direct_f32_ok(x, w) -> bool:
+    """Can ``gemm_direct_f32`` take these operands? (Whole steps of K, 16-byte pieces of rows, 32-bit byte offsets.)"""
+    return rows_f32_ok(x, w) and x.shape[1] % DIRECT_F32_STEP == 0 and w.numel() * 4 < DIRECT_REACH and \
+        x.shape[0] * x.stride(0) * 4 < DIRECT_REACH
+
+
+def gemm_direct_f32(x, w, out, shape: int = -1) -> torch.Tensor:
+    """``x [M, K] @ w[N, K].T`` on float32 values with the matrix cores' full-precision instruction, operands straight from
+    memory into LDS. ``shape``: 0 = blocks of 128 x 128, 1 = 64 x 64, 2 = 32 x 64; -1 lets the library choose."""
+    _gpu(x, "x", torch.float32)
+    _gpu(w, "w", torch.float32)
+    _gpu(out, "out", torch.float32)
+    m, k = x.shape
+    n = w.shape[0]
+    if not (w.shape == (n, k) and w.is_contiguous() and direct_f32_ok(x, w)):
+        raise KernelError(f"gemm_direct_f32: x [M,K] and w [N,K], 16-byte aligned rows, K % {DIRECT_F32_STEP} == 0, got K={k}")
+    if not (out.shape == (m, n) and out.is_contiguous() and out.data_ptr() % 16 == 0):
+        raise KernelError(f"gemm_direct_f32: out must be contiguous and 16-byte aligned [{m},{n}]")
+    if not (-1 <= shape <= 2):
+        raise KernelError("gemm_direct_f32: shape 0, 1 or 2, or -1")
+    _check(_fn("gemm_f32", "dryft_gemm_direct_f32")(_ptr(x), x.stride(0), _ptr(w), _ptr(out), m, n, k, int(shape), _stream()),
+           "gemm_direct_f32")
     return out
 
 

@@ -418,6 +418,14 @@ class GQAAttention(Mixer):
             ops.attn_causal_bf16(q, line.k, line.v, line.page_table, ctx.seq_slot, ctx.cu_rows, tile_cu,
                                  ctx.seq_start, ctx.n_seqs, max_tiles, out, self.n_heads, self.n_kv,
                                  self.head_dim, self.scale, window)
+        elif ops.attn_f32_takes(q, line.k, line.v, self.head_dim):
+            if ctx.max_q_len == 1:
+                ops.attn_f32(q, line.k, line.v, line.page_table, out, self.n_heads, self.n_kv, self.head_dim, self.scale,
+                             window, row_slot=ctx.row_slot, row_pos=ctx.row_pos)
+            else:
+                tile_cu, max_tiles = ctx.tiles(ops.ATTN_F32_TILE)
+                ops.attn_f32(q, line.k, line.v, line.page_table, out, self.n_heads, self.n_kv, self.head_dim, self.scale,
+                             window, tiles=(ctx.seq_slot, ctx.cu_rows, tile_cu, ctx.seq_start, ctx.n_seqs, max_tiles))
         else:
             ops.attn_rows(q, line.k, line.v, line.page_table, ctx.row_slot, ctx.row_pos, out, self.n_heads, self.n_kv,
                           self.head_dim, self.scale, window)

@@ -4,9 +4,10 @@ The reference hands every projection to a vendor library (F.linear,
 engine/dryft_qwen3/model.py:153, 179-180, 237, 258-261). Here:
 
 * float32: this library's own kernels, so the 32-bit path has no reduced-precision matrix
-  mode anywhere: plain multiply-adds that read every weight once for at most 16 rows, the
-  matrix cores' full-precision instruction (``v_mfma_f32_16x16x4_f32``) in blocks of
-  128 x 128 for more, and a plain tiled kernel for sizes those do not take;
+  mode anywhere: the matrix cores' full-precision instruction (``v_mfma_f32_16x16x4_f32``),
+  with K split over a workgroup's waves (or plain multiply-adds, ``streams_f32``) for at most 16 rows, operands straight into LDS in
+  blocks chosen by the number of workgroups for more (``K`` a multiple of 32; else blocks of
+  128 x 128 through registers), and a plain tiled kernel for sizes those do not take;
 * bfloat16, at most 16 rows (decoding at small batch): this library's weight-streaming
   matrix-core kernel, which stages whole cache lines through LDS and can leave its result
   as float32 partial sums over K for the consumer to add;
@@ -63,6 +64,30 @@ def stream_plan(n: int, k: int, may_split: bool) -> tuple[int, int, int]:
     want = (k_blocks + 4 * _STREAM_BLOCKS_PER_WAVE - 1) // (4 * _STREAM_BLOCKS_PER_WAVE)
     splits = max(1, min(want, _STREAM_WORKGROUPS // tiles, k_blocks // 8, 16)) if may_split else 1
     return (splits, 1, 2) if splits > 1 else (1, 2, 2)
+
+
+def rows_f32_splits(n: int, k: int) -> int:
+    """Splits of K across workgroups for at most 16 rows of float32 values (16 outputs a workgroup): as many as give every
+    compute unit a workgroup, each at least 512 values of K."""
+    return max(1, min(_COMPUTE_UNITS // ((n + 15) // 16), k // 512, 16))
+
+
+def streams_f32(m: int, n: int, k: int) -> bool:
+    """Does a product of at most 16 rows of float32 values go to the plain multiply-adds that read whole lines, or to the
+    matrix cores with K split over a workgroup's waves? The first is bound by its arithmetic, the rows of x, and by K walked
+    chunk by chunk; the second by its trips to memory (three of them from K = 2,560 on) and by reading the rows of x again in
+    every workgroup. In a captured chain on rotating cold weights, us, first against second: 6,144 x 1,024 at 1 / 4 / 8 / 16
+    rows 7.2 / 9.3 / 11.8 / 17.3 against 9.0 / 9.8 / 10.5 / 12.3; 4,096 x 1,024 5.8 / 8.0 / 10.3 / 15.7 against 6.4 / 6.6 / 6.9 /
+    7.7; 151,936 x 1,024 105 / 120 / 183 / 352 against 136 / 139 / 155 / 182; 19,456 x 2,560 37 / 43 / 52 / 96 against 54 / 58 /
+    64 / 78; 2,560 x 9,728 29 / 41 / 48 / 70 against 35 / 37 / 42 / 50."""
+    return m == 1 or (n >= 6144 and (m <= 4 or (m <= 8 and k >= 2560)))
+
+
+def swiglu_f32_ok(h: torch.Tensor, w_gate_up: torch.Tensor) -> bool:
+    """Does the float32 gate/up product run with its activation in one kernel? The matrix cores' form only, so up to eight
+    rows not from K = 2,560 on: 19,456 x 2,560 at 4 rows 56 us against 43 and 3 for the activation; 6,144 x 1,024 9.9 against
+    9.3 and 3."""
+    return h.shape[0] <= STREAM_ROWS and ops.rows_f32_ok(h, w_gate_up) and not (h.shape[0] <= 8 and h.shape[1] >= 2560)
 
 
 def wide_plan(n: int, k: int, may_split: bool) -> tuple[int, int, int]:
@@ -181,12 +206,18 @@ def linear(x: torch.Tensor, w: torch.Tensor, *, out_dtype: torch.dtype | None = 
     n = w.shape[0]
     out_dtype = out_dtype or x.dtype
     if x.dtype == torch.float32:
+        if m <= STREAM_ROWS and ops.rows_f32_ok(x, w):
+            splits = rows_f32_splits(n, k) if allow_partials else 1
+            if splits > 1:
+                partials = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
+                return Partials(ops.gemm_rows_f32(x, w, partials, splits), splits)
+            product = ops.gemm_stream_f32 if streams_f32(m, n, k) else ops.gemm_rows_f32
+            return product(x, w, torch.empty((m, n), dtype=torch.float32, device=x.device))
         out = torch.empty((m, n), dtype=torch.float32, device=x.device)
-        if k % 4 == 0 and w.data_ptr() % 16 == 0:
-            if m <= STREAM_ROWS:
-                return ops.gemm_rows_f32(x, w, out)
-            if x.stride(0) % 4 == 0 and x.data_ptr() % 16 == 0:
-                return ops.gemm_block_f32(x, w, out, shape=0)
+        if ops.rows_f32_ok(x, w):
+            if ops.direct_f32_ok(x, w):
+                return ops.gemm_direct_f32(x, w, out)
+            return ops.gemm_block_f32(x, w, out, shape=0)
         return ops.gemm_tiled(x, w, out)
     few_ok = few_rows_ok(x, w)
     if out_dtype == torch.float32 and not allow_partials and m > STREAM_ROWS and n <= ops.NARROW_OUTPUTS and few_ok:

@@ -12,7 +12,7 @@ from ..csrc import ops
 from ..weights.spec import VECTOR
 from . import register_part
 from .base import FeedForward, Partials, matrix
-from .linear import STREAM_ROWS, few_rows_ok, linear, panel_swiglu_ok, tall_swiglu_ok
+from .linear import STREAM_ROWS, few_rows_ok, linear, panel_swiglu_ok, swiglu_f32_ok, tall_swiglu_ok
 
 
 class SwiGLU(FeedForward):
@@ -44,6 +44,8 @@ class SwiGLU(FeedForward):
             ops.relu_mul(linear(h, self.w_gate_up), act)
         elif h.dtype == torch.bfloat16 and h.shape[0] <= STREAM_ROWS and few_rows_ok(h, self.w_gate_up):
             ops.gemm_stream_swiglu_bf16(h, self.w_gate_up, act)       # the same for any K that is a multiple of 8
+        elif h.dtype == torch.float32 and swiglu_f32_ok(h, self.w_gate_up):
+            ops.gemm_rows_swiglu_f32(h, self.w_gate_up, act)
         else:
             ops.silu_mul(linear(h, self.w_gate_up), act)
         return linear(act, self.w_down, allow_partials=True)
