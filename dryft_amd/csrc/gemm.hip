@@ -805,6 +805,72 @@ static int panel_entry(const void* x, int64_t x_stride, const void* w, void* y, 
   }
 }
 
+// -------------------------------------------------------------------------------------------- few
+// The fused gate/up product with its activation for at most 16 rows and few outputs (a shared expert's, a small model's),
+// where the panel product has less than half as many workgroups as the chip has compute units and each walks all of K. Here a
+// workgroup takes eight outputs (their gate rows and then their up rows, 16 rows of W, as a wave of the panel product) and
+// its WAVES waves split K in runs of whole blocks of 64, operands straight from memory in the matrix cores' layout, four
+// blocks in flight (lane (c, g) takes the 32 bytes from 16 g on of row c, for both operands alike); the waves' sums meet in
+// LDS and are added in the order 0, 1, .... Bound by its trips to memory. In a captured chain on rotating cold weights, us
+// at 1 / 4 / 16 rows, against the panel product: 512 outputs of K 2,048 4.5 / 4.9 / 5.9 (5.6 / 5.7 / 5.9), 1,024 of 2,048
+// 5.1 / 5.5 / 6.8 (8.3 / 8.4 / 8.7), 2,048 of 2,048 5.9 / 6.2 / 7.2 (8.8 / 8.8 / 9.1), 3,072 of 1,024 5.6 / 5.8 / 7.0 (6.3 /
+// 5.9 / 6.1), 4,096 of 2,048 9.1 / 9.6 / 12.1 (10.7 / 9.3 / 9.6): each workgroup reads the rows of x again, so the more rows
+// and the more workgroups, the less it pays (`gemm_few_glu_ok` in ops.py draws the line).
+template <int WAVES>
+__global__ __launch_bounds__(WAVES * WAVE) void gemm_few_glu_kernel(const bf16_t* __restrict__ x, int64_t x_stride,
+                                                                    const bf16_t* __restrict__ w, bf16_t* __restrict__ y,
+                                                                    int M, int N, int K, GateAct act) {
+  __shared__ f32x4 sums[WAVES][WAVE];
+  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, c = lane % 16, g = lane / 16;
+  const int n0 = blockIdx.x * 8;
+  const int64_t w_row = (c < 8 ? 0 : N) + min(n0 + (c & 7), N - 1);
+  const bf16_t* wp = w + w_row * K + 16 * g;
+  const bf16_t* xp = x + (int64_t)min(c, M - 1) * x_stride + 16 * g;
+  const int per = ((K + 63) / 64 + WAVES - 1) / WAVES * 64;
+  const int k_begin = min(wave * per, K), k_end = min(k_begin + per, K);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int k0 = k_begin; k0 < k_end; k0 += 256) {
+    bf16x8 wv[8], xv[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {                          // K is a multiple of 8; beyond the run: times zeros
+      const int k = k0 + 64 * (u / 2) + 8 * (u % 2);
+      const bool in = k + 16 * g < k_end;
+      wv[u] = in ? *(const bf16x8*)(wp + k) : zero8g();
+      xv[u] = in ? *(const bf16x8*)(xp + k) : zero8g();
+    }
+    __builtin_amdgcn_sched_barrier(0);                     // every load of the four blocks before the first product
+#pragma unroll
+    for (int u = 0; u < 8; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[u], xv[u], acc, 0, 0, 0);
+  }
+  sums[wave][lane] = acc;
+  __syncthreads();
+  if (wave != 0) return;
+#pragma unroll
+  for (int v = 1; v < WAVES; ++v) acc += sums[v][lane];
+  // acc[i] is row 4g + i of the workgroup's 16 for row c of x
+  swiglu_store4(y + (int64_t)min(c, M - 1) * N, n0, N, g, acc, c < M, act);
+}
+
+// M <= 16, K a multiple of 8, rows at 16-byte addresses; W = [Wg; Wu] of 2N rows; silu, relu, or with limit > 0 the clamped
+// unit, as the panel product's.
+DRYFT_API int dryft_gemm_few_glu_bf16(const void* x, int64_t x_stride, const void* w, void* y, int M, int N, int K, int relu,
+                                      float limit, float alpha, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (M > 16 || K < 8 || K % 8 || x_stride % 8 || (((uintptr_t)x | (uintptr_t)w) & 15) || limit < 0.f || (relu && limit > 0.f))
+    return -1;
+  GateAct act;
+  act.relu = relu;
+  act.limit = limit;
+  act.alpha = alpha;
+  const dim3 grid((N + 7) / 8);
+#define FEW(W) hipLaunchKernelGGL((gemm_few_glu_kernel<W>), grid, dim3(W * WAVE), 0, stream, (const bf16_t*)x, x_stride,   \
+                                  (const bf16_t*)w, (bf16_t*)y, M, N, K, act)
+  if (K <= 1024) FEW(4);                                   // so that a wave's run is one trip to memory up to K = 2,048
+  else FEW(8);
+#undef FEW
+  return DRYFT_LAUNCH_CHECK();
+}
+
 // --------------------------------------------------------------------------------------------- mid
 // The projections back to the hidden width (few outputs, a long K) for short prompts, 65 to 256 rows: there the
 // vendor library takes 20 to 50 us for matrices that stream in 4 to 10 (Qwen3-4B: o 20 to 25 us, down 27 to 53),

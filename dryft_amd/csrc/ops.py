@@ -83,6 +83,7 @@ _SIGNATURES = {
                  "dryft_gemm_direct_f32": [_P, _L, _P, _P, _I, _I, _I, _I, _P]},
     "gemm": {"dryft_gemm_tiled": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _P],
              "dryft_gemm_stream_bf16": [_P, _L, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
+             "dryft_gemm_few_glu_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _F, _F, _P],
              "dryft_gemm_stream_swiglu_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _P],
              "dryft_gemm_wide_bf16": [_P, _L, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
              "dryft_gemm_panel_swiglu_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _P],
@@ -983,6 +984,42 @@ def gemm_wide_bf16(x, w, out, partials=None, group_blocks: int = 2, splits: int 
             raise KernelError(f"gemm_wide: out must be contiguous [{m},{n}]")
     _check(_fn("gemm", "dryft_gemm_wide_bf16")(_ptr(x), x.stride(0), _ptr(w), _ptr(out), _ptr(partials), m, n, k,
                                                int(group_blocks), int(depth), int(splits), out_f32, _stream()), "gemm_wide_bf16")
+
+
+def gemm_few_glu_ok(x, w_gate_up) -> bool:
+    """Does the fused gate/up product go to the kernel that splits K over a workgroup's waves? (Figures beside it.) Its
+    workgroups read the rows of x again: up to eight rows where the panel product has fewer than 128 workgroups, up to
+    sixteen where it has at most 64."""
+    m, k = x.shape
+    n = w_gate_up.shape[0] // 2
+    if m > 16 or k % 8 or x.stride(0) % 8 or x.data_ptr() % 16 or w_gate_up.data_ptr() % 16:
+        return False
+    workgroups = -(-n // (8 * gemm_panel_waves(n)))
+    return workgroups < 128 if m <= 8 else workgroups <= 64
+
+
+def gemm_few_glu_bf16(x, w_gate_up, out, clamped: tuple[float, float] | None = None, relu: bool = False) -> torch.Tensor:
+    """The fused gate/up product with its activation for at most 16 rows and few outputs; the units are those of
+    ``gemm_panel_swiglu_bf16``. K a multiple of 8."""
+    if relu and clamped is not None:
+        raise KernelError("gemm_few_glu: relu or the clamped unit, not both")
+    _gpu(x, "x", torch.bfloat16)
+    _gpu(w_gate_up, "w_gate_up", torch.bfloat16)
+    _gpu(out, "out", torch.bfloat16)
+    m, k = x.shape
+    two_n = w_gate_up.shape[0]
+    if not (two_n % 2 == 0 and w_gate_up.shape == (two_n, k) and w_gate_up.is_contiguous() and x.stride(1) == 1):
+        raise KernelError("gemm_few_glu: x [M,K] row-major, w [2N,K] contiguous")
+    if not (m <= 16 and k % 8 == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w_gate_up.data_ptr() % 16 == 0):
+        raise KernelError(f"gemm_few_glu: needs M <= 16, K % 8 == 0 and 16-byte aligned rows, got M={m} K={k}")
+    if not (out.shape == (m, two_n // 2) and out.is_contiguous() and out.data_ptr() % 4 == 0):
+        raise KernelError(f"gemm_few_glu: out contiguous [{m},{two_n // 2}] at a 4-byte address")
+    limit, alpha = clamped if clamped is not None else (0.0, 0.0)
+    if clamped is not None and not limit > 0:
+        raise KernelError(f"gemm_few_glu: the clamp's limit must be positive, got {limit}")
+    _check(_fn("gemm", "dryft_gemm_few_glu_bf16")(_ptr(x), x.stride(0), _ptr(w_gate_up), _ptr(out), m, two_n // 2, k,
+                                                  int(bool(relu)), float(limit), float(alpha), _stream()), "gemm_few_glu_bf16")
+    return out
 
 
 PANEL_GROUP = 128     # values of K the panel kernel moves at a time; K must be a multiple of it

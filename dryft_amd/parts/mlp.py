@@ -36,7 +36,9 @@ class SwiGLU(FeedForward):
 
     def forward(self, h, ctx):
         act = torch.empty((h.shape[0], self.inter), dtype=h.dtype, device=h.device)
-        if h.dtype == torch.bfloat16 and panel_swiglu_ok(h, self.w_gate_up):
+        if h.dtype == torch.bfloat16 and ops.gemm_few_glu_ok(h, self.w_gate_up):
+            ops.gemm_few_glu_bf16(h, self.w_gate_up, act, relu=self.relu)             # few rows and outputs, in one kernel
+        elif h.dtype == torch.bfloat16 and panel_swiglu_ok(h, self.w_gate_up):
             ops.gemm_panel_swiglu_bf16(h, self.w_gate_up, act, relu=self.relu)        # product and activation in one kernel
         elif h.dtype == torch.bfloat16 and tall_swiglu_ok(h, self.w_gate_up):
             ops.gemm_tall_swiglu_bf16(h, self.w_gate_up, act, relu=self.relu)         # the same at 65 to 256 rows
@@ -80,7 +82,9 @@ class ClampedGLU(FeedForward):
 
     def forward(self, h, ctx):
         act = torch.empty((h.shape[0], self.inter), dtype=h.dtype, device=h.device)
-        if h.dtype == torch.bfloat16 and panel_swiglu_ok(h, self.w_gate_up):
+        if h.dtype == torch.bfloat16 and ops.gemm_few_glu_ok(h, self.w_gate_up):
+            ops.gemm_few_glu_bf16(h, self.w_gate_up, act, clamped=(self.limit, self.alpha))
+        elif h.dtype == torch.bfloat16 and panel_swiglu_ok(h, self.w_gate_up):
             # up to 64 rows: product and unit in one kernel, the unit on the float accumulators
             ops.gemm_panel_swiglu_bf16(h, self.w_gate_up, act, clamped=(self.limit, self.alpha))
         else:
