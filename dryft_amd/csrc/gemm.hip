@@ -1287,6 +1287,188 @@ DRYFT_API int dryft_gemm_tall_bf16(const void* x, int64_t x_stride, const void* 
   return tall_tiles<2, false>(x, x_stride, w, partials, M, N, K, tiles, splits, per, stream);
 }
 
+// -------------------------------------------------------------------------------------------- many
+// The fused gate/up product with its activation for prompts of more than 256 rows, y[M, N] = T(T(silu(x . Wg^T)) *
+// (x . Wu^T)). Four waves own a tile of 256 rows of x by 256 rows of W, wave (wm, wn) half of either: 8 x 8 tiles of 16 x 16
+// whose sums fill the 256 accumulation registers, so one workgroup runs on a compute unit and one wave on a SIMD. A wave's
+// half of the rows of W are the gate rows of 64 outputs and then their up rows: gate and up of an output meet in one lane.
+// K goes by in steps of 64 values (rows of 128 bytes, piece p of row r at place p ^ ((r / 2) % 8), as in gemm_mid),
+// operands straight from memory into one of two places in LDS. Operands are read from LDS half a step (32 values of K)
+// ahead of the matrix instructions that use them. A step has one barrier, between its halves: there everybody has read all
+// of this step (its place is free for the step after the next, whose loads are issued one by one under the second half's
+// instructions) and the next step has arrived.
+// The matrix instructions are written as asm with the sums tied to accumulation registers: left to the compiler they move
+// through copies at the loop's head (164 of them and 90 waits for 128 instructions). What the hazard rules want around them
+// holds by distance: the operands are waited for as any register that a load writes; the sums are zeroed before a wait and a
+// barrier, and read after 32 idle cycles.
+// Bound by the matrix cores' clock and what they wait: 1.0 to 1.2 PFLOP/s of 2.5 nominal. Alone, us, beside the vendor
+// library's product and the activation kernel: 2,048 rows, 2 x 9,728 of K 2,560 201 (227 + 23); 12,806 rows 999 (951 + 135);
+// 5,099 rows, 2 x 8,192 of 2,048 271 (244 + 47); 2,048 rows, 2 x 3,072 of 1,024 32 (30 + 8); 517 rows, 2 x 9,728 of 2,560 69
+// (54 + 8). In whole steps it is ahead at 2,048 rows (12 layers 6.75 -> 6.53 ms) and level at 12,806, so it serves products
+// below 2.5e11 operations (the rule: linear.py). Tried beside it: one workgroup a unit that walks several tiles and fetches
+// the next one's first steps under the stores (10 % slower: the branches it needs break the order of instructions), tiles of
+// 256 x 128 with three steps in LDS (194 at 2,048 rows, but 1,165 at 12,806, and slower in the step), 256 x 192 (206), 128 x
+// 128 (219), other orders of tiles and places in LDS (the same).
+#define MANY_STEP 64
+#define MANY_TILES 8                         // of 16 rows of either operand, a wave
+#define MANY_LDS (2 * 2 * 32 * MANY_TILES * 2 * MANY_STEP)
+
+__device__ __forceinline__ void mfma_in_place(f32x4& acc, const bf16x8& a, const bf16x8& b) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+}
+
+__global__ __launch_bounds__(256, 1) void gemm_many_glu_kernel(const bf16_t* __restrict__ x, int64_t x_stride,
+                                                               const bf16_t* __restrict__ w, bf16_t* __restrict__ y, int M,
+                                                               int N, int K, int m_tiles, int n_tiles, GateAct act) {
+  extern __shared__ __align__(16) unsigned char many_lds[];
+  constexpr int MT = MANY_TILES, NT = MANY_TILES, STAGES = 2;
+  constexpr int RB = 2 * MANY_STEP, BM = 32 * MT, BN = 32 * NT, X_BYTES = BM * RB, STAGE_BYTES = (BM + BN) * RB;
+  constexpr int X_LOADS = BM / 32, W_LOADS = BN / 32, LOADS = X_LOADS + W_LOADS;      // of 1 KB (8 rows), per wave and step
+  constexpr int HALF = 8 * NT;                             // outputs of a wave: as many gate rows, then as many up rows
+  constexpr int GROUP = 8;                                 // tiles of rows that share their rows of W while those are near
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int lane = threadIdx.x % WAVE, c = lane % 16, g = lane / 16;
+  const int wm = wave / 2, wn = wave % 2;
+  // Workgroups go to the eight dies in turn, each die with an L2 of its own: a die gets neighbouring tiles, column by column
+  // of GROUP tiles of rows. The grid is 8 * ceil(tiles / 8); those beyond the last tile leave at once.
+  const int total = m_tiles * n_tiles, a_die = (total + 7) / 8;
+  const int id = (int)(blockIdx.x % 8) * a_die + (int)(blockIdx.x / 8);
+  if (id >= total) return;
+  const int group = id / (GROUP * n_tiles), in_group = id % (GROUP * n_tiles);
+  const int group_tiles = min(GROUP, m_tiles - group * GROUP);
+  const int m0 = (group * GROUP + in_group % group_tiles) * BM, n0 = in_group / group_tiles * 2 * HALF;
+  const int steps = K / MANY_STEP;
+  uint32_t x_from[X_LOADS], w_from[W_LOADS];
+#pragma unroll
+  for (int i = 0; i < X_LOADS; ++i) {
+    const int r = 8 * (wave * X_LOADS + i) + lane / 8;     // row of the tile's part of x
+    x_from[i] = (uint32_t)min(m0 + r, M - 1) * (uint32_t)x_stride * 2u + (((lane % 8) ^ ((r >> 1) & 7)) << 4);
+  }
+#pragma unroll
+  for (int i = 0; i < W_LOADS; ++i) {
+    const int r = 8 * (wave * W_LOADS + i) + lane / 8;     // row of the tile's part of W: wave column, gate or up, output
+    const int in_wave = r % (2 * HALF), o = n0 + r / (2 * HALF) * HALF + in_wave % HALF;
+    const int row = (in_wave < HALF ? 0 : N) + min(o, N - 1);
+    w_from[i] = (uint32_t)row * (uint32_t)K * 2u + (((lane % 8) ^ ((r >> 1) & 7)) << 4);
+  }
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)many_lds);
+  auto load_one = [&](int i, int step, int stage) __attribute__((always_inline)) {
+    const int64_t at = (int64_t)min(step, steps - 1) * RB;             // past the end: the last step again, read by nobody
+    if (i < X_LOADS)
+      panel_load16((const unsigned char*)x + at, x_from[i], lds0 + stage * STAGE_BYTES + (wave * X_LOADS + i) * 1024);
+    else
+      panel_load16((const unsigned char*)w + at, w_from[i - X_LOADS],
+                   lds0 + stage * STAGE_BYTES + X_BYTES + (wave * W_LOADS + i - X_LOADS) * 1024);
+  };
+  f32x4 acc[MT][NT];                                       // [tile of 16 rows][NT / 2 tiles of gates, then of ups]
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int sw = (c >> 1) & 7;                             // row 16 t + c of any tile is swizzled like row c
+  const unsigned char* xr = many_lds + (16 * MT * wm + c) * RB;
+  const unsigned char* wr = many_lds + X_BYTES + (16 * NT * wn + c) * RB;
+  bf16x8 a[2][NT], b[2][MT];
+  auto read_pair = [&](int u, int stage, int t) __attribute__((always_inline)) {     // tile t of either operand
+    const int place = ((4 * u + g) ^ sw) << 4;
+    if (t < NT) a[u][t] = *(const bf16x8*)(wr + stage * STAGE_BYTES + 16 * t * RB + place);
+    b[u][t] = *(const bf16x8*)(xr + stage * STAGE_BYTES + 16 * t * RB + place);
+  };
+#pragma unroll
+  for (int f = 0; f < STAGES; ++f)
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) load_one(i, f, f);
+  panel_wait<(STAGES - 1) * LOADS>();
+  __syncthreads();
+  int cur = 0;
+#pragma unroll
+  for (int t = 0; t < MT; ++t) read_pair(0, 0, t);
+  for (int s = 0; s < steps; ++s) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {                         // the second half's reads under the first half's products
+      read_pair(1, cur, m);
+#pragma unroll
+      for (int n = 0; n < NT; ++n) mfma_in_place(acc[m][n], a[0][n], b[0][m]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // every operand of this step has been read, and the next step's loads have arrived: lgkmcnt(0) and vmcnt(0)
+    __builtin_amdgcn_s_waitcnt(0x0070);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    constexpr int PER = (LOADS + MT - 1) / MT;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {                         // the next step's first half under the second half's products
+#pragma unroll
+      for (int i = 0; i < PER; ++i)
+        if (m * PER + i < LOADS) load_one(m * PER + i, s + STAGES, cur);
+      read_pair(0, cur ^ 1, m);
+#pragma unroll
+      for (int n = 0; n < NT; ++n) mfma_in_place(acc[m][n], a[1][n], b[1][m]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    cur ^= 1;
+  }
+  panel_wait<0>();                                         // the loads past the end have landed before the waves leave
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");       // and the last sums may be read
+  __builtin_amdgcn_sched_barrier(0);
+  // acc[m][n][i] is the gate of output 16 n + 4g + i of the wave's for row 16 m + c, acc[m][n + NT / 2][i] its up
+  const bool clamped = act.limit > 0.f, whole = N % 4 == 0;
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int row = m0 + 16 * (MT * wm + m) + c;
+    __builtin_amdgcn_sched_barrier(0);
+    if (row >= M) continue;
+#pragma unroll
+    for (int n = 0; n < NT / 2; ++n) {
+      const int o = n0 + HALF * wn + 16 * n + 4 * g;
+      bf16_t v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float gate = acc[m][n][i], up = acc[m][n + NT / 2][i];
+        v[i] = act.relu ? float_to_bf16(fmaxf(gate, 0.f) * up)
+               : clamped ? float_to_bf16(clamped_unit(gate, up, act))
+                         : float_to_bf16(rounded_as<bf16_t>(silu_for_bf16(rounded_as<bf16_t>(gate))) * rounded_as<bf16_t>(up));
+      }
+      bf16_t* to = y + (int64_t)row * N + o;
+      if (whole) {                                         // then o + 3 < N where o < N, and the address is a multiple of 8
+        if (o < N) *(uint2*)to = uint2{v[0].bits | ((uint32_t)v[1].bits << 16), v[2].bits | ((uint32_t)v[3].bits << 16)};
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (o + i < N) to[i] = v[i];
+      }
+    }
+  }
+}
+
+// Any M. W = [Wg; Wu] of 2N rows; silu, relu, or with limit > 0 the clamped unit, as the panel product's. K a multiple of
+// 64; x and W within reach of 32-bit byte offsets.
+DRYFT_API int dryft_gemm_many_glu_bf16(const void* x, int64_t x_stride, const void* w, void* y, int M, int N, int K,
+                                       int relu, float limit, float alpha, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (K <= 0 || K % MANY_STEP || x_stride % 8 || (((uintptr_t)x | (uintptr_t)w) & 15) || ((uintptr_t)y & 7) ||
+      (int64_t)2 * N * K * 2 >= (int64_t)4 << 30 || (int64_t)M * x_stride * 2 >= (int64_t)4 << 30 || limit < 0.f ||
+      (relu && limit > 0.f))
+    return -1;
+  GateAct act;
+  act.relu = relu;
+  act.limit = limit;
+  act.alpha = alpha;
+  static bool raised = false;                              // more dynamic LDS than the default limit allows
+  if (!raised) {
+    if (hipFuncSetAttribute((const void*)gemm_many_glu_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, MANY_LDS) != hipSuccess)
+      return -2;
+    raised = true;
+  }
+  const int m_tiles = (M + 32 * MANY_TILES - 1) / (32 * MANY_TILES), n_tiles = (N + 16 * MANY_TILES - 1) / (16 * MANY_TILES);
+  if ((int64_t)m_tiles * n_tiles > 1 << 28) return -1;
+  hipLaunchKernelGGL(gemm_many_glu_kernel, dim3(8 * ((m_tiles * n_tiles + 7) / 8)), dim3(256), MANY_LDS, stream,
+                     (const bf16_t*)x, x_stride, (const bf16_t*)w, (bf16_t*)y, M, N, K, m_tiles, n_tiles, act);
+  return DRYFT_LAUNCH_CHECK();
+}
+
 // ------------------------------------------------------------------------------------------- block
 // Many rows: a workgroup owns a block of rows by outputs (128 x 128 with four waves, 256 x 256 with eight) and
 // walks K in steps of 64. Its threads copy the block's rows of x and of W for one step into LDS (whole cache

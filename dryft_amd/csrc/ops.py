@@ -83,6 +83,7 @@ _SIGNATURES = {
                  "dryft_gemm_direct_f32": [_P, _L, _P, _P, _I, _I, _I, _I, _P]},
     "gemm": {"dryft_gemm_tiled": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _P],
              "dryft_gemm_stream_bf16": [_P, _L, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
+             "dryft_gemm_many_glu_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _F, _F, _P],
              "dryft_gemm_few_glu_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _F, _F, _P],
              "dryft_gemm_stream_swiglu_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _P],
              "dryft_gemm_wide_bf16": [_P, _L, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
@@ -1065,6 +1066,33 @@ def gemm_panel_swiglu_bf16(x, w_gate_up, out, waves: int = 0, clamped: tuple[flo
         return out
     _check(_fn("gemm", "dryft_gemm_panel_swiglu_bf16")(_ptr(x), x.stride(0), _ptr(w_gate_up), _ptr(out), m, two_n // 2, k,
                                                        int(waves), int(bool(relu)), _stream()), "gemm_panel_swiglu_bf16")
+    return out
+
+
+MANY_STEP = 64      # values of K gemm_many_glu moves at a time; K must be a multiple of it
+
+
+def gemm_many_glu_bf16(x, w_gate_up, out, clamped: tuple[float, float] | None = None, relu: bool = False) -> torch.Tensor:
+    """The fused gate/up product with its activation for many rows; the units are those of ``gemm_panel_swiglu_bf16``."""
+    if relu and clamped is not None:
+        raise KernelError("gemm_many_glu: relu or the clamped unit, not both")
+    _gpu(x, "x", torch.bfloat16)
+    _gpu(w_gate_up, "w_gate_up", torch.bfloat16)
+    _gpu(out, "out", torch.bfloat16)
+    m, k = x.shape
+    two_n = w_gate_up.shape[0]
+    if not (two_n % 2 == 0 and w_gate_up.shape == (two_n, k) and w_gate_up.is_contiguous() and x.stride(1) == 1):
+        raise KernelError("gemm_many_glu: x [M,K] row-major, w [2N,K] contiguous")
+    if not (k % MANY_STEP == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w_gate_up.data_ptr() % 16 == 0):
+        raise KernelError(f"gemm_many_glu: needs K % {MANY_STEP} == 0 and 16-byte aligned rows, got K={k}")
+    if not (out.shape == (m, two_n // 2) and out.is_contiguous() and out.data_ptr() % 8 == 0):
+        raise KernelError(f"gemm_many_glu: out contiguous [{m},{two_n // 2}] at an 8-byte address")
+    limit, alpha = clamped if clamped is not None else (0.0, 0.0)
+    if clamped is not None and not limit > 0:
+        raise KernelError(f"gemm_many_glu: the clamp's limit must be positive, got {limit}")
+    _check(_fn("gemm", "dryft_gemm_many_glu_bf16")(_ptr(x), x.stride(0), _ptr(w_gate_up), _ptr(out), m, two_n // 2, k,
+                                                   int(bool(relu)), float(limit), float(alpha), _stream()),
+           "gemm_many_glu_bf16")
     return out
 
 

@@ -22,7 +22,8 @@ engine/dryft_qwen3/model.py:153, 179-180, 237, 258-261). Here:
   for sizes the vendor library does not take;
 * bfloat16, 65 to 256 rows (short prompts, decoding at large batch) where the consumer adds partial sums and K is a
   multiple of 64: this library's kernel whose waves each own rows of x, operands straight into LDS (``tall_plan``);
-  the fused gate/up product of as many rows goes to its other form (``tall_swiglu_ok``);
+  the fused gate/up product of as many rows goes to its other form (``tall_swiglu_ok``), of more rows to this library's
+  kernel of 256 rows a workgroup where that fills the chip (``many_glu_ok``);
 * bfloat16, more than 16 rows, float32 results of at most 64 outputs (gates, routers, low-rank projections): this
   library's kernel that reads the rows once and splits K over the waves of a workgroup;
 * bfloat16, otherwise (prompts, decoding at large batch): the vendor library through
@@ -36,6 +37,7 @@ from __future__ import annotations
 
 import contextlib
 import functools
+import math
 import os
 import tempfile
 
@@ -187,6 +189,27 @@ def tall_swiglu_ok(x: torch.Tensor, w_gate_up: torch.Tensor) -> bool:
     m, k = x.shape
     return WIDE_ROWS < m <= ops.TALL_ROWS and k % ops.TALL_GROUP == 0 and few_rows_ok(x, w_gate_up) and \
         within_direct_reach(x, w_gate_up) and w_gate_up.numel() * w_gate_up.element_size() <= _TALL_SWIGLU_BYTES
+
+
+@functools.lru_cache(maxsize=None)
+def _many_glu_pays(m: int, n: int, k: int) -> bool:
+    """Is the fused gate/up product of many rows (256 rows by 128 outputs a workgroup) expected to be ahead of the vendor
+    library's product and the activation kernel? Not from 2.5e11 operations on (there the library reaches 1.3 PFLOP/s, and a
+    step of 12,806 rows of Qwen3-4B takes the same time with either), nor where the tiles fill the last round of the compute
+    units badly. Times in us: 1.67 per step of 64 values of K and round of the compute units and 6 to fill and drain, from 2,048
+    and 5,099 rows of three shapes; the library at 0.94 PFLOP/s, the activation at 4.6 TB/s. (What both took: beside the
+    kernel.) The prompt of 2,048 tokens through 12 layers of Qwen3-4B: 6.75 -> 6.53 ms."""
+    flops = 4.0 * m * n * k
+    rounds = -(-(-(-m // 256) * -(-n // 128)) // _COMPUTE_UNITS)
+    library = flops / 0.94e9 + m * n * 6 / 4.6e6 + 3
+    return flops < 2.5e11 and 6 + 1.67 * (k // ops.MANY_STEP) * rounds < 0.97 * library
+
+
+def many_glu_ok(x: torch.Tensor, w_gate_up: torch.Tensor) -> bool:
+    """``_many_glu_pays``, and the operands suit the kernel."""
+    m, k = x.shape
+    return m > ops.TALL_ROWS and k % ops.MANY_STEP == 0 and few_rows_ok(x, w_gate_up) and \
+        within_direct_reach(x, w_gate_up) and _many_glu_pays(m, w_gate_up.shape[0] // 2, k)
 
 
 def within_direct_reach(x: torch.Tensor, w: torch.Tensor) -> bool:

@@ -12,7 +12,7 @@ from ..csrc import ops
 from ..weights.spec import VECTOR
 from . import register_part
 from .base import FeedForward, Partials, matrix
-from .linear import STREAM_ROWS, few_rows_ok, linear, panel_swiglu_ok, swiglu_f32_ok, tall_swiglu_ok
+from .linear import STREAM_ROWS, few_rows_ok, linear, many_glu_ok, panel_swiglu_ok, swiglu_f32_ok, tall_swiglu_ok
 
 
 class SwiGLU(FeedForward):
@@ -42,6 +42,8 @@ class SwiGLU(FeedForward):
             ops.gemm_panel_swiglu_bf16(h, self.w_gate_up, act, relu=self.relu)        # product and activation in one kernel
         elif h.dtype == torch.bfloat16 and tall_swiglu_ok(h, self.w_gate_up):
             ops.gemm_tall_swiglu_bf16(h, self.w_gate_up, act, relu=self.relu)         # the same at 65 to 256 rows
+        elif h.dtype == torch.bfloat16 and many_glu_ok(h, self.w_gate_up):
+            ops.gemm_many_glu_bf16(h, self.w_gate_up, act, relu=self.relu)     # and beyond
         elif self.relu:
             ops.relu_mul(linear(h, self.w_gate_up), act)
         elif h.dtype == torch.bfloat16 and h.shape[0] <= STREAM_ROWS and few_rows_ok(h, self.w_gate_up):
@@ -87,6 +89,8 @@ class ClampedGLU(FeedForward):
         elif h.dtype == torch.bfloat16 and panel_swiglu_ok(h, self.w_gate_up):
             # up to 64 rows: product and unit in one kernel, the unit on the float accumulators
             ops.gemm_panel_swiglu_bf16(h, self.w_gate_up, act, clamped=(self.limit, self.alpha))
+        elif h.dtype == torch.bfloat16 and many_glu_ok(h, self.w_gate_up):
+            ops.gemm_many_glu_bf16(h, self.w_gate_up, act, clamped=(self.limit, self.alpha))
         else:
             ops.glu_clamped(linear(h, self.w_gate_up), act, self.limit, self.alpha)
         return linear(act, self.w_down, allow_partials=True)
