@@ -285,11 +285,37 @@ __global__ __launch_bounds__(256) void stream_norm_kernel(const void* __restrict
     store_from_float(y + base + i, (held[i] - mean) * inv * load_vector(w, i, w_f32) + (bias ? bias[i] : 0.f));
 }
 
-// The same for rows whose width is a multiple of 8 with 16-byte aligned operands: a thread owns runs of 8
-// contiguous values, moves them with 16-byte loads and stores, and asks for four partial sums at a time, so that a
-// row of a decoding step (latency, not bandwidth) costs a few trips to memory instead of one per value and part.
-template <typename T, typename D>
-__global__ __launch_bounds__(256) void stream_norm_vec_kernel(const void* __restrict__ x_in, int x_kind,
+// d += sum_p parts[p] of eight neighbouring values, in the order 0, 1, ...; eight parts' loads in flight
+template <typename D>
+__device__ __forceinline__ void add_parts8(const D* at, int n_parts, int64_t stride, float (&d)[8]) {
+  constexpr int AHEAD = sizeof(D) == 4 ? 8 : 1;             // a delta in the 16-bit dtype is one tensor: no registers for more
+  for (int p0 = 0; p0 < n_parts; p0 += AHEAD) {
+    float t[AHEAD][8];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+      if (p0 + u < n_parts) load8_as_float(at + (p0 + u) * stride, t[u]);
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+      if (p0 + u < n_parts) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) d[j] += t[u][j];
+      }
+  }
+}
+
+__device__ __forceinline__ void load8_vector(const void* p, int i, int is_f32, float (&v)[8]) {
+  if (is_f32) load8_as_float((const float*)p + i, v);
+  else load8_as_float((const bf16_t*)p + i, v);
+}
+
+// The same for rows whose width is a multiple of 8 with 16-byte aligned operands. What a row of a decoding step costs is
+// trips to memory one after the other, not bytes: a thread owns RUNS runs of 8 neighbouring values, asks for all its
+// operands at once (the weights too, which nothing needs before the sums) and keeps the row in registers between the passes.
+// Four rows of 2,048 in decoding steps, partial sums as delta: 4.4-4.8 us where a form that held the row in LDS and read the
+// weights after the sums took 5.2; 5,099 rows are bound by their bytes and take 23-28 us in both forms.
+#define STREAM_NORM_THREADS 512
+template <typename T, typename D, int RUNS>
+__global__ __launch_bounds__(STREAM_NORM_THREADS) void stream_norm_vec_kernel(const void* __restrict__ x_in, int x_kind,
                                                               const D* __restrict__ delta, int n_partials,
                                                               int64_t partial_stride, const void* __restrict__ wb,
                                                               int wb_f32, const T* __restrict__ extra,
@@ -297,132 +323,115 @@ __global__ __launch_bounds__(256) void stream_norm_vec_kernel(const void* __rest
                                                               const void* __restrict__ w, int w_f32,
                                                               const float* __restrict__ bias, float* __restrict__ x_out, T* __restrict__ y, int width,
                                                               float eps, int form, int groups) {
-  extern __shared__ __attribute__((aligned(16))) float held[];
-  __shared__ float scratch[16], sums[STREAM_NORM_MAX_GROUPS];
+  __shared__ float scratch[16], sums[STREAM_NORM_MAX_GROUPS], squares[RUNS * STREAM_NORM_THREADS];
+  constexpr bool EARLY = RUNS == 1;                        // longer rows have no registers for all weights at once
   const int64_t base = (int64_t)blockIdx.x * width;
-  float inv_d = 1.f, mean_d = 0.f;
-  if (n_partials > 0) {
-    float ss = 0.f, sd = 0.f;
-    for (int i = threadIdx.x * 8; i < width; i += blockDim.x * 8) {
-      float d[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      int p = 0;
-      for (; p + 4 <= n_partials; p += 4) {               // four loads in flight; added in the order 0, 1, ...
-        float t[4][8];
+  const bool normed = y != nullptr && !(form & 4);
+  float v[RUNS][8], d[RUNS][8], wv[RUNS][8], wbv[RUNS][8], bv[RUNS][8];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) load8_as_float(delta + (p + u) * partial_stride + base + i, t[u]);
+  for (int r = 0; r < RUNS; ++r) {
+    const int i = (r * blockDim.x + threadIdx.x) * 8;
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+    for (int j = 0; j < 8; ++j) v[r][j] = d[r][j] = bv[r][j] = 0.f;
+    if (i >= width) continue;
+    if (x_kind == 2) load8_as_float((const float*)x_in + base + i, v[r]);
+    else if (x_kind == 1) load8_as_float((const T*)x_in + base + i, v[r]);
+    if (EARLY && wb != nullptr) load8_vector(wb, i, wb_f32, wbv[r]);
+    if (EARLY && normed) load8_vector(w, i, w_f32, wv[r]);
+    if (EARLY && normed && bias != nullptr) load8_as_float(bias + i, bv[r]);
+    add_parts8(delta + base + i, n_partials, partial_stride, d[r]);
+  }
+  if (n_partials > 0 && wb != nullptr) {
+    float mean = 0.f, ss = 0.f;
+    if (form & 1) {
+      float sd = 0.f;
 #pragma unroll
-          for (int j = 0; j < 8; ++j) d[j] += t[u][j];
-      }
-      for (; p < n_partials; ++p) {
-        float t[8];
-        load8_as_float(delta + p * partial_stride + base + i, t);
+      for (int r = 0; r < RUNS; ++r)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) d[j] += t[j];
-      }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) { ss += d[j] * d[j]; sd += d[j]; }
-      store8_from_float(held + i, d);
+        for (int j = 0; j < 8; ++j) sd += d[r][j];         // values beyond the row are zeros
+      mean = block_sum(sd, scratch) / (float)width;
     }
-    if (wb != nullptr) {
-      if (form & 1) {
-        mean_d = block_sum(sd, scratch) / (float)width;
-        ss = 0.f;
-        for (int i = threadIdx.x * 8; i < width; i += blockDim.x * 8) {
-          float d[8];
-          load8_as_float(held + i, d);
 #pragma unroll
-          for (int j = 0; j < 8; ++j) ss += (d[j] - mean_d) * (d[j] - mean_d);
-        }
+    for (int r = 0; r < RUNS; ++r)
+      if ((int)(r * blockDim.x + threadIdx.x) * 8 < width) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) ss += (d[r][j] - mean) * (d[r][j] - mean);
       }
-      inv_d = rsqrtf(block_sum(ss, scratch) / (float)width + eps);
+    const float inv = rsqrtf(block_sum(ss, scratch) / (float)width + eps);
+#pragma unroll
+    for (int r = 0; r < RUNS; ++r) {
+      const int i = (r * blockDim.x + threadIdx.x) * 8;
+      if (!EARLY && i < width) load8_vector(wb, i, wb_f32, wbv[r]);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) d[r][j] = i < width ? (d[r][j] - mean) * inv * wbv[r][j] : 0.f;
     }
   }
   float ss = 0.f, sv = 0.f;
-  for (int i = threadIdx.x * 8; i < width; i += blockDim.x * 8) {
-    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, t[8];
-    if (x_kind == 2) load8_as_float((const float*)x_in + base + i, v);
-    else if (x_kind == 1) load8_as_float((const T*)x_in + base + i, v);
-    if (n_partials > 0) {
-      load8_as_float(held + i, t);
-      if (wb != nullptr) {
-        float wv[8];
-        if (wb_f32) load8_as_float((const float*)wb + i, wv); else load8_as_float((const bf16_t*)wb + i, wv);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] += (t[j] - mean_d) * inv_d * wv[j];
-      } else {
+  for (int r = 0; r < RUNS; ++r) {
+    const int i = (r * blockDim.x + threadIdx.x) * 8;
+    if (i >= width) continue;
+    float t[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] += t[j];
-      }
-    }
+    for (int j = 0; j < 8; ++j) v[r][j] += d[r][j];
     if (extra != nullptr) {
       load8_as_float(extra + base + i, t);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] += t[j];
+      for (int j = 0; j < 8; ++j) v[r][j] += t[j];
     }
     if (vec != nullptr) {
-      if (vec_f32) load8_as_float((const float*)vec + i, t); else load8_as_float((const bf16_t*)vec + i, t);
+      load8_vector(vec, i, vec_f32, t);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] += t[j];
+      for (int j = 0; j < 8; ++j) v[r][j] += t[j];
     }
-    store8_from_float(held + i, v);
-    if (x_out != nullptr) store8_from_float(x_out + base + i, v);
+    if (x_out != nullptr) store8_from_float(x_out + base + i, v[r]);
+    float own = 0.f;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) { ss += v[j] * v[j]; sv += v[j]; }
+    for (int j = 0; j < 8; ++j) { own += v[r][j] * v[r][j]; sv += v[r][j]; }
+    ss += own;
+    if (groups > 1) squares[r * blockDim.x + threadIdx.x] = own;
   }
   if (y == nullptr) return;
-  if (form & 4) {
-    for (int i = threadIdx.x * 8; i < width; i += blockDim.x * 8) {
-      float v[8];
-      load8_as_float(held + i, v);
-      store8_from_float(y + base + i, v);
+  float mean = 0.f, inv = 1.f;
+  const int len = width / groups;
+  if (normed && groups > 1) {
+    // a part's sum of squares from those of its runs, where runs lie in one part; the launcher sends other widths elsewhere
+    __syncthreads();
+    const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, waves = blockDim.x / WAVE, runs = len / 8;
+    for (int p = wave; p < groups; p += waves) {
+      float own = 0.f;
+      for (int k = lane; k < runs; k += WAVE) own += squares[p * runs + k];
+      own = wave_sum(own);
+      if (lane == 0) sums[p] = rsqrtf(own / (float)len + eps);
     }
-    return;
+    __syncthreads();
+  } else if (normed) {
+    if (form & 2) {
+      mean = block_sum(sv, scratch) / (float)width;
+      ss = 0.f;
+#pragma unroll
+      for (int r = 0; r < RUNS; ++r)
+        if ((int)(r * blockDim.x + threadIdx.x) * 8 < width) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) ss += (v[r][j] - mean) * (v[r][j] - mean);
+        }
+    }
+    inv = rsqrtf(block_sum(ss, scratch) / (float)width + eps);
   }
-  if (groups > 1) {
-    const int cuts = part_squares(held, width, groups, sums), len = width / groups;
-    for (int i = threadIdx.x * 8; i < width; i += blockDim.x * 8) {
-      float v[8], wv[8];
-      load8_as_float(held + i, v);
-      if (w_f32) load8_as_float((const float*)w + i, wv); else load8_as_float((const bf16_t*)w + i, wv);
-      if (len % 8 == 0) {                    // eight neighbours lie in one part
-        const float inv = part_inverse(sums, cuts, i / len, len, eps);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] *= inv * wv[j];
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] *= part_inverse(sums, cuts, (i + j) / len, len, eps) * wv[j];
+  for (int r = 0; r < RUNS; ++r) {
+    const int i = (r * blockDim.x + threadIdx.x) * 8;
+    if (i >= width) continue;
+    if (normed) {
+      if (!EARLY) {
+        load8_vector(w, i, w_f32, wv[r]);
+        if (bias != nullptr) load8_as_float(bias + i, bv[r]);
       }
-      store8_from_float(y + base + i, v);
-    }
-    return;
-  }
-  float mean = 0.f;
-  if (form & 2) {
-    mean = block_sum(sv, scratch) / (float)width;
-    ss = 0.f;
-    for (int i = threadIdx.x * 8; i < width; i += blockDim.x * 8) {
-      float v[8];
-      load8_as_float(held + i, v);
+      if (groups > 1) inv = sums[i / len];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) ss += (v[j] - mean) * (v[j] - mean);
+      for (int j = 0; j < 8; ++j) v[r][j] = (v[r][j] - mean) * inv * wv[r][j] + bv[r][j];
     }
-  }
-  const float inv = rsqrtf(block_sum(ss, scratch) / (float)width + eps);
-  for (int i = threadIdx.x * 8; i < width; i += blockDim.x * 8) {
-    float v[8], wv[8];
-    load8_as_float(held + i, v);
-    if (w_f32) load8_as_float((const float*)w + i, wv); else load8_as_float((const bf16_t*)w + i, wv);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = (v[j] - mean) * inv * wv[j];
-    if (bias != nullptr) {
-      float bv[8];
-      load8_as_float(bias + i, bv);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] += bv[j];
-    }
-    store8_from_float(y + base + i, v);
+    store8_from_float(y + base + i, v[r]);
   }
 }
 
@@ -446,19 +455,28 @@ DRYFT_API int dryft_stream_norm(const void* x_in, int x_kind, const void* delta,
   hipLaunchKernelGGL((stream_norm_kernel<TT, DD>), grid, block, lds, stream, x_in, x_kind, (const DD*)delta,        \
                      n_partials, partial_stride, wb, wb_f32, (const TT*)extra, vec, vec_f32, w, w_f32, bias, x_out, \
                      (TT*)y, width, eps, form, groups)
-#define SNV(TT, DD)                                                                                                  \
-  hipLaunchKernelGGL((stream_norm_vec_kernel<TT, DD>), grid, block, lds, stream, x_in, x_kind, (const DD*)delta,    \
+  const int runs = width / 8, per = (runs + STREAM_NORM_THREADS - 1) / STREAM_NORM_THREADS;    // at most four a thread
+  const dim3 threads((((runs + per - 1) / per) + WAVE - 1) / WAVE * WAVE);
+#define SNR(TT, DD, R)                                                                                               \
+  hipLaunchKernelGGL((stream_norm_vec_kernel<TT, DD, R>), grid, threads, 0, stream, x_in, x_kind, (const DD*)delta,  \
                      n_partials, partial_stride, wb, wb_f32, (const TT*)extra, vec, vec_f32, w, w_f32, bias, x_out, \
                      (TT*)y, width, eps, form, groups)
+#define SNV(TT, DD)                                                                                                  \
+  do {                                                                                                               \
+    if (per <= 1) SNR(TT, DD, 1);                                                                                     \
+    else if (per <= 2) SNR(TT, DD, 2);                                                                                \
+    else SNR(TT, DD, 4);                                                                                              \
+  } while (0)
   const bool aligned = (((uintptr_t)x_in | (uintptr_t)delta | (uintptr_t)wb | (uintptr_t)extra | (uintptr_t)vec |
                          (uintptr_t)w | (uintptr_t)bias | (uintptr_t)x_out | (uintptr_t)y) & 15) == 0 && partial_stride % 4 == 0;
-  if (width % 8 == 0 && aligned) {
+  if (width % 8 == 0 && aligned && (groups == 1 || (width / groups) % 8 == 0)) {
     if (is_f32) SNV(float, float);
     else if (delta_kind == 2) SNV(bf16_t, float);
     else SNV(bf16_t, bf16_t);
     return DRYFT_LAUNCH_CHECK();
   }
 #undef SNV
+#undef SNR
   if (is_f32) SN(float, float);
   else if (delta_kind == 2) SN(bf16_t, float);
   else SN(bf16_t, bf16_t);
@@ -499,6 +517,52 @@ __global__ __launch_bounds__(256) void rms_pair_mean_kernel(const DA* __restrict
     out[base + i] = 0.5f * (held[i] * inv_a * wa[i] + held[width + i] * inv_b * wb[i]);
 }
 
+// The same for rows whose width is a multiple of 8 with 16-byte aligned operands, in registers: every operand asked for at
+// once, one trip to memory where the kernel above takes one per part and pass. Four rows of 2,048 in decoding
+// steps: 4.7 us where the kernel above takes 14.7; 5,099 rows: 24.6 and 39.1 us.
+template <typename DA, typename DB, int RUNS>
+__global__ __launch_bounds__(STREAM_NORM_THREADS) void rms_pair_mean_vec_kernel(
+    const DA* __restrict__ a, int a_parts, int64_t a_stride, const float* __restrict__ a_bias, const float* __restrict__ wa,
+    const DB* __restrict__ b, int b_parts, int64_t b_stride, const float* __restrict__ b_bias, const float* __restrict__ wb,
+    float* __restrict__ out, int width, float eps) {
+  __shared__ float scratch[16];
+  constexpr bool EARLY = RUNS == 1;
+  const int64_t base = (int64_t)blockIdx.x * width;
+  float x[RUNS][8], y[RUNS][8], xw[RUNS][8], yw[RUNS][8];
+  float sa = 0.f, sb = 0.f;
+#pragma unroll
+  for (int r = 0; r < RUNS; ++r) {
+    const int i = (r * blockDim.x + threadIdx.x) * 8;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[r][j] = y[r][j] = 0.f;
+    if (i >= width) continue;
+    if (a_bias) load8_as_float(a_bias + i, x[r]);
+    if (b_bias) load8_as_float(b_bias + i, y[r]);
+    if (EARLY) {
+      load8_as_float(wa + i, xw[r]);
+      load8_as_float(wb + i, yw[r]);
+    }
+    add_parts8(a + base + i, a_parts, a_stride, x[r]);
+    add_parts8(b + base + i, b_parts, b_stride, y[r]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) { sa += x[r][j] * x[r][j]; sb += y[r][j] * y[r][j]; }
+  }
+  const float inv_a = rsqrtf(block_sum(sa, scratch) / (float)width + eps);
+  const float inv_b = rsqrtf(block_sum(sb, scratch) / (float)width + eps);
+#pragma unroll
+  for (int r = 0; r < RUNS; ++r) {
+    const int i = (r * blockDim.x + threadIdx.x) * 8;
+    if (i >= width) continue;
+    if (!EARLY) {
+      load8_as_float(wa + i, xw[r]);
+      load8_as_float(wb + i, yw[r]);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[r][j] = 0.5f * (x[r][j] * inv_a * xw[r][j] + y[r][j] * inv_b * yw[r][j]);
+    store8_from_float(out + base + i, x[r]);
+  }
+}
+
 // a_kind / b_kind: 1 = activation dtype [rows, width], 2 = float partial sums [parts, rows, width].
 DRYFT_API int dryft_rms_pair_mean(const void* a, int a_kind, int a_parts, int64_t a_stride, const float* a_bias,
                                   const float* wa, const void* b, int b_kind, int b_parts, int64_t b_stride,
@@ -509,6 +573,27 @@ DRYFT_API int dryft_rms_pair_mean(const void* a, int a_kind, int a_parts, int64_
   dim3 grid(n_rows), block(256);
   const size_t lds = (size_t)2 * width * sizeof(float);
   const bool fa = is_f32 || a_kind == 2, fb = is_f32 || b_kind == 2;
+  const uintptr_t all = (uintptr_t)a | (uintptr_t)b | (uintptr_t)a_bias | (uintptr_t)b_bias | (uintptr_t)wa | (uintptr_t)wb |
+                        (uintptr_t)out;
+  if (width % 8 == 0 && (all & 15) == 0 && (a_parts == 1 || a_stride % 8 == 0) && (b_parts == 1 || b_stride % 8 == 0)) {
+    const int runs = width / 8, per = (runs + STREAM_NORM_THREADS - 1) / STREAM_NORM_THREADS;  // at most two a thread
+    const dim3 threads((((runs + per - 1) / per) + WAVE - 1) / WAVE * WAVE);
+#define PMV(DA, DB, R)                                                                                                \
+  hipLaunchKernelGGL((rms_pair_mean_vec_kernel<DA, DB, R>), grid, threads, 0, stream, (const DA*)a, a_parts, a_stride, \
+                     a_bias, wa, (const DB*)b, b_parts, b_stride, b_bias, wb, out, width, eps)
+#define PMR(DA, DB)                 \
+  do {                              \
+    if (per <= 1) PMV(DA, DB, 1);   \
+    else PMV(DA, DB, 2);            \
+  } while (0)
+    if (fa && fb) PMR(float, float);
+    else if (fa) PMR(float, bf16_t);
+    else if (fb) PMR(bf16_t, float);
+    else PMR(bf16_t, bf16_t);
+#undef PMR
+#undef PMV
+    return DRYFT_LAUNCH_CHECK();
+  }
 #define PM(DA, DB)                                                                                                    \
   hipLaunchKernelGGL((rms_pair_mean_kernel<DA, DB>), grid, block, lds, stream, (const DA*)a, a_parts, a_stride, a_bias, \
                      wa, (const DB*)b, b_parts, b_stride, b_bias, wb, out, width, eps)
