@@ -17,7 +17,9 @@
 // are the same for every column: they wait in LDS, one run per lane of a column (runs a bank apart), read 16
 // bytes at a time. Operands come in batches of eight tokens: while the wave walks one batch, the next one's loads
 // are in flight; the unit lengths (a sum over D per token) are taken by four lanes a vector as the batch goes to LDS.
-#include "common.h"
+//
+// Most walks of 17 rows and more go sixteen rows at a time on the matrix cores instead (chunk_walk.h).
+#include "chunk_walk.h"
 
 #define DELTA_MAX_DIM 256
 #define DELTA_BATCH 8            // tokens whose operands are brought into LDS together
@@ -322,4 +324,18 @@ DRYFT_API int dryft_delta_steps(const void* qkv, int64_t qkv_stride, int q_col, 
 #undef DELTA_CASE
 #undef DELTA_LAUNCH
   return DRYFT_LAUNCH_CHECK();
+}
+
+// Whole sequences, sixteen tokens at a time on the matrix cores; -2 for shapes that the kernel does not take.
+DRYFT_API int dryft_delta_chunks(const void* qkv, int64_t qkv_stride, int q_col, int k_col, int v_col, const float* gates,
+                                 int64_t gate_stride, int a_col, int b_col, const float* dt_bias, const float* a_log,
+                                 const int* seq_slot, const int* cu_rows, const int* q_len, float* state, float* out,
+                                 int n_seqs, int H, int G, int D, int P, float q_scale, float unit_eps, int write_state,
+                                 int is_f32, hipStream_t stream) {
+  if (n_seqs <= 0) return 0;
+  if (H <= 0 || G <= 0 || H % G || D <= 0 || P <= 0) return -1;
+  if (!chunk_walk_takes(qkv, qkv_stride, q_col, k_col, D)) return -2;
+  return chunk_walk_run<true>(qkv, qkv_stride, q_col, k_col, v_col, gates, gate_stride, a_col, b_col, dt_bias, a_log, nullptr,
+                              seq_slot, cu_rows, q_len, state, out, n_seqs, H, G, D, P, q_scale, unit_eps, write_state, is_f32,
+                              stream);
 }

@@ -13,7 +13,9 @@
 // a column as still leave every lane eight rows and the chip a wave per SIMD. B and C of a token are the same for
 // every column: they wait in LDS, one run per lane of a column (runs a bank apart), read 16 bytes at a time.
 // Operands come in batches of eight tokens; the next batch's loads are in flight while the wave walks this one.
-#include "common.h"
+//
+// Most walks of 17 rows and more go sixteen rows at a time on the matrix cores instead (chunk_walk.h).
+#include "chunk_walk.h"
 
 #define SSM_MAX_STATE 256
 #define SSM_BATCH 8              // tokens whose operands are brought into LDS together
@@ -303,4 +305,16 @@ DRYFT_API int dryft_gate_part_norm(const float* y, const void* z, int64_t z_stri
     hipLaunchKernelGGL(gate_part_norm_kernel<bf16_t>, grid, block, 0, stream, y, (const bf16_t*)z, z_stride, z_col, w,
                        row_slot, (bf16_t*)out, inner, parts, eps);
   return DRYFT_LAUNCH_CHECK();
+}
+
+// Whole sequences, sixteen tokens at a time on the matrix cores; -2 for shapes that the kernel does not take.
+DRYFT_API int dryft_ssm_chunks(const void* xbc, int64_t xbc_stride, int x_col, int b_col, int c_col, const float* dt_raw,
+                               int64_t dt_stride, const float* dt_bias, const float* a_log, const float* d_skip,
+                               const int* seq_slot, const int* cu_rows, const int* q_len, float* state, float* y, int n_seqs,
+                               int H, int P, int N, int G, int write_state, int is_f32, hipStream_t stream) {
+  if (n_seqs <= 0) return 0;
+  if (H <= 0 || P <= 0 || N <= 0 || G <= 0 || H % G) return -1;
+  if (!chunk_walk_takes(xbc, xbc_stride, c_col, b_col, N)) return -2;
+  return chunk_walk_run<false>(xbc, xbc_stride, c_col, b_col, x_col, dt_raw, dt_stride, 0, 0, dt_bias, a_log, d_skip, seq_slot,
+                               cu_rows, q_len, state, y, n_seqs, H, G, N, P, 1.f, 0.f, write_state, is_f32, stream);
 }

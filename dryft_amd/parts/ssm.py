@@ -83,12 +83,12 @@ class StateSpaceMixer(Mixer):
         dt_raw = linear(h, self.w_dt, out_dtype=torch.float32)
         xbc = short_conv(proj, self.inner, self.conv_channels, self.conv_w, ctx, line.get("tail"), writes_cache,
                          out_bias=self.conv_b, silu=True, weight_t=self.conv_wt)
-        # a long prompt runs as segments side by side (the rows of sequences that sit out are then not visited)
+        # long walks go by chunks, or as segments side by side (the rows of sequences that sit out are then not visited)
         segments = ctx.segments() if writes_cache else None
         y = torch.empty((rows, self.inner), dtype=torch.float32, device=h.device)
         ops.ssm_scan(xbc, 0, self.inner, self.inner + GN, dt_raw, self.dt_bias, self.a_log, self.d_skip, ctx.seq_slot,
                      ctx.cu_rows, ctx.q_len, ctx.n_seqs, line["state"].state, y, self.n_heads, self.head_dim,
-                     self.n_state, self.groups, writes_cache, segments=segments)
+                     self.n_state, self.groups, writes_cache, segments=segments, longest=ctx.max_q_len)
         out = torch.empty((rows, self.inner), dtype=h.dtype, device=h.device)
         ops.gate_part_norm(y, proj, 0, self.out_norm, ctx.row_slot, out, self.norm_parts, self.norm_eps)
         return linear(out, self.w_o, allow_partials=True)

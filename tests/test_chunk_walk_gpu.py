@@ -1,0 +1,73 @@
+"""The delta rule and the state-space recurrence sixteen rows at a time, against 64-bit walks row by row: lengths around a
+chunk and the ring of chunks, states at the edges of the kernel's two sizes, columns that do not fill a wave, sequences that
+sit out, decays that forget at once and that hardly forget, and rows that the general walk takes instead."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+LENGTHS = (33, 0, 17, 1, 300, 16, 64, 49)       # the second sits out
+# float32 sums of up to 128 products and 16 tokens a chunk, a few 2^-24 each; a state that forgets nothing in 300 rows
+# carries the roundings of all 19 chunks: 32 x 2^-24 of the outputs' size, the largest of some 10^5 values.
+TOL = 64 * 2.0 ** -24
+
+
+def walk(kind, x, gates, dt_bias, a_log, skip, state, H, G, D, P, eps):
+    x, gates = x.double(), gates.double()
+    dt = torch.nn.functional.softplus(gates[:, :H] + dt_bias.double())
+    decay, beta = torch.exp(-a_log.double().exp() * dt), torch.sigmoid(gates[:, H:])
+    q, k = (t.reshape(-1, G, D).repeat_interleave(H // G, 1) for t in (x[:, :G * D], x[:, G * D:2 * G * D]))
+    v = x[:, 2 * G * D:].reshape(-1, H, P)
+    if kind == "delta":
+        unit = lambda t: t / (t.pow(2).sum(-1, keepdim=True) + eps).sqrt()
+        q, k = unit(q) * D ** -0.5, unit(k)
+    S, out = state.double().clone(), []
+    for t in range(x.shape[0]):
+        S = S * decay[t][:, None, None]
+        u = beta[t][:, None] * (v[t] - (S * k[t][:, :, None]).sum(1)) if kind == "delta" else dt[t][:, None] * v[t]
+        S = S + k[t][:, :, None] * u[:, None, :]
+        out.append((S * q[t][:, :, None]).sum(1) + (0 if kind == "delta" else skip.double()[:, None] * v[t]))
+    return torch.stack(out).flatten(1) if out else x.new_zeros(0, H * P), S
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kind,H,G,D,P,rate,pad", [("delta", 4, 2, 128, 128, None, 0), ("delta", 2, 1, 64, 40, -9.0, 8), ("delta", 3, 3, 8, 5, 6.0, 0),
+                                                   ("delta", 2, 2, 72, 16, None, 0), ("delta", 2, 1, 64, 32, None, 1), ("state", 4, 2, 128, 64, None, 0),
+                                                   ("state", 3, 1, 64, 72, -9.0, 8), ("state", 2, 1, 24, 8, 6.0, 0), ("state", 2, 1, 128, 33, None, 0)])
+def test_walk_by_chunks(dtype, kind, H, G, D, P, rate, pad):
+    from dryft_amd.csrc import ops
+    g = torch.Generator().manual_seed(D + P + H)
+    rows, n, eps = sum(LENGTHS), len(LENGTHS), 1e-6
+    width = 2 * G * D + H * P
+    x = torch.randn(rows, (width + 7) // 8 * 8 + pad, generator=g).to(dtype)
+    gates = torch.randn(rows, 2 * H, generator=g)
+    dt_bias, skip = torch.randn(H, generator=g), torch.randn(H, generator=g)
+    a_log = torch.randn(H, generator=g) if rate is None else torch.full((H,), rate)
+    state = torch.randn(n + 2, H, D, P, generator=g)
+    slots = [3, -1, 0, 5, 1, 9, 2, 7]
+    cu = torch.tensor([0] + torch.tensor(LENGTHS).cumsum(0).tolist(), dtype=torch.int32)
+    dev = lambda t: t.to(DEV)
+    got_state, out = dev(state.clone()), torch.full((rows, H * P), 7.0, device=DEV)
+    facts = (dev(torch.tensor(slots, dtype=torch.int32)), dev(cu), dev(torch.tensor(LENGTHS, dtype=torch.int32)), n, got_state, out)
+    seg_cu = torch.tensor([0] + [-(-q // 64) * (s >= 0) for q, s in zip(LENGTHS, slots)]).cumsum(0).to(torch.int32)
+    segments = (64, dev(seg_cu), int(seg_cu[-1])) if kind == "delta" else None
+    xd = dev(x)
+    by_chunks = ops._walks_by_chunks(xd, 0, G * D, D, P, H, n, max(LENGTHS), segments is not None,
+                                     ops._DELTA_WALK_US if kind == "delta" else ops._SSM_WALK_US)
+    assert by_chunks == (pad != 1)                                    # rows that do not begin at 16 bytes: the general walk
+    if kind == "delta":
+        ops.delta_steps(xd, 0, G * D, 2 * G * D, dev(gates), 0, H, dev(dt_bias), dev(a_log), *facts, H, G, D, P, D ** -0.5, eps, True,
+                        segments=segments, longest=max(LENGTHS))
+    else:
+        ops.ssm_scan(xd, 2 * G * D, G * D, 0, dev(gates), dev(dt_bias), dev(a_log), dev(skip), *facts, H, P, D, G, True,
+                     segments=segments, longest=max(LENGTHS))
+    out, got_state = out.double().cpu(), got_state.double().cpu()
+    for s, (slot, q) in enumerate(zip(slots, LENGTHS)):
+        r = slice(int(cu[s]), int(cu[s]) + q)
+        if slot < 0:
+            continue
+        want, S = walk(kind, x[r, :width], gates[r], dt_bias, a_log, skip, state[slot], H, G, D, P, eps)
+        assert float((out[r] - want).abs().max()) <= TOL * float(want.pow(2).mean().sqrt()) * 4, (slot, q)
+        assert float((got_state[slot] - S).abs().max()) <= TOL * float(S.pow(2).mean().sqrt()) * 4, (slot, q)
+    for slot in set(range(n + 2)) - set(slots):                       # nobody else's state is touched
+        assert torch.equal(got_state[slot], state[slot].double())
