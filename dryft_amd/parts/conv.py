@@ -28,8 +28,10 @@ def short_conv(u: torch.Tensor, col: int, channels: int, weight: torch.Tensor, c
     taps = weight.shape[1]
     tail = tail_line.state if taps > 1 else None
     out = torch.empty((u.shape[0], channels), dtype=u.dtype, device=u.device)
+    # a step of one row a sequence reads every earlier input from the tail, which then moves on in the same launch
+    one_row = writes_cache and taps > 1 and ctx.max_q_len == 1
     ops.causal_conv(u, col, channels, in_bias, weight, out_bias, silu, ctx.row_slot, ctx.row_seq, ctx.row_pos,
-                    ctx.seq_start, tail, out, weight_t=weight_t)
-    if writes_cache and taps > 1:
+                    ctx.seq_start, tail, out, weight_t=weight_t, moves_tail=one_row)
+    if writes_cache and taps > 1 and not one_row:
         ops.conv_tail(u, col, channels, in_bias, taps, ctx.seq_slot, ctx.cu_rows, ctx.q_len, ctx.n_seqs, tail)
     return out
