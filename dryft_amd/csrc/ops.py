@@ -110,10 +110,10 @@ _SIGNATURES = {
                "dryft_latent_rope_kv": [_P, _P, _P, _L, _I, _P, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I,
                                         _I, _I, _I, _I, _I, _P],
                "dryft_head_gate": [_P, _P, _L, _I, _P, _I, _I, _I, _I, _I, _I, _P]},
-    "moe": {"dryft_moe_route": [_P, _L, _P, _I, _I, _I, _I, _F, _P, _P, _I, _I, _I, _I, _P, _P],
+    "moe": {"dryft_moe_route": [_P, _L, _P, _I, _I, _I, _I, _F, _P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P],
             "dryft_moe_plan": [_P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _P],
             "dryft_moe_product": [_P, _L, _P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _F, _F, _F, _I, _I, _I, _P],
-            "dryft_moe_table_route": [_P, _P, _P, _P, _I, _I, _I, _I, _P],
+            "dryft_moe_table_route": [_P, _P, _P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P],
             "dryft_moe_combine": [_P, _P, _P, _P, _P, _L, _I, _P, _I, _I, _I, _I, _P]},
     "conv": {"dryft_conv_max_taps": [],
              "dryft_causal_conv": [_P, _L, _I, _P, _P, _P, _P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _P],
@@ -2105,14 +2105,15 @@ MOE_TILE = 64
 
 def moe_route(logits, correction, n_experts: int, groups: int, keep: int, scale: float, chosen, weights, *,
               softmax: bool = False, group_best: bool = False, renorm: bool = True, chosen_softmax: bool = False,
-              logit_bias=None) -> None:
+              logit_bias=None, plan: "MoePlan | None" = None) -> None:
     """Per row of float32 ``logits`` (their first ``n_experts`` columns): the ``top`` experts by ``sigmoid + correction``
     among the ``keep`` best of ``groups`` groups (a group's score: its two largest such scores), and their weights
     ``sigmoid / (sum of the chosen sigmoids + 1e-20) * scale``. ``chosen`` int32 and ``weights`` float32 ``[rows, top]``.
     ``softmax``: scores are the softmax over all experts instead; ``correction`` None: none; ``group_best``: a group
     scores as its best expert; ``renorm`` off: the weights are the scores times ``scale`` as they are.
     ``chosen_softmax``: the logits plus ``logit_bias`` (float32 ``[experts]``, optional) decide, and a chosen expert weighs
-    ``exp(its logit)`` over the sum of the chosen ones' exponentials, times ``scale``."""
+    ``exp(its logit)`` over the sum of the chosen ones' exponentials, times ``scale``. ``plan``: filled from ``chosen``, in
+    the same launch for few rows."""
     if chosen_softmax and (softmax or correction is not None) or (logit_bias is not None and not chosen_softmax):
         raise KernelError("moe_route: chosen_softmax goes alone, and a bias on the logits only with it")
     if logit_bias is not None:
@@ -2133,7 +2134,9 @@ def moe_route(logits, correction, n_experts: int, groups: int, keep: int, scale:
     _check(_fn("moe", "dryft_moe_route")(_ptr(logits), logits.stride(0), _ptr(correction), n_experts, groups, keep, top,
                                          float(scale), _ptr(chosen), _ptr(weights), rows,
                                          2 if chosen_softmax else int(bool(softmax)), int(bool(group_best)),
-                                         int(bool(renorm)), _ptr(logit_bias), _stream()), "moe_route")
+                                         int(bool(renorm)), _ptr(logit_bias), *_plan_pointers(plan, rows, top), _stream()),
+           "moe_route")
+    _plan_many(chosen, n_experts, plan)
 
 
 class MoePlan:
@@ -2150,6 +2153,30 @@ class MoePlan:
         self.place_of = torch.empty(n_pairs, **i32)
         self.tiles = torch.empty((3, self.max_tiles), **i32)        # expert | first place | places
         self.n_tiles = torch.empty(1, **i32)
+        self.done = False                                           # a router has filled it
+
+    def pointers(self) -> tuple:
+        return (_ptr(self.sorted_pair), _ptr(self.place_of), _ptr(self.tiles[0]), _ptr(self.tiles[1]), _ptr(self.tiles[2]),
+                _ptr(self.n_tiles))
+
+
+MOE_FEW_ROWS, MOE_FEW_PAIRS = 16, 64     # steps that route and plan in one launch: a wave a row, a lane a pair
+
+
+def _plan_pointers(plan: "MoePlan | None", rows: int, top: int) -> tuple:
+    """Where a router leaves the plan itself; zeros where ``_plan_many`` follows with a launch of its own, or no plan is asked for."""
+    if plan is None:
+        return (0,) * 6
+    if plan.n_pairs != rows * top:
+        raise KernelError(f"a plan of {plan.n_pairs} pairs for {rows} rows of {top}")
+    plan.done = 0 < rows <= MOE_FEW_ROWS and plan.n_pairs <= MOE_FEW_PAIRS
+    return plan.pointers() if plan.done else (0,) * 6
+
+
+def _plan_many(chosen, n_experts: int, plan: "MoePlan | None") -> None:
+    if plan is not None and not plan.done:
+        _check(_fn("moe", "dryft_moe_plan")(_ptr(chosen), plan.n_pairs, n_experts, *plan.pointers(), plan.max_tiles, _stream()),
+               "moe_plan")
 
 
 def moe_plan(chosen, n_experts: int) -> MoePlan:
@@ -2157,15 +2184,13 @@ def moe_plan(chosen, n_experts: int) -> MoePlan:
     if not chosen.is_contiguous():
         raise KernelError("moe_plan: chosen must be contiguous")
     plan = MoePlan(chosen.numel(), n_experts, chosen.device, most_places=chosen.shape[0] if chosen.dim() == 2 else None)
-    _check(_fn("moe", "dryft_moe_plan")(_ptr(chosen), plan.n_pairs, n_experts, _ptr(plan.sorted_pair), _ptr(plan.place_of),
-                                        _ptr(plan.tiles[0]), _ptr(plan.tiles[1]), _ptr(plan.tiles[2]), _ptr(plan.n_tiles),
-                                        plan.max_tiles, _stream()), "moe_plan")
+    _plan_many(chosen, n_experts, plan)
     return plan
 
 
-def moe_table_route(tokens, table, n_experts: int, chosen, weights) -> None:
+def moe_table_route(tokens, table, n_experts: int, chosen, weights, plan: "MoePlan | None" = None) -> None:
     """A router that is a table: row ``r`` goes to the experts ``table[tokens[r]]`` (int32 ``[vocab, top]``), each with
-    weight ``1 / top``. ``chosen`` int32 and ``weights`` float32 ``[rows, top]``."""
+    weight ``1 / top``. ``chosen`` int32 and ``weights`` float32 ``[rows, top]``. ``plan``: as in ``moe_route``."""
     _gpu(tokens, "tokens", torch.int32)
     _gpu(table, "table", torch.int32)
     _gpu(chosen, "chosen", torch.int32)
@@ -2175,7 +2200,9 @@ def moe_table_route(tokens, table, n_experts: int, chosen, weights) -> None:
             table.is_contiguous() and chosen.is_contiguous() and weights.shape == (rows, top) and weights.is_contiguous()):
         raise KernelError("moe_table_route: tokens [rows], table [vocab, top], chosen and weights [rows, top], contiguous")
     _check(_fn("moe", "dryft_moe_table_route")(_ptr(tokens), _ptr(table), _ptr(chosen), _ptr(weights), rows, top,
-                                               table.shape[0], n_experts, _stream()), "moe_table_route")
+                                               table.shape[0], n_experts, *_plan_pointers(plan, rows, top), _stream()),
+           "moe_table_route")
+    _plan_many(chosen, n_experts, plan)
 
 
 def moe_products(a, w, plan: MoePlan, out, top: int, glu: tuple | None = None, act: str | None = None) -> None:

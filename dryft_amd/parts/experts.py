@@ -129,16 +129,15 @@ class RoutedExperts(FeedForward):
         dev = h.device
         chosen = torch.empty((rows, top), dtype=torch.int32, device=dev)
         weights = torch.empty((rows, top), dtype=torch.float32, device=dev)
-        logits = None
+        logits, plan = None, ops.MoePlan(rows * top, E, dev, most_places=rows)
         if self.router == "table":
-            ops.moe_table_route(ctx.tokens, self.table, E, chosen, weights)
+            ops.moe_table_route(ctx.tokens, self.table, E, chosen, weights, plan=plan)
         else:
             logits = linear(h, self.w_router, out_dtype=torch.float32)
             ops.moe_route(logits, self.correction, E, self.groups[0], self.groups[1], self.route_scale, chosen, weights,
                           softmax=self.score == "softmax", group_best=self.group_score == "best",
                           renorm=self.renormalize, chosen_softmax=self.score == "chosen_softmax",
-                          logit_bias=self.router_bias)
-        plan = ops.moe_plan(chosen, E)
+                          logit_bias=self.router_bias, plan=plan)
         act = torch.empty((rows * top, self.inter), dtype=h.dtype, device=dev)
         if self.gated:
             ops.moe_products(h, self.w_gate_up, plan, act, top, glu=self.glu)
