@@ -1,6 +1,6 @@
 // Causal grouped-query attention over the paged cache, one workgroup per (row, query head), with
-// float arithmetic throughout. It serves the float32 path of the model and, in bfloat16, head
-// sizes the matrix-core kernels do not take. Formula (reference: engine/dryft_qwen3/model.py:172-177,
+// float arithmetic throughout. It serves the head sizes and options that the matrix-core
+// kernels do not take, in bfloat16 and in float32. Formula (reference: engine/dryft_qwen3/model.py:172-177,
 // 254-257; kernels/attn_decode.py:180-196):
 //
 //   s[j] = (q . k[j]) * scale  for  lo <= j <= pos,   p = softmax(s),   o = sum_j p[j] v[j]

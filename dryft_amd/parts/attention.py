@@ -338,7 +338,8 @@ class GQAAttention(Mixer):
             out = self._forward_general(h, ctx, line, writes_cache)
             return add_bias(out, self.o_bias, h.dtype) if self.has_bias else out
         rows = h.shape[0]
-        # bfloat16 on the matrix cores where they take the head size; float32 and the other head sizes on the plain kernel
+        # bfloat16 on the matrix cores where they take the head size; in float32 on the 32-bit matrix
+        # kernels where those do, everything else on the plain one
         matrix_cores = h.dtype == torch.bfloat16 and self.head_dim % MATRIX_CORE_HEAD_STEP == 0
         decoding = matrix_cores and ctx.max_q_len == 1
         fused_decoding = decoding and self.n_heads // self.n_kv <= 16
