@@ -102,3 +102,39 @@ def test_attn_f32(case, dead, way):
     close(out, torch.cat([want[b, :ql] for b, ql in enumerate(q_lens)]), torch.float32, what=f"attn_f32 {way} {case}")
     for b in dead:
         assert not out[int(cu[b]):int(cu[b + 1])].any()
+
+
+@pytest.mark.parametrize("D", [32, 128, 256])
+@pytest.mark.parametrize("way", ["rows", "tiles"])
+def test_attn_f32_scores_without_a_number(D, way):
+    """Scores of NaN, +inf and -inf: a row is a number exactly where the softmax over its keys is one (-inf beside other
+    scores weighs nothing, also where the first hundreds of keys are of that kind)."""
+    n_heads, n_kv = 4, 2
+    lengths = [70, 64, 300, 40, 50, 33]
+    torch.manual_seed(D)
+    B, L = len(lengths), max(lengths)
+    k, v, q = torch.randn(B, L, n_kv, D), torch.randn(B, L, n_kv, D), torch.randn(B, L, n_heads, D)
+    q[..., 0] = q[..., 0].abs() + 0.1
+    endless = lambda sign: torch.tensor([sign * float("inf")] + [0.0] * (D - 1))
+    k[0, 40] = float("nan")                       # rows from 40 on
+    k[1, 10, 0] = endless(1)                      # of one kv head, rows from 10 on
+    k[2, :290] = endless(-1)                      # whole waves without a finite score; from row 290 on there is one
+    k[3] = endless(-1)                            # nothing else
+    q[4, 7, 1] = float("nan")                     # one query
+    q_pos = torch.tensor([[t if t < n else -1 for t in range(L)] for n in lengths])
+    want = attention_ref(q, k, v, lengths, q_pos, D ** -0.5)
+    k_pages, v_pages, table, slots = build_pages(k, v, lengths, sum((n + 63) // 64 for n in lengths) + 1, B, seed=2, poison=1e4)
+    i32 = lambda values: torch.tensor(np.asarray(values), dtype=torch.int32, device=DEV)
+    packed = torch.cat([q[b, :n] for b, n in enumerate(lengths)]).contiguous().to(DEV)
+    out = torch.zeros_like(packed)
+    if way == "rows":
+        index = dict(row_slot=i32([s for s, n in zip(slots, lengths) for _ in range(n)]),
+                     row_pos=i32([t for n in lengths for t in range(n)]))
+    else:
+        tiles = [-(-n // 16) for n in lengths]
+        index = dict(tiles=(i32(slots), i32(np.concatenate([[0], np.cumsum(lengths)])), i32(np.concatenate([[0], np.cumsum(tiles)])),
+                            i32([0] * B), B, sum(tiles)))
+    ops().attn_f32(packed, k_pages.to(DEV), v_pages.to(DEV), table.to(DEV), out, n_heads, n_kv, D, D ** -0.5, 0, **index)
+    out, want = out.cpu(), torch.cat([want[b, :n] for b, n in enumerate(lengths)])
+    assert torch.equal(out.isnan(), want.isnan()) and 0 < int(want.isnan().sum()) < want.numel()
+    close(out.nan_to_num(0.0), want.nan_to_num(0.0), torch.float32, what=f"attn_f32 {way}, scores without a number")
