@@ -188,7 +188,8 @@ __global__ __launch_bounds__((OWNERS + 5) * WAVE) void chunk_walk_kernel(
         float ss = 0.f;
 #pragma unroll
         for (int i = 0; i < PER; ++i) ss += v[i] * v[i];
-        const uint32_t bits = __float_as_uint(rsqrtf(lanes_sum<8>(ss) + unit_eps));
+        // rows beyond the end are zeros and stay so whatever unit_eps is: their factor is 1, not 1 / sqrt(0)
+        const uint32_t bits = tok < left ? __float_as_uint(rsqrtf(lanes_sum<8>(ss) + unit_eps)) : __float_as_uint(1.f);
         const float power = __uint_as_float(bits & 0x7f800000u), rest = __uint_as_float((bits & 0x7fffffu) | 0x3f800000u);
 #pragma unroll
         for (int i = 0; i < PER; ++i) v[i] *= power;

@@ -71,3 +71,45 @@ def test_walk_by_chunks(dtype, kind, H, G, D, P, rate, pad):
         assert float((got_state[slot] - S).abs().max()) <= TOL * float(S.pow(2).mean().sqrt()) * 4, (slot, q)
     for slot in set(range(n + 2)) - set(slots):                       # nobody else's state is touched
         assert torch.equal(got_state[slot], state[slot].double())
+
+
+def drawn(kind, H, G, D, P, lengths, dtype, seed):
+    """Inputs of a step of these sequences, each in the slot of its own number."""
+    g = torch.Generator().manual_seed(seed)
+    rows = sum(lengths)
+    return dict(x=torch.randn(rows, (2 * G * D + H * P + 7) // 8 * 8, generator=g).to(dtype), gates=torch.randn(rows, 2 * H, generator=g),
+                dt_bias=torch.randn(H, generator=g), a_log=torch.randn(H, generator=g), skip=torch.randn(H, generator=g),
+                state=torch.randn(len(lengths), H, D, P, generator=g))
+
+
+def by_chunks(kind, d, H, G, D, P, lengths, eps):
+    """Outputs and states of the step, by chunks."""
+    from dryft_amd.csrc import ops
+    n, longest = len(lengths), max(lengths)
+    dev, ints = (lambda t: t.to(DEV)), (lambda v: torch.tensor(v, dtype=torch.int32, device=DEV))
+    x, state, out = dev(d["x"]), dev(d["state"].clone()), torch.full((d["x"].shape[0], H * P), 7.0, device=DEV)
+    assert ops._walks_by_chunks(x, 0, G * D, D, P, H, n, longest, False, None)
+    facts = (ints(list(range(n))), ints([0] + torch.tensor(lengths).cumsum(0).tolist()), ints(lengths), n, state, out)
+    if kind == "delta":
+        ops.delta_steps(x, 0, G * D, 2 * G * D, dev(d["gates"]), 0, H, dev(d["dt_bias"]), dev(d["a_log"]), *facts, H, G, D, P, D ** -0.5,
+                        eps, True, longest=longest)
+    else:
+        ops.ssm_scan(x, 2 * G * D, G * D, 0, dev(d["gates"]), dev(d["dt_bias"]), dev(d["a_log"]), dev(d["skip"]), *facts, H, P, D, G, True,
+                     longest=longest)
+    return out.double().cpu(), state.double().cpu()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,G,D,P", [(4, 2, 128, 128), (2, 1, 64, 40), (3, 3, 24, 5)])
+def test_unit_vectors_without_an_eps(dtype, H, G, D, P):
+    """Lengths that do not fill their last chunk: the zeros that do have no direction, and no say in anything."""
+    lengths = (17, 33, 16, 1)
+    d = drawn("delta", H, G, D, P, lengths, dtype, D + P)
+    out, state = by_chunks("delta", d, H, G, D, P, lengths, 0.0)
+    at = 0
+    for s, q in enumerate(lengths):
+        want, S = walk("delta", d["x"][at:at + q, :2 * G * D + H * P], d["gates"][at:at + q], d["dt_bias"], d["a_log"], d["skip"], d["state"][s],
+                       H, G, D, P, 0.0)
+        assert float((out[at:at + q] - want).abs().max()) <= TOL * float(want.pow(2).mean().sqrt()) * 4, q
+        assert float((state[s] - S).abs().max()) <= TOL * float(S.pow(2).mean().sqrt()) * 4, q
+        at += q
