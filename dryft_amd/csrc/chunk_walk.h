@@ -312,19 +312,48 @@ __global__ __launch_bounds__((OWNERS + 5) * WAVE) void chunk_walk_kernel(
       o[r] = grown_q[r] * ((qs[0][r] + qs[1][r]) + (qs[2][r] + qs[3][r])) + (DELTA ? 0.f : skip * v);
     }
     values(n + 1);                                           // beyond the end: the last row once more
+    const cw_f4 rhs = u;
     if (DELTA) {
       const vf4 w = *(const vf4*)(lds.inv[n & 1][c] + 4 * g);
-      const cw_f4 rhs = u;
       u = cw_f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int r = 0; r < 4; ++r) u = cw_mfma(w[r], rhs[r], u);
     }
+    const vf4 a = *(const vf4*)(lds.att[b][0][c] + 4 * g) + *(const vf4*)(lds.att[b][1][c] + 4 * g);
+    const cw_f4 carried = o;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o = cw_mfma(a[r], u[r], o);
+    // A factor 0 keeps a token from those before it only while its u is a number. Where one is none (a bad row of the input),
+    // its column is summed again over the tokens up to each one's own, as a walk row by row would.
+    const uint64_t strays = __ballot(!(fabsf(u[0]) < INFINITY && fabsf(u[1]) < INFINITY && fabsf(u[2]) < INFINITY && fabsf(u[3]) < INFINITY));
+    if (strays) {
+      const bool again = (((strays >> c) | (strays >> (c + 16)) | (strays >> (c + 32)) | (strays >> (c + 48))) & 1) != 0;
+      auto up_to_own = [&](const float (*one)[N + 4], const float (*two)[N + 4], cw_f4 x, cw_f4 sum) __attribute__((always_inline)) {
+#pragma unroll 1
+        for (int j4 = 0; j4 < N; j4 += 4)
+#pragma unroll
+          for (int jr = 0; jr < 4; ++jr) {
+            const float xj = __shfl(x[jr], c + 4 * j4, WAVE);        // token j4 + jr of this column
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const int i = 4 * g + r, j = j4 + jr;
+              if (j <= i) sum[r] += (one[i][j] + (two != nullptr ? two[i][j] : 0.f)) * xj;
+            }
+          }
+        return sum;
+      };
+      if (DELTA) {
+        const cw_f4 own = up_to_own(lds.inv[n & 1], nullptr, rhs, cw_f4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+        for (int r = 0; r < 4; ++r) u[r] = again ? own[r] : u[r];
+      }
+      const cw_f4 own = up_to_own(lds.att[b][0], lds.att[b][1], u, carried);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = again ? own[r] : o[r];
+    }
     cw_f4 eu;
 #pragma unroll
     for (int r = 0; r < 4; ++r) eu[r] = to_end[r] * u[r];
-    const vf4 a = *(const vf4*)(lds.att[b][0][c] + 4 * g) + *(const vf4*)(lds.att[b][1][c] + 4 * g);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) o = cw_mfma(a[r], u[r], o);
 #pragma unroll
     for (int t = 0; t < DT; ++t) {
       S[t] *= all;

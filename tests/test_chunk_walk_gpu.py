@@ -113,3 +113,32 @@ def test_unit_vectors_without_an_eps(dtype, H, G, D, P):
         assert float((out[at:at + q] - want).abs().max()) <= TOL * float(want.pow(2).mean().sqrt()) * 4, q
         assert float((state[s] - S).abs().max()) <= TOL * float(S.pow(2).mean().sqrt()) * 4, q
         at += q
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kind,H,G,D,P", [("delta", 2, 1, 128, 40), ("delta", 2, 1, 64, 32), ("state", 2, 1, 128, 40), ("state", 2, 2, 24, 32)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+def test_a_bad_row_leaves_the_rows_before_it_alone(kind, H, G, D, P, dtype, bad):
+    """One value of one row that is no number (in q, k, v or a gate): what becomes none is what becomes none row by row, in
+    outputs and states, and everything else is what it would be."""
+    parts = {"q": 1, "k": G * D + 2, "v": 2 * G * D + P - 1, "v2": 2 * G * D + P + 3}
+    lengths = (40, 33, 35, 20) + ((18, 50) if bad != bad else ())
+    d = drawn(kind, H, G, D, P, lengths, dtype, D + P)
+    cu = [0] + torch.tensor(lengths).cumsum(0).tolist()
+    for s, (part, row) in enumerate(zip(parts, (21, 16, 18, 9))):
+        d["x"][cu[s] + row, parts[part]] = bad
+    if bad != bad:
+        d["gates"][cu[4] + 5, 0] = bad
+        d["gates"][cu[5] + 31, H] = bad                       # of the delta rule alone
+    out, state = by_chunks(kind, d, H, G, D, P, lengths, 1e-6)
+    lost = 0
+    for s, q in enumerate(lengths):
+        r = slice(cu[s], cu[s] + q)
+        want, S = walk(kind, d["x"][r, :2 * G * D + H * P], d["gates"][r], d["dt_bias"], d["a_log"], d["skip"], d["state"][s], H, G, D, P, 1e-6)
+        for got, ref in ((out[r], want), (state[s], S)):
+            assert torch.equal(got.isfinite(), ref.isfinite()), (s, (got.isfinite() != ref.isfinite()).nonzero()[:4])
+            rest = ref[ref.isfinite()]
+            lost += ref.numel() - rest.numel()
+            if rest.numel():
+                assert float((got[ref.isfinite()] - rest).abs().max()) <= TOL * float(rest.pow(2).mean().sqrt()) * 4, s
+    assert lost
