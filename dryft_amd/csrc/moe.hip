@@ -44,6 +44,8 @@ __device__ __forceinline__ float wave_most(float v) {
 // choice scores are s itself; `group_best`: a group scores as its single largest choice score; without `renorm`
 // the weights are s * scale as they are. `softmax` = 2: no scores at all; the logits themselves (plus `logit_bias`, if
 // there is one) decide; a chosen expert weighs exp(its logit) over the sum of the chosen ones' exponentials, times scale.
+// A row none of whose choice scores is a number has no largest one: its experts are then the first `top`, with weights that
+// are no numbers, so that every entry of `chosen` names an expert and the row's output shows that it has none.
 template <int PER>
 __device__ __forceinline__ void route_row(const float* __restrict__ logits, int64_t stride,
                                           const float* __restrict__ correction, int n_experts, int groups, int keep, int top,
@@ -125,9 +127,9 @@ __device__ __forceinline__ void route_row(const float* __restrict__ logits, int6
     for (int i = 0; i < top; ++i) {
       const float best = wave_most(c[0]);
       const uint64_t at = __ballot(lane < n_experts && c[0] == best);
-      const int e = at ? __ffsll((unsigned long long)at) - 1 : 0x7fffffff;
-      float sv = at ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s[0]), e & (WAVE - 1))) : 0.f;
-      if (lane == e) c[0] = NEG;
+      const int e = at ? __ffsll((unsigned long long)at) - 1 : i;
+      float sv = at ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s[0]), e)) : __builtin_nanf("");
+      if (at && lane == e) c[0] = NEG;
       if (softmax == 2) {              // the first chosen logit is the largest
         if (i == 0) first = sv;
         sv = expf(sv - first);
@@ -156,6 +158,7 @@ __device__ __forceinline__ void route_row(const float* __restrict__ logits, int6
     for (int j = 0; j < PER; ++j)
       if (lane + WAVE * j == a.i) { sv = s[j]; c[j] = NEG; }
     sv = wave_sum(sv);
+    if (a.i == 0x7fffffff) { a.i = i; sv = __builtin_nanf(""); }
     if (softmax == 2) {                // the first chosen logit is the largest
       if (i == 0) first = sv;
       sv = expf(sv - first);
@@ -186,8 +189,8 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict_
 }
 
 // The plan of a step of at most MOE_TILE pairs, by one wave and in registers: lane p holds pair p's expert, and no expert
-// has more than one tile. Places run by expert, then by pair. A pair whose expert does not exist (every score of its row
-// was not a number) gets a place and no tile.
+// has more than one tile. Places run by expert, then by pair. A pair whose expert does not exist (no router here leaves
+// one) gets a place behind all others and no tile.
 #define MOE_FEW_PAIRS 64
 #define MOE_FEW_ROWS 16
 __device__ __forceinline__ void plan_few(int expert, int n_pairs, int n_experts, int* __restrict__ sorted_pair,
@@ -291,10 +294,12 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
                                                         int* __restrict__ tile_expert, int* __restrict__ tile_start,
                                                         int* __restrict__ tile_rows, int* __restrict__ n_tiles,
                                                         int max_tiles) {
-  __shared__ int counts[MOE_MAX_EXPERTS], cursor[MOE_MAX_EXPERTS];
-  for (int e = threadIdx.x; e < n_experts; e += blockDim.x) counts[e] = 0;
+  __shared__ int counts[MOE_MAX_EXPERTS + 1], cursor[MOE_MAX_EXPERTS + 1];
+  // experts that do not exist share the entry behind the last one: a place and no tile, as in plan_few
+  auto expert_of = [&](int p) { return (unsigned)chosen[p] < (unsigned)n_experts ? chosen[p] : n_experts; };
+  for (int e = threadIdx.x; e <= n_experts; e += blockDim.x) counts[e] = 0;
   __syncthreads();
-  for (int p = threadIdx.x; p < n_pairs; p += blockDim.x) atomicAdd(&counts[chosen[p]], 1);
+  for (int p = threadIdx.x; p < n_pairs; p += blockDim.x) atomicAdd(&counts[expert_of(p)], 1);
   __syncthreads();
   if (threadIdx.x == 0) {
     int at = 0, nt = 0;
@@ -308,11 +313,12 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
       }
       at += counts[e];
     }
+    cursor[n_experts] = at;
     *n_tiles = nt;
   }
   __syncthreads();
   for (int p = threadIdx.x; p < n_pairs; p += blockDim.x) {
-    const int place = atomicAdd(&cursor[chosen[p]], 1);
+    const int place = atomicAdd(&cursor[expert_of(p)], 1);
     sorted_pair[place] = p;
     place_of[p] = place;
   }

@@ -50,3 +50,49 @@ def test_route_and_plan(experts, top):
         ops.moe_table_route(tokens.to(DEV), table.to(DEV), experts, chosen, weights, plan=plan)
         assert torch.equal(chosen.cpu(), table[tokens.long()].clamp(0, experts - 1)) and bool((weights == 1 / top).all())
         check_plan(plan, chosen, experts)
+
+
+@pytest.mark.parametrize("kind", ["sigmoid", "softmax", "chosen_softmax"])
+@pytest.mark.parametrize("experts,top,rows", [(1, 1, 3), (16, 4, 4), (16, 4, 40), (64, 8, 9), (130, 5, 7), (130, 5, 40), (512, 4, 33)])
+def test_a_row_without_a_number(kind, experts, top, rows):
+    """A row whose scores are no numbers (with softmax one logit does that) names experts that exist, its output is no number,
+    and the other rows' experts, weights and outputs are what they are beside a row of numbers."""
+    from dryft_amd.csrc import ops
+    g = torch.Generator().manual_seed(experts + rows)
+    good = torch.randn(rows, experts, generator=g)
+    bad = good.clone()
+    if kind == "softmax":
+        bad[1, experts // 2] = float("nan")
+    else:
+        bad[1] = float("nan")
+    x, w = torch.randn(rows, 64, generator=g).to(torch.bfloat16).to(DEV), torch.randn(experts, 32, 64, generator=g).to(torch.bfloat16).to(DEV)
+
+    def run(logits):
+        chosen, weights = torch.empty((rows, top), dtype=torch.int32, device=DEV), torch.empty((rows, top), device=DEV)
+        plan = ops.MoePlan(rows * top, experts, chosen.device, most_places=rows)
+        ops.moe_route(logits.to(DEV), None, experts, 1, 1, 1.0, chosen, weights, softmax=kind == "softmax",
+                      chosen_softmax=kind == "chosen_softmax", plan=plan)
+        check_plan(plan, chosen, experts)
+        y, out = torch.empty((rows * top, 32), device=DEV), torch.empty((rows, 32), dtype=torch.bfloat16, device=DEV)
+        ops.moe_products(x, w, plan, y, top)
+        ops.moe_combine(y, plan, weights, None, None, 0, out)
+        return chosen.cpu(), weights.cpu(), out.cpu()
+
+    want, got = run(good), run(bad)
+    others = [r for r in range(rows) if r != 1]
+    assert all(torch.equal(a[others], b[others]) for a, b in zip(got, want))
+    chosen, weights, out = got
+    assert chosen[1].tolist() == list(range(top)) and weights[1].isnan().all() and out[1].isnan().all()
+
+
+@pytest.mark.parametrize("rows", [5, 40])
+def test_plan_of_pairs_without_an_expert(rows):
+    """Entries that name no expert get a place behind all others, at any number of pairs."""
+    from dryft_amd.csrc import ops
+    g = torch.Generator().manual_seed(rows)
+    chosen = torch.randint(0, 9, (rows, 3), generator=g, dtype=torch.int32)
+    chosen[1, 0], chosen[2], chosen[4, 1] = 9, -1, 0x7fffffff
+    plan = ops.moe_plan(chosen.to(DEV), 9)
+    check_plan(plan, chosen, 9)
+    places = plan.place_of.cpu().view(rows, 3)
+    assert sorted(places[(chosen < 0) | (chosen >= 9)].tolist()) == list(range(3 * rows - 5, 3 * rows))
