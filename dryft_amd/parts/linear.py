@@ -237,6 +237,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, *, out_dtype: torch.dtype | None = 
             product = ops.gemm_stream_f32 if streams_f32(m, n, k) else ops.gemm_rows_f32
             return product(x, w, torch.empty((m, n), dtype=torch.float32, device=x.device))
         out = torch.empty((m, n), dtype=torch.float32, device=x.device)
+        if m <= STREAM_ROWS and k % 4 == 0 and w.data_ptr() % 16 == 0:
+            return ops.gemm_stream_f32(x, w, out)         # rows of x at any address: that kernel reads them value by value
         if ops.rows_f32_ok(x, w):
             if ops.direct_f32_ok(x, w):
                 return ops.gemm_direct_f32(x, w, out)

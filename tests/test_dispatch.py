@@ -1,6 +1,7 @@
 """Which matrix-product kernel a shape goes to, decided on the host: checked here with tensors that have shapes but
 no storage."""
 
+import pytest
 import torch
 
 
@@ -52,6 +53,26 @@ def test_gate_up_kernel_by_rows_and_size():
     assert tall_swiglu_ok(fake(65, 2560), w) and tall_swiglu_ok(fake(256, 2560), w) and not tall_swiglu_ok(fake(257, 2560), w)
     assert not tall_swiglu_ok(fake(128, 5120), fake(2 * 17408, 5120))           # beyond 256 MiB: the vendor library
     assert not tall_swiglu_ok(fake(128, 2592), fake(512, 2592))                 # K no multiple of 64
+
+
+@pytest.mark.parametrize("rows,k,offset,stride,want", [(3, 64, 0, 64, "few"), (3, 64, 1, 64, "gemm_stream_f32"), (3, 64, 0, 67, "gemm_stream_f32"),
+                                                       (16, 36, 3, 39, "gemm_stream_f32"), (3, 66, 0, 66, "gemm_tiled"),
+                                                       (17, 64, 1, 64, "gemm_tiled"), (17, 64, 0, 64, "gemm_direct_f32"),
+                                                       (17, 36, 0, 36, "gemm_block_f32")])
+def test_float32_products_by_where_the_rows_lie(monkeypatch, rows, k, offset, stride, want):
+    """Up to 16 rows that do not start at 16-byte addresses go to the kernel that reads them value by value."""
+    from dryft_amd.csrc import ops
+    from dryft_amd.parts import linear as linear_module
+    called = []
+    for name in ("gemm_rows_f32", "gemm_stream_f32", "gemm_direct_f32", "gemm_block_f32", "gemm_tiled"):
+        monkeypatch.setattr(ops, name, lambda x, w, out, *a, name=name, **b: called.append(name) or out)
+    held = torch.empty(rows * stride + 8)
+    first = (-held.data_ptr() % 16) // 4 + offset
+    x = held[first:].as_strided((rows, k), (stride, 1))
+    w = torch.empty(40 * k + 4)
+    w = w[(-w.data_ptr() % 16) // 4:][:40 * k].view(40, k)
+    linear_module.linear(x, w)
+    assert called in ([want], ["gemm_rows_f32" if want == "few" else want])
 
 
 def test_every_entry_point_is_called_with_as_many_arguments_as_it_declares():
