@@ -320,12 +320,14 @@ static int launch_direct(const float* x, int64_t x_stride, const float* w, float
 }
 
 // Which block: 0 = 128 x 128, 1 = 64 x 64, 2 = 32 x 64 (rows of x by rows of W): the one whose busiest compute unit has the
-// fewest outputs to do, the larger one where two are within a twelfth (it reads the caches less).
+// fewest outputs to do, the larger one where two are within a twelfth (it reads the caches less). Blocks of few rows do not
+// take more rows than a grid has places for them.
 DRYFT_API int dryft_gemm_direct_f32_shape(int M, int N) {
   const int bm[3] = {128, 64, 32}, bn[3] = {128, 64, 64};
   int best = 0;
   double least = 1e30;
   for (int s = 0; s < 3; ++s) {
+    if (((int64_t)M + bm[s] - 1) / bm[s] > 65535) continue;
     const int64_t blocks = (int64_t)((M + bm[s] - 1) / bm[s]) * ((N + bn[s] - 1) / bn[s]);
     const double work = (double)((blocks + 255) / 256) * bm[s] * bn[s];
     if (work < least * (11.0 / 12.0)) {

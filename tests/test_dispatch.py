@@ -75,6 +75,14 @@ def test_float32_products_by_where_the_rows_lie(monkeypatch, rows, k, offset, st
     assert called in ([want], ["gemm_rows_f32" if want == "few" else want])
 
 
+@pytest.mark.parametrize("rows,outputs", [(2_097_120, 64), (2_097_121, 32), (4_194_241, 64), (5_000_000, 64), (8_388_480, 64)])
+def test_float32_blocks_of_many_rows_fit_a_grid(rows, outputs):
+    """The block that the library chooses has no more than 65,535 blocks of rows as long as one of the three has."""
+    from dryft_amd.csrc import ops
+    shape = ops._fn("gemm_f32", "dryft_gemm_direct_f32_shape")(rows, outputs)
+    assert -(-rows // (128, 64, 32)[shape]) <= 65535
+
+
 def test_every_entry_point_is_called_with_as_many_arguments_as_it_declares():
     """The table of ctypes signatures against the ``extern "C"`` declarations in the HIP sources: every entry point the
     Python side calls exists in its library's source and takes as many arguments as the table lists."""
