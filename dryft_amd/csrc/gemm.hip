@@ -1304,8 +1304,8 @@ DRYFT_API int dryft_gemm_tall_bf16(const void* x, int64_t x_stride, const void* 
 // Bound by the matrix cores' clock and what they wait: 1.0 to 1.2 PFLOP/s of 2.5 nominal. Alone, us, beside the vendor
 // library's product and the activation kernel: 2,048 rows, 2 x 9,728 of K 2,560 201 (227 + 23); 12,806 rows 999 (951 + 135);
 // 5,099 rows, 2 x 8,192 of 2,048 271 (244 + 47); 2,048 rows, 2 x 3,072 of 1,024 32 (30 + 8); 517 rows, 2 x 9,728 of 2,560 69
-// (54 + 8). In whole steps it is ahead at 2,048 rows (12 layers 6.75 -> 6.53 ms) and level at 12,806, so it serves products
-// below 2.5e11 operations (the rule: linear.py). Tried beside it: one workgroup a unit that walks several tiles and fetches
+// (54 + 8). A round of 256 tiles takes 1.5 us a step of K and some 9 us to fill, drain and store; it serves steps that fill their
+// rounds (the rule, with both sides in whole steps: linear.py). Tried beside it: one workgroup a unit that walks several tiles and fetches
 // the next one's first steps under the stores (10 % slower: the branches it needs break the order of instructions), tiles of
 // 256 x 128 with three steps in LDS (194 at 2,048 rows, but 1,165 at 12,806, and slower in the step), 256 x 192 (206), 128 x
 // 128 (219), other orders of tiles and places in LDS (the same).

@@ -191,18 +191,28 @@ def tall_swiglu_ok(x: torch.Tensor, w_gate_up: torch.Tensor) -> bool:
         within_direct_reach(x, w_gate_up) and w_gate_up.numel() * w_gate_up.element_size() <= _TALL_SWIGLU_BYTES
 
 
-@functools.lru_cache(maxsize=None)
+_MANY_TILE = (256, 128)         # rows and outputs of a workgroup of gemm_many_glu; one runs on a compute unit
+_MANY_FILLED = 0.89
+_MANY_DEPTHS = (1536, 3072)
+
+
 def _many_glu_pays(m: int, n: int, k: int) -> bool:
-    """Is the fused gate/up product of many rows (256 rows by 128 outputs a workgroup) expected to be ahead of the vendor
-    library's product and the activation kernel? Not from 2.5e11 operations on (there the library reaches 1.3 PFLOP/s, and a
-    step of 12,806 rows of Qwen3-4B takes the same time with either), nor where the tiles fill the last round of the compute
-    units badly. Times in us: 1.67 per step of 64 values of K and round of the compute units and 6 to fill and drain, from 2,048
-    and 5,099 rows of three shapes; the library at 0.94 PFLOP/s, the activation at 4.6 TB/s. (What both took: beside the
-    kernel.) The prompt of 2,048 tokens through 12 layers of Qwen3-4B: 6.75 -> 6.53 ms."""
-    flops = 4.0 * m * n * k
-    rounds = -(-(-(-m // 256) * -(-n // 128)) // _COMPUTE_UNITS)
-    library = flops / 0.94e9 + m * n * 6 / 4.6e6 + 3
-    return flops < 2.5e11 and 6 + 1.67 * (k // ops.MANY_STEP) * rounds < 0.97 * library
+    """Is the fused gate/up product of many rows ahead of the vendor library's product and the activation kernel, whether
+    ``library_tuning`` has chosen the library's kernels or not? Where its rounds of workgroups are nearly full. A full round
+    keeps up with the library's best (1.3 to 1.4 PFLOP/s) and saves the activation's pass, some 11 us a round; places of the
+    last round that stay empty, and rows of a tile that are not there, cost as much as filled ones, where the library goes to
+    smaller tiles. Time against the library's, as it comes / tuned, product and activation in a chain on rotating weights, 199
+    sizes: with 0.89 to 1 of the rounds filled 0.94 / 0.97 on average (0.68 to 1.03 / 0.84 to 1.05), from 0.85 on 0.96 / 0.99
+    (up to 1.03), from 0.74 on 1.01 / 1.01 (up to 1.10), from 0.6 on 1.08 / 1.06. Whole steps of 12 layers of Qwen3-4B (2 x 9,728 of 2,560): 2,560 rows 0.868 /
+    0.987, 5,099 0.932 / 0.992, 6,144 0.959 / 1.006, 8,192 0.953 / 0.995, 9,472 0.955 / 0.985, 12,806 0.992 / 0.996, 768 0.987 /
+    0.986, 1,536 0.999 / 0.991 of the time; left to the library:
+    1,188 rows 1.044 / 1.034, 1,368 1.010 / 1.021, 2,126 1.012 / 1.013, and 2,048 0.963 / 1.020 (0.79 filled).
+    The depths are those at which this holds. At K = 1,024 filling and draining a tile takes a quarter of its time (Qwen3-0.6B,
+    full rounds, whole steps: 0.995 to 1.006 / 1.008 to 1.024); at K = 4,096 the activation is a tenth of the product and the
+    library reaches 1.5 PFLOP/s (Qwen3-8B likewise: 0.958 to 1.002 / 1.012 to 1.023)."""
+    rows, outputs = _MANY_TILE
+    rounds = -(-(-(-m // rows) * -(-n // outputs)) // _COMPUTE_UNITS)
+    return _MANY_DEPTHS[0] <= k <= _MANY_DEPTHS[1] and m * n >= _MANY_FILLED * rounds * _COMPUTE_UNITS * rows * outputs
 
 
 def many_glu_ok(x: torch.Tensor, w_gate_up: torch.Tensor) -> bool:

@@ -83,6 +83,19 @@ def test_float32_blocks_of_many_rows_fit_a_grid(rows, outputs):
     assert -(-rows // (128, 64, 32)[shape]) <= 65535
 
 
+@pytest.mark.parametrize("rows,outputs,depth,ours", [
+    (1188, 9728, 2560, False), (1368, 9728, 2560, False), (2126, 9728, 2560, False), (2842, 9728, 2560, False),
+    (2048, 6144, 2048, False), (3072, 6144, 2048, False), (1557, 8192, 2048, False), (2150, 3072, 1024, False), (4360, 3072, 1024, False),
+    (1530, 12288, 4096, False), (6144, 12288, 4096, False), (12806, 12288, 4096, False),
+    (768, 9728, 2560, True), (2560, 9728, 2560, True), (4096, 9728, 2560, True), (5099, 9728, 2560, True), (8192, 9728, 2560, True),
+    (1280, 6144, 2048, True), (1024, 8192, 2048, True), (5099, 8192, 2048, True), (8447, 8960, 1536, True)])
+def test_gate_up_of_many_rows_goes_where_it_was_measured_ahead(rows, outputs, depth, ours):
+    """Rounds of tiles that are nearly full stay here, at sizes beyond 2.5e11 operations too; sizes that were 1 to 10 % slower
+    than the vendor library, as it comes or tuned, go there."""
+    from dryft_amd.parts.linear import many_glu_ok
+    assert many_glu_ok(fake(rows, depth), fake(2 * outputs, depth)) == ours
+
+
 def test_every_entry_point_is_called_with_as_many_arguments_as_it_declares():
     """The table of ctypes signatures against the ``extern "C"`` declarations in the HIP sources: every entry point the
     Python side calls exists in its library's source and takes as many arguments as the table lists."""
