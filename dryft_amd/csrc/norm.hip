@@ -323,7 +323,8 @@ __global__ __launch_bounds__(STREAM_NORM_THREADS) void stream_norm_vec_kernel(co
                                                               const void* __restrict__ w, int w_f32,
                                                               const float* __restrict__ bias, float* __restrict__ x_out, T* __restrict__ y, int width,
                                                               float eps, int form, int groups) {
-  __shared__ float scratch[16], sums[STREAM_NORM_MAX_GROUPS], squares[RUNS * STREAM_NORM_THREADS];
+  // of a run of 8 values: the squares that belong to the part it begins in, and those of the next part, if it reaches there
+  __shared__ float scratch[16], sums[STREAM_NORM_MAX_GROUPS], squares[RUNS * STREAM_NORM_THREADS], beyond[RUNS * STREAM_NORM_THREADS];
   constexpr bool EARLY = RUNS == 1;                        // longer rows have no registers for all weights at once
   const int64_t base = (int64_t)blockIdx.x * width;
   const bool normed = y != nullptr && !(form & 4);
@@ -367,6 +368,7 @@ __global__ __launch_bounds__(STREAM_NORM_THREADS) void stream_norm_vec_kernel(co
     }
   }
   float ss = 0.f, sv = 0.f;
+  const int len = width / groups;
 #pragma unroll
   for (int r = 0; r < RUNS; ++r) {
     const int i = (r * blockDim.x + threadIdx.x) * 8;
@@ -389,18 +391,28 @@ __global__ __launch_bounds__(STREAM_NORM_THREADS) void stream_norm_vec_kernel(co
 #pragma unroll
     for (int j = 0; j < 8; ++j) { own += v[r][j] * v[r][j]; sv += v[r][j]; }
     ss += own;
-    if (groups > 1) squares[r * blockDim.x + threadIdx.x] = own;
+    if (groups > 1) {
+      float next = 0.f;
+      if (len % 8 != 0) {
+        const int left = len - i % len;                    // values up to the end of the part
+        own = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) (j < left ? own : next) += v[r][j] * v[r][j];
+      }
+      squares[r * blockDim.x + threadIdx.x] = own;
+      beyond[r * blockDim.x + threadIdx.x] = next;
+    }
   }
   if (y == nullptr) return;
   float mean = 0.f, inv = 1.f;
-  const int len = width / groups;
   if (normed && groups > 1) {
-    // a part's sum of squares from those of its runs, where runs lie in one part; the launcher sends other widths elsewhere
+    // a part's sum of squares from those of the runs that begin in it and the one that reaches into it (parts of 8 or more)
     __syncthreads();
-    const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, waves = blockDim.x / WAVE, runs = len / 8;
+    const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, waves = blockDim.x / WAVE;
     for (int p = wave; p < groups; p += waves) {
-      float own = 0.f;
-      for (int k = lane; k < runs; k += WAVE) own += squares[p * runs + k];
+      const int first = (p * len + 7) / 8, end = ((p + 1) * len + 7) / 8;
+      float own = lane == 0 && p * len % 8 != 0 ? beyond[first - 1] : 0.f;
+      for (int k = first + lane; k < end; k += WAVE) own += squares[k];
       own = wave_sum(own);
       if (lane == 0) sums[p] = rsqrtf(own / (float)len + eps);
     }
@@ -428,8 +440,10 @@ __global__ __launch_bounds__(STREAM_NORM_THREADS) void stream_norm_vec_kernel(co
         if (bias != nullptr) load8_as_float(bias + i, bv[r]);
       }
       if (groups > 1) inv = sums[i / len];
+      const int left = groups > 1 ? len - i % len : 8;
+      const float inv_next = left < 8 ? sums[i / len + 1] : inv;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[r][j] = (v[r][j] - mean) * inv * wv[r][j] + bv[r][j];
+      for (int j = 0; j < 8; ++j) v[r][j] = (v[r][j] - mean) * (j < left ? inv : inv_next) * wv[r][j] + bv[r][j];
     }
     store8_from_float(y + base + i, v[r]);
   }
@@ -469,7 +483,7 @@ DRYFT_API int dryft_stream_norm(const void* x_in, int x_kind, const void* delta,
   } while (0)
   const bool aligned = (((uintptr_t)x_in | (uintptr_t)delta | (uintptr_t)wb | (uintptr_t)extra | (uintptr_t)vec |
                          (uintptr_t)w | (uintptr_t)bias | (uintptr_t)x_out | (uintptr_t)y) & 15) == 0 && partial_stride % 4 == 0;
-  if (width % 8 == 0 && aligned && (groups == 1 || (width / groups) % 8 == 0)) {
+  if (width % 8 == 0 && aligned && (groups == 1 || width / groups >= 8)) {
     if (is_f32) SNV(float, float);
     else if (delta_kind == 2) SNV(bf16_t, float);
     else SNV(bf16_t, bf16_t);

@@ -51,6 +51,22 @@ def test_stream_norm_runs(dtype, width, parts, groups):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("width,groups", [(2040, 8), (72, 8), (3000, 24), (40, 10), (504, 56), (4104, 36), (8200, 8), (12296, 8),
+                                          (16376, 8)])
+def test_parts_that_end_within_a_run(dtype, width, groups):
+    """Parts whose length is no multiple of 8: runs of eight values that reach into the next part, once and twice in a row."""
+    from dryft_amd.csrc import ops
+    g = torch.Generator().manual_seed(width)
+    x, w = torch.randn(3, width, generator=g) * torch.linspace(0.1, 3, width), torch.randn(width, generator=g)
+    d = torch.randn(2, 3, width, generator=g)
+    x_out, y = torch.empty(3, width, device=DEV), torch.empty(3, width, dtype=dtype, device=DEV)
+    ops.stream_norm(x.to(DEV), (d.to(DEV), 2), None, None, None, w.to(DEV), EPS, x_out, y, dtype, groups=groups)
+    want = x.double() + d.double().sum(0)
+    close(x_out, want, 2e-6)
+    close(y, normed(want, w.double(), False, groups), TOL[dtype])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("width,parts", [(8, 1), (520, 9), (4096, 8), (4104, 3), (8192, 12)])
 def test_pair_mean_runs(dtype, width, parts):
     from dryft_amd.csrc import ops
