@@ -59,6 +59,29 @@ _QKV_PARTIAL_ROWS = 256         # decoding steps of up to so many rows take the 
 _PROMPT_PARTIAL_ROWS = 256      # and so do prompt steps of at most so many rows
 
 
+_UNITS = 256                    # compute units: steps of at most so many (row, head) pairs have one for each
+
+
+def float32_form(rows: int, n_heads: int, n_kv: int, head_dim: int, longest: int, keys: int) -> str:
+    """Which kernel a float32 step of ``rows`` rows, at most ``longest`` of one sequence, over at most ``keys`` keys takes:
+    ``plain`` (``attn_rows``), or the matrix cores' by ``rows`` or by ``tiles`` of 16 rows of a sequence.
+
+    Tiles read a key once for their rows, in as many workgroups fewer: they pay where (row, head) pairs outnumber the compute
+    units, and cost a sixteenth of the chip where they do not. Microseconds between launches that stream 32 MB, plain / rows /
+    tiles, 16 heads on 8 of 128: 16 rows at 200 keys 12.3 / 12.3 / 16.2, at 1,024 44 / 40 / 49, at 4,096 163 / 131 / 177; 33 rows
+    at 200 keys 21 / 22 / 16, at 4,096 369 / 247 / 177. One row, plain / rows, 20 keys 8.1 / 6.9, 280 20.5 / 15.8, 1,024 51 / 39;
+    without the launches between, 4,096 164 / 126, 16,384 642 / 478.
+    The plain kernel is ahead in short contexts where a row's work on the matrix cores is long (heads of more than 128: no
+    registers to ask for the values with the keys) or its columns fill two workgroups (groups of more than 16): 8 heads on 1 of
+    256, one row, 20 / 150 / 280 / 512 keys 11.2 / 17.7 / 29.6 / 39.6 against 11.8 / 21.3 / 28.6 / 40.1; 16 on 4 of 192 at 150 /
+    280 15.4 / 25.3 against 17.3 / 23.2; 32 on 1 of 128 at 20 / 150 / 512 / 768 7.8 / 11.7 / 24.7 / 35.4 against 8.9 / 14.2 /
+    26.5 / 33.3. With two heads a group it is not (16 on 8 of 256, 20 / 150 keys: 12.1 / 19.3 against 10.6 / 19.9)."""
+    group, few = n_heads // n_kv, rows * n_heads <= _UNITS
+    if few and (group > 16 or head_dim > 128 and group >= 4) and keys <= (512 if group > 16 else 256):
+        return "plain"
+    return "rows" if longest == 1 or few else "tiles"
+
+
 def add_bias(delta, bias: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     """``delta + bias`` per row in ``dtype``; ``delta`` is a tensor or ``Partials`` (added up on the way in)."""
     data = delta.data if isinstance(delta, Partials) else delta
@@ -410,6 +433,8 @@ class GQAAttention(Mixer):
         ops.qk_norm_rope_kv(qkv, self.q_norm, self.k_norm, self.qk_norm_eps or 0.0, cos, sin, self.rotary_dim,
                             ctx.row_slot, ctx.row_pos, q, line.k, line.v, line.page_table, writes_cache,
                             self.n_heads, self.n_kv, self.head_dim)
+        form = float32_form(rows, self.n_heads, self.n_kv, self.head_dim, ctx.max_q_len,
+                            min(window or ctx.max_kv_len, ctx.max_kv_len)) if h.dtype == torch.float32 else None
         if decoding:
             ops.attn_split_bf16(q, line.k, line.v, line.page_table, ctx.seq_slot, ctx.cu_rows, ctx.kv_len,
                                 ctx.n_seqs, part_o, part_ml, splits, out, self.n_heads, self.n_kv, self.head_dim,
@@ -419,8 +444,8 @@ class GQAAttention(Mixer):
             ops.attn_causal_bf16(q, line.k, line.v, line.page_table, ctx.seq_slot, ctx.cu_rows, tile_cu,
                                  ctx.seq_start, ctx.n_seqs, max_tiles, out, self.n_heads, self.n_kv,
                                  self.head_dim, self.scale, window)
-        elif ops.attn_f32_takes(q, line.k, line.v, self.head_dim):
-            if ctx.max_q_len == 1:
+        elif ops.attn_f32_takes(q, line.k, line.v, self.head_dim) and form != "plain":
+            if form == "rows":
                 ops.attn_f32(q, line.k, line.v, line.page_table, out, self.n_heads, self.n_kv, self.head_dim, self.scale,
                              window, row_slot=ctx.row_slot, row_pos=ctx.row_pos)
             else:

@@ -96,6 +96,18 @@ def test_gate_up_of_many_rows_goes_where_it_was_measured_ahead(rows, outputs, de
     assert many_glu_ok(fake(rows, depth), fake(2 * outputs, depth)) == ours
 
 
+@pytest.mark.parametrize("rows,heads,kv,size,longest,keys,form", [
+    (1, 16, 8, 128, 1, 20, "rows"), (4, 16, 8, 128, 1, 4096, "rows"), (64, 32, 8, 128, 1, 280, "rows"),       # decoding
+    (16, 16, 8, 128, 16, 200, "rows"), (5, 32, 8, 128, 5, 4096, "rows"), (17, 16, 8, 128, 17, 17, "tiles"),   # steps of few rows
+    (33, 16, 8, 128, 33, 4096, "tiles"), (525, 16, 8, 128, 253, 253, "tiles"), (20, 32, 8, 128, 5, 64, "tiles"),
+    (1, 32, 1, 128, 1, 150, "plain"), (8, 32, 1, 128, 1, 512, "plain"), (1, 32, 1, 128, 1, 1024, "rows"), (16, 32, 1, 128, 1, 64, "rows"),
+    (1, 8, 1, 256, 1, 150, "plain"), (17, 8, 1, 256, 17, 17, "plain"), (1, 8, 1, 256, 1, 512, "rows"), (40, 8, 1, 256, 40, 40, "tiles"),
+    (4, 16, 4, 192, 1, 150, "plain"), (4, 16, 8, 256, 1, 150, "rows"), (5, 16, 8, 256, 5, 200, "rows")])
+def test_float32_attention_goes_where_it_was_measured_ahead(rows, heads, kv, size, longest, keys, form):
+    from dryft_amd.parts.attention import float32_form
+    assert float32_form(rows, heads, kv, size, longest, keys) == form
+
+
 def test_every_entry_point_is_called_with_as_many_arguments_as_it_declares():
     """The table of ctypes signatures against the ``extern "C"`` declarations in the HIP sources: every entry point the
     Python side calls exists in its library's source and takes as many arguments as the table lists."""
