@@ -13,9 +13,11 @@
 // positions of a half page in the order that gives a lane its eight of both tiles of 16 keys as 32 contiguous bytes
 // (value_column). So scores never leave registers, and every line of a page is read once by one wave for all columns, where
 // the kernel of one workgroup a (row, head) (attn_rows.hip) read every key with 16 bytes a line and request, once per head
-// of the group. Qwen3-0.6B, 4 sequences, us in the step: decoding at
-// 10 to 280 keys 14.9 against that kernel's 18.6 (what is left are four trips to memory one after the other and 13 of 16
-// columns unused), 525 prompt rows 29.5 against 123.
+// of the group. Between launches that stream other memory, us, against that kernel: Qwen3-0.6B's heads, one sequence, one row at
+// 20 / 280 / 1,024 keys 6.9 / 15.8 / 39 (8.1 / 20.5 / 51), four sequences of 150 prompt rows 35 (115); in a traced serving pass
+// decoding at 10 to 280 keys 14.6, 525 prompt rows 36.8. What is left in decoding are four trips to memory one after the
+// other, 14 of 16 columns unused (a group of two), and keys that no second workgroup shares: 4,096 keys take 126 us. Which steps
+// take which form, and where the other kernel stays ahead: `float32_form` in parts/attention.py.
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;

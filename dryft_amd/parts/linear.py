@@ -5,8 +5,8 @@ engine/dryft_qwen3/model.py:153, 179-180, 237, 258-261). Here:
 
 * float32: this library's own kernels, so the 32-bit path has no reduced-precision matrix
   mode anywhere: the matrix cores' full-precision instruction (``v_mfma_f32_16x16x4_f32``),
-  with K split over a workgroup's waves (or plain multiply-adds, ``streams_f32``) for at most 16 rows, operands straight into LDS in
-  blocks chosen by the number of workgroups for more (``K`` a multiple of 32; else blocks of
+  with K split over a workgroup's waves (or plain multiply-adds, ``streams_f32``) for at most 16 rows, operands straight
+  into LDS in blocks chosen by the number of workgroups for more (``K`` a multiple of 32; else blocks of
   128 x 128 through registers), and a plain tiled kernel for sizes those do not take;
 * bfloat16, at most 16 rows (decoding at small batch): this library's weight-streaming
   matrix-core kernel, which stages whole cache lines through LDS and can leave its result
@@ -23,7 +23,7 @@ engine/dryft_qwen3/model.py:153, 179-180, 237, 258-261). Here:
 * bfloat16, 65 to 256 rows (short prompts, decoding at large batch) where the consumer adds partial sums and K is a
   multiple of 64: this library's kernel whose waves each own rows of x, operands straight into LDS (``tall_plan``);
   the fused gate/up product of as many rows goes to its other form (``tall_swiglu_ok``), of more rows to this library's
-  kernel of 256 rows a workgroup where that fills the chip (``many_glu_ok``);
+  kernel of 256 rows a workgroup where its rounds of workgroups are nearly full (``many_glu_ok``);
 * bfloat16, more than 16 rows, float32 results of at most 64 outputs (gates, routers, low-rank projections): this
   library's kernel that reads the rows once and splits K over the waves of a workgroup;
 * bfloat16, otherwise (prompts, decoding at large batch): the vendor library through
@@ -37,7 +37,6 @@ from __future__ import annotations
 
 import contextlib
 import functools
-import math
 import os
 import tempfile
 
@@ -203,10 +202,10 @@ def _many_glu_pays(m: int, n: int, k: int) -> bool:
     last round that stay empty, and rows of a tile that are not there, cost as much as filled ones, where the library goes to
     smaller tiles. Time against the library's, as it comes / tuned, product and activation in a chain on rotating weights, 199
     sizes: with 0.89 to 1 of the rounds filled 0.94 / 0.97 on average (0.68 to 1.03 / 0.84 to 1.05), from 0.85 on 0.96 / 0.99
-    (up to 1.03), from 0.74 on 1.01 / 1.01 (up to 1.10), from 0.6 on 1.08 / 1.06. Whole steps of 12 layers of Qwen3-4B (2 x 9,728 of 2,560): 2,560 rows 0.868 /
-    0.987, 5,099 0.932 / 0.992, 6,144 0.959 / 1.006, 8,192 0.953 / 0.995, 9,472 0.955 / 0.985, 12,806 0.992 / 0.996, 768 0.987 /
-    0.986, 1,536 0.999 / 0.991 of the time; left to the library:
-    1,188 rows 1.044 / 1.034, 1,368 1.010 / 1.021, 2,126 1.012 / 1.013, and 2,048 0.963 / 1.020 (0.79 filled).
+    (up to 1.03), from 0.74 on 1.01 / 1.01 (up to 1.10), from 0.6 on 1.08 / 1.06. Whole steps of 12 layers of Qwen3-4B (2 x
+    9,728 of 2,560): 2,560 rows 0.868 / 0.987, 5,099 0.932 / 0.992, 6,144 0.959 / 1.006, 8,192 0.953 / 0.995, 9,472 0.955 /
+    0.985, 12,806 0.992 / 0.996, 768 0.987 / 0.986, 1,536 0.999 / 0.991 of the time; left to the library: 1,188 rows 1.044 /
+    1.034, 1,368 1.010 / 1.021, 2,126 1.012 / 1.013, and 2,048 0.963 / 1.020 (0.79 filled).
     The depths are those at which this holds. At K = 1,024 filling and draining a tile takes a quarter of its time (Qwen3-0.6B,
     full rounds, whole steps: 0.995 to 1.006 / 1.008 to 1.024); at K = 4,096 the activation is a tenth of the product and the
     library reaches 1.5 PFLOP/s (Qwen3-8B likewise: 0.958 to 1.002 / 1.012 to 1.023)."""
