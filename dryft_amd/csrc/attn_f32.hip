@@ -95,7 +95,6 @@ __global__ __launch_bounds__(WAVES * WAVE) void attn_f32_kernel(AttnF32 a) {
 #pragma unroll
   for (int t = 0; t < DT; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;                            // l: over the keys of this lane alone
-  bool saw = false;                                        // has this lane's column seen a key, whatever its score
   constexpr bool V_EARLY = DT <= 8;                        // wider heads have no registers for the values that soon
   int u = lo_all / 32 + wave;
   int page = 32 * u <= last_pos ? table[u / 2] : -1;
@@ -103,7 +102,6 @@ __global__ __launch_bounds__(WAVES * WAVE) void attn_f32_kernel(AttnF32 a) {
     const int here = page;
     page = 32 * (u + WAVES) <= last_pos ? table[(u + WAVES) / 2] : -1;
     if (here < 0) continue;
-    saw |= 32 * u <= pos && 32 * u + 31 >= lo_col;
     const int64_t base = ((int64_t)here * a.n_kv + kvh) * PAGE_TOKENS * D;
     const float* kp = a.k_pages + base + (int64_t)(32 * (u & 1) + c) * D + 4 * g;
     const float* vp = a.v_pages + base + (int64_t)c * PAGE_TOKENS + 32 * (u & 1) + 8 * g;
@@ -177,7 +175,6 @@ __global__ __launch_bounds__(WAVES * WAVE) void attn_f32_kernel(AttnF32 a) {
   }
   l += __shfl_xor(l, 16, WAVE);
   l += __shfl_xor(l, 32, WAVE);
-  if (saw && l == 0.f) l = -1.f;                           // keys, but every score -inf: not the 0 of a wave without keys
   // o[t][i] is feature 16 t + 4g + i of column c
 #pragma unroll
   for (int t = 0; t < DT; ++t)
@@ -196,17 +193,15 @@ __global__ __launch_bounds__(WAVES * WAVE) void attn_f32_kernel(AttnF32 a) {
 #pragma unroll
     for (int v = 0; v < WAVES; ++v) top = fmaxf(top, merge_m[v * 16 + col]);
     float sum = 0.f, total = 0.f;
-    bool any = false;
 #pragma unroll
     for (int v = 0; v < WAVES; ++v) {
-      const float mv = merge_m[v * 16 + col], lv = merge_l[v * 16 + col];
+      const float mv = merge_m[v * 16 + col];
       const float wgt = mv == -INFINITY ? 0.f : expf(mv - top);
-      any |= lv != 0.f;
-      total += wgt * lv;
+      total += wgt * merge_l[v * 16 + col];
       sum += wgt * merge_o[(v * 16 + col) * OS + d];
     }
-    // a score that is no number or +inf, or nothing but -inf: no number, as the softmax has none; no key at all: 0
-    a.out[out_at + col * out_step + d] = any ? sum / total : 0.f;
+    // whatever the total is: a score of NaN or +inf, or none but -inf (0 / 0), leaves no number, as in the softmax
+    a.out[out_at + col * out_step + d] = sum / total;
   }
 }
 
