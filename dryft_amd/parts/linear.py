@@ -207,10 +207,11 @@ def _many_glu_pays(m: int, n: int, k: int) -> bool:
     9,728 of 2,560): 2,560 rows 0.868 / 0.987, 5,099 0.932 / 0.992, 6,144 0.959 / 1.006, 8,192 0.953 / 0.995, 9,472 0.955 /
     0.985, 12,806 0.992 / 0.996, 768 0.987 / 0.986, 1,536 0.999 / 0.991 of the time; left to the library: 1,188 rows 1.044 /
     1.034, 1,368 1.010 / 1.021, 2,126 1.012 / 1.013, and 2,048 0.963 / 1.020 (0.79 filled).
-    Beyond 1.5e12 operations neither is ahead throughout (13,824 rows 0.999 / 0.995; 16,384 1.009 / 1.006, 20,480 0.978 / 0.983,
-    32,000 1.019 / 1.016): the library. The depths are those at which this holds. At K = 1,024 filling and draining a tile takes a quarter of its time (Qwen3-0.6B,
-    full rounds, whole steps: 0.995 to 1.006 / 1.008 to 1.024); at K = 4,096 the activation is a tenth of the product and the
-    library reaches 1.5 PFLOP/s (Qwen3-8B likewise: 0.958 to 1.002 / 1.012 to 1.023)."""
+    At 13,824 rows it is still level (0.999 / 0.995); beyond 1.5e12 operations neither is ahead throughout (16,384 rows 1.009 /
+    1.006, 20,480 0.978 / 0.983, 32,000 1.019 / 1.016), and the library takes them.
+    The depths are those at which this holds. At K = 1,024 filling and draining a tile takes a quarter of its time
+    (Qwen3-0.6B, full rounds, whole steps: 0.995 to 1.006 / 1.008 to 1.024); at K = 4,096 the activation is a tenth of the
+    product and the library reaches 1.5 PFLOP/s (Qwen3-8B likewise: 0.958 to 1.002 / 1.012 to 1.023)."""
     rows, outputs = _MANY_TILE
     rounds = -(-(-(-m // rows) * -(-n // outputs)) // _COMPUTE_UNITS)
     return _MANY_DEPTHS[0] <= k <= _MANY_DEPTHS[1] and 4.0 * m * n * k <= _MANY_FLOPS and \
