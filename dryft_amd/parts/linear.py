@@ -193,7 +193,7 @@ def tall_swiglu_ok(x: torch.Tensor, w_gate_up: torch.Tensor) -> bool:
 _MANY_TILE = (256, 128)         # rows and outputs of a workgroup of gemm_many_glu; one runs on a compute unit
 _MANY_FILLED = 0.89
 _MANY_DEPTHS = (1536, 3072)
-_MANY_FLOPS = 1.5e12
+_MANY_FLOPS = 1.1e12
 
 
 def _many_glu_pays(m: int, n: int, k: int) -> bool:
@@ -205,10 +205,10 @@ def _many_glu_pays(m: int, n: int, k: int) -> bool:
     sizes: with 0.89 to 1 of the rounds filled 0.94 / 0.97 on average (0.68 to 1.03 / 0.84 to 1.05), from 0.85 on 0.96 / 0.99
     (up to 1.03), from 0.74 on 1.01 / 1.01 (up to 1.10), from 0.6 on 1.08 / 1.06. Whole steps of 12 layers of Qwen3-4B (2 x
     9,728 of 2,560): 2,560 rows 0.868 / 0.987, 5,099 0.932 / 0.992, 6,144 0.959 / 1.006, 8,192 0.953 / 0.995, 9,472 0.955 /
-    0.985, 12,806 0.992 / 0.996, 768 0.987 / 0.986, 1,536 0.999 / 0.991 of the time; left to the library: 1,188 rows 1.044 /
+    0.985, 10,752 0.978 / 0.999, 768 0.987 / 0.986, 1,536 0.999 / 0.991 of the time; left to the library: 1,188 rows 1.044 /
     1.034, 1,368 1.010 / 1.021, 2,126 1.012 / 1.013, and 2,048 0.963 / 1.020 (0.79 filled).
-    At 13,824 rows it is still level (0.999 / 0.995); beyond 1.5e12 operations neither is ahead throughout (16,384 rows 1.009 /
-    1.006, 20,480 0.978 / 0.983, 32,000 1.019 / 1.016), and the library takes them.
+    Beyond 1.1e12 operations the library takes them: 12,806 rows are 0.992 / 0.996 on one card and up to 1.02 on others, 13,824
+    0.999 / 0.995, 16,384 1.009 / 1.006, 20,480 0.978 / 0.983, 32,000 1.019 / 1.016.
     The depths are those at which this holds. At K = 1,024 filling and draining a tile takes a quarter of its time
     (Qwen3-0.6B, full rounds, whole steps: 0.995 to 1.006 / 1.008 to 1.024); at K = 4,096 the activation is a tenth of the
     product and the library reaches 1.5 PFLOP/s (Qwen3-8B likewise: 0.958 to 1.002 / 1.012 to 1.023)."""

@@ -87,7 +87,7 @@ def test_float32_blocks_of_many_rows_fit_a_grid(rows, outputs):
     (1188, 9728, 2560, False), (1368, 9728, 2560, False), (2126, 9728, 2560, False), (2842, 9728, 2560, False),
     (2048, 6144, 2048, False), (3072, 6144, 2048, False), (1557, 8192, 2048, False), (2150, 3072, 1024, False), (4360, 3072, 1024, False),
     (1530, 12288, 4096, False), (6144, 12288, 4096, False), (12806, 12288, 4096, False),
-    (16384, 9728, 2560, False), (32000, 9728, 2560, False), (12806, 9728, 2560, True),
+    (16384, 9728, 2560, False), (32000, 9728, 2560, False), (12806, 9728, 2560, False), (10752, 9728, 2560, True),
     (768, 9728, 2560, True), (2560, 9728, 2560, True), (4096, 9728, 2560, True), (5099, 9728, 2560, True), (8192, 9728, 2560, True),
     (1280, 6144, 2048, True), (1024, 8192, 2048, True), (5099, 8192, 2048, True), (8447, 8960, 1536, True)])
 def test_gate_up_of_many_rows_goes_where_it_was_measured_ahead(rows, outputs, depth, ours):
