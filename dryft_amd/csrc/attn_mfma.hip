@@ -1,6 +1,6 @@
 // bfloat16 attention on the matrix cores (v_mfma_f32_16x16x32_bf16), reading keys and values from
 // the paged cache: a causal kernel for steps that bring many rows per sequence, and a split
-// kernel plus a combine for steps that bring one row per sequence. They stand where the reference
+// kernel for steps that bring one row per sequence. They stand where the reference
 // uses a library's flash attention for prompts (engine/dryft_qwen3/model.py:172-177) and its
 // split-KV kernel for decoding (kernels/attn_decode.py:36-118). Scores, running maximum, exponentials,
 // row sums and the output accumulator are float; probabilities are rounded to bfloat16 for the
@@ -942,17 +942,23 @@ __global__ __launch_bounds__(256, RP == 1 && !DIFF ? 4 : 2) void attn_causal_dir
 // ---------------------------------------------------------------------------------------------------
 // One row per sequence. Grid: (sequences, kv heads * head blocks, splits); four waves per workgroup.
 // The 16 "rows" of a wave are up to 16 query heads that share the kv head. A split covers a run of
-// pages; its waves take them in turn, each page's loads issued before the previous page's second
-// product so that memory stays busy, and merge their results in LDS. Each split writes an
-// unnormalised partial (o, m, l); the combine kernel merges splits in a fixed order, so results do
-// not depend on timing.
+// pages; its waves take half pages in turn, two of them on their way, and merge their results in LDS. Each split writes
+// an unnormalised partial (o, m, l), and the workgroup that ends last of a sequence's splits merges them in a fixed order,
+// so results do not depend on timing.
+// Bound by trips to memory one after the other where contexts are short (scalars, page numbers, projection and page,
+// partials, and back) and by the keys' way from memory where they are long. In a captured chain on rotating cold caches, us
+// before (whole pages, heads by the workgroup together, a combine kernel of its own) and now, 32 query heads on 8 of 128: one
+// sequence of 517 keys 13.3 / 9.3, of 2,000 15.0 / 11.3, eight of 1,600 to 2,048 (60 MB) 25.3 / 21.2, 64 of 97 to 475 (75 MB)
+// 29.7 / 27.9; 16 on 8, three of 150 to 410 11.5 / 9.0; 16 on 4 with q given ready, four of 501 to 2,048 12.8 / 10.8.
 // One q or k head of one row, as the fused projection left it: RMSNorm over the head (optional), then the
 // rotation of pairs (j, j + rot/2), with the same roundings as the stand-alone kernel (rope_kv.hip). One wave, in
 // two halves so that a caller can put other loads between them: `head_load` issues every load (head_dim <= 256:
 // at most 4 values per lane), `head_finish` computes. `tmp` is the wave's own LDS scratch of head_dim floats. The
 // result is written as bfloat16 to `dst` (in LDS) and, if given, to `dst2` (in global memory).
+#define HELD_PARTS 4                 // partial sums of the projection that are asked for at once
+template <int U>                     // values a lane: feature lane + 64 u of the head
 struct HeadRegs {
-  float x[4], wt[4], cs[4], sn[4];
+  uint32_t x[HELD_PARTS][U], wt[U], cs[U], sn[U];      // bits as they lie in memory: nothing waits for them before head_finish
 };
 
 // Where a row of the fused projection's output lies: as bfloat16 values, or as `parts` float partial sums over K,
@@ -962,57 +968,111 @@ struct ProjectedRow {
   const float* sums;
   int parts;
   int64_t part_stride;
-  __device__ __forceinline__ float at(int64_t i) const {
-    if (sums == nullptr) return bf16_to_float(values[i]);
-    float v = sums[i];
-    for (int s = 1; s < parts; ++s) v += sums[s * part_stride + i];
-    return rounded_as<bf16_t>(v);
-  }
 };
 
-__device__ __forceinline__ void head_load(HeadRegs& r, const ProjectedRow& src, int64_t first, const void* __restrict__ w,
+// Partial sums s0 .. s0 + 3 of a lane's values; a part beyond the last is read as the last one and not added.
+template <int U>
+__device__ __forceinline__ void load_parts(uint32_t (&x)[HELD_PARTS][U], const ProjectedRow& src, int s0, int64_t first, int head_dim) {
+  const int lane = threadIdx.x % WAVE;
+#pragma unroll
+  for (int s = 0; s < HELD_PARTS; ++s)
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      x[s][u] = __float_as_uint(src.sums[min(s0 + s, src.parts - 1) * src.part_stride + first + min(lane + WAVE * u, head_dim - 1)]);
+}
+
+// A lane's values of a row as the projection's epilogue would have left them, from what load_projected asked for.
+template <int U, bool SUMS>
+__device__ __forceinline__ void load_projected(uint32_t (&x)[HELD_PARTS][U], const ProjectedRow& src, int64_t first, int head_dim) {
+  const int lane = threadIdx.x % WAVE;
+  if (SUMS) {
+    load_parts<U>(x, src, 0, first, head_dim);
+    return;
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) x[0][u] = src.values[first + min(lane + WAVE * u, head_dim - 1)].bits;
+}
+template <int U, bool SUMS>
+__device__ __forceinline__ void projected(float (&v)[U], uint32_t (&x)[HELD_PARTS][U], const ProjectedRow& src, int64_t first,
+                                          int head_dim) {
+  if (!SUMS) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = __uint_as_float(x[0][u] << 16);
+    return;
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) v[u] = __uint_as_float(x[0][u]);
+#pragma unroll
+  for (int s = 1; s < HELD_PARTS; ++s)
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (s < src.parts) v[u] += __uint_as_float(x[s][u]);
+  for (int s0 = HELD_PARTS; s0 < src.parts; s0 += HELD_PARTS) {
+    load_parts<U>(x, src, s0, first, head_dim);
+#pragma unroll
+    for (int s = 0; s < HELD_PARTS; ++s)
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (s0 + s < src.parts) v[u] += __uint_as_float(x[s][u]);
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) v[u] = rounded_as<bf16_t>(v[u]);
+}
+
+// Every load of a head is unconditional, from a clamped and valid place, and nothing is computed here from what comes back:
+// a head is one trip to memory, and the caller's own loads go out behind it before anything waits. (Loops of a load and an
+// addition, and loads whose type was only known at run time, made it up to eight trips, 0.7 us each.)
+template <int U, bool SUMS>
+__device__ __forceinline__ void head_load(HeadRegs<U>& r, const ProjectedRow& src, int64_t first, const void* __restrict__ w,
                                           int w_f32, int has_norm, const bf16_t* __restrict__ cos_t,
                                           const bf16_t* __restrict__ sin_t, int rot, int pos, int head_dim) {
   const int lane = threadIdx.x % WAVE;
   const int half = rot / 2;
+  load_projected<U, SUMS>(r.x, src, first, head_dim);
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int i = lane + WAVE * u;
-    const bool in = i < head_dim;
-    r.x[u] = in ? src.at(first + i) : 0.f;
-    r.wt[u] = (in && has_norm) ? load_vector(w, i, w_f32) : 1.f;
-    const int j = i < half ? i : i - half;
-    r.cs[u] = (in && i < rot) ? bf16_to_float(cos_t[(int64_t)pos * half + j]) : 1.f;
-    r.sn[u] = (in && i < rot) ? bf16_to_float(sin_t[(int64_t)pos * half + j]) : 0.f;
+  for (int u = 0; u < U; ++u) {
+    const int i = min(lane + WAVE * u, head_dim - 1);
+    r.wt[u] = r.cs[u] = r.sn[u] = 0;
+    if (has_norm) r.wt[u] = w_f32 ? ((const uint32_t*)w)[i] : (uint32_t)((const uint16_t*)w)[i];
+    if (rot > 0) {
+      const int j = min(i < half ? i : i - half, half - 1);
+      r.cs[u] = cos_t[(int64_t)pos * half + j].bits;
+      r.sn[u] = sin_t[(int64_t)pos * half + j].bits;
+    }
   }
 }
 
-__device__ __forceinline__ void head_finish(HeadRegs& r, int has_norm, float eps, int rot, int head_dim, float* tmp,
-                                            bf16_t* dst, bf16_t* dst2) {
+template <int U, bool SUMS>
+__device__ __forceinline__ void head_finish(HeadRegs<U>& r, const ProjectedRow& src, int64_t first, int has_norm, int w_f32,
+                                            float eps, int rot, int head_dim, float* tmp, bf16_t* dst, bf16_t* dst2) {
   const int lane = threadIdx.x % WAVE;
   const int half = rot / 2;
+  float x[U];
+  projected<U, SUMS>(x, r.x, src, first, head_dim);
   if (has_norm) {
     float ss = 0.f;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) ss += r.x[u] * r.x[u];
+    for (int u = 0; u < U; ++u) ss += lane + WAVE * u < head_dim ? x[u] * x[u] : 0.f;
     ss = wave_sum(ss);
     const float inv = rsqrtf(ss / (float)head_dim + eps);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) r.x[u] = rounded_as<bf16_t>(rounded_as<bf16_t>(r.x[u] * inv) * r.wt[u]);
+    for (int u = 0; u < U; ++u)
+      x[u] = rounded_as<bf16_t>(rounded_as<bf16_t>(x[u] * inv) * __uint_as_float(w_f32 ? r.wt[u] : r.wt[u] << 16));
   }
 #pragma unroll
-  for (int u = 0; u < 4; ++u)
-    if (lane + WAVE * u < head_dim) tmp[lane + WAVE * u] = r.x[u];
+  for (int u = 0; u < U; ++u)
+    if (lane + WAVE * u < head_dim) tmp[lane + WAVE * u] = x[u];
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
   __builtin_amdgcn_wave_barrier();
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
+  for (int u = 0; u < U; ++u) {
     const int i = lane + WAVE * u;
     if (i >= head_dim) continue;
-    float o = r.x[u];
+    float o = x[u];
     if (i < rot) {
       const float other = tmp[i < half ? i + half : i - half];
-      const float a = rounded_as<bf16_t>(o * r.cs[u]), b = rounded_as<bf16_t>(other * r.sn[u]);
+      const float a = rounded_as<bf16_t>(o * __uint_as_float(r.cs[u] << 16));
+      const float b = rounded_as<bf16_t>(other * __uint_as_float(r.sn[u] << 16));
       o = i < half ? a - b : a + b;
     }
     const bf16_t v = float_to_bf16(o);
@@ -1039,160 +1099,444 @@ struct FusedQKV {
   int write_kv;
 };
 
+// A row's query heads of one kv head, its new key and its new value for one wave alone: lane 16 h + j takes features 8 j ..
+// 8 j + 7 of head h of four, so that heads are whole lines, the sum of squares and the rotation's pairs stay within 16 lanes
+// (moves within a row, no LDS), and four heads are one pass. They end in the wave's own piece of LDS, from where it takes its
+// operands: no wave waits for another. (Heads spread over the workgroup's waves with a barrier before the keys: 64 sequences
+// of 97 to 475 keys 30 us against 26. Heads in the operands' layout, features of a head over four lanes and eleven of sixteen
+// columns idle: 28.) Sums and roundings in the order of head_finish. Heads of 128 features that turn as a whole.
+#define DIRECT_HEAD 128
+#define DIRECT_PASSES 3
+struct HeadPass {
+  vf4 x[2][2];                       // two partial sums of the projection (or, in x[0][0], eight bfloat16 values)
+  bf16x8 w;
+};
+
+// `col`: the lane's first value in the row; `w`: at the lane's first value (any valid place without a norm). More than two
+// partial sums are added here, a trip to memory each, for models whose projection is split so often.
+template <bool SUMS>
+__device__ __forceinline__ void pass_load(HeadPass& r, const ProjectedRow& src, int64_t col, const bf16_t* w) {
+  if (!SUMS) {
+    r.x[0][0] = *(const vf4*)(src.values + col);
+    r.w = load8(w);
+    return;
+  }
+  auto part = [&](int at, int s) {
+    const float* p = src.sums + s * src.part_stride + col;
+    r.x[at][0] = *(const vf4*)p;
+    r.x[at][1] = *(const vf4*)(p + 4);
+  };
+  part(0, 0);
+  part(1, min(1, src.parts - 1));
+  r.w = load8(w);
+  for (int s = 2; s < src.parts; ++s) {
+    r.x[0][0] += r.x[1][0];
+    r.x[0][1] += r.x[1][1];
+    part(1, s);
+  }
+}
+
+// `plain`: neither normed nor turned (the value).
+template <bool SUMS>
+__device__ __forceinline__ bf16x8 pass_finish(const HeadPass& r, int parts, bool norm, float eps, bf16x8 cs, bf16x8 sn, bool plain) {
+  const bool upper = threadIdx.x % 16 >= 8;                   // the second half of a head's features
+  float x[8];
+  bf16x8 raw;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float one = r.x[0][i / 4][i % 4], two = r.x[1][i / 4][i % 4];
+    raw[i] = SUMS ? to_bf16(parts > 1 ? one + two : one) : __builtin_bit_cast(bf16x8, r.x[0][0])[i];
+    x[i] = (float)raw[i];
+  }
+  if (norm) {
+    float ss[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float far = dpp_move<0x128>(x[i]);                // row_ror:8: the feature 64 further on or back
+      const float lo = upper ? far : x[i], hi = upper ? x[i] : far;
+      ss[i] = fmaf(hi, hi, lo * lo);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ss[i] += dpp_move<0x124>(ss[i]);   // row_ror:4, the halves being equal: lane j ^ 4
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ss[i] += dpp_move<0x4E>(ss[i]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ss[i] += dpp_move<0xB1>(ss[i]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ss[i] += ss[i + 4];
+    const float inv = rsqrtf(((ss[0] + ss[2]) + (ss[1] + ss[3])) / (float)DIRECT_HEAD + eps);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = rounded_as<bf16_t>(rounded_as<bf16_t>(x[i] * inv) * (float)r.w[i]);
+  }
+  bf16x8 out;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float far = dpp_move<0x128>(x[i]);
+    const float mine = rounded_as<bf16_t>(x[i] * (float)cs[i]), theirs = rounded_as<bf16_t>(far * (float)sn[i]);
+    out[i] = to_bf16(upper ? mine + theirs : mine - theirs);
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) out[i] = plain ? raw[i] : out[i];
+  return out;
+}
+
 #define SPLIT_WAVES 4
 #define SPLIT_MAX_D 256
 
+// Values that workgroups of one launch hand to one another: stores and loads that pass by the caches which the chip's
+// compute dies keep for themselves.
+__device__ __forceinline__ void store_far(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ float load_far(const float* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// One row's splits added up by one wave: o = sum_s w_s o_s of the lane's features lane + 64 u, returns sum_s w_s l_s with
+// w_s = 2^(m_s - max m) (attn_decode.py:102-118). The outputs of the first splits are asked for along with the weights.
+#define COMBINE_MAX_SPLITS 64
+template <int U>
+__device__ __forceinline__ float combined(float (&o)[U], const float* po, const float* ml, int n, int head_dim, const float* sink,
+                                          int head) {
+  constexpr int HELD = U <= 2 ? 16 : 8;
+  const int lane = threadIdx.x % WAVE;
+  asm volatile("" : "+v"(n));                 // or the compiler keeps every comparison with n in scalar registers it has not got
+  float held[HELD][U];
+  int at[U];                                                  // of the split that is asked for next; stays at the last one
+#pragma unroll
+  for (int u = 0; u < U; ++u) at[u] = min(lane + WAVE * u, head_dim - 1);
+  auto ask = [&](int s0) {
+#pragma unroll
+    for (int s = 0; s < HELD; ++s) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        held[s][u] = load_far(po + at[u]);
+        at[u] += s0 + s < n - 1 ? head_dim : 0;
+      }
+    }
+  };
+  const int mine = min(lane, n - 1);
+  float ms = load_far(ml + 2 * mine), ls = load_far(ml + 2 * mine + 1);
+  ask(0);
+  if (lane >= n) ms = -INFINITY;
+  float m = fmaxf(ms, dpp_move<0xB1>(ms));                    // over 16 lanes by moves within the row (lanes_sum)
+  m = fmaxf(m, dpp_move<0x4E>(m));
+  m = fmaxf(m, dpp_move<0x141>(m));
+  m = fmaxf(m, dpp_move<0x140>(m));
+  if (n > 16) {
+    m = fmaxf(m, __shfl_xor(m, 16, WAVE));
+    m = fmaxf(m, __shfl_xor(m, 32, WAVE));
+  }
+  const float w = ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - m);
+  float l = lanes_sum<16>(w * ls);
+  if (n > 16) {
+    l += __shfl_xor(l, 16, WAVE);
+    l += __shfl_xor(l, 32, WAVE);
+  }
+  m = __shfl(m, 0, WAVE);
+  l = __shfl(l, 0, WAVE);
+  if (sink != nullptr && m != -INFINITY) l += sink_term(sink, head, m);
+#pragma unroll
+  for (int u = 0; u < U; ++u) o[u] = 0.f;
+  for (int s0 = 0; s0 < n; s0 += HELD) {
+    if (s0 > 0) ask(s0);
+#pragma unroll
+    for (int s = 0; s < HELD; ++s) {
+      const float ws = __shfl(w, min(s0 + s, WAVE - 1), WAVE);          // 0 beyond the last split
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (s0 + s < n) o[u] += ws * held[s][u];      // a split without keys has weight 0 and holds finite values
+    }
+  }
+  return l;
+}
+
+// Half a page, 32 keys, for one wave: loads, scores, online softmax and the second product, as for whole pages above. Halves
+// keep what is on its way in half the registers, so that the next half's keys and values are asked for before this one's are
+// looked at (whole pages spill: 64 sequences of 97 to 475 keys 44 us against 28).
+template <int KB>
+struct HalfPage {
+  bf16x8 k[2][KB], v[2 * KB];
+};
+
 template <int KB, bool FULL>
+__device__ __forceinline__ void load_half(HalfPage<KB>& f, const bf16_t* k_page, const bf16_t* v_page, int half, int head_dim) {
+  const int lane = threadIdx.x % WAVE, c = lane % 16, g = lane / 16;
+  const bf16_t* k = k_page + (32 * half + c) * head_dim;
+  const bf16_t* v = v_page + 32 * half + 8 * g;
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) f.k[t][kb] = load8(k + 16 * t * head_dim + (FULL ? 32 * kb + 8 * g : min(32 * kb + 8 * g, head_dim - 8)));
+#pragma unroll
+  for (int dt = 0; dt < 2 * KB; ++dt) f.v[dt] = load8(v + (FULL ? 16 * dt + c : min(16 * dt + c, head_dim - 1)) * PAGE_TOKENS);
+}
+
+// The key and value at position `pos`, which may not have reached memory yet, into the half page that holds it: key pos is row
+// pos % 16 of a tile of 16, as a value it is one element of one lane group (value_column).
+template <int KB>
+__device__ __forceinline__ void put_own(HalfPage<KB>& f, const bf16x8 (&key)[KB], const float (&value)[2 * KB], int pos) {
+  const int lane = threadIdx.x % WAVE, c = lane % 16, g = lane / 16;
+  const int t = pos % 32 / 16, col = value_column(pos % PAGE_TOKENS) % 32;
+  const bool mine = c == pos % 16;
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    if (mine && t == 0) f.k[0][kb] = key[kb];
+    if (mine && t == 1) f.k[1][kb] = key[kb];
+  }
+  const uint32_t keep = col % 2 ? 0x0000ffffu : 0xffff0000u;
+  const int shift = col % 2 ? 16 : 0;
+#pragma unroll
+  for (int dt = 0; dt < 2 * KB; ++dt) {
+    const uint32_t v = (uint32_t)float_to_bf16(value[dt]).bits << shift;
+    vu4 w = __builtin_bit_cast(vu4, f.v[dt]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (g == col / 8 && i == col % 8 / 2) w[i] = (w[i] & keep) | v;
+    f.v[dt] = __builtin_bit_cast(bf16x8, w);
+  }
+}
+
+template <int KB>
+__device__ __forceinline__ void half_update(RowBlock<KB>& st, const HalfPage<KB>& f, float scale_log2, int key0, int lo, int pos,
+                                            ScoreCap cap) {
+  const int g = (threadIdx.x % WAVE) / 16;
+  f32x4 s[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) s[t] = MFMA16(f.k[t][kb], st.q[kb], s[t]);
+  }
+  float lane_max = -INFINITY;
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int j = key0 + 16 * t + 4 * g + i;
+      if (cap.cap > 0.f) s[t][i] = cap.cap * fast_tanh(s[t][i] * cap.pre);
+      if (cap.rel != nullptr) {
+        const int dist = min(max(pos - j, 0), cap.n_dist - 1);
+        s[t][i] = fmaf(s[t][i], cap.rel_scale, cap.rel[(int64_t)dist * cap.rel_stride]);
+      }
+      s[t][i] = j >= lo && j <= pos ? s[t][i] : -INFINITY;
+      lane_max = fmaxf(lane_max, s[t][i]);
+    }
+  lane_max *= scale_log2;
+  if (__any(lane_max > st.m + MAX_SLACK)) {                   // see page_softmax
+    float row_max = fmaxf(lane_max, __shfl_xor(lane_max, 16, WAVE));
+    row_max = fmaxf(row_max, __shfl_xor(row_max, 32, WAVE));
+    const float m_new = fmaxf(st.m, row_max);
+    const float alpha = m_new == -INFINITY ? 1.f : fast_exp2(st.m - m_new);
+    st.l *= alpha;
+    st.m = m_new;
+#pragma unroll
+    for (int dt = 0; dt < 2 * KB; ++dt) st.o[dt] *= alpha;
+  }
+  const float m_ref = st.m == -INFINITY ? 0.f : st.m;
+  bf16x8 p;
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float e = fast_exp2(fmaf(s[t][i], scale_log2, -m_ref));
+      st.l += e;
+      p[4 * t + i] = to_bf16(e);
+    }
+#pragma unroll
+  for (int dt = 0; dt < 2 * KB; ++dt) st.o[dt] = MFMA16(f.v[dt], p, st.o[dt]);
+}
+
+// MODE: q is given ready, or the row's q, k and v come straight from the projection (FusedQKV, no score options or pairs),
+// by all waves together or by each for itself (HeadPass; bfloat16 weights, at most 10 query heads a kv head, 16-byte aligned).
+enum SplitMode { READY_Q, FUSED_LDS, FUSED_DIRECT };
+template <int KB, bool FULL, SplitMode MODE, bool SUMS>
 // The fused form appends the row's key and value through k_pages_w / v_pages_w, which are the same buffers as
 // k_pages / v_pages: none of the four is declared restrict.
 __global__ __launch_bounds__(64 * SPLIT_WAVES, 2) void attn_split_kernel(
     const bf16_t* __restrict__ q, const bf16_t* k_pages, const bf16_t* v_pages,
     const int* __restrict__ page_table, int max_pages, const int* __restrict__ seq_slot,
-    const int* __restrict__ cu_rows, const int* __restrict__ kv_len, float* __restrict__ part_o,
-    float* __restrict__ part_ml, int n_heads, int n_kv, int head_dim, float scale, int window, int n_splits,
-    FusedQKV fused, bf16_t* k_pages_w, bf16_t* v_pages_w, bf16_t* __restrict__ out, ScoreOptions opt) {
-  ScoreCap cap = score_cap(opt, scale, n_heads);
+    const int* __restrict__ cu_rows, const int* __restrict__ kv_len, float* part_o, float* part_ml, int* arrivals, int n_heads,
+    int n_kv, int group, int blocks, int any_dim, float scale, int window, int n_splits, FusedQKV fused, bf16_t* k_pages_w, bf16_t* v_pages_w,
+    bf16_t* __restrict__ out, ScoreOptions opt, MapPair pair) {
+  constexpr bool FUSED = MODE != READY_Q;
+  constexpr int U = (KB + 1) / 2;                              // features of a head that a lane holds outside the tiles
+  const int head_dim = FULL ? 32 * KB : any_dim;
+  ScoreCap cap = FUSED ? ScoreCap{} : score_cap(opt, scale, n_heads);
   __shared__ float merge_o[SPLIT_WAVES][16][32 * KB + 1];
   __shared__ float merge_ml[SPLIT_WAVES][16][2];
-  __shared__ __attribute__((aligned(16))) bf16_t q_lds[16][32 * KB];
-  __shared__ __attribute__((aligned(16))) bf16_t kv_new[2][32 * KB];   // the row's own key (normed, rotated) and value
+  __shared__ __attribute__((aligned(16))) bf16_t q_lds[MODE == FUSED_LDS ? 16 : 1][32 * KB];
+  __shared__ __attribute__((aligned(16))) bf16_t kv_new[2][MODE == FUSED_LDS ? 32 * KB : 8];   // the row's own key (normed, rotated) and value
+  __shared__ int came_last;
   const int seq = blockIdx.x, split = blockIdx.z;
-  const int group = n_heads / n_kv, blocks = (group + 15) / 16;
-  const int kvh = blockIdx.y / blocks, hb = blockIdx.y % blocks;
-  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, c = lane % 16, g = lane / 16;
+  const int kvh = blocks == 1 ? blockIdx.y : blockIdx.y / blocks, hb = blockIdx.y - kvh * blocks;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE, c = lane % 16, g = lane / 16;
   const int slot = seq_slot[seq];
-  const int head = kvh * group + hb * 16 + c;
-  const bool row_valid = hb * 16 + c < group;
   const int64_t row = cu_rows[seq];
-  // pages of this split, taken by its waves in turn
-  int pos = 0, lo = 0, pg = 0, pg1 = -1, pg_hi = 0, pg_first = 0;
-  const int* table = page_table + (int64_t)max(slot, 0) * max_pages;
-  if (slot >= 0) {
-    pos = kv_len[seq] - 1;                                     // the row's own position
-    lo = first_seen(pos, window, opt.chunk);
-    const int pg_lo = lo / PAGE_TOKENS;
-    pg_hi = pos / PAGE_TOKENS;
-    const int per = (pg_hi - pg_lo + n_splits) / n_splits;     // ceil(pages / splits)
-    pg1 = min(pg_hi, pg_lo + split * per + per - 1);
-    pg_first = pg_lo + split * per;
-    pg = pg_first + wave;
+  const int pos = kv_len[seq] - 1;                             // the row's own position
+  const int first_head = kvh * group + hb * 16, rows = min(16, group - hb * 16);
+  const int head = first_head + c;
+  const bool row_valid = c < rows;
+  const bool pairs = !FUSED && pair.v_dim > 0;
+  if (slot < 0) {                                              // a sequence that sits out: zeros, once
+    const int width = pairs ? pair.v_dim : head_dim, per_row = pairs ? 2 : 1;
+    bf16_t* o = out + (row * n_heads + first_head) / per_row * width;
+    if (split == 0)
+      for (int i = threadIdx.x; i < rows / per_row * width; i += blockDim.x) o[i] = float_to_bf16(0.f);
+    return;
   }
+  // pages of this split, taken by its waves in turn; splits past the sequence's end have none and nothing to say
+  const int lo = first_seen(pos, window, FUSED ? 0 : opt.chunk);
+  const int pg_lo = lo / PAGE_TOKENS, pg_hi = pos / PAGE_TOKENS;
+  const int per = (pg_hi - pg_lo + n_splits) / n_splits;       // ceil(pages / splits)
+  const int pg_first = pg_lo + split * per, pg1 = min(pg_hi, pg_first + per - 1);
+  if (pg_first > pg_hi) return;
+  const int live_splits = (pg_hi - pg_lo + per) / per;
+  // a wave takes every fourth half page; AHEAD of them are on their way
+  constexpr int AHEAD = KB <= 4 ? 2 : 1;
+  int unit = 2 * pg_first + wave;
+  const int unit_end = min(2 * pg1 + 2, pos / 32 + 1);
+  const int* table = page_table + (int64_t)slot * max_pages;
   const float scale_log2 = (cap.cap > 0.f || cap.rel != nullptr ? 1.f : scale) * 1.44269504088896340736f;
-  cap = for_head(cap, min(head, n_heads - 1));                 // a lane's row is a head here; absent rows read a valid column
+  if (!FUSED) cap = for_head(cap, min(head, n_heads - 1));     // a lane's row is a head here; absent rows read a valid column
   const int64_t page_elems = (int64_t)PAGE_TOKENS * head_dim;
-  PageK<KB> kf;
-  PageV<KB> vf;
-  int page = pg <= pg1 ? table[pg] : -1;
+  HalfPage<KB> held[AHEAD];
+  int held_page[AHEAD];
+#pragma unroll
+  for (int a = 0; a < AHEAD; ++a) held_page[a] = unit + SPLIT_WAVES * a < unit_end ? table[(unit + SPLIT_WAVES * a) / 2] : -1;
+  auto ask = [&](int a, int u, int page) {
+    const int64_t at = ((int64_t)page * n_kv + kvh) * page_elems;
+    load_half<KB, FULL>(held[a], k_pages + at, v_pages + at, u % 2, head_dim);
+  };
   RowBlock<KB> st;
-  bool values_asked = false;                      // the values of the wave's first page are on their way already
-  const bool fused_on = fused.qkv != nullptr;
-  // exactly one split has the row's own page among its pages (splits past the sequence's end have none)
-  const bool owns_last = fused_on && slot >= 0 && pg_first <= pg_hi && pg1 == pg_hi;
-  if (fused_on) {
-    // The row's q, k and v come straight from the projection. The waves norm and rotate the query heads this
-    // workgroup serves into LDS. The workgroup whose pages include the row's own position also norms and rotates
-    // the new key, appends key and value to the cache, and keeps both in LDS: the wave that reads that page puts
-    // them into its operands itself, so nothing has to wait for memory. The loads of a wave's first head are
-    // issued before those of its first page of keys and waited for first, so the two latencies overlap.
-    float* tmp = &merge_o[wave][0][0];                          // free until the merge
-    ProjectedRow src_row;
-    src_row.values = fused.parts > 0 ? nullptr : fused.qkv + row * fused.stride;
-    src_row.sums = fused.parts > 0 ? (const float*)fused.qkv + row * fused.stride : nullptr;
-    src_row.parts = fused.parts;
-    src_row.part_stride = fused.part_stride;
-    HeadRegs first;
-    const bool has_first = slot >= 0 && wave < group;
-    if (has_first)
-      head_load(first, src_row, (int64_t)(kvh * group + wave) * head_dim, fused.q_w, fused.w_f32, fused.has_norm,
-                fused.cos_t, fused.sin_t, fused.rot, pos, head_dim);
-    if (page >= 0) {
-      // the first page's values too: asked for behind the barrier below they would cost a trip to memory of their own
-      load_page_k<KB, FULL>(kf, k_pages + ((int64_t)page * n_kv + kvh) * page_elems, head_dim);
-      load_page_v<KB, FULL>(vf, v_pages + ((int64_t)page * n_kv + kvh) * page_elems, head_dim);
-      values_asked = true;
+  const bool owns_last = FUSED && pg1 == pg_hi;                // exactly one split has the row's own page among its pages
+  const ProjectedRow src_row = {SUMS ? nullptr : fused.qkv + row * fused.stride,
+                                SUMS ? (const float*)fused.qkv + row * fused.stride : nullptr, fused.parts, fused.part_stride};
+  bf16x8 own_key[KB] = {};
+  float own_value[2 * KB] = {};
+  // the wave that reads the half page in which the row's own key belongs
+  const bool owner = MODE == FUSED_DIRECT && owns_last && fused.write_kv && (pos / 32 - unit) % SPLIT_WAVES == 0;
+  const int page_own = owner ? table[pg_hi] : -1;
+  if constexpr (MODE == FUSED_DIRECT) {
+    const int j = lane % 16, limit = owner ? group + 2 : group;          // heads: queries, then the key, then the value
+    const bf16_t *cs_at = fused.cos_t + (int64_t)pos * (DIRECT_HEAD / 2) + j % 8 * 8, *sn_at = fused.sin_t + (int64_t)pos * (DIRECT_HEAD / 2) + j % 8 * 8;
+    HeadPass pass[DIRECT_PASSES] = {};
+    bf16x8 cs = load8(cs_at), sn = load8(sn_at);
+#pragma unroll
+    for (int p = 0; p < DIRECT_PASSES; ++p) {
+      if (p > 0 && 4 * p >= limit) continue;
+      const int h = 4 * p + lane / 16;
+      const int64_t col = (int64_t)(h < group ? kvh * group + h : h == group ? n_heads + kvh : n_heads + n_kv + kvh) * DIRECT_HEAD + 8 * j;
+      pass_load<SUMS>(pass[p], src_row, col, fused.has_norm ? (const bf16_t*)(h < group ? fused.q_w : fused.k_w) + 8 * j : cs_at);
     }
-    if (has_first)
-      head_finish(first, fused.has_norm, fused.eps, fused.rot, head_dim, tmp, &q_lds[wave][0], nullptr);
-    if (slot >= 0) {
-      for (int r = wave + SPLIT_WAVES; r < group; r += SPLIT_WAVES) {
-        HeadRegs more;
-        head_load(more, src_row, (int64_t)(kvh * group + r) * head_dim, fused.q_w, fused.w_f32, fused.has_norm,
-                  fused.cos_t, fused.sin_t, fused.rot, pos, head_dim);
-        head_finish(more, fused.has_norm, fused.eps, fused.rot, head_dim, tmp, &q_lds[r][0], nullptr);
-      }
-      if (owns_last) {
-        const int page_last = table[pg_hi];
-        const int64_t base = ((int64_t)max(page_last, 0) * n_kv + kvh) * page_elems;
+#pragma unroll
+    for (int a = 0; a < AHEAD; ++a)
+      if (held_page[a] >= 0) ask(a, unit + SPLIT_WAVES * a, held_page[a]);
+    bf16_t* heads = (bf16_t*)&merge_o[wave][0][0];              // free until the merge
+#pragma unroll
+    for (int p = 0; p < DIRECT_PASSES; ++p) {
+      if (p > 0 && 4 * p >= limit) continue;
+      const int h = 4 * p + lane / 16;
+      const bf16x8 v = pass_finish<SUMS>(pass[p], src_row.parts, fused.has_norm, fused.eps, cs, sn, h > group);
+      if (h < limit) *(bf16x8*)(heads + h * DIRECT_HEAD + 8 * j) = v;
+      if (owner && page_own >= 0) {
         const int at = pos % PAGE_TOKENS;
-        const bool store = fused.write_kv && page_last >= 0;
-        if (wave == SPLIT_WAVES - 1) {
-          HeadRegs key;
-          head_load(key, src_row, (int64_t)(n_heads + kvh) * head_dim, fused.k_w, fused.w_f32, fused.has_norm,
-                    fused.cos_t, fused.sin_t, fused.rot, pos, head_dim);
-          head_finish(key, fused.has_norm, fused.eps, fused.rot, head_dim, tmp, &kv_new[0][0],
-                      store ? k_pages_w + base + (int64_t)at * head_dim : nullptr);
-        }
-        if (wave == SPLIT_WAVES - 2) {
-          const int64_t vs = (int64_t)(n_heads + n_kv + kvh) * head_dim;
-          for (int i = lane; i < head_dim; i += WAVE) {
-            const bf16_t v = float_to_bf16(src_row.at(vs + i));
-            kv_new[1][i] = v;
-            if (store) v_pages_w[base + (int64_t)i * PAGE_TOKENS + value_column(at)] = v;
+        const int64_t base = ((int64_t)page_own * n_kv + kvh) * page_elems;
+        if (h == group) *(bf16x8*)(k_pages_w + base + (int64_t)at * DIRECT_HEAD + 8 * j) = v;
+        if (h == group + 1) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const __bf16 feature = v[i];
+            v_pages_w[base + (int64_t)(8 * j + i) * PAGE_TOKENS + value_column(at)].bits = __builtin_bit_cast(uint16_t, feature);
           }
         }
       }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    init_rows<KB>(st, heads + min(c, group - 1) * DIRECT_HEAD, c < group, head_dim);
+    if (owner) {
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) own_key[kb] = load8(heads + group * DIRECT_HEAD + 32 * kb + 8 * g);
+#pragma unroll
+      for (int dt = 0; dt < 2 * KB; ++dt) own_value[dt] = bf16_to_float(heads[(group + 1) * DIRECT_HEAD + 16 * dt + c]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  } else if (FUSED) {
+    // The waves norm and rotate the query heads this workgroup serves into LDS. The workgroup whose pages include the
+    // row's own position also norms and rotates the new key, appends key and value to the cache, and keeps both in LDS: the
+    // wave that reads that half page puts them into its operands itself, so nothing has to wait for memory. All loads of a
+    // wave's first head, of the new key or value and of the first half pages go out before anything waits, so that their
+    // latencies overlap.
+    float* tmp = &merge_o[wave][0][0];                          // free until the merge
+    const bool makes_key = owns_last && wave == SPLIT_WAVES - 1, makes_value = owns_last && wave == SPLIT_WAVES - 2;
+    const int64_t key_at = (int64_t)(n_heads + kvh) * head_dim, value_at = (int64_t)(n_heads + n_kv + kvh) * head_dim;
+    const int page_last = owns_last ? table[pg_hi] : -1;
+    HeadRegs<U> first, fresh;
+    const int64_t first_at = (int64_t)(kvh * group + wave) * head_dim;
+    if (wave < group)
+      head_load<U, SUMS>(first, src_row, first_at, fused.q_w, fused.w_f32, fused.has_norm, fused.cos_t, fused.sin_t, fused.rot, pos,
+                   head_dim);
+    if (makes_key)
+      head_load<U, SUMS>(fresh, src_row, key_at, fused.k_w, fused.w_f32, fused.has_norm, fused.cos_t, fused.sin_t, fused.rot, pos,
+                   head_dim);
+    if (makes_value) load_projected<U, SUMS>(fresh.x, src_row, value_at, head_dim);
+#pragma unroll
+    for (int a = 0; a < AHEAD; ++a)
+      if (held_page[a] >= 0) ask(a, unit + SPLIT_WAVES * a, held_page[a]);
+    if (wave < group)
+      head_finish<U, SUMS>(first, src_row, first_at, fused.has_norm, fused.w_f32, fused.eps, fused.rot, head_dim, tmp, &q_lds[wave][0],
+                     nullptr);
+    const int64_t base = ((int64_t)max(page_last, 0) * n_kv + kvh) * page_elems;
+    const int at = pos % PAGE_TOKENS;
+    const bool store = fused.write_kv && page_last >= 0;
+    if (makes_key)
+      head_finish<U, SUMS>(fresh, src_row, key_at, fused.has_norm, fused.w_f32, fused.eps, fused.rot, head_dim, tmp, &kv_new[0][0],
+                     store ? k_pages_w + base + (int64_t)at * head_dim : nullptr);
+    if (makes_value) {
+      float v[U];
+      projected<U, SUMS>(v, fresh.x, src_row, value_at, head_dim);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int i = lane + WAVE * u;
+        if (i >= head_dim) continue;
+        kv_new[1][i] = float_to_bf16(v[u]);
+        if (store) v_pages_w[base + (int64_t)i * PAGE_TOKENS + value_column(at)] = float_to_bf16(v[u]);
+      }
+    }
+    for (int r = wave + SPLIT_WAVES; r < group; r += SPLIT_WAVES) {
+      const int64_t more_at = (int64_t)(kvh * group + r) * head_dim;
+      head_load<U, SUMS>(first, src_row, more_at, fused.q_w, fused.w_f32, fused.has_norm, fused.cos_t, fused.sin_t, fused.rot, pos,
+                   head_dim);
+      head_finish<U, SUMS>(first, src_row, more_at, fused.has_norm, fused.w_f32, fused.eps, fused.rot, head_dim, tmp, &q_lds[r][0],
+                     nullptr);
     }
     __syncthreads();
-    init_rows<KB>(st, &q_lds[c][0], row_valid && slot >= 0, head_dim);
+    init_rows<KB>(st, &q_lds[MODE == FUSED_LDS ? c : 0][0], row_valid, head_dim);
   } else {
-    if (page >= 0) load_page_k<KB, FULL>(kf, k_pages + ((int64_t)page * n_kv + kvh) * page_elems, head_dim);
-    init_rows<KB>(st, q + (row * n_heads + head) * head_dim, row_valid && slot >= 0, head_dim);
+    init_rows<KB>(st, q + (row * n_heads + head) * head_dim, row_valid, head_dim);
+#pragma unroll
+    for (int a = 0; a < AHEAD; ++a)
+      if (held_page[a] >= 0) ask(a, unit + SPLIT_WAVES * a, held_page[a]);
   }
-  while (pg <= pg1) {
-    const int pg_next = pg + SPLIT_WAVES;
-    const int page_next = pg_next <= pg1 ? table[pg_next] : -1;
-    if (page >= 0) {
-      if (!values_asked) load_page_v<KB, FULL>(vf, v_pages + ((int64_t)page * n_kv + kvh) * page_elems, head_dim);
-      values_asked = false;
-      if (fused_on && fused.write_kv && pg == pg_hi) {
-        // this page holds the row's own position, whose key and value may not have reached memory yet: take them
-        // from LDS. Key `at` is row at%16 of key tile at/16; as a value it is one element of one lane group.
-        const int at = pos % PAGE_TOKENS;
-        if (c == at % 16) {
+  for (; unit < unit_end; unit += AHEAD * SPLIT_WAVES) {
 #pragma unroll
-          for (int t = 0; t < 4; ++t)
-            if (t == at / 16) {
+    for (int a = 0; a < AHEAD; ++a) {
+      const int here = unit + SPLIT_WAVES * a, next = here + AHEAD * SPLIT_WAVES;
+      if (here >= unit_end) break;
+      const int page_next = next < unit_end ? table[next / 2] : -1;
+      if (FUSED && owns_last && fused.write_kv && here == pos / 32) {
+        if (MODE == FUSED_LDS) {
 #pragma unroll
-              for (int kb = 0; kb < KB; ++kb) {
-                const int d = FULL ? 32 * kb + 8 * g : min(32 * kb + 8 * g, head_dim - 8);
-                kf.k[t][kb] = load8(&kv_new[0][d]);
-              }
-            }
+          for (int kb = 0; kb < KB; ++kb) own_key[kb] = load8(&kv_new[0][FULL ? 32 * kb + 8 * g : min(32 * kb + 8 * g, head_dim - 8)]);
+#pragma unroll
+          for (int dt = 0; dt < 2 * KB; ++dt) own_value[dt] = bf16_to_float(kv_new[1][FULL ? 16 * dt + c : min(16 * dt + c, head_dim - 1)]);
         }
-        const int col = value_column(at), hsel = col / 32, gsel = (col % 32) / 8, esel = col % 8;
-        if (g == gsel) {
-#pragma unroll
-          for (int dt = 0; dt < 2 * KB; ++dt) {
-            const int d = FULL ? 16 * dt + c : min(16 * dt + c, head_dim - 1);
-            const __bf16 nv = __builtin_bit_cast(__bf16, kv_new[1][d].bits);
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-              for (int e = 0; e < 8; ++e)
-                if (h == hsel && e == esel) vf.v[dt][h][e] = nv;
-          }
-        }
+        put_own<KB>(held[a], own_key, own_value, pos);
       }
-      f32x4 s[4];
-      page_scores<KB>(s, kf, st);
-      if (page_next >= 0)
-        load_page_k<KB, FULL>(kf, k_pages + ((int64_t)page_next * n_kv + kvh) * page_elems, head_dim);
-      page_update<KB>(st, s, vf, head_dim, scale_log2, pg * PAGE_TOKENS, lo, pos, true, cap);
-    } else if (page_next >= 0) {
-      load_page_k<KB, FULL>(kf, k_pages + ((int64_t)page_next * n_kv + kvh) * page_elems, head_dim);
+      if (held_page[a] >= 0) half_update<KB>(st, held[a], scale_log2, 32 * here, lo, pos, cap);
+      held_page[a] = page_next;
+      if (page_next >= 0) ask(a, next, page_next);
     }
-    pg = pg_next;
-    page = page_next;
   }
   // merge the four waves' results: o = sum_w 2^(m_w - m) o_w, l likewise
   const float l_wave = row_sum<KB>(st);
@@ -1207,7 +1551,7 @@ __global__ __launch_bounds__(64 * SPLIT_WAVES, 2) void attn_split_kernel(
     }
   }
   __syncthreads();
-  const int rows = min(16, group - hb * 16);
+  const bool alone = live_splits == 1 && !pairs;
   for (int idx = threadIdx.x; idx < rows * head_dim; idx += blockDim.x) {     // all heads of the block at once
     const int r = idx / head_dim, d = idx % head_dim;
     float m = -INFINITY;
@@ -1221,132 +1565,66 @@ __global__ __launch_bounds__(64 * SPLIT_WAVES, 2) void attn_split_kernel(
       l += wgt * merge_ml[w][r][1];
       o += wgt * merge_o[w][r][d];
     }
-    if (n_splits == 1 && out != nullptr) {                 // nothing to combine: this is the result
-      if (opt.sink != nullptr && m != -INFINITY) l += sink_term(opt.sink, kvh * group + hb * 16 + r, m);
-      out[(row * n_heads + kvh * group + hb * 16 + r) * head_dim + d] = float_to_bf16(l > 0.f ? o / l : 0.f);
+    if (alone) {                                           // nothing to combine: this is the result
+      if (!FUSED && opt.sink != nullptr && m != -INFINITY) l += sink_term(opt.sink, first_head + r, m);
+      out[(row * n_heads + first_head + r) * head_dim + d] = float_to_bf16(l > 0.f ? o / l : 0.f);
       continue;
     }
-    const int64_t at = ((int64_t)seq * n_heads + kvh * group + hb * 16 + r) * n_splits + split;
-    part_o[at * head_dim + d] = o;
+    const int64_t at = ((int64_t)seq * n_heads + first_head + r) * n_splits + split;
+    store_far(part_o + at * head_dim + d, o);
     if (d == 0) {
-      part_ml[at * 2] = m;       // in units of log2(e)
-      part_ml[at * 2 + 1] = l;
+      store_far(part_ml + at * 2, m);       // in units of log2(e)
+      store_far(part_ml + at * 2 + 1, l);
     }
   }
-}
-
-// out[seq_row, head, :] = sum_s w_s o_s / sum_s w_s l_s,  w_s = 2^(m_s - max m)  (attn_decode.py:102-118)
-#define COMBINE_MAX_SPLITS 64
-#define COMBINE_THREADS 128          // head sizes up to 256: two features a thread
-template <int COMBINE_HELD>          // how many splits a thread asks for before it knows their weights
-__global__ __launch_bounds__(COMBINE_THREADS) void attn_combine_kernel(const float* __restrict__ part_o,
-                                                           const float* __restrict__ part_ml,
-                                                           const int* __restrict__ seq_slot,
-                                                           const int* __restrict__ cu_rows, bf16_t* __restrict__ out,
-                                                           int n_heads, int head_dim, int n_splits,
-                                                           const float* __restrict__ sink) {
-  __shared__ float wgt[COMBINE_MAX_SPLITS];
-  __shared__ float inv_l;
-  const int seq = blockIdx.x, head = blockIdx.y, tid = threadIdx.x;
-  const int64_t row = cu_rows[seq];
-  bf16_t* o = out + (row * n_heads + head) * head_dim;
-  const float* ml = part_ml + ((int64_t)seq * n_heads + head) * n_splits * 2;
-  const float* po = part_o + ((int64_t)seq * n_heads + head) * n_splits * head_dim;
-  const bool live = seq_slot[seq] >= 0;
-  // The partial outputs are asked for before the weights are known, so that one trip to memory serves both (the
-  // kernel moves almost nothing: what it costs is its trips to memory one after the other). A thread holds the first
-  // COMBINE_HELD splits of its (at most two) features; further splits are read after the weights.
-  float held[2][COMBINE_HELD];
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const int d = min(tid + k * COMBINE_THREADS, head_dim - 1);        // every load unconditional, from a valid place
-#pragma unroll
-    for (int s = 0; s < COMBINE_HELD; ++s) held[k][s] = po[min(s, n_splits - 1) * head_dim + d];
-  }
-  if (tid < WAVE) {                       // the first wave turns (m_s, l_s) into weights
-    const float ms = (live && tid < n_splits) ? ml[2 * tid] : -INFINITY;
-    const float ls = (live && tid < n_splits) ? ml[2 * tid + 1] : 0.f;
-    const float m = wave_max(ms);
-    const float w = (ms == -INFINITY) ? 0.f : exp2f(ms - m);
-    float l = wave_sum(w * ls);
-    if (sink != nullptr && m != -INFINITY) l += sink_term(sink, head, m);
-    if (tid < n_splits) wgt[tid] = w;
-    if (tid == 0) inv_l = l > 0.f ? 1.f / l : 0.f;
+  if (alone) return;
+  // The workgroup that comes last of a row's splits adds them up, in their order, so that results do not depend on timing.
+  // Nobody waits: the others are gone by then. What they wrote went past the caches that the compute dies do not share
+  // (store_far), and is counted only once it has arrived.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int* count = arrivals + (int64_t)seq * gridDim.y + blockIdx.y;
+    const int before = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    came_last = before == live_splits - 1;
+    if (came_last) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next launch
   }
   __syncthreads();
+  if (!came_last) return;
+  if (!pairs) {
+    for (int r = wave; r < rows; r += SPLIT_WAVES) {
+      float o[U];
+      const int64_t at = ((int64_t)seq * n_heads + first_head + r) * n_splits;
+      const float l = combined<U>(o, part_o + at * head_dim, part_ml + 2 * at, live_splits, head_dim, FUSED ? nullptr : opt.sink, first_head + r);
+      const float inv_l = l > 0.f ? 1.f / l : 0.f;
 #pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const int d = tid + k * COMBINE_THREADS;
-    if (d >= head_dim) continue;
-    float num = 0.f;
-#pragma unroll
-    for (int s = 0; s < COMBINE_HELD; ++s)
-      if (s < n_splits) num += wgt[s] * held[k][s];      // a split without keys has weight 0 and holds finite values
-    for (int s = COMBINE_HELD; s < n_splits; ++s) num += wgt[s] * po[s * head_dim + d];
-    o[d] = float_to_bf16(num * inv_l);
-  }
-}
-
-// The same for the two maps of a head (MapPair above): query heads 2 h and 2 h + 1 of the partial results become one
-// row of v_dim features, o = a1 - lambda * a2 divided by its root mean square and times post.
-template <int COMBINE_HELD>
-__global__ __launch_bounds__(COMBINE_THREADS) void attn_combine_maps_kernel(const float* __restrict__ part_o,
-                                                                const float* __restrict__ part_ml,
-                                                                const int* __restrict__ seq_slot,
-                                                                const int* __restrict__ cu_rows, bf16_t* __restrict__ out,
-                                                                int n_heads, int head_dim, int n_splits,
-                                                                const float* __restrict__ sink, MapPair pair) {
-  __shared__ float wgt[2][COMBINE_MAX_SPLITS];
-  __shared__ float scratch[16];
-  const int seq = blockIdx.x, head = blockIdx.y, tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
-  const int64_t row = cu_rows[seq];
-  const float* ml = part_ml + ((int64_t)seq * n_heads + 2 * head) * n_splits * 2;
-  const float* po = part_o + ((int64_t)seq * n_heads + 2 * head) * n_splits * head_dim;
-  const int64_t map_stride = (int64_t)n_splits * head_dim;
-  const bool live = seq_slot[seq] >= 0;
-  float held[2][2][COMBINE_HELD];                             // [map][feature of the thread][split]
-#pragma unroll
-  for (int m = 0; m < 2; ++m)
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const int d = min(tid + k * COMBINE_THREADS, head_dim - 1);
-#pragma unroll
-      for (int s = 0; s < COMBINE_HELD; ++s) held[m][k][s] = po[m * map_stride + min(s, n_splits - 1) * head_dim + d];
+      for (int u = 0; u < U; ++u)
+        if (lane + WAVE * u < head_dim) out[(row * n_heads + first_head + r) * head_dim + lane + WAVE * u] = float_to_bf16(o[u] * inv_l);
     }
-  {                                       // wave m turns map m's (m_s, l_s) into weights, the sum's inverse included
-    const float* mine = ml + (int64_t)wave * n_splits * 2;
-    const float ms = (live && lane < n_splits) ? mine[2 * lane] : -INFINITY;
-    const float ls = (live && lane < n_splits) ? mine[2 * lane + 1] : 0.f;
-    const float m = wave_max(ms);
-    const float w = (ms == -INFINITY) ? 0.f : exp2f(ms - m);
-    float l = wave_sum(w * ls);
-    if (sink != nullptr && m != -INFINITY) l += sink_term(sink, 2 * head + wave, m);
-    if (lane < n_splits) wgt[wave][lane] = l > 0.f ? w / l : 0.f;
+    return;
   }
-  __syncthreads();
-  float o[2], ss = 0.f;
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const int d = tid + k * COMBINE_THREADS;
-    float a[2];
+  // the two maps of a head (MapPair above), neighbouring rows here: o = a1 - lambda * a2 divided by its root mean square and
+  // times post
+  for (int p = wave; p < rows / 2; p += SPLIT_WAVES) {
+    float a[2][U], ss = 0.f;
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
-      a[m] = 0.f;
+      const int64_t at = ((int64_t)seq * n_heads + first_head + 2 * p + m) * n_splits;
+      const float l = combined<U>(a[m], part_o + at * head_dim, part_ml + 2 * at, live_splits, head_dim, nullptr, 0);
+      const float inv_l = l > 0.f ? 1.f / l : 0.f;
 #pragma unroll
-      for (int s = 0; s < COMBINE_HELD; ++s)
-        if (s < n_splits) a[m] += wgt[m][s] * held[m][k][s];
-      if (d < head_dim)
-        for (int s = COMBINE_HELD; s < n_splits; ++s) a[m] += wgt[m][s] * po[m * map_stride + s * head_dim + d];
+      for (int u = 0; u < U; ++u) a[m][u] *= inv_l;
     }
-    o[k] = a[0] - pair.lambda * a[1];
-    ss += d < pair.v_dim ? o[k] * o[k] : 0.f;
-  }
-  ss = block_sum(ss, scratch);
-  const float r = pair.post / sqrtf(ss / (float)pair.v_dim + pair.eps);
 #pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const int d = tid + k * COMBINE_THREADS;
-    if (d < pair.v_dim) out[(row * (n_heads / 2) + head) * pair.v_dim + d] = float_to_bf16(o[k] * r);
+    for (int u = 0; u < U; ++u) {
+      a[0][u] -= pair.lambda * a[1][u];
+      ss += lane + WAVE * u < pair.v_dim ? a[0][u] * a[0][u] : 0.f;
+    }
+    const float r = pair.post / sqrtf(wave_sum(ss) / (float)pair.v_dim + pair.eps);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (lane + WAVE * u < pair.v_dim)
+        out[(row * (n_heads / 2) + first_head / 2 + p) * pair.v_dim + lane + WAVE * u] = float_to_bf16(a[0][u] * r);
   }
 }
 
@@ -1508,60 +1786,62 @@ DRYFT_API int dryft_attn_causal_projected_bf16(const void* qkv, int64_t qkv_stri
                       max_tiles, out, n_heads, n_kv, head_dim, scale, window, mode, projected, stream);
 }
 
+// Can each wave take the heads for itself? (16-byte pieces; queries, key and value in DIRECT_PASSES passes.)
+static bool direct_heads_ok(const FusedQKV& f, int group, int head_dim) {
+  const int piece = f.parts > 0 ? 4 : 8;
+  uintptr_t at = (uintptr_t)f.qkv | (uintptr_t)f.cos_t | (uintptr_t)f.sin_t;
+  if (f.has_norm) at |= (uintptr_t)f.q_w | (uintptr_t)f.k_w;
+  return head_dim == DIRECT_HEAD && f.rot == head_dim && group + 2 <= 4 * DIRECT_PASSES && !(f.has_norm && f.w_f32) && at % 16 == 0 &&
+         f.stride % piece == 0 && f.part_stride % piece == 0;
+}
+
 static int launch_split(const void* q, const void* k_pages, const void* v_pages, const int* page_table, int max_pages,
                         const int* seq_slot, const int* cu_rows, const int* kv_len, int n_seqs, float* part_o,
-                        float* part_ml, int n_splits, void* out, int n_heads, int n_kv, int head_dim, float scale,
+                        float* part_ml, int n_splits, int* arrivals, void* out, int n_heads, int n_kv, int head_dim, float scale,
                         int window, FusedQKV fused, hipStream_t stream, ScoreOptions opt = {0.f, nullptr},
-                        const MapPair* pair = nullptr) {
+                        MapPair pair = {0, 0, 0.f, 0.f, 0.f}) {
   if (n_seqs <= 0) return 0;
   if (!head_shape_ok(n_heads, n_kv, head_dim) || n_splits < 1 || n_splits > COMBINE_MAX_SPLITS) return -1;
+  if (arrivals == nullptr && (n_splits > 1 || pair.v_dim > 0)) return -1;
   const int group = n_heads / n_kv, blocks = (group + 15) / 16;
   if (fused.qkv != nullptr && (blocks != 1 || fused.rot > head_dim || (fused.rot & 1))) return -1;
   dim3 grid(n_seqs, n_kv * blocks, n_splits), block(64 * SPLIT_WAVES);
-#define LAUNCH_SPLIT(FULLV)                                                                                        \
-  hipLaunchKernelGGL((attn_split_kernel<KB, FULLV>), grid, block, 0, stream, (const bf16_t*)q, (const bf16_t*)k_pages, \
-                     (const bf16_t*)v_pages, page_table, max_pages, seq_slot, cu_rows, kv_len, part_o, part_ml,    \
-                     n_heads, n_kv, head_dim, scale, window, n_splits, fused, (bf16_t*)k_pages, (bf16_t*)v_pages,       \
-                     (bf16_t*)(pair != nullptr ? nullptr : out), opt)
-  if (head_dim % 32 == 0) {
-    DISPATCH_KB(head_dim / 32, LAUNCH_SPLIT(true));
+#define LAUNCH_SPLIT(FULLV, MODEV, SUMSV)                                                                          \
+  hipLaunchKernelGGL((attn_split_kernel<KB, FULLV, MODEV, SUMSV>), grid, block, 0, stream, (const bf16_t*)q, (const bf16_t*)k_pages, \
+                     (const bf16_t*)v_pages, page_table, max_pages, seq_slot, cu_rows, kv_len, part_o, part_ml, arrivals, \
+                     n_heads, n_kv, group, blocks, head_dim, scale, window, n_splits, fused, (bf16_t*)k_pages, (bf16_t*)v_pages,       \
+                     (bf16_t*)out, opt, pair)
+  const bool full = head_dim % 32 == 0;
+#define LAUNCH_ANY(MODEV, SUMSV)                                                       \
+  if (full) { DISPATCH_KB(head_dim / 32, LAUNCH_SPLIT(true, MODEV, SUMSV)); }          \
+  else { DISPATCH_KB((head_dim + 31) / 32, LAUNCH_SPLIT(false, MODEV, SUMSV)); }
+#define LAUNCH_DIRECT(SUMSV) { constexpr int KB = DIRECT_HEAD / 32; LAUNCH_SPLIT(true, FUSED_DIRECT, SUMSV); }
+  if (fused.qkv == nullptr) {
+    LAUNCH_ANY(READY_Q, false)
+  } else if (direct_heads_ok(fused, group, head_dim)) {
+    if (fused.parts > 0) LAUNCH_DIRECT(true)
+    else LAUNCH_DIRECT(false)
+  } else if (fused.parts > 0) {
+    LAUNCH_ANY(FUSED_LDS, true)
   } else {
-    DISPATCH_KB((head_dim + 31) / 32, LAUNCH_SPLIT(false));
+    LAUNCH_ANY(FUSED_LDS, false)
   }
+#undef LAUNCH_ANY
+#undef LAUNCH_DIRECT
 #undef LAUNCH_SPLIT
-  int rc = DRYFT_LAUNCH_CHECK();
-  if (rc) return rc;
-  if (pair != nullptr) {
-#define COMBINE_MAPS(HELD)                                                                                          \
-  hipLaunchKernelGGL(attn_combine_maps_kernel<HELD>, dim3(n_seqs, n_heads / 2), dim3(COMBINE_THREADS), 0, stream,    \
-                     part_o, part_ml, seq_slot, cu_rows, (bf16_t*)out, n_heads, head_dim, n_splits, opt.sink, *pair)
-    if (n_splits <= 4) COMBINE_MAPS(4);
-    else if (n_splits <= 8) COMBINE_MAPS(8);
-    else COMBINE_MAPS(16);
-#undef COMBINE_MAPS
-    return DRYFT_LAUNCH_CHECK();
-  }
-  if (n_splits == 1) return rc;
-#define COMBINE(HELD)                                                                                              \
-  hipLaunchKernelGGL(attn_combine_kernel<HELD>, dim3(n_seqs, n_heads), dim3(COMBINE_THREADS), 0, stream, part_o,   \
-                     part_ml, seq_slot, cu_rows, (bf16_t*)out, n_heads, head_dim, n_splits, opt.sink)
-  if (n_splits <= 4) COMBINE(4);
-  else if (n_splits <= 8) COMBINE(8);
-  else if (n_splits <= 16) COMBINE(16);
-  else COMBINE(32);
-#undef COMBINE
   return DRYFT_LAUNCH_CHECK();
 }
 
+// `arrivals`: zeros, one for each sequence, kv head and block of 16 of its query heads; zeros again after the launch.
 DRYFT_API int dryft_attn_split_bf16(const void* q, const void* k_pages, const void* v_pages, const int* page_table,
                                     int max_pages, const int* seq_slot, const int* cu_rows, const int* kv_len,
-                                    int n_seqs, float* part_o, float* part_ml, int n_splits, void* out, int n_heads,
+                                    int n_seqs, float* part_o, float* part_ml, int n_splits, int* arrivals, void* out, int n_heads,
                                     int n_kv, int head_dim, float scale, int window, float softcap, const float* sink,
                                     int chunk, const float* rel, int n_dist, hipStream_t stream) {
   FusedQKV none = {};
   if (chunk < 0 || (chunk > 0 && window > 0) || (rel != nullptr && n_dist <= 0)) return -1;
   return launch_split(q, k_pages, v_pages, page_table, max_pages, seq_slot, cu_rows, kv_len, n_seqs, part_o, part_ml,
-                      n_splits, out, n_heads, n_kv, head_dim, scale, window, none, stream,
+                      n_splits, arrivals, out, n_heads, n_kv, head_dim, scale, window, none, stream,
                       ScoreOptions{softcap, sink, chunk, rel, n_dist});
 }
 
@@ -1574,14 +1854,14 @@ DRYFT_API int dryft_attn_decode_fused_bf16(const void* qkv, int64_t qkv_stride, 
                                            int w_f32, int has_norm, float eps, const void* cos_t, const void* sin_t,
                                            int rot, int write_kv, void* k_pages, void* v_pages, const int* page_table,
                                            int max_pages, const int* seq_slot, const int* cu_rows, const int* kv_len,
-                                           int n_seqs, float* part_o, float* part_ml, int n_splits, void* out,
+                                           int n_seqs, float* part_o, float* part_ml, int n_splits, int* arrivals, void* out,
                                            int n_heads, int n_kv, int head_dim, float scale, int window,
                                            hipStream_t stream) {
   if (qkv == nullptr || qkv_parts < 0) return -1;
   FusedQKV fused = {(const bf16_t*)qkv, qkv_stride, qkv_parts, qkv_part_stride, q_w, k_w, w_f32, has_norm, eps,
                     (const bf16_t*)cos_t, (const bf16_t*)sin_t, rot, write_kv};
   return launch_split(nullptr, k_pages, v_pages, page_table, max_pages, seq_slot, cu_rows, kv_len, n_seqs, part_o,
-                      part_ml, n_splits, out, n_heads, n_kv, head_dim, scale, window, fused, stream);
+                      part_ml, n_splits, arrivals, out, n_heads, n_kv, head_dim, scale, window, fused, stream);
 }
 
 static int pair_ok(const MapPair& p, int n_heads, int n_kv, int head_dim) {
@@ -1619,13 +1899,13 @@ DRYFT_API int dryft_attn_causal_diff_bf16(const void* q, const void* k_pages, co
 // page's row, with zeros around it, so that the maps of all heads of a kv head share the 16 rows of a tile.
 DRYFT_API int dryft_attn_split_diff_bf16(const void* q, const void* k_pages, const void* v_pages, const int* page_table,
                                          int max_pages, const int* seq_slot, const int* cu_rows, const int* kv_len,
-                                         int n_seqs, float* part_o, float* part_ml, int n_splits, void* out, int n_heads,
+                                         int n_seqs, float* part_o, float* part_ml, int n_splits, int* arrivals, void* out, int n_heads,
                                          int n_kv, int head_dim, int v_dim, float scale, int window, float lambda,
                                          float post, float eps, hipStream_t stream) {
   FusedQKV none = {};
   const MapPair pair = {8, v_dim, lambda, post, eps};          // where the maps' keys sit is in q
   if (!pair_ok(pair, n_heads, n_kv, head_dim)) return -1;
   return launch_split(q, k_pages, v_pages, page_table, max_pages, seq_slot, cu_rows, kv_len, n_seqs, part_o, part_ml,
-                      n_splits, out, n_heads, n_kv, head_dim, scale, window, none, stream,
-                      ScoreOptions{0.f, nullptr, 0, nullptr, 0}, &pair);
+                      n_splits, arrivals, out, n_heads, n_kv, head_dim, scale, window, none, stream,
+                      ScoreOptions{0.f, nullptr, 0, nullptr, 0}, pair);
 }

@@ -63,17 +63,17 @@ _SIGNATURES = {
     "attn_rows": {"dryft_attn_rows": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _F, _P, _I, _I, _P, _I, _I, _I, _P]},
     "attn_mfma": {"dryft_attn_causal_diff_bf16": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _P, _I, _I, _I, _I, _I, _F,
                                                   _I, _F, _F, _F, _I, _P],
-                  "dryft_attn_split_diff_bf16": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _P, _P, _I, _P, _I, _I, _I, _I, _F, _I,
+                  "dryft_attn_split_diff_bf16": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _P, _P, _I, _P, _P, _I, _I, _I, _I, _F, _I,
                                                  _F, _F, _F, _P],
                   "dryft_attn_causal_bf16": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _P, _I, _I, _I, _F, _I, _I, _F, _P,
                                              _I, _P, _I, _P],
                   "dryft_attn_causal_takes_projection": [_I, _I],
                   "dryft_attn_causal_projected_bf16": [_P, _L, _P, _I, _I, _F, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _I,
                                                        _I, _P, _I, _I, _I, _F, _I, _I, _P],
-                  "dryft_attn_split_bf16": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _P, _P, _I, _P, _I, _I, _I, _F, _I,
+                  "dryft_attn_split_bf16": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _P, _P, _I, _P, _P, _I, _I, _I, _F, _I,
                                             _F, _P, _I, _P, _I, _P],
                   "dryft_attn_decode_fused_bf16": [_P, _L, _I, _L, _P, _P, _I, _I, _F, _P, _P, _I, _I, _P, _P, _P, _I, _P, _P,
-                                                   _P, _I, _P, _P, _I, _P, _I, _I, _I, _F, _I, _P]},
+                                                   _P, _I, _P, _P, _I, _P, _P, _I, _I, _I, _F, _I, _P]},
     "attn_f32": {"dryft_attn_f32_rows": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _F, _I, _P],
                  "dryft_attn_f32_tiles": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _P, _I, _I, _I, _F, _I, _P]},
     "gemm_f32": {"dryft_gemm_stream_f32": [_P, _L, _P, _P, _I, _I, _I, _P],
@@ -792,9 +792,26 @@ def attn_causal_projected_bf16(qkv, q_weight, eps: float, cos, sin, k_pages, v_p
         _stream()), "attn_causal_projected_bf16")
 
 
+def split_arrivals(n_seqs: int, n_heads: int, n_kv: int) -> int:
+    """How many counters a step of one row per sequence needs: one for each sequence, kv head and block of 16 of the query
+    heads that share it."""
+    return n_seqs * n_kv * ((n_heads // n_kv + 15) // 16)
+
+
+def _arrivals(given, n_seqs: int, n_heads: int, n_kv: int, needed: bool, like):
+    if given is None:
+        return torch.zeros(split_arrivals(n_seqs, n_heads, n_kv), dtype=torch.int32, device=like.device) if needed else None
+    _gpu(given, "arrivals", torch.int32)
+    if not (given.is_contiguous() and given.numel() >= split_arrivals(n_seqs, n_heads, n_kv)):
+        raise KernelError(f"arrivals: needs {split_arrivals(n_seqs, n_heads, n_kv)} contiguous entries")
+    return given
+
+
 def attn_split_bf16(q, k_pages, v_pages, page_table, seq_slot, cu_rows, kv_len, n_seqs: int, part_o, part_ml,
                     n_splits: int, out, n_heads: int, n_kv: int, head_dim: int, scale: float, window: int,
-                    softcap: float = 0.0, sink=None, chunk: int = 0, rel=None) -> None:
+                    softcap: float = 0.0, sink=None, chunk: int = 0, rel=None, arrivals=None) -> None:
+    """``arrivals``: zeros that the splits of a sequence count themselves with (``split_arrivals`` of them, int32), zeros
+    again afterwards; None: made for the call."""
     _check_sink(sink, n_heads)
     _check_rel(rel, n_heads)
     _gpu(q, "q", torch.bfloat16)
@@ -815,15 +832,17 @@ def attn_split_bf16(q, k_pages, v_pages, page_table, seq_slot, cu_rows, kv_len, 
         raise KernelError("attn_split: grid too large")
     _check(_fn("attn_mfma", "dryft_attn_split_bf16")(
         _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(page_table), page_table.shape[1], _ptr(seq_slot), _ptr(cu_rows),
-        _ptr(kv_len), n_seqs, _ptr(part_o), _ptr(part_ml), n_splits, _ptr(out), n_heads, n_kv, head_dim, float(scale),
+        _ptr(kv_len), n_seqs, _ptr(part_o), _ptr(part_ml), n_splits,
+        _ptr(_arrivals(arrivals, n_seqs, n_heads, n_kv, n_splits > 1, q)), _ptr(out), n_heads, n_kv, head_dim, float(scale),
         int(window), float(softcap), _ptr(sink), int(chunk), _ptr(rel), rel.shape[0] if rel is not None else 0,
         _stream()), "attn_split_bf16")
 
 
 def attn_decode_fused_bf16(qkv, q_weight, k_weight, eps: float, cos, sin, rot: int, write_kv: bool, k_pages, v_pages,
                            page_table, seq_slot, cu_rows, kv_len, n_seqs: int, part_o, part_ml, n_splits: int, out,
-                           n_heads: int, n_kv: int, head_dim: int, scale: float, window: int, qkv_parts: int = 0) -> None:
-    """One row per sequence: q/k norm, rotation, append to the cache and attention in one kernel (plus the combine).
+                           n_heads: int, n_kv: int, head_dim: int, scale: float, window: int, qkv_parts: int = 0,
+                           arrivals=None) -> None:
+    """One row per sequence: q/k norm, rotation, append to the cache and attention in one kernel.
 
     ``qkv`` is the fused projection's output ``[n_seqs rows, (heads + 2 kv heads) * head_dim]``; row ``i`` belongs to
     sequence ``i`` (``cu_rows[i] == i``). It may also be that product left as float32 partial sums over K,
@@ -878,7 +897,8 @@ def attn_decode_fused_bf16(qkv, q_weight, k_weight, eps: float, cos, sin, rot: i
         _ptr(qkv), row_stride, int(qkv_parts), part_stride, _ptr(q_weight), _ptr(k_weight), w_f32, int(has_norm),
         float(eps), _ptr(cos), _ptr(sin),
         int(rot), int(write_kv), _ptr(k_pages), _ptr(v_pages), _ptr(page_table), page_table.shape[1], _ptr(seq_slot),
-        _ptr(cu_rows), _ptr(kv_len), n_seqs, _ptr(part_o), _ptr(part_ml), n_splits, _ptr(out), n_heads, n_kv, head_dim,
+        _ptr(cu_rows), _ptr(kv_len), n_seqs, _ptr(part_o), _ptr(part_ml), n_splits,
+        _ptr(_arrivals(arrivals, n_seqs, n_heads, n_kv, n_splits > 1, qkv)), _ptr(out), n_heads, n_kv, head_dim,
         float(scale), int(window), _stream()), "attn_decode_fused_bf16")
 
 
@@ -1552,7 +1572,7 @@ def attn_causal_diff_bf16(q, k_pages, v_pages, page_table, seq_slot, cu_rows, ti
 
 def attn_split_diff_bf16(q, k_pages, v_pages, page_table, seq_slot, cu_rows, kv_len, n_seqs: int, part_o, part_ml,
                          n_splits: int, out, n_heads: int, n_kv: int, map_dim: int, v_dim: int, scale: float, window: int,
-                         lam: float, post: float, eps: float) -> None:
+                         lam: float, post: float, eps: float, arrivals=None) -> None:
     """The same for steps of one row per sequence; ``q [rows, heads, 2, page width]`` holds map ``m`` at ``m * map_dim`` and
     zeros elsewhere."""
     page_dim = _diff_operands("attn_split_diff", q, k_pages, v_pages, page_table, out, n_heads, n_kv, map_dim, v_dim,
@@ -1570,7 +1590,8 @@ def attn_split_diff_bf16(q, k_pages, v_pages, page_table, seq_slot, cu_rows, kv_
         raise KernelError("attn_split_diff: grid too large")
     _check(_fn("attn_mfma", "dryft_attn_split_diff_bf16")(
         _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(page_table), page_table.shape[1], _ptr(seq_slot), _ptr(cu_rows),
-        _ptr(kv_len), n_seqs, _ptr(part_o), _ptr(part_ml), n_splits, _ptr(out), 2 * n_heads, n_kv, page_dim, v_dim,
+        _ptr(kv_len), n_seqs, _ptr(part_o), _ptr(part_ml), n_splits,
+        _ptr(_arrivals(arrivals, n_seqs, 2 * n_heads, n_kv, True, q)), _ptr(out), 2 * n_heads, n_kv, page_dim, v_dim,
         float(scale), int(window), float(lam), float(post), float(eps), _stream()), "attn_split_diff_bf16")
 
 

@@ -55,6 +55,7 @@ from .rope import HalfRotaryPositions, PairRotaryPositions, RotaryPositions
 
 _RESIDENT_WORKGROUPS = 512     # of the split kernel: two per compute unit (its registers allow no more)
 _MAX_SPLITS = 32
+_SHORT_SPLITS = 16             # of contexts up to 128 pages
 _QKV_PARTIAL_ROWS = 256         # decoding steps of up to so many rows take the projection as partial sums over K
 _PROMPT_PARTIAL_ROWS = 256      # and so do prompt steps of at most so many rows
 
@@ -109,9 +110,18 @@ def keys_seen(spans: list[tuple[int, int]], window: int | None, chunk: int | Non
 def key_splits(n_seqs: int, blocks: int, span: int) -> int:
     """How many ways each sequence's keys are split in decoding (``blocks`` workgroups a sequence and split, ``span`` keys
     at most): as many as run at the same time, and no more. Workgroups beyond what the chip holds at once start when
-    the first ones end, which costs more than the longer walk of fewer, larger splits."""
+    the first ones end, which costs more than the longer walk of fewer, larger splits. Nor more than sixteen before a split
+    holds eight pages, since one workgroup adds them all up at the end: 32 heads on 8 of 128, us at 16 / 24 / 32 splits, one
+    sequence of 2,000 keys 11.3 / 11.3 / 13.4, of 4,000 13.6 / 14.6 / 15.1, of 16,000 28.0 / 25.7 / 24.9; two of 2,000 13.4 /
+    14.2 / 15.9."""
     pages = max(1, (span + 63) // 64)
-    return max(1, min(_RESIDENT_WORKGROUPS // (n_seqs * blocks), _MAX_SPLITS, pages))
+    return max(1, min(_RESIDENT_WORKGROUPS // (n_seqs * blocks), max(_SHORT_SPLITS, pages // 8), _MAX_SPLITS, pages))
+
+
+def split_counters(ctx: StepContext, n_heads: int, n_kv: int) -> torch.Tensor:
+    """What the splits of a decoding step count themselves with: zeros between launches, one set per step context (its
+    launches run one after another)."""
+    return ctx.kept_zeros((ops.split_arrivals(ctx.n_seqs, n_heads, n_kv),), torch.int32)
 
 
 def distance_row(n: int, rows: int, far: int) -> int:
@@ -324,7 +334,8 @@ class GQAAttention(Mixer):
             part_ml = torch.empty((ctx.n_seqs, H, splits, 2), dtype=torch.float32, device=h.device)
             ops.attn_split_bf16(q, line.k, line.v, line.page_table, ctx.seq_slot, ctx.cu_rows, ctx.kv_len, ctx.n_seqs,
                                 part_o, part_ml, splits, out, H, G, D, self.scale, window, softcap=self.softcap,
-                                sink=self.sink, chunk=self.chunk or 0, rel=self.rel)
+                                sink=self.sink, chunk=self.chunk or 0, rel=self.rel,
+                                arrivals=split_counters(ctx, H, G))
         elif matrix_cores:
             # the tiled kernel never visits the rows of sequences that sit out; they must hold something finite
             out = ctx.kept_zeros((rows, H, Dv), h.dtype) if ctx.some_sit_out() else \
@@ -404,7 +415,8 @@ class GQAAttention(Mixer):
             ops.attn_decode_fused_bf16(qkv.data if parts else qkv, self.q_norm, self.k_norm, self.qk_norm_eps or 0.0, cos, sin, self.rotary_dim,
                                        writes_cache, line.k, line.v, line.page_table, ctx.seq_slot, ctx.cu_rows,
                                        ctx.kv_len, ctx.n_seqs, part_o, part_ml, splits, out, self.n_heads, self.n_kv,
-                                       self.head_dim, self.scale, window, qkv_parts=parts)
+                                       self.head_dim, self.scale, window, qkv_parts=parts,
+                                       arrivals=split_counters(ctx, self.n_heads, self.n_kv))
             return linear(out.view(rows, self.q_dim), self.w_o, allow_partials=True)
         if prompt_parts and isinstance(qkv, Partials):
             q = torch.empty((rows, self.n_heads, self.head_dim), dtype=h.dtype, device=h.device)
@@ -438,7 +450,7 @@ class GQAAttention(Mixer):
         if decoding:
             ops.attn_split_bf16(q, line.k, line.v, line.page_table, ctx.seq_slot, ctx.cu_rows, ctx.kv_len,
                                 ctx.n_seqs, part_o, part_ml, splits, out, self.n_heads, self.n_kv, self.head_dim,
-                                self.scale, window)
+                                self.scale, window, arrivals=split_counters(ctx, self.n_heads, self.n_kv))
         elif matrix_cores:
             tile_cu, max_tiles = ctx.tiles(ops.ATTN_ROW_TILE)
             ops.attn_causal_bf16(q, line.k, line.v, line.page_table, ctx.seq_slot, ctx.cu_rows, tile_cu,

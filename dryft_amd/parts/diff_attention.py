@@ -32,7 +32,7 @@ from ..csrc import ops
 from ..limits import MATRIX_CORE_HEAD_STEP, MAX_HEAD_DIM
 from ..weights.spec import VECTOR
 from . import register_part
-from .attention import key_splits, keys_seen
+from .attention import key_splits, keys_seen, split_counters
 from .base import Mixer, Partials, StepContext, matrix
 from .linear import linear
 from .rope import PairRotaryPositions
@@ -124,7 +124,7 @@ class DifferentialAttention(Mixer):
             part_ml = torch.empty((ctx.n_seqs, 2 * H, splits, 2), dtype=torch.float32, device=h.device)
             ops.attn_split_diff_bf16(q, line.k, line.v, line.page_table, ctx.seq_slot, ctx.cu_rows, ctx.kv_len, ctx.n_seqs,
                                      part_o, part_ml, splits, out, H, G, step, Dv, self.scale, window, self.lam, post,
-                                     self.norm_eps)
+                                     self.norm_eps, arrivals=split_counters(ctx, 2 * H, G))
         elif wide:
             tile_cu, max_tiles = ctx.tiles(ops.ATTN_ROW_TILE)
             ops.attn_causal_diff_bf16(q, line.k, line.v, line.page_table, ctx.seq_slot, ctx.cu_rows, tile_cu, ctx.seq_start,

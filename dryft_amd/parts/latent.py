@@ -32,7 +32,7 @@ from ..csrc import ops
 from ..limits import MATRIX_CORE_HEAD_STEP, MAX_HEAD_DIM
 from ..weights.spec import VECTOR
 from . import register_part
-from .attention import GQAAttention
+from .attention import GQAAttention, split_counters
 from .base import Mixer, StepContext, matrix
 from .linear import linear
 from .rope import PairRotaryPositions
@@ -118,7 +118,8 @@ class LatentAttention(Mixer):
             part_o = torch.empty((ctx.n_seqs, H, splits, D), dtype=torch.float32, device=h.device)
             part_ml = torch.empty((ctx.n_seqs, H, splits, 2), dtype=torch.float32, device=h.device)
             ops.attn_split_bf16(q, line.k, line.v, line.page_table, ctx.seq_slot, ctx.cu_rows, ctx.kv_len, ctx.n_seqs,
-                                part_o, part_ml, splits, out, H, H, D, self.scale, window, sink=self.sink)
+                                part_o, part_ml, splits, out, H, H, D, self.scale, window, sink=self.sink,
+                                arrivals=split_counters(ctx, H, H))
         elif self._matrix_cores():
             # the tiled kernel never visits the rows of sequences that sit out; they must hold something finite
             out = ctx.kept_zeros((rows, H, D), h.dtype) if ctx.some_sit_out() else \

@@ -1,0 +1,108 @@
+"""Attention of decoding steps: heads that each wave takes for itself, and splits whose last workgroup adds them up."""
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def step(n_heads, n_kv, D, lengths, seed, dead=None):
+    """Pages, slots and the projection's output of one decoding step; sequence ``dead`` sits out."""
+    gen = torch.Generator().manual_seed(seed)
+    rng = np.random.default_rng(seed)
+    B, max_pages = len(lengths), -(-max(lengths) // 64)
+    table = torch.tensor(rng.permutation((B + 1) * max_pages).reshape(B + 1, max_pages), dtype=torch.int32, device=DEV)
+    slots = [int(x) for x in rng.permutation(B + 1)[:B]]
+    if dead is not None:
+        slots[dead] = -1
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    n_pages = (B + 1) * max_pages
+    k = torch.randn(n_pages, n_kv, 64, D, generator=gen).to(torch.bfloat16).to(DEV)
+    v = torch.randn(n_pages, n_kv, D, 64, generator=gen).to(torch.bfloat16).to(DEV)
+    qkv = (2 * torch.randn(B, (n_heads + 2 * n_kv) * D, generator=gen)).to(torch.bfloat16)
+    wq, wk = ((1 + 0.1 * torch.randn(D, generator=gen)).to(torch.bfloat16).to(DEV) for _ in range(2))
+    ang = torch.arange(512).float()[:, None] * (1.0 / (1e4 ** (torch.arange(0, D, 2).float() / D)))[None]
+    cos, sin = ang.cos().to(torch.bfloat16).to(DEV), ang.sin().to(torch.bfloat16).to(DEV)
+    return dict(table=table, slots=i32(slots), cu=i32(list(range(B + 1))), kv_len=i32(lengths), pos=i32([n - 1 for n in lengths]),
+                k=k, v=v, qkv=qkv, wq=wq, wk=wk, cos=cos, sin=sin)
+
+
+def buffers(B, n_heads, splits, D):
+    return (torch.full((B * n_heads * splits * D,), float("nan"), device=DEV),
+            torch.full((B * n_heads * splits * 2,), float("nan"), device=DEV))
+
+
+# 10 query heads a kv head are the most that a wave takes for itself, in three passes of four heads, key and value; 2 and 3
+# share a pass with key and value, 4 and 7 do not; a position in every quarter of a page and on both sides of its ends
+@pytest.mark.parametrize("group", [1, 2, 3, 4, 7, 10, 11])
+@pytest.mark.parametrize("parts", [0, 1, 2, 5])
+def test_heads_of_a_wave_equal_the_kernel_of_their_own(group, parts):
+    from dryft_amd.csrc import ops as o
+    n_kv, D, splits = 2, 128, 3
+    n_heads, lengths = group * n_kv, [1, 32, 33, 64, 65, 97, 200, 17, 448]
+    s = step(n_heads, n_kv, D, lengths, 10 * group + parts, dead=3)
+    B, scale = len(lengths), D ** -0.5
+    po, pml = buffers(B, n_heads, splits, D)
+    if parts:
+        gen = torch.Generator().manual_seed(parts)
+        given = torch.randn(parts, *s["qkv"].shape, generator=gen).to(DEV)
+        total = given[0].clone()
+        for p in given[1:]:
+            total += p
+        plain = total.to(torch.bfloat16)
+    else:
+        given = plain = s["qkv"].to(DEV)
+    k1, v1, k2, v2 = s["k"].clone(), s["v"].clone(), s["k"].clone(), s["v"].clone()
+    q = torch.empty(B, n_heads, D, dtype=torch.bfloat16, device=DEV)
+    out1, out2 = (torch.full((B, n_heads, D), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    o.qk_norm_rope_kv(plain, s["wq"], s["wk"], 1e-6, s["cos"], s["sin"], D, s["slots"], s["pos"], q, k1, v1, s["table"], True,
+                      n_heads, n_kv, D)
+    o.attn_split_bf16(q, k1, v1, s["table"], s["slots"], s["cu"], s["kv_len"], B, po, pml, splits, out1, n_heads, n_kv, D,
+                      scale, 0)
+    arrivals = torch.zeros(o.split_arrivals(B, n_heads, n_kv), dtype=torch.int32, device=DEV)
+    for _ in range(2):                                        # the second launch finds the counters as the first left them
+        o.attn_decode_fused_bf16(given, s["wq"], s["wk"], 1e-6, s["cos"], s["sin"], D, True, k2, v2, s["table"], s["slots"],
+                                 s["cu"], s["kv_len"], B, po, pml, splits, out2, n_heads, n_kv, D, scale, 0, qkv_parts=parts,
+                                 arrivals=arrivals)
+        assert torch.equal(k1, k2) and torch.equal(v1, v2)
+        assert torch.equal(out1, out2)
+        assert not arrivals.any()
+    assert not out2[3].any(), "a sequence that sits out holds zeros"
+
+
+# fewer pages than splits, pages that do not divide among them, more than 16 splits, one and two blocks of 16 query heads
+@pytest.mark.parametrize("n_heads,n_kv,D,window", [(8, 2, 128, 0), (20, 1, 64, 0), (6, 3, 48, 70), (4, 1, 256, 0), (2, 2, 112, 0)])
+@pytest.mark.parametrize("splits", [1, 2, 5, 17, 33])
+def test_splits_added_by_the_last_workgroup(n_heads, n_kv, D, window, splits):
+    from dryft_amd.csrc import ops as o
+    lengths = [1, 31, 64, 65, 300, 1100]
+    s = step(n_heads, n_kv, D, lengths, D + splits, dead=1)
+    B, scale, group = len(lengths), D ** -0.5, n_heads // n_kv
+    gen = torch.Generator().manual_seed(splits)
+    q = torch.randn(B, n_heads, D, generator=gen).to(torch.bfloat16).to(DEV)
+    po, pml = buffers(B, n_heads, splits, D)
+    out = torch.full((B, n_heads, D), float("nan"), dtype=torch.bfloat16, device=DEV)
+    arrivals = torch.zeros(o.split_arrivals(B, n_heads, n_kv), dtype=torch.int32, device=DEV)
+    o.attn_split_bf16(q, s["k"], s["v"], s["table"], s["slots"], s["cu"], s["kv_len"], B, po, pml, splits, out, n_heads, n_kv, D,
+                      scale, window, arrivals=arrivals)
+    assert not arrivals.any() and not out[1].any()
+    for b, n in enumerate(lengths):
+        if b == 1:
+            continue
+        pages = s["table"][int(s["slots"][b]), :-(-n // 64)].long()
+        keys = s["k"][pages].permute(1, 0, 2, 3).reshape(n_kv, -1, D)[:, :n].double()
+        at = torch.tensor([value_column(p) for p in range(64)], device=DEV)
+        values = s["v"][pages][..., at].permute(1, 0, 3, 2).reshape(n_kv, -1, D)[:, :n].double()
+        lo = max(0, n - window) if window else 0
+        scores = torch.matmul(q[b].double().view(n_kv, group, D), keys.transpose(1, 2)) * scale
+        scores[..., :lo] = -torch.inf
+        want = torch.matmul(torch.softmax(scores, -1), values).reshape(n_heads, D)
+        # probabilities and the result are rounded to bfloat16: each half an ulp, 2^-9, of values up to the largest
+        assert float((out[b].double() - want).abs().max()) <= 2 * 2.0 ** -9 * float(values.abs().max())
+
+
+def value_column(pos):
+    o = pos & 31
+    return (pos & 32) + 8 * ((o >> 2) & 3) + 4 * (o >> 4) + (o & 3)
