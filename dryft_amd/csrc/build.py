@@ -26,10 +26,11 @@ ARCH = "gfx950"
 HIPCC_FLAGS = ["-O3", f"--offload-arch={ARCH}", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden",
                "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 MODULES = ("batch", "embed", "norm", "activation", "rope_kv", "attn_rows", "attn_f32", "attn_mfma", "gemm",
-           "gemm_f32", "sampling", "mlstm",
+           "gemm_lines", "gemm_f32", "sampling", "mlstm",
            "rglru", "hyper", "wkv", "latent", "moe", "conv", "ssm", "delta", "linattn", "mla")
 _HEADERS = ("common.h",)                       # every library includes these
-_OWN_HEADERS = {"sampling": ("sampling.h",), "delta": ("chunk_walk.h",), "ssm": ("chunk_walk.h",)}    # and some a header of their own
+_OWN_HEADERS = {"gemm": ("gate_unit.h",), "gemm_lines": ("gate_unit.h",), "sampling": ("sampling.h",),
+                "delta": ("chunk_walk.h",), "ssm": ("chunk_walk.h",)}    # and some a header of their own
 
 _loaded: dict[str, ctypes.CDLL] = {}
 _lock = threading.Lock()

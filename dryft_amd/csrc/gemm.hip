@@ -8,7 +8,7 @@
 //    weight is read once and multiplied on the matrix cores; K may be split across workgroups into
 //    float partial sums that the consumer adds in a fixed order. gemm_panel (M <= 64) is the fused gate/up
 //    product, gemm_mid (M <= 256) the projections back to the hidden width for short prompts.
-#include "common.h"
+#include "gate_unit.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
@@ -563,29 +563,11 @@ __device__ __forceinline__ void panel_wait() {
   asm volatile("" ::: "memory");
 }
 
-// silu for the epilogues whose result is rounded to bfloat16 at once: the hardware's exp2 and reciprocal (about an
-// ulp of float each) instead of the library's exp and an exact division, a fifth of the instructions; the ends of
-// the range come out right (exp2 = inf gives -0, exp2 = 0 gives g). Of all 65,280 finite bfloat16 gates one comes out a bfloat16
-// step from the rounded 64-bit result, and results below 1e-36 come out as 0 (from -87.5 down; by exact division from -89).
-__device__ __forceinline__ float silu_for_bf16(float g) {
-  return g * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f));
-}
-
 // The end of the fused gate/up products: of one row, a lane with g < 2 holds the gates of four neighbouring outputs
 // n .. n + 3 (n = first + 4 g), the lane 32 further on their ups. The two lanes share the work: the first takes
 // outputs n and n + 1, the second n + 2 and n + 3, each after one exchange of two values.
 // y[n + i] = T(T(silu(gate)) * up), two values in one store where N is even.
-// With `act.limit` > 0 the unit is the clamped one instead: g = min(gate, limit), u = clamp(up, -limit, limit),
-// y = T(g * sigmoid(alpha g) * (u + 1)), from the float accumulators, rounded once.
-// With `act.relu` it is T(max(gate, 0) * up), also from the accumulators and rounded once.
-struct GateAct {
-  float limit = 0.f, alpha = 0.f;
-  int relu = 0;
-};
-__device__ __forceinline__ float clamped_unit(float gate, float up, const GateAct& act) {
-  const float gc = fminf(gate, act.limit), uc = fminf(fmaxf(up, -act.limit), act.limit);
-  return gc * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(gc * act.alpha * -1.4426950408889634f)) * (uc + 1.f);
-}
+// (or the unit that `act` names).
 __device__ __forceinline__ void swiglu_store4(bf16_t* __restrict__ y_row, int first, int N, int g, const f32x4& acc,
                                               bool row_there, GateAct act = {}) {
   const bool second = g >= 2;
@@ -594,13 +576,7 @@ __device__ __forceinline__ void swiglu_store4(bf16_t* __restrict__ y_row, int fi
   const float gate0 = second ? got0 : acc[0], gate1 = second ? got1 : acc[1];
   const float up0 = second ? acc[2] : got0, up1 = second ? acc[3] : got1;
   const int n = first + 4 * (g & 1) + (second ? 2 : 0);
-  const bool clamped = act.limit > 0.f;
-  const bf16_t v0 = act.relu ? float_to_bf16(fmaxf(gate0, 0.f) * up0)
-                    : clamped ? float_to_bf16(clamped_unit(gate0, up0, act))
-                            : float_to_bf16(rounded_as<bf16_t>(silu_for_bf16(rounded_as<bf16_t>(gate0))) * rounded_as<bf16_t>(up0));
-  const bf16_t v1 = act.relu ? float_to_bf16(fmaxf(gate1, 0.f) * up1)
-                    : clamped ? float_to_bf16(clamped_unit(gate1, up1, act))
-                            : float_to_bf16(rounded_as<bf16_t>(silu_for_bf16(rounded_as<bf16_t>(gate1))) * rounded_as<bf16_t>(up1));
+  const bf16_t v0 = gate_unit(gate0, up0, act), v1 = gate_unit(gate1, up1, act);
   if (!row_there || n >= N) return;
   if (N % 2 == 0) {                                        // then n + 1 < N too, and the address is a multiple of 4
     *(uint32_t*)(y_row + n) = (uint32_t)v0.bits | ((uint32_t)v1.bits << 16);
@@ -804,72 +780,6 @@ static int panel_entry(const void* x, int64_t x_stride, const void* w, void* y, 
     case 3: return panel_waves<3>(x, x_stride, w, y, M, N, K, waves, stream, act);
     default: return panel_waves<4>(x, x_stride, w, y, M, N, K, waves, stream, act);
   }
-}
-
-// -------------------------------------------------------------------------------------------- few
-// The fused gate/up product with its activation for at most 16 rows and few outputs (a shared expert's, a small model's),
-// where the panel product has less than half as many workgroups as the chip has compute units and each walks all of K. Here a
-// workgroup takes eight outputs (their gate rows and then their up rows, 16 rows of W, as a wave of the panel product) and
-// its WAVES waves split K in runs of whole blocks of 64, operands straight from memory in the matrix cores' layout, four
-// blocks in flight (lane (c, g) takes the 32 bytes from 16 g on of row c, for both operands alike); the waves' sums meet in
-// LDS and are added in the order 0, 1, .... Bound by its trips to memory. In a captured chain on rotating cold weights, us
-// at 1 / 4 / 16 rows, against the panel product: 512 outputs of K 2,048 4.5 / 4.9 / 5.9 (5.6 / 5.7 / 5.9), 1,024 of 2,048
-// 5.1 / 5.5 / 6.8 (8.3 / 8.4 / 8.7), 2,048 of 2,048 5.9 / 6.2 / 7.2 (8.8 / 8.8 / 9.1), 3,072 of 1,024 5.6 / 5.8 / 7.0 (6.3 /
-// 5.9 / 6.1), 4,096 of 2,048 9.1 / 9.6 / 12.1 (10.7 / 9.3 / 9.6): each workgroup reads the rows of x again, so the more rows
-// and the more workgroups, the less it pays (`gemm_few_glu_ok` in ops.py draws the line).
-template <int WAVES>
-__global__ __launch_bounds__(WAVES * WAVE) void gemm_few_glu_kernel(const bf16_t* __restrict__ x, int64_t x_stride,
-                                                                    const bf16_t* __restrict__ w, bf16_t* __restrict__ y,
-                                                                    int M, int N, int K, GateAct act) {
-  __shared__ f32x4 sums[WAVES][WAVE];
-  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, c = lane % 16, g = lane / 16;
-  const int n0 = blockIdx.x * 8;
-  const int64_t w_row = (c < 8 ? 0 : N) + min(n0 + (c & 7), N - 1);
-  const bf16_t* wp = w + w_row * K + 16 * g;
-  const bf16_t* xp = x + (int64_t)min(c, M - 1) * x_stride + 16 * g;
-  const int per = ((K + 63) / 64 + WAVES - 1) / WAVES * 64;
-  const int k_begin = min(wave * per, K), k_end = min(k_begin + per, K);
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int k0 = k_begin; k0 < k_end; k0 += 256) {
-    bf16x8 wv[8], xv[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {                          // K is a multiple of 8; beyond the run: times zeros
-      const int k = k0 + 64 * (u / 2) + 8 * (u % 2);
-      const bool in = k + 16 * g < k_end;
-      wv[u] = in ? *(const bf16x8*)(wp + k) : zero8g();
-      xv[u] = in ? *(const bf16x8*)(xp + k) : zero8g();
-    }
-    __builtin_amdgcn_sched_barrier(0);                     // every load of the four blocks before the first product
-#pragma unroll
-    for (int u = 0; u < 8; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[u], xv[u], acc, 0, 0, 0);
-  }
-  sums[wave][lane] = acc;
-  __syncthreads();
-  if (wave != 0) return;
-#pragma unroll
-  for (int v = 1; v < WAVES; ++v) acc += sums[v][lane];
-  // acc[i] is row 4g + i of the workgroup's 16 for row c of x
-  swiglu_store4(y + (int64_t)min(c, M - 1) * N, n0, N, g, acc, c < M, act);
-}
-
-// M <= 16, K a multiple of 8, rows at 16-byte addresses; W = [Wg; Wu] of 2N rows; silu, relu, or with limit > 0 the clamped
-// unit, as the panel product's.
-DRYFT_API int dryft_gemm_few_glu_bf16(const void* x, int64_t x_stride, const void* w, void* y, int M, int N, int K, int relu,
-                                      float limit, float alpha, hipStream_t stream) {
-  if (M <= 0 || N <= 0) return 0;
-  if (M > 16 || K < 8 || K % 8 || x_stride % 8 || (((uintptr_t)x | (uintptr_t)w) & 15) || limit < 0.f || (relu && limit > 0.f))
-    return -1;
-  GateAct act;
-  act.relu = relu;
-  act.limit = limit;
-  act.alpha = alpha;
-  const dim3 grid((N + 7) / 8);
-#define FEW(W) hipLaunchKernelGGL((gemm_few_glu_kernel<W>), grid, dim3(W * WAVE), 0, stream, (const bf16_t*)x, x_stride,   \
-                                  (const bf16_t*)w, (bf16_t*)y, M, N, K, act)
-  if (K <= 1024) FEW(4);                                   // so that a wave's run is one trip to memory up to K = 2,048
-  else FEW(8);
-#undef FEW
-  return DRYFT_LAUNCH_CHECK();
 }
 
 // --------------------------------------------------------------------------------------------- mid
@@ -1415,7 +1325,7 @@ __global__ __launch_bounds__(256, 1) void gemm_many_glu_kernel(const bf16_t* __r
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");       // and the last sums may be read
   __builtin_amdgcn_sched_barrier(0);
   // acc[m][n][i] is the gate of output 16 n + 4g + i of the wave's for row 16 m + c, acc[m][n + NT / 2][i] its up
-  const bool clamped = act.limit > 0.f, whole = N % 4 == 0;
+  const bool whole = N % 4 == 0;
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
     const int row = m0 + 16 * (MT * wm + m) + c;
@@ -1428,9 +1338,7 @@ __global__ __launch_bounds__(256, 1) void gemm_many_glu_kernel(const bf16_t* __r
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float gate = acc[m][n][i], up = acc[m][n + NT / 2][i];
-        v[i] = act.relu ? float_to_bf16(fmaxf(gate, 0.f) * up)
-               : clamped ? float_to_bf16(clamped_unit(gate, up, act))
-                         : float_to_bf16(rounded_as<bf16_t>(silu_for_bf16(rounded_as<bf16_t>(gate))) * rounded_as<bf16_t>(up));
+        v[i] = gate_unit(gate, up, act);
       }
       bf16_t* to = y + (int64_t)row * N + o;
       if (whole) {                                         // then o + 3 < N where o < N, and the address is a multiple of 8

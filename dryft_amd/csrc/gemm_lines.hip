@@ -1,0 +1,319 @@
+// Matrix products of at most 16 rows in bfloat16 whose sums are whole when a workgroup ends: y[M,N] = x[M,K] . W[N,K]^T, and the
+// gated units of feed-forwards on top of such products.
+//
+// Decoding steps are chains of launches, each too short to hide the trips to memory at its ends, so this kernel is built to
+// make as few of them as it can and to leave nothing for a launch of its own afterwards:
+//
+//  * A load instruction brings four weight rows, 256 contiguous bytes of each, and its registers are a matrix-core operand
+//    as they are. v_mfma_f32_16x16x32_bf16 takes 16 rows of 32 values; "row" c of the operand is here piece c % 4 of weight
+//    row c / 4 (8 values of every 32), and the rows of x are cut the same way. Of the 16 x 16 products those of equal pieces
+//    count: a quarter of the matrix cores' work, of which there is plenty, buys whole cache lines without a way through LDS.
+//    (Eight pieces of two rows: 1 to 3 % faster at one row, 5 to 15 % slower at four and eight.)
+//  * K is split over the waves of a workgroup (blocks of 128 values in turn, so that together they read on without gaps) and
+//    over nothing else; the waves' sums meet in LDS.
+//  * The end of the kernel may be what a layer does next: the residual sum r <- T(r + y), the rows for the next product,
+//    T(r * w) with the next norm's weight w, and the workgroup's sums of r^2 (`NextNorm`). The next product multiplies its
+//    float sums by rsqrt(mean(r^2) + eps) (`LateNorm`), so that the norm between two products needs no launch: r * w is rounded
+//    once, where the norm's own kernel rounds r / rms(r) and then the product with w.
+//
+// Bound by the weights' bytes and by the two ends of a launch. In a captured chain on rotating cold weights, us at 1 / 4 / 8 rows,
+// against the line-staging kernel with its splits of K: 2,560 x 4,096 5.7 / 5.8 / 6.2 (6.4 / 6.3 / 6.6), 2,560 x 9,728 10.1 / 10.3 /
+// 10.9 (11.4 / 11.5 / 11.8), 6,144 x 2,560 7.3 / 7.3 / 8.0 (8.1 / 8.2 / 8.5), 1,024 x 3,072 3.7 / 3.8 / 4.3 (4.2 / 4.3 / 4.4), 2,048 x
+// 2,048 4.0 / 4.0 / 4.1 (4.5), 8,192 x 2,048 7.5 / 7.5 / 8.5 (9.2 / 9.3 / 9.4), 2,048 x 8,192 8.1 / 8.3 / 8.5 (8.7 / 8.8 / 9.0), 65,536 x
+// 2,048 42 / 42 / 45 (51 / 50 / 51), 151,936 x 2,560 115 / 121 / 132 (126 / 134 / 147). A product, the residual sum and the norm after
+// it, against the line-staging kernel and the norm's launch: 2,560 x 4,096 6.6 / 6.8 / 7.2 (9.6 / 9.7 / 10.2), 2,560 x 9,728 10.9 /
+// 11.0 / 11.8 (15.3 / 15.4 / 15.6), 1,024 x 3,072 4.6 / 4.7 / 5.1 (7.4 / 7.4 / 7.8).
+#include "gate_unit.h"
+#include <type_traits>
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+#define LATE_ROWS 16           // rows that the sums have places for: squares[count][LATE_ROWS]
+#define LATE_MOST 1024         // workgroups that may have left sums
+
+struct LateNorm {
+  const float* squares = nullptr;   // null: the product as it is
+  int count = 0;
+  float eps = 0.f, inverse_width = 0.f;
+};
+
+struct NextNorm {
+  bf16_t* residual = nullptr;       // r, updated in place
+  bf16_t* rows = nullptr;           // T(r * w); null: no norm follows
+  float* squares = nullptr;
+  const void* weight = nullptr;
+  int weight_f32 = 0;
+};
+
+// The sums of squares of a workgroup of WAVES waves: asked for when the object is made, ahead of the product's operands, and
+// added up by `finish`. A group of 16 lanes takes four rows (groups beyond row M none), 16 workgroups' sums at a time.
+template <int WAVES>
+struct LateSums {
+  static constexpr int HELD = WAVES >= 8 ? 2 : 16 / WAVES;    // loads out at once: 256 workgroups' sums
+  f32x4 held[HELD];
+  const LateNorm& late;
+  const bool wanted;
+  __device__ __forceinline__ f32x4 asked(int from, int lane) const {
+    return *(const f32x4*)(late.squares + from * LATE_ROWS + 4 * (lane / 16));
+  }
+  __device__ __forceinline__ LateSums(const LateNorm& l, int M, int wave, int lane)
+      : late(l), wanted(l.squares != nullptr && 4 * (lane / 16) < M) {
+#pragma unroll
+    for (int i = 0; i < HELD; ++i) {
+      const int from = 16 * (wave + WAVES * i) + lane % 16;
+      held[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (wanted && from < late.count) held[i] = asked(from, lane);
+    }
+  }
+  __device__ __forceinline__ void finish(float (*sums)[LATE_ROWS], int wave, int lane) {
+    if (late.squares == nullptr) return;
+    f32x4 s = held[0];
+#pragma unroll
+    for (int i = 1; i < HELD; ++i) s += held[i];
+    if (wanted)
+      for (int from = 16 * (wave + WAVES * HELD) + lane % 16; from < late.count; from += 16 * WAVES) s += asked(from, lane);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s[j] = lanes_sum<16>(s[j]);
+    if (lane % 16 == 0)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) sums[wave][4 * (lane / 16) + j] = s[j];
+  }
+};
+
+template <int WAVES>
+__device__ __forceinline__ float late_scale(const LateNorm& late, const float (*sums)[LATE_ROWS], int row) {
+  float s = 0.f;
+#pragma unroll
+  for (int u = 0; u < WAVES; ++u) s += sums[u][row];
+  return rsqrtf(s * late.inverse_width + late.eps);
+}
+
+__device__ __forceinline__ bf16x8 zero8() {
+  bf16x8 z;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) z[i] = (__bf16)0.f;
+  return z;
+}
+
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void each(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    each<N, I + 1>(f);
+  }
+}
+
+// ROWS weight rows a workgroup (with GLU half of them gate rows and then their up rows), X groups of four rows of x, DEPTH blocks
+// of 128 values of K of a wave on their way at a time
+template <int ROWS, int X, int WAVES, int DEPTH, bool GLU>
+__global__ __launch_bounds__(64 * WAVES) void gemm_lines_kernel(const bf16_t* __restrict__ x, int64_t x_stride,
+                                                                const bf16_t* __restrict__ w, void* __restrict__ y, int y_f32,
+                                                                int M, int N, int K, LateNorm late, NextNorm next, GateAct act) {
+  constexpr int T = (ROWS + 3) / 4, BLOCK = 128, OUT = GLU ? ROWS / 2 : ROWS;
+  __shared__ float sums[WAVES][T][X][4][4], late_sums[WAVES][LATE_ROWS], squares[GLU ? 1 : ROWS][LATE_ROWS];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
+  const int c = lane % 16, g = lane / 16, piece = c % 4;
+  const int n0 = blockIdx.x * OUT;
+  LateSums<WAVES> squared(late, M, wave, lane);
+  const int at = 32 * g + 8 * piece;                       // of this lane within a block
+  const bf16_t* wp[T];
+  const bf16_t* xp[X];
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+    const int row = min(4 * t + c / 4, ROWS - 1);          // past the workgroup's rows and the matrix's: the last one again
+    wp[t] = w + (int64_t)(GLU && row >= OUT ? N + min(n0 + row - OUT, N - 1) : min(n0 + row, N - 1)) * K;
+  }
+#pragma unroll
+  for (int i = 0; i < X; ++i) xp[i] = x + (int64_t)min(4 * i + c / 4, M - 1) * x_stride;
+  f32x4 acc[T][X];
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int i = 0; i < X; ++i) acc[t][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int blocks = (K + BLOCK - 1) / BLOCK, mine = (blocks - wave + WAVES - 1) / WAVES;    // wave, wave + WAVES, ...
+  bf16x8 a[DEPTH][T], b[DEPTH][X];
+  auto fetch = [&](auto slot, int i) {
+    constexpr int d = decltype(slot)::value;
+    int k = (wave + i * WAVES) * BLOCK + at;
+    k = k < K ? k : 0;                                     // beyond K (a multiple of 8): any values, zeros when they are used
+#pragma unroll
+    for (int j = 0; j < X; ++j) b[d][j] = *(const bf16x8*)(xp[j] + k);
+#pragma unroll
+    for (int t = 0; t < T; ++t) a[d][t] = __builtin_nontemporal_load((const bf16x8*)(wp[t] + k));
+  };
+  auto multiply = [&](auto slot, int i) {
+    constexpr int d = decltype(slot)::value;
+    const int k0 = (wave + i * WAVES) * BLOCK;
+    if (k0 + BLOCK > K && k0 + at >= K) {
+#pragma unroll
+      for (int j = 0; j < X; ++j) b[d][j] = zero8();
+#pragma unroll
+      for (int t = 0; t < T; ++t) a[d][t] = zero8();
+    }
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int j = 0; j < X; ++j) acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d][t], b[d][j], acc[t][j], 0, 0, 0);
+  };
+  each<DEPTH>([&](auto d) { if (d.value < mine) fetch(d, d.value); });
+  int i = 0;
+  for (; i + 2 * DEPTH <= mine; i += DEPTH)
+    each<DEPTH>([&](auto d) {
+      multiply(d, i + d.value);
+      fetch(d, i + d.value + DEPTH);
+    });
+  for (; i < mine; i += DEPTH)
+    each<DEPTH>([&](auto d) {
+      if (i + d.value < mine) {
+        multiply(d, i + d.value);
+        if (i + d.value + DEPTH < mine) fetch(d, i + d.value + DEPTH);
+      }
+    });
+  // a lane holds the products of x's row c / 4, piece c % 4, with the four pieces of weight row g: one of them counts, and the
+  // pieces add up over four lanes
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int j = 0; j < X; ++j) {
+      const f32x4 s = acc[t][j];
+      const float low = (piece & 1) ? s[1] : s[0], high = (piece & 1) ? s[3] : s[2];
+      const float one = lanes_sum<4>((piece & 2) ? high : low);
+      if (piece == 0) sums[wave][t][j][g][c / 4] = one;
+    }
+  squared.finish(late_sums, wave, lane);
+  __syncthreads();
+  for (int e = threadIdx.x; e < OUT * LATE_ROWS; e += 64 * WAVES) {
+    const int out = e % OUT, m = e / OUT, n = n0 + out;
+    float r2 = 0.f;
+    if (m < M && m < 4 * X && n < N) {
+      const float scale = late.squares != nullptr ? late_scale<WAVES>(late, late_sums, m) : 1.f;
+      auto whole = [&](int row) {
+        float v = 0.f;
+#pragma unroll
+        for (int u = 0; u < WAVES; ++u) v += sums[u][row / 4][m / 4][row % 4][m % 4];
+        return v * scale;
+      };
+      const float v = whole(out);
+      const int64_t place = (int64_t)m * N + n;
+      if constexpr (GLU) {
+        ((bf16_t*)y)[place] = gate_unit(v, whole(out + OUT), act);
+      } else if (next.rows != nullptr) {
+        const float r = rounded_as<bf16_t>(bf16_to_float(next.residual[place]) + v);
+        next.residual[place] = float_to_bf16(r);
+        next.rows[place] = float_to_bf16(r * load_vector(next.weight, n, next.weight_f32));
+        r2 = r * r;
+      } else if (y_f32) {
+        ((float*)y)[place] = v;
+      } else {
+        ((bf16_t*)y)[place] = float_to_bf16(v);
+      }
+    }
+    if constexpr (!GLU) squares[out][m] = r2;
+  }
+  if constexpr (!GLU) {
+    if (next.rows == nullptr) return;
+    __syncthreads();
+    if (threadIdx.x < LATE_ROWS) {
+      float s = 0.f;
+#pragma unroll
+      for (int u = 0; u < ROWS; ++u) s += squares[u][threadIdx.x];
+      next.squares[(int64_t)blockIdx.x * LATE_ROWS + threadIdx.x] = s;
+    }
+  }
+}
+
+template <int ROWS, int X, int WAVES, bool GLU>
+static int launch_lines(const void* x, int64_t x_stride, const void* w, void* y, int y_f32, int M, int N, int K, LateNorm late,
+                        NextNorm next, GateAct act, hipStream_t stream) {
+  constexpr int T = (ROWS + 3) / 4, OUT = GLU ? ROWS / 2 : ROWS;
+  // registers for the operands on their way: eight waves have 256 a lane, four are to share a compute unit with others
+  constexpr int room = (WAVES == 8 ? 232 : X * T > 8 ? 164 : 124) - 28 - 4 * T * X - 2 * (T + X);
+  constexpr int fit = room / (4 * (T + X));
+  constexpr int DEPTH = fit < 1 ? 1 : fit > 10 ? 10 : fit;
+  hipLaunchKernelGGL((gemm_lines_kernel<ROWS, X, WAVES, DEPTH, GLU>), dim3((N + OUT - 1) / OUT), dim3(64 * WAVES), 0, stream,
+                     (const bf16_t*)x, x_stride, (const bf16_t*)w, y, y_f32, M, N, K, late, next, act);
+  return DRYFT_LAUNCH_CHECK();
+}
+
+template <int ROWS, int WAVES, bool GLU>
+static int lines_by_rows(const void* x, int64_t x_stride, const void* w, void* y, int y_f32, int M, int N, int K, LateNorm late,
+                         NextNorm next, GateAct act, hipStream_t stream) {
+  if (M <= 4) return launch_lines<ROWS, 1, WAVES, GLU>(x, x_stride, w, y, y_f32, M, N, K, late, next, act, stream);
+  if (M <= 8) return launch_lines<ROWS, 2, WAVES, GLU>(x, x_stride, w, y, y_f32, M, N, K, late, next, act, stream);
+  return launch_lines<ROWS, 4, WAVES, GLU>(x, x_stride, w, y, y_f32, M, N, K, late, next, act, stream);
+}
+
+// Rows of a workgroup, and its waves: up to 3,072 outputs the fewest rows that leave every compute unit one workgroup (of eight
+// waves, with registers for ten blocks on their way); 2,560 x 9,728 in 320 workgroups of eight rows instead of 256 of ten: 13.9 against
+// 10.1 us, the units that get two of them work on alone. Beyond, four waves, several workgroups a unit, of as many rows as make
+// their rounds fullest. Each workgroup reads the rows of x again: with more than four of them and a large matrix 20 weight rows
+// share that (151,936 x 2,560 at 8 rows 132 us against 139 with 12; at 4 rows 121 either way; 10,240 x 5,120 at 8 18.9 against 20.4
+// with 10; 5,120 x 8,192 16.8 against 16.6: the line).
+#define LINES_LARGE ((int64_t)40 << 20)
+struct LinesShape {
+  int rows, waves;
+};
+static LinesShape lines_shape(int M, int N, int K) {
+  if (N <= 3072) return {N <= 1024 ? 4 : N <= 2048 ? 8 : N <= 2560 ? 10 : 12, 8};
+  if (M > 4 && (int64_t)N * K >= LINES_LARGE) return {20, 4};
+  int best = 12;
+  int64_t least = INT64_MAX;
+  for (int rows = 12; rows >= 8; rows -= 2) {
+    const int64_t rounds = ((N + rows - 1) / rows + 255) / 256;
+    if (rounds * rows < least) {
+      least = rounds * rows;
+      best = rows;
+    }
+  }
+  return {best, 4};
+}
+
+// How many workgroups the product takes, and so how many rows of sums of squares it leaves.
+DRYFT_API int dryft_gemm_lines_blocks(int M, int N, int K) {
+  const int rows = lines_shape(M, N, K).rows;
+  return (N + rows - 1) / rows;
+}
+
+static bool lines_refuse(const void* x, int64_t x_stride, const void* w, int M, int K, const float* late_squares, int late_count) {
+  return M > LATE_ROWS || K <= 0 || K % 8 || x_stride % 8 || (((uintptr_t)x | (uintptr_t)w) & 15) ||
+         (late_squares != nullptr && (late_count < 1 || late_count > LATE_MOST || ((uintptr_t)late_squares & 15)));
+}
+
+// M <= 16, K a multiple of 8, rows of x and W at 16-byte addresses. y as float (y_f32) or bfloat16, or with `rows` the residual sum,
+// the next product's rows and squares[blocks][16] instead. late_squares: those of the product before, whose width is K.
+DRYFT_API int dryft_gemm_lines_bf16(const void* x, int64_t x_stride, const void* w, void* y, int y_f32, int M, int N, int K,
+                                    const float* late_squares, int late_count, float late_eps, void* residual, void* rows,
+                                    float* squares, const void* weight, int weight_f32, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (lines_refuse(x, x_stride, w, M, K, late_squares, late_count)) return -1;
+  const LateNorm late{late_squares, late_count, late_eps, 1.f / (float)K};
+  const NextNorm next{(bf16_t*)residual, (bf16_t*)rows, squares, weight, weight_f32};
+  const LinesShape shape = lines_shape(M, N, K);
+#define LINES(ROWS, W) case ROWS + 32 * W: return lines_by_rows<ROWS, W, false>(x, x_stride, w, y, y_f32, M, N, K, late, next, {}, stream);
+  switch (shape.rows + 32 * shape.waves) {
+    LINES(4, 8) LINES(8, 8) LINES(10, 8) LINES(12, 8) LINES(8, 4) LINES(10, 4) LINES(12, 4) LINES(20, 4)
+    default: return -1;
+  }
+#undef LINES
+}
+
+// y[M,N] = the gated unit of x . Wg^T and x . Wu^T with W = [Wg; Wu] of 2N rows. Up to 1,024 outputs four a workgroup of eight waves,
+// beyond eight a workgroup of four. Us at 1 / 4 / 8 / 16 rows against the panel product (gemm.hip): 9,728 outputs of K 2,560 17.4 /
+// 17.2 / 18.3 / 21.4 (19.7 / 19.9 / 20.0 / 20.2), 12,288 of 4,096 33.0 / 32.4 / 33.0 / 37.2 (37.7 / 36.2 / 36.4 / 36.5), 8,192 of 2,048
+// 12.2 / 12.4 / 14.0 / 16.4 (12.7 / 12.7 / 12.7 / 12.8), 4,096 of 2,048 7.4 / 7.7 / 8.0 / 9.1 (9.3 / 9.3 / 9.5 / 9.7); 3,072 of 1,024 4.5 / 4.6
+// / 4.9 / 5.7 (6.3 / 5.9 / - / 6.1), and against a kernel that took each operand's rows 32 bytes at a time 1,024 of 2,048 4.0 / 4.1 / 4.2 / 4.7
+// (5.1 / 5.4 / 5.9 / 6.7), 512 of 2,048 3.5 / 3.6 / 3.8 / 4.4 (4.7 / 5.1 / 5.4 / 6.1): `gemm_few_glu_ok` in ops.py draws the line.
+DRYFT_API int dryft_gemm_lines_glu_bf16(const void* x, int64_t x_stride, const void* w, void* y, int M, int N, int K,
+                                        const float* late_squares, int late_count, float late_eps, int relu, float limit, float alpha,
+                                        hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (lines_refuse(x, x_stride, w, M, K, late_squares, late_count) || limit < 0.f || (relu && limit > 0.f)) return -1;
+  const LateNorm late{late_squares, late_count, late_eps, 1.f / (float)K};
+  GateAct act;
+  act.relu = relu;
+  act.limit = limit;
+  act.alpha = alpha;
+  if (N <= 1024) return lines_by_rows<8, 8, true>(x, x_stride, w, y, 0, M, N, K, late, {}, act, stream);
+  return lines_by_rows<16, 4, true>(x, x_stride, w, y, 0, M, N, K, late, {}, act, stream);
+}

@@ -81,10 +81,12 @@ _SIGNATURES = {
                  "dryft_gemm_rows_swiglu_f32": [_P, _L, _P, _P, _I, _I, _I, _P],
                  "dryft_gemm_direct_f32_shape": [_I, _I],
                  "dryft_gemm_direct_f32": [_P, _L, _P, _P, _I, _I, _I, _I, _P]},
+    "gemm_lines": {"dryft_gemm_lines_blocks": [_I, _I, _I],
+                   "dryft_gemm_lines_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _P, _I, _F, _P, _P, _P, _P, _I, _P],
+                   "dryft_gemm_lines_glu_bf16": [_P, _L, _P, _P, _I, _I, _I, _P, _I, _F, _I, _F, _F, _P]},
     "gemm": {"dryft_gemm_tiled": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _P],
              "dryft_gemm_stream_bf16": [_P, _L, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
              "dryft_gemm_many_glu_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _F, _F, _P],
-             "dryft_gemm_few_glu_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _F, _F, _P],
              "dryft_gemm_stream_swiglu_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _P],
              "dryft_gemm_wide_bf16": [_P, _L, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
              "dryft_gemm_panel_swiglu_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _P],
@@ -1011,39 +1013,108 @@ def gemm_wide_bf16(x, w, out, partials=None, group_blocks: int = 2, splits: int 
                                                int(group_blocks), int(depth), int(splits), out_f32, _stream()), "gemm_wide_bf16")
 
 
-def gemm_few_glu_ok(x, w_gate_up) -> bool:
-    """Does the fused gate/up product go to the kernel that splits K over a workgroup's waves? (Figures beside it.) Its
-    workgroups read the rows of x again: up to eight rows where the panel product has fewer than 128 workgroups, up to
-    sixteen where it has at most 64."""
+LINES_ROWS = 16       # the most rows the kernel that loads matrix-core operands as whole lines takes
+
+
+def lines_ok(x, w) -> bool:
+    """Can the kernel that loads matrix-core operands as whole lines take these? At most 16 rows, 16-byte pieces of rows."""
+    return x.shape[0] <= LINES_ROWS and x.shape[1] % 8 == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and \
+        w.data_ptr() % 16 == 0
+
+
+def _lines_operands(who: str, x, w) -> None:
+    _gpu(x, "x", torch.bfloat16)
+    _gpu(w, "w", torch.bfloat16)
+    if not (w.dim() == 2 and w.shape[1] == x.shape[1] and w.is_contiguous() and x.stride(1) == 1):
+        raise KernelError(f"{who}: x [M,K] row-major, w [N,K] contiguous")
+    if not lines_ok(x, w):
+        raise KernelError(f"{who}: needs M <= {LINES_ROWS}, K % 8 == 0 and 16-byte aligned rows, got M={x.shape[0]} K={x.shape[1]}")
+
+
+def _late(who: str, late) -> tuple[int, int, float]:
+    """``late``: None, or ``(squares [count, 16], eps)``."""
+    if late is None:
+        return 0, 0, 0.0
+    squares, eps = late
+    _gpu(squares, "squares", torch.float32)
+    if not (squares.dim() == 2 and squares.shape[1] == LINES_ROWS and squares.is_contiguous() and 1 <= squares.shape[0] <= LATE_MOST):
+        raise KernelError(f"{who}: the sums of squares must be contiguous [1 to {LATE_MOST}, {LINES_ROWS}]")
+    return _ptr(squares), squares.shape[0], float(eps)
+
+
+LATE_MOST = 1024      # workgroups whose sums of squares a product adds up
+
+
+def gemm_lines_bf16(x, w, out, late: tuple | None = None) -> torch.Tensor:
+    """``x [M<=16, K] @ w[N, K].T`` into ``out`` (float32 or bfloat16) by the kernel that loads matrix-core operands as whole
+    lines and splits K over the waves of a workgroup alone. With ``late = (squares, eps)`` row ``m`` of the result is multiplied
+    by ``rsqrt(squares[:, m].sum() / K + eps)``."""
+    _lines_operands("gemm_lines", x, w)
+    _gpu(out, "out")
     m, k = x.shape
-    n = w_gate_up.shape[0] // 2
-    if m > 16 or k % 8 or x.stride(0) % 8 or x.data_ptr() % 16 or w_gate_up.data_ptr() % 16:
+    n = w.shape[0]
+    if not (out.shape == (m, n) and out.is_contiguous() and out.dtype in (torch.float32, torch.bfloat16)):
+        raise KernelError(f"gemm_lines: out must be contiguous [{m},{n}]")
+    _check(_fn("gemm_lines", "dryft_gemm_lines_bf16")(
+        _ptr(x), x.stride(0), _ptr(w), _ptr(out), _float_flag(out, "out"), m, n, k, *_late("gemm_lines", late), 0, 0, 0, 0, 0,
+        _stream()), "gemm_lines_bf16")
+    return out
+
+
+def gemm_lines_blocks(m: int, n: int, k: int) -> int:
+    """How many workgroups ``gemm_lines_bf16`` takes, and so rows of sums of squares ``gemm_lines_next_bf16`` leaves."""
+    return int(_fn("gemm_lines", "dryft_gemm_lines_blocks")(int(m), int(n), int(k)))
+
+
+def gemm_lines_next_bf16(x, w, residual, weight, late: tuple | None = None) -> tuple[torch.Tensor, torch.Tensor]:
+    """The product of ``gemm_lines_bf16`` added to ``residual [M, N]`` (in place, the float sum rounded once), and what the next
+    product reads in the norm's place: ``(rows, squares)`` with ``rows = T(residual * weight)`` and ``squares [count, 16]`` float
+    sums of the residual's squares over each workgroup's columns."""
+    _lines_operands("gemm_lines_next", x, w)
+    m, k = x.shape
+    n = w.shape[0]
+    _gpu(residual, "residual", torch.bfloat16)
+    _gpu(weight, "weight")
+    if not (residual.shape == (m, n) and residual.is_contiguous() and weight.shape == (n,) and weight.is_contiguous()):
+        raise KernelError(f"gemm_lines_next: residual contiguous [{m},{n}], weight [{n}]")
+    rows = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
+    squares = torch.empty((gemm_lines_blocks(m, n, k), LINES_ROWS), dtype=torch.float32, device=x.device)
+    _check(_fn("gemm_lines", "dryft_gemm_lines_bf16")(
+        _ptr(x), x.stride(0), _ptr(w), 0, 0, m, n, k, *_late("gemm_lines_next", late), _ptr(residual), _ptr(rows), _ptr(squares),
+        _ptr(weight), _float_flag(weight, "weight"), _stream()), "gemm_lines_next_bf16")
+    return rows, squares
+
+
+def gemm_few_glu_ok(x, w_gate_up) -> bool:
+    """Does the fused gate/up product go to the kernel that loads matrix-core operands as whole lines? (Figures beside it.) Its
+    workgroups read the rows of x again: up to four rows always, up to eight up to 4,096 outputs and from K = 2,560 on, where
+    the panel product takes several trips to memory a workgroup, up to sixteen up to 4,096 outputs."""
+    if not lines_ok(x, w_gate_up):
         return False
-    workgroups = -(-n // (8 * gemm_panel_waves(n)))
-    return workgroups < 128 if m <= 8 else workgroups <= 64
+    m, k = x.shape
+    return m <= 4 or w_gate_up.shape[0] // 2 <= 4096 or (m <= 8 and k >= 2560)
 
 
-def gemm_few_glu_bf16(x, w_gate_up, out, clamped: tuple[float, float] | None = None, relu: bool = False) -> torch.Tensor:
-    """The fused gate/up product with its activation for at most 16 rows and few outputs; the units are those of
-    ``gemm_panel_swiglu_bf16``. K a multiple of 8."""
+def gemm_few_glu_bf16(x, w_gate_up, out, clamped: tuple[float, float] | None = None, relu: bool = False,
+                      late: tuple | None = None) -> torch.Tensor:
+    """The fused gate/up product with its activation for at most 16 rows; the units are those of
+    ``gemm_panel_swiglu_bf16``, ``late`` as in ``gemm_lines_bf16``. K a multiple of 8."""
     if relu and clamped is not None:
         raise KernelError("gemm_few_glu: relu or the clamped unit, not both")
-    _gpu(x, "x", torch.bfloat16)
-    _gpu(w_gate_up, "w_gate_up", torch.bfloat16)
+    _lines_operands("gemm_few_glu", x, w_gate_up)
     _gpu(out, "out", torch.bfloat16)
     m, k = x.shape
     two_n = w_gate_up.shape[0]
-    if not (two_n % 2 == 0 and w_gate_up.shape == (two_n, k) and w_gate_up.is_contiguous() and x.stride(1) == 1):
-        raise KernelError("gemm_few_glu: x [M,K] row-major, w [2N,K] contiguous")
-    if not (m <= 16 and k % 8 == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w_gate_up.data_ptr() % 16 == 0):
-        raise KernelError(f"gemm_few_glu: needs M <= 16, K % 8 == 0 and 16-byte aligned rows, got M={m} K={k}")
-    if not (out.shape == (m, two_n // 2) and out.is_contiguous() and out.data_ptr() % 4 == 0):
-        raise KernelError(f"gemm_few_glu: out contiguous [{m},{two_n // 2}] at a 4-byte address")
+    if two_n % 2:
+        raise KernelError("gemm_few_glu: w_gate_up must be [2N,K]")
+    if not (out.shape == (m, two_n // 2) and out.is_contiguous()):
+        raise KernelError(f"gemm_few_glu: out contiguous [{m},{two_n // 2}]")
     limit, alpha = clamped if clamped is not None else (0.0, 0.0)
     if clamped is not None and not limit > 0:
         raise KernelError(f"gemm_few_glu: the clamp's limit must be positive, got {limit}")
-    _check(_fn("gemm", "dryft_gemm_few_glu_bf16")(_ptr(x), x.stride(0), _ptr(w_gate_up), _ptr(out), m, two_n // 2, k,
-                                                  int(bool(relu)), float(limit), float(alpha), _stream()), "gemm_few_glu_bf16")
+    _check(_fn("gemm_lines", "dryft_gemm_lines_glu_bf16")(
+        _ptr(x), x.stride(0), _ptr(w_gate_up), _ptr(out), m, two_n // 2, k, *_late("gemm_few_glu", late), int(bool(relu)),
+        float(limit), float(alpha), _stream()), "gemm_few_glu_bf16")
     return out
 
 

@@ -8,9 +8,11 @@ engine/dryft_qwen3/model.py:153, 179-180, 237, 258-261). Here:
   with K split over a workgroup's waves (or plain multiply-adds, ``streams_f32``) for at most 16 rows, operands straight
   into LDS in blocks chosen by the number of workgroups for more (``K`` a multiple of 32; else blocks of
   128 x 128 through registers), and a plain tiled kernel for sizes those do not take;
-* bfloat16, at most 16 rows (decoding at small batch): this library's weight-streaming
+* bfloat16, at most 16 rows (decoding at small batch): this library's kernel whose loads bring whole cache lines that are
+  matrix-core operands as they are, with K split over a workgroup's waves (``lines_pay``), or its weight-streaming
   matrix-core kernel, which stages whole cache lines through LDS and can leave its result
   as float32 partial sums over K for the consumer to add;
+* the gated units of feed-forwards at most 16 rows likewise (``ops.gemm_few_glu_ok``);
 * bfloat16, at most 64 rows, the fused gate/up product with its activation: this library's kernel that brings
   its operands straight into LDS (``panel_swiglu_ok``; K a multiple of 128, else the two kernels below);
 * bfloat16, 33 to 64 rows, where the consumer adds partial sums (q/k/v of decoding steps, the projections back to
@@ -89,6 +91,24 @@ def swiglu_f32_ok(h: torch.Tensor, w_gate_up: torch.Tensor) -> bool:
     rows not from K = 2,560 on: 19,456 x 2,560 at 4 rows 56 us against 43 and 3 for the activation; 6,144 x 1,024 9.9 against
     9.3 and 3."""
     return h.shape[0] <= STREAM_ROWS and ops.rows_f32_ok(h, w_gate_up) and not (h.shape[0] <= 8 and h.shape[1] >= 2560)
+
+
+def lines_pay(m: int, n: int, k: int) -> bool:
+    """Does a product of at most 16 rows go to the kernel that loads matrix-core operands as whole lines (figures beside it), or
+    to the line-staging one? Every workgroup of the first reads the rows of x again, a workgroup of the second more weight rows
+    for them. Up to four rows the first is ahead everywhere, up to eight but for heads of little depth (151,936 x 1,024 at 8 rows
+    62 us against 59). At 16 rows: ahead on matrices that leave either a launch's ends (2,048 x 2,048 4.5 against 5.3 us, 3,072 x
+    2,048 5.4 / 6.1, 4,096 x 1,024 4.8 / 5.0, 1,024 x 3,072 4.8 / 5.1) and on those large enough for its workgroups of 20 weight
+    rows (10,240 x 5,120 21 / 25, 5,120 x 25,600 52 / 59, 65,536 x 2,048 58 / 60, 151,936 x 2,560 165 / 174), behind between them
+    (2,560 x 4,096 7.4 / 7.1, 8,192 x 2,048 10.8 / 10.0) and on 151,936 x 1,024 (72 / 69)."""
+    if m <= 4:
+        return True
+    if k <= 1024 and n > 32768:
+        return False
+    return m <= 8 or n * k <= _LINES_SMALL or n * k >= _LINES_LARGE
+
+
+_LINES_SMALL, _LINES_LARGE = 8 << 20, 40 << 20
 
 
 def wide_plan(n: int, k: int, may_split: bool) -> tuple[int, int, int]:
@@ -263,6 +283,11 @@ def linear(x: torch.Tensor, w: torch.Tensor, *, out_dtype: torch.dtype | None = 
     library_ok = k % 8 == 0 and n % 8 == 0 and x.is_contiguous() and out_dtype == x.dtype
     if m <= STREAM_ROWS and few_ok:
         splits, group, depth = stream_plan(n, k, allow_partials)
+        if lines_pay(m, n, k):
+            # whole sums; where the consumer adds float partial sums it is given one, unrounded
+            if splits > 1:
+                return Partials(ops.gemm_lines_bf16(x, w, torch.empty((1, m, n), dtype=torch.float32, device=x.device)[0])[None], 1)
+            return ops.gemm_lines_bf16(x, w, torch.empty((m, n), dtype=out_dtype, device=x.device))
         if splits > 1:
             partials = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
             ops.gemm_stream_bf16(x, w, None, partials, group, splits, depth)
