@@ -50,7 +50,7 @@ from ..weights.spec import VECTOR
 from . import register_part
 from .base import Mixer, Partials, StepContext, matrix
 from .conv import conv_need, short_conv
-from .linear import linear
+from .linear import linear, linear_for_sum
 from .rope import HalfRotaryPositions, PairRotaryPositions, RotaryPositions
 
 _RESIDENT_WORKGROUPS = 512     # of the split kernel: two per compute unit (its registers allow no more)
@@ -357,10 +357,10 @@ class GQAAttention(Mixer):
                 out = gated
             else:
                 out = ops.sigmoid_gate(out.view(rows, self.o_dim), proj[:, g_col:g_col + self.o_dim], gated)
-            return linear(out, self.w_o, allow_partials=True)
+            return linear_for_sum(out, self.w_o, allow_partials=True)
         if wide:
-            return linear(out.view(rows, H * wide), self.w_o_padded, allow_partials=True)
-        return linear(out.view(rows, self.o_dim), self.w_o, allow_partials=True)
+            return linear_for_sum(out.view(rows, H * wide), self.w_o_padded, allow_partials=True)
+        return linear_for_sum(out.view(rows, self.o_dim), self.w_o, allow_partials=True)
 
     def forward_split(self, h: torch.Tensor, ctx: StepContext, line, writes_cache: bool):
         if self.has_bias:
@@ -394,9 +394,9 @@ class GQAAttention(Mixer):
             rows <= _PROMPT_PARTIAL_ROWS and \
             ops.rows_to_cache_takes(rows, self.head_dim, self.rotary_dim, True)
         if prompt_parts:
-            qkv = linear(h, self.w_qkv, allow_partials=True)
+            qkv = linear_for_sum(h, self.w_qkv, allow_partials=True)
         else:
-            qkv = linear(h, self.w_qkv, allow_partials=fused_decoding, partial_rows=_QKV_PARTIAL_ROWS)
+            qkv = linear_for_sum(h, self.w_qkv, allow_partials=fused_decoding, partial_rows=_QKV_PARTIAL_ROWS)
         window = self.window or 0
         # The tiled prompt kernels never visit the rows of sequences that sit out, and the projection after them reads
         # every row: where the step may hold such sequences the output lives in a tensor that started as zeros, so
@@ -417,7 +417,7 @@ class GQAAttention(Mixer):
                                        ctx.kv_len, ctx.n_seqs, part_o, part_ml, splits, out, self.n_heads, self.n_kv,
                                        self.head_dim, self.scale, window, qkv_parts=parts,
                                        arrivals=split_counters(ctx, self.n_heads, self.n_kv))
-            return linear(out.view(rows, self.q_dim), self.w_o, allow_partials=True)
+            return linear_for_sum(out.view(rows, self.q_dim), self.w_o, allow_partials=True)
         if prompt_parts and isinstance(qkv, Partials):
             q = torch.empty((rows, self.n_heads, self.head_dim), dtype=h.dtype, device=h.device)
             ops.rows_to_cache_from_partials(qkv.data, self.q_norm, self.k_norm, self.qk_norm_eps or 0.0, cos, sin,
@@ -427,7 +427,7 @@ class GQAAttention(Mixer):
             ops.attn_causal_bf16(q, line.k, line.v, line.page_table, ctx.seq_slot, ctx.cu_rows, tile_cu,
                                  ctx.seq_start, ctx.n_seqs, max_tiles, out, self.n_heads, self.n_kv,
                                  self.head_dim, self.scale, window)
-            return linear(out.view(rows, self.q_dim), self.w_o, allow_partials=True)
+            return linear_for_sum(out.view(rows, self.q_dim), self.w_o, allow_partials=True)
         if matrix_cores and not decoding and cos is not None and \
                 ops.attn_causal_takes_projection(self.head_dim, self.rotary_dim):
             # the prompt kernel norms and rotates the queries on their way in: only keys and values go to the cache here
@@ -440,7 +440,7 @@ class GQAAttention(Mixer):
                                            line.page_table, ctx.seq_slot, ctx.cu_rows, tile_cu, ctx.seq_start,
                                            ctx.n_seqs, max_tiles, out, self.n_heads, self.n_kv, self.head_dim,
                                            self.scale, window)
-            return linear(out.view(rows, self.q_dim), self.w_o, allow_partials=True)
+            return linear_for_sum(out.view(rows, self.q_dim), self.w_o, allow_partials=True)
         q = torch.empty((rows, self.n_heads, self.head_dim), dtype=h.dtype, device=h.device)
         ops.qk_norm_rope_kv(qkv, self.q_norm, self.k_norm, self.qk_norm_eps or 0.0, cos, sin, self.rotary_dim,
                             ctx.row_slot, ctx.row_pos, q, line.k, line.v, line.page_table, writes_cache,
@@ -467,7 +467,7 @@ class GQAAttention(Mixer):
         else:
             ops.attn_rows(q, line.k, line.v, line.page_table, ctx.row_slot, ctx.row_pos, out, self.n_heads, self.n_kv,
                           self.head_dim, self.scale, window)
-        return linear(out.view(rows, self.q_dim), self.w_o, allow_partials=True)
+        return linear_for_sum(out.view(rows, self.q_dim), self.w_o, allow_partials=True)
 
     def flops(self, rows, spans):
         """The projections, and both attention products over the keys each row sees."""

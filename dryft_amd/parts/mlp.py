@@ -12,7 +12,7 @@ from ..csrc import ops
 from ..weights.spec import VECTOR
 from . import register_part
 from .base import FeedForward, Partials, matrix
-from .linear import STREAM_ROWS, few_rows_ok, linear, many_glu_ok, panel_swiglu_ok, swiglu_f32_ok, tall_swiglu_ok
+from .linear import STREAM_ROWS, few_rows_ok, linear, linear_for_sum, many_glu_ok, panel_swiglu_ok, swiglu_f32_ok, tall_swiglu_ok
 
 
 class SwiGLU(FeedForward):
@@ -52,7 +52,7 @@ class SwiGLU(FeedForward):
             ops.gemm_rows_swiglu_f32(h, self.w_gate_up, act)
         else:
             ops.silu_mul(linear(h, self.w_gate_up), act)
-        return linear(act, self.w_down, allow_partials=True)
+        return linear_for_sum(act, self.w_down, allow_partials=True)
 
 
 class ReGLU(SwiGLU):
@@ -93,7 +93,7 @@ class ClampedGLU(FeedForward):
             ops.gemm_many_glu_bf16(h, self.w_gate_up, act, clamped=(self.limit, self.alpha))
         else:
             ops.glu_clamped(linear(h, self.w_gate_up), act, self.limit, self.alpha)
-        return linear(act, self.w_down, allow_partials=True)
+        return linear_for_sum(act, self.w_down, allow_partials=True)
 
 
 class SquaredReLU(FeedForward):
@@ -116,7 +116,7 @@ class SquaredReLU(FeedForward):
     def forward(self, h, ctx):
         act = torch.empty((h.shape[0], self.inter), dtype=h.dtype, device=h.device)
         ops.relu_squared(linear(h, self.w_up), act)
-        return linear(act, self.w_down, allow_partials=True)
+        return linear_for_sum(act, self.w_down, allow_partials=True)
 
 
 class PolyNormMLP(FeedForward):
@@ -140,10 +140,10 @@ class PolyNormMLP(FeedForward):
         return ("gemm", "activation")
 
     def forward(self, h, ctx):
-        z = linear(h, self.w_up, allow_partials=True)
+        z = linear_for_sum(h, self.w_up, allow_partials=True)
         act = torch.empty((h.shape[0], self.inter), dtype=h.dtype, device=h.device)
         ops.poly_norm((z.data, z.count) if isinstance(z, Partials) else z, self.act, self.eps, act)
-        return linear(act, self.w_down, allow_partials=True)
+        return linear_for_sum(act, self.w_down, allow_partials=True)
 
 
 register_part("swiglu", SwiGLU)
