@@ -11,82 +11,46 @@
 //    (Eight pieces of two rows: 1 to 3 % faster at one row, 5 to 15 % slower at four and eight.)
 //  * K is split over the waves of a workgroup (blocks of 128 values in turn, so that together they read on without gaps) and
 //    over nothing else; the waves' sums meet in LDS.
-//  * The end of the kernel may be what a layer does next: the residual sum r <- T(r + y), the rows for the next product,
-//    T(r * w) with the next norm's weight w, and the workgroup's sums of r^2 (`NextNorm`). The next product multiplies its
-//    float sums by rsqrt(mean(r^2) + eps) (`LateNorm`), so that the norm between two products needs no launch: r * w is rounded
-//    once, where the norm's own kernel rounds r / rms(r) and then the product with w.
+//  * The end of the kernel may be what a layer does next: the residual sum r <- T(r + y) and each workgroup's sums of r^2
+//    (`Residual`). The next product, given r and those sums (`LateNorm`), takes its rows through the norm on their way to the matrix
+//    cores, T(T(r * rsqrt(mean(r^2) + eps)) * weight) as the norm's own kernel rounds, while its weights are on their way: the norm
+//    between two products needs no launch.
 //
 // Bound by the weights' bytes and by the two ends of a launch. In a captured chain on rotating cold weights, us at 1 / 4 / 8 rows,
 // against the line-staging kernel with its splits of K: 2,560 x 4,096 5.7 / 5.8 / 6.2 (6.4 / 6.3 / 6.6), 2,560 x 9,728 10.1 / 10.3 /
 // 10.9 (11.4 / 11.5 / 11.8), 6,144 x 2,560 7.3 / 7.3 / 8.0 (8.1 / 8.2 / 8.5), 1,024 x 3,072 3.7 / 3.8 / 4.3 (4.2 / 4.3 / 4.4), 2,048 x
 // 2,048 4.0 / 4.0 / 4.1 (4.5), 8,192 x 2,048 7.5 / 7.5 / 8.5 (9.2 / 9.3 / 9.4), 2,048 x 8,192 8.1 / 8.3 / 8.5 (8.7 / 8.8 / 9.0), 65,536 x
-// 2,048 42 / 42 / 45 (51 / 50 / 51), 151,936 x 2,560 115 / 121 / 132 (126 / 134 / 147). A product, the residual sum and the norm after
-// it, against the line-staging kernel and the norm's launch: 2,560 x 4,096 6.6 / 6.8 / 7.2 (9.6 / 9.7 / 10.2), 2,560 x 9,728 10.9 /
-// 11.0 / 11.8 (15.3 / 15.4 / 15.6), 1,024 x 3,072 4.6 / 4.7 / 5.1 (7.4 / 7.4 / 7.8).
+// 2,048 42 / 42 / 45 (51 / 50 / 51), 151,936 x 2,560 115 / 121 / 132 (126 / 134 / 147).
+// The norm on the way, instead of launches of its own (3.4 to 4.6 us and the gap before each, two a layer), whole passes of 96
+// decoding steps through 12 layers of Qwen3-4B: one sequence 79.7 -> 73.5 ms, eight 135.4 -> 131.2 ms; 64 steps of three sequences
+// through Qwen3-0.6B 62.6 -> 56.4 ms.
 #include "gate_unit.h"
 #include <type_traits>
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
-#define LATE_ROWS 16           // rows that the sums have places for: squares[count][LATE_ROWS]
+#define LINES_ROWS 16          // the most rows of x
+#define LATE_ROWS 8            // rows that the sums of squares have places for: squares[count][LATE_ROWS]
 #define LATE_MOST 1024         // workgroups that may have left sums
 
 struct LateNorm {
-  const float* squares = nullptr;   // null: the product as it is
+  const float* squares = nullptr;
   int count = 0;
-  float eps = 0.f, inverse_width = 0.f;
+  float eps = 0.f;
+  const bf16_t* weight = nullptr;
 };
 
-struct NextNorm {
-  bf16_t* residual = nullptr;       // r, updated in place
-  bf16_t* rows = nullptr;           // T(r * w); null: no norm follows
+struct Residual {
+  bf16_t* rows = nullptr;           // r, updated in place; null: the product is stored
   float* squares = nullptr;
-  const void* weight = nullptr;
-  int weight_f32 = 0;
 };
 
-// The sums of squares of a workgroup of WAVES waves: asked for when the object is made, ahead of the product's operands, and
-// added up by `finish`. A group of 16 lanes takes four rows (groups beyond row M none), 16 workgroups' sums at a time.
-template <int WAVES>
-struct LateSums {
-  static constexpr int HELD = WAVES >= 8 ? 2 : 16 / WAVES;    // loads out at once: 256 workgroups' sums
-  f32x4 held[HELD];
-  const LateNorm& late;
-  const bool wanted;
-  __device__ __forceinline__ f32x4 asked(int from, int lane) const {
-    return *(const f32x4*)(late.squares + from * LATE_ROWS + 4 * (lane / 16));
-  }
-  __device__ __forceinline__ LateSums(const LateNorm& l, int M, int wave, int lane)
-      : late(l), wanted(l.squares != nullptr && 4 * (lane / 16) < M) {
+// A fragment of a row through the norm: T(T(r * inverse) * weight), eight values
+__device__ __forceinline__ bf16x8 normed8(bf16x8 r, float inverse, bf16x8 weight) {
 #pragma unroll
-    for (int i = 0; i < HELD; ++i) {
-      const int from = 16 * (wave + WAVES * i) + lane % 16;
-      held[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (wanted && from < late.count) held[i] = asked(from, lane);
-    }
-  }
-  __device__ __forceinline__ void finish(float (*sums)[LATE_ROWS], int wave, int lane) {
-    if (late.squares == nullptr) return;
-    f32x4 s = held[0];
-#pragma unroll
-    for (int i = 1; i < HELD; ++i) s += held[i];
-    if (wanted)
-      for (int from = 16 * (wave + WAVES * HELD) + lane % 16; from < late.count; from += 16 * WAVES) s += asked(from, lane);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) s[j] = lanes_sum<16>(s[j]);
-    if (lane % 16 == 0)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) sums[wave][4 * (lane / 16) + j] = s[j];
-  }
-};
-
-template <int WAVES>
-__device__ __forceinline__ float late_scale(const LateNorm& late, const float (*sums)[LATE_ROWS], int row) {
-  float s = 0.f;
-#pragma unroll
-  for (int u = 0; u < WAVES; ++u) s += sums[u][row];
-  return rsqrtf(s * late.inverse_width + late.eps);
+  for (int i = 0; i < 8; ++i) r[i] = (__bf16)((float)(__bf16)((float)r[i] * inverse) * (float)weight[i]);
+  return r;
 }
 
 __device__ __forceinline__ bf16x8 zero8() {
@@ -106,16 +70,31 @@ __device__ __forceinline__ void each(F&& f) {
 
 // ROWS weight rows a workgroup (with GLU half of them gate rows and then their up rows), X groups of four rows of x, DEPTH blocks
 // of 128 values of K of a wave on their way at a time
-template <int ROWS, int X, int WAVES, int DEPTH, bool GLU>
+template <int ROWS, int X, int WAVES, int DEPTH, bool GLU, bool LATE>
 __global__ __launch_bounds__(64 * WAVES) void gemm_lines_kernel(const bf16_t* __restrict__ x, int64_t x_stride,
                                                                 const bf16_t* __restrict__ w, void* __restrict__ y, int y_f32,
-                                                                int M, int N, int K, LateNorm late, NextNorm next, GateAct act) {
+                                                                int M, int N, int K, LateNorm late, Residual residual, GateAct act) {
   constexpr int T = (ROWS + 3) / 4, BLOCK = 128, OUT = GLU ? ROWS / 2 : ROWS;
-  __shared__ float sums[WAVES][T][X][4][4], late_sums[WAVES][LATE_ROWS], squares[GLU ? 1 : ROWS][LATE_ROWS];
+  __shared__ float sums[WAVES][T][X][4][4], late_sums[LATE ? WAVES : 1][LATE_ROWS], squares[GLU ? 1 : ROWS][LATE_ROWS];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
   const int c = lane % 16, g = lane / 16, piece = c % 4;
   const int n0 = blockIdx.x * OUT;
-  LateSums<WAVES> squared(late, M, wave, lane);
+  f32x4 late_held[X];                                      // sums of squares, asked for ahead of everything
+  if constexpr (LATE) {
+#pragma unroll
+    for (int i = 0; i < X; ++i) {
+      late_held[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int from = threadIdx.x + 64 * WAVES; from < late.count; from += 64 * WAVES)
+        late_held[i] += *(const f32x4*)(late.squares + from * LATE_ROWS + 4 * i);
+    }
+    const int from = min((int)threadIdx.x, late.count - 1);
+#pragma unroll
+    for (int i = 0; i < X; ++i) {
+      const f32x4 one = *(const f32x4*)(late.squares + from * LATE_ROWS + 4 * i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) late_held[i][j] += (int)threadIdx.x < late.count ? one[j] : 0.f;
+    }
+  }
   const int at = 32 * g + 8 * piece;                       // of this lane within a block
   const bf16_t* wp[T];
   const bf16_t* xp[X];
@@ -132,19 +111,25 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_lines_kernel(const bf16_t* __
 #pragma unroll
     for (int i = 0; i < X; ++i) acc[t][i] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int blocks = (K + BLOCK - 1) / BLOCK, mine = (blocks - wave + WAVES - 1) / WAVES;    // wave, wave + WAVES, ...
-  bf16x8 a[DEPTH][T], b[DEPTH][X];
+  bf16x8 a[DEPTH][T], b[DEPTH][X], norm[LATE ? DEPTH : 1];
+  float inverse[X];
   auto fetch = [&](auto slot, int i) {
     constexpr int d = decltype(slot)::value;
     int k = (wave + i * WAVES) * BLOCK + at;
     k = k < K ? k : 0;                                     // beyond K (a multiple of 8): any values, zeros when they are used
 #pragma unroll
     for (int j = 0; j < X; ++j) b[d][j] = *(const bf16x8*)(xp[j] + k);
+    if constexpr (LATE) norm[d] = *(const bf16x8*)(late.weight + k);
 #pragma unroll
     for (int t = 0; t < T; ++t) a[d][t] = __builtin_nontemporal_load((const bf16x8*)(wp[t] + k));
   };
   auto multiply = [&](auto slot, int i) {
     constexpr int d = decltype(slot)::value;
     const int k0 = (wave + i * WAVES) * BLOCK;
+    if constexpr (LATE) {
+#pragma unroll
+      for (int j = 0; j < X; ++j) b[d][j] = normed8(b[d][j], inverse[j], norm[d]);
+    }
     if (k0 + BLOCK > K && k0 + at >= K) {
 #pragma unroll
       for (int j = 0; j < X; ++j) b[d][j] = zero8();
@@ -156,7 +141,28 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_lines_kernel(const bf16_t* __
 #pragma unroll
       for (int j = 0; j < X; ++j) acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d][t], b[d][j], acc[t][j], 0, 0, 0);
   };
-  each<DEPTH>([&](auto d) { if (d.value < mine) fetch(d, d.value); });
+  // ahead of a norm every slot is filled, past the wave's blocks too (with any values): the compiler then knows how many loads lie
+  // behind the sums of squares, and waits for no operand to add those up
+  each<DEPTH>([&](auto d) { if (LATE || d.value < mine) fetch(d, d.value); });
+  if constexpr (LATE) {
+#pragma unroll
+    for (int i = 0; i < X; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float v = lanes_sum<16>(late_held[i][j]);
+        v += __shfl_xor(v, 16, WAVE);
+        v += __shfl_xor(v, 32, WAVE);
+        if (lane == 0) late_sums[wave][4 * i + j] = v;
+      }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < X; ++i) {
+      float v = 0.f;
+#pragma unroll
+      for (int u = 0; u < WAVES; ++u) v += late_sums[u][4 * i + c / 4];
+      inverse[i] = rsqrtf(v / (float)K + late.eps);
+    }
+  }
   int i = 0;
   for (; i + 2 * DEPTH <= mine; i += DEPTH)
     each<DEPTH>([&](auto d) {
@@ -181,67 +187,68 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_lines_kernel(const bf16_t* __
       const float one = lanes_sum<4>((piece & 2) ? high : low);
       if (piece == 0) sums[wave][t][j][g][c / 4] = one;
     }
-  squared.finish(late_sums, wave, lane);
   __syncthreads();
-  for (int e = threadIdx.x; e < OUT * LATE_ROWS; e += 64 * WAVES) {
+  for (int e = threadIdx.x; e < OUT * 4 * X; e += 64 * WAVES) {
     const int out = e % OUT, m = e / OUT, n = n0 + out;
     float r2 = 0.f;
-    if (m < M && m < 4 * X && n < N) {
-      const float scale = late.squares != nullptr ? late_scale<WAVES>(late, late_sums, m) : 1.f;
+    if (m < M && n < N) {
       auto whole = [&](int row) {
         float v = 0.f;
 #pragma unroll
         for (int u = 0; u < WAVES; ++u) v += sums[u][row / 4][m / 4][row % 4][m % 4];
-        return v * scale;
+        return v;
       };
       const float v = whole(out);
       const int64_t place = (int64_t)m * N + n;
       if constexpr (GLU) {
         ((bf16_t*)y)[place] = gate_unit(v, whole(out + OUT), act);
-      } else if (next.rows != nullptr) {
-        const float r = rounded_as<bf16_t>(bf16_to_float(next.residual[place]) + v);
-        next.residual[place] = float_to_bf16(r);
-        next.rows[place] = float_to_bf16(r * load_vector(next.weight, n, next.weight_f32));
-        r2 = r * r;
+      } else if (residual.rows != nullptr) {
+        const bf16_t r = float_to_bf16(bf16_to_float(residual.rows[place]) + v);
+        residual.rows[place] = r;
+        r2 = bf16_to_float(r) * bf16_to_float(r);
       } else if (y_f32) {
         ((float*)y)[place] = v;
       } else {
         ((bf16_t*)y)[place] = float_to_bf16(v);
       }
     }
-    if constexpr (!GLU) squares[out][m] = r2;
+    if constexpr (!GLU && X <= 2) squares[out][m] = r2;
   }
-  if constexpr (!GLU) {
-    if (next.rows == nullptr) return;
+  if constexpr (!GLU && X <= 2) {
+    if (residual.rows == nullptr) return;
     __syncthreads();
-    if (threadIdx.x < LATE_ROWS) {
+    if (threadIdx.x < 4 * X) {
       float s = 0.f;
 #pragma unroll
       for (int u = 0; u < ROWS; ++u) s += squares[u][threadIdx.x];
-      next.squares[(int64_t)blockIdx.x * LATE_ROWS + threadIdx.x] = s;
+      residual.squares[(int64_t)blockIdx.x * LATE_ROWS + threadIdx.x] = s;
     }
   }
 }
 
-template <int ROWS, int X, int WAVES, bool GLU>
+template <int ROWS, int X, int WAVES, bool GLU, bool LATE>
 static int launch_lines(const void* x, int64_t x_stride, const void* w, void* y, int y_f32, int M, int N, int K, LateNorm late,
-                        NextNorm next, GateAct act, hipStream_t stream) {
+                        Residual residual, GateAct act, hipStream_t stream) {
   constexpr int T = (ROWS + 3) / 4, OUT = GLU ? ROWS / 2 : ROWS;
   // registers for the operands on their way: eight waves have 256 a lane, four are to share a compute unit with others
-  constexpr int room = (WAVES == 8 ? 232 : X * T > 8 ? 164 : 124) - 28 - 4 * T * X - 2 * (T + X);
-  constexpr int fit = room / (4 * (T + X));
-  constexpr int DEPTH = fit < 1 ? 1 : fit > 10 ? 10 : fit;
-  hipLaunchKernelGGL((gemm_lines_kernel<ROWS, X, WAVES, DEPTH, GLU>), dim3((N + OUT - 1) / OUT), dim3(64 * WAVES), 0, stream,
-                     (const bf16_t*)x, x_stride, (const bf16_t*)w, y, y_f32, M, N, K, late, next, act);
+  constexpr int room = (WAVES == 8 ? 232 : X * T > 8 || LATE ? 164 : 124) - 28 - 4 * T * X - 2 * (T + X) - (LATE ? 5 * X : 0);
+  constexpr int fit = room / (4 * (T + X + (LATE ? 1 : 0)));
+  constexpr int most = LATE ? 4 : 10, DEPTH = fit < 1 ? 1 : fit > most ? most : fit;
+  hipLaunchKernelGGL((gemm_lines_kernel<ROWS, X, WAVES, DEPTH, GLU, LATE>), dim3((N + OUT - 1) / OUT), dim3(64 * WAVES), 0, stream,
+                     (const bf16_t*)x, x_stride, (const bf16_t*)w, y, y_f32, M, N, K, late, residual, act);
   return DRYFT_LAUNCH_CHECK();
 }
 
 template <int ROWS, int WAVES, bool GLU>
 static int lines_by_rows(const void* x, int64_t x_stride, const void* w, void* y, int y_f32, int M, int N, int K, LateNorm late,
-                         NextNorm next, GateAct act, hipStream_t stream) {
-  if (M <= 4) return launch_lines<ROWS, 1, WAVES, GLU>(x, x_stride, w, y, y_f32, M, N, K, late, next, act, stream);
-  if (M <= 8) return launch_lines<ROWS, 2, WAVES, GLU>(x, x_stride, w, y, y_f32, M, N, K, late, next, act, stream);
-  return launch_lines<ROWS, 4, WAVES, GLU>(x, x_stride, w, y, y_f32, M, N, K, late, next, act, stream);
+                         Residual residual, GateAct act, hipStream_t stream) {
+  if (late.squares != nullptr) {
+    if (M <= 4) return launch_lines<ROWS, 1, WAVES, GLU, true>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
+    return launch_lines<ROWS, 2, WAVES, GLU, true>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
+  }
+  if (M <= 4) return launch_lines<ROWS, 1, WAVES, GLU, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
+  if (M <= 8) return launch_lines<ROWS, 2, WAVES, GLU, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
+  return launch_lines<ROWS, 4, WAVES, GLU, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
 }
 
 // Rows of a workgroup, and its waves: up to 3,072 outputs the fewest rows that leave every compute unit one workgroup (of eight
@@ -275,22 +282,23 @@ DRYFT_API int dryft_gemm_lines_blocks(int M, int N, int K) {
   return (N + rows - 1) / rows;
 }
 
-static bool lines_refuse(const void* x, int64_t x_stride, const void* w, int M, int K, const float* late_squares, int late_count) {
-  return M > LATE_ROWS || K <= 0 || K % 8 || x_stride % 8 || (((uintptr_t)x | (uintptr_t)w) & 15) ||
-         (late_squares != nullptr && (late_count < 1 || late_count > LATE_MOST || ((uintptr_t)late_squares & 15)));
+static bool lines_refuse(const void* x, int64_t x_stride, const void* w, int M, int K, const LateNorm& late) {
+  return M > LINES_ROWS || K <= 0 || K % 8 || x_stride % 8 || (((uintptr_t)x | (uintptr_t)w) & 15) ||
+         (late.squares != nullptr && (M > LATE_ROWS || late.count < 1 || late.count > LATE_MOST || late.weight == nullptr ||
+                                      (((uintptr_t)late.squares | (uintptr_t)late.weight) & 15)));
 }
 
-// M <= 16, K a multiple of 8, rows of x and W at 16-byte addresses. y as float (y_f32) or bfloat16, or with `rows` the residual sum,
-// the next product's rows and squares[blocks][16] instead. late_squares: those of the product before, whose width is K.
+// M <= 16, K a multiple of 8, rows of x and W at 16-byte addresses. y as float (y_f32) or bfloat16, or with `residual` the sum
+// residual[M, N] + y in place and squares[blocks][8] (M <= 8). late_squares: those of the product that left x (M <= 8).
 DRYFT_API int dryft_gemm_lines_bf16(const void* x, int64_t x_stride, const void* w, void* y, int y_f32, int M, int N, int K,
-                                    const float* late_squares, int late_count, float late_eps, void* residual, void* rows,
-                                    float* squares, const void* weight, int weight_f32, hipStream_t stream) {
+                                    const float* late_squares, int late_count, float late_eps, const void* late_weight,
+                                    void* residual_rows, float* squares, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (lines_refuse(x, x_stride, w, M, K, late_squares, late_count)) return -1;
-  const LateNorm late{late_squares, late_count, late_eps, 1.f / (float)K};
-  const NextNorm next{(bf16_t*)residual, (bf16_t*)rows, squares, weight, weight_f32};
+  const LateNorm late{late_squares, late_count, late_eps, (const bf16_t*)late_weight};
+  const Residual residual{(bf16_t*)residual_rows, squares};
+  if (lines_refuse(x, x_stride, w, M, K, late) || (residual_rows != nullptr && (squares == nullptr || M > LATE_ROWS))) return -1;
   const LinesShape shape = lines_shape(M, N, K);
-#define LINES(ROWS, W) case ROWS + 32 * W: return lines_by_rows<ROWS, W, false>(x, x_stride, w, y, y_f32, M, N, K, late, next, {}, stream);
+#define LINES(ROWS, W) case ROWS + 32 * W: return lines_by_rows<ROWS, W, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, {}, stream);
   switch (shape.rows + 32 * shape.waves) {
     LINES(4, 8) LINES(8, 8) LINES(10, 8) LINES(12, 8) LINES(8, 4) LINES(10, 4) LINES(12, 4) LINES(20, 4)
     default: return -1;
@@ -305,11 +313,11 @@ DRYFT_API int dryft_gemm_lines_bf16(const void* x, int64_t x_stride, const void*
 // / 4.9 / 5.7 (6.3 / 5.9 / - / 6.1), and against a kernel that took each operand's rows 32 bytes at a time 1,024 of 2,048 4.0 / 4.1 / 4.2 / 4.7
 // (5.1 / 5.4 / 5.9 / 6.7), 512 of 2,048 3.5 / 3.6 / 3.8 / 4.4 (4.7 / 5.1 / 5.4 / 6.1): `gemm_few_glu_ok` in ops.py draws the line.
 DRYFT_API int dryft_gemm_lines_glu_bf16(const void* x, int64_t x_stride, const void* w, void* y, int M, int N, int K,
-                                        const float* late_squares, int late_count, float late_eps, int relu, float limit, float alpha,
-                                        hipStream_t stream) {
+                                        const float* late_squares, int late_count, float late_eps, const void* late_weight, int relu,
+                                        float limit, float alpha, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (lines_refuse(x, x_stride, w, M, K, late_squares, late_count) || limit < 0.f || (relu && limit > 0.f)) return -1;
-  const LateNorm late{late_squares, late_count, late_eps, 1.f / (float)K};
+  const LateNorm late{late_squares, late_count, late_eps, (const bf16_t*)late_weight};
+  if (lines_refuse(x, x_stride, w, M, K, late) || limit < 0.f || (relu && limit > 0.f)) return -1;
   GateAct act;
   act.relu = relu;
   act.limit = limit;

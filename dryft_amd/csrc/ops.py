@@ -82,8 +82,8 @@ _SIGNATURES = {
                  "dryft_gemm_direct_f32_shape": [_I, _I],
                  "dryft_gemm_direct_f32": [_P, _L, _P, _P, _I, _I, _I, _I, _P]},
     "gemm_lines": {"dryft_gemm_lines_blocks": [_I, _I, _I],
-                   "dryft_gemm_lines_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _P, _I, _F, _P, _P, _P, _P, _I, _P],
-                   "dryft_gemm_lines_glu_bf16": [_P, _L, _P, _P, _I, _I, _I, _P, _I, _F, _I, _F, _F, _P]},
+                   "dryft_gemm_lines_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _P, _I, _F, _P, _P, _P, _P],
+                   "dryft_gemm_lines_glu_bf16": [_P, _L, _P, _P, _I, _I, _I, _P, _I, _F, _P, _I, _F, _F, _P]},
     "gemm": {"dryft_gemm_tiled": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _P],
              "dryft_gemm_stream_bf16": [_P, _L, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
              "dryft_gemm_many_glu_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _F, _F, _P],
@@ -1031,24 +1031,28 @@ def _lines_operands(who: str, x, w) -> None:
         raise KernelError(f"{who}: needs M <= {LINES_ROWS}, K % 8 == 0 and 16-byte aligned rows, got M={x.shape[0]} K={x.shape[1]}")
 
 
-def _late(who: str, late) -> tuple[int, int, float]:
-    """``late``: None, or ``(squares [count, 16], eps)``."""
-    if late is None:
-        return 0, 0, 0.0
-    squares, eps = late
-    _gpu(squares, "squares", torch.float32)
-    if not (squares.dim() == 2 and squares.shape[1] == LINES_ROWS and squares.is_contiguous() and 1 <= squares.shape[0] <= LATE_MOST):
-        raise KernelError(f"{who}: the sums of squares must be contiguous [1 to {LATE_MOST}, {LINES_ROWS}]")
-    return _ptr(squares), squares.shape[0], float(eps)
-
-
+LATE_ROWS = 8         # the most rows of a product that takes its rows through a norm, or leaves their sums of squares
 LATE_MOST = 1024      # workgroups whose sums of squares a product adds up
+
+
+def _late(who: str, late, x) -> tuple:
+    """``late``: None, or ``(squares [count, 8], eps, weight [K])`` of the norm that the rows of ``x`` go through."""
+    if late is None:
+        return 0, 0, 0.0, 0
+    squares, eps, weight = late
+    _gpu(squares, "squares", torch.float32)
+    _gpu(weight, "weight", torch.bfloat16)
+    if not (squares.dim() == 2 and squares.shape[1] == LATE_ROWS and squares.is_contiguous() and 1 <= squares.shape[0] <= LATE_MOST):
+        raise KernelError(f"{who}: the sums of squares must be contiguous [1 to {LATE_MOST}, {LATE_ROWS}]")
+    if not (x.shape[0] <= LATE_ROWS and weight.shape == (x.shape[1],) and weight.is_contiguous() and weight.data_ptr() % 16 == 0):
+        raise KernelError(f"{who}: a norm on the way takes up to {LATE_ROWS} rows and a contiguous weight [{x.shape[1]}]")
+    return _ptr(squares), squares.shape[0], float(eps), _ptr(weight)
 
 
 def gemm_lines_bf16(x, w, out, late: tuple | None = None) -> torch.Tensor:
     """``x [M<=16, K] @ w[N, K].T`` into ``out`` (float32 or bfloat16) by the kernel that loads matrix-core operands as whole
-    lines and splits K over the waves of a workgroup alone. With ``late = (squares, eps)`` row ``m`` of the result is multiplied
-    by ``rsqrt(squares[:, m].sum() / K + eps)``."""
+    lines and splits K over the waves of a workgroup alone. With ``late = (squares, eps, weight)`` the rows of ``x`` go through
+    the norm first: ``T(T(x * rsqrt(squares[:, m].sum() / K + eps)) * weight)``."""
     _lines_operands("gemm_lines", x, w)
     _gpu(out, "out")
     m, k = x.shape
@@ -1056,43 +1060,41 @@ def gemm_lines_bf16(x, w, out, late: tuple | None = None) -> torch.Tensor:
     if not (out.shape == (m, n) and out.is_contiguous() and out.dtype in (torch.float32, torch.bfloat16)):
         raise KernelError(f"gemm_lines: out must be contiguous [{m},{n}]")
     _check(_fn("gemm_lines", "dryft_gemm_lines_bf16")(
-        _ptr(x), x.stride(0), _ptr(w), _ptr(out), _float_flag(out, "out"), m, n, k, *_late("gemm_lines", late), 0, 0, 0, 0, 0,
+        _ptr(x), x.stride(0), _ptr(w), _ptr(out), _float_flag(out, "out"), m, n, k, *_late("gemm_lines", late, x), 0, 0,
         _stream()), "gemm_lines_bf16")
     return out
 
 
 def gemm_lines_blocks(m: int, n: int, k: int) -> int:
-    """How many workgroups ``gemm_lines_bf16`` takes, and so rows of sums of squares ``gemm_lines_next_bf16`` leaves."""
+    """How many workgroups ``gemm_lines_bf16`` takes, and so rows of sums of squares ``gemm_lines_add_bf16`` leaves."""
     return int(_fn("gemm_lines", "dryft_gemm_lines_blocks")(int(m), int(n), int(k)))
 
 
-def gemm_lines_next_bf16(x, w, residual, weight, late: tuple | None = None) -> tuple[torch.Tensor, torch.Tensor]:
-    """The product of ``gemm_lines_bf16`` added to ``residual [M, N]`` (in place, the float sum rounded once), and what the next
-    product reads in the norm's place: ``(rows, squares)`` with ``rows = T(residual * weight)`` and ``squares [count, 16]`` float
-    sums of the residual's squares over each workgroup's columns."""
-    _lines_operands("gemm_lines_next", x, w)
+def gemm_lines_add_bf16(x, w, residual) -> torch.Tensor:
+    """The product of ``gemm_lines_bf16`` of up to 8 rows added to ``residual [M, N]`` (in place, the float sum rounded once);
+    returns what a norm of the sum needs, ``squares [count, 8]``: float sums of its squares over each workgroup's columns."""
+    _lines_operands("gemm_lines_add", x, w)
     m, k = x.shape
     n = w.shape[0]
     _gpu(residual, "residual", torch.bfloat16)
-    _gpu(weight, "weight")
-    if not (residual.shape == (m, n) and residual.is_contiguous() and weight.shape == (n,) and weight.is_contiguous()):
-        raise KernelError(f"gemm_lines_next: residual contiguous [{m},{n}], weight [{n}]")
-    rows = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
-    squares = torch.empty((gemm_lines_blocks(m, n, k), LINES_ROWS), dtype=torch.float32, device=x.device)
+    if not (m <= LATE_ROWS and residual.shape == (m, n) and residual.is_contiguous()):
+        raise KernelError(f"gemm_lines_add: up to {LATE_ROWS} rows, residual contiguous [{m},{n}]")
+    squares = torch.empty((gemm_lines_blocks(m, n, k), LATE_ROWS), dtype=torch.float32, device=x.device)
     _check(_fn("gemm_lines", "dryft_gemm_lines_bf16")(
-        _ptr(x), x.stride(0), _ptr(w), 0, 0, m, n, k, *_late("gemm_lines_next", late), _ptr(residual), _ptr(rows), _ptr(squares),
-        _ptr(weight), _float_flag(weight, "weight"), _stream()), "gemm_lines_next_bf16")
-    return rows, squares
+        _ptr(x), x.stride(0), _ptr(w), 0, 0, m, n, k, 0, 0, 0.0, 0, _ptr(residual), _ptr(squares), _stream()), "gemm_lines_add_bf16")
+    return squares
 
 
-def gemm_few_glu_ok(x, w_gate_up) -> bool:
+def few_glu_pays(m: int, n: int, k: int) -> bool:
     """Does the fused gate/up product go to the kernel that loads matrix-core operands as whole lines? (Figures beside it.) Its
     workgroups read the rows of x again: up to four rows always, up to eight up to 4,096 outputs and from K = 2,560 on, where
     the panel product takes several trips to memory a workgroup, up to sixteen up to 4,096 outputs."""
-    if not lines_ok(x, w_gate_up):
-        return False
-    m, k = x.shape
-    return m <= 4 or w_gate_up.shape[0] // 2 <= 4096 or (m <= 8 and k >= 2560)
+    return m <= LINES_ROWS and k % 8 == 0 and (m <= 4 or n <= 4096 or (m <= 8 and k >= 2560))
+
+
+def gemm_few_glu_ok(x, w_gate_up) -> bool:
+    """``few_glu_pays``, and the operands suit the kernel."""
+    return lines_ok(x, w_gate_up) and few_glu_pays(x.shape[0], w_gate_up.shape[0] // 2, x.shape[1])
 
 
 def gemm_few_glu_bf16(x, w_gate_up, out, clamped: tuple[float, float] | None = None, relu: bool = False,
@@ -1113,7 +1115,7 @@ def gemm_few_glu_bf16(x, w_gate_up, out, clamped: tuple[float, float] | None = N
     if clamped is not None and not limit > 0:
         raise KernelError(f"gemm_few_glu: the clamp's limit must be positive, got {limit}")
     _check(_fn("gemm_lines", "dryft_gemm_lines_glu_bf16")(
-        _ptr(x), x.stride(0), _ptr(w_gate_up), _ptr(out), m, two_n // 2, k, *_late("gemm_few_glu", late), int(bool(relu)),
+        _ptr(x), x.stride(0), _ptr(w_gate_up), _ptr(out), m, two_n // 2, k, *_late("gemm_few_glu", late, x), int(bool(relu)),
         float(limit), float(alpha), _stream()), "gemm_few_glu_bf16")
     return out
 

@@ -12,7 +12,7 @@ import torch
 
 from ..config.plan import ModelPlan
 from ..parts import block_class, build_part
-from ..parts.base import Deferred, Part, Partials, StepContext
+from ..parts.base import Deferred, Part, Partials, Product, StepContext
 from ..weights.spec import TensorSpec
 from ..csrc import ops
 
@@ -157,9 +157,12 @@ class DecoderModel:
         ctx.embedded = x
         pending = None
         for i, run in enumerate(self.plan.schedule):
+            block = self.blocks[run.layer]
+            if isinstance(pending, Product) and (run.enter is not None or not getattr(block, "takes_products", False)):
+                pending = pending.made()
             if run.enter is not None:
                 pending = self.stream_parts[run.enter[0]].enter(pending, run.enter[1], ctx)
-            x, pending = self.blocks[run.layer].forward(x, pending, ctx, cache.line(run.cache_line), run.writes_cache)
+            x, pending = block.forward(x, pending, ctx, cache.line(run.cache_line), run.writes_cache)
             if tap is not None:
                 tap(i, _settled(x, pending))
         if rows is not None:
@@ -168,7 +171,7 @@ class DecoderModel:
             x, pending = _pick_rows(x, rows), _pick_rows(pending, rows)
         if pending is None:
             return self.final_norm.forward(x)
-        _, h = self.final_norm.add_forward(x, pending)
+        _, h = self.final_norm.add_forward(x, pending.made() if isinstance(pending, Product) else pending)
         return h
 
     def logits(self, hidden: torch.Tensor, rows: torch.Tensor | None = None) -> torch.Tensor:
@@ -188,6 +191,8 @@ def _held_tensors(part):
 
 def _settled(x: torch.Tensor, pending) -> torch.Tensor:
     """The residual stream with what is pending added, float32."""
+    if isinstance(pending, Product):
+        pending = pending.made()
     if isinstance(pending, Deferred) or x.dtype == torch.float32 and pending is not None:
         from ..parts.stream import settle
         return settle(x, pending)
@@ -204,6 +209,8 @@ def _pick_rows(x, rows: torch.Tensor):
         return None
     if isinstance(x, Deferred):
         return x.picked(lambda t: _pick_rows(t, rows))
+    if isinstance(x, Product):
+        return Product(_pick_rows(x.x, rows), x.w)
     if isinstance(x, Partials):
         parts = x.data[:x.count]
         picked = torch.empty((x.count, rows.numel(), parts.shape[2]), dtype=parts.dtype, device=parts.device)

@@ -48,9 +48,9 @@ from ..csrc import ops
 from ..limits import MATRIX_CORE_HEAD_STEP, MAX_HEAD_DIM
 from ..weights.spec import VECTOR
 from . import register_part
-from .base import Mixer, Partials, StepContext, matrix
+from .base import LateNormed, Mixer, Partials, Product, StepContext, matrix
 from .conv import conv_need, short_conv
-from .linear import linear, linear_for_sum
+from .linear import lines_pay, linear, linear_for_sum
 from .rope import HalfRotaryPositions, PairRotaryPositions, RotaryPositions
 
 _RESIDENT_WORKGROUPS = 512     # of the split kernel: two per compute unit (its registers allow no more)
@@ -367,16 +367,33 @@ class GQAAttention(Mixer):
             return self._forward_general(h, ctx, line, writes_cache), self.o_bias
         return self.forward(h, ctx, line, writes_cache), None
 
-    def forward(self, h: torch.Tensor, ctx: StepContext, line: KVLine, writes_cache: bool):
-        if self.extended or (self.positions and not isinstance(ctx.positions[self.positions], RotaryPositions)):
+    def _plain(self, ctx: StepContext) -> bool:
+        return not (self.extended or (self.positions and not isinstance(ctx.positions[self.positions], RotaryPositions)))
+
+    def _fused_decoding(self, ctx: StepContext, dtype: torch.dtype) -> bool:
+        return dtype == torch.bfloat16 and self.head_dim % MATRIX_CORE_HEAD_STEP == 0 and ctx.max_q_len == 1 and \
+            self.n_heads // self.n_kv <= 16
+
+    def takes_late(self, rows: int, ctx: StepContext) -> bool:
+        """Decoding steps of few rows whose projection goes to the kernel that can scale its sums."""
+        n, k = self.w_qkv.shape
+        return self._plain(ctx) and self._fused_decoding(ctx, self.w_qkv.dtype) and rows <= ops.LATE_ROWS and k % 8 == 0 and \
+            lines_pay(rows, n, k) and self.w_qkv.data_ptr() % 16 == 0
+
+    def forward(self, h: torch.Tensor, ctx: StepContext, line: KVLine, writes_cache: bool, leave_product: bool = False):
+        """``leave_product``: the output projection may be left unmade (``Product``)."""
+        if not self._plain(ctx):
             out = self._forward_general(h, ctx, line, writes_cache)
             return add_bias(out, self.o_bias, h.dtype) if self.has_bias else out
+        late = None
+        if isinstance(h, LateNormed):
+            h, late = h.rows, h.late
         rows = h.shape[0]
         # bfloat16 on the matrix cores where they take the head size; in float32 on the 32-bit matrix
         # kernels where those do, everything else on the plain one
         matrix_cores = h.dtype == torch.bfloat16 and self.head_dim % MATRIX_CORE_HEAD_STEP == 0
         decoding = matrix_cores and ctx.max_q_len == 1
-        fused_decoding = decoding and self.n_heads // self.n_kv <= 16
+        fused_decoding = self._fused_decoding(ctx, h.dtype)
         # The kernel that norms, rotates, appends and attends in one adds up partial sums of the projection on its way
         # in, so K may be split over workgroups. Measured on Qwen3-4B's sizes, a decoding step with the split against
         # without: 2.980 against 3.008 ms at 8 sequences, 4.63 against 4.74 at 32, 6.75 against 6.86 at 64, 8.92 against
@@ -393,7 +410,9 @@ class GQAAttention(Mixer):
         prompt_parts = matrix_cores and not decoding and writes_cache and cos is not None and \
             rows <= _PROMPT_PARTIAL_ROWS and \
             ops.rows_to_cache_takes(rows, self.head_dim, self.rotary_dim, True)
-        if prompt_parts:
+        if late is not None:
+            qkv = ops.gemm_lines_bf16(h, self.w_qkv, torch.empty((rows, self.w_qkv.shape[0]), dtype=h.dtype, device=h.device), late=late)
+        elif prompt_parts:
             qkv = linear_for_sum(h, self.w_qkv, allow_partials=True)
         else:
             qkv = linear_for_sum(h, self.w_qkv, allow_partials=fused_decoding, partial_rows=_QKV_PARTIAL_ROWS)
@@ -417,7 +436,8 @@ class GQAAttention(Mixer):
                                        ctx.kv_len, ctx.n_seqs, part_o, part_ml, splits, out, self.n_heads, self.n_kv,
                                        self.head_dim, self.scale, window, qkv_parts=parts,
                                        arrivals=split_counters(ctx, self.n_heads, self.n_kv))
-            return linear_for_sum(out.view(rows, self.q_dim), self.w_o, allow_partials=True)
+            out = out.view(rows, self.q_dim)
+            return Product(out, self.w_o) if leave_product else linear_for_sum(out, self.w_o, allow_partials=True)
         if prompt_parts and isinstance(qkv, Partials):
             q = torch.empty((rows, self.n_heads, self.head_dim), dtype=h.dtype, device=h.device)
             ops.rows_to_cache_from_partials(qkv.data, self.q_norm, self.k_norm, self.qk_norm_eps or 0.0, cos, sin,

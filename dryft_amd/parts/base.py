@@ -132,6 +132,34 @@ class Partials:
 
 
 @dataclass
+class Product:
+    """A matrix product ``x @ w.T`` not made yet: for a norm that adds it to the residual stream and can have the product's own
+    kernel do that. ``made`` makes it as the part that left it would have."""
+
+    x: torch.Tensor
+    w: torch.Tensor
+
+    def made(self):
+        from .linear import linear_for_sum
+        return linear_for_sum(self.x, self.w)
+
+
+@dataclass
+class LateNormed:
+    """Rows ahead of a norm, which the product that reads them takes them through: ``squares`` are float sums of their squares
+    (``[count, 8]``), ``weight`` and ``eps`` the norm's."""
+
+    rows: torch.Tensor
+    squares: torch.Tensor
+    eps: float
+    weight: torch.Tensor
+
+    @property
+    def late(self) -> tuple:
+        return self.squares, self.eps, self.weight
+
+
+@dataclass
 class Deferred:
     """What has still to be added to a float32 residual stream before the next norm reads it, so that one kernel
     can do all of it: a branch's output ``delta`` (a tensor or ``Partials``) that is normed with ``norm`` first (None:

@@ -3,13 +3,18 @@
 ``PreNormBlock``: ``x = x + mixer(norm(x))``; ``x = x + ffn(norm(x))`` (reference:
 engine/dryft_qwen3/model.py:151-184). Each residual sum is folded into the norm that
 follows it, so a block receives the previous block's not-yet-added output as
-``pending`` and hands its own feed-forward output on in the same way.
+``pending`` and hands its own feed-forward output on in the same way. Of few rows the
+products at the ends of mixer and feed-forward are handed on unmade: the norm after them
+has the product's kernel add the residual, and the product after the norm takes the rows
+through it (``LateNormed``).
 """
 
 from __future__ import annotations
 
+from inspect import signature
+
 from . import register_block
-from .base import FeedForward, Mixer, Norm
+from .base import FeedForward, Mixer, Norm, Product
 
 
 class PreNormBlock:
@@ -17,18 +22,33 @@ class PreNormBlock:
 
     def __init__(self, mixer_norm: Norm, mixer: Mixer, ffn_norm: Norm, ffn: FeedForward):
         self.mixer_norm, self.mixer, self.ffn_norm, self.ffn = mixer_norm, mixer, ffn_norm, ffn
+        # the parts that know the option (a class of the user's that replaces the call need not)
+        self._leaves = {id(part): "leave_product" in signature(part.forward).parameters for part in (mixer, ffn)}
+        self._folds = {id(norm): "late" in signature(norm.add_forward).parameters for norm in (mixer_norm, ffn_norm)}
 
     def parts(self):
         return {"mixer_norm": self.mixer_norm, "mixer": self.mixer, "ffn_norm": self.ffn_norm, "ffn": self.ffn}
+
+    takes_products = True
 
     def forward(self, x, pending, ctx, line, writes_cache: bool):
         if pending is None:
             h = self.mixer_norm.forward(x)
         else:
-            x, h = self.mixer_norm.add_forward(x, pending)
-        mixed = self.mixer.forward(h, ctx, line, writes_cache)
-        x, h = self.ffn_norm.add_forward(x, mixed)
-        return x, self.ffn.forward(h, ctx)
+            x, h = self._added(self.mixer_norm, x, pending, self.mixer, ctx)
+        mixed = self.mixer.forward(h, ctx, line, writes_cache, **self._left(self.mixer))
+        x, h = self._added(self.ffn_norm, x, mixed, self.ffn, ctx)
+        return x, self.ffn.forward(h, ctx, **self._left(self.ffn))
+
+    def _left(self, part) -> dict:
+        return {"leave_product": True} if self._leaves[id(part)] else {}
+
+    def _added(self, norm: Norm, x, delta, reader, ctx):
+        if not isinstance(delta, Product):
+            return norm.add_forward(x, delta)
+        if not self._folds[id(norm)]:
+            return norm.add_forward(x, delta.made())
+        return norm.add_forward(x, delta, late=self._leaves[id(reader)] and reader.takes_late(x.shape[0], ctx))
 
 
 register_block("prenorm", PreNormBlock)

@@ -11,7 +11,7 @@ import torch
 from ..csrc import ops
 from ..weights.spec import VECTOR
 from . import register_part
-from .base import FeedForward, Partials, matrix
+from .base import FeedForward, LateNormed, Partials, Product, matrix
 from .linear import STREAM_ROWS, few_rows_ok, linear, linear_for_sum, many_glu_ok, panel_swiglu_ok, swiglu_f32_ok, tall_swiglu_ok
 
 
@@ -34,10 +34,16 @@ class SwiGLU(FeedForward):
     def kernel_modules(self, dtype):
         return ("gemm", "activation")
 
-    def forward(self, h, ctx):
+    def takes_late(self, rows: int, ctx) -> bool:
+        return rows <= ops.LATE_ROWS and ops.few_glu_pays(rows, self.inter, self.hidden) and self.w_gate_up.data_ptr() % 16 == 0
+
+    def forward(self, h, ctx, leave_product: bool = False):
+        late = None
+        if isinstance(h, LateNormed):
+            h, late = h.rows, h.late
         act = torch.empty((h.shape[0], self.inter), dtype=h.dtype, device=h.device)
         if h.dtype == torch.bfloat16 and ops.gemm_few_glu_ok(h, self.w_gate_up):
-            ops.gemm_few_glu_bf16(h, self.w_gate_up, act, relu=self.relu)             # few rows and outputs, in one kernel
+            ops.gemm_few_glu_bf16(h, self.w_gate_up, act, relu=self.relu, late=late)  # few rows, in one kernel
         elif h.dtype == torch.bfloat16 and panel_swiglu_ok(h, self.w_gate_up):
             ops.gemm_panel_swiglu_bf16(h, self.w_gate_up, act, relu=self.relu)        # product and activation in one kernel
         elif h.dtype == torch.bfloat16 and tall_swiglu_ok(h, self.w_gate_up):
@@ -52,7 +58,7 @@ class SwiGLU(FeedForward):
             ops.gemm_rows_swiglu_f32(h, self.w_gate_up, act)
         else:
             ops.silu_mul(linear(h, self.w_gate_up), act)
-        return linear_for_sum(act, self.w_down, allow_partials=True)
+        return Product(act, self.w_down) if leave_product else linear_for_sum(act, self.w_down, allow_partials=True)
 
 
 class ReGLU(SwiGLU):
