@@ -147,28 +147,36 @@ class DecoderModel:
     def forward(self, tokens: torch.Tensor, ctx: StepContext, cache, rows: torch.Tensor | None = None,
                 tap=None) -> torch.Tensor:
         """Hidden states after the final norm, ``[rows, hidden]``: of every row of the step, or of ``rows`` alone
-        (int32 indices into the step's rows, on the device), which are picked before the final norm so that it runs
-        over nothing else. ``tap(i, stream)``, when given, is called after run ``i`` of the schedule with the residual
+        (int32 indices into the step's rows, on the device), which are picked behind the last mixer where its block can
+        go on with them, else before the final norm. ``tap(i, stream)``, when given, is called after run ``i`` of the schedule with the residual
         stream as that run leaves it (float32, everything pending added): a way to look, not part of the step."""
         ctx.positions = self.positions
         ctx.tokens = tokens
         ctx.shared.clear()
         x = self.embedding.forward(tokens)
         ctx.embedded = x
-        pending = None
+        pending, picked = None, False
+        last = len(self.plan.schedule) - 1 if rows is not None and 0 < rows.numel() < tokens.numel() and tap is None else None
         for i, run in enumerate(self.plan.schedule):
             block = self.blocks[run.layer]
             if isinstance(pending, Product) and (run.enter is not None or not getattr(block, "takes_products", False)):
                 pending = pending.made()
             if run.enter is not None:
                 pending = self.stream_parts[run.enter[0]].enter(pending, run.enter[1], ctx)
-            x, pending = block.forward(x, pending, ctx, cache.line(run.cache_line), run.writes_cache)
+            more = {}
+            if last is not None and i == last and getattr(block, "picks_rows", False):
+                # nobody reads the other rows behind the last mixer: nor does its feed-forward need them (prompts
+                # through 12 layers of Qwen3-4B: 2,048 tokens 6.67 -> 6.29 ms, 12,800 in six prompts 30.5 -> 28.9)
+                more["pick"] = lambda t: _pick_rows(t, rows)
+                picked = True
+            x, pending = block.forward(x, pending, ctx, cache.line(run.cache_line), run.writes_cache, **more)
             if tap is not None:
                 tap(i, _settled(x, pending))
         if rows is not None:
             if rows.numel() == 0:                              # nothing is wanted: the layers have run, that is all
                 return x[:0]
-            x, pending = _pick_rows(x, rows), _pick_rows(pending, rows)
+            if not picked:
+                x, pending = _pick_rows(x, rows), _pick_rows(pending, rows)
         if pending is None:
             return self.final_norm.forward(x)
         _, h = self.final_norm.add_forward(x, pending.made() if isinstance(pending, Product) else pending)

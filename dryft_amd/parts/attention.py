@@ -436,8 +436,7 @@ class GQAAttention(Mixer):
                                        ctx.kv_len, ctx.n_seqs, part_o, part_ml, splits, out, self.n_heads, self.n_kv,
                                        self.head_dim, self.scale, window, qkv_parts=parts,
                                        arrivals=split_counters(ctx, self.n_heads, self.n_kv))
-            out = out.view(rows, self.q_dim)
-            return Product(out, self.w_o) if leave_product else linear_for_sum(out, self.w_o, allow_partials=True)
+            return self._projected(out, rows, leave_product)
         if prompt_parts and isinstance(qkv, Partials):
             q = torch.empty((rows, self.n_heads, self.head_dim), dtype=h.dtype, device=h.device)
             ops.rows_to_cache_from_partials(qkv.data, self.q_norm, self.k_norm, self.qk_norm_eps or 0.0, cos, sin,
@@ -447,7 +446,7 @@ class GQAAttention(Mixer):
             ops.attn_causal_bf16(q, line.k, line.v, line.page_table, ctx.seq_slot, ctx.cu_rows, tile_cu,
                                  ctx.seq_start, ctx.n_seqs, max_tiles, out, self.n_heads, self.n_kv,
                                  self.head_dim, self.scale, window)
-            return linear_for_sum(out.view(rows, self.q_dim), self.w_o, allow_partials=True)
+            return self._projected(out, rows, leave_product)
         if matrix_cores and not decoding and cos is not None and \
                 ops.attn_causal_takes_projection(self.head_dim, self.rotary_dim):
             # the prompt kernel norms and rotates the queries on their way in: only keys and values go to the cache here
@@ -460,7 +459,7 @@ class GQAAttention(Mixer):
                                            line.page_table, ctx.seq_slot, ctx.cu_rows, tile_cu, ctx.seq_start,
                                            ctx.n_seqs, max_tiles, out, self.n_heads, self.n_kv, self.head_dim,
                                            self.scale, window)
-            return linear_for_sum(out.view(rows, self.q_dim), self.w_o, allow_partials=True)
+            return self._projected(out, rows, leave_product)
         q = torch.empty((rows, self.n_heads, self.head_dim), dtype=h.dtype, device=h.device)
         ops.qk_norm_rope_kv(qkv, self.q_norm, self.k_norm, self.qk_norm_eps or 0.0, cos, sin, self.rotary_dim,
                             ctx.row_slot, ctx.row_pos, q, line.k, line.v, line.page_table, writes_cache,
@@ -487,7 +486,11 @@ class GQAAttention(Mixer):
         else:
             ops.attn_rows(q, line.k, line.v, line.page_table, ctx.row_slot, ctx.row_pos, out, self.n_heads, self.n_kv,
                           self.head_dim, self.scale, window)
-        return linear_for_sum(out.view(rows, self.q_dim), self.w_o, allow_partials=True)
+        return self._projected(out, rows, leave_product)
+
+    def _projected(self, out: torch.Tensor, rows: int, leave_product: bool):
+        out = out.view(rows, self.q_dim)
+        return Product(out, self.w_o) if leave_product else linear_for_sum(out, self.w_o, allow_partials=True)
 
     def flops(self, rows, spans):
         """The projections, and both attention products over the keys each row sees."""

@@ -237,6 +237,8 @@ class Mixer(Part):
 
 
 class FeedForward(Part):
+    row_wise = False    # does a row's output depend on that row of ``h`` alone, and on nothing that ``ctx`` says of the rows?
+
     def forward(self, h: torch.Tensor, ctx: StepContext):
         raise NotImplementedError
 

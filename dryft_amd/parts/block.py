@@ -31,12 +31,19 @@ class PreNormBlock:
 
     takes_products = True
 
-    def forward(self, x, pending, ctx, line, writes_cache: bool):
+    @property
+    def picks_rows(self) -> bool:
+        """Can the block go on from its mixer with a choice of its rows (``pick`` gathers them)?"""
+        return self.ffn.row_wise
+
+    def forward(self, x, pending, ctx, line, writes_cache: bool, pick=None):
         if pending is None:
             h = self.mixer_norm.forward(x)
         else:
             x, h = self._added(self.mixer_norm, x, pending, self.mixer, ctx)
         mixed = self.mixer.forward(h, ctx, line, writes_cache, **self._left(self.mixer))
+        if pick is not None:
+            x, mixed = pick(x), pick(mixed)
         x, h = self._added(self.ffn_norm, x, mixed, self.ffn, ctx)
         return x, self.ffn.forward(h, ctx, **self._left(self.ffn))
 

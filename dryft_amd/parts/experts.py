@@ -124,6 +124,10 @@ class RoutedExperts(FeedForward):
     def kernel_modules(self, dtype):
         return ("gemm", "activation", "moe")
 
+    @property
+    def row_wise(self) -> bool:
+        return self.router != "table"                                  # a table is read by the rows' tokens
+
     def forward(self, h, ctx):
         rows, E, top = h.shape[0], self.n_experts, self.top
         dev = h.device

@@ -101,11 +101,18 @@ class HyperBlock:
     def parts(self):
         return {role: getattr(self, role) for role in self.roles}
 
-    def forward(self, x, pending, ctx: StepContext, line, writes_cache: bool):
+    @property
+    def picks_rows(self) -> bool:
+        """Can the block go on from its mixer with a choice of its rows (``pick`` gathers them)?"""
+        return self.ffn is not None and self.ffn.row_wise
+
+    def forward(self, x, pending, ctx: StepContext, line, writes_cache: bool, pick=None):
         x, h = read_streams(x, as_deferred(pending), self.mixer_route, self.mixer_norm, ctx.dtype)
         pending = Deferred(delta=self.mixer.forward(h, ctx, line, writes_cache), route=self.mixer_route)
         if self.ffn is None:
             return x, pending
+        if pick is not None:
+            x, pending = pick(x), pick(pending)
         x, h = read_streams(x, pending, self.ffn_route, self.ffn_norm, ctx.dtype)
         return x, Deferred(delta=self.ffn.forward(h, ctx), route=self.ffn_route)
 

@@ -17,6 +17,7 @@ from .linear import STREAM_ROWS, few_rows_ok, linear, linear_for_sum, many_glu_o
 
 class SwiGLU(FeedForward):
     relu = False              # relu in the place of silu (``ReGLU``)
+    row_wise = True
 
     def __init__(self, hidden_size: int, intermediate_size: int):
         self.hidden, self.inter = int(hidden_size), int(intermediate_size)
@@ -71,6 +72,8 @@ class ClampedGLU(FeedForward):
     """``down( g * sigmoid(alpha * g) * (u + 1) )`` with ``g = min(gate(h), limit)`` and
     ``u = clamp(up(h), -limit, limit)``, dense, no bias. Gate and up are one product, as above."""
 
+    row_wise = True
+
     def __init__(self, hidden_size: int, intermediate_size: int, limit: float, alpha: float = 1.702):
         self.hidden, self.inter = int(hidden_size), int(intermediate_size)
         self.limit, self.alpha = float(limit), float(alpha)
@@ -105,6 +108,8 @@ class ClampedGLU(FeedForward):
 class SquaredReLU(FeedForward):
     """``down( relu(up(h))^2 )``, dense, no gate, no bias."""
 
+    row_wise = True
+
     def __init__(self, hidden_size: int, intermediate_size: int):
         self.hidden, self.inter = int(hidden_size), int(intermediate_size)
         self.w_up: torch.Tensor | None = None
@@ -129,6 +134,8 @@ class PolyNormMLP(FeedForward):
     """``down( c0 N(z) + c1 N(z^2) + c2 N(z^3) + c3 )`` with ``z = up(h)``, powers element by element and ``N`` the division
     of a token's vector by its root mean square (``eps`` inside the root); dense, no bias. Tensor ``act`` holds the four
     numbers. ``z`` reaches the polynomial as the float partial sums of its product where that is split over K."""
+
+    row_wise = True
 
     def __init__(self, hidden_size: int, intermediate_size: int, eps: float):
         self.hidden, self.inter, self.eps = int(hidden_size), int(intermediate_size), float(eps)

@@ -174,12 +174,19 @@ class SandwichBlock:
     def parts(self):
         return {role: getattr(self, role) for role in self.roles}
 
-    def forward(self, x, pending, ctx: StepContext, line, writes_cache: bool):
+    @property
+    def picks_rows(self) -> bool:
+        """Can the block go on from its mixer with a choice of its rows (``pick`` gathers them)?"""
+        return self.ffn is not None and self.ffn.row_wise
+
+    def forward(self, x, pending, ctx: StepContext, line, writes_cache: bool, pick=None):
         # the embedding's output starts the stream and is read again later: it is never updated in place
         x, h = self.mixer_norm.add_forward(x, pending, ctx.dtype, in_place=x is not ctx.embedded)
         pending = Deferred(delta=self.mixer.forward(h, ctx, line, writes_cache), norm=self.mixer_post_norm)
         if self.ffn is None:
             return x, pending
+        if pick is not None:
+            x, pending = pick(x), pick(pending)
         x, h = self.ffn_norm.add_forward(x, pending, ctx.dtype)
         return x, Deferred(delta=self.ffn.forward(h, ctx), norm=self.ffn_post_norm)
 
@@ -202,11 +209,18 @@ class PostNormBlock:
     def parts(self):
         return {role: getattr(self, role) for role in self.roles}
 
-    def forward(self, x, pending, ctx: StepContext, line, writes_cache: bool):
+    @property
+    def picks_rows(self) -> bool:
+        """Can the block go on from its mixer with a choice of its rows (``pick`` gathers them)?"""
+        return self.ffn is not None and self.ffn.row_wise
+
+    def forward(self, x, pending, ctx: StepContext, line, writes_cache: bool, pick=None):
         x, h = read_plain(x, pending, ctx.dtype)
         pending = Deferred(delta=self.mixer.forward(h, ctx, line, writes_cache), norm=self.mixer_post_norm)
         if self.ffn is None:
             return x, pending
+        if pick is not None:
+            x, pending = pick(x), pick(pending)
         x, h = read_plain(x, pending, ctx.dtype)
         return x, Deferred(delta=self.ffn.forward(h, ctx), norm=self.ffn_post_norm)
 
@@ -266,12 +280,19 @@ class PreNormBlock:
     def parts(self):
         return {role: getattr(self, role) for role in self.roles}
 
-    def forward(self, x, pending, ctx: StepContext, line, writes_cache: bool):
+    @property
+    def picks_rows(self) -> bool:
+        """Can the block go on from its mixer with a choice of its rows (``pick`` gathers them)?"""
+        return self.ffn is not None and self.ffn.row_wise and self.side is None
+
+    def forward(self, x, pending, ctx: StepContext, line, writes_cache: bool, pick=None):
         # the embedding's output starts the stream and other parts may read it again: never updated in place
         x, h = self.mixer_norm.add_forward(x, pending, ctx.dtype, in_place=x is not ctx.embedded)
         delta, bias = self.mixer.forward_split(h, ctx, line, writes_cache)
         pending = Deferred(delta=delta, vector=bias)
         if self.ffn is not None:
+            if pick is not None:
+                x, pending = pick(x), pick(pending)
             x, h = self.ffn_norm.add_forward(x, pending, ctx.dtype)
             pending = Deferred(delta=self.ffn.forward(h, ctx))
         if self.side is not None:
