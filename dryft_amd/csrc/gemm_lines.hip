@@ -1,4 +1,4 @@
-// Matrix products of at most 16 rows in bfloat16 whose sums are whole when a workgroup ends: y[M,N] = x[M,K] . W[N,K]^T, and the
+// Matrix products of at most 16 rows in bfloat16, 4 in float32, whose sums are whole when a workgroup ends: y[M,N] = x[M,K] . W[N,K]^T, and the
 // gated units of feed-forwards on top of such products.
 //
 // Decoding steps are chains of launches, each too short to hide the trips to memory at its ends, so this kernel is built to
@@ -30,35 +30,70 @@
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
-#define LINES_ROWS 16          // the most rows of x
+#define LINES_ROWS 16          // the most rows of x, in bfloat16
+#define LINES_ROWS_F32 4       // and in float32
 #define LATE_ROWS 8            // rows that the sums of squares have places for: squares[count][LATE_ROWS]
 #define LATE_MOST 1024         // workgroups that may have left sums
 
+template <typename E>
 struct LateNorm {
   const float* squares = nullptr;
   int count = 0;
   float eps = 0.f;
-  const bf16_t* weight = nullptr;
+  const E* weight = nullptr;
 };
 
+template <typename E>
 struct Residual {
-  bf16_t* rows = nullptr;           // r, updated in place; null: the product is stored
+  E* rows = nullptr;                // r, updated in place; null: the product is stored
   float* squares = nullptr;
 };
 
-// A fragment of a row through the norm: T(T(r * inverse) * weight), eight values
-__device__ __forceinline__ bf16x8 normed8(bf16x8 r, float inverse, bf16x8 weight) {
+// Sixteen bytes of a row are an operand of one matrix instruction of 32 values in bfloat16, or a value for each of four
+// instructions of four values in float32 (32-bit factors and sums).
+template <typename E>
+struct Fragment;
+template <>
+struct Fragment<bf16_t> {
+  typedef bf16x8 type;
+  static constexpr int VALUES = 8;
+  static constexpr int SUMS = 1;
+  static __device__ __forceinline__ void multiply(bf16x8 a, bf16x8 b, f32x4 (&acc)[SUMS]) {
+    acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[0], 0, 0, 0);
+  }
+  static __device__ __forceinline__ f32x4 sum(const f32x4 (&acc)[SUMS]) { return acc[0]; }
+  static __device__ __forceinline__ bf16x8 zero() {
+    bf16x8 z;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) r[i] = (__bf16)((float)(__bf16)((float)r[i] * inverse) * (float)weight[i]);
-  return r;
-}
-
-__device__ __forceinline__ bf16x8 zero8() {
-  bf16x8 z;
+    for (int i = 0; i < 8; ++i) z[i] = (__bf16)0.f;
+    return z;
+  }
+  // a fragment of a row through the norm: T(T(r * inverse) * weight)
+  static __device__ __forceinline__ bf16x8 normed(bf16x8 r, float inverse, bf16x8 weight) {
 #pragma unroll
-  for (int i = 0; i < 8; ++i) z[i] = (__bf16)0.f;
-  return z;
-}
+    for (int i = 0; i < 8; ++i) r[i] = (__bf16)((float)(__bf16)((float)r[i] * inverse) * (float)weight[i]);
+    return r;
+  }
+};
+template <>
+struct Fragment<float> {
+  typedef f32x4 type;
+  static constexpr int VALUES = 4;
+  // a sum for each of the four: no instruction waits for the one before, and sums a quarter as long are rounded less (against 64
+  // bits, relative to the result's norm, K = 1,024: 1.0e-7 instead of 1.6e-7; 9,728: 1.8e-7 instead of 3.3e-7)
+  static constexpr int SUMS = 4;
+  static __device__ __forceinline__ void multiply(f32x4 a, f32x4 b, f32x4 (&acc)[SUMS]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], acc[i], 0, 0, 0);
+  }
+  static __device__ __forceinline__ f32x4 sum(const f32x4 (&acc)[SUMS]) { return (acc[0] + acc[1]) + (acc[2] + acc[3]); }
+  static __device__ __forceinline__ f32x4 zero() { return f32x4{0.f, 0.f, 0.f, 0.f}; }
+  static __device__ __forceinline__ f32x4 normed(f32x4 r, float inverse, f32x4 weight) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = r[i] * inverse * weight[i];
+    return r;
+  }
+};
 
 template <int N, int I = 0, typename F>
 __device__ __forceinline__ void each(F&& f) {
@@ -69,12 +104,15 @@ __device__ __forceinline__ void each(F&& f) {
 }
 
 // ROWS weight rows a workgroup (with GLU half of them gate rows and then their up rows), X groups of four rows of x, DEPTH blocks
-// of 128 values of K of a wave on their way at a time
-template <int ROWS, int X, int WAVES, int DEPTH, bool GLU, bool LATE>
-__global__ __launch_bounds__(64 * WAVES) void gemm_lines_kernel(const bf16_t* __restrict__ x, int64_t x_stride,
-                                                                const bf16_t* __restrict__ w, void* __restrict__ y, int y_f32,
-                                                                int M, int N, int K, LateNorm late, Residual residual, GateAct act) {
-  constexpr int T = (ROWS + 3) / 4, BLOCK = 128, OUT = GLU ? ROWS / 2 : ROWS;
+// of 256 bytes of K of a wave on their way at a time
+template <typename E, int ROWS, int X, int WAVES, int DEPTH, bool GLU, bool LATE>
+__global__ __launch_bounds__(64 * WAVES) void gemm_lines_kernel(const E* __restrict__ x, int64_t x_stride,
+                                                                const E* __restrict__ w, void* __restrict__ y, int y_f32,
+                                                                int M, int N, int K, LateNorm<E> late, Residual<E> residual,
+                                                                GateAct act) {
+  typedef Fragment<E> F;
+  typedef typename F::type frag;
+  constexpr int T = (ROWS + 3) / 4, BLOCK = 16 * F::VALUES, OUT = GLU ? ROWS / 2 : ROWS;
   __shared__ float sums[WAVES][T][X][4][4], late_sums[LATE ? WAVES : 1][LATE_ROWS], squares[GLU ? 1 : ROWS][LATE_ROWS];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
   const int c = lane % 16, g = lane / 16, piece = c % 4;
@@ -95,9 +133,9 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_lines_kernel(const bf16_t* __
       for (int j = 0; j < 4; ++j) late_held[i][j] += (int)threadIdx.x < late.count ? one[j] : 0.f;
     }
   }
-  const int at = 32 * g + 8 * piece;                       // of this lane within a block
-  const bf16_t* wp[T];
-  const bf16_t* xp[X];
+  const int at = F::VALUES * (4 * g + piece);                       // of this lane within a block
+  const E* wp[T];
+  const E* xp[X];
 #pragma unroll
   for (int t = 0; t < T; ++t) {
     const int row = min(4 * t + c / 4, ROWS - 1);          // past the workgroup's rows and the matrix's: the last one again
@@ -105,41 +143,43 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_lines_kernel(const bf16_t* __
   }
 #pragma unroll
   for (int i = 0; i < X; ++i) xp[i] = x + (int64_t)min(4 * i + c / 4, M - 1) * x_stride;
-  f32x4 acc[T][X];
+  f32x4 acc[T][X][F::SUMS];
 #pragma unroll
   for (int t = 0; t < T; ++t)
 #pragma unroll
-    for (int i = 0; i < X; ++i) acc[t][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < X; ++i)
+#pragma unroll
+      for (int u = 0; u < F::SUMS; ++u) acc[t][i][u] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int blocks = (K + BLOCK - 1) / BLOCK, mine = (blocks - wave + WAVES - 1) / WAVES;    // wave, wave + WAVES, ...
-  bf16x8 a[DEPTH][T], b[DEPTH][X], norm[LATE ? DEPTH : 1];
+  frag a[DEPTH][T], b[DEPTH][X], norm[LATE ? DEPTH : 1];
   float inverse[X];
   auto fetch = [&](auto slot, int i) {
     constexpr int d = decltype(slot)::value;
     int k = (wave + i * WAVES) * BLOCK + at;
-    k = k < K ? k : 0;                                     // beyond K (a multiple of 8): any values, zeros when they are used
+    k = k < K ? k : 0;                                     // beyond K (a multiple of a fragment): any values, zeros when they are used
 #pragma unroll
-    for (int j = 0; j < X; ++j) b[d][j] = *(const bf16x8*)(xp[j] + k);
-    if constexpr (LATE) norm[d] = *(const bf16x8*)(late.weight + k);
+    for (int j = 0; j < X; ++j) b[d][j] = *(const frag*)(xp[j] + k);
+    if constexpr (LATE) norm[d] = *(const frag*)(late.weight + k);
 #pragma unroll
-    for (int t = 0; t < T; ++t) a[d][t] = __builtin_nontemporal_load((const bf16x8*)(wp[t] + k));
+    for (int t = 0; t < T; ++t) a[d][t] = __builtin_nontemporal_load((const frag*)(wp[t] + k));
   };
   auto multiply = [&](auto slot, int i) {
     constexpr int d = decltype(slot)::value;
     const int k0 = (wave + i * WAVES) * BLOCK;
     if constexpr (LATE) {
 #pragma unroll
-      for (int j = 0; j < X; ++j) b[d][j] = normed8(b[d][j], inverse[j], norm[d]);
+      for (int j = 0; j < X; ++j) b[d][j] = F::normed(b[d][j], inverse[j], norm[d]);
     }
     if (k0 + BLOCK > K && k0 + at >= K) {
 #pragma unroll
-      for (int j = 0; j < X; ++j) b[d][j] = zero8();
+      for (int j = 0; j < X; ++j) b[d][j] = F::zero();
 #pragma unroll
-      for (int t = 0; t < T; ++t) a[d][t] = zero8();
+      for (int t = 0; t < T; ++t) a[d][t] = F::zero();
     }
 #pragma unroll
     for (int t = 0; t < T; ++t)
 #pragma unroll
-      for (int j = 0; j < X; ++j) acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d][t], b[d][j], acc[t][j], 0, 0, 0);
+      for (int j = 0; j < X; ++j) F::multiply(a[d][t], b[d][j], acc[t][j]);
   };
   // ahead of a norm every slot is filled, past the wave's blocks too (with any values): the compiler then knows how many loads lie
   // behind the sums of squares, and waits for no operand to add those up
@@ -182,7 +222,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_lines_kernel(const bf16_t* __
   for (int t = 0; t < T; ++t)
 #pragma unroll
     for (int j = 0; j < X; ++j) {
-      const f32x4 s = acc[t][j];
+      const f32x4 s = F::sum(acc[t][j]);
       const float low = (piece & 1) ? s[1] : s[0], high = (piece & 1) ? s[3] : s[2];
       const float one = lanes_sum<4>((piece & 2) ? high : low);
       if (piece == 0) sums[wave][t][j][g][c / 4] = one;
@@ -201,15 +241,16 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_lines_kernel(const bf16_t* __
       const float v = whole(out);
       const int64_t place = (int64_t)m * N + n;
       if constexpr (GLU) {
-        ((bf16_t*)y)[place] = gate_unit(v, whole(out + OUT), act);
+        if constexpr (sizeof(E) == 4) ((float*)y)[place] = v / (1.f + expf(-v)) * whole(out + OUT);
+        else ((bf16_t*)y)[place] = gate_unit(v, whole(out + OUT), act);
       } else if (residual.rows != nullptr) {
-        const bf16_t r = float_to_bf16(bf16_to_float(residual.rows[place]) + v);
-        residual.rows[place] = r;
-        r2 = bf16_to_float(r) * bf16_to_float(r);
+        const float r = rounded_as<E>(load_as_float(residual.rows + place) + v);
+        store_from_float(residual.rows + place, r);
+        r2 = r * r;
       } else if (y_f32) {
         ((float*)y)[place] = v;
       } else {
-        ((bf16_t*)y)[place] = float_to_bf16(v);
+        store_from_float((E*)y + place, v);
       }
     }
     if constexpr (!GLU && X <= 2) squares[out][m] = r2;
@@ -226,29 +267,35 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_lines_kernel(const bf16_t* __
   }
 }
 
-template <int ROWS, int X, int WAVES, bool GLU, bool LATE>
-static int launch_lines(const void* x, int64_t x_stride, const void* w, void* y, int y_f32, int M, int N, int K, LateNorm late,
-                        Residual residual, GateAct act, hipStream_t stream) {
+template <typename E, int ROWS, int X, int WAVES, bool GLU, bool LATE>
+static int launch_lines(const void* x, int64_t x_stride, const void* w, void* y, int y_f32, int M, int N, int K, LateNorm<E> late,
+                        Residual<E> residual, GateAct act, hipStream_t stream) {
   constexpr int T = (ROWS + 3) / 4, OUT = GLU ? ROWS / 2 : ROWS;
   // registers for the operands on their way: eight waves have 256 a lane, four are to share a compute unit with others
-  constexpr int room = (WAVES == 8 ? 232 : X * T > 8 || LATE ? 164 : 124) - 28 - 4 * T * X - 2 * (T + X) - (LATE ? 5 * X : 0);
+  constexpr int held = 4 * T * X * Fragment<E>::SUMS;
+  constexpr int room = (WAVES == 8 || held > 64 ? 232 : held > 32 || LATE ? 164 : 124) - 28 - held - 2 * (T + X) - (LATE ? 5 * X : 0);
   constexpr int fit = room / (4 * (T + X + (LATE ? 1 : 0)));
   constexpr int most = LATE ? 4 : 10, DEPTH = fit < 1 ? 1 : fit > most ? most : fit;
-  hipLaunchKernelGGL((gemm_lines_kernel<ROWS, X, WAVES, DEPTH, GLU, LATE>), dim3((N + OUT - 1) / OUT), dim3(64 * WAVES), 0, stream,
-                     (const bf16_t*)x, x_stride, (const bf16_t*)w, y, y_f32, M, N, K, late, residual, act);
+  hipLaunchKernelGGL((gemm_lines_kernel<E, ROWS, X, WAVES, DEPTH, GLU, LATE>), dim3((N + OUT - 1) / OUT), dim3(64 * WAVES), 0, stream,
+                     (const E*)x, x_stride, (const E*)w, y, y_f32, M, N, K, late, residual, act);
   return DRYFT_LAUNCH_CHECK();
 }
 
-template <int ROWS, int WAVES, bool GLU>
-static int lines_by_rows(const void* x, int64_t x_stride, const void* w, void* y, int y_f32, int M, int N, int K, LateNorm late,
-                         Residual residual, GateAct act, hipStream_t stream) {
-  if (late.squares != nullptr) {
-    if (M <= 4) return launch_lines<ROWS, 1, WAVES, GLU, true>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
-    return launch_lines<ROWS, 2, WAVES, GLU, true>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
+template <typename E, int ROWS, int WAVES, bool GLU>
+static int lines_by_rows(const void* x, int64_t x_stride, const void* w, void* y, int y_f32, int M, int N, int K, LateNorm<E> late,
+                         Residual<E> residual, GateAct act, hipStream_t stream) {
+  if constexpr (sizeof(E) == 4) {
+    if (late.squares != nullptr) return launch_lines<E, ROWS, 1, WAVES, GLU, true>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
+    return launch_lines<E, ROWS, 1, WAVES, GLU, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
+  } else {
+    if (late.squares != nullptr) {
+      if (M <= 4) return launch_lines<E, ROWS, 1, WAVES, GLU, true>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
+      return launch_lines<E, ROWS, 2, WAVES, GLU, true>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
+    }
+    if (M <= 4) return launch_lines<E, ROWS, 1, WAVES, GLU, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
+    if (M <= 8) return launch_lines<E, ROWS, 2, WAVES, GLU, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
+    return launch_lines<E, ROWS, 4, WAVES, GLU, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
   }
-  if (M <= 4) return launch_lines<ROWS, 1, WAVES, GLU, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
-  if (M <= 8) return launch_lines<ROWS, 2, WAVES, GLU, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
-  return launch_lines<ROWS, 4, WAVES, GLU, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
 }
 
 // Rows of a workgroup, and its waves: up to 3,072 outputs the fewest rows that leave every compute unit one workgroup (of eight
@@ -257,13 +304,13 @@ static int lines_by_rows(const void* x, int64_t x_stride, const void* w, void* y
 // their rounds fullest. Each workgroup reads the rows of x again: with more than four of them and a large matrix 20 weight rows
 // share that (151,936 x 2,560 at 8 rows 132 us against 139 with 12; at 4 rows 121 either way; 10,240 x 5,120 at 8 18.9 against 20.4
 // with 10; 5,120 x 8,192 16.8 against 16.6: the line).
-#define LINES_LARGE ((int64_t)40 << 20)
+#define LINES_LARGE ((int64_t)80 << 20)      // bytes of W
 struct LinesShape {
   int rows, waves;
 };
-static LinesShape lines_shape(int M, int N, int K) {
+static LinesShape lines_shape(int M, int N, int64_t row_bytes, bool is_f32) {
   if (N <= 3072) return {N <= 1024 ? 4 : N <= 2048 ? 8 : N <= 2560 ? 10 : 12, 8};
-  if (M > 4 && (int64_t)N * K >= LINES_LARGE) return {20, 4};
+  if (!is_f32 && M > 4 && N * row_bytes >= LINES_LARGE) return {20, 4};      // float32: no registers for so many sums
   int best = 12;
   int64_t least = INT64_MAX;
   for (int rows = 12; rows >= 8; rows -= 2) {
@@ -277,33 +324,63 @@ static LinesShape lines_shape(int M, int N, int K) {
 }
 
 // How many workgroups the product takes, and so how many rows of sums of squares it leaves.
-DRYFT_API int dryft_gemm_lines_blocks(int M, int N, int K) {
-  const int rows = lines_shape(M, N, K).rows;
+DRYFT_API int dryft_gemm_lines_blocks(int M, int N, int K, int is_f32) {
+  const int rows = lines_shape(M, N, (int64_t)K * (is_f32 ? 4 : 2), is_f32).rows;
   return (N + rows - 1) / rows;
 }
 
-static bool lines_refuse(const void* x, int64_t x_stride, const void* w, int M, int K, const LateNorm& late) {
-  return M > LINES_ROWS || K <= 0 || K % 8 || x_stride % 8 || (((uintptr_t)x | (uintptr_t)w) & 15) ||
+template <typename E>
+static bool lines_refuse(const void* x, int64_t x_stride, const void* w, int M, int K, const LateNorm<E>& late) {
+  constexpr int V = Fragment<E>::VALUES;
+  return M > (V == 8 ? LINES_ROWS : LINES_ROWS_F32) || K <= 0 || K % V || x_stride % V || (((uintptr_t)x | (uintptr_t)w) & 15) ||
          (late.squares != nullptr && (M > LATE_ROWS || late.count < 1 || late.count > LATE_MOST || late.weight == nullptr ||
                                       (((uintptr_t)late.squares | (uintptr_t)late.weight) & 15)));
+}
+
+template <typename E>
+static int lines(const void* x, int64_t x_stride, const void* w, void* y, int y_f32, int M, int N, int K, const float* late_squares,
+                 int late_count, float late_eps, const void* late_weight, void* residual_rows, float* squares, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  const LateNorm<E> late{late_squares, late_count, late_eps, (const E*)late_weight};
+  const Residual<E> residual{(E*)residual_rows, squares};
+  if (lines_refuse(x, x_stride, w, M, K, late) || (residual_rows != nullptr && (squares == nullptr || M > LATE_ROWS))) return -1;
+  const LinesShape shape = lines_shape(M, N, (int64_t)K * sizeof(E), sizeof(E) == 4);
+#define LINES(ROWS, W) case ROWS + 32 * W: return lines_by_rows<E, ROWS, W, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, {}, stream);
+  switch (shape.rows + 32 * shape.waves) {
+    LINES(4, 8) LINES(8, 8) LINES(10, 8) LINES(12, 8) LINES(8, 4) LINES(10, 4) LINES(12, 4)
+    case 20 + 32 * 4:
+      if constexpr (sizeof(E) == 2) return lines_by_rows<E, 20, 4, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, {}, stream);
+    default: return -1;
+  }
+#undef LINES
+}
+
+template <typename E>
+static int lines_glu(const void* x, int64_t x_stride, const void* w, void* y, int M, int N, int K, const float* late_squares,
+                     int late_count, float late_eps, const void* late_weight, GateAct act, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  const LateNorm<E> late{late_squares, late_count, late_eps, (const E*)late_weight};
+  if (lines_refuse(x, x_stride, w, M, K, late) || act.limit < 0.f || (act.relu && act.limit > 0.f)) return -1;
+  if (N <= 1024) return lines_by_rows<E, 8, 8, true>(x, x_stride, w, y, 0, M, N, K, late, {}, act, stream);
+  return lines_by_rows<E, 16, 4, true>(x, x_stride, w, y, 0, M, N, K, late, {}, act, stream);
 }
 
 // M <= 16, K a multiple of 8, rows of x and W at 16-byte addresses. y as float (y_f32) or bfloat16, or with `residual` the sum
 // residual[M, N] + y in place and squares[blocks][8] (M <= 8). late_squares: those of the product that left x (M <= 8).
 DRYFT_API int dryft_gemm_lines_bf16(const void* x, int64_t x_stride, const void* w, void* y, int y_f32, int M, int N, int K,
                                     const float* late_squares, int late_count, float late_eps, const void* late_weight,
-                                    void* residual_rows, float* squares, hipStream_t stream) {
-  if (M <= 0 || N <= 0) return 0;
-  const LateNorm late{late_squares, late_count, late_eps, (const bf16_t*)late_weight};
-  const Residual residual{(bf16_t*)residual_rows, squares};
-  if (lines_refuse(x, x_stride, w, M, K, late) || (residual_rows != nullptr && (squares == nullptr || M > LATE_ROWS))) return -1;
-  const LinesShape shape = lines_shape(M, N, K);
-#define LINES(ROWS, W) case ROWS + 32 * W: return lines_by_rows<ROWS, W, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, {}, stream);
-  switch (shape.rows + 32 * shape.waves) {
-    LINES(4, 8) LINES(8, 8) LINES(10, 8) LINES(12, 8) LINES(8, 4) LINES(10, 4) LINES(12, 4) LINES(20, 4)
-    default: return -1;
-  }
-#undef LINES
+                                    void* residual, float* squares, hipStream_t stream) {
+  return lines<bf16_t>(x, x_stride, w, y, y_f32, M, N, K, late_squares, late_count, late_eps, late_weight, residual, squares, stream);
+}
+
+// The same in float32: M <= 4, K a multiple of 4. Us at 1 / 4 rows, against the kernels of gemm_f32.hip: 4,096 x 1,024 5.6 / 5.5 (6.0 /
+// 6.7), 1,024 x 3,072 4.9 / 5.1 (5.8 / 6.2), 151,936 x 1,024 106 / 114 (105 / 123), 6,144 x 2,560 13.3 / 13.6 (13.4 / 18.5), 2,560 x 9,728
+// 20.7 / 20.9 (32 / 39), 3,072 gated outputs of 1,024 7.4 / 7.6 (9.6 / 10.3). At 8 rows the sums of two groups of four leave one
+// workgroup a unit: 151,936 x 1,024 217 us against 157.
+DRYFT_API int dryft_gemm_lines_f32(const void* x, int64_t x_stride, const void* w, void* y, int M, int N, int K,
+                                   const float* late_squares, int late_count, float late_eps, const void* late_weight,
+                                   void* residual, float* squares, hipStream_t stream) {
+  return lines<float>(x, x_stride, w, y, 1, M, N, K, late_squares, late_count, late_eps, late_weight, residual, squares, stream);
 }
 
 // y[M,N] = the gated unit of x . Wg^T and x . Wu^T with W = [Wg; Wu] of 2N rows. Up to 1,024 outputs four a workgroup of eight waves,
@@ -315,13 +392,16 @@ DRYFT_API int dryft_gemm_lines_bf16(const void* x, int64_t x_stride, const void*
 DRYFT_API int dryft_gemm_lines_glu_bf16(const void* x, int64_t x_stride, const void* w, void* y, int M, int N, int K,
                                         const float* late_squares, int late_count, float late_eps, const void* late_weight, int relu,
                                         float limit, float alpha, hipStream_t stream) {
-  if (M <= 0 || N <= 0) return 0;
-  const LateNorm late{late_squares, late_count, late_eps, (const bf16_t*)late_weight};
-  if (lines_refuse(x, x_stride, w, M, K, late) || limit < 0.f || (relu && limit > 0.f)) return -1;
   GateAct act;
   act.relu = relu;
   act.limit = limit;
   act.alpha = alpha;
-  if (N <= 1024) return lines_by_rows<8, 8, true>(x, x_stride, w, y, 0, M, N, K, late, {}, act, stream);
-  return lines_by_rows<16, 4, true>(x, x_stride, w, y, 0, M, N, K, late, {}, act, stream);
+  return lines_glu<bf16_t>(x, x_stride, w, y, M, N, K, late_squares, late_count, late_eps, late_weight, act, stream);
+}
+
+// silu(x . Wg^T) * (x . Wu^T) in float32: M <= 4, K a multiple of 4
+DRYFT_API int dryft_gemm_lines_swiglu_f32(const void* x, int64_t x_stride, const void* w, void* y, int M, int N, int K,
+                                          const float* late_squares, int late_count, float late_eps, const void* late_weight,
+                                          hipStream_t stream) {
+  return lines_glu<float>(x, x_stride, w, y, M, N, K, late_squares, late_count, late_eps, late_weight, {}, stream);
 }

@@ -81,7 +81,9 @@ _SIGNATURES = {
                  "dryft_gemm_rows_swiglu_f32": [_P, _L, _P, _P, _I, _I, _I, _P],
                  "dryft_gemm_direct_f32_shape": [_I, _I],
                  "dryft_gemm_direct_f32": [_P, _L, _P, _P, _I, _I, _I, _I, _P]},
-    "gemm_lines": {"dryft_gemm_lines_blocks": [_I, _I, _I],
+    "gemm_lines": {"dryft_gemm_lines_blocks": [_I, _I, _I, _I],
+                   "dryft_gemm_lines_f32": [_P, _L, _P, _P, _I, _I, _I, _P, _I, _F, _P, _P, _P, _P],
+                   "dryft_gemm_lines_swiglu_f32": [_P, _L, _P, _P, _I, _I, _I, _P, _I, _F, _P, _P],
                    "dryft_gemm_lines_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _P, _I, _F, _P, _P, _P, _P],
                    "dryft_gemm_lines_glu_bf16": [_P, _L, _P, _P, _I, _I, _I, _P, _I, _F, _P, _I, _F, _F, _P]},
     "gemm": {"dryft_gemm_tiled": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _P],
@@ -1013,26 +1015,28 @@ def gemm_wide_bf16(x, w, out, partials=None, group_blocks: int = 2, splits: int 
                                                int(group_blocks), int(depth), int(splits), out_f32, _stream()), "gemm_wide_bf16")
 
 
-LINES_ROWS = 16       # the most rows the kernel that loads matrix-core operands as whole lines takes
+LINES_ROWS = 16       # the most rows the kernel that loads matrix-core operands as whole lines takes in bfloat16
+LINES_ROWS_F32 = 4    # and in float32
+LATE_ROWS = 8         # the most rows of a product that takes its rows through a norm, or leaves their sums of squares
+LATE_MOST = 1024      # workgroups whose sums of squares a product adds up
 
 
 def lines_ok(x, w) -> bool:
-    """Can the kernel that loads matrix-core operands as whole lines take these? At most 16 rows, 16-byte pieces of rows."""
-    return x.shape[0] <= LINES_ROWS and x.shape[1] % 8 == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and \
-        w.data_ptr() % 16 == 0
+    """Can the kernel that loads matrix-core operands as whole lines take these? At most 16 rows in bfloat16 and 4 in float32,
+    16-byte pieces of rows."""
+    piece = 4 if x.dtype == torch.float32 else 8
+    return x.shape[0] <= (LINES_ROWS_F32 if piece == 4 else LINES_ROWS) and x.shape[1] % piece == 0 and x.stride(0) % piece == 0 and \
+        x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
 
 
 def _lines_operands(who: str, x, w) -> None:
-    _gpu(x, "x", torch.bfloat16)
-    _gpu(w, "w", torch.bfloat16)
+    _gpu(x, "x")
+    _float_flag(x, "x")
+    _gpu(w, "w", x.dtype)
     if not (w.dim() == 2 and w.shape[1] == x.shape[1] and w.is_contiguous() and x.stride(1) == 1):
         raise KernelError(f"{who}: x [M,K] row-major, w [N,K] contiguous")
     if not lines_ok(x, w):
-        raise KernelError(f"{who}: needs M <= {LINES_ROWS}, K % 8 == 0 and 16-byte aligned rows, got M={x.shape[0]} K={x.shape[1]}")
-
-
-LATE_ROWS = 8         # the most rows of a product that takes its rows through a norm, or leaves their sums of squares
-LATE_MOST = 1024      # workgroups whose sums of squares a product adds up
+        raise KernelError(f"{who}: needs few rows of 16-byte aligned pieces, got M={x.shape[0]} K={x.shape[1]} in {x.dtype}")
 
 
 def _late(who: str, late, x) -> tuple:
@@ -1041,7 +1045,7 @@ def _late(who: str, late, x) -> tuple:
         return 0, 0, 0.0, 0
     squares, eps, weight = late
     _gpu(squares, "squares", torch.float32)
-    _gpu(weight, "weight", torch.bfloat16)
+    _gpu(weight, "weight", x.dtype)
     if not (squares.dim() == 2 and squares.shape[1] == LATE_ROWS and squares.is_contiguous() and 1 <= squares.shape[0] <= LATE_MOST):
         raise KernelError(f"{who}: the sums of squares must be contiguous [1 to {LATE_MOST}, {LATE_ROWS}]")
     if not (x.shape[0] <= LATE_ROWS and weight.shape == (x.shape[1],) and weight.is_contiguous() and weight.data_ptr() % 16 == 0):
@@ -1049,39 +1053,46 @@ def _late(who: str, late, x) -> tuple:
     return _ptr(squares), squares.shape[0], float(eps), _ptr(weight)
 
 
-def gemm_lines_bf16(x, w, out, late: tuple | None = None) -> torch.Tensor:
-    """``x [M<=16, K] @ w[N, K].T`` into ``out`` (float32 or bfloat16) by the kernel that loads matrix-core operands as whole
-    lines and splits K over the waves of a workgroup alone. With ``late = (squares, eps, weight)`` the rows of ``x`` go through
-    the norm first: ``T(T(x * rsqrt(squares[:, m].sum() / K + eps)) * weight)``."""
-    _lines_operands("gemm_lines", x, w)
-    _gpu(out, "out")
+def _lines(who: str, x, w, out, late, residual, squares) -> None:
     m, k = x.shape
     n = w.shape[0]
-    if not (out.shape == (m, n) and out.is_contiguous() and out.dtype in (torch.float32, torch.bfloat16)):
-        raise KernelError(f"gemm_lines: out must be contiguous [{m},{n}]")
-    _check(_fn("gemm_lines", "dryft_gemm_lines_bf16")(
-        _ptr(x), x.stride(0), _ptr(w), _ptr(out), _float_flag(out, "out"), m, n, k, *_late("gemm_lines", late, x), 0, 0,
-        _stream()), "gemm_lines_bf16")
+    tail = (*_late(who, late, x), _ptr(residual), _ptr(squares), _stream())
+    if x.dtype == torch.float32:
+        rc = _fn("gemm_lines", "dryft_gemm_lines_f32")(_ptr(x), x.stride(0), _ptr(w), _ptr(out), m, n, k, *tail)
+    else:
+        rc = _fn("gemm_lines", "dryft_gemm_lines_bf16")(_ptr(x), x.stride(0), _ptr(w), _ptr(out),
+                                                        int(out is not None and out.dtype == torch.float32), m, n, k, *tail)
+    _check(rc, who)
+
+
+def gemm_lines(x, w, out, late: tuple | None = None) -> torch.Tensor:
+    """``x @ w[N, K].T`` of few rows (``lines_ok``) into ``out`` (float32 or the dtype of ``x``) by the kernel that loads matrix-core
+    operands as whole lines and splits K over the waves of a workgroup alone. With ``late = (squares, eps, weight)`` the rows of
+    ``x`` go through the norm first: ``T(T(x * rsqrt(squares[:, m].sum() / K + eps)) * weight)``."""
+    _lines_operands("gemm_lines", x, w)
+    _gpu(out, "out")
+    if not (out.shape == (x.shape[0], w.shape[0]) and out.is_contiguous() and out.dtype in (torch.float32, x.dtype)):
+        raise KernelError(f"gemm_lines: out must be contiguous [{x.shape[0]},{w.shape[0]}]")
+    _lines("gemm_lines", x, w, out, late, None, None)
     return out
 
 
-def gemm_lines_blocks(m: int, n: int, k: int) -> int:
-    """How many workgroups ``gemm_lines_bf16`` takes, and so rows of sums of squares ``gemm_lines_add_bf16`` leaves."""
-    return int(_fn("gemm_lines", "dryft_gemm_lines_blocks")(int(m), int(n), int(k)))
+def gemm_lines_blocks(m: int, n: int, k: int, dtype: torch.dtype) -> int:
+    """How many workgroups ``gemm_lines`` takes, and so rows of sums of squares ``gemm_lines_add`` leaves."""
+    return int(_fn("gemm_lines", "dryft_gemm_lines_blocks")(int(m), int(n), int(k), int(dtype == torch.float32)))
 
 
-def gemm_lines_add_bf16(x, w, residual) -> torch.Tensor:
-    """The product of ``gemm_lines_bf16`` of up to 8 rows added to ``residual [M, N]`` (in place, the float sum rounded once);
+def gemm_lines_add(x, w, residual) -> torch.Tensor:
+    """The product of ``gemm_lines`` of up to 8 rows added to ``residual [M, N]`` (in place, the float sum rounded once);
     returns what a norm of the sum needs, ``squares [count, 8]``: float sums of its squares over each workgroup's columns."""
     _lines_operands("gemm_lines_add", x, w)
     m, k = x.shape
     n = w.shape[0]
-    _gpu(residual, "residual", torch.bfloat16)
+    _gpu(residual, "residual", x.dtype)
     if not (m <= LATE_ROWS and residual.shape == (m, n) and residual.is_contiguous()):
         raise KernelError(f"gemm_lines_add: up to {LATE_ROWS} rows, residual contiguous [{m},{n}]")
-    squares = torch.empty((gemm_lines_blocks(m, n, k), LATE_ROWS), dtype=torch.float32, device=x.device)
-    _check(_fn("gemm_lines", "dryft_gemm_lines_bf16")(
-        _ptr(x), x.stride(0), _ptr(w), 0, 0, m, n, k, 0, 0, 0.0, 0, _ptr(residual), _ptr(squares), _stream()), "gemm_lines_add_bf16")
+    squares = torch.empty((gemm_lines_blocks(m, n, k, x.dtype), LATE_ROWS), dtype=torch.float32, device=x.device)
+    _lines("gemm_lines_add", x, w, None, None, residual, squares)
     return squares
 
 
@@ -1103,6 +1114,7 @@ def gemm_few_glu_bf16(x, w_gate_up, out, clamped: tuple[float, float] | None = N
     ``gemm_panel_swiglu_bf16``, ``late`` as in ``gemm_lines_bf16``. K a multiple of 8."""
     if relu and clamped is not None:
         raise KernelError("gemm_few_glu: relu or the clamped unit, not both")
+    _gpu(x, "x", torch.bfloat16)
     _lines_operands("gemm_few_glu", x, w_gate_up)
     _gpu(out, "out", torch.bfloat16)
     m, k = x.shape
@@ -1390,7 +1402,7 @@ def rows_f32_ok(x, w) -> bool:
 
 def gemm_rows_f32(x, w, out, splits: int = 1) -> torch.Tensor:
     """``x [M<=16, K] @ w[N, K].T`` on float32 values with the matrix cores' full-precision instruction, every weight
-    read once; ``K`` a multiple of 4 and ``w`` 16-byte aligned. ``splits`` > 1: ``out`` is ``[splits, M, N]`` and receives
+    read once; ``K`` a multiple of 4 and ``w`` 16-byte aligned (whole products of up to 4 rows: ``gemm_lines``). ``splits`` > 1: ``out`` is ``[splits, M, N]`` and receives
     sums over as many runs of K. Rows of ``x`` that do not start at 16-byte addresses go to ``gemm_stream_f32``."""
     _gpu(x, "x", torch.float32)
     _gpu(w, "w", torch.float32)
@@ -1407,6 +1419,8 @@ def gemm_rows_f32(x, w, out, splits: int = 1) -> torch.Tensor:
         if splits > 1:
             raise KernelError("gemm_rows_f32: splits need rows of x at 16-byte addresses")
         return gemm_stream_f32(x, w, out)
+    if splits == 1 and lines_ok(x, w):
+        return gemm_lines(x, w, out)
     _check(_fn("gemm_f32", "dryft_gemm_rows_f32")(_ptr(x), x.stride(0), _ptr(w), _ptr(out), m, n, k, int(splits), _stream()),
            "gemm_rows_f32")
     return out
@@ -1431,9 +1445,9 @@ def gemm_stream_f32(x, w, out) -> torch.Tensor:
     return out
 
 
-def gemm_rows_swiglu_f32(x, w_gate_up, out) -> torch.Tensor:
+def gemm_rows_swiglu_f32(x, w_gate_up, out, late: tuple | None = None) -> torch.Tensor:
     """``silu(x @ Wg.T) * (x @ Wu.T)`` for ``w_gate_up = [Wg; Wu]`` and at most 16 rows of float32 values, in one kernel;
-    operands as ``rows_f32_ok`` wants them."""
+    operands as ``rows_f32_ok`` wants them. ``late`` as in ``gemm_lines``, up to 4 rows."""
     _gpu(x, "x", torch.float32)
     _gpu(w_gate_up, "w_gate_up", torch.float32)
     _gpu(out, "out", torch.float32)
@@ -1445,6 +1459,13 @@ def gemm_rows_swiglu_f32(x, w_gate_up, out) -> torch.Tensor:
         raise KernelError(f"gemm_rows_swiglu_f32: needs M <= 16, K % 4 == 0 and 16-byte aligned rows, got M={m} K={k}")
     if not (out.shape == (m, two_n // 2) and out.is_contiguous()):
         raise KernelError(f"gemm_rows_swiglu_f32: out must be contiguous [{m},{two_n // 2}]")
+    if lines_ok(x, w_gate_up):
+        _check(_fn("gemm_lines", "dryft_gemm_lines_swiglu_f32")(_ptr(x), x.stride(0), _ptr(w_gate_up), _ptr(out), m, two_n // 2, k,
+                                                                *_late("gemm_rows_swiglu_f32", late, x), _stream()),
+               "gemm_rows_swiglu_f32")
+        return out
+    if late is not None:
+        raise KernelError(f"gemm_rows_swiglu_f32: a norm on the way takes up to {LINES_ROWS_F32} rows")
     _check(_fn("gemm_f32", "dryft_gemm_rows_swiglu_f32")(_ptr(x), x.stride(0), _ptr(w_gate_up), _ptr(out), m, two_n // 2, k,
                                                          _stream()), "gemm_rows_swiglu_f32")
     return out

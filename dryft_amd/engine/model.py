@@ -94,7 +94,7 @@ class DecoderModel:
         mods = {"batch", "embed"}
         for part, _ in self._bindings:
             mods.update(part.kernel_modules(self.dtype))
-        if "gemm" in mods and self.dtype == torch.bfloat16:
+        if "gemm" in mods:
             mods.add("gemm_lines")
         if self.dtype == torch.float32:
             mods.update(name + "_f32" for name, plain in (("gemm", "gemm"), ("attn", "attn_rows")) if plain in mods)

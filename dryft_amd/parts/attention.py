@@ -375,10 +375,13 @@ class GQAAttention(Mixer):
             self.n_heads // self.n_kv <= 16
 
     def takes_late(self, rows: int, ctx: StepContext) -> bool:
-        """Decoding steps of few rows whose projection goes to the kernel that can scale its sums."""
+        """Steps of few rows whose projection goes to the kernel that can take its rows through a norm."""
         n, k = self.w_qkv.shape
-        return self._plain(ctx) and self._fused_decoding(ctx, self.w_qkv.dtype) and rows <= ops.LATE_ROWS and k % 8 == 0 and \
-            lines_pay(rows, n, k) and self.w_qkv.data_ptr() % 16 == 0
+        if not self._plain(ctx) or self.w_qkv.data_ptr() % 16:
+            return False
+        if self.w_qkv.dtype == torch.float32:
+            return rows <= ops.LINES_ROWS_F32 and k % 4 == 0
+        return self._fused_decoding(ctx, self.w_qkv.dtype) and rows <= ops.LATE_ROWS and k % 8 == 0 and lines_pay(rows, n, k)
 
     def forward(self, h: torch.Tensor, ctx: StepContext, line: KVLine, writes_cache: bool, leave_product: bool = False):
         """``leave_product``: the output projection may be left unmade (``Product``)."""
@@ -411,7 +414,7 @@ class GQAAttention(Mixer):
             rows <= _PROMPT_PARTIAL_ROWS and \
             ops.rows_to_cache_takes(rows, self.head_dim, self.rotary_dim, True)
         if late is not None:
-            qkv = ops.gemm_lines_bf16(h, self.w_qkv, torch.empty((rows, self.w_qkv.shape[0]), dtype=h.dtype, device=h.device), late=late)
+            qkv = ops.gemm_lines(h, self.w_qkv, torch.empty((rows, self.w_qkv.shape[0]), dtype=h.dtype, device=h.device), late=late)
         elif prompt_parts:
             qkv = linear_for_sum(h, self.w_qkv, allow_partials=True)
         else:

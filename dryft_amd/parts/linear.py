@@ -4,7 +4,7 @@ The reference hands every projection to a vendor library (F.linear,
 engine/dryft_qwen3/model.py:153, 179-180, 237, 258-261). Here:
 
 * float32: this library's own kernels, so the 32-bit path has no reduced-precision matrix
-  mode anywhere: the matrix cores' full-precision instruction (``v_mfma_f32_16x16x4_f32``),
+  mode anywhere: up to 4 rows the kernel of whole lines (below, on the 32-bit instruction); else the matrix cores' full-precision instruction (``v_mfma_f32_16x16x4_f32``),
   with K split over a workgroup's waves (or plain multiply-adds, ``streams_f32``) for at most 16 rows, operands straight
   into LDS in blocks chosen by the number of workgroups for more (``K`` a multiple of 32; else blocks of
   128 x 128 through registers), and a plain tiled kernel for sizes those do not take;
@@ -76,7 +76,7 @@ def rows_f32_splits(n: int, k: int) -> int:
 
 
 def streams_f32(m: int, n: int, k: int) -> bool:
-    """Does a product of at most 16 rows of float32 values go to the plain multiply-adds that read whole lines, or to the
+    """Does a product of 5 to 16 rows of float32 values (or of any up to 16 that the kernel of whole lines refuses) go to the plain multiply-adds that read whole lines, or to the
     matrix cores with K split over a workgroup's waves? The first is bound by its arithmetic, the rows of x, and by K walked
     chunk by chunk; the second by its trips to memory (three of them from K = 2,560 on) and by reading the rows of x again in
     every workgroup. In a captured chain on rotating cold weights, us, first against second: 6,144 x 1,024 at 1 / 4 / 8 / 16
@@ -87,10 +87,11 @@ def streams_f32(m: int, n: int, k: int) -> bool:
 
 
 def swiglu_f32_ok(h: torch.Tensor, w_gate_up: torch.Tensor) -> bool:
-    """Does the float32 gate/up product run with its activation in one kernel? The matrix cores' form only, so up to eight
-    rows not from K = 2,560 on: 19,456 x 2,560 at 4 rows 56 us against 43 and 3 for the activation; 6,144 x 1,024 9.9 against
+    """Does the float32 gate/up product run with its activation in one kernel? Up to four rows always; beyond, the matrix cores'
+    form only, so up to eight rows not from K = 2,560 on: 19,456 x 2,560 at 4 rows 56 us against 43 and 3 for the activation; 6,144 x 1,024 9.9 against
     9.3 and 3."""
-    return h.shape[0] <= STREAM_ROWS and ops.rows_f32_ok(h, w_gate_up) and not (h.shape[0] <= 8 and h.shape[1] >= 2560)
+    return ops.lines_ok(h, w_gate_up) or \
+        (h.shape[0] <= STREAM_ROWS and ops.rows_f32_ok(h, w_gate_up) and not (h.shape[0] <= 8 and h.shape[1] >= 2560))
 
 
 def lines_pay(m: int, n: int, k: int) -> bool:
@@ -263,6 +264,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, *, out_dtype: torch.dtype | None = 
     n = w.shape[0]
     out_dtype = out_dtype or x.dtype
     if x.dtype == torch.float32:
+        if ops.lines_ok(x, w):
+            return ops.gemm_rows_f32(x, w, torch.empty((m, n), dtype=torch.float32, device=x.device))
         if m <= STREAM_ROWS and ops.rows_f32_ok(x, w):
             splits = rows_f32_splits(n, k) if allow_partials else 1
             if splits > 1:
@@ -286,7 +289,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, *, out_dtype: torch.dtype | None = 
         splits, group, depth = stream_plan(n, k, allow_partials)
         if lines_pay(m, n, k):
             # whole sums; unrounded where the caller would have been given float partial sums
-            return ops.gemm_lines_bf16(x, w, torch.empty((m, n), dtype=torch.float32 if splits > 1 else out_dtype, device=x.device))
+            return ops.gemm_lines(x, w, torch.empty((m, n), dtype=torch.float32 if splits > 1 else out_dtype, device=x.device))
         if splits > 1:
             partials = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
             ops.gemm_stream_bf16(x, w, None, partials, group, splits, depth)

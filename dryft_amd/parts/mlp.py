@@ -36,7 +36,11 @@ class SwiGLU(FeedForward):
         return ("gemm", "activation")
 
     def takes_late(self, rows: int, ctx) -> bool:
-        return rows <= ops.LATE_ROWS and ops.few_glu_pays(rows, self.inter, self.hidden) and self.w_gate_up.data_ptr() % 16 == 0
+        if self.w_gate_up.data_ptr() % 16:
+            return False
+        if self.w_gate_up.dtype == torch.float32:
+            return not self.relu and rows <= ops.LINES_ROWS_F32 and self.hidden % 4 == 0
+        return rows <= ops.LATE_ROWS and ops.few_glu_pays(rows, self.inter, self.hidden)
 
     def forward(self, h, ctx, leave_product: bool = False):
         late = None
@@ -56,7 +60,7 @@ class SwiGLU(FeedForward):
         elif h.dtype == torch.bfloat16 and h.shape[0] <= STREAM_ROWS and few_rows_ok(h, self.w_gate_up):
             ops.gemm_stream_swiglu_bf16(h, self.w_gate_up, act)       # the same for any K that is a multiple of 8
         elif h.dtype == torch.float32 and swiglu_f32_ok(h, self.w_gate_up):
-            ops.gemm_rows_swiglu_f32(h, self.w_gate_up, act)
+            ops.gemm_rows_swiglu_f32(h, self.w_gate_up, act, late=late)
         else:
             ops.silu_mul(linear(h, self.w_gate_up), act)
         return Product(act, self.w_down) if leave_product else linear_for_sum(act, self.w_down, allow_partials=True)

@@ -39,7 +39,7 @@ class RMSNorm(Norm):
         kernel then does the sum, and the reader's the norm."""
         if isinstance(delta, Product):
             if late and self.late_ok(res, delta):
-                return res, LateNormed(res, ops.gemm_lines_add_bf16(delta.x, delta.w, res), self.eps, self.weight)
+                return res, LateNormed(res, ops.gemm_lines_add(delta.x, delta.w, res), self.eps, self.weight)
             delta = delta.made()
         y = torch.empty_like(res)
         if isinstance(delta, Partials):
@@ -50,9 +50,9 @@ class RMSNorm(Norm):
 
     def late_ok(self, res: torch.Tensor, product: Product) -> bool:
         m, n = res.shape
-        return res.dtype == product.x.dtype == self.weight.dtype == torch.bfloat16 and 0 < m <= ops.LATE_ROWS and \
-            res.is_contiguous() and res.data_ptr() % 16 == 0 and n % 8 == 0 and self.weight.data_ptr() % 16 == 0 and \
-            ops.lines_ok(product.x, product.w) and ops.gemm_lines_blocks(m, n, product.x.shape[1]) <= ops.LATE_MOST
+        return res.dtype == product.x.dtype == self.weight.dtype and 0 < m <= ops.LATE_ROWS and res.is_contiguous() and \
+            res.data_ptr() % 16 == 0 and self.weight.data_ptr() % 16 == 0 and ops.lines_ok(product.x, product.w) and \
+            ops.gemm_lines_blocks(m, n, product.x.shape[1], res.dtype) <= ops.LATE_MOST
 
 
 register_part("rmsnorm", RMSNorm)

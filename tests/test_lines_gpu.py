@@ -13,10 +13,10 @@ def ops():
     return ops
 
 
-def operands(m, n, k, seed, stride=0):
+def operands(m, n, k, seed, stride=0, dtype=torch.bfloat16):
     torch.manual_seed(seed)
-    x = torch.randn(m, stride or k, device=DEV).to(torch.bfloat16)[:, :k]
-    w = (torch.randn(n, k, device=DEV) * k ** -0.5).to(torch.bfloat16)
+    x = torch.randn(m, stride or k, device=DEV).to(dtype)[:, :k]
+    w = (torch.randn(n, k, device=DEV) * k ** -0.5).to(dtype)
     return x, w
 
 
@@ -36,16 +36,35 @@ CASES = [(1, 1, 8), (4, 3, 24), (5, 4, 120), (3, 5, 128), (8, 1024, 136), (9, 10
 def test_product(m, n, k):
     x, w = operands(m, n, k, m + n + k, stride=k + 8)
     want, bound = product(x, w)
-    out = ops().gemm_lines_bf16(x, w, torch.full((m, n), float("nan"), device=DEV))
+    out = ops().gemm_lines(x, w, torch.full((m, n), float("nan"), device=DEV))
     assert (out.double() - want).abs().le(bound).all()
-    rounded = ops().gemm_lines_bf16(x, w, torch.full((m, n), float("nan"), device=DEV).to(torch.bfloat16))
+    rounded = ops().gemm_lines(x, w, torch.full((m, n), float("nan"), device=DEV).to(torch.bfloat16))
     assert torch.equal(rounded, out.to(torch.bfloat16))
+
+
+CASES_F32 = [(1, 1, 4), (2, 3, 12), (3, 5, 60), (4, 4, 64), (4, 1024, 68), (1, 1025, 516), (2, 2049, 644), (3, 2561, 36), (4, 3073, 1284),
+             (4, 5120, 8192)]
+
+
+@pytest.mark.parametrize("m,n,k", CASES_F32)
+def test_float32_product_and_residual_sum(m, n, k):
+    o = ops()
+    x, w = operands(m, n, k, m + n + k, stride=k + 4, dtype=torch.float32)
+    want, bound = product(x, w)
+    out = o.gemm_lines(x, w, torch.full((m, n), float("nan"), device=DEV))
+    assert (out.double() - want).abs().le(bound).all()
+    residual = torch.randn(m, n, device=DEV)
+    summed = residual + out                                     # the same sums, added and rounded once
+    squares = o.gemm_lines_add(x, w, residual)
+    assert torch.equal(residual, summed)
+    total = (residual.double() ** 2).sum(1)
+    assert (squares.double().sum(0)[:m] - total).abs().le(n * 2.0 ** -24 * total).all()
 
 
 def late_rows(r, squares, eps, weight):
     """The norm by its formula with its two roundings, from the sums of squares given."""
     inverse = torch.rsqrt(squares.sum(0)[:r.shape[0]] / r.shape[1] + eps)[:, None]
-    return ((r.float() * inverse).to(torch.bfloat16).float() * weight.float()).to(torch.bfloat16)
+    return ((r.float() * inverse).to(r.dtype).float() * weight.float()).to(r.dtype)
 
 
 @pytest.mark.parametrize("m,n,k", [c for c in CASES if c[0] <= 8])
@@ -55,7 +74,7 @@ def test_residual_sum_and_its_squares(m, n, k):
     residual = torch.randn(m, n, device=DEV).to(torch.bfloat16)
     want, bound = product(x, w)
     want = residual.double() + want
-    squares = o.gemm_lines_add_bf16(x, w, residual)
+    squares = o.gemm_lines_add(x, w, residual)
     assert (residual.double() - want).abs().le(2.0 ** -8 * want.abs() + 1.01 * bound).all()        # one rounding
     total = (residual.double() ** 2).sum(1)
     assert (squares.double().sum(0)[:m] - total).abs().le(n * 2.0 ** -24 * total).all()
@@ -65,23 +84,28 @@ def test_residual_sum_and_its_squares(m, n, k):
 @pytest.mark.parametrize("m,n,k,count", [(1, 1, 8, 1), (3, 9, 136, 2), (4, 1025, 1032, 256), (5, 3073, 2560, 257), (8, 2561, 520, 512),
                                          (7, 4099, 1288, 1024), (8, 5123, 8200, 700), (2, 40, 2048, 63)])
 @pytest.mark.parametrize("glu", [False, True])
-def test_norm_on_the_way(m, n, k, count, glu):
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_norm_on_the_way(m, n, k, count, glu, dtype):
     """Against the same product of rows that were normed ahead. A root that is off by a unit in its last place may round a value
     of the row the other way: by powers of two it is exact."""
     o = ops()
-    torch.manual_seed(count)
-    r, w = operands(m, 2 * n if glu else n, k, m + n + k + 2)
-    weight = (1 + 0.3 * torch.randn(k, device=DEV)).to(torch.bfloat16)
+    if dtype == torch.float32:
+        m = min(m, o.LINES_ROWS_F32)
+    r, w = operands(m, 2 * n if glu else n, k, m + n + k + 2, dtype=dtype)
+    weight = (1 + 0.3 * torch.randn(k, device=DEV)).to(dtype)
     squares = torch.full((count, 8), float("nan"), device=DEV)
     squares[:, :m] = 0
     squares[count // 2, :m] = k * 4.0 ** (torch.arange(m, device=DEV) % 3 - 1)
     rows = late_rows(r, squares, 0.0, weight)
-    if glu:
+    if glu and dtype == torch.float32:
+        got = o.gemm_rows_swiglu_f32(r, w, torch.empty((m, n), device=DEV), late=(squares, 0.0, weight))
+        want = o.gemm_rows_swiglu_f32(rows, w, torch.empty((m, n), device=DEV))
+    elif glu:
         got = o.gemm_few_glu_bf16(r, w, torch.empty((m, n), dtype=torch.bfloat16, device=DEV), late=(squares, 0.0, weight))
         want = o.gemm_few_glu_bf16(rows, w, torch.empty((m, n), dtype=torch.bfloat16, device=DEV))
     else:
-        got = o.gemm_lines_bf16(r, w, torch.empty((m, n), device=DEV), late=(squares, 0.0, weight))
-        want = o.gemm_lines_bf16(rows, w, torch.empty((m, n), device=DEV))
+        got = o.gemm_lines(r, w, torch.empty((m, n), device=DEV), late=(squares, 0.0, weight))
+        want = o.gemm_lines(rows, w, torch.empty((m, n), device=DEV))
     assert torch.equal(got, want)
 
 
@@ -89,16 +113,19 @@ def test_refusals():
     o = ops()
     x, w = operands(17, 8, 64, 0)
     with pytest.raises(o.KernelError):
-        o.gemm_lines_bf16(x, w, torch.empty((17, 8), device=DEV))
+        o.gemm_lines(x, w, torch.empty((17, 8), device=DEV))
+    x, w = operands(5, 8, 64, 0, dtype=torch.float32)
+    with pytest.raises(o.KernelError):
+        o.gemm_lines(x, w, torch.empty((5, 8), device=DEV))
     x, w = operands(2, 8, 60, 0)
     with pytest.raises(o.KernelError):
-        o.gemm_lines_bf16(x, w, torch.empty((2, 8), device=DEV))
+        o.gemm_lines(x, w, torch.empty((2, 8), device=DEV))
     x, w = operands(2, 8, 64, 0)
     weight = torch.ones(64, dtype=torch.bfloat16, device=DEV)
     with pytest.raises(o.KernelError):
-        o.gemm_lines_bf16(x, w, torch.empty((2, 8), device=DEV), late=(torch.zeros((1025, 8), device=DEV), 0.0, weight))
+        o.gemm_lines(x, w, torch.empty((2, 8), device=DEV), late=(torch.zeros((1025, 8), device=DEV), 0.0, weight))
     x, w = operands(9, 8, 64, 0)
     with pytest.raises(o.KernelError):
-        o.gemm_lines_bf16(x, w, torch.empty((9, 8), device=DEV), late=(torch.zeros((4, 8), device=DEV), 0.0, weight))
+        o.gemm_lines(x, w, torch.empty((9, 8), device=DEV), late=(torch.zeros((4, 8), device=DEV), 0.0, weight))
     with pytest.raises(o.KernelError):
-        o.gemm_lines_add_bf16(x, w, torch.zeros((9, 8), dtype=torch.bfloat16, device=DEV))
+        o.gemm_lines_add(x, w, torch.zeros((9, 8), dtype=torch.bfloat16, device=DEV))
