@@ -313,13 +313,12 @@ __device__ __forceinline__ void v_tile_write(int tile_index, int kvh, const T* _
     }
     base[threadIdx.x] = where;
     in_page[threadIdx.x] = at;
-  }
-  __syncthreads();
-  if (threadIdx.x < V_TILE_ROWS / 32) {                     // is this block of 32 rows one aligned block of a page?
-    const int t0 = 32 * threadIdx.x;
-    bool ok = base[t0] >= 0 && in_page[t0] % 32 == 0;
-    for (int j = 1; j < 32; ++j) ok = ok && base[t0 + j] == base[t0] && in_page[t0 + j] == in_page[t0] + j;
-    block_ok[threadIdx.x] = ok;
+    // is a block of 32 rows one aligned block of a page? A wave holds both blocks' rows, and each asks its block's first
+    const int64_t block_where = __shfl(where, threadIdx.x & 32, WAVE);
+    const int block_at = __shfl(at, threadIdx.x & 32, WAVE);
+    const bool fits = block_where >= 0 && block_at % 32 == 0 && where == block_where && at == block_at + (int)(threadIdx.x & 31);
+    const uint64_t all = __ballot(fits);
+    if (threadIdx.x % 32 == 0) block_ok[threadIdx.x / 32] = (uint32_t)(all >> threadIdx.x) == 0xffffffffu;
   }
   __syncthreads();
   for (int e = threadIdx.x; e < head_dim * (V_TILE_ROWS / 8); e += blockDim.x) {
