@@ -276,8 +276,19 @@ static int launch_lines(const void* x, int64_t x_stride, const void* w, void* y,
   constexpr int room = (WAVES == 8 || held > 64 ? 232 : held > 32 || LATE ? 164 : 124) - 28 - held - 2 * (T + X) - (LATE ? 5 * X : 0);
   constexpr int fit = room / (4 * (T + X + (LATE ? 1 : 0)));
   constexpr int most = LATE ? 4 : 10, DEPTH = fit < 1 ? 1 : fit > most ? most : fit;
-  hipLaunchKernelGGL((gemm_lines_kernel<E, ROWS, X, WAVES, DEPTH, GLU, LATE>), dim3((N + OUT - 1) / OUT), dim3(64 * WAVES), 0, stream,
-                     (const E*)x, x_stride, (const E*)w, y, y_f32, M, N, K, late, residual, act);
+  // Ahead of a norm five to eight rows are work for the vector units too, and waves side by side hide it better than blocks on their
+  // way: one block a wave, us at 8 rows against two or three, 6,144 x 2,560 8.4 (10.0), 4,096 x 1,024 5.0 (6.1), 3,072 gated outputs
+  // of 1,024 5.5 (6.1); gated outputs of a long K want two (9,728 of 2,560 20.6, with one 21.5).
+#define GO(D)                                                                                                                  \
+  hipLaunchKernelGGL((gemm_lines_kernel<E, ROWS, X, WAVES, D, GLU, LATE>), dim3((N + OUT - 1) / OUT), dim3(64 * WAVES), 0, stream, \
+                     (const E*)x, x_stride, (const E*)w, y, y_f32, M, N, K, late, residual, act)
+  if constexpr (LATE && X == 2 && WAVES == 4) {
+    if (!GLU || K <= 1024) GO(1);
+    else GO(DEPTH);
+  } else {
+    GO(DEPTH);
+  }
+#undef GO
   return DRYFT_LAUNCH_CHECK();
 }
 
