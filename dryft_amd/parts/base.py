@@ -243,6 +243,16 @@ class FeedForward(Part):
         raise NotImplementedError
 
 
+def works_row_by_row(ffn) -> bool:
+    """``row_wise``, as said by the class whose ``forward`` runs (one that replaces ``forward`` has to say it again)."""
+    for cls in type(ffn).__mro__:
+        if "row_wise" in vars(cls):
+            return bool(ffn.row_wise)
+        if "forward" in vars(cls):
+            return False
+    return False
+
+
 class StreamPart(Part):
     """Acts on the residual stream between two runs of the schedule (where a pass over a run of layers begins, say):
     a run that names it hands over what is still to be added to the stream and gets back what is to be added now."""

@@ -14,7 +14,7 @@ from __future__ import annotations
 from inspect import signature
 
 from . import register_block
-from .base import FeedForward, Mixer, Norm, Product
+from .base import FeedForward, Mixer, Norm, Product, works_row_by_row
 
 
 class PreNormBlock:
@@ -23,39 +23,40 @@ class PreNormBlock:
     def __init__(self, mixer_norm: Norm, mixer: Mixer, ffn_norm: Norm, ffn: FeedForward):
         self.mixer_norm, self.mixer, self.ffn_norm, self.ffn = mixer_norm, mixer, ffn_norm, ffn
         # the parts that know the option (a class of the user's that replaces the call need not)
-        self._leaves = {id(part): "leave_product" in signature(part.forward).parameters for part in (mixer, ffn)}
-        self._folds = {id(norm): "late" in signature(norm.add_forward).parameters for norm in (mixer_norm, ffn_norm)}
+        self._leaves = {role: "leave_product" in signature(part.forward).parameters for role, part in (("mixer", mixer), ("ffn", ffn))}
+        self._folds = {role: "late" in signature(norm.add_forward).parameters for role, norm in (("mixer", mixer_norm), ("ffn", ffn_norm))}
 
     def parts(self):
         return {"mixer_norm": self.mixer_norm, "mixer": self.mixer, "ffn_norm": self.ffn_norm, "ffn": self.ffn}
 
-    takes_products = True
-
     @property
     def picks_rows(self) -> bool:
         """Can the block go on from its mixer with a choice of its rows (``pick`` gathers them)?"""
-        return self.ffn.row_wise
+        return works_row_by_row(self.ffn)
 
-    def forward(self, x, pending, ctx, line, writes_cache: bool, pick=None):
+    def forward(self, x, pending, ctx, line, writes_cache: bool, pick=None, leave_product: bool = False):
+        """``pick`` gathers the rows that go on behind the mixer; ``leave_product``: the feed-forward's last product may be handed
+        on unmade."""
         if pending is None:
             h = self.mixer_norm.forward(x)
         else:
-            x, h = self._added(self.mixer_norm, x, pending, self.mixer, ctx)
-        mixed = self.mixer.forward(h, ctx, line, writes_cache, **self._left(self.mixer))
+            x, h = self._added("mixer", x, pending, ctx)
+        mixed = self.mixer.forward(h, ctx, line, writes_cache, **self._left("mixer"))
         if pick is not None:
             x, mixed = pick(x), pick(mixed)
-        x, h = self._added(self.ffn_norm, x, mixed, self.ffn, ctx)
-        return x, self.ffn.forward(h, ctx, **self._left(self.ffn))
+        x, h = self._added("ffn", x, mixed, ctx)
+        return x, self.ffn.forward(h, ctx, **(self._left("ffn") if leave_product else {}))
 
-    def _left(self, part) -> dict:
-        return {"leave_product": True} if self._leaves[id(part)] else {}
+    def _left(self, role: str) -> dict:
+        return {"leave_product": True} if self._leaves[role] else {}
 
-    def _added(self, norm: Norm, x, delta, reader, ctx):
+    def _added(self, reader: str, x, delta, ctx):
+        norm, part = (self.mixer_norm, self.mixer) if reader == "mixer" else (self.ffn_norm, self.ffn)
         if not isinstance(delta, Product):
             return norm.add_forward(x, delta)
-        if not self._folds[id(norm)]:
+        if not self._folds[reader]:
             return norm.add_forward(x, delta.made())
-        return norm.add_forward(x, delta, late=self._leaves[id(reader)] and reader.takes_late(x.shape[0], ctx))
+        return norm.add_forward(x, delta, late=self._leaves[reader] and part.takes_late(x.shape[0], ctx))
 
 
 register_block("prenorm", PreNormBlock)

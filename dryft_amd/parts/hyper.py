@@ -18,7 +18,7 @@ import torch
 from ..csrc import ops
 from ..weights.spec import VECTOR
 from . import register_block, register_part
-from .base import Deferred, FeedForward, Mixer, Norm, Part, Partials, StepContext
+from .base import Deferred, FeedForward, Mixer, Norm, Part, Partials, StepContext, works_row_by_row
 from .stream import as_deferred
 
 
@@ -104,7 +104,7 @@ class HyperBlock:
     @property
     def picks_rows(self) -> bool:
         """Can the block go on from its mixer with a choice of its rows (``pick`` gathers them)?"""
-        return self.ffn is not None and self.ffn.row_wise
+        return self.ffn is not None and works_row_by_row(self.ffn)
 
     def forward(self, x, pending, ctx: StepContext, line, writes_cache: bool, pick=None):
         x, h = read_streams(x, as_deferred(pending), self.mixer_route, self.mixer_norm, ctx.dtype)

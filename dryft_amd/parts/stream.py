@@ -27,7 +27,7 @@ import torch
 from ..csrc import ops
 from ..weights.spec import VECTOR
 from . import register_block, register_part
-from .base import Deferred, FeedForward, Mixer, Norm, Part, Partials, StepContext, StreamPart, matrix
+from .base import Deferred, FeedForward, Mixer, Norm, Part, Partials, StepContext, StreamPart, matrix, works_row_by_row
 from .linear import linear, linear_for_sum
 
 
@@ -177,7 +177,7 @@ class SandwichBlock:
     @property
     def picks_rows(self) -> bool:
         """Can the block go on from its mixer with a choice of its rows (``pick`` gathers them)?"""
-        return self.ffn is not None and self.ffn.row_wise
+        return self.ffn is not None and works_row_by_row(self.ffn)
 
     def forward(self, x, pending, ctx: StepContext, line, writes_cache: bool, pick=None):
         # the embedding's output starts the stream and is read again later: it is never updated in place
@@ -212,7 +212,7 @@ class PostNormBlock:
     @property
     def picks_rows(self) -> bool:
         """Can the block go on from its mixer with a choice of its rows (``pick`` gathers them)?"""
-        return self.ffn is not None and self.ffn.row_wise
+        return self.ffn is not None and works_row_by_row(self.ffn)
 
     def forward(self, x, pending, ctx: StepContext, line, writes_cache: bool, pick=None):
         x, h = read_plain(x, pending, ctx.dtype)
@@ -283,7 +283,7 @@ class PreNormBlock:
     @property
     def picks_rows(self) -> bool:
         """Can the block go on from its mixer with a choice of its rows (``pick`` gathers them)?"""
-        return self.ffn is not None and self.ffn.row_wise and self.side is None
+        return self.ffn is not None and works_row_by_row(self.ffn) and self.side is None
 
     def forward(self, x, pending, ctx: StepContext, line, writes_cache: bool, pick=None):
         # the embedding's output starts the stream and other parts may read it again: never updated in place
