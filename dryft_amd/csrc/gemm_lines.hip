@@ -283,8 +283,13 @@ static int launch_lines(const void* x, int64_t x_stride, const void* w, void* y,
   hipLaunchKernelGGL((gemm_lines_kernel<E, ROWS, X, WAVES, D, GLU, LATE>), dim3((N + OUT - 1) / OUT), dim3(64 * WAVES), 0, stream, \
                      (const E*)x, x_stride, (const E*)w, y, y_f32, M, N, K, late, residual, act)
   if constexpr (LATE && X == 2 && WAVES == 4) {
-    if (!GLU || K <= 1024) GO(1);
-    else GO(DEPTH);
+    if constexpr (GLU) {
+      if (K > 1024) {
+        GO(DEPTH);
+        return DRYFT_LAUNCH_CHECK();
+      }
+    }
+    GO(1);
   } else {
     GO(DEPTH);
   }

@@ -8,13 +8,11 @@ plan gives, and layers run in the order of the schedule.
 
 from __future__ import annotations
 
-from inspect import signature
-
 import torch
 
 from ..config.plan import ModelPlan
 from ..parts import block_class, build_part
-from ..parts.base import Deferred, Part, Partials, Product, StepContext
+from ..parts.base import Deferred, Part, Partials, Product, StepContext, accepts
 from ..weights.spec import TensorSpec
 from ..csrc import ops
 
@@ -41,7 +39,7 @@ class DecoderModel:
                 raise ValueError(f"block {layer.block!r} needs parts {missing}")
             parts = {role: build_part(layer.parts[role]) for role in cls.roles}
             self.blocks.append(cls(**parts))
-            self._options.append(frozenset(signature(self.blocks[-1].forward).parameters))
+            self._options.append(frozenset(o for o in ("pick", "leave_product") if accepts(self.blocks[-1].forward, o)))
             for role in cls.roles:
                 self._bindings.append((parts[role], layer.parts[role].tensors))
         self._bindings.append((self.final_norm, plan.final_norm.tensors))

@@ -8,6 +8,8 @@ maps logical tensor names to checkpoint names and wires the parts together.
 
 from __future__ import annotations
 
+import functools
+import inspect
 from dataclasses import dataclass, field
 from typing import Any
 
@@ -241,6 +243,16 @@ class FeedForward(Part):
 
     def forward(self, h: torch.Tensor, ctx: StepContext):
         raise NotImplementedError
+
+
+@functools.lru_cache(maxsize=None)
+def _parameters(function) -> frozenset[str]:
+    return frozenset(inspect.signature(function).parameters)
+
+
+def accepts(method, name: str) -> bool:
+    """Does a part's or block's method take the argument ``name``? (Looked up once a function: models ask per layer.)"""
+    return name in _parameters(getattr(method, "__func__", method))
 
 
 def works_row_by_row(ffn) -> bool:

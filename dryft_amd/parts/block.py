@@ -11,10 +11,8 @@ through it (``LateNormed``).
 
 from __future__ import annotations
 
-from inspect import signature
-
 from . import register_block
-from .base import FeedForward, Mixer, Norm, Product, works_row_by_row
+from .base import FeedForward, Mixer, Norm, Product, accepts, works_row_by_row
 
 
 class PreNormBlock:
@@ -23,8 +21,8 @@ class PreNormBlock:
     def __init__(self, mixer_norm: Norm, mixer: Mixer, ffn_norm: Norm, ffn: FeedForward):
         self.mixer_norm, self.mixer, self.ffn_norm, self.ffn = mixer_norm, mixer, ffn_norm, ffn
         # the parts that know the option (a class of the user's that replaces the call need not)
-        self._leaves = {role: "leave_product" in signature(part.forward).parameters for role, part in (("mixer", mixer), ("ffn", ffn))}
-        self._folds = {role: "late" in signature(norm.add_forward).parameters for role, norm in (("mixer", mixer_norm), ("ffn", ffn_norm))}
+        self._leaves = {role: accepts(part.forward, "leave_product") for role, part in (("mixer", mixer), ("ffn", ffn))}
+        self._folds = {role: accepts(norm.add_forward, "late") for role, norm in (("mixer", mixer_norm), ("ffn", ffn_norm))}
 
     def parts(self):
         return {"mixer_norm": self.mixer_norm, "mixer": self.mixer, "ffn_norm": self.ffn_norm, "ffn": self.ffn}
