@@ -6,7 +6,7 @@
 //    sizes the matrix-core kernel refuses.
 //  * gemm_stream (M <= 16) and gemm_wide (M <= 64): bfloat16, few rows (decoding, output head): every
 //    weight is read once and multiplied on the matrix cores; K may be split across workgroups into
-//    float partial sums that the consumer adds in a fixed order. gemm_panel (M <= 64) is the fused gate/up
+//    float partial sums that the consumer adds in a fixed order. gemm_panel (M <= 96) is the fused gate/up
 //    product, gemm_mid (M <= 256) the projections back to the hidden width for short prompts.
 #include "gate_unit.h"
 
@@ -532,7 +532,7 @@ DRYFT_API int dryft_gemm_wide_swiglu_bf16(const void* x, int64_t x_stride, const
 }
 
 // ------------------------------------------------------------------------------------------- panel
-// The fused gate/up product with its activation for steps of up to 64 rows, with the operands going from memory straight
+// The fused gate/up product with its activation for steps of up to 96 rows, with the operands going from memory straight
 // into LDS (global_load_lds_dwordx4: 16 bytes a lane, no registers in between and nothing for the waves to store),
 // two groups of K ahead of the one that is multiplied. A workgroup of four to eight waves owns 8 outputs a wave
 // (each wave the gate rows and the up rows of its own) and all MT tiles of 16 rows of x. A group is
@@ -551,8 +551,22 @@ DRYFT_API int dryft_gemm_wide_swiglu_bf16(const void* x, int64_t x_stride, const
 // with depths of their own (26 at best). The plain product of the same form was no faster than what serves it now.
 // Walking K from a different starting group in every workgroup took Qwen3-8B's gate/up (rows 8,192 bytes apart)
 // from 44 to 38 us at 8 to 40 rows; at Qwen3-4B's 5,120 bytes it changes nothing.
+// The caches are told that the weights are read once (panel_load16_once): in a captured chain on rotating cold weights, us at 17 /
+// 33 / 64 rows, 9,728 outputs of K 2,560 19.5 / 20.7 / 23.4 (without 20.9 / 21.5 / 23.6), 12,288 of 4,096 35.9 / 36.6 / 38.2 (39.2 /
+// 39.3 / 40.9), 8,192 of 2,048 12.9 / 13.3 / 15.4 (13.9 / 13.7 / 15.2). At 65 to 96 rows it loads 80 or 96 rows of x where the tall form below
+// loads 128: at 65 / 80 / 96 rows the first 23.7 / 24.4 / 26.3 (26.0 / 27.2 / 28.3), the second 39.2 / 39.0 / 40.5 (44.5 / 47.8 / 45.3),
+// 3,072 of 1,024 8.5 / 8.8 / 9.7 (9.9 / 10.0 / 10.2); at 112 it is behind (31.8 / 29.8, 52 / 45, 11.3 / 10.4).
 __device__ __forceinline__ void panel_load16(const void* base, uint32_t offset, uint32_t lds_base) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(offset), "s"(base) : "memory", "m0");
+}
+// The same for weights, which no other workgroup reads: the caches give their lines up first (nt), so that the rows of x, which
+// every workgroup of a die reads, stay in its L2.
+template <bool ONCE>
+__device__ __forceinline__ void panel_load16_once(const void* base, uint32_t offset, uint32_t lds_base) {
+  if constexpr (ONCE)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds_base), "v"(offset), "s"(base) : "memory", "m0");
+  else
+    panel_load16(base, offset, lds_base);
 }
 
 // s_waitcnt vmcnt(N) alone (vmcnt sits in bits 3:0 and 15:14 of the immediate, the other counters stay at their
@@ -587,7 +601,9 @@ __device__ __forceinline__ void swiglu_store4(bf16_t* __restrict__ y_row, int fi
 }
 
 #define PANEL_GROUP 128                      // values of K in a group; K must be a multiple of it
-#define PANEL_STAGES 3
+#define PANEL_ROWS 96
+// Groups of K in LDS: three, or two where a third does not fit (96 rows of x and 128 of W).
+constexpr int panel_stages(int mt, int waves) { return 3 * (16 * waves + 16 * mt) * 2 * PANEL_GROUP <= 160 * 1024 ? 3 : 2; }
 
 // WAVES waves, 8 outputs each: a wave's 16 weight rows are the gate rows of its 8 outputs and then their up rows, so
 // that gate and up of an output meet in lanes 32 apart and no LDS pass is needed at the end. The launcher picks
@@ -598,7 +614,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_panel_swiglu_kernel(const bf1
                                                                        bf16_t* __restrict__ y, int M, int N, int K,
                                                                        GateAct act) {
   extern __shared__ __align__(16) unsigned char panel_lds[];
-  constexpr int STAGES = PANEL_STAGES;
+  constexpr int STAGES = panel_stages(MT, WAVES);
   constexpr int RB = 2 * PANEL_GROUP;                      // bytes of a row in a group
   constexpr int X_ALL = 4 * MT;                            // 1 KB pieces of x in a group, dealt to the waves in turn
   constexpr int X_LOADS = (X_ALL + WAVES - 1) / WAVES;     // every wave issues this many
@@ -634,7 +650,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_panel_swiglu_kernel(const bf1
     const unsigned char* xb = (const unsigned char*)x + (int64_t)gk * RB;
     const uint32_t at = lds0 + stage * STAGE_BYTES;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) panel_load16(wb, w_from[i], at + (16 * wave + 4 * i) * RB);
+    for (int i = 0; i < 4; ++i) panel_load16_once<true>(wb, w_from[i], at + (16 * wave + 4 * i) * RB);
 #pragma unroll
     for (int i = 0; i < X_LOADS; ++i) panel_load16(xb, x_from[i], at + W_BYTES + x_piece[i] * 1024);
   };
@@ -698,7 +714,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_panel_swiglu_kernel(const bf1
 template <int MT, int WAVES>
 static int launch_panel_swiglu(const void* x, int64_t x_stride, const void* w, void* y, int M, int N, int K,
                                hipStream_t stream, GateAct act) {
-  constexpr int lds = PANEL_STAGES * (16 * WAVES + 16 * MT) * 2 * PANEL_GROUP;
+  constexpr int lds = panel_stages(MT, WAVES) * (16 * WAVES + 16 * MT) * 2 * PANEL_GROUP;
   static_assert(lds <= 160 * 1024, "the stages must fit a compute unit's LDS");
   static bool raised = false;                              // more dynamic LDS than the default limit allows
   auto kernel = gemm_panel_swiglu_kernel<MT, WAVES>;
@@ -743,7 +759,7 @@ DRYFT_API int dryft_gemm_panel_waves(int N) {
   return best;
 }
 
-// M <= 64. y[M, N] = T(T(silu(x . Wg^T)) * (x . Wu^T)) with W = [Wg; Wu] of 2N rows (relu: T(max(x . Wg^T, 0) *
+// M <= 96. y[M, N] = T(T(silu(x . Wg^T)) * (x . Wu^T)) with W = [Wg; Wu] of 2N rows (relu: T(max(x . Wg^T, 0) *
 // (x . Wu^T))); K a multiple of 128; x and W
 // within reach of 32-bit byte offsets; waves: 4 to 8, or 0 for dryft_gemm_panel_waves' choice.
 static int panel_entry(const void* x, int64_t x_stride, const void* w, void* y, int M, int N, int K, int waves,
@@ -770,7 +786,7 @@ DRYFT_API int dryft_gemm_panel_glu_clamped_bf16(const void* x, int64_t x_stride,
 static int panel_entry(const void* x, int64_t x_stride, const void* w, void* y, int M, int N, int K, int waves,
                        GateAct act, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (M > 64 || K <= 0 || K % PANEL_GROUP || x_stride % 8 || (((uintptr_t)x | (uintptr_t)w) & 15) ||
+  if (M > PANEL_ROWS || K <= 0 || K % PANEL_GROUP || x_stride % 8 || (((uintptr_t)x | (uintptr_t)w) & 15) ||
       (int64_t)2 * N * K * 2 >= (int64_t)4 << 30 || (int64_t)M * x_stride * 2 >= (int64_t)4 << 30)
     return -1;
   if (waves == 0) waves = dryft_gemm_panel_waves(N);
@@ -778,7 +794,9 @@ static int panel_entry(const void* x, int64_t x_stride, const void* w, void* y, 
     case 1: return panel_waves<1>(x, x_stride, w, y, M, N, K, waves, stream, act);
     case 2: return panel_waves<2>(x, x_stride, w, y, M, N, K, waves, stream, act);
     case 3: return panel_waves<3>(x, x_stride, w, y, M, N, K, waves, stream, act);
-    default: return panel_waves<4>(x, x_stride, w, y, M, N, K, waves, stream, act);
+    case 4: return panel_waves<4>(x, x_stride, w, y, M, N, K, waves, stream, act);
+    case 5: return panel_waves<5>(x, x_stride, w, y, M, N, K, waves, stream, act);
+    default: return panel_waves<6>(x, x_stride, w, y, M, N, K, waves, stream, act);
   }
 }
 

@@ -1132,6 +1132,7 @@ def gemm_few_glu_bf16(x, w_gate_up, out, clamped: tuple[float, float] | None = N
     return out
 
 
+PANEL_ROWS = 96       # the most rows the panel kernel takes
 PANEL_GROUP = 128     # values of K the panel kernel moves at a time; K must be a multiple of it
 DIRECT_REACH = 1 << 32    # bytes: the kernels that bring operands straight into LDS address them by 32-bit offsets
 
@@ -1143,7 +1144,7 @@ def gemm_panel_waves(n_outputs: int) -> int:
 
 def gemm_panel_swiglu_bf16(x, w_gate_up, out, waves: int = 0, clamped: tuple[float, float] | None = None,
                            relu: bool = False) -> torch.Tensor:
-    """``silu(x @ Wg.T) * (x @ Wu.T)`` for ``w_gate_up = [Wg; Wu]``, at most 64 rows, by the kernel whose operands go
+    """``silu(x @ Wg.T) * (x @ Wu.T)`` for ``w_gate_up = [Wg; Wu]``, at most 96 rows, by the kernel whose operands go
     from memory straight into LDS. K must be a multiple of 128. ``waves`` (4 to 8, 8 outputs each) per workgroup;
     0 lets the library choose. ``clamped = (limit, alpha)``: the clamped gated unit in the epilogue instead,
     ``g * sigmoid(alpha * g) * (u + 1)`` with ``g = min(x @ Wg.T, limit)`` and ``u = clamp(x @ Wu.T, -limit, limit)``.
@@ -1157,8 +1158,8 @@ def gemm_panel_swiglu_bf16(x, w_gate_up, out, waves: int = 0, clamped: tuple[flo
     two_n = w_gate_up.shape[0]
     if not (two_n % 2 == 0 and w_gate_up.shape == (two_n, k) and w_gate_up.is_contiguous() and x.stride(1) == 1):
         raise KernelError("gemm_panel_swiglu: x [M,K] row-major, w [2N,K] contiguous")
-    if not (m <= 64 and k % PANEL_GROUP == 0 and x.stride(0) % 8 == 0):
-        raise KernelError(f"gemm_panel_swiglu: needs M <= 64 and K % {PANEL_GROUP} == 0, got M={m} K={k}")
+    if not (m <= PANEL_ROWS and k % PANEL_GROUP == 0 and x.stride(0) % 8 == 0):
+        raise KernelError(f"gemm_panel_swiglu: needs M <= {PANEL_ROWS} and K % {PANEL_GROUP} == 0, got M={m} K={k}")
     if not (x.data_ptr() % 16 == 0 and w_gate_up.data_ptr() % 16 == 0):
         raise KernelError("gemm_panel_swiglu: operands must be 16-byte aligned")
     if not (out.shape == (m, two_n // 2) and out.is_contiguous()):

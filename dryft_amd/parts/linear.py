@@ -13,7 +13,7 @@ engine/dryft_qwen3/model.py:153, 179-180, 237, 258-261). Here:
   matrix-core kernel, which stages whole cache lines through LDS and can leave its result
   as float32 partial sums over K for the consumer to add;
 * the gated units of feed-forwards at most 16 rows likewise (``ops.gemm_few_glu_ok``);
-* bfloat16, at most 64 rows, the fused gate/up product with its activation: this library's kernel that brings
+* bfloat16, at most 96 rows, the fused gate/up product with its activation: this library's kernel that brings
   its operands straight into LDS (``panel_swiglu_ok``; K a multiple of 128, else the two kernels below);
 * bfloat16, 33 to 64 rows, where the consumer adds partial sums (q/k/v of decoding steps, the projections back to
   the hidden width) and K is a multiple of 64: this library's kernel that splits K and brings its operands straight
@@ -24,7 +24,7 @@ engine/dryft_qwen3/model.py:153, 179-180, 237, 258-261). Here:
   for sizes the vendor library does not take;
 * bfloat16, 65 to 256 rows (short prompts, decoding at large batch) where the consumer adds partial sums and K is a
   multiple of 64: this library's kernel whose waves each own rows of x, operands straight into LDS (``tall_plan``);
-  the fused gate/up product of as many rows goes to its other form (``tall_swiglu_ok``), of more rows to this library's
+  the fused gate/up product of 97 to 256 rows goes to its other form (``tall_swiglu_ok``), of more rows to this library's
   kernel of 256 rows a workgroup where its rounds of workgroups are nearly full (``many_glu_ok``);
 * bfloat16, more than 16 rows, float32 results of at most 64 outputs (gates, routers, low-rank projections): this
   library's kernel that reads the rows once and splits K over the waves of a workgroup;
@@ -209,15 +209,19 @@ def few_rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 def panel_swiglu_ok(x: torch.Tensor, w_gate_up: torch.Tensor) -> bool:
     """Does the fused gate/up product with its activation go to the kernel that brings its operands straight into
-    LDS? Up to 64 rows, K a multiple of its group. In-graph times on rotating cold weights, us, against the
-    line-staging kernel (up to 16 rows) or the vendor library plus the activation kernel (more): Qwen3-4B's sizes
-    20.3 against 21.5 at 8 rows, 20.3 against 22.4 at 16, 21.2 against 26.8 at 24, 24.9 against 30.7 at 64;
-    Qwen3-8B's 36.7 against 37.8, 36.8 against 38.0, 37.6 against 52.1, 39.9 against 52.7; Qwen3-32B's 96.9 against
-    98.4, 95.0 against 103.8, 97.6 against 100.9, 107.8 against 110.4."""
+    LDS? K a multiple of its group, up to 64 rows, and up to 96 where the matrix is at most 384 MiB. In-graph times on
+    rotating cold weights, us, against the line-staging kernel (up to 16 rows) or the vendor library plus the activation
+    kernel (more), Qwen3-4B's sizes: 20.3 against 21.5 at 8 rows, 19.5 against 22.4 at 16 and 17, 20.2 against 27 at 32,
+    23.4 against 30.7 at 64; Qwen3-8B's 36.7 against 37.8, 35.9 against 38.0, 34.4 against 52, 38.2 against 52.7. At 65 to 96
+    rows against the kernel whose waves own rows of x (Qwen3-4B's 23.7 to 26.3 against 26.0 to 28.3, Qwen3-8B's 39 to 40.5
+    against 44 to 48) and the library (2 x 17,408 of 5,120, 340 MiB: 79.9 / 84.3 / 89.8 against 95.0 / 93.4 / 98.4 at 65 / 80 /
+    96 rows; 2 x 25,600 of 5,120, 500 MiB: 106.9 / 110.5 / 118.9 against 108.8 / 109.8 / 113.8, left to the library)."""
     m, k = x.shape
-    return m <= WIDE_ROWS and k % ops.PANEL_GROUP == 0 and few_rows_ok(x, w_gate_up) and within_direct_reach(x, w_gate_up)
+    return (m <= WIDE_ROWS or (m <= ops.PANEL_ROWS and w_gate_up.numel() * w_gate_up.element_size() <= _PANEL_BYTES)) and \
+        k % ops.PANEL_GROUP == 0 and few_rows_ok(x, w_gate_up) and within_direct_reach(x, w_gate_up)
 
 
+_PANEL_BYTES = 384 << 20        # gate/up matrices up to here go there at 65 to 96 rows too
 _TALL_SMALL_BYTES = 128 << 20   # matrices from here on go to the kernel whose waves own rows of x already at 33 to 64 rows.
 # Whole decoding steps, ms, against the shared-activation kernel or the vendor library there: Qwen3-14B (down, 178 MB) 10.99
 # against 11.19 at 64 sequences, the same at 48. With every matrix beyond 48 MiB sent there Qwen3-14B gains more (10.89; 9.97

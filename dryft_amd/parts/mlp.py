@@ -52,7 +52,7 @@ class SwiGLU(FeedForward):
         elif h.dtype == torch.bfloat16 and panel_swiglu_ok(h, self.w_gate_up):
             ops.gemm_panel_swiglu_bf16(h, self.w_gate_up, act, relu=self.relu)        # product and activation in one kernel
         elif h.dtype == torch.bfloat16 and tall_swiglu_ok(h, self.w_gate_up):
-            ops.gemm_tall_swiglu_bf16(h, self.w_gate_up, act, relu=self.relu)         # the same at 65 to 256 rows
+            ops.gemm_tall_swiglu_bf16(h, self.w_gate_up, act, relu=self.relu)         # the same at more rows, up to 256
         elif h.dtype == torch.bfloat16 and many_glu_ok(h, self.w_gate_up):
             ops.gemm_many_glu_bf16(h, self.w_gate_up, act, relu=self.relu)     # and beyond
         elif self.relu:
@@ -100,7 +100,7 @@ class ClampedGLU(FeedForward):
         if h.dtype == torch.bfloat16 and ops.gemm_few_glu_ok(h, self.w_gate_up):
             ops.gemm_few_glu_bf16(h, self.w_gate_up, act, clamped=(self.limit, self.alpha))
         elif h.dtype == torch.bfloat16 and panel_swiglu_ok(h, self.w_gate_up):
-            # up to 64 rows: product and unit in one kernel, the unit on the float accumulators
+            # up to 64 or 96 rows: product and unit in one kernel, the unit on the float accumulators
             ops.gemm_panel_swiglu_bf16(h, self.w_gate_up, act, clamped=(self.limit, self.alpha))
         elif h.dtype == torch.bfloat16 and many_glu_ok(h, self.w_gate_up):
             ops.gemm_many_glu_bf16(h, self.w_gate_up, act, clamped=(self.limit, self.alpha))

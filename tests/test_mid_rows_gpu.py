@@ -1,0 +1,34 @@
+"""Products of 17 to 128 rows whose operands go straight into LDS, at the edges of their tiles of rows and of outputs."""
+
+import math
+
+import pytest
+import torch
+
+from test_kernels_gpu import close
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("m", [65, 80, 81, 96])
+@pytest.mark.parametrize("inter,k,waves", [(47, 128, 0), (100, 640, 5), (136, 256, 8), (1024, 2560, 4)])
+@pytest.mark.parametrize("unit", ["silu", "relu", "clamped"])
+def test_panel_of_up_to_96_rows(m, inter, k, waves, unit):
+    """Five and six tiles of rows, three stages in LDS and (eight waves at 96 rows) two; rows of x wider apart than K."""
+    from dryft_amd.csrc import ops
+    torch.manual_seed(m + inter + k)
+    x = torch.randn(m, k + 8).to(torch.bfloat16)
+    w = (torch.randn(2 * inter, k) * 2 / math.sqrt(k)).to(torch.bfloat16)
+    gu = x[:, :k].double() @ w.double().T
+    if unit == "silu":                                          # the product and silu are rounded first
+        gu = gu.to(torch.bfloat16).double()
+        want = torch.nn.functional.silu(gu[:, :inter]).to(torch.bfloat16).double() * gu[:, inter:]
+    elif unit == "relu":
+        want = gu[:, :inter].clamp(min=0) * gu[:, inter:]
+    else:
+        g, u = gu[:, :inter].clamp(max=1.5), gu[:, inter:].clamp(-1.5, 1.5)
+        want = g * torch.sigmoid(1.702 * g) * (u + 1)
+    out = torch.full((m, inter), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.gemm_panel_swiglu_bf16(x.to(DEV)[:, :k], w.to(DEV), out, waves, (1.5, 1.702) if unit == "clamped" else None, unit == "relu")
+    close(out, want, torch.bfloat16, ulps=4.0, what=f"panel, {unit}")        # a rounding of each factor, and its own
