@@ -7,7 +7,7 @@
 //  * gemm_stream (M <= 16) and gemm_wide (M <= 64): bfloat16, few rows (decoding, output head): every
 //    weight is read once and multiplied on the matrix cores; K may be split across workgroups into
 //    float partial sums that the consumer adds in a fixed order. gemm_panel (M <= 96) is the fused gate/up
-//    product, gemm_mid (M <= 256) the projections back to the hidden width for short prompts.
+//    product, gemm_mid (17 to 128 rows) the others of decoding at larger batch and of short prompts.
 #include "gate_unit.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
@@ -801,30 +801,32 @@ static int panel_entry(const void* x, int64_t x_stride, const void* w, void* y, 
 }
 
 // --------------------------------------------------------------------------------------------- mid
-// The projections back to the hidden width (few outputs, a long K) for short prompts, 65 to 256 rows: there the
-// vendor library takes 20 to 50 us for matrices that stream in 4 to 10 (Qwen3-4B: o 20 to 25 us, down 27 to 53),
-// because its tiles are too few for the chip. Here a workgroup of four waves owns 64 outputs (16 rows of W a wave)
-// and all rows of x, K is split over workgroups into float partial sums that the consumer adds in a fixed order,
-// and the operands go from memory straight into LDS as in the panel product (groups of 64 values of K: rows of
-// 128 bytes, piece p of row r at place p ^ ((r / 2) % 8); three groups in LDS; a wave fetches its own 16 rows of W
-// and its share of the rows of x; every workgroup walks its part of K from a starting group of its own). Every
-// workgroup reads all of x (from L2), which is why this form stops paying at about 250 rows and never pays for the
-// products with many outputs (q/k/v, gate/up). Measured, weights from memory, us at 80 / 128 / 192 rows against the
-// vendor library: Qwen3-4B's o 10.9 / 12.8 / 17.3 (21 / 25 / 19), down 19.1 / 21.0 / 28.5 (27 / 53 / 34); Qwen3-8B's o
-// 13.5 / 15.4 / 20.6 (21 / 25 / 34), down 29 / 38 / 53 (38 / 67 / 90); Qwen3-32B's o 26 / 29 / 39 (30 / 45 / 61), down
-// 72 / 88 / 111 (173 / 181 / 209). Since the tall product below took the steps of 65 to 256 rows (its workgroups take
-// in fewer bytes of x for a row of W), this one serves those of 33 to 64 rows.
+// Products of 17 to 128 rows. A workgroup owns 16 rows of W a wave (WAVES 4, 5, 6 or 8) and all rows of x; K may be split over
+// workgroups into float partial sums that the consumer adds in a fixed order; the operands go from memory straight into
+// LDS as in the panel product (groups of 64 values of K: rows of 128 bytes, piece p of row r at place p ^ ((r / 2) % 8);
+// a wave fetches its own 16 rows of W and its share of the rows of x; every workgroup walks its part of K from a starting
+// group of its own).
+// Bound by what a compute unit takes in (some 35 KB a microsecond of weights from memory and rows of x from the L2 together)
+// and by the ends of the launch. So the rows of W a workgroup and the runs of K are chosen together (`mid_plan`, linear.py), to
+// give each compute unit one workgroup that takes in the fewest bytes; with 64 rows of W whatever the sizes and three stages it
+// was, us at 64 rows: 6,144 x 2,560 11.6, 2,560 x 9,728 14.4, 6,144 x 4,096 16.1 (two stages, gemm_wide), now 10.0, 12.9, 12.2.
+// Four groups of K in LDS: with three the bytes on their way do not cover the trip to memory (2,560 x 9,728 at 24 rows 14.5, four
+// 11.5, five 11.4, eight 12.1); beyond 64 rows three, as a group is larger. Weights are read as lines not kept (nt) where the L2 is
+// short: matrices of 40 MiB on at any number of rows (4,096 x 12,288 at 64 24.0 / 22.0), from 8 MiB on up to 32 rows (2,560 x
+// 9,728 at 17 11.9 / 11.3, 4,096 x 4,096 8.1 / 7.7); else they are a little slower (6,144 x 2,560 at 64 11.8 / 12.2).
+// Whole products with more workgroups than units (the output head) run two or three on a unit: there two stages from 49 rows on
+// and three below leave the room, and nt. 151,936 x 2,560 at 17 / 64 / 96 rows 143 / 176 / 197 (gemm_wide and, beyond 64 rows,
+// gemm_block 158 / 207 / 294), 65,536 x 2,048 48 / 53 / 56 (65 / 70 / 84), 151,936 x 1,024 at 64 69 (94).
+// Operands in the matrix cores' layout straight from memory into registers, without LDS, 16 rows of 64 bytes a load: 1.4 to 1.8
+// times as long (a compute unit looks up a line, or half of one, every 8 cycles or so); K over the waves too, with one
+// sum at the end: the same.
 #define MID_GROUP 64
-#define MID_STAGES 3
-#define MID_WAVES 4
 
-template <int MT>
-__global__ __launch_bounds__(64 * MID_WAVES) void gemm_mid_kernel(const bf16_t* __restrict__ x, int64_t x_stride,
-                                                                  const bf16_t* __restrict__ w,
-                                                                  float* __restrict__ partials, int M, int N, int K,
-                                                                  int groups_per_split) {
+template <int MT, int WAVES, int STAGES, bool ONCE>
+__global__ __launch_bounds__(64 * WAVES) void gemm_mid_kernel(const bf16_t* __restrict__ x, int64_t x_stride,
+                                                              const bf16_t* __restrict__ w, float* __restrict__ partials,
+                                                              int M, int N, int K, int groups_per_split) {
   extern __shared__ __align__(16) unsigned char mid_lds[];
-  constexpr int STAGES = MID_STAGES, WAVES = MID_WAVES;
   constexpr int RB = 2 * MID_GROUP;                        // bytes of a row in a group
   constexpr int X_ALL = 2 * MT;                            // 1 KB pieces (8 rows) of x in a group
   constexpr int X_LOADS = (X_ALL + WAVES - 1) / WAVES;     // every wave issues this many
@@ -857,7 +859,7 @@ __global__ __launch_bounds__(64 * MID_WAVES) void gemm_mid_kernel(const bf16_t* 
     const unsigned char* xb = (const unsigned char*)x + (int64_t)gk * RB;
     const uint32_t at = lds0 + stage * STAGE_BYTES;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) panel_load16(wb, w_from[i], at + (16 * wave + 8 * i) * RB);
+    for (int i = 0; i < 2; ++i) panel_load16_once<ONCE>(wb, w_from[i], at + (16 * wave + 8 * i) * RB);
 #pragma unroll
     for (int i = 0; i < X_LOADS; ++i) panel_load16(xb, x_from[i], at + W_BYTES + x_piece[i] * 1024);
   };
@@ -915,40 +917,68 @@ __global__ __launch_bounds__(64 * MID_WAVES) void gemm_mid_kernel(const bf16_t* 
   }
 }
 
-template <int MT>
+template <int MT, int WAVES, int STAGES, bool ONCE>
 static int launch_mid(const void* x, int64_t x_stride, const void* w, float* partials, int M, int N, int K, int splits,
-                      int groups_per_split, hipStream_t stream) {
-  constexpr int lds = MID_STAGES * (16 * MID_WAVES + 16 * MT) * 2 * MID_GROUP;
+                      hipStream_t stream) {
+  constexpr int lds = STAGES * (16 * WAVES + 16 * MT) * 2 * MID_GROUP;
   static_assert(lds <= 160 * 1024, "the stages must fit a compute unit's LDS");
   static bool raised = false;                              // more dynamic LDS than the default limit allows
-  auto kernel = gemm_mid_kernel<MT>;
+  auto kernel = gemm_mid_kernel<MT, WAVES, STAGES, ONCE>;
   if (lds > 64 * 1024 && !raised) {
     if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return -2;
     raised = true;
   }
-  dim3 grid((N + 16 * MID_WAVES - 1) / (16 * MID_WAVES), splits), block(64 * MID_WAVES);
+  const int groups = K / MID_GROUP;
+  dim3 grid((N + 16 * WAVES - 1) / (16 * WAVES), splits), block(64 * WAVES);
   hipLaunchKernelGGL(kernel, grid, block, lds, stream, (const bf16_t*)x, x_stride, (const bf16_t*)w, partials, M, N, K,
-                     groups_per_split);
+                     (groups + splits - 1) / splits);
   return DRYFT_LAUNCH_CHECK();
 }
 
-// M <= 256. partials[splits, M, N] = float partial sums of x . W^T over `splits` equal runs of groups of 64 values of K
-// (the last run may be shorter, none may be empty); K a multiple of 64; x and W within reach of 32-bit byte offsets.
+template <int MT, int WAVES>
+static int mid_stages(const void* x, int64_t x_stride, const void* w, float* partials, int M, int N, int K, int splits,
+                      hipStream_t stream) {
+  const int64_t bytes = (int64_t)N * K * 2;
+  const bool once = bytes >= (40 << 20) || (M <= 32 && bytes >= (8 << 20));
+  constexpr int ONE_EACH = MT <= 4 ? 4 : 3, SEVERAL = MT <= 3 ? 3 : 2;
+  if ((int64_t)((N + 16 * WAVES - 1) / (16 * WAVES)) * splits > 256)
+    return launch_mid<MT, WAVES, SEVERAL, true>(x, x_stride, w, partials, M, N, K, splits, stream);
+  if (once) return launch_mid<MT, WAVES, ONE_EACH, true>(x, x_stride, w, partials, M, N, K, splits, stream);
+  return launch_mid<MT, WAVES, ONE_EACH, false>(x, x_stride, w, partials, M, N, K, splits, stream);
+}
+
+template <int MT>
+static int mid_waves(const void* x, int64_t x_stride, const void* w, float* partials, int M, int N, int K, int splits,
+                     int waves, hipStream_t stream) {
+  switch (waves) {
+    case 4: return mid_stages<MT, 4>(x, x_stride, w, partials, M, N, K, splits, stream);
+    case 5: return mid_stages<MT, 5>(x, x_stride, w, partials, M, N, K, splits, stream);
+    case 6: return mid_stages<MT, 6>(x, x_stride, w, partials, M, N, K, splits, stream);
+    case 8: return mid_stages<MT, 8>(x, x_stride, w, partials, M, N, K, splits, stream);
+    default: return -1;
+  }
+}
+
+// M <= 256 (beyond 128 four waves only). partials[splits, M, N] = float partial sums of x . W^T over `splits` equal runs of groups
+// of 64 values of K (the last run may be shorter, none may be empty); a workgroup owns 16 `waves` outputs (4, 5, 6 or 8 waves); K a
+// multiple of 64; x and W within reach of 32-bit byte offsets.
 DRYFT_API int dryft_gemm_mid_bf16(const void* x, int64_t x_stride, const void* w, float* partials, int M, int N, int K,
-                                  int splits, hipStream_t stream) {
+                                  int splits, int waves, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   if (M > 256 || K <= 0 || K % MID_GROUP || splits < 1 || x_stride % 8 || (((uintptr_t)x | (uintptr_t)w) & 15) ||
       ((uintptr_t)partials & 15) || (int64_t)N * K * 2 >= (int64_t)4 << 30 || (int64_t)M * x_stride * 2 >= (int64_t)4 << 30)
     return -1;
   const int groups = K / MID_GROUP, per = (groups + splits - 1) / splits;
   if ((groups + per - 1) / per != splits) return -1;       // a run would be empty
-  if (M <= 32) return launch_mid<2>(x, x_stride, w, partials, M, N, K, splits, per, stream);
-  if (M <= 48) return launch_mid<3>(x, x_stride, w, partials, M, N, K, splits, per, stream);
-  if (M <= 64) return launch_mid<4>(x, x_stride, w, partials, M, N, K, splits, per, stream);
-  if (M <= 96) return launch_mid<6>(x, x_stride, w, partials, M, N, K, splits, per, stream);
-  if (M <= 128) return launch_mid<8>(x, x_stride, w, partials, M, N, K, splits, per, stream);
-  if (M <= 192) return launch_mid<12>(x, x_stride, w, partials, M, N, K, splits, per, stream);
-  return launch_mid<16>(x, x_stride, w, partials, M, N, K, splits, per, stream);
+  if (M <= 32) return mid_waves<2>(x, x_stride, w, partials, M, N, K, splits, waves, stream);
+  if (M <= 48) return mid_waves<3>(x, x_stride, w, partials, M, N, K, splits, waves, stream);
+  if (M <= 64) return mid_waves<4>(x, x_stride, w, partials, M, N, K, splits, waves, stream);
+  if (M <= 80) return mid_waves<5>(x, x_stride, w, partials, M, N, K, splits, waves, stream);
+  if (M <= 96) return mid_waves<6>(x, x_stride, w, partials, M, N, K, splits, waves, stream);
+  if (M <= 128) return mid_waves<8>(x, x_stride, w, partials, M, N, K, splits, waves, stream);
+  if (waves != 4) return -1;
+  if (M <= 192) return launch_mid<12, 4, 3, false>(x, x_stride, w, partials, M, N, K, splits, stream);
+  return launch_mid<16, 4, 3, false>(x, x_stride, w, partials, M, N, K, splits, stream);
 }
 
 // -------------------------------------------------------------------------------------------- tall

@@ -97,7 +97,7 @@ _SIGNATURES = {
              "dryft_gemm_tall_swiglu_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _P],
              "dryft_gemm_tall_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _P],
              "dryft_gemm_tall_tiles": [_I],
-             "dryft_gemm_mid_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _P],
+             "dryft_gemm_mid_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _P],
              "dryft_gemm_block_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _I, _P],
              "dryft_gemm_block_f32": [_P, _L, _P, _P, _I, _I, _I, _I, _P],
              "dryft_gemm_wide_swiglu_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _P],
@@ -1262,6 +1262,8 @@ def gemm_tall_bf16(x, w, partials, splits: int, tiles: int) -> torch.Tensor:
 
 
 MID_ROWS = 256      # the most rows gemm_mid takes
+MID_MOST = 128      # the most it takes with other than 4 waves
+MID_WAVES = (4, 5, 6, 8)
 MID_GROUP = 64      # values of K it walks at a time; K must be a multiple, and the splits are runs of such groups
 
 
@@ -1274,10 +1276,10 @@ def gemm_mid_splits(k: int, splits: int) -> int:
     return splits
 
 
-def gemm_mid_bf16(x, w, partials, splits: int) -> torch.Tensor:
+def gemm_mid_bf16(x, w, partials, splits: int, waves: int = 4) -> torch.Tensor:
     """Float partial sums ``partials[splits, M, N]`` of ``x @ w.T`` over ``splits`` runs of K, for 1 to 256 rows, by the
     kernel whose operands go from memory straight into LDS. K must be a multiple of 64 and ``splits`` one that
-    ``gemm_mid_splits`` returns."""
+    ``gemm_mid_splits`` returns; a workgroup owns ``16 * waves`` outputs (4, 5, 6 or 8 waves; beyond 128 rows 4)."""
     _gpu(x, "x", torch.bfloat16)
     _gpu(w, "w", torch.bfloat16)
     _gpu(partials, "partials", torch.float32)
@@ -1293,8 +1295,10 @@ def gemm_mid_bf16(x, w, partials, splits: int) -> torch.Tensor:
         raise KernelError(f"gemm_mid: {splits} splits would leave a run of K = {k} empty")
     if not (partials.shape == (splits, m, n) and partials.is_contiguous()):
         raise KernelError(f"gemm_mid: partials must be [{splits},{m},{n}]")
+    if not (waves in MID_WAVES and (m <= MID_MOST or waves == 4)):
+        raise KernelError(f"gemm_mid: waves 4, 5, 6 or 8, beyond {MID_MOST} rows 4")
     _check(_fn("gemm", "dryft_gemm_mid_bf16")(_ptr(x), x.stride(0), _ptr(w), _ptr(partials), m, n, k, int(splits),
-                                              _stream()), "gemm_mid_bf16")
+                                              int(waves), _stream()), "gemm_mid_bf16")
     return partials
 
 

@@ -15,15 +15,13 @@ engine/dryft_qwen3/model.py:153, 179-180, 237, 258-261). Here:
 * the gated units of feed-forwards at most 16 rows likewise (``ops.gemm_few_glu_ok``);
 * bfloat16, at most 96 rows, the fused gate/up product with its activation: this library's kernel that brings
   its operands straight into LDS (``panel_swiglu_ok``; K a multiple of 128, else the two kernels below);
-* bfloat16, 33 to 64 rows, where the consumer adds partial sums (q/k/v of decoding steps, the projections back to
-  the hidden width) and K is a multiple of 64: this library's kernel that splits K and brings its operands straight
-  into LDS (``small_mid_plan``);
-* bfloat16, 17 to 64 rows otherwise: this library's shared-activation kernel where the consumer adds
-  partial sums (the projections back to the hidden width, which give the vendor library too
-  few tiles to fill the chip), where the result is wanted in float32 (the output head) and
-  for sizes the vendor library does not take;
-* bfloat16, 65 to 256 rows (short prompts, decoding at large batch) where the consumer adds partial sums and K is a
-  multiple of 64: this library's kernel whose waves each own rows of x, operands straight into LDS (``tall_plan``);
+* bfloat16, 17 to 128 rows, where the consumer adds partial sums (q/k/v of decoding steps and short prompts, the projections
+  back to the hidden width) or the result is wanted in float32 (the output head), K a multiple of 64: this library's kernel
+  that brings its operands straight into LDS, K split over workgroups (``mid_plan``);
+* bfloat16, 17 to 64 rows, such products of other K, and sizes the vendor library does not take: this library's
+  shared-activation kernel;
+* bfloat16, 129 to 256 rows (short prompts, decoding at large batch; large matrices from 65) where the consumer adds partial sums
+  and K is a multiple of 64: this library's kernel whose waves each own rows of x, operands straight into LDS (``tall_plan``);
   the fused gate/up product of 97 to 256 rows goes to its other form (``tall_swiglu_ok``), of more rows to this library's
   kernel of 256 rows a workgroup where its rounds of workgroups are nearly full (``many_glu_ok``);
 * bfloat16, more than 16 rows, float32 results of at most 64 outputs (gates, routers, low-rank projections): this
@@ -49,8 +47,7 @@ from .base import Partials
 
 STREAM_ROWS = 16                # the most rows the line-staging kernel takes; up to here it beats the vendor library
 WIDE_ROWS = 64                  # the most rows the shared-activation kernel takes
-_SMALL_MID_BYTES = 48 << 20     # the largest matrix that goes there
-SMALL_MID_ROWS = 32             # above so many rows (and up to WIDE_ROWS) split products go to the direct-to-LDS kernel
+_SMALL_MID_BYTES = 48 << 20     # the largest matrix for which workgroups of 64 outputs come into question
 _STREAM_BLOCKS_PER_WAVE = 5     # measured on the projection shapes of 4B to 32B models inside captured graphs:
 _STREAM_WORKGROUPS = 1536       # short walks over K, as long as the launch stays under about six workgroups a unit
 _COMPUTE_UNITS = 256            # of the MI355X
@@ -189,17 +186,54 @@ def _tall_plan(loaded: int, n: int, k: int) -> tuple[int, int]:
 
 
 def small_mid_plan(n: int, k: int) -> int:
-    """Splits of K across workgroups for the kernel that brings its operands straight into LDS, at 33 to 64 rows (64
-    outputs a workgroup): as many as give every compute unit one workgroup; 1 where the product stays with the
-    shared-activation kernel or the vendor library. Measured alone in a captured graph at 64 rows, us, against the
-    better of those two: Qwen3-4B's q/k/v 11.7 (13.7), o 8.1 (10.2), down 14.3 (15.6); Qwen3-8B's 16.0 (17.8), 9.9 (11.6),
-    23.3 (25.5); and a decoding step of 64 sequences with it 6.28 against 6.50 ms (Qwen3-4B), 7.58 against 7.71
-    (Qwen3-8B). On larger matrices the same kernel is ahead alone (Qwen3-14B's q/k/v 20.5 against 25.0) and behind in
-    the step (11.27 against 11.18 ms; Qwen3-32B 21.9 against 21.5), so matrices beyond 48 MiB stay where they were."""
+    """Splits of K that give every compute unit one workgroup of 64 outputs: what ``mid_plan`` weighs wider workgroups
+    against. 1 beyond 48 MiB, where those are always ahead."""
     if n * k * 2 > _SMALL_MID_BYTES:
         return 1
     blocks = (n + 63) // 64
     return ops.gemm_mid_splits(k, max(1, min(16, _COMPUTE_UNITS // blocks)))
+
+
+def mid_pays(m: int, n: int, k: int, may_split: bool) -> bool:
+    """Does a product of 17 to 128 rows go to the kernel of ``mid_plan``, or beyond 64 rows to the one whose waves own rows of x? To
+    the first, but for split products of large matrices (5,120 x 25,600, 250 MiB, at 77 / 96 / 128 rows 59 / 69 / 80 us against
+    54 / 58 / 63; 5,120 x 17,408, 170 MiB, 36 / 38 / 42 against 38 / 40 / 43) and beyond 96 rows of small ones, whose partial sums
+    weigh more than they (steps of 128 sequences through Qwen3-0.6B, 4 to 8 MiB, 2,295 against 2,284 us; Qwen3-4B's, 12 layers,
+    20 MiB on, 1,707 against 1,812)."""
+    size = n * k * 2
+    return m <= WIDE_ROWS or not may_split or (size <= 192 << 20 and (m <= 96 or size >= 16 << 20))
+
+
+def mid_plan(m: int, n: int, k: int, may_split: bool) -> tuple[int, int]:
+    return _mid_plan(-(-m // 16) if m <= 96 else 8, n, k, may_split)
+
+
+@functools.lru_cache(maxsize=1024)
+def _mid_plan(tiles: int, n: int, k: int, may_split: bool) -> tuple[int, int]:
+    """(waves of 16 outputs a workgroup, splits of K across workgroups) for the kernel that brings its operands straight into
+    LDS, with ``tiles`` of 16 rows of x: the pair with the lowest modelled time, in us: 3 + rounds * (30 * MB of W a workgroup
+    takes in + 10 * MB of x it takes in) + 0.6 * MB of partial sums, rounds being how often the workgroups fill the compute
+    units. Fitted to times in a captured chain on rotating cold weights of 19 sizes (1,024 x 1,024 to 5,120 x 25,600) at
+    17 to 128 rows, where partial sums count 0.3; its choice is there within 3 % of the best pair on average (worst 12 %), and
+    14 % ahead of what served these sizes before. The kernel that adds them up on its way in counts for the rest: steps of 64
+    / 96 sequences through Qwen3-0.6B 1,587 / 2,032 us with 0.3, 1,558 / 1,982 with 0.6, 1,555 / 1,972 with 0.8, of 128 through
+    Qwen3-4B (12 layers) 1,732, 1,707 and 1,716. Against ``gemm_wide`` at 17 to 32 rows, 64 rows a workgroup and three stages at 33 to
+    64, and ``gemm_tall`` beyond, us: 6,144 x 2,560 at 17 / 32 / 64 / 96 rows 8.2 / 8.7 / 10.0 / 11.5 (10.2 / 10.9 / 11.7 / 13.2),
+    2,560 x 9,728 10.5 / 11.1 / 12.8 / 14.7 (13.1 / 12.9 / 14.5 / 15.7), 4,096 x 1,024 4.0 / 4.2 / 5.0 / 5.7 (5.3 / 5.8 / 5.0 / 7.0),
+    10,240 x 5,120 19.7 / 21.0 / 23.8 / 26.2 (36.6 / 35.5 / 42.2 / 27.5)."""
+    groups = k // ops.MID_GROUP
+    best, best_cost = (4, 1), float("inf")
+    for waves in ops.MID_WAVES:
+        blocks = -(-n // (16 * waves))
+        wants = (1,) if not may_split else (small_mid_plan(n, k),) if waves == 4 else range(1, min(groups, 16) + 1)
+        for splits in {ops.gemm_mid_splits(k, want) for want in wants}:
+            rounds = -(-(blocks * splits) // _COMPUTE_UNITS)
+            if splits > 1 and rounds > 1:
+                continue
+            cost = rounds * 16 * (30 * waves + 10 * tiles) * -(-groups // splits) * 128e-6 + 0.6e-6 * splits * 16 * tiles * n * 4
+            if cost < best_cost:
+                best, best_cost = (waves, splits), cost
+    return best
 
 
 def few_rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -222,11 +256,6 @@ def panel_swiglu_ok(x: torch.Tensor, w_gate_up: torch.Tensor) -> bool:
 
 
 _PANEL_BYTES = 384 << 20        # gate/up matrices up to here go there at 65 to 96 rows too
-_TALL_SMALL_BYTES = 128 << 20   # matrices from here on go to the kernel whose waves own rows of x already at 33 to 64 rows.
-# Whole decoding steps, ms, against the shared-activation kernel or the vendor library there: Qwen3-14B (down, 178 MB) 10.99
-# against 11.19 at 64 sequences, the same at 48. With every matrix beyond 48 MiB sent there Qwen3-14B gains more (10.89; 9.97
-# against 10.09 at 48), Qwen3-32B a little (20.35 against 20.63; 19.01 against 19.10), and Qwen3-8B (q/k/v 50 MB, down 100 MB)
-# loses (7.60 against 7.54 at 64), though each of its products alone is faster: so only the large ones.
 _TALL_SWIGLU_BYTES = 256 << 20  # gate/up matrices up to here go to the kernel whose waves own rows of x at 65 to 256 rows
 
 
@@ -329,18 +358,12 @@ def linear(x: torch.Tensor, w: torch.Tensor, *, out_dtype: torch.dtype | None = 
         out = torch.empty((m, n), dtype=out_dtype, device=x.device)
         ops.gemm_stream_bf16(x, w, out, None, group, 1, depth)
         return out
-    if SMALL_MID_ROWS < m <= WIDE_ROWS and allow_partials and few_ok and k % ops.MID_GROUP == 0 and \
-            within_direct_reach(x, w):
-        splits = small_mid_plan(n, k)
-        if splits > 1:
-            partials = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
-            ops.gemm_mid_bf16(x, w, partials, splits)
-            return Partials(partials, splits)
-        if n * k * 2 >= _TALL_SMALL_BYTES:
-            tiles, splits = tall_plan(m, n, k)
-            partials = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
-            ops.gemm_tall_bf16(x, w, partials, splits, tiles)
-            return Partials(partials, splits)
+    if m <= ops.MID_MOST and (allow_partials or out_dtype == torch.float32) and few_ok and k % ops.MID_GROUP == 0 and \
+            within_direct_reach(x, w) and mid_pays(m, n, k, allow_partials):
+        waves, splits = mid_plan(m, n, k, allow_partials)
+        partials = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
+        ops.gemm_mid_bf16(x, w, partials, splits, waves)
+        return Partials(partials, splits) if allow_partials else partials[0]
     if m <= WIDE_ROWS and few_ok:
         splits, group, depth = wide_plan(n, k, allow_partials)
         if splits > 1:

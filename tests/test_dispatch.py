@@ -125,3 +125,15 @@ def test_every_entry_point_is_called_with_as_many_arguments_as_it_declares():
             assert name in declared, f"{module}.hip declares no {name}"
             count = len([a for a in declared[name].split(",") if a.strip()])
             assert count == len(signature), f"{name}: declared with {count} arguments, called with {len(signature)}"
+
+
+@pytest.mark.parametrize("rows", [17, 32, 33, 64, 65, 96, 97, 128])
+@pytest.mark.parametrize("n,k", [(6144, 2560), (2560, 9728), (1024, 64), (5120, 17408), (151936, 1024), (96, 4096)])
+def test_products_of_17_to_128_rows_fill_the_units_once(rows, n, k):
+    """A plan that splits K leaves no run empty and needs one round of workgroups; a whole product has one run."""
+    from dryft_amd.csrc import ops
+    from dryft_amd.parts.linear import mid_plan
+    waves, splits = mid_plan(rows, n, k, True)
+    assert waves in ops.MID_WAVES and ops.gemm_mid_splits(k, splits) == splits
+    assert splits == 1 or -(-n // (16 * waves)) * splits <= 256
+    assert mid_plan(rows, n, k, False)[1] == 1

@@ -32,3 +32,21 @@ def test_panel_of_up_to_96_rows(m, inter, k, waves, unit):
     out = torch.full((m, inter), float("nan"), dtype=torch.bfloat16, device=DEV)
     ops.gemm_panel_swiglu_bf16(x.to(DEV)[:, :k], w.to(DEV), out, waves, (1.5, 1.702) if unit == "clamped" else None, unit == "relu")
     close(out, want, torch.bfloat16, ulps=4.0, what=f"panel, {unit}")        # a rounding of each factor, and its own
+
+
+@pytest.mark.parametrize("m", [17, 33, 64, 65, 81, 97, 128])
+@pytest.mark.parametrize("n,k,waves,splits", [(77, 64, 5, 1), (97, 320, 6, 5), (100, 192, 8, 3), (2560, 1664, 5, 7),
+                                              (33000, 128, 8, 1), (20500, 192, 4, 1), (4200, 1024, 4, 4), (2056, 2048, 8, 16)])
+def test_products_of_17_to_128_rows(m, n, k, waves, splits):
+    """Every width of a workgroup, runs of K of one group and of unequal length, weights kept and read once, launches of more
+    workgroups than compute units (two stages in LDS); a row of x wider than K."""
+    from dryft_amd.csrc import ops
+    torch.manual_seed(m + n + k)
+    x, w = torch.randn(m, k + 8).to(torch.bfloat16).to(DEV)[:, :k], (torch.randn(n, k) / math.sqrt(k)).to(torch.bfloat16).to(DEV)
+    assert ops.gemm_mid_splits(k, splits) == splits
+    parts = torch.full((splits, m, n), float("nan"), dtype=torch.float32, device=DEV)
+    ops.gemm_mid_bf16(x, w, parts, splits, waves)
+    per = -(-(k // 64) // splits)
+    for s in range(splits):
+        a, b = 64 * per * s, min(k, 64 * per * (s + 1))
+        close(parts[s], x[:, a:b].double() @ w[:, a:b].double().T, torch.float32, what=f"run {s}")
