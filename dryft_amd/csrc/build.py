@@ -29,7 +29,7 @@ MODULES = ("batch", "embed", "norm", "activation", "rope_kv", "attn_rows", "attn
            "gemm_lines", "gemm_f32", "sampling", "mlstm",
            "rglru", "hyper", "wkv", "latent", "moe", "conv", "ssm", "delta", "linattn", "mla")
 _HEADERS = ("common.h",)                       # every library includes these
-_OWN_HEADERS = {"gemm": ("gate_unit.h",), "gemm_lines": ("gate_unit.h",), "sampling": ("sampling.h",),
+_OWN_HEADERS = {"gemm": ("gate_unit.h",), "gemm_lines": ("gate_unit.h",), "moe": ("gate_unit.h",), "sampling": ("sampling.h",),
                 "delta": ("chunk_walk.h",), "ssm": ("chunk_walk.h",)}    # and some a header of their own
 
 _loaded: dict[str, ctypes.CDLL] = {}

@@ -1,7 +1,7 @@
 // Routed experts on the device: the router's choice, the sort of (row, expert) pairs by expert, the grouped
 // products over each expert's rows, and the weighted sum per row. No step of it needs the host, so a step that
 // holds it can be captured.
-#include "common.h"
+#include "gate_unit.h"
 
 #define MOE_MAX_EXPERTS 512
 #define MOE_PER_LANE (MOE_MAX_EXPERTS / WAVE)
@@ -583,116 +583,195 @@ __global__ __launch_bounds__(256) void moe_product_mfma_kernel(const bf16_t* __r
   }
 }
 
-// For steps of few rows (decoding), where a tile holds at most 16 places. A workgroup takes 16 outputs of a tile (for
-// the gated unit 16 gate rows and their 16 up rows) and its WAVES waves split K in runs of whole blocks of 64, with the
-// operand rows straight from memory (they are few and stay in the vector cache) and four blocks in flight; the waves'
-// sums meet in LDS and are added in the order 0, 1, .... What bounds it is the trip to memory, not the 2 to 17 MB that a
-// step reads: with one wave walking all of K the same product is eight trips one after the other in a quarter as many
-// workgroups (in a decoding step, 4 places of 16 experts of 2 x 512 x 2048: 24.3 us, now 8.3; 16 places 26.0, now 16.6; the
-// products back to the width, 2048 x 512: 6.1, now 4.9, and 9.3, now 9.1). Eight waves where that leaves a wave two blocks
-// or more, else four. Tiles of more places are walked 16 places at a time.
-template <typename O, bool GLU, int WAVES>
-__global__ __launch_bounds__(WAVES * WAVE) void moe_product_few_kernel(const bf16_t* __restrict__ a, int64_t a_stride,
-                                                              const bf16_t* __restrict__ w,
-                                                              const int* __restrict__ sorted_pair,
-                                                              const int* __restrict__ tile_expert,
-                                                              const int* __restrict__ tile_start,
-                                                              const int* __restrict__ tile_rows,
-                                                              const int* __restrict__ n_tiles, O* __restrict__ out,
-                                                              int top, int n_out, int k_dim, float limit, float alpha, float offset, int act) {
-  __shared__ f32x4 sums[WAVES][GLU ? 2 : 1][WAVE];
-  const int tile = blockIdx.x;
-  if (tile >= *n_tiles) return;
-  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, c = lane % 16, g = lane / 16;
-  const int n0 = blockIdx.y * 16;                             // the grid has no workgroup without outputs
-  const int expert = tile_expert[tile], start = tile_start[tile], count = tile_rows[tile];
-  const int w_rows = GLU ? 2 * n_out : n_out;
-  const bf16_t* we = w + (int64_t)expert * w_rows * k_dim;
-  const int n_mine = min(n0 + c, n_out - 1);
-  const bf16_t* w_gate = we + (int64_t)n_mine * k_dim + 16 * g;
-  const bf16_t* w_up = we + ((int64_t)n_out + n_mine) * k_dim + 16 * g;
-  const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-  const int per = ((k_dim + 63) / 64 + WAVES - 1) / WAVES * 64;          // a wave's run of K, whole blocks
-  const int k_begin = min(wave * per, k_dim), k_end = min(k_begin + per, k_dim);
-  for (int m0 = 0; m0 < count; m0 += 16) {
-    const int place = start + min(m0 + c, count - 1);
-    const bf16_t* x = a + (int64_t)(top > 0 ? sorted_pair[place] / top : place) * a_stride + 16 * g;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f}, acc_up = {0.f, 0.f, 0.f, 0.f};
-    for (int k0 = k_begin; k0 < k_end; k0 += 256) {
-      bf16x8 wg[8], wu[8], xv[8];
+// For steps of few rows (decoding), where no expert has more than 16 places. A workgroup takes 16 rows of an expert's weights (for the
+// gated unit 8 gate rows and their 8 up rows). Operands as in gemm_lines.hip: a load brings four weight rows, 256 contiguous bytes of
+// each, which are a matrix-core operand as they are ("row" c of it is piece c % 4 of weight row c / 4), the places' rows are cut
+// the same way, and of the 16 x 16 products those of equal pieces count. K is split over the waves in blocks of 128 values
+// in turn; their sums meet in LDS and are added in the order 0, 1, ....
+// The shared expert, which takes every row, rides along as workgroups of its own behind the routed ones: two launches fewer a step.
+// What bounds it is the weights (4.2 to 67 MB) and the trips to memory ahead of them (the tile, its rows, their operands).
+// A pass takes up to four places of an expert (eight where a step has more than four rows); more are walked pass by pass: with
+// sixteen a pass the registers leave half as many workgroups (the product back to the width at 12 rows 14.1 us, with eight 10.5).
+// In a captured chain on rotating weights of 16 experts, four of them a row (2 x 512 and 512 of 2,048, the shared one 1,024), us
+// at 1 / 2 / 4 / 8 / 16 rows against a kernel that took the operands' rows 32 bytes at a time: gate and up 6.6 / 7.9 / 11.2 / 13.3 / 14.1
+// (8.9 / 9.9 / 17.6 / 19.6 / 25.9), down 4.9 / 5.9 / 8.3 / 9.8 / 10.5 (5.5 / 6.6 / 9.1 / 10.1 / 10.8), both with the shared expert, whose
+// two launches were its own, 12.6 / 16.1 / 20.7 / 25.1 / 32.2 (20.2 / 23.6 / 33.6 / 36.2 / 43.3).
+struct SharedExpert {
+  const bf16_t* a = nullptr;                                  // [rows, k]; null: there is none
+  int64_t a_stride = 0;
+  const bf16_t* w = nullptr;                                  // [n, k], with the gated unit [2 n, k]
+  bf16_t* out = nullptr;                                      // [rows, n]
+  int rows = 0, n = 0, k = 0;
+  GateAct unit;
+};
+#define MOE_LINE_ROWS 16
+#define MOE_LINE_WAVES 4                                       // eight: 20.8 / 22.7 us of a layer at 4 rows, 25 / 37 at 8
+#define MOE_LINE_AHEAD 4                                       // blocks of K of a wave on their way
+
+template <typename O, bool GLU, int X>
+__global__ __launch_bounds__(MOE_LINE_WAVES * WAVE) void moe_lines_kernel(const bf16_t* __restrict__ a, int64_t a_stride,
+                                                                 const bf16_t* __restrict__ w, const int* __restrict__ sorted_pair,
+                                                                 const int* __restrict__ tile_expert, const int* __restrict__ tile_start,
+                                                                 const int* __restrict__ tile_rows, const int* __restrict__ n_tiles,
+                                                                 int max_tiles, O* __restrict__ out, int top, int n_routed, int k_routed,
+                                                                 float limit, float alpha, float offset, int act, SharedExpert both) {
+  constexpr int T = MOE_LINE_ROWS / 4, OUT = GLU ? MOE_LINE_ROWS / 2 : MOE_LINE_ROWS, AHEAD = MOE_LINE_AHEAD, WAVES = MOE_LINE_WAVES;
+  __shared__ float sums[WAVES][T][X][4][4];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
+  const int c = lane % 16, g = lane / 16, piece = c % 4;
+  const int blocks = (n_routed + OUT - 1) / OUT, routed = max_tiles * blocks;
+  const bool shared = (int)blockIdx.x >= routed;
+  int block = (int)blockIdx.x - routed, start = 0, count = both.rows, n = both.n, k_dim = both.k;
+  const bf16_t* wb = both.w;
+  if (!shared) {
+    const int tile = blockIdx.x / blocks;
+    if (tile >= *n_tiles) return;
+    block = blockIdx.x % blocks;
+    start = tile_start[tile];
+    count = tile_rows[tile];
+    n = n_routed;
+    k_dim = k_routed;
+    wb = w + (int64_t)tile_expert[tile] * (GLU ? 2 * n : n) * k_dim;
+  }
+  const int n0 = block * OUT, at = 8 * (4 * g + piece);       // of this lane within a block of K
+  const bf16_t* wp[T];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int k = k0 + 64 * u;
-        const bool in0 = k + 16 * g < k_end, in1 = k + 16 * g + 8 < k_end;     // K is a multiple of 8
-        wg[2 * u] = in0 ? *(const bf16x8*)(w_gate + k) : zero;
-        wg[2 * u + 1] = in1 ? *(const bf16x8*)(w_gate + k + 8) : zero;
-        wu[2 * u] = (GLU && in0) ? *(const bf16x8*)(w_up + k) : zero;
-        wu[2 * u + 1] = (GLU && in1) ? *(const bf16x8*)(w_up + k + 8) : zero;
-        xv[2 * u] = in0 ? *(const bf16x8*)(x + k) : zero;
-        xv[2 * u + 1] = in1 ? *(const bf16x8*)(x + k + 8) : zero;
+  for (int t = 0; t < T; ++t) {                               // past the outputs: the last row again
+    const int row = 4 * t + c / 4;
+    wp[t] = wb + (int64_t)(GLU && row >= OUT ? n + min(n0 + row - OUT, n - 1) : min(n0 + row, n - 1)) * k_dim;
+  }
+  const int k_blocks = (k_dim + 127) / 128, mine = (k_blocks - wave + WAVES - 1) / WAVES;
+  for (int m0 = 0; m0 < count; m0 += 4 * X) {
+    const bf16_t* xp[X];
+#pragma unroll
+    for (int i = 0; i < X; ++i) {
+      const int place = start + min(m0 + 4 * i + c / 4, count - 1);
+      xp[i] = shared ? both.a + place * both.a_stride : a + (int64_t)(top > 0 ? sorted_pair[place] / top : place) * a_stride;
+    }
+    f32x4 acc[T][X];
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int i = 0; i < X; ++i) acc[t][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i0 = 0; i0 < mine; i0 += AHEAD) {
+      bf16x8 wv[AHEAD][T], xv[AHEAD][X];
+#pragma unroll
+      for (int d = 0; d < AHEAD; ++d) {
+        if (d > 0 && i0 + d >= mine) continue;
+        int k = (wave + (i0 + d) * WAVES) * 128 + at;
+        k = k < k_dim ? k : 0;                                // beyond K (a multiple of 8): any values, zeros below
+#pragma unroll
+        for (int t = 0; t < T; ++t) wv[d][t] = __builtin_nontemporal_load((const bf16x8*)(wp[t] + k));
+#pragma unroll
+        for (int i = 0; i < X; ++i) xv[d][i] = *(const bf16x8*)(xp[i] + k);
       }
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wg[u], xv[u], acc, 0, 0, 0);
-        if (GLU) acc_up = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wu[u], xv[u], acc_up, 0, 0, 0);
+      for (int d = 0; d < AHEAD; ++d) {
+        if (d > 0 && i0 + d >= mine) continue;
+        if ((wave + (i0 + d) * WAVES) * 128 + at >= k_dim) {
+          const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+          for (int t = 0; t < T; ++t) wv[d][t] = zero;
+#pragma unroll
+          for (int i = 0; i < X; ++i) xv[d][i] = zero;
+        }
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+          for (int i = 0; i < X; ++i) acc[t][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[d][t], xv[d][i], acc[t][i], 0, 0, 0);
       }
     }
-    sums[wave][0][lane] = acc;
-    if (GLU) sums[wave][GLU ? 1 : 0][lane] = acc_up;
+    // a lane holds the products of place c / 4, piece c % 4, with the four pieces of weight row g: one counts, and the pieces add up
+    // over four lanes
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int i = 0; i < X; ++i) {
+        const f32x4 s = acc[t][i];
+        const float low = (piece & 1) ? s[1] : s[0], high = (piece & 1) ? s[3] : s[2];
+        const float one = lanes_sum<4>((piece & 2) ? high : low);
+        if (piece == 0) sums[wave][t][i][g][c / 4] = one;
+      }
     __syncthreads();
-    // wave 0 holds the sums: entry i of lane (c, g) is output 4 g + i of place c
-    if (wave == 0 && m0 + c < count) {
+    for (int e = threadIdx.x; e < OUT * 4 * X; e += WAVES * WAVE) {
+      const int o = e % OUT, m = e / OUT;
+      if (m0 + m >= count || n0 + o >= n) continue;
+      auto whole = [&](int row) {
+        float v = 0.f;
 #pragma unroll
-      for (int v = 1; v < WAVES; ++v) {
-        acc += sums[v][0][lane];
-        if (GLU) acc_up += sums[v][GLU ? 1 : 0][lane];
+        for (int u = 0; u < WAVES; ++u) v += sums[u][row / 4][m / 4][row % 4][m % 4];
+        return v;
+      };
+      float v = whole(o);
+      const int64_t to = (int64_t)(start + m0 + m) * n + n0 + o;
+      if (GLU && shared) {
+        both.out[to] = gate_unit(v, whole(o + OUT), both.unit);
+        continue;
       }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int n = n0 + 4 * g + i;
-        if (n >= n_out) continue;
-        float v = acc[i];
-        if (GLU) {
-          const float gv = fminf(rounded_as<bf16_t>(v), limit);
-          const float uv = fminf(fmaxf(rounded_as<bf16_t>(acc_up[i]), -limit), limit);
-          v = gv / (1.f + expf(-alpha * gv)) * (uv + offset);
-        } else if (act == 1) {
-          const float r = fmaxf(rounded_as<bf16_t>(v), 0.f);
-          v = r * r;
-        }
-        store_from_float(out + (int64_t)(start + m0 + c) * n_out + n, v);
+      if (GLU) {
+        const float gv = fminf(rounded_as<bf16_t>(v), limit);
+        const float uv = fminf(fmaxf(rounded_as<bf16_t>(whole(o + OUT)), -limit), limit);
+        v = gv / (1.f + expf(-alpha * gv)) * (uv + offset);
+      } else if (act == 1) {
+        const float r = fmaxf(rounded_as<bf16_t>(v), 0.f);
+        v = r * r;
       }
+      if (shared) store_from_float(both.out + to, v);
+      else store_from_float(out + to, v);
     }
     __syncthreads();                                          // the sums have been read
   }
 }
 
+// shared_w: a shared expert's weights of the same product, for all shared_rows rows of shared_a ([shared_n, shared_k], with glu [2
+// shared_n, shared_k], its unit by shared_limit and shared_alpha as in GateAct); shared_out in bfloat16. Only where no expert
+// has more than 16 places, in bfloat16, shared_k a multiple of 8.
 DRYFT_API int dryft_moe_product(const void* a, int64_t a_stride, const void* w, const int* sorted_pair,
                                 const int* tile_expert, const int* tile_start, const int* tile_rows, const int* n_tiles,
                                 int max_tiles, void* out, int out_is_f32, int top, int n_out, int k_dim, int glu,
-                                float limit, float alpha, float offset, int act, int most_places, int is_f32, hipStream_t stream) {
+                                float limit, float alpha, float offset, int act, int most_places, int is_f32, const void* shared_a,
+                                int64_t shared_stride, const void* shared_w, void* shared_out, int shared_rows, int shared_n,
+                                int shared_k, float shared_limit, float shared_alpha, hipStream_t stream) {
   if (max_tiles <= 0) return 0;
   if (n_out <= 0 || k_dim <= 0 || (glu && out_is_f32 && !is_f32)) return -1;
   dim3 grid(max_tiles, (n_out + MOE_TN - 1) / MOE_TN), block(256);
-  if (!is_f32 && k_dim % 8 == 0 && a_stride % 8 == 0 && (((uintptr_t)a | (uintptr_t)w) & 15) == 0) {
-    const dim3 few(max_tiles, (n_out + 15) / 16);
-    if (most_places <= 16 && few.y <= 65535) {           // no expert can get more places than that
-#define MOE_FEW_WAVES(O, G, W)                                                                                    \
-  hipLaunchKernelGGL((moe_product_few_kernel<O, G, W>), few, dim3(W * WAVE), 0, stream, (const bf16_t*)a, a_stride, \
-                     (const bf16_t*)w, sorted_pair, tile_expert, tile_start, tile_rows, n_tiles, (O*)out, top, n_out, \
-                     k_dim, limit, alpha, offset, act)
-#define MOE_FEW(O, G)                                                                                             \
-  do {                                                                                                            \
-    if (k_dim >= 1024) MOE_FEW_WAVES(O, G, 8);                                                                     \
-    else MOE_FEW_WAVES(O, G, 4);                                                                                   \
+  const bool lined = !is_f32 && k_dim % 8 == 0 && a_stride % 8 == 0 && (((uintptr_t)a | (uintptr_t)w) & 15) == 0;
+  SharedExpert both;
+  if (shared_w != nullptr) {
+    if (!lined || most_places > 16 || shared_rows <= 0 || shared_n <= 0 || shared_k <= 0 || shared_k % 8 || shared_stride % 8 ||
+        (((uintptr_t)shared_a | (uintptr_t)shared_w) & 15) || shared_limit < 0.f)
+      return -1;
+    both.a = (const bf16_t*)shared_a;
+    both.a_stride = shared_stride;
+    both.w = (const bf16_t*)shared_w;
+    both.out = (bf16_t*)shared_out;
+    both.rows = shared_rows;
+    both.n = shared_n;
+    both.k = shared_k;
+    both.unit.limit = shared_limit;
+    both.unit.alpha = shared_alpha;
+  }
+  if (lined) {
+    const int outs = glu ? MOE_LINE_ROWS / 2 : MOE_LINE_ROWS;
+    const int64_t few = (int64_t)max_tiles * ((n_out + outs - 1) / outs) + (shared_w != nullptr ? (shared_n + outs - 1) / outs : 0);
+    if (most_places <= 16 && few <= 1 << 24) {           // no expert can get more places than that
+#define MOE_LINES_X(O, G, XV)                                                                                        \
+  hipLaunchKernelGGL((moe_lines_kernel<O, G, XV>), dim3((unsigned)few), dim3(MOE_LINE_WAVES * WAVE), 0, stream,       \
+                     (const bf16_t*)a, a_stride, (const bf16_t*)w, sorted_pair, tile_expert, tile_start, tile_rows, n_tiles, \
+                     max_tiles, (O*)out, top, n_out, k_dim, limit, alpha, offset, act, both)
+#define MOE_LINES(O, G)                                                                                              \
+  do {                                                                                                               \
+    if (most_places <= 4) MOE_LINES_X(O, G, 1);                                                                       \
+    else MOE_LINES_X(O, G, 2);                                                                                        \
   } while (0)
-      if (glu) MOE_FEW(bf16_t, true);
-      else if (out_is_f32) MOE_FEW(float, false);
-      else MOE_FEW(bf16_t, false);
-#undef MOE_FEW_WAVES
-#undef MOE_FEW
+      if (glu) MOE_LINES(bf16_t, true);
+      else if (out_is_f32) MOE_LINES(float, false);
+      else MOE_LINES(bf16_t, false);
+#undef MOE_LINES
+#undef MOE_LINES_X
       return DRYFT_LAUNCH_CHECK();
     }
+    if (shared_w != nullptr) return -1;
 #define MOE_MFMA(O, G)                                                                                            \
   hipLaunchKernelGGL((moe_product_mfma_kernel<O, G>), grid, block, 0, stream, (const bf16_t*)a, a_stride,          \
                      (const bf16_t*)w, sorted_pair, tile_expert, tile_start, tile_rows, n_tiles, (O*)out, top, n_out, \

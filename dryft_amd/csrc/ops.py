@@ -116,7 +116,8 @@ _SIGNATURES = {
                "dryft_head_gate": [_P, _P, _L, _I, _P, _I, _I, _I, _I, _I, _I, _P]},
     "moe": {"dryft_moe_route": [_P, _L, _P, _I, _I, _I, _I, _F, _P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P],
             "dryft_moe_plan": [_P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _P],
-            "dryft_moe_product": [_P, _L, _P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _F, _F, _F, _I, _I, _I, _P],
+            "dryft_moe_product": [_P, _L, _P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _F, _F, _F, _I, _I, _I, _P, _L, _P, _P, _I,
+                                  _I, _I, _F, _F, _P],
             "dryft_moe_table_route": [_P, _P, _P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P],
             "dryft_moe_combine": [_P, _P, _P, _P, _P, _L, _I, _P, _I, _I, _I, _I, _P]},
     "conv": {"dryft_conv_max_taps": [],
@@ -2325,13 +2326,24 @@ def moe_table_route(tokens, table, n_experts: int, chosen, weights, plan: "MoePl
     _plan_many(chosen, n_experts, plan)
 
 
-def moe_products(a, w, plan: MoePlan, out, top: int, glu: tuple | None = None, act: str | None = None) -> None:
+def moe_takes_shared(a, w, plan: MoePlan, shared_w) -> bool:
+    """Can ``moe_products`` make a shared expert's product in the same launch? Steps of few rows in bfloat16."""
+    return a.dtype == torch.bfloat16 and shared_w.dtype == torch.bfloat16 and 0 < plan.most_places <= MOE_FEW_ROWS and \
+        a.shape[1] % 8 == 0 and w.shape[2] % 8 == 0 and shared_w.shape[1] % 8 == 0 and a.stride(0) % 8 == 0 and \
+        a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and shared_w.data_ptr() % 16 == 0
+
+
+def moe_products(a, w, plan: MoePlan, out, top: int, glu: tuple | None = None, act: str | None = None,
+                 shared: tuple | None = None) -> None:
     """``out[place] = W_e a_row`` for every place of the plan, ``e`` the place's expert. ``top`` > 0: ``a`` is
     ``[rows, K]`` and a place's operand is row ``pair // top``; ``top`` == 0: ``a`` is ``[pairs, K]`` in place order.
     ``w`` is ``[experts, N, K]``; with ``glu = (limit, alpha)`` it holds gate rows then up rows (``N = 2 I``) and
     ``out [pairs, I]`` receives the clamped gated unit of the two, ``g sigmoid(alpha g) (u + 1)``; ``glu = (limit, alpha,
     offset)`` puts ``offset`` in the place of that 1 (``(inf, 1, 0)`` is ``silu(gate) * up``). ``out`` may be float32
-    for a plain product. ``act="relu2"`` (no gate): ``out`` receives the square of relu of the product."""
+    for a plain product. ``act="relu2"`` (no gate): ``out`` receives the square of relu of the product.
+    ``shared = (a_s [rows, K_s], w_s, out_s [rows, N_s], (limit, alpha) or None)``: the same product of another matrix for
+    all rows, in the same launch (``moe_takes_shared``), stored in bfloat16; its gated unit is the clamped one or ``silu(gate) *
+    up`` with the roundings of ``gemm_panel_swiglu_bf16``."""
     if act not in (None, "relu2") or (act and glu):
         raise KernelError("moe_products: act is None or 'relu2', and goes without a gate")
     _gpu(a, "a")
@@ -2350,11 +2362,27 @@ def moe_products(a, w, plan: MoePlan, out, top: int, glu: tuple | None = None, a
     if glu and out.dtype != a.dtype:
         raise KernelError("moe_products: the gated unit is stored in the activation dtype")
     limit, alpha, offset = (tuple(glu) + (1.0,))[:3] if glu else (0.0, 0.0, 0.0)
+    ride = (0, 0, 0, 0, 0, 0, 0, 0.0, 0.0)
+    if shared is not None:
+        a_s, w_s, out_s, clamped = shared
+        if not moe_takes_shared(a, w, plan, w_s):
+            raise KernelError("moe_products: a shared expert rides along with bfloat16 steps of few rows at 16-byte addresses")
+        for name, t in (("shared a", a_s), ("shared w", w_s), ("shared out", out_s)):
+            _gpu(t, name, torch.bfloat16)
+        n_s, k_s = (w_s.shape[0] // 2 if glu else w_s.shape[0]), w_s.shape[1]
+        if not (w_s.dim() == 2 and w_s.is_contiguous() and (not glu or w_s.shape[0] % 2 == 0) and a_s.dim() == 2 and a_s.shape[1] == k_s and
+                a_s.stride(1) == 1 and a_s.stride(0) % 8 == 0 and a_s.data_ptr() % 16 == 0 and 0 < a_s.shape[0] <= MOE_FEW_ROWS and
+                out_s.shape == (a_s.shape[0], n_s) and out_s.is_contiguous()):
+            raise KernelError("moe_products: shared a [rows, K] at 16-byte addresses, w contiguous [N, K], out contiguous [rows, N]")
+        if clamped is not None and not clamped[0] > 0:
+            raise KernelError(f"moe_products: the clamp's limit must be positive, got {clamped[0]}")
+        ride = (_ptr(a_s), a_s.stride(0), _ptr(w_s), _ptr(out_s), a_s.shape[0], n_s, k_s) + \
+            ((float(clamped[0]), float(clamped[1])) if clamped is not None else (0.0, 0.0))
     _check(_fn("moe", "dryft_moe_product")(
         _ptr(a), a.stride(0), _ptr(w), _ptr(plan.sorted_pair), _ptr(plan.tiles[0]), _ptr(plan.tiles[1]),
         _ptr(plan.tiles[2]), _ptr(plan.n_tiles), plan.max_tiles, _ptr(out), 1 if out.dtype == torch.float32 else 0,
         int(top), n_out, k, 1 if glu else 0, float(limit), float(alpha), float(offset), 1 if act else 0, plan.most_places,
-        _float_flag(a, "a"), _stream()),
+        _float_flag(a, "a"), *ride, _stream()),
         "moe_products")
 
 

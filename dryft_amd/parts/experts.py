@@ -23,7 +23,8 @@ times ``route_scale``.
 
 On the device throughout, so a step can be captured: the router picks, a small kernel sorts the (row, expert) pairs
 by expert and cuts each expert's run into tiles, and two grouped products walk the tiles (gate/up with the unit in
-the epilogue, then down); a last kernel adds each row's weighted outputs and the shared expert in a fixed order.
+the epilogue, then down); a last kernel adds each row's weighted outputs and the shared expert in a fixed order. In steps of
+few rows the shared expert's products are made in the launches of the routed ones.
 """
 
 from __future__ import annotations
@@ -34,7 +35,7 @@ from ..csrc import ops
 from ..weights.spec import INT_TABLE, VECTOR
 from . import register_part
 from .base import FeedForward, Partials, matrix
-from .linear import linear
+from .linear import lines_pay, linear
 from .mlp import ClampedGLU, SquaredReLU, SwiGLU
 
 
@@ -143,20 +144,43 @@ class RoutedExperts(FeedForward):
                           renorm=self.renormalize, chosen_softmax=self.score == "chosen_softmax",
                           logit_bias=self.router_bias, plan=plan)
         act = torch.empty((rows * top, self.inter), dtype=h.dtype, device=dev)
-        if self.gated:
-            ops.moe_products(h, self.w_gate_up, plan, act, top, glu=self.glu)
-        else:
-            ops.moe_products(h, self.w_gate_up, plan, act, top, act="relu2")
+        unit = dict(glu=self.glu) if self.gated else dict(act="relu2")
         y = torch.empty((rows * top, self.hidden), dtype=torch.float32, device=dev)
-        ops.moe_products(act, self.w_down, plan, y, 0)
         shared = None
-        if self.shared is not None:
-            shared = self.shared.forward(h, ctx)
-            if isinstance(shared, Partials):
-                shared = shared.summed(h.dtype)
+        if self._shared_rides(h, plan):
+            w_in, clamped = self._shared_unit()
+            shared_act = torch.empty((rows, self.shared.inter), dtype=h.dtype, device=dev)
+            shared = torch.empty((rows, self.hidden), dtype=h.dtype, device=dev)
+            ops.moe_products(h, self.w_gate_up, plan, act, top, shared=(h, w_in, shared_act, clamped), **unit)
+            ops.moe_products(act, self.w_down, plan, y, 0, shared=(shared_act, self.shared.w_down, shared, None))
+        else:
+            ops.moe_products(h, self.w_gate_up, plan, act, top, **unit)
+            ops.moe_products(act, self.w_down, plan, y, 0)
+            if self.shared is not None:
+                shared = self.shared.forward(h, ctx)
+                if isinstance(shared, Partials):
+                    shared = shared.summed(h.dtype)
         out = torch.empty((rows, self.hidden), dtype=h.dtype, device=dev)
         ops.moe_combine(y, plan, weights, shared, logits if self.shared_gate else None, E, out)
         return out
+
+    def _shared_unit(self):
+        """The shared expert's first matrix, and (limit, alpha) where its unit is the clamped one."""
+        if not self.gated:
+            return self.shared.w_up, None
+        return self.shared.w_gate_up, (self.shared.limit, self.shared.alpha) if self.unit == "clamped" else None
+
+    def _shared_rides(self, h, plan) -> bool:
+        """Are the shared expert's products made in the launches of the routed ones? Steps of few rows whose own products would
+        go to the same kind of kernel (``few_glu_pays``, ``lines_pay``), and only where the shared expert is as it was made."""
+        shared = self.shared
+        if shared is None or type(shared) not in (ClampedGLU, SwiGLU, SquaredReLU) or "forward" in vars(shared):
+            return False
+        rows, w_in = h.shape[0], self._shared_unit()[0]
+        return ops.moe_takes_shared(h, self.w_gate_up, plan, w_in) and self.inter % 8 == 0 and shared.inter % 8 == 0 and \
+            self.w_down.data_ptr() % 16 == 0 and shared.w_down.data_ptr() % 16 == 0 and \
+            (ops.few_glu_pays(rows, shared.inter, self.hidden) if self.gated else lines_pay(rows, shared.inter, self.hidden)) and \
+            lines_pay(rows, self.hidden, shared.inter)
 
     def reads_whole(self) -> bool:
         return True

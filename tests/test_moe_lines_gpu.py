@@ -1,0 +1,77 @@
+"""Experts' products of few rows, with a shared expert in the same launch: at the edges of their tiles, passes and blocks of K."""
+
+import math
+
+import pytest
+import torch
+
+from test_kernels_gpu import close
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def unit_of(z, kind):
+    """The unit in 64 bits on a product's rounded results."""
+    z = z.to(torch.bfloat16).double()
+    if kind == "relu2":
+        return z.clamp(min=0) ** 2
+    g, u = z[:, :z.shape[1] // 2], z[:, z.shape[1] // 2:]
+    if kind == "silu":
+        return torch.nn.functional.silu(g) * u
+    g, u = g.clamp(max=1.5), u.clamp(-1.5, 1.5)
+    return g * torch.sigmoid(1.702 * g) * (u + 1)
+
+
+@pytest.mark.parametrize("rows,experts,top", [(1, 4, 4), (3, 5, 2), (4, 16, 4), (5, 3, 3), (8, 2, 1), (9, 2, 1), (16, 1, 1), (16, 16, 4)])
+@pytest.mark.parametrize("k,inter,shared_inter", [(8, 8, 16), (136, 24, 72), (512, 72, 8), (1160, 136, 200)])
+@pytest.mark.parametrize("kind", ["silu", "clamped", "relu2"])
+def test_experts_and_the_shared_one(rows, experts, top, k, inter, shared_inter, kind):
+    from dryft_amd.csrc import ops
+    torch.manual_seed(rows * 1000 + k + inter)
+    halves = 1 if kind == "relu2" else 2
+    x = torch.randn(rows, k + 8).to(torch.bfloat16)[:, :k]                     # rows wider apart than K
+    w = (torch.randn(experts, halves * inter, k) * 2 / math.sqrt(k)).to(torch.bfloat16)
+    down = (torch.randn(experts, k, inter) / math.sqrt(inter)).to(torch.bfloat16)
+    ws = (torch.randn(halves * shared_inter, k) * 2 / math.sqrt(k)).to(torch.bfloat16)
+    down_s = (torch.randn(k, shared_inter) / math.sqrt(shared_inter)).to(torch.bfloat16)
+    chosen = torch.stack([torch.randperm(experts)[:top] for _ in range(rows)]).to(torch.int32)
+    plan = ops.moe_plan(chosen.to(DEV), experts)
+    n = rows * top
+    act, y = torch.full((n, inter), float("nan"), dtype=torch.bfloat16, device=DEV), torch.full((n, k), float("nan"), device=DEV)
+    act_s = torch.full((rows, shared_inter), float("nan"), dtype=torch.bfloat16, device=DEV)
+    y_s = torch.full((rows, k), float("nan"), dtype=torch.bfloat16, device=DEV)
+    how = dict(act="relu2") if kind == "relu2" else dict(glu=(float("inf"), 1.0, 0.0) if kind == "silu" else (1.5, 1.702))
+    ride = (x.to(DEV) if x.is_contiguous() else torch.nn.functional.pad(x, (0, 8)).to(DEV)[:, :k], ws.to(DEV), act_s,
+            (1.5, 1.702) if kind == "clamped" else None)
+    ops.moe_products(ride[0], w.to(DEV), plan, act, top, shared=ride, **how)
+    ops.moe_products(act, down.to(DEV), plan, y, 0, shared=(act_s, down_s.to(DEV), y_s, None))
+    place = plan.place_of.cpu().view(rows, top)
+    a = act.cpu().double()
+    for r in range(rows):
+        for t in range(top):
+            e, p = int(chosen[r, t]), int(place[r, t])
+            # the unit's argument is a bfloat16 step off where its sum lies between two
+            close(act[p:p + 1], unit_of(x[r:r + 1].double() @ w[e].double().T, kind), torch.bfloat16, ulps=4.0, what=f"row {r} expert {e}")
+            close(y[p:p + 1], a[p:p + 1] @ down[e].double().T, torch.float32, what=f"row {r} expert {e}, back")
+    close(act_s, unit_of(x.double() @ ws.double().T, kind), torch.bfloat16, ulps=4.0, what="shared")
+    close(y_s, act_s.cpu().double() @ down_s.double().T, torch.bfloat16, what="shared, back")
+
+
+def test_a_replaced_shared_expert_is_called():
+    """A shared expert whose ``forward`` was replaced on the object runs as it says, ahead of everything that rides along."""
+    from dryft_amd.csrc import ops
+    from dryft_amd.parts.experts import RoutedExperts
+    part = RoutedExperts(64, 4, 2, 16, unit="silu", shared=(24,), correction=False)
+    part.compute_dtype = torch.bfloat16
+    torch.manual_seed(0)
+    part.load({name: torch.randn(*spec[0]).to(torch.bfloat16).to(DEV) * 0.1 for name, spec in part.tensor_specs().items()})
+    h, ctx = torch.randn(3, 64).to(torch.bfloat16).to(DEV), None
+    plain = part.forward(h, ctx)
+    plan = ops.MoePlan(6, 4, DEV, most_places=3)
+    assert part._shared_rides(h, plan)
+    made = part.shared.forward
+    part.shared.forward = lambda rows, step: 0 * made(rows, step).summed(torch.bfloat16) if hasattr(made(rows, step), "summed") else 0 * made(rows, step)
+    assert not part._shared_rides(h, plan)
+    without = part.forward(h, ctx)
+    assert not torch.equal(plain, without)
