@@ -49,6 +49,17 @@ struct Residual {
   float* squares = nullptr;
 };
 
+// Further products of the same rows in the same launch, workgroups of their own behind the first product's: small ones (gates, step
+// sizes, low-rank projections) are all trips to memory as launches of their own.
+#define LINES_BESIDE 3
+template <typename E>
+struct Beside {
+  int count = 0;
+  const E* w[LINES_BESIDE] = {};
+  void* y[LINES_BESIDE] = {};
+  int n[LINES_BESIDE] = {}, y_f32[LINES_BESIDE] = {};
+};
+
 // Sixteen bytes of a row are an operand of one matrix instruction of 32 values in bfloat16, or a value for each of four
 // instructions of four values in float32 (32-bit factors and sums).
 template <typename E>
@@ -105,18 +116,32 @@ __device__ __forceinline__ void each(F&& f) {
 
 // ROWS weight rows a workgroup (with GLU half of them gate rows and then their up rows), X groups of four rows of x, DEPTH blocks
 // of 256 bytes of K of a wave on their way at a time
-template <typename E, int ROWS, int X, int WAVES, int DEPTH, bool GLU, bool LATE>
+template <typename E, int ROWS, int X, int WAVES, int DEPTH, bool GLU, bool LATE, bool MORE>
 __global__ __launch_bounds__(64 * WAVES) void gemm_lines_kernel(const E* __restrict__ x, int64_t x_stride,
                                                                 const E* __restrict__ w, void* __restrict__ y, int y_f32,
                                                                 int M, int N, int K, LateNorm<E> late, Residual<E> residual,
-                                                                GateAct act) {
+                                                                GateAct act, Beside<E> beside) {
   typedef Fragment<E> F;
   typedef typename F::type frag;
   constexpr int T = (ROWS + 3) / 4, BLOCK = 16 * F::VALUES, OUT = GLU ? ROWS / 2 : ROWS;
   __shared__ float sums[WAVES][T][X][4][4], late_sums[LATE ? WAVES : 1][LATE_ROWS], squares[GLU ? 1 : ROWS][LATE_ROWS];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
   const int c = lane % 16, g = lane / 16, piece = c % 4;
-  const int n0 = blockIdx.x * OUT;
+  int block = blockIdx.x;
+  if constexpr (MORE) {                                    // whose outputs these are
+#pragma unroll
+    for (int p = 0; p < LINES_BESIDE; ++p) {
+      const int blocks = (N + OUT - 1) / OUT;
+      if (p < beside.count && block >= blocks) {
+        block -= blocks;
+        w = beside.w[p];
+        y = beside.y[p];
+        N = beside.n[p];
+        y_f32 = beside.y_f32[p];
+      }
+    }
+  }
+  const int n0 = block * OUT;
   f32x4 late_held[X];                                      // sums of squares, asked for ahead of everything
   if constexpr (LATE) {
 #pragma unroll
@@ -267,9 +292,9 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_lines_kernel(const E* __restr
   }
 }
 
-template <typename E, int ROWS, int X, int WAVES, bool GLU, bool LATE>
+template <typename E, int ROWS, int X, int WAVES, bool GLU, bool LATE, bool MORE = false>
 static int launch_lines(const void* x, int64_t x_stride, const void* w, void* y, int y_f32, int M, int N, int K, LateNorm<E> late,
-                        Residual<E> residual, GateAct act, hipStream_t stream) {
+                        Residual<E> residual, GateAct act, hipStream_t stream, const Beside<E>& beside) {
   constexpr int T = (ROWS + 3) / 4, OUT = GLU ? ROWS / 2 : ROWS;
   // registers for the operands on their way: eight waves have 256 a lane, four are to share a compute unit with others
   constexpr int held = 4 * T * X * Fragment<E>::SUMS;
@@ -279,9 +304,11 @@ static int launch_lines(const void* x, int64_t x_stride, const void* w, void* y,
   // Ahead of a norm five to eight rows are work for the vector units too, and waves side by side hide it better than blocks on their
   // way: one block a wave, us at 8 rows against two or three, 6,144 x 2,560 8.4 (10.0), 4,096 x 1,024 5.0 (6.1), 3,072 gated outputs
   // of 1,024 5.5 (6.1); gated outputs of a long K want two (9,728 of 2,560 20.6, with one 21.5).
+  int blocks = (N + OUT - 1) / OUT;
+  for (int p = 0; p < beside.count; ++p) blocks += (beside.n[p] + OUT - 1) / OUT;
 #define GO(D)                                                                                                                  \
-  hipLaunchKernelGGL((gemm_lines_kernel<E, ROWS, X, WAVES, D, GLU, LATE>), dim3((N + OUT - 1) / OUT), dim3(64 * WAVES), 0, stream, \
-                     (const E*)x, x_stride, (const E*)w, y, y_f32, M, N, K, late, residual, act)
+  hipLaunchKernelGGL((gemm_lines_kernel<E, ROWS, X, WAVES, D, GLU, LATE, MORE>), dim3(blocks), dim3(64 * WAVES), 0, stream,          \
+                     (const E*)x, x_stride, (const E*)w, y, y_f32, M, N, K, late, residual, act, beside)
   if constexpr (LATE && X == 2 && WAVES == 4) {
     if constexpr (GLU) {
       if (K > 1024) {
@@ -299,18 +326,25 @@ static int launch_lines(const void* x, int64_t x_stride, const void* w, void* y,
 
 template <typename E, int ROWS, int WAVES, bool GLU>
 static int lines_by_rows(const void* x, int64_t x_stride, const void* w, void* y, int y_f32, int M, int N, int K, LateNorm<E> late,
-                         Residual<E> residual, GateAct act, hipStream_t stream) {
+                         Residual<E> residual, GateAct act, hipStream_t stream, const Beside<E>& beside = {}) {
   if constexpr (sizeof(E) == 4) {
-    if (late.squares != nullptr) return launch_lines<E, ROWS, 1, WAVES, GLU, true>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
-    return launch_lines<E, ROWS, 1, WAVES, GLU, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
+    if (late.squares != nullptr) return launch_lines<E, ROWS, 1, WAVES, GLU, true>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream, beside);
+    return launch_lines<E, ROWS, 1, WAVES, GLU, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream, beside);
   } else {
     if (late.squares != nullptr) {
-      if (M <= 4) return launch_lines<E, ROWS, 1, WAVES, GLU, true>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
-      return launch_lines<E, ROWS, 2, WAVES, GLU, true>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
+      if (M <= 4) return launch_lines<E, ROWS, 1, WAVES, GLU, true>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream, beside);
+      return launch_lines<E, ROWS, 2, WAVES, GLU, true>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream, beside);
     }
-    if (M <= 4) return launch_lines<E, ROWS, 1, WAVES, GLU, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
-    if (M <= 8) return launch_lines<E, ROWS, 2, WAVES, GLU, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
-    return launch_lines<E, ROWS, 4, WAVES, GLU, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream);
+    if constexpr (!GLU) {
+      if (beside.count > 0) {
+        if (M <= 4) return launch_lines<E, ROWS, 1, WAVES, GLU, false, true>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream, beside);
+        if (M <= 8) return launch_lines<E, ROWS, 2, WAVES, GLU, false, true>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream, beside);
+        return launch_lines<E, ROWS, 4, WAVES, GLU, false, true>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream, beside);
+      }
+    }
+    if (M <= 4) return launch_lines<E, ROWS, 1, WAVES, GLU, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream, beside);
+    if (M <= 8) return launch_lines<E, ROWS, 2, WAVES, GLU, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream, beside);
+    return launch_lines<E, ROWS, 4, WAVES, GLU, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, act, stream, beside);
   }
 }
 
@@ -360,17 +394,20 @@ static bool lines_refuse(const void* x, int64_t x_stride, const void* w, int M, 
 
 template <typename E>
 static int lines(const void* x, int64_t x_stride, const void* w, void* y, int y_f32, int M, int N, int K, const float* late_squares,
-                 int late_count, float late_eps, const void* late_weight, void* residual_rows, float* squares, hipStream_t stream) {
+                 int late_count, float late_eps, const void* late_weight, void* residual_rows, float* squares, hipStream_t stream,
+                 const Beside<E>& beside = {}) {
   if (M <= 0 || N <= 0) return 0;
   const LateNorm<E> late{late_squares, late_count, late_eps, (const E*)late_weight};
   const Residual<E> residual{(E*)residual_rows, squares};
   if (lines_refuse(x, x_stride, w, M, K, late) || (residual_rows != nullptr && (squares == nullptr || M > LATE_ROWS))) return -1;
-  const LinesShape shape = lines_shape(M, N, (int64_t)K * sizeof(E), sizeof(E) == 4);
-#define LINES(ROWS, W) case ROWS + 32 * W: return lines_by_rows<E, ROWS, W, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, {}, stream);
+  int outputs = N;
+  for (int p = 0; p < beside.count; ++p) outputs += beside.n[p];
+  const LinesShape shape = lines_shape(M, outputs, (int64_t)K * sizeof(E), sizeof(E) == 4);
+#define LINES(ROWS, W) case ROWS + 32 * W: return lines_by_rows<E, ROWS, W, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, {}, stream, beside);
   switch (shape.rows + 32 * shape.waves) {
     LINES(4, 8) LINES(8, 8) LINES(10, 8) LINES(12, 8) LINES(8, 4) LINES(10, 4) LINES(12, 4)
     case 20 + 32 * 4:
-      if constexpr (sizeof(E) == 2) return lines_by_rows<E, 20, 4, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, {}, stream);
+      if constexpr (sizeof(E) == 2) return lines_by_rows<E, 20, 4, false>(x, x_stride, w, y, y_f32, M, N, K, late, residual, {}, stream, beside);
     default: return -1;
   }
 #undef LINES
@@ -392,6 +429,26 @@ DRYFT_API int dryft_gemm_lines_bf16(const void* x, int64_t x_stride, const void*
                                     const float* late_squares, int late_count, float late_eps, const void* late_weight,
                                     void* residual, float* squares, hipStream_t stream) {
   return lines<bf16_t>(x, x_stride, w, y, y_f32, M, N, K, late_squares, late_count, late_eps, late_weight, residual, squares, stream);
+}
+
+// The products of x [M, K] with up to four matrices w[p] [n[p], K], each y[p] as float (y_f32[p]) or bfloat16, in one launch:
+// gates, step sizes and the second mixer of two side by side, launches of 2.3 to 6 us and the gap before each, ride along with a
+// layer's first product. Passes of 24 decoding steps of four sequences and their prompts, ms: barilix-w2048 (nine launches fewer a
+// step) 20.8 -> 20.4, piralix-w2048 (two of its first six layers) 10.29 -> 10.14, fubinex-w2048 (four) 17.50 -> 17.26.
+DRYFT_API int dryft_gemm_lines_beside_bf16(const void* x, int64_t x_stride, int M, int K, int count, const void* const* w, void* const* y,
+                                           const int* n, const int* y_f32, hipStream_t stream) {
+  if (count < 1 || count > 1 + LINES_BESIDE) return -1;
+  Beside<bf16_t> beside;
+  beside.count = count - 1;
+  for (int p = 0; p < count; ++p)
+    if (n[p] <= 0 || ((uintptr_t)w[p] & 15)) return -1;
+  for (int p = 1; p < count; ++p) {
+    beside.w[p - 1] = (const bf16_t*)w[p];
+    beside.y[p - 1] = y[p];
+    beside.n[p - 1] = n[p];
+    beside.y_f32[p - 1] = y_f32[p];
+  }
+  return lines<bf16_t>(x, x_stride, w[0], y[0], y_f32[0], M, n[0], K, nullptr, 0, 0.f, nullptr, nullptr, nullptr, stream, beside);
 }
 
 // The same in float32: M <= 4, K a multiple of 4. Us at 1 / 4 rows, against the kernels of gemm_f32.hip: 4,096 x 1,024 5.6 / 5.5 (6.0 /

@@ -84,6 +84,7 @@ _SIGNATURES = {
     "gemm_lines": {"dryft_gemm_lines_blocks": [_I, _I, _I, _I],
                    "dryft_gemm_lines_f32": [_P, _L, _P, _P, _I, _I, _I, _P, _I, _F, _P, _P, _P, _P],
                    "dryft_gemm_lines_swiglu_f32": [_P, _L, _P, _P, _I, _I, _I, _P, _I, _F, _P, _P],
+                   "dryft_gemm_lines_beside_bf16": [_P, _L, _I, _I, _I, _P, _P, _P, _P, _P],
                    "dryft_gemm_lines_bf16": [_P, _L, _P, _P, _I, _I, _I, _I, _P, _I, _F, _P, _P, _P, _P],
                    "dryft_gemm_lines_glu_bf16": [_P, _L, _P, _P, _I, _I, _I, _P, _I, _F, _P, _I, _F, _F, _P]},
     "gemm": {"dryft_gemm_tiled": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _P],
@@ -1095,6 +1096,29 @@ def gemm_lines_add(x, w, residual) -> torch.Tensor:
     squares = torch.empty((gemm_lines_blocks(m, n, k, x.dtype), LATE_ROWS), dtype=torch.float32, device=x.device)
     _lines("gemm_lines_add", x, w, None, None, residual, squares)
     return squares
+
+
+LINES_TOGETHER = 4       # the most products of the same rows in one launch
+
+
+def gemm_lines_beside(x, products: list) -> None:
+    """``out = x @ w.T`` for every ``(w, out)`` of up to ``LINES_TOGETHER``, bfloat16 operands of at most 16 rows, in one launch;
+    ``out`` bfloat16 or float32."""
+    if not 1 <= len(products) <= LINES_TOGETHER:
+        raise KernelError(f"gemm_lines_beside: 1 to {LINES_TOGETHER} products")
+    _gpu(x, "x", torch.bfloat16)
+    m, k = x.shape
+    for w, out in products:
+        _lines_operands("gemm_lines_beside", x, w)
+        _gpu(out, "out")
+        if not (out.dtype in (torch.bfloat16, torch.float32) and out.shape == (m, w.shape[0]) and out.is_contiguous()):
+            raise KernelError(f"gemm_lines_beside: out contiguous [{m},{w.shape[0]}] in bfloat16 or float32")
+    count = len(products)
+    pointers, numbers = ctypes.c_void_p * count, ctypes.c_int * count
+    _check(_fn("gemm_lines", "dryft_gemm_lines_beside_bf16")(
+        _ptr(x), x.stride(0), m, k, count, pointers(*(_ptr(w) for w, _ in products)), pointers(*(_ptr(out) for _, out in products)),
+        numbers(*(w.shape[0] for w, _ in products)), numbers(*(int(out.dtype == torch.float32) for _, out in products)), _stream()),
+        "gemm_lines_beside_bf16")
 
 
 def few_glu_pays(m: int, n: int, k: int) -> bool:

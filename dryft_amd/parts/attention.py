@@ -274,7 +274,10 @@ class GQAAttention(Mixer):
             (("activation",) if self.output_gate or self.value_mix else ()) + (("latent",) if self.head_gate else ()) + \
             (("conv", "norm") if self.conv_taps or self.has_bias else ())
 
-    def _forward_general(self, h: torch.Tensor, ctx: StepContext, line, writes_cache: bool):
+    def first_products(self, ctx: StepContext) -> list:
+        return [] if self._plain(ctx.positions) else [(self.w_qkv, None)]
+
+    def _forward_general(self, h: torch.Tensor, ctx: StepContext, line, writes_cache: bool, made: list | None = None):
         """Every option, in float arithmetic on the kernel that takes one (row, head) a workgroup. Returns the output
         projection's result without its bias."""
         rows, H, G, D, Dv = h.shape[0], self.n_heads, self.n_kv, self.head_dim, self.value_dim
@@ -291,7 +294,7 @@ class GQAAttention(Mixer):
             cos, sin, rot = table.cos, table.sin, table.dims
             if rot > D:
                 raise ValueError(f"the position encoding rotates {rot} features, a head has {D}")
-        proj = linear(h, self.w_qkv)                                    # q | k | v | gate
+        proj = made[0] if made else linear(h, self.w_qkv)               # q | k | v | gate
         src = proj
         if self.conv_w is not None:
             # biases and the short convolution: q | k | v as one run of channels, each with its own history
@@ -362,10 +365,10 @@ class GQAAttention(Mixer):
             return linear(out.view(rows, H * wide), self.w_o_padded, allow_partials=True)
         return linear(out.view(rows, self.o_dim), self.w_o, allow_partials=True)
 
-    def forward_split(self, h: torch.Tensor, ctx: StepContext, line, writes_cache: bool):
+    def forward_split(self, h: torch.Tensor, ctx: StepContext, line, writes_cache: bool, made: list | None = None):
         if self.has_bias:
-            return self._forward_general(h, ctx, line, writes_cache), self.o_bias
-        return self.forward(h, ctx, line, writes_cache), None
+            return self._forward_general(h, ctx, line, writes_cache, made), self.o_bias
+        return self.forward(h, ctx, line, writes_cache, **({"made": made} if made else {})), None
 
     def _plain(self, positions) -> bool:
         return not (self.extended or (self.positions and not isinstance(positions[self.positions], RotaryPositions)))
@@ -383,10 +386,11 @@ class GQAAttention(Mixer):
             return rows <= ops.LINES_ROWS_F32 and k % 4 == 0
         return self._fused_decoding(ctx, self.w_qkv.dtype) and rows <= ops.LATE_ROWS and k % 8 == 0 and lines_pay(rows, n, k)
 
-    def forward(self, h: torch.Tensor, ctx: StepContext, line: KVLine, writes_cache: bool, leave_product: bool = False):
-        """``leave_product``: the output projection may be left unmade (``Product``)."""
+    def forward(self, h: torch.Tensor, ctx: StepContext, line: KVLine, writes_cache: bool, leave_product: bool = False,
+                made: list | None = None):
+        """``leave_product``: the output projection may be left unmade (``Product``). ``made``: see ``first_products``."""
         if not self._plain(ctx.positions):
-            out = self._forward_general(h, ctx, line, writes_cache)
+            out = self._forward_general(h, ctx, line, writes_cache, made)
             return add_bias(out, self.o_bias, h.dtype) if self.has_bias else out
         late = None
         if isinstance(h, LateNormed):

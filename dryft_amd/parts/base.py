@@ -256,6 +256,11 @@ class Mixer(Part):
         (a float32 vector of the output's width)."""
         return self.forward(h, ctx, line, writes_cache), None
 
+    def first_products(self, ctx: StepContext) -> list:
+        """The products of ``h`` that the mixer begins with, ``(w, out dtype or None)``, where ``forward`` and ``forward_split``
+        take them ``made``: for a caller that makes several mixers' together. Empty: none such."""
+        return []
+
 
 class FeedForward(Part):
     row_wise = False    # does a row's output depend on that row of ``h`` alone, and on nothing that ``ctx`` says of the rows?

@@ -27,7 +27,7 @@ from ..weights.spec import VECTOR
 from . import register_part
 from .base import Mixer, StepContext, matrix
 from .conv import conv_need, short_conv
-from .linear import linear
+from .linear import linear, linears
 
 
 class GatedDeltaMixer(Mixer):
@@ -77,8 +77,8 @@ class GatedDeltaMixer(Mixer):
 
     def forward(self, h: torch.Tensor, ctx: StepContext, line, writes_cache: bool):
         rows = h.shape[0]
-        proj = linear(h, self.w_in)                                        # q | k | v | gate, in the activation dtype
-        gates = linear(h, self.w_gates, out_dtype=torch.float32)            # a | b stay float32 from here on
+        # q | k | v | gate, in the activation dtype; a | b stay float32 from here on
+        proj, gates = linears(h, [(self.w_in, None), (self.w_gates, torch.float32)])
         qkv = short_conv(proj, 0, self.conv_channels, self.conv_w, ctx, line.get("tail"), writes_cache, silu=True,
                          weight_t=self.conv_wt)
         # the rows of sequences that sit out are not visited by the walk; the read-out norms whatever they hold

@@ -387,6 +387,23 @@ def linear(x: torch.Tensor, w: torch.Tensor, *, out_dtype: torch.dtype | None = 
     return ops.gemm_tiled(x, w, out)
 
 
+def linears(x: torch.Tensor, products: list) -> list:
+    """``linear(x, w, out_dtype=dtype)`` for every ``(w, dtype)`` of ``products`` (``dtype`` None: that of ``x``): in one launch
+    for few rows whose products go to the kernel of whole lines anyway, alone and as one matrix."""
+    m, k = x.shape
+    if together_pay(x, [w for w, _ in products]):
+        outs = [torch.empty((m, w.shape[0]), dtype=dtype or x.dtype, device=x.device) for w, dtype in products]
+        ops.gemm_lines_beside(x, [(w, out) for (w, _), out in zip(products, outs)])
+        return outs
+    return [linear(x, w, out_dtype=dtype) for w, dtype in products]
+
+
+def together_pay(x: torch.Tensor, weights: list) -> bool:
+    m, k = x.shape
+    return x.dtype == torch.bfloat16 and 1 < len(weights) <= ops.LINES_TOGETHER and \
+        all(ops.lines_ok(x, w) and lines_pay(m, w.shape[0], k) for w in weights) and lines_pay(m, sum(w.shape[0] for w in weights), k)
+
+
 @contextlib.contextmanager
 def library_tuning():
     """While open, the vendor library times its candidate kernels for every product shape it meets for the

@@ -26,7 +26,7 @@ from ..csrc import ops
 from ..weights.spec import VECTOR
 from . import register_part
 from .base import Mixer, StepContext, matrix
-from .linear import linear
+from .linear import linear, linears
 from .rope import HalfRotaryPositions
 
 
@@ -96,14 +96,20 @@ class LinearAttention(Mixer):
             raise ValueError(f"position tables cover {table.n_positions} positions, the step reaches {ctx.max_kv_len}")
         return table.cos, table.sin, table.dims
 
-    def forward(self, h: torch.Tensor, ctx: StepContext, line, writes_cache: bool):
+    def first_products(self, ctx: StepContext) -> list:
+        # q | k | v | gate; the decay stays float32 from here on
+        return [(self.w_in, None)] + ([(self.w_down, torch.float32)] if self.channel_decay else [])
+
+    def forward_split(self, h, ctx, line, writes_cache, made=None):
+        return self.forward(h, ctx, line, writes_cache, **({"made": made} if made else {})), None
+
+    def forward(self, h: torch.Tensor, ctx: StepContext, line, writes_cache: bool, made: list | None = None):
         rows = h.shape[0]
-        proj = linear(h, self.w_in)                                       # q | k | v | gate
+        proj, *low = made or linears(h, self.first_products(ctx))
         logs = None
         if self.channel_decay:
-            low = linear(h, self.w_down, out_dtype=torch.float32)          # the decay stays float32 from here on
             logs = torch.empty((rows, self.qk_dim), dtype=torch.float32, device=h.device)
-            ops.log_decay(low, self.w_up, self.decay_bias, logs, 1.0 / self.channel_decay[1])
+            ops.log_decay(low[0], self.w_up, self.decay_bias, logs, 1.0 / self.channel_decay[1])
         cols = (0, self.qk_dim, 2 * self.qk_dim)
         g_col = 2 * self.qk_dim + self.v_dim
         tables = self._tables(ctx)

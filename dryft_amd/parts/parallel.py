@@ -17,7 +17,8 @@ import torch
 from ..csrc import ops
 from ..weights.spec import VECTOR
 from . import build_part, register_part
-from .base import Mixer, Partials, StepContext
+from .base import Mixer, Partials, StepContext, accepts
+from .linear import linears, together_pay
 
 
 class ParallelMixer(Mixer):
@@ -72,9 +73,9 @@ class ParallelMixer(Mixer):
         return tuple(sorted(mods))
 
     def forward(self, h: torch.Tensor, ctx: StepContext, line, writes_cache: bool):
-        outs = []
+        outs, made = [], self._first_products(h, ctx)
         for name in self.names:
-            delta, bias = self.mixers[name].forward_split(h, ctx, self._line(name, line), writes_cache)
+            delta, bias = self.mixers[name].forward_split(h, ctx, self._line(name, line), writes_cache, **made.get(name, {}))
             outs += [(delta.data, delta.count) if isinstance(delta, Partials) else delta, bias,
                      self.out_weight[name] if self.scales is None else self.scales[name]]
         out = torch.empty((1, h.shape[0], self.hidden), dtype=torch.float32, device=h.device)
@@ -83,6 +84,16 @@ class ParallelMixer(Mixer):
         else:
             ops.scaled_pair(*outs, out[0], h.dtype)
         return Partials(out, 1)                # float32, for the norm that takes it into the stream
+
+    def _first_products(self, h: torch.Tensor, ctx: StepContext) -> dict:
+        """The products that both mixers begin with, made in one launch where that pays: what goes into their calls, by name."""
+        lists = {name: mixer.first_products(ctx) for name, mixer in self.mixers.items()
+                 if accepts(mixer, "forward_split", "made") and accepts(mixer, "forward", "made")}
+        every = [one for products in lists.values() for one in products]
+        if len(lists) < 2 or not all(lists.values()) or not together_pay(h, [w for w, _ in every]):
+            return {}
+        made = iter(linears(h, every))
+        return {name: {"made": [next(made) for _ in products]} for name, products in lists.items()}
 
     def reads_whole(self) -> bool:
         return True

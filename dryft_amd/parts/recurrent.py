@@ -22,7 +22,7 @@ from ..csrc import ops
 from ..weights.spec import VECTOR
 from . import register_part
 from .base import Mixer, StepContext, matrix
-from .linear import linear
+from .linear import linear, linears
 
 
 _MAX_SEGMENTS = 8
@@ -75,8 +75,8 @@ class MatrixMemory(Mixer):
 
     def forward(self, h: torch.Tensor, ctx: StepContext, line, writes_cache: bool):
         rows = h.shape[0]
-        proj = linear(h, self.w_in)                                       # q | k | v | g, in the activation dtype
-        gates = linear(h, self.w_gates, out_dtype=torch.float32)           # the gates stay float32 from here on
+        # q | k | v | g, in the activation dtype; the gates stay float32 from here on
+        proj, gates = linears(h, [(self.w_in, None), (self.w_gates, torch.float32)])
         o_raw = torch.empty((rows, self.n_heads, self.value_dim), dtype=torch.float32, device=h.device)
         # steps of many rows in bfloat16: a chunk of tokens at a time on the matrix cores; single tokens, float32
         # and sizes without 16-byte pieces: token by token in float arithmetic

@@ -28,7 +28,7 @@ from ..weights.spec import VECTOR
 from . import register_part
 from .base import Mixer, StepContext, matrix
 from .conv import conv_need, short_conv
-from .linear import linear
+from .linear import linear, linears
 
 
 class StateSpaceMixer(Mixer):
@@ -77,10 +77,15 @@ class StateSpaceMixer(Mixer):
     def kernel_modules(self, dtype):
         return ("gemm", "conv", "ssm")
 
-    def forward(self, h: torch.Tensor, ctx: StepContext, line, writes_cache: bool):
+    def first_products(self, ctx: StepContext) -> list:
+        return [(self.w_in, None), (self.w_dt, torch.float32)]
+
+    def forward_split(self, h, ctx, line, writes_cache, made=None):
+        return self.forward(h, ctx, line, writes_cache, **({"made": made} if made else {})), None
+
+    def forward(self, h: torch.Tensor, ctx: StepContext, line, writes_cache: bool, made: list | None = None):
         rows, GN = h.shape[0], self.groups * self.n_state
-        proj = linear(h, self.w_in)
-        dt_raw = linear(h, self.w_dt, out_dtype=torch.float32)
+        proj, dt_raw = made or linears(h, self.first_products(ctx))
         xbc = short_conv(proj, self.inner, self.conv_channels, self.conv_w, ctx, line.get("tail"), writes_cache,
                          out_bias=self.conv_b, silu=True, weight_t=self.conv_wt)
         # long walks go by chunks, or as segments side by side (the rows of sequences that sit out are then not visited)

@@ -135,3 +135,33 @@ def test_replaced_calls_are_not_kept():
     del part.forward
     gc.collect()
     assert gone() is None and works_row_by_row(part)
+
+
+@pytest.mark.parametrize("name", ["forward", "forward_split"])
+def test_mixers_side_by_side_with_a_replaced_call_begin_alone(monkeypatch, name):
+    """Two mixers' first products are made together only where the calls that run take them."""
+    from dryft_amd.parts import parallel
+
+    class Begins(Mixer):
+        def first_products(self, ctx):
+            return [(torch.eye(4), None)]
+
+        def forward(self, h, ctx, line, writes_cache, made=None):
+            self.made = made
+            return (made[0] if made else h) * 2
+
+        def forward_split(self, h, ctx, line, writes_cache, made=None):
+            return self.forward(h, ctx, line, writes_cache, **({"made": made} if made else {})), None
+
+    monkeypatch.setattr(parallel, "together_pay", lambda h, weights: len(weights) == 2)
+    monkeypatch.setattr(parallel, "linears", lambda h, products: [h @ w.T for w, _ in products])
+    both = parallel.ParallelMixer.__new__(parallel.ParallelMixer)
+    both.mixers = {"left": Begins(), "right": Begins()}
+    h = torch.ones(2, 4)
+    assert {n: len(m["made"]) for n, m in both._first_products(h, STEP).items()} == {"left": 1, "right": 1}
+    if name == "forward":
+        both.mixers["left"].forward = lambda h, ctx, line, writes_cache: 3 * h
+    else:
+        both.mixers["left"].forward_split = lambda h, ctx, line, writes_cache: (3 * h, None)
+    assert both._first_products(h, STEP) == {}
+    assert torch.equal(both.mixers["left"].forward_split(h, STEP, None, True)[0], 3 * h)
