@@ -18,8 +18,10 @@
 // bytes at a time. Operands come in batches of eight tokens: while the wave walks one batch, the next one's loads
 // are in flight; the unit lengths (a sum over D per token) are taken by four lanes a vector as the batch goes to LDS.
 //
-// Most walks of 17 rows and more go sixteen rows at a time on the matrix cores instead (chunk_walk.h).
+// Most walks of 17 rows and more go sixteen rows at a time on the matrix cores instead (chunk_walk.h), steps of one row a sequence
+// through a kernel of their own that ends with the read-out's norm and gate (token_step.h).
 #include "chunk_walk.h"
+#include "token_step.h"
 
 #define DELTA_MAX_DIM 256
 #define DELTA_BATCH 8            // tokens whose operands are brought into LDS together
@@ -324,6 +326,18 @@ DRYFT_API int dryft_delta_steps(const void* qkv, int64_t qkv_stride, int q_col, 
 #undef DELTA_CASE
 #undef DELTA_LAUNCH
   return DRYFT_LAUNCH_CHECK();
+}
+
+// Steps of one row a sequence, with the read-out: out[row, head] = o / sqrt(mean(o^2) + eps) * weight * silu(out_gate) in the
+// activation dtype; -2 for sizes that the kernel does not take.
+DRYFT_API int dryft_delta_token(const void* qkv, int64_t qkv_stride, int q_col, int k_col, int v_col, const float* gates,
+                                int64_t gate_stride, int a_col, int b_col, const float* dt_bias, const float* a_log,
+                                const int* seq_slot, const int* cu_rows, const int* q_len, float* state, const void* out_gate,
+                                int64_t out_gate_stride, const float* weight, float eps, void* out, int n_seqs, int H, int G, int D,
+                                int P, float q_scale, float unit_eps, int write_state, int is_f32, hipStream_t stream) {
+  const TokenStep a = {qkv_stride, q_col, k_col, v_col, gates, gate_stride, a_col, b_col, dt_bias, a_log, nullptr, seq_slot, cu_rows,
+                       q_len, state, H, G, D, P, q_scale, unit_eps, write_state, out_gate_stride, weight, eps};
+  return token_step_run<true>(qkv, out_gate, out, a, n_seqs, is_f32, stream);
 }
 
 // Whole sequences, sixteen tokens at a time on the matrix cores; -2 for shapes that the kernel does not take.

@@ -126,11 +126,14 @@ _SIGNATURES = {
              "dryft_conv_step": [_P, _L, _I, _P, _P, _P, _P, _I, _I, _P, _P, _P, _P, _I, _I, _I, _P],
              "dryft_conv_tail": [_P, _L, _I, _P, _I, _P, _P, _P, _P, _I, _I, _I, _P]},
     "ssm": {"dryft_ssm_max_state": [],
+            "dryft_ssm_token": [_P, _L, _I, _I, _I, _P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
             "dryft_ssm_scan": [_P, _L, _I, _I, _I, _P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I,
                                _I, _P, _P, _I, _P],
             "dryft_ssm_chunks": [_P, _L, _I, _I, _I, _P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
             "dryft_gate_part_norm": [_P, _P, _L, _I, _P, _P, _P, _I, _I, _I, _F, _I, _P]},
     "delta": {"dryft_delta_max_dim": [],
+              "dryft_delta_token": [_P, _L, _I, _I, _I, _P, _L, _I, _I, _P, _P, _P, _P, _P, _P, _P, _L, _P, _F, _P, _I, _I, _I, _I, _I, _F, _F, _I,
+                                    _I, _P],
               "dryft_delta_steps": [_P, _L, _I, _I, _I, _P, _L, _I, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I,
                                     _F, _F, _I, _P, _I, _I, _P, _P, _I, _P],
               "dryft_delta_chunks": [_P, _L, _I, _I, _I, _P, _L, _I, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I,
@@ -2672,6 +2675,16 @@ def _walks_by_chunks(x, k_col: int, q_col: int, rows_of_state: int, columns: int
     return by_chunks < cut_fixed + cut_row * longest + cut_values * 1e-6 * x.shape[0] * n_heads * rows_of_state * columns
 
 
+def token_step_takes(state) -> bool:
+    """Can a step of one row a sequence go to the kernel that takes a (sequence, head) a workgroup? By the state's sizes ``[slots,
+    heads, rows, columns]``."""
+    return state.shape[2] <= TOKEN_MAX_DIM and state.shape[3] in (32, 64, 128, 256) and state.shape[1] <= 65535 and \
+        state.data_ptr() % 16 == 0
+
+
+TOKEN_MAX_DIM = 256
+
+
 def ssm_scan(xbc, x_col: int, b_col: int, c_col: int, dt_raw, dt_bias, a_log, d_skip, seq_slot, cu_rows, q_len,
              n_seqs: int, state, y, n_heads: int, head_dim: int, n_state: int, groups: int, write_state: bool,
              segments=None, longest: int = 0) -> None:
@@ -2711,6 +2724,12 @@ def ssm_scan(xbc, x_col: int, b_col: int, c_col: int, dt_raw, dt_bias, a_log, d_
             _ptr(xbc), xbc.stride(0), x_col, b_col, c_col, _ptr(dt_raw), dt_raw.stride(0), _ptr(dt_bias), _ptr(a_log),
             _ptr(d_skip), _ptr(seq_slot), _ptr(cu_rows), _ptr(q_len), _ptr(state), _ptr(y), n_seqs, n_heads, head_dim,
             n_state, groups, int(bool(write_state)), _float_flag(xbc, "xbc"), _stream()), "ssm_chunks")
+        return
+    if segments is None and longest == 1 and token_step_takes(state):
+        _check(_fn("ssm", "dryft_ssm_token")(
+            _ptr(xbc), xbc.stride(0), x_col, b_col, c_col, _ptr(dt_raw), dt_raw.stride(0), _ptr(dt_bias), _ptr(a_log),
+            _ptr(d_skip), _ptr(seq_slot), _ptr(cu_rows), _ptr(q_len), _ptr(state), _ptr(y), n_seqs, n_heads, head_dim,
+            n_state, groups, int(bool(write_state)), _float_flag(xbc, "xbc"), _stream()), "ssm_token")
         return
     seg_state = seg_decay = None
     if segments is not None:
@@ -2798,6 +2817,41 @@ def delta_steps(qkv, q_col: int, k_col: int, v_col: int, gates, a_col: int, b_co
         _ptr(a_log), _ptr(seq_slot), _ptr(cu_rows), _ptr(q_len), _ptr(state), _ptr(out), n_seqs, n_heads, n_groups,
         key_dim, value_dim, float(q_scale), float(unit_eps), int(bool(write_state)), _ptr(seg_cu), max_segs, seg_rows,
         _ptr(seg_state), _ptr(seg_trans), _float_flag(qkv, "qkv"), _stream()), "delta_steps")
+
+
+def delta_token(qkv, q_col: int, k_col: int, v_col: int, gates, a_col: int, b_col: int, dt_bias, a_log, seq_slot, cu_rows, q_len,
+                n_seqs: int, state, gate, weight, norm_eps: float, out, n_heads: int, n_groups: int, key_dim: int, value_dim: int,
+                q_scale: float, unit_eps: float, write_state: bool) -> None:
+    """``delta_steps`` for a step in which no sequence has more than one row (``token_step_takes``), and ``wkv_out`` on what it reads:
+    ``out`` ``[rows, heads * value_dim]`` in the dtype of ``qkv`` (rows of sequences that sit out become zeros), ``gate`` a run of
+    columns of a tensor of that dtype, ``weight`` float32 ``[heads * value_dim]``."""
+    _gpu(qkv, "qkv")
+    rows, inner = qkv.shape[0], n_heads * value_dim
+    if not (qkv.dim() == 2 and qkv.stride(1) == 1 and min(q_col, k_col, v_col) >= 0 and
+            max(q_col + n_groups * key_dim, k_col + n_groups * key_dim, v_col + inner) <= qkv.shape[1]):
+        raise KernelError("delta_token: q, k or v lie outside the columns of qkv")
+    _gpu(gates, "gates", torch.float32)
+    if not (gates.dim() == 2 and gates.shape[0] == rows and gates.stride(1) == 1 and min(a_col, b_col) >= 0 and
+            max(a_col, b_col) + n_heads <= gates.shape[1]):
+        raise KernelError("delta_token: gates must be float32 [rows, columns] that hold a and b for every head")
+    _f32_vector(dt_bias, "dt_bias", n_heads)
+    _f32_vector(a_log, "a_log", n_heads)
+    _f32_vector(weight, "weight", inner)
+    _seq_facts(seq_slot, cu_rows, q_len, n_seqs)
+    _gpu(state, "state", torch.float32)
+    _gpu(gate, "gate", qkv.dtype)
+    _gpu(out, "out", qkv.dtype)
+    if not (state.dim() == 4 and state.shape[1:] == (n_heads, key_dim, value_dim) and state.is_contiguous() and token_step_takes(state)):
+        raise KernelError(f"delta_token: state must be contiguous float32 [slots, {n_heads}, {key_dim}, {value_dim}] of sizes it takes")
+    if not (gate.shape == (rows, inner) and gate.stride(1) == 1 and out.shape == (rows, inner) and out.is_contiguous()):
+        raise KernelError(f"delta_token: gate [rows, {inner}] with unit column stride, out contiguous [rows, {inner}]")
+    if not (n_groups > 0 and n_heads % n_groups == 0):
+        raise KernelError("delta_token: heads a multiple of the key heads")
+    _check(_fn("delta", "dryft_delta_token")(
+        _ptr(qkv), qkv.stride(0), q_col, k_col, v_col, _ptr(gates), gates.stride(0), a_col, b_col, _ptr(dt_bias), _ptr(a_log),
+        _ptr(seq_slot), _ptr(cu_rows), _ptr(q_len), _ptr(state), _ptr(gate), gate.stride(0), _ptr(weight), float(norm_eps), _ptr(out),
+        n_seqs, n_heads, n_groups, key_dim, value_dim, float(q_scale), float(unit_eps), int(bool(write_state)),
+        _float_flag(qkv, "qkv"), _stream()), "delta_token")
 
 
 # ------------------------------------------------------------------------------------------ linear attention

@@ -14,8 +14,10 @@
 // every column: they wait in LDS, one run per lane of a column (runs a bank apart), read 16 bytes at a time.
 // Operands come in batches of eight tokens; the next batch's loads are in flight while the wave walks this one.
 //
-// Most walks of 17 rows and more go sixteen rows at a time on the matrix cores instead (chunk_walk.h).
+// Most walks of 17 rows and more go sixteen rows at a time on the matrix cores instead (chunk_walk.h), steps of one row a sequence
+// through a kernel of their own (token_step.h).
 #include "chunk_walk.h"
+#include "token_step.h"
 
 #define SSM_MAX_STATE 256
 #define SSM_BATCH 8              // tokens whose operands are brought into LDS together
@@ -290,6 +292,16 @@ DRYFT_API int dryft_ssm_scan(const void* xbc, int64_t xbc_stride, int x_col, int
 #undef SSM_CASE
 #undef SSM_LAUNCH
   return DRYFT_LAUNCH_CHECK();
+}
+
+// Steps of one row a sequence; -2 for sizes that the kernel does not take.
+DRYFT_API int dryft_ssm_token(const void* xbc, int64_t xbc_stride, int x_col, int b_col, int c_col, const float* dt_raw,
+                              int64_t dt_stride, const float* dt_bias, const float* a_log, const float* d_skip, const int* seq_slot,
+                              const int* cu_rows, const int* q_len, float* state, float* y, int n_seqs, int H, int P, int N, int G,
+                              int write_state, int is_f32, hipStream_t stream) {
+  const TokenStep a = {xbc_stride, c_col, b_col, x_col, dt_raw, dt_stride, 0, 0, dt_bias, a_log, d_skip, seq_slot, cu_rows,
+                       q_len, state, H, G, N, P, 1.f, 0.f, write_state, 0, nullptr, 0.f};
+  return token_step_run<false>(xbc, nullptr, y, a, n_seqs, is_f32, stream);
 }
 
 DRYFT_API int dryft_gate_part_norm(const float* y, const void* z, int64_t z_stride, int z_col, const float* w,

@@ -81,6 +81,14 @@ class GatedDeltaMixer(Mixer):
         proj, gates = linears(h, [(self.w_in, None), (self.w_gates, torch.float32)])
         qkv = short_conv(proj, 0, self.conv_channels, self.conv_w, ctx, line.get("tail"), writes_cache, silu=True,
                          weight_t=self.conv_wt)
+        if ctx.max_q_len == 1 and ops.token_step_takes(line["memory"].state):
+            # one row a sequence: the walk and its read-out in one launch
+            out = torch.empty((rows, self.v_dim), dtype=h.dtype, device=h.device)
+            ops.delta_token(qkv, 0, self.qk_dim, 2 * self.qk_dim, gates, 0, self.n_heads, self.dt_bias, self.a_log, ctx.seq_slot,
+                            ctx.cu_rows, ctx.q_len, ctx.n_seqs, line["memory"].state, proj[:, self.conv_channels:], self.out_norm,
+                            self.norm_eps, out, self.n_heads, self.n_kv, self.key_dim, self.value_dim, self.key_dim ** -0.5,
+                            self.unit_eps, writes_cache)
+            return linear(out, self.w_o, allow_partials=True)
         # the rows of sequences that sit out are not visited by the walk; the read-out norms whatever they hold
         o_raw = ctx.kept_zeros((rows, self.v_dim), torch.float32) if ctx.some_sit_out() else \
             torch.empty((rows, self.v_dim), dtype=torch.float32, device=h.device)
