@@ -30,7 +30,7 @@ MODULES = ("batch", "embed", "norm", "activation", "rope_kv", "attn_rows", "attn
            "rglru", "hyper", "wkv", "latent", "moe", "conv", "ssm", "delta", "linattn", "mla")
 _HEADERS = ("common.h",)                       # every library includes these
 _OWN_HEADERS = {"gemm": ("gate_unit.h",), "gemm_lines": ("gate_unit.h",), "moe": ("gate_unit.h",), "sampling": ("sampling.h",),
-                "delta": ("chunk_walk.h", "token_step.h"), "ssm": ("chunk_walk.h", "token_step.h")}    # and some a header of their own
+                "delta": ("chunk_walk.h", "token_step.h"), "ssm": ("chunk_walk.h", "token_step.h"), "mlstm": ("token_step.h",)}    # and some a header of their own
 
 _loaded: dict[str, ctypes.CDLL] = {}
 _lock = threading.Lock()

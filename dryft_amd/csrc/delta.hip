@@ -336,8 +336,8 @@ DRYFT_API int dryft_delta_token(const void* qkv, int64_t qkv_stride, int q_col, 
                                 int64_t out_gate_stride, const float* weight, float eps, void* out, int n_seqs, int H, int G, int D,
                                 int P, float q_scale, float unit_eps, int write_state, int is_f32, hipStream_t stream) {
   const TokenStep a = {qkv_stride, q_col, k_col, v_col, gates, gate_stride, a_col, b_col, dt_bias, a_log, nullptr, seq_slot, cu_rows,
-                       q_len, state, H, G, D, P, q_scale, unit_eps, write_state, out_gate_stride, weight, eps};
-  return token_step_run<true>(qkv, out_gate, out, a, n_seqs, is_f32, stream);
+                       q_len, state, H, G, D, P, q_scale, unit_eps, write_state, out_gate_stride, weight, eps, 0.f, nullptr, nullptr, 0};
+  return token_step_run<TOKEN_DELTA>(qkv, out_gate, out, a, n_seqs, is_f32, stream);
 }
 
 // Whole sequences, sixteen tokens at a time on the matrix cores; -2 for shapes that the kernel does not take.

@@ -16,8 +16,10 @@
 // lane of a wave the same entries), whose product with q goes through the same reduction as one more column.
 // Tokens are staged through LDS a tile at a time. n and m are kept once per run of 64 value columns
 // ([.., heads, runs, D] and [.., heads, runs]): every workgroup reads and writes its own copy, so none ever
-// reads what another has already updated.
+// reads what another has already updated. Steps of one row a sequence go to a kernel of their own that ends with the read-out's norm
+// and gate (token_step.h).
 #include "common.h"
+#include "token_step.h"
 
 #define MLSTM_COLS 64            // value columns a workgroup owns
 #define MLSTM_RED (MLSTM_COLS + 1)  // a wave's partial sums: its columns, then n . q
@@ -154,6 +156,20 @@ DRYFT_API int dryft_mlstm_steps(const void* proj, int64_t proj_stride, int q_col
 #undef ML_T
 #undef ML
   return DRYFT_LAUNCH_CHECK();
+}
+
+// Steps of one row a sequence, with what mlstm_out_kernel does to the read-out; -2 for sizes that the kernel does not take.
+DRYFT_API int dryft_mlstm_token(const void* proj, int64_t proj_stride, int q_col, int k_col, int v_col, int g_col, const float* gates,
+                                const float* bias_i, const float* bias_f, float cap, const int* seq_slot, const int* cu_rows,
+                                const int* q_len, int n_seqs, float* state_s, float* state_n, float* state_m, const float* weight,
+                                float eps, void* out, int n_heads, int dim, int v_dim, float q_scale, int write_state, int is_f32,
+                                hipStream_t stream) {
+  if (!(cap > 0.f)) return -1;
+  const int64_t row_bytes = is_f32 ? sizeof(float) : sizeof(bf16_t);
+  const TokenStep a = {proj_stride, q_col, k_col, v_col, gates, 2 * n_heads, 0, n_heads, bias_i, bias_f, nullptr, seq_slot, cu_rows,
+                       q_len, state_s, n_heads, n_heads, dim, v_dim, q_scale, 0.f, write_state, proj_stride, weight, eps, cap,
+                       state_n, state_m, (v_dim + MLSTM_COLS - 1) / MLSTM_COLS};
+  return token_step_run<TOKEN_MEMORY>(proj, (const char*)proj + g_col * row_bytes, out, a, n_seqs, is_f32, stream);
 }
 
 // out[row, head * v_dim + c] = T( o / sqrt(mean_c(o^2) + eps) * w[head * v_dim + c] * sigmoid(g) ): each head's

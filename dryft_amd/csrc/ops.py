@@ -38,6 +38,7 @@ _SIGNATURES = {
                    "dryft_blend_columns": [_P, _L, _P, _L, _P, _I, _I, _I, _P]},
     "mlstm": {"dryft_mlstm_steps": [_P, _L, _I, _I, _I, _P, _P, _P, _F, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _F,
                                     _I, _I, _P],
+              "dryft_mlstm_token": [_P, _L, _I, _I, _I, _I, _P, _P, _P, _F, _P, _P, _P, _I, _P, _P, _P, _P, _F, _P, _I, _I, _I, _F, _I, _I, _P],
               "dryft_mlstm_chunks_takes": [_I, _I, _I, _I, _I, _L],
               "dryft_mlstm_chunks": [_P, _L, _I, _I, _I, _P, _P, _P, _F, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _F,
                                      _I, _I, _P, _I, _P, _P],
@@ -1826,6 +1827,40 @@ def mlstm_steps(proj, q_col: int, k_col: int, v_col: int, gates, bias_i, bias_f,
         _ptr(proj), proj.stride(0), q_col, k_col, v_col, _ptr(gates), _ptr(bias_i), _ptr(bias_f), float(cap),
         _ptr(seq_slot), _ptr(cu_rows), _ptr(q_len), n_seqs, _ptr(state_s), _ptr(state_n), _ptr(state_m), _ptr(o_raw),
         n_heads, dim, v_dim, float(q_scale), int(bool(write_state)), is_f32, _stream()), "mlstm_steps")
+
+
+def mlstm_token(proj, q_col: int, k_col: int, v_col: int, g_col: int, gates, bias_i, bias_f, cap: float, seq_slot, cu_rows, q_len,
+                n_seqs: int, state_s, state_n, state_m, weight, eps: float, out, n_heads: int, dim: int, v_dim: int, q_scale: float,
+                write_state: bool) -> None:
+    """``mlstm_steps`` for a step in which no sequence has more than one row (``token_step_takes``), and ``mlstm_out`` on what it
+    reads: ``out`` ``[rows, heads * v_dim]`` in the dtype of ``proj``, rows of sequences that sit out become zeros."""
+    _gpu(proj, "proj")
+    rows, inner = proj.shape[0], n_heads * v_dim
+    if not (proj.dim() == 2 and proj.stride(1) == 1 and min(q_col, k_col, v_col, g_col) >= 0 and
+            max(q_col + n_heads * dim, k_col + n_heads * dim, v_col + inner, g_col + inner) <= proj.shape[1]):
+        raise KernelError("mlstm_token: q, k, v or the gate lie outside the projection's columns")
+    _gpu(gates, "gates", torch.float32)
+    if not (gates.shape == (rows, 2 * n_heads) and gates.is_contiguous()):
+        raise KernelError(f"mlstm_token: gates must be contiguous float32 [{rows}, {2 * n_heads}]")
+    _f32_vector(bias_i, "bias_i", n_heads)
+    _f32_vector(bias_f, "bias_f", n_heads)
+    _f32_vector(weight, "weight", inner)
+    _seq_facts(seq_slot, cu_rows, q_len, n_seqs)
+    slots, runs = state_m.shape[0], -(-v_dim // MLSTM_COLUMNS)
+    for name, t, shape in (("state_s", state_s, (slots, n_heads, dim, v_dim)),
+                           ("state_n", state_n, (slots, n_heads, runs, dim)), ("state_m", state_m, (slots, n_heads, runs))):
+        _gpu(t, name, torch.float32)
+        if not (tuple(t.shape) == shape and t.is_contiguous()):
+            raise KernelError(f"{name}: must be contiguous float32 {shape}, got {tuple(t.shape)}")
+    if not token_step_takes(state_s):
+        raise KernelError(f"mlstm_token: a state of {dim} x {v_dim} goes token by token to mlstm_steps")
+    _gpu(out, "out", proj.dtype)
+    if not (out.shape == (rows, inner) and out.is_contiguous()):
+        raise KernelError(f"mlstm_token: out must be contiguous [{rows}, {inner}]")
+    _check(_fn("mlstm", "dryft_mlstm_token")(
+        _ptr(proj), proj.stride(0), q_col, k_col, v_col, g_col, _ptr(gates), _ptr(bias_i), _ptr(bias_f), float(cap), _ptr(seq_slot),
+        _ptr(cu_rows), _ptr(q_len), n_seqs, _ptr(state_s), _ptr(state_n), _ptr(state_m), _ptr(weight), float(eps), _ptr(out), n_heads,
+        dim, v_dim, float(q_scale), int(bool(write_state)), _float_flag(proj, "proj"), _stream()), "mlstm_token")
 
 
 def mlstm_out(o_raw, proj, g_col: int, weight, row_slot, out, n_heads: int, v_dim: int, eps: float) -> None:

@@ -300,8 +300,8 @@ DRYFT_API int dryft_ssm_token(const void* xbc, int64_t xbc_stride, int x_col, in
                               const int* cu_rows, const int* q_len, float* state, float* y, int n_seqs, int H, int P, int N, int G,
                               int write_state, int is_f32, hipStream_t stream) {
   const TokenStep a = {xbc_stride, c_col, b_col, x_col, dt_raw, dt_stride, 0, 0, dt_bias, a_log, d_skip, seq_slot, cu_rows,
-                       q_len, state, H, G, N, P, 1.f, 0.f, write_state, 0, nullptr, 0.f};
-  return token_step_run<false>(xbc, nullptr, y, a, n_seqs, is_f32, stream);
+                       q_len, state, H, G, N, P, 1.f, 0.f, write_state, 0, nullptr, 0.f, 0.f, nullptr, nullptr, 0};
+  return token_step_run<TOKEN_SSM>(xbc, nullptr, y, a, n_seqs, is_f32, stream);
 }
 
 DRYFT_API int dryft_gate_part_norm(const float* y, const void* z, int64_t z_stride, int z_col, const float* w,

@@ -77,6 +77,14 @@ class MatrixMemory(Mixer):
         rows = h.shape[0]
         # q | k | v | g, in the activation dtype; the gates stay float32 from here on
         proj, gates = linears(h, [(self.w_in, None), (self.w_gates, torch.float32)])
+        if ctx.max_q_len == 1 and ops.token_step_takes(line["memory"].state):
+            # one row a sequence: the walk and its read-out in one launch
+            out = torch.empty((rows, self.v_dim), dtype=h.dtype, device=h.device)
+            ops.mlstm_token(proj, 0, self.qk_dim, 2 * self.qk_dim, 2 * self.qk_dim + self.v_dim, gates, self.bias_i, self.bias_f,
+                            self.gate_cap, ctx.seq_slot, ctx.cu_rows, ctx.q_len, ctx.n_seqs, line["memory"].state,
+                            line["normaliser"].state, line["maximum"].state, self.out_norm, self.norm_eps, out, self.n_heads,
+                            self.key_dim, self.value_dim, self.key_dim ** -0.5, writes_cache)
+            return linear(out, self.w_o, allow_partials=True)
         o_raw = torch.empty((rows, self.n_heads, self.value_dim), dtype=torch.float32, device=h.device)
         # steps of many rows in bfloat16: a chunk of tokens at a time on the matrix cores; single tokens, float32
         # and sizes without 16-byte pieces: token by token in float arithmetic

@@ -1,4 +1,4 @@
-"""One row a sequence through the delta rule (with its read-out) and the state-space recurrence, against 64-bit walks: the narrowest
+"""One row a sequence through the delta rule and the matrix memory (with their read-outs) and the state-space recurrence, against 64-bit walks: the narrowest
 and widest states, rows that do not fill the row groups, several heads a group, sequences that sit out or have no row, states left
 as they were."""
 import pytest
@@ -59,3 +59,49 @@ def test_one_row_a_sequence(dtype, write, kind, H, G, D, P, rate):
     for slot in range(n + 2):
         if not write or slot not in {s for s, q in zip(SLOTS, ROWS) if q}:
             assert torch.equal(got_state[slot], state[slot].double())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("write", [True, False])
+@pytest.mark.parametrize("H,D,P,bias", [(4, 128, 256, 0.0), (2, 256, 64, 9.0), (3, 8, 32, -30.0), (2, 130, 128, 0.0)])
+def test_one_row_of_a_matrix_memory(dtype, write, H, D, P, bias):
+    from dryft_amd.csrc import ops
+    g = torch.Generator().manual_seed(D + P + H)
+    n, rows, eps, cap, runs = len(SLOTS), sum(ROWS), 1e-6, 15.0, -(-P // 64)
+    x = torch.randn(rows, 2 * H * D + 2 * H * P + 3, generator=g).to(dtype)
+    gates, weight = torch.randn(rows, 2 * H, generator=g), torch.randn(H * P, generator=g)
+    bi, bf = torch.randn(H, generator=g), torch.randn(H, generator=g) + bias       # forget gates: hardly, half, at once
+    S0, N0 = torch.randn(n + 2, H, D, P, generator=g), torch.randn(n + 2, H, 1, D, generator=g).repeat(1, 1, runs, 1)
+    m0 = torch.randn(n + 2, H, 1, generator=g).repeat(1, 1, runs)
+    dev, ints = (lambda t: t.to(DEV)), (lambda v: torch.tensor(v, dtype=torch.int32, device=DEV))
+    cu = [0] + torch.tensor(ROWS).cumsum(0).tolist()
+    S, N, m, out = dev(S0.clone()), dev(N0.clone()), dev(m0.clone()), torch.full((rows, H * P), 7.0, device=DEV, dtype=dtype)
+    ops.mlstm_token(dev(x), 0, H * D, 2 * H * D, 2 * H * D + H * P, dev(gates), dev(bi), dev(bf), cap, ints(SLOTS), ints(cu), ints(ROWS), n,
+                    S, N, m, dev(weight), eps, out, H, D, P, D ** -0.5, write)
+    out, S, N, m = (t.double().cpu() for t in (out, S, N, m))
+    for s, (slot, q) in enumerate(zip(SLOTS, ROWS)):
+        r = cu[s]
+        if slot < 0 or not q:
+            assert slot >= 0 or not out[r].any()
+            continue
+        xs = x[r].double()
+        qv, k = xs[:H * D].view(H, D) * D ** -0.5, xs[H * D:2 * H * D].view(H, D)
+        v, gate = (xs[2 * H * D + i * H * P:2 * H * D + (i + 1) * H * P].view(H, P) for i in (0, 1))
+        soft = lambda t: cap * torch.tanh(t.double() / cap)
+        gi, gf = soft(gates[r, :H].double() + bi.double()), torch.nn.functional.logsigmoid(soft(gates[r, H:].double() + bf.double()))
+        mm = torch.maximum(gf + m0[slot, :, 0].double(), gi)
+        keep, take = torch.exp(gf + m0[slot, :, 0].double() - mm)[:, None], torch.exp(gi - mm)[:, None]
+        want_n = keep * N0[slot, :, 0].double() + take * k
+        want_s = keep[:, :, None] * S0[slot].double() + (take * k)[:, :, None] * v[:, None, :]
+        o = (want_s * qv[:, :, None]).sum(1) / (torch.maximum((want_n * qv).sum(1).abs(), torch.exp(-mm)) + 1e-6)[:, None]
+        by = (o.pow(2).mean(-1, keepdim=True) + eps).rsqrt() * weight.double().view(H, P) * torch.sigmoid(gate)
+        # the read-out's sums as in TOL, of each head's own size after its norm (the normaliser's error cancels in the norm)
+        tol = TOL * 4 * by.abs().amax() / (o.pow(2).mean(-1) + eps).rsqrt().amin() * (o.pow(2).mean(-1) + eps).rsqrt().amax() + 1e-5
+        tol = tol + ((o * by).abs() * 2.0 ** -8 if dtype == torch.bfloat16 else 0.0)
+        assert bool(((out[r].view(H, P) - o * by).abs() <= tol).all()), (slot, float((out[r].view(H, P) - o * by).abs().max()))
+        if write:
+            assert float((S[slot] - want_s).abs().max()) <= TOL * 4 * float(want_s.pow(2).mean().sqrt()) + TOL
+            assert float((N[slot] - want_n[:, None]).abs().max()) <= TOL * 4 and float((m[slot] - mm[:, None]).abs().max()) <= TOL * 4
+    for slot in range(n + 2):
+        if not write or slot not in {s for s, q in zip(SLOTS, ROWS) if q}:
+            assert all(torch.equal(a[slot], b[slot].double()) for a, b in ((S, S0), (N, N0), (m, m0)))
