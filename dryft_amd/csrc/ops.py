@@ -48,6 +48,7 @@ _SIGNATURES = {
               "dryft_rglru_tile_rows": [],
               "dryft_rglru_scan_tiles": [_P, _P, _P, _L, _I, _I, _P, _P, _I, _P, _P, _P, _P, _I, _I, _P, _P, _P, _I, _I,
                                          _I, _P],
+              "dryft_rglru_token": [_P, _L, _I, _I, _P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _F, _P, _P, _P, _P, _I, _I, _I, _I, _P],
               "dryft_rglru_scan": [_P, _P, _L, _I, _I, _P, _P, _I, _P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _P]},
     "rope_kv": {"dryft_qk_norm_rope_kv": [_P, _L, _P, _P, _I, _I, _F, _P, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I,
                                           _I, _I, _I, _I, _I, _P],
@@ -1954,6 +1955,57 @@ def rglru_scan(coef, proj, x_col: int, y_col: int, x_bias, y_bias, taps: int, se
         _ptr(coef), _ptr(proj), proj.stride(0), x_col, y_col, _ptr(x_bias), _ptr(y_bias), taps, _ptr(seq_slot),
         _ptr(cu_rows), _ptr(q_len), _ptr(row_slot), n_seqs, _ptr(state), _ptr(tail) if taps > 1 else 0, _ptr(out), rows,
         width, int(bool(write_state)), _float_flag(proj, "proj"), _stream()), "rglru_scan")
+
+
+RGLRU_TOKEN_BLOCK = 256
+
+
+def rglru_token_takes(proj, state, gate_a, gate_i, vectors, blocks: int) -> bool:
+    """Does ``rglru_token`` take these tensors, and gain by it: bfloat16, blocks of a multiple of 32 channels up to ``RGLRU_TOKEN_BLOCK``, the state, the
+    gates and the ``vectors`` (gate biases, lam, y_bias) at 16-byte addresses; up to 16 rows only blocks of at most 128 channels (4 rows of
+    blocks of 256: 18.4 us against 13.9 for gates and walk, 64 rows 25 against 121; 4 rows of blocks of 128 8.1 against 12.1)."""
+    size = state.shape[1] // blocks if blocks > 0 else 0
+    return proj.dtype == torch.bfloat16 and size % 32 == 0 and 0 < size <= (RGLRU_TOKEN_BLOCK if proj.shape[0] > 16 else 128) and \
+        all(t.data_ptr() % 16 == 0 for t in (state, gate_a, gate_i, *vectors))
+
+
+def rglru_token(proj, x_col: int, y_col: int, x_bias, y_bias, conv_w, conv_b, taps: int, gate_a, gate_a_bias, gate_i, gate_i_bias, lam,
+                decay_scale: float, row_slot, state, tail, out, width: int, blocks: int, write_state: bool) -> None:
+    """``rglru_gates`` and ``rglru_scan`` for a step in which no sequence has more than one row (``rglru_token_takes``)."""
+    _gpu(proj, "proj", torch.bfloat16)
+    rows = proj.shape[0]
+    if not (proj.dim() == 2 and proj.stride(1) == 1 and min(x_col, y_col) >= 0 and max(x_col, y_col) + width <= proj.shape[1]):
+        raise KernelError("rglru_token: a branch lies outside the projection's columns")
+    if blocks <= 0 or width % blocks or not 1 <= taps <= RGLRU_MAX_TAPS:
+        raise KernelError(f"rglru_token: {width} channels in {blocks} blocks, {taps} taps")
+    size = width // blocks
+    for name, t in (("gate_a", gate_a), ("gate_i", gate_i)):
+        _gpu(t, name, proj.dtype)
+        if not (tuple(t.shape) == (blocks, size, size) and t.is_contiguous()):
+            raise KernelError(f"{name}: must be contiguous [{blocks}, {size}, {size}]")
+    for name, t in (("x_bias", x_bias), ("y_bias", y_bias), ("conv_b", conv_b), ("gate_a_bias", gate_a_bias),
+                    ("gate_i_bias", gate_i_bias), ("lam", lam)):
+        _f32_vector(t, name, width)
+    _f32_vector(conv_w, "conv_w", width * taps)
+    _gpu(row_slot, "row_slot", torch.int32)
+    if not (row_slot.is_contiguous() and row_slot.numel() >= rows):
+        raise KernelError(f"row_slot: needs {rows} contiguous entries")
+    _gpu(state, "state", torch.float32)
+    if not (state.dim() == 2 and state.shape[1] == width and state.is_contiguous()):
+        raise KernelError(f"state: must be contiguous float32 [slots, {width}]")
+    if taps > 1:
+        _gpu(tail, "tail", torch.float32)
+        if not (tuple(tail.shape) == (state.shape[0], taps - 1, width) and tail.is_contiguous()):
+            raise KernelError(f"tail: must be contiguous float32 [slots, {taps - 1}, {width}]")
+    _gpu(out, "out", proj.dtype)
+    if not (tuple(out.shape) == (rows, width) and out.is_contiguous()):
+        raise KernelError(f"out: must be contiguous [{rows}, {width}]")
+    if not rglru_token_takes(proj, state, gate_a, gate_i, (gate_a_bias, gate_i_bias, lam, y_bias), blocks):
+        raise KernelError(f"rglru_token: blocks of {size} channels, {rows} rows or addresses that it does not take")
+    _check(_fn("rglru", "dryft_rglru_token")(
+        _ptr(proj), proj.stride(0), x_col, y_col, _ptr(x_bias), _ptr(y_bias), _ptr(conv_w), _ptr(conv_b), taps, _ptr(gate_a),
+        _ptr(gate_a_bias), _ptr(gate_i), _ptr(gate_i_bias), _ptr(lam), float(decay_scale), _ptr(row_slot), _ptr(state),
+        _ptr(tail) if taps > 1 else 0, _ptr(out), rows, width, blocks, int(bool(write_state)), _stream()), "rglru_token")
 
 
 RGLRU_TILE = 64         # tokens of a sequence that one workgroup of the tiled walk takes (``ctx.tiles``)

@@ -10,7 +10,7 @@
 // store (zero when a sequence starts); everything above is float arithmetic and only out is rounded.
 // Two kernels: the gates of every row at once (a workgroup takes a few rows of one block, so that each
 // gate weight it reads serves all of them), then the walk over a sequence's rows, one thread a channel,
-// which also leaves the state for the next step.
+// which also leaves the state for the next step. Steps of one row a sequence take both in one launch (rglru_token_kernel).
 #include "common.h"
 
 #define RG_ROWS 8               // rows a gates workgroup takes
@@ -392,6 +392,181 @@ __global__ __launch_bounds__(256) void rglru_gates_mfma_kernel(
     *(vf4*)dst = va;
     *(vf4*)(dst + width) = vb;
   }
+}
+
+// ---------------------------------------------------------------------------------------------------
+// Steps of one row a sequence (decoding) in bfloat16: gates, walk and convolution memory in one launch, with the formulas and the order
+// of the sums of the kernels above. A workgroup takes 16 rows of one block of at most RG_TOKEN_BLOCK channels, a wave 16 of its outputs.
+// Everything is asked for at the start, the convolution's inputs first. Rows of 128 or 256 weights come as whole lines, four rows of 256
+// bytes a load: lane (c, g) holds 16-byte piece 4 (c % 4) + g of row 4 (c / 4) + j, which the matrix instruction takes as 16 operand rows
+// of a quarter row each; against quarter s of u, register s of a lane is the part of output 4 g + j that this quarter gives (as 16 rows of
+// 64 bytes a load the weights of 128 / 256 channels took 3 / 13 us more: half lines cost a look-up each). All outputs of a block stay in one
+// workgroup: a second one would read the convolution's memory while the first moves it on.
+// Bound by trips to memory one after the other: a row's slot, its inputs; the weights are 2 x 32 KB a workgroup at 128 channels.
+// 2,048 channels in blocks of 128, 4 / 16 / 64 / 256 rows: 8.1, 11.0, 11.4 and 12.9 us, where gates and walk took 12.1, 15.7, 57 and 62.
+// Blocks of 256: 18.4, 23.7, 25 and 28 us against 13.9, 23.5, 121 and 136, since up to 16 rows the gates' outputs go over four workgroups
+// there: such steps keep the two launches.
+#define RG_TOKEN_BLOCK 256
+
+template <int KB, int TAPS, bool LINES>
+__global__ __launch_bounds__(128 * KB) void rglru_token_kernel(
+    const bf16_t* __restrict__ proj, int64_t proj_stride, int x_col, int y_col, const float* __restrict__ x_bias,
+    const float* __restrict__ y_bias, const float* __restrict__ conv_w, const float* __restrict__ conv_b, int taps,
+    const bf16_t* __restrict__ gate_a, const float* __restrict__ gate_a_bias, const bf16_t* __restrict__ gate_i,
+    const float* __restrict__ gate_i_bias, const float* __restrict__ lam, float decay_scale, const int* __restrict__ row_slot,
+    float* __restrict__ state, float* __restrict__ tail, bf16_t* __restrict__ out, int n_rows, int width, int block_size,
+    int write_state) {
+  __shared__ __attribute__((aligned(16))) float u_s[16][RG_TOKEN_BLOCK + RG_MM_PAD];
+  const int r0 = blockIdx.x * 16, b = blockIdx.y, rows = min(16, n_rows - r0), kbs = block_size / 32, keep = taps - 1;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE, waves = blockDim.x / WAVE, c = lane % 16, g = lane / 16;
+  // the convolution: a wave takes 64 channels of a row; the inputs before the step's one are the memory's, oldest first
+  const int chunks = (block_size + WAVE - 1) / WAVE;
+  int sl = -1, at = 0;
+  float win[TAPS], cw[TAPS], cb, xb, x;
+  auto ask = [&](int unit) {
+    const int rr = unit / chunks, cc = unit % chunks * WAVE + lane;
+    sl = row_slot[r0 + rr];
+    at = b * block_size + min(cc, block_size - 1);
+    const float* tl = tail + (int64_t)max(sl, 0) * keep * width + at;
+#pragma unroll
+    for (int k = 0; k < TAPS - 1; ++k) {
+      if (k >= keep) break;
+      win[k] = tl[(int64_t)k * width];
+    }
+#pragma unroll
+    for (int k = 0; k < TAPS; ++k) {
+      if (k < taps) cw[k] = conv_w[at * taps + k];
+    }
+    x = load_as_float(proj + (int64_t)(r0 + rr) * proj_stride + x_col + at);
+    xb = x_bias[at];
+    cb = conv_b[at];
+  };
+  auto convolve = [&](int unit) {
+    const int rr = unit / chunks, cc = unit % chunks * WAVE + lane;
+    if (cc >= block_size) return;
+    const float now = x + xb;
+    float u = cb;
+#pragma unroll
+    for (int k = 0; k < TAPS; ++k) {
+      if (k < keep) u += cw[k] * win[k];
+      if (k == keep) u += cw[k] * now;
+    }
+    u_s[rr][cc] = sl >= 0 ? u : 0.f;
+    if (!write_state || sl < 0) return;
+    float* tl = tail + (int64_t)sl * keep * width + at;
+#pragma unroll
+    for (int k = 0; k < TAPS - 1; ++k) {
+      if (k < keep) tl[(int64_t)k * width] = k + 1 < keep ? win[k + 1] : now;
+    }
+  };
+  const int units = rows * chunks;
+  if (wave < units) ask(wave);
+  // the wave's outputs 16 * wave .. + 15 (waves = block_size / 16), the lane's row and its four outputs of it
+  const int64_t first = ((int64_t)b * block_size + 16 * wave) * block_size;
+  bf16x8 fa[KB], fi[KB];
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    if (kb >= kbs) continue;
+    const int64_t w = first + (LINES ? (4 * (c / 4) + kb % 4) * block_size + 128 * (kb / 4) + 8 * (4 * (c % 4) + g)
+                                     : c * block_size + 32 * kb + 8 * g);
+    fa[kb] = *(const bf16x8*)(gate_a + w);
+    fi[kb] = *(const bf16x8*)(gate_i + w);
+  }
+  const int o = 16 * wave + 4 * g, ch = b * block_size + o;
+  const int64_t row = r0 + c;
+  const int64_t some = min(row, (int64_t)n_rows - 1);
+  const int slot = row_slot[some];
+  const vf4 ab = *(const vf4*)(gate_a_bias + ch), ib = *(const vf4*)(gate_i_bias + ch), la = *(const vf4*)(lam + ch);
+  const vf4 yb = *(const vf4*)(y_bias + ch);
+  vf4 S = *(const vf4*)(state + (int64_t)max(slot, 0) * width + ch);
+  bf16_t y[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) y[i] = proj[some * proj_stride + y_col + ch + i];
+  for (int unit = wave; unit < units; unit += waves) {
+    if (unit != wave) ask(unit);
+    convolve(unit);
+  }
+  __syncthreads();
+  f32x4 acc_a = f32x4{0.f, 0.f, 0.f, 0.f}, acc_i = f32x4{0.f, 0.f, 0.f, 0.f};
+  bf16x8 ub[KB];
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    if (kb >= kbs) continue;
+    const vf4 lo = *(const vf4*)(&u_s[c][32 * kb + 8 * g]), hi = *(const vf4*)(&u_s[c][32 * kb + 8 * g + 4]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) { ub[kb][j] = (__bf16)lo[j]; ub[kb][4 + j] = (__bf16)hi[j]; }
+    if constexpr (!LINES) {
+      acc_a = MFMA16(fa[kb], ub[kb], acc_a);
+      acc_i = MFMA16(fi[kb], ub[kb], acc_i);
+    }
+  }
+  if constexpr (LINES) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        f32x4 pa = f32x4{0.f, 0.f, 0.f, 0.f}, pi = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kk = 0; kk < KB / 4; ++kk) {
+          pa = MFMA16(fa[4 * kk + j], ub[4 * kk + s], pa);
+          pi = MFMA16(fi[4 * kk + j], ub[4 * kk + s], pi);
+        }
+        acc_a[j] += pa[s];
+        acc_i[j] += pi[s];
+      }
+    }
+  }
+  if (c >= rows) return;
+  bf16_t* dst = out + row * width + ch;
+  if (slot < 0) {                                          // the rows of a sequence that sits out hold zeros
+#pragma unroll
+    for (int i = 0; i < 4; ++i) store_from_float(dst + i, 0.f);
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float r = 1.f / (1.f + expf(-(acc_a[i] + ab[i])));
+    const float gi = 1.f / (1.f + expf(-(acc_i[i] + ib[i])));
+    const float log_a = -decay_scale * soft_plus(la[i]) * r;
+    S[i] = expf(log_a) * S[i] + sqrtf(-expm1f(2.f * log_a)) * gi * u_s[c][o + i];
+    store_from_float(dst + i, S[i] * gelu_tanh(load_as_float(y + i) + yb[i]));
+  }
+  if (write_state) *(vf4*)(state + (int64_t)slot * width + ch) = S;
+}
+
+// -2: blocks and addresses that the kernel does not take.
+DRYFT_API int dryft_rglru_token(const void* proj, int64_t proj_stride, int x_col, int y_col, const float* x_bias, const float* y_bias,
+                                const float* conv_w, const float* conv_b, int taps, const void* gate_a, const float* gate_a_bias,
+                                const void* gate_i, const float* gate_i_bias, const float* lam, float decay_scale, const int* row_slot,
+                                float* state, float* tail, void* out, int n_rows, int width, int blocks, int write_state,
+                                hipStream_t stream) {
+  if (n_rows <= 0) return 0;
+  if (blocks <= 0 || width % blocks || taps < 1 || taps > RG_MAX_TAPS) return -1;
+  const int block_size = width / blocks;
+  if (block_size % 32 || block_size > RG_TOKEN_BLOCK || blocks > 65535 ||
+      (((uintptr_t)gate_a | (uintptr_t)gate_i | (uintptr_t)gate_a_bias | (uintptr_t)gate_i_bias | (uintptr_t)lam | (uintptr_t)y_bias |
+        (uintptr_t)state) & 15))
+    return -2;
+  const dim3 grid((n_rows + 15) / 16, blocks), block(block_size / 16 * WAVE);
+#define RG_TOKEN_(KB, TAPS, LINES)                                                                                                       \
+  hipLaunchKernelGGL((rglru_token_kernel<KB, TAPS, LINES>), grid, block, 0, stream, (const bf16_t*)proj, proj_stride, x_col, y_col, x_bias, y_bias, \
+                     conv_w, conv_b, taps, (const bf16_t*)gate_a, gate_a_bias, (const bf16_t*)gate_i, gate_i_bias, lam, decay_scale, \
+                     row_slot, state, tail, (bf16_t*)out, n_rows, width, block_size, write_state)
+#define RG_TOKEN(KB, LINES)                   \
+  if (taps <= 4) RG_TOKEN_(KB, 4, LINES);     \
+  else RG_TOKEN_(KB, RG_MAX_TAPS, LINES)
+  if (block_size == 128) {
+    RG_TOKEN(4, true);
+  } else if (block_size == 256) {
+    RG_TOKEN(8, true);
+  } else if (block_size < 128) {
+    RG_TOKEN(4, false);
+  } else {
+    RG_TOKEN(8, false);
+  }
+#undef RG_TOKEN
+#undef RG_TOKEN_
+  return DRYFT_LAUNCH_CHECK();
 }
 
 DRYFT_API int dryft_rglru_gates(const void* proj, int64_t proj_stride, int x_col, const float* x_bias,

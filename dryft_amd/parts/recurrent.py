@@ -160,6 +160,14 @@ class GatedLinearRecurrence(Mixer):
         rows, W = h.shape[0], self.width
         proj = linear(h, self.w_in)
         tail = line["tail"].state if self.taps > 1 else None
+        if ctx.max_q_len == 1 and ops.rglru_token_takes(proj, line["state"].state, self.gate_a, self.gate_i,
+                                                        (self.gate_a_bias, self.gate_i_bias, self.lam, self.y_bias), self.blocks):
+            # one row a sequence: gates, walk and the convolution's memory in one launch
+            out = torch.empty((rows, W), dtype=h.dtype, device=h.device)
+            ops.rglru_token(proj, W, 0, self.x_bias, self.y_bias, self.conv, self.conv_bias, self.taps, self.gate_a, self.gate_a_bias,
+                            self.gate_i, self.gate_i_bias, self.lam, self.decay_scale, ctx.row_slot, line["state"].state, tail, out, W,
+                            self.blocks, writes_cache)
+            return linear(out, self.w_o, allow_partials=True)
         coef = torch.empty((rows, 2, W), dtype=torch.float32, device=h.device)
         ops.rglru_gates(proj, W, self.x_bias, self.conv, self.conv_bias, self.taps, self.gate_a, self.gate_a_bias,
                         self.gate_i, self.gate_i_bias, self.lam, self.decay_scale, ctx.row_slot, ctx.row_seq,

@@ -105,3 +105,46 @@ def test_one_row_of_a_matrix_memory(dtype, write, H, D, P, bias):
     for slot in range(n + 2):
         if not write or slot not in {s for s, q in zip(SLOTS, ROWS) if q}:
             assert all(torch.equal(a[slot], b[slot].double()) for a, b in ((S, S0), (N, N0), (m, m0)))
+
+
+@pytest.mark.parametrize("write", [True, False])
+@pytest.mark.parametrize("rows,size,taps", [(1, 128, 4), (5, 32, 1), (16, 96, 5), (17, 256, 4), (33, 128, 16), (17, 160, 2)])
+def test_one_row_of_a_gated_linear_recurrence(write, rows, size, taps):
+    """Against the formulas in 64 bits; the convolution is rounded to bfloat16 where the gates multiply it, on both sides."""
+    from dryft_amd.csrc import ops
+    g = torch.Generator().manual_seed(rows + size)
+    blocks, scale = 3, 8.0
+    W = blocks * size
+    proj = torch.randn(rows, 2 * W + 5, generator=g).bfloat16()
+    xb, yb, cb, ab, ib, lam = (torch.randn(W, generator=g) for _ in range(6))
+    conv, tail, S = torch.randn(W, taps, generator=g), torch.randn(rows + 1, max(taps - 1, 1), W, generator=g), torch.randn(rows + 1, W, generator=g)
+    wa, wi = ((torch.randn(blocks, size, size, generator=g) * size ** -0.5).bfloat16() for _ in range(2))
+    slots = torch.randperm(rows + 1, generator=g)[:rows]
+    slots[rows // 2] = -1 if rows > 1 else slots[0]
+    dev = lambda t: t.to(DEV)
+    got_s, got_t, out = dev(S.clone()), dev(tail.clone()), torch.full((rows, W), 7.0, device=DEV, dtype=torch.bfloat16)
+    wad, wid, vectors = dev(wa), dev(wi), [dev(v) for v in (ab, ib, lam, yb)]
+    assert ops.rglru_token_takes(dev(proj), got_s, wad, wid, vectors, blocks)
+    ops.rglru_token(dev(proj), W, 0, dev(xb), vectors[3], dev(conv), dev(cb), taps, wad, vectors[0], wid, vectors[1], vectors[2], scale,
+                    dev(slots.int()), got_s, got_t if taps > 1 else None, out, W, blocks, write)
+    out, got_s, got_t = (t.double().cpu() for t in (out, got_s, got_t))
+    live = slots >= 0
+    assert not out[~live].any()
+    rs, at, p = live.nonzero()[:, 0], slots[live], proj.double()
+    window = torch.cat([tail.double()[at][:, :taps - 1], (p[rs, W:2 * W] + xb.double())[:, None]], 1)
+    u = cb.double() + (window * conv.double().t()).sum(1)
+    ub = u.float().bfloat16().double().view(-1, blocks, size)
+    gate = lambda w, b: torch.sigmoid((ub.transpose(0, 1) @ w.double().transpose(1, 2).contiguous()).transpose(0, 1).reshape(-1, W) + b.double())
+    log_a = -scale * torch.nn.functional.softplus(lam.double()) * gate(wa, ab)
+    want_s = log_a.exp() * S.double()[at] + (-torch.expm1(2 * log_a)).sqrt() * gate(wi, ib) * u
+    want = want_s * torch.nn.functional.gelu(p[rs, :W] + yb.double(), approximate="tanh")
+    # sums of up to 256 float products; an input of the gates whose float sum lies next to a boundary of bfloat16 may round the other way
+    # (2^-8 of it, times a weight of size^-1/2, through a slope of scale * softplus * 1/4 at most)
+    tol = 2.0 ** -8 * 4 * size ** -0.5 * scale * float(torch.nn.functional.softplus(lam).max()) / 4 * float(want_s.abs().max())
+    assert float((out[live] - want).abs().max()) <= tol + 2.0 ** -8 * float(want.abs().max())
+    if write:
+        assert float((got_s[at] - want_s).abs().max()) <= tol and float((got_s[at] - want_s).pow(2).mean().sqrt()) <= 1e-3
+        if taps > 1:
+            assert float((got_t[at] - window[:, 1:]).abs().max()) <= 2.0 ** -20
+    untouched = [s for s in range(rows + 1) if not write or s not in at.tolist()]
+    assert torch.equal(got_s[untouched], S.double()[untouched]) and torch.equal(got_t[untouched], tail.double()[untouched])
