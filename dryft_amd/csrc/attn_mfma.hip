@@ -987,6 +987,113 @@ struct FusedQKV {
   int write_kv;
 };
 
+// What the split kernel needs to take a row's queries, key and value straight from a projection whose heads turn by float32 tables:
+// the work of the kernels in rope_kv.hip for neighbouring pairs, for halves behind a per-head norm, and for two maps a head, in their
+// order and with their one rounding.
+struct TurnedQKV {
+  const bf16_t* src;                 // [rows, stride]; heads of `dim` features from q_col and k_col, of v_dim from v_col
+  int64_t stride;
+  int parts;                         // > 0: src points to float partial sums [parts, rows, stride] instead, added up in order and rounded
+  int64_t part_stride;
+  int q_col, k_col, v_col;
+  const float* bias;                 // one number a column of src, or null
+  const float *q_w, *k_w;            // per-head norm ahead of the turn, or null
+  float eps;
+  int unit_after;                    // divide by the root mean square behind the turn
+  const float *cos_t, *sin_t;
+  int rot, pairs;                    // features 2i and 2i + 1 turn together, or i and i + rot / 2
+  int dim, v_dim;
+  int map_dim;                       // > 0: query and key heads are pairs of maps, the second from feature map_dim of a page's row
+  int write_kv;
+  const bf16_t* gate;                // sigmoid gate of the output, [rows, gate_stride] with n_heads * head_dim columns, or null
+  int64_t gate_stride;
+};
+
+// A lane's features lane + 64 u of a head, what turns with them, and their factors: bits as they lie in memory.
+template <int U>
+struct TurnedRegs {
+  float x[U], other[U];
+  float b[U], b_other[U], w[U], w_other[U], cs[U], sn[U];
+};
+
+__device__ __forceinline__ int turns_with(const TurnedQKV& t, int i) {
+  return i >= t.rot ? i : t.pairs ? i ^ 1 : i < t.rot / 2 ? i + t.rot / 2 : i - t.rot / 2;
+}
+
+// A feature as it lies in memory; `projected_value` of it is the feature. More than one partial sum is waited for here.
+template <bool SUMS>
+__device__ __forceinline__ float projected_raw(const TurnedQKV& t, int64_t at) {
+  if (!SUMS) return __uint_as_float((uint32_t)t.src[at].bits);
+  const float* sums = (const float*)t.src;
+  float v = sums[at];
+  for (int s = 1; s < t.parts; ++s) v += sums[s * t.part_stride + at];
+  return v;
+}
+template <bool SUMS>
+__device__ __forceinline__ float projected_value(float raw) {
+  return SUMS ? rounded_as<bf16_t>(raw) : __uint_as_float(__float_as_uint(raw) << 16);
+}
+
+template <int U, bool SUMS>
+__device__ __forceinline__ void turned_load(TurnedRegs<U>& h, const TurnedQKV& t, int64_t row, int col, const float* __restrict__ w,
+                                            int pos) {
+  const int lane = threadIdx.x % WAVE, half = t.rot / 2;
+  const int64_t first = row * t.stride + col;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int i = min(lane + WAVE * u, t.dim - 1), j = turns_with(t, i);
+    h.x[u] = projected_raw<SUMS>(t, first + i);
+    h.other[u] = projected_raw<SUMS>(t, first + j);
+    h.b[u] = h.b_other[u] = h.sn[u] = 0.f;
+    h.w[u] = h.w_other[u] = h.cs[u] = 1.f;
+    if (t.bias != nullptr) { h.b[u] = t.bias[col + i]; h.b_other[u] = t.bias[col + j]; }
+    if (w != nullptr) { h.w[u] = w[i]; h.w_other[u] = w[j]; }
+    if (half > 0) {
+      const int f = min(t.pairs ? i / 2 : i < half ? i : i - half, half - 1);
+      h.cs[u] = t.cos_t[(int64_t)pos * half + f];
+      h.sn[u] = t.sin_t[(int64_t)pos * half + f];
+    }
+  }
+}
+
+// The head, zeros around it, to `row_lds` (`width` values, features from `at`) and, if given, the features to `dst`.
+template <int U, bool SUMS>
+__device__ __forceinline__ void turned_finish(const TurnedRegs<U>& h, const TurnedQKV& t, bool normed, int at, int width, bool clear,
+                                              bf16_t* row_lds, bf16_t* dst) {
+  const int lane = threadIdx.x % WAVE, half = t.rot / 2;
+  float x[U], o[U], ss = 0.f;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    x[u] = projected_value<SUMS>(h.x[u]) + h.b[u];
+    ss += lane + WAVE * u < t.dim ? x[u] * x[u] : 0.f;
+  }
+  const float inv = normed ? rsqrtf(wave_sum(ss) / (float)t.dim + t.eps) : 1.f;
+  ss = 0.f;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int i = lane + WAVE * u;
+    const float own = normed ? x[u] * inv * h.w[u] : x[u];
+    const float other = (projected_value<SUMS>(h.other[u]) + h.b_other[u]) * (normed ? inv * h.w_other[u] : 1.f);
+    const bool first = t.pairs ? (i & 1) == 0 : i < half;
+    o[u] = i >= t.rot ? own : first ? own * h.cs[u] - other * h.sn[u] : own * h.cs[u] + other * h.sn[u];
+    ss += i < t.dim ? o[u] * o[u] : 0.f;
+  }
+  const float unit = t.unit_after ? rsqrtf(wave_sum(ss) / (float)t.dim + t.eps) : 1.f;
+  if (clear) {
+    for (int i = lane; i < width; i += WAVE) row_lds[i] = float_to_bf16(0.f);
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");   // another lane's feature may follow this lane's zero
+    __builtin_amdgcn_wave_barrier();
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int i = lane + WAVE * u;
+    if (i >= t.dim) continue;
+    const bf16_t v = float_to_bf16(o[u] * unit);
+    row_lds[at + i] = v;
+    if (dst != nullptr) dst[at + i] = v;
+  }
+}
+
 // A row's query heads of one kv head, its new key and its new value for one wave alone: lane 16 h + j takes features 8 j ..
 // 8 j + 7 of head h of four, so that heads are whole lines, the sum of squares and the rotation's pairs stay within 16 lanes
 // (moves within a row, no LDS), and four heads are one pass. They end in the wave's own piece of LDS, from where it takes its
@@ -1246,7 +1353,10 @@ __device__ __forceinline__ void half_update(RowBlock<KB>& st, const HalfPage<KB>
 //
 // MODE: q is given ready, or the row's q, k and v come straight from the projection (FusedQKV, no score options or pairs),
 // by all waves together or by each for itself (HeadPass; bfloat16 weights, at most 10 query heads a kv head, 16-byte aligned).
-enum SplitMode { READY_Q, FUSED_LDS, FUSED_DIRECT };
+// Or they come from a projection whose heads turn by float32 tables (TurnedQKV, all options): a launch and its wait less. 16 query
+// heads on 4 of 128, us with the turn in a launch of its own / here: one sequence of 1,000 keys and heads of 64 9.0 / 7.4, four of 501 to
+// 2,048 with a gate behind 14.1 / 11.5, 64 of 300 27.4 / 16.3; two maps of 64 a head, one of 2,000 12.5 / 10.8, 64 of 300 28.8 / 17.6.
+enum SplitMode { READY_Q, FUSED_LDS, FUSED_DIRECT, TURNED };
 template <int KB, bool FULL, SplitMode MODE, bool SUMS>
 // The fused form appends the row's key and value through k_pages_w / v_pages_w, which are the same buffers as
 // k_pages / v_pages: none of the four is declared restrict.
@@ -1255,15 +1365,15 @@ __global__ __launch_bounds__(64 * SPLIT_WAVES, 2) void attn_split_kernel(
     const int* __restrict__ page_table, int max_pages, const int* __restrict__ seq_slot,
     const int* __restrict__ cu_rows, const int* __restrict__ kv_len, float* part_o, float* part_ml, int* arrivals, int n_heads,
     int n_kv, int group, int blocks, int any_dim, float scale, int window, int n_splits, FusedQKV fused, bf16_t* k_pages_w, bf16_t* v_pages_w,
-    bf16_t* __restrict__ out, ScoreOptions opt, MapPair pair) {
-  constexpr bool FUSED = MODE != READY_Q;
+    bf16_t* __restrict__ out, ScoreOptions opt, MapPair pair, TurnedQKV turned) {
+  constexpr bool FUSED = MODE == FUSED_LDS || MODE == FUSED_DIRECT, TURN = MODE == TURNED, IN_LDS = MODE == FUSED_LDS || TURN;
   constexpr int U = (KB + 1) / 2;                              // features of a head that a lane holds outside the tiles
   const int head_dim = FULL ? 32 * KB : any_dim;
   ScoreCap cap = FUSED ? ScoreCap{} : score_cap(opt, scale, n_heads);
   __shared__ __attribute__((aligned(16))) float merge_o[SPLIT_WAVES][16][32 * KB + 1];   // ahead of the merge a wave's heads, in pieces of 16 bytes
   __shared__ float merge_ml[SPLIT_WAVES][16][2];
-  __shared__ __attribute__((aligned(16))) bf16_t q_lds[MODE == FUSED_LDS ? 16 : 1][32 * KB];
-  __shared__ __attribute__((aligned(16))) bf16_t kv_new[2][MODE == FUSED_LDS ? 32 * KB : 8];   // the row's own key (normed, rotated) and value
+  __shared__ __attribute__((aligned(16))) bf16_t q_lds[IN_LDS ? 16 : 1][32 * KB];
+  __shared__ __attribute__((aligned(16))) bf16_t kv_new[2][IN_LDS ? 32 * KB : 8];   // the row's own key (normed, rotated) and value
   __shared__ int came_last;
   const int seq = blockIdx.x, split = blockIdx.z;
   const int kvh = blocks == 1 ? blockIdx.y : blockIdx.y / blocks, hb = blockIdx.y - kvh * blocks;
@@ -1306,7 +1416,7 @@ __global__ __launch_bounds__(64 * SPLIT_WAVES, 2) void attn_split_kernel(
     load_half<KB, FULL>(held[a], k_pages + at, v_pages + at, u % 2, head_dim);
   };
   RowBlock<KB> st;
-  const bool owns_last = FUSED && pg1 == pg_hi;                // exactly one split has the row's own page among its pages
+  const bool owns_last = (FUSED || TURN) && pg1 == pg_hi, appends = TURN ? turned.write_kv : FUSED && fused.write_kv;               // exactly one split has the row's own page among its pages
   const ProjectedRow src_row = {SUMS ? nullptr : fused.qkv + row * fused.stride,
                                 SUMS ? (const float*)fused.qkv + row * fused.stride : nullptr, fused.parts, fused.part_stride};
   bf16x8 own_key[KB] = {};
@@ -1411,6 +1521,65 @@ __global__ __launch_bounds__(64 * SPLIT_WAVES, 2) void attn_split_kernel(
     }
     __syncthreads();
     init_rows<KB>(st, &q_lds[MODE == FUSED_LDS ? c : 0][0], row_valid, head_dim);
+  } else if constexpr (TURN) {
+    // As above; the second map of a new key is made by a wave of its own, and two query heads a wave are on their way. Wide heads:
+    // one, and the first half pages only behind them, or there are no registers for it all (one sequence of 1,000 keys, 256
+    // features, 17.7 us in two launches: 23.6 asked ahead, 19.8 behind).
+    constexpr int HEADS_AHEAD = KB <= 4 ? 2 : 1;
+    constexpr bool PAGES_AHEAD = KB <= (FULL ? 5 : 3);
+    const int maps = turned.map_dim > 0 ? 2 : 1, at = pos % PAGE_TOKENS, page_last = owns_last && appends ? table[pg_hi] : -1;
+    const bool makes_value = owns_last && appends && wave == SPLIT_WAVES - 2;
+    const int map_made = wave == SPLIT_WAVES - 1 ? 0 : wave == SPLIT_WAVES - 3 ? 1 : maps;        // of the new key
+    const bool makes_key = owns_last && appends && map_made < maps;
+    TurnedRegs<U> held_q[HEADS_AHEAD], fresh;
+    float value[U];
+#pragma unroll
+    for (int n = 0; n < HEADS_AHEAD; ++n)
+      if (wave + SPLIT_WAVES * n < rows)
+        turned_load<U, SUMS>(held_q[n], turned, row, turned.q_col + (first_head + wave + SPLIT_WAVES * n) * turned.dim, turned.q_w, pos);
+    if (makes_key) turned_load<U, SUMS>(fresh, turned, row, turned.k_col + (kvh * maps + map_made) * turned.dim, turned.k_w, pos);
+    if (makes_value) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        value[u] = projected_raw<SUMS>(turned, row * turned.stride + turned.v_col + kvh * turned.v_dim + min(lane + WAVE * u, turned.v_dim - 1));
+    }
+#pragma unroll
+    for (int a = 0; a < AHEAD; ++a)
+      if (PAGES_AHEAD && held_page[a] >= 0) ask(a, unit + SPLIT_WAVES * a, held_page[a]);
+    for (int r = wave; r < rows; r += HEADS_AHEAD * SPLIT_WAVES) {
+#pragma unroll
+      for (int n = 0; n < HEADS_AHEAD; ++n) {
+        const int rr = r + SPLIT_WAVES * n;
+        if (rr >= rows) continue;
+        if (r != wave) turned_load<U, SUMS>(held_q[n], turned, row, turned.q_col + (first_head + rr) * turned.dim, turned.q_w, pos);
+        turned_finish<U, SUMS>(held_q[n], turned, turned.q_w != nullptr, (first_head + rr) % maps * turned.map_dim, 32 * KB, true, &q_lds[rr][0],
+                         nullptr);
+      }
+    }
+    const int64_t base = ((int64_t)max(page_last, 0) * n_kv + kvh) * page_elems;
+    // a row's maps come from two waves: each clears its own half of the row
+    if (makes_key) {
+      const int from = map_made == 0 ? 0 : turned.map_dim, to = maps == 2 && map_made == 0 ? turned.map_dim : 32 * KB;
+      for (int i = from + lane; i < to; i += WAVE) kv_new[0][i] = float_to_bf16(0.f);
+      turned_finish<U, SUMS>(fresh, turned, turned.k_w != nullptr, from, 0, false, &kv_new[0][0],
+                       page_last >= 0 ? k_pages_w + base + (int64_t)at * head_dim : nullptr);
+    }
+    if (makes_value) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int i = lane + WAVE * u;
+        float v = projected_value<SUMS>(value[u]);
+        if (turned.bias != nullptr && i < turned.v_dim) v += turned.bias[turned.v_col + kvh * turned.v_dim + i];
+        const bf16_t b = float_to_bf16(i < turned.v_dim ? v : 0.f);
+        if (i < 32 * KB) kv_new[1][i] = b;
+        if (page_last >= 0 && i < turned.v_dim) v_pages_w[base + (int64_t)i * PAGE_TOKENS + value_column(at)] = b;
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < AHEAD; ++a)
+      if (!PAGES_AHEAD && held_page[a] >= 0) ask(a, unit + SPLIT_WAVES * a, held_page[a]);
+    __syncthreads();
+    init_rows<KB>(st, &q_lds[c][0], row_valid, head_dim);
   } else {
     init_rows<KB>(st, q + (row * n_heads + head) * head_dim, row_valid, head_dim);
 #pragma unroll
@@ -1423,8 +1592,8 @@ __global__ __launch_bounds__(64 * SPLIT_WAVES, 2) void attn_split_kernel(
       const int here = unit + SPLIT_WAVES * a, next = here + AHEAD * SPLIT_WAVES;
       if (here >= unit_end) break;
       const int page_next = next < unit_end ? table[next / 2] : -1;
-      if (FUSED && owns_last && fused.write_kv && here == pos / 32) {
-        if (MODE == FUSED_LDS) {
+      if ((FUSED || TURN) && owns_last && appends && here == pos / 32) {
+        if (IN_LDS) {
 #pragma unroll
           for (int kb = 0; kb < KB; ++kb) own_key[kb] = load8(&kv_new[0][FULL ? 32 * kb + 8 * g : min(32 * kb + 8 * g, head_dim - 8)]);
 #pragma unroll
@@ -1451,6 +1620,13 @@ __global__ __launch_bounds__(64 * SPLIT_WAVES, 2) void attn_split_kernel(
   }
   __syncthreads();
   const bool alone = live_splits == 1 && !pairs;
+  auto put = [&](int r, int d, float o) {                  // feature d of head r of the block
+    const int64_t at = (int64_t)(first_head + r) * head_dim + d;
+    bf16_t v = float_to_bf16(o);
+    if (TURN && turned.gate != nullptr)
+      v = float_to_bf16(bf16_to_float(v) * (1.f / (1.f + expf(-bf16_to_float(turned.gate[row * turned.gate_stride + at])))));
+    out[row * n_heads * head_dim + at] = v;
+  };
   // Below, a row that has summed nothing (l = 0: no page, or nothing but scores of -inf) becomes zeros; a total that is no number
   // divides as it is, so that a bad key or query shows at every length and number of splits.
   for (int idx = threadIdx.x; idx < rows * head_dim; idx += blockDim.x) {     // all heads of the block at once
@@ -1468,7 +1644,7 @@ __global__ __launch_bounds__(64 * SPLIT_WAVES, 2) void attn_split_kernel(
     }
     if (alone) {                                           // nothing to combine: this is the result
       if (!FUSED && opt.sink != nullptr && m != -INFINITY) l += sink_term(opt.sink, first_head + r, m);
-      out[(row * n_heads + first_head + r) * head_dim + d] = float_to_bf16(l == 0.f ? 0.f : o / l);
+      put(r, d, l == 0.f ? 0.f : o / l);
       continue;
     }
     const int64_t at = ((int64_t)seq * n_heads + first_head + r) * n_splits + split;
@@ -1500,7 +1676,7 @@ __global__ __launch_bounds__(64 * SPLIT_WAVES, 2) void attn_split_kernel(
       const float inv_l = l == 0.f ? 0.f : 1.f / l;
 #pragma unroll
       for (int u = 0; u < U; ++u)
-        if (lane + WAVE * u < head_dim) out[(row * n_heads + first_head + r) * head_dim + lane + WAVE * u] = float_to_bf16(o[u] * inv_l);
+        if (lane + WAVE * u < head_dim) put(r, lane + WAVE * u, o[u] * inv_l);
     }
     return;
   }
@@ -1700,7 +1876,7 @@ static int launch_split(const void* q, const void* k_pages, const void* v_pages,
                         const int* seq_slot, const int* cu_rows, const int* kv_len, int n_seqs, float* part_o,
                         float* part_ml, int n_splits, int* arrivals, void* out, int n_heads, int n_kv, int head_dim, float scale,
                         int window, FusedQKV fused, hipStream_t stream, ScoreOptions opt = {0.f, nullptr},
-                        MapPair pair = {0, 0, 0.f, 0.f, 0.f}) {
+                        MapPair pair = {0, 0, 0.f, 0.f, 0.f}, const TurnedQKV* turned = nullptr) {
   if (n_seqs <= 0) return 0;
   if (!head_shape_ok(n_heads, n_kv, head_dim) || n_splits < 1 || n_splits > COMBINE_MAX_SPLITS) return -1;
   if (arrivals == nullptr && (n_splits > 1 || pair.v_dim > 0)) return -1;
@@ -1711,13 +1887,20 @@ static int launch_split(const void* q, const void* k_pages, const void* v_pages,
   hipLaunchKernelGGL((attn_split_kernel<KB, FULLV, MODEV, SUMSV>), grid, block, 0, stream, (const bf16_t*)q, (const bf16_t*)k_pages, \
                      (const bf16_t*)v_pages, page_table, max_pages, seq_slot, cu_rows, kv_len, part_o, part_ml, arrivals, \
                      n_heads, n_kv, group, blocks, head_dim, scale, window, n_splits, fused, (bf16_t*)k_pages, (bf16_t*)v_pages,       \
-                     (bf16_t*)out, opt, pair)
+                     (bf16_t*)out, opt, pair, turned != nullptr ? *turned : TurnedQKV{})
   const bool full = head_dim % 32 == 0;
 #define LAUNCH_ANY(MODEV, SUMSV)                                                       \
   if (full) { DISPATCH_KB(head_dim / 32, LAUNCH_SPLIT(true, MODEV, SUMSV)); }          \
   else { DISPATCH_KB((head_dim + 31) / 32, LAUNCH_SPLIT(false, MODEV, SUMSV)); }
 #define LAUNCH_DIRECT(SUMSV) { constexpr int KB = DIRECT_HEAD / 32; LAUNCH_SPLIT(true, FUSED_DIRECT, SUMSV); }
-  if (fused.qkv == nullptr) {
+  if (turned != nullptr) {
+    if (blocks != 1) return -1;
+    if (turned->parts > 0) {
+      LAUNCH_ANY(TURNED, true)
+    } else {
+      LAUNCH_ANY(TURNED, false)
+    }
+  } else if (fused.qkv == nullptr) {
     LAUNCH_ANY(READY_Q, false)
   } else if (direct_heads_ok(fused, group, head_dim)) {
     if (fused.parts > 0) LAUNCH_DIRECT(true)
@@ -1809,4 +1992,34 @@ DRYFT_API int dryft_attn_split_diff_bf16(const void* q, const void* k_pages, con
   return launch_split(q, k_pages, v_pages, page_table, max_pages, seq_slot, cu_rows, kv_len, n_seqs, part_o, part_ml,
                       n_splits, arrivals, out, n_heads, n_kv, head_dim, scale, window, none, stream,
                       ScoreOptions{0.f, nullptr, 0, nullptr, 0}, pair);
+}
+
+// One row per sequence with queries, key and value straight from the projection, turned by float32 tables (TurnedQKV): the work of
+// dryft_rope_pairs_kv (pairs), dryft_norm_rope_half_kv (halves) or, with map_dim > 0, dryft_rope_maps_kv, then of
+// dryft_attn_split_bf16 or dryft_attn_split_diff_bf16, then (gate != null) of dryft_sigmoid_gate. n_heads counts the rows of
+// queries (two a head where there are maps), head_dim is the pages' width. At most 16 rows of queries a kv head.
+DRYFT_API int dryft_attn_turned_bf16(const void* src, int64_t stride, int parts, int64_t part_stride, int q_col, int k_col, int v_col, const float* bias,
+                                     const float* q_w, const float* k_w, float eps, int unit_after, const float* cos_t,
+                                     const float* sin_t, int rot, int pairs, int dim, int v_dim, int map_dim, int write_kv,
+                                     const void* gate, int64_t gate_stride, void* k_pages, void* v_pages, const int* page_table,
+                                     int max_pages, const int* seq_slot, const int* cu_rows, const int* kv_len, int n_seqs,
+                                     float* part_o, float* part_ml, int n_splits, int* arrivals, void* out, int n_heads, int n_kv,
+                                     int head_dim, float scale, int window, float softcap, const float* sink, int chunk,
+                                     const float* rel, int n_dist, float lambda, float post, float pair_eps, hipStream_t stream) {
+  if (src == nullptr || dim <= 0 || v_dim <= 0 || dim > head_dim || v_dim > head_dim || rot < 0 || rot % 2 || rot > dim || map_dim < 0 ||
+      parts < 0 || chunk < 0 || (chunk > 0 && window > 0) || (rel != nullptr && n_dist <= 0) || n_kv <= 0 || n_heads > 16 * n_kv ||
+      (gate != nullptr && (map_dim > 0 || v_dim != head_dim)))
+    return -1;
+  MapPair pair = {0, 0, 0.f, 0.f, 0.f};
+  if (map_dim > 0) {
+    pair = {8, v_dim, lambda, post, pair_eps};
+    if (!pair_ok(pair, n_heads, n_kv, head_dim) || map_dim < dim || map_dim + dim > head_dim || softcap != 0.f || sink || chunk || rel)
+      return -1;
+  }
+  const TurnedQKV turned = {(const bf16_t*)src, stride, parts, part_stride, q_col, k_col, v_col, bias, q_w, k_w, eps, unit_after, cos_t, sin_t, rot, pairs,
+                            dim, v_dim, map_dim, write_kv, (const bf16_t*)gate, gate_stride};
+  FusedQKV none = {};
+  return launch_split(nullptr, k_pages, v_pages, page_table, max_pages, seq_slot, cu_rows, kv_len, n_seqs, part_o, part_ml, n_splits,
+                      arrivals, out, n_heads, n_kv, head_dim, scale, window, none, stream,
+                      ScoreOptions{softcap, sink, chunk, rel, n_dist}, pair, &turned);
 }

@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import ctypes
 from ctypes import c_float, c_int, c_int64, c_void_p
+from typing import NamedTuple
 
 import torch
 
@@ -72,6 +73,8 @@ _SIGNATURES = {
                   "dryft_attn_causal_takes_projection": [_I, _I],
                   "dryft_attn_causal_projected_bf16": [_P, _L, _P, _I, _I, _F, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _I,
                                                        _I, _P, _I, _I, _I, _F, _I, _I, _P],
+                  "dryft_attn_turned_bf16": [_P, _L, _I, _L, _I, _I, _I, _P, _P, _P, _F, _I, _P, _P, _I, _I, _I, _I, _I, _I, _P, _L, _P, _P, _P, _I, _P, _P,
+                                             _P, _I, _P, _P, _I, _P, _P, _I, _I, _I, _F, _I, _F, _P, _I, _P, _I, _F, _F, _F, _P],
                   "dryft_attn_split_bf16": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _P, _P, _I, _P, _P, _I, _I, _I, _F, _I,
                                             _F, _P, _I, _P, _I, _P],
                   "dryft_attn_decode_fused_bf16": [_P, _L, _I, _L, _P, _P, _I, _I, _F, _P, _P, _I, _I, _P, _P, _P, _I, _P, _P,
@@ -1678,6 +1681,107 @@ def map_difference(a, out, v_dim: int, lam: float, post: float, eps: float) -> t
     _check(_fn("rope_kv", "dryft_map_difference")(_ptr(a), _ptr(out), out.numel() // v_dim, v_dim, float(lam), float(post),
                                                   float(eps), _float_flag(a, "a"), _stream()), "map_difference")
     return out
+
+
+ROWS_A_KV_HEAD = 16         # rows of queries of a kv head that ``attn_turned_bf16`` takes (two maps are two rows)
+
+
+def turns_in_attention(n_seqs: int, rows_a_kv_head: int, page_dim: int) -> bool:
+    """Does ``attn_turned_bf16`` take a step of so many sequences, and gain by it? A wave turns every fourth row of queries, one or two
+    at a time: 16 rows of 128 features for 8 sequences of 1,000 keys 16.1 us against 15.2 for the turn in a launch of its own, 8 rows
+    of 64 (two maps) 10.8 against 12.5. Heads beyond 192 features leave it no registers: 8 x 1,000 keys 30 against 25. From 32
+    sequences on the other launch's rows cost more than either: 16 rows of 224 29 against 41, of 128 for 64 sequences 24 against 34."""
+    return rows_a_kv_head <= ROWS_A_KV_HEAD and (n_seqs >= 32 or (rows_a_kv_head <= 8 and page_dim <= 192))
+
+
+class Turned(NamedTuple):
+    """Queries, keys and values in a projection ``src`` (bfloat16 ``[rows, columns]``, or float32 partial sums of it ``[parts, rows,
+    columns]``): heads of ``dim`` features from ``q_col`` and
+    ``k_col``, values of ``v_dim`` from ``v_col``, ``bias`` float32 over the columns; heads divided by their root mean square and
+    weighted (``q_weight``, ``k_weight`` float32, None: they pass) before the first ``rot`` features turn by float32 tables
+    ``[positions, rot / 2]``, neighbours together (``pairs``) or halves; ``unit_after``: divided by the root mean square behind that.
+    ``gate``: columns of a bfloat16 tensor whose sigmoid multiplies the output."""
+    src: torch.Tensor
+    q_col: int
+    k_col: int
+    v_col: int
+    dim: int
+    v_dim: int
+    cos: torch.Tensor | None
+    sin: torch.Tensor | None
+    rot: int
+    pairs: bool
+    bias: torch.Tensor | None = None
+    q_weight: torch.Tensor | None = None
+    k_weight: torch.Tensor | None = None
+    eps: float = 0.0
+    unit_after: bool = False
+    gate: torch.Tensor | None = None
+
+
+def attn_turned_bf16(turned: Turned, write_kv: bool, k_pages, v_pages, page_table, seq_slot, cu_rows, kv_len, n_seqs: int, part_o,
+                     part_ml, n_splits: int, out, n_heads: int, n_kv: int, page_dim: int, scale: float, window: int, softcap: float = 0.0,
+                     sink=None, chunk: int = 0, rel=None, maps: tuple | None = None, arrivals=None) -> None:
+    """One row per sequence: the turn of queries and keys, the append to the cache and attention (what ``rope_pairs_kv``,
+    ``norm_rope_half_kv`` or ``rope_maps_kv`` and then ``attn_split_bf16`` or ``attn_split_diff_bf16`` do, and ``sigmoid_gate`` behind
+    them where there is a gate) in one launch. ``maps = (map_dim, lam, post, eps)``: two maps a head. At most 16 rows of queries
+    (maps counted) a kv head. ``page_dim`` is the width of keys' and values' pages; ``out [rows, heads, page_dim]`` (with maps
+    ``[rows, heads, v_dim]``)."""
+    t, per = turned, 2 if maps else 1
+    parts = t.src.shape[0] if t.src.dim() == 3 else 0
+    _gpu(t.src, "src", torch.float32 if parts else torch.bfloat16)
+    rows, columns = t.src.shape[-2:]
+    if not (t.src.dim() in (2, 3) and t.src.stride(-1) == 1 and min(t.q_col, t.k_col, t.v_col) >= 0 and
+            max(t.q_col + per * n_heads * t.dim, t.k_col + per * n_kv * t.dim, t.v_col + n_kv * t.v_dim) <= columns):
+        raise KernelError("attn_turned: q, k or v lie outside the columns of src")
+    if t.rot % 2 or not 0 <= t.rot <= t.dim or not 0 < t.dim <= page_dim or not 0 < t.v_dim <= page_dim:
+        raise KernelError(f"attn_turned: heads of {t.dim} and {t.v_dim} features, {t.rot} of them turned, in pages of {page_dim}")
+    if t.rot:
+        for name, table in (("cos", t.cos), ("sin", t.sin)):
+            _gpu(table, name, torch.float32)
+            if not (table.dim() == 2 and table.shape[1] == t.rot // 2 and table.is_contiguous()):
+                raise KernelError(f"{name}: must be contiguous float32 [positions, {t.rot // 2}]")
+    if t.bias is not None:
+        _f32_vector(t.bias, "bias", columns)
+    if t.unit_after and (t.q_weight is not None or t.k_weight is not None):
+        raise KernelError("attn_turned: a norm before the turn or one after it")
+    for name, w in (("q_weight", t.q_weight), ("k_weight", t.k_weight)):
+        if w is not None:
+            _f32_vector(w, name, t.dim)
+    map_dim, lam, post, pair_eps = maps if maps else (0, 0.0, 0.0, 0.0)
+    if maps and not (map_dim >= t.dim and map_dim % 8 == 0 and map_dim + t.dim <= page_dim):
+        raise KernelError("attn_turned: pages too narrow for the maps")
+    _gpu(out, "out", torch.bfloat16)
+    if not (out.is_contiguous() and out.numel() == rows * n_heads * (t.v_dim if maps else page_dim)):
+        raise KernelError("attn_turned: out must be contiguous, a row of every head")
+    if t.gate is not None:
+        _gpu(t.gate, "gate", torch.bfloat16)
+        if maps or t.v_dim != page_dim or not (t.gate.shape == (rows, n_heads * page_dim) and t.gate.stride(1) == 1):
+            raise KernelError(f"attn_turned: gate [rows, {n_heads * page_dim}] with unit column stride, heads as wide as the pages")
+    _check_sink(sink, n_heads)
+    _check_rel(rel, n_heads)
+    _check_pages(k_pages, v_pages, page_table, n_kv, page_dim, torch.bfloat16)
+    if not (n_kv > 0 and n_heads % n_kv == 0 and per * n_heads <= ROWS_A_KV_HEAD * n_kv):
+        raise KernelError("attn_turned: at most 16 rows of queries a kv head")
+    for name, f, n in (("seq_slot", seq_slot, n_seqs), ("cu_rows", cu_rows, n_seqs + 1), ("kv_len", kv_len, n_seqs)):
+        _gpu(f, name, torch.int32)
+        if not (f.numel() >= n):
+            raise KernelError(f"{name}: needs {n} entries")
+    _gpu(part_o, "part_o", torch.float32)
+    _gpu(part_ml, "part_ml", torch.float32)
+    entries = n_seqs * per * n_heads * n_splits
+    if part_o.numel() < entries * page_dim or part_ml.numel() < entries * 2:
+        raise KernelError("attn_turned: partial buffers too small")
+    if not (n_splits <= 65535 and n_kv <= 65535):
+        raise KernelError("attn_turned: grid too large")
+    _check(_fn("attn_mfma", "dryft_attn_turned_bf16")(
+        _ptr(t.src), t.src.stride(-2), parts, t.src.stride(0) if parts else 0, t.q_col, t.k_col, t.v_col, _ptr(t.bias), _ptr(t.q_weight), _ptr(t.k_weight), float(t.eps),
+        int(bool(t.unit_after)), _ptr(t.cos), _ptr(t.sin), t.rot, int(bool(t.pairs)), t.dim, t.v_dim, int(map_dim), int(bool(write_kv)),
+        _ptr(t.gate), t.gate.stride(0) if t.gate is not None else 0, _ptr(k_pages), _ptr(v_pages), _ptr(page_table),
+        page_table.shape[1], _ptr(seq_slot), _ptr(cu_rows), _ptr(kv_len), n_seqs, _ptr(part_o), _ptr(part_ml), n_splits,
+        _ptr(_arrivals(arrivals, n_seqs, per * n_heads, n_kv, n_splits > 1 or bool(maps), t.src)), _ptr(out), per * n_heads, n_kv,
+        page_dim, float(scale), int(window), float(softcap), _ptr(sink), int(chunk), _ptr(rel), rel.shape[0] if rel is not None else 0,
+        float(lam), float(post), float(pair_eps), _stream()), "attn_turned_bf16")
 
 
 def attn_causal_diff_bf16(q, k_pages, v_pages, page_table, seq_slot, cu_rows, tile_cu, seq_start, n_seqs: int,

@@ -311,12 +311,38 @@ class GQAAttention(Mixer):
                     raise ValueError(f"values {name!r}: no earlier layer of this step has left values of this shape")
                 ops.blend_columns(v_cols, earlier, self.vmix)
         wide = self.page_dim()
+        by_pairs = isinstance(table, PairRotaryPositions)
+        if by_pairs and (self.qk_norm_eps is not None or self.qk_unit_eps is not None or wide):
+            raise NotImplementedError("per-head q/k norms and padded pages do not go with the rotation over "
+                                      "neighbouring pairs")
+        # bfloat16 on the matrix cores where they take the sizes (keys and values of one width, a multiple of 16, as
+        # they are or padded); float32, and the other sizes, on the kernel that takes one (row, head) a workgroup
+        matrix_cores = h.dtype == torch.bfloat16 and (wide or (D == Dv and D % MATRIX_CORE_HEAD_STEP == 0))
+        window = self.window or 0
+        g_col = self.q_dim + self.kv_dim + self.v_dim
+        if matrix_cores and ctx.max_q_len == 1 and ops.turns_in_attention(ctx.n_seqs, H // G, wide or D):
+            # one row a sequence: turn, append, attention and a gate of every feature in one launch
+            P = wide or D
+            gate = proj[:, g_col:g_col + self.o_dim] if self.output_gate and not self.head_gate and not wide else None
+            turned = ops.Turned(src, 0, self.q_dim, self.q_dim + self.kv_dim, D, Dv, cos, sin, rot, by_pairs,
+                                q_weight=self.q_norm if self.qk_norm_eps is not None else None,
+                                k_weight=self.k_norm if self.qk_norm_eps is not None else None,
+                                eps=self.qk_unit_eps or self.qk_norm_eps or 0.0, unit_after=self.qk_unit_eps is not None, gate=gate)
+            out = torch.empty((rows, H, P), dtype=h.dtype, device=h.device)
+            splits = self.decode_splits(ctx.n_seqs, ctx.max_kv_len)
+            part_o = torch.empty((ctx.n_seqs, H, splits, P), dtype=torch.float32, device=h.device)
+            part_ml = torch.empty((ctx.n_seqs, H, splits, 2), dtype=torch.float32, device=h.device)
+            ops.attn_turned_bf16(turned, writes_cache, line.k, line.v, line.page_table, ctx.seq_slot, ctx.cu_rows, ctx.kv_len,
+                                 ctx.n_seqs, part_o, part_ml, splits, out, H, G, P, self.scale, window, softcap=self.softcap,
+                                 sink=self.sink, chunk=self.chunk or 0, rel=self.rel, arrivals=split_counters(ctx, H, G))
+            if self.output_gate and gate is None:
+                gated = torch.empty((rows, self.o_dim), dtype=h.dtype, device=h.device)
+                ops.head_gate(out, proj, g_col, gated, H, self.value_dim, per_element=not self.head_gate)
+                return linear(gated, self.w_o, allow_partials=True)
+            return linear(out.view(rows, H * P), self.w_o_padded if wide else self.w_o, allow_partials=True)
         q = torch.zeros((rows, H, wide), dtype=h.dtype, device=h.device) if wide else \
             torch.empty((rows, H, D), dtype=h.dtype, device=h.device)
-        if isinstance(table, PairRotaryPositions):
-            if self.qk_norm_eps is not None or self.qk_unit_eps is not None or wide:
-                raise NotImplementedError("per-head q/k norms and padded pages do not go with the rotation over "
-                                          "neighbouring pairs")
+        if by_pairs:
             ops.rope_pairs_kv(src, 0, self.q_dim, self.q_dim + self.kv_dim, cos, sin, rot, ctx.row_slot, ctx.row_pos, q,
                               line.k, line.v, line.page_table, writes_cache, H, G, D, Dv)
         else:
@@ -324,12 +350,8 @@ class GQAAttention(Mixer):
                                   self.qk_unit_eps or self.qk_norm_eps or 0.0, cos, sin, rot, ctx.row_slot, ctx.row_pos, q,
                                   line.k, line.v, line.page_table, writes_cache, H, G, D, Dv, page_dim=wide,
                                   unit_after=self.qk_unit_eps is not None)
-        # bfloat16 on the matrix cores where they take the sizes (keys and values of one width, a multiple of 16, as
-        # they are or padded); float32, and the other sizes, on the kernel that takes one (row, head) a workgroup
-        matrix_cores = h.dtype == torch.bfloat16 and (wide or (D == Dv and D % MATRIX_CORE_HEAD_STEP == 0))
         if wide:
             D = Dv = wide                        # what the attention kernels see; o_dim keeps the values' own width
-        window = self.window or 0
         if matrix_cores and ctx.max_q_len == 1:
             out = torch.empty((rows, H, Dv), dtype=h.dtype, device=h.device)
             splits = self.decode_splits(ctx.n_seqs, ctx.max_kv_len)
@@ -354,7 +376,6 @@ class GQAAttention(Mixer):
                           chunk=self.chunk or 0, rel=self.rel)
         if self.output_gate:
             gated = torch.empty((rows, self.o_dim), dtype=h.dtype, device=h.device)
-            g_col = self.q_dim + self.kv_dim + self.v_dim
             if self.head_gate or wide:           # this kernel also packs heads that are padded
                 ops.head_gate(out, proj, g_col, gated, H, self.value_dim, per_element=not self.head_gate)
                 out = gated

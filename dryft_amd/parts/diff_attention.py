@@ -110,11 +110,21 @@ class DifferentialAttention(Mixer):
             proj = (proj.data, proj.count)
         wide, step = self.page_dim(), self.map_width()
         decoding = bool(wide) and ctx.max_q_len == 1
+        window, post = self.window or 0, 1.0 - self.diff
+        if decoding and ops.turns_in_attention(ctx.n_seqs, 2 * H // G, wide):
+            # one row a sequence: turn, append and attention in one launch
+            out = torch.empty((rows, H, Dv), dtype=h.dtype, device=h.device)
+            splits = key_splits(ctx.n_seqs, G, self.window or ctx.max_kv_len)
+            part_o = torch.empty((ctx.n_seqs, 2 * H, splits, wide), dtype=torch.float32, device=h.device)
+            part_ml = torch.empty((ctx.n_seqs, 2 * H, splits, 2), dtype=torch.float32, device=h.device)
+            turned = ops.Turned(proj[0][:proj[1]] if isinstance(proj, tuple) else proj, 0, self.q_dim, self.q_dim + self.k_dim, D, Dv, cos, sin, rot, True, bias=self.in_bias)
+            ops.attn_turned_bf16(turned, writes_cache, line.k, line.v, line.page_table, ctx.seq_slot, ctx.cu_rows, ctx.kv_len,
+                                 ctx.n_seqs, part_o, part_ml, splits, out, H, G, wide, self.scale, window,
+                                 maps=(step, self.lam, post, self.norm_eps), arrivals=split_counters(ctx, 2 * H, G))
+            return linear(out.view(rows, self.o_dim), self.w_o, allow_partials=True)
         q = torch.empty((rows, H, 2, wide if decoding else step), dtype=h.dtype, device=h.device)
         ops.rope_maps_kv(proj, 0, self.q_dim, self.q_dim + self.k_dim, self.in_bias, cos, sin, rot, ctx.row_slot, ctx.row_pos, q,
                          step if decoding else 0, line.k, step, line.v, line.page_table, writes_cache, H, G, D, Dv)
-        window = self.window or 0
-        post = 1.0 - self.diff
         # the tiled prompt kernel never visits the rows of sequences that sit out; they must hold something finite
         out = ctx.kept_zeros((rows, H, Dv), h.dtype) if wide and not decoding and ctx.some_sit_out() else \
             torch.empty((rows, H, Dv), dtype=h.dtype, device=h.device)
