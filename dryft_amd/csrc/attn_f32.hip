@@ -15,9 +15,13 @@
 // the kernel of one workgroup a (row, head) (attn_rows.hip) read every key with 16 bytes a line and request, once per head
 // of the group. Between launches that stream other memory, us, against that kernel: Qwen3-0.6B's heads, one sequence, one row at
 // 20 / 280 / 1,024 keys 6.9 / 15.8 / 39 (8.1 / 20.5 / 51), four sequences of 150 prompt rows 35 (115); in a traced serving pass
-// decoding at 10 to 280 keys 14.6, 525 prompt rows 36.8. What is left in decoding are four trips to memory one after the
-// other, 14 of 16 columns unused (a group of two), and keys that no second workgroup shares: 4,096 keys take 126 us. Which steps
-// take which form, and where the other kernel stays ahead: `float32_form` in parts/attention.py.
+// decoding at 10 to 280 keys 14.6, 525 prompt rows 36.8.
+// In decoding a compute unit takes in 35 KB/us, a half page of 128 features is 32 KB, and few rows leave most units without work: then
+// a row's keys go over several workgroups (SPLIT) of fewer waves (by what a unit takes in at once: 2, 4 or 8), whose last one adds up
+// their partial results. 16 heads on 8 of 128, one workgroup a row and kv head / split, us: one sequence of 280 / 1,024 / 4,096 keys 15.1
+// / 37.0 / 126 and 10.6 / 11.5 / 17.9, four 15.3 / 39 / 135 and 10.9 / 14.2 / 35, four of 20 / 150 6.1 / 10.6 and 6.2 / 10.7; 8 on 1 of
+// 64, four of 150 / 1,024 7.8 / 22.2 and 7.2 / 10.3. Which steps take which form, and where the other kernel stays ahead:
+// `float32_form` and `float32_splits` in parts/attention.py.
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
@@ -39,9 +43,20 @@ struct AttnF32 {
   int n_heads, n_kv, head_dim;
   float scale;
   int window;
+  int n_splits;                   // splits of a decoding row's keys, their partial results, and counters that are zeros between launches
+  float* part_o;                  // [rows, n_heads, n_splits, D]
+  float* part_ml;                 // [rows, n_heads, n_splits, 2]
+  int* arrivals;                  // [rows, kv heads * blocks of 16 heads]
 };
 
-template <int DT, int WAVES, bool TILES>
+// Values that workgroups of one launch hand to one another: past the caches that the chip's compute dies keep for themselves.
+__device__ __forceinline__ void store_far(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ float load_far(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+#define F32_SPLIT_WAVES(DT) ((DT) <= 4 ? 8 : (DT) <= 8 ? 4 : 2)
+#define F32_MAX_SPLITS 32
+
+template <int DT, int WAVES, bool TILES, bool SPLIT = false>
 __global__ __launch_bounds__(WAVES * WAVE) void attn_f32_kernel(AttnF32 a) {
   extern __shared__ __align__(16) float attn_f32_lds[];
   constexpr int D = 16 * DT, OS = D + 1;
@@ -78,6 +93,7 @@ __global__ __launch_bounds__(WAVES * WAVE) void attn_f32_kernel(AttnF32 a) {
     columns = min(16, group - h0);
     first_pos = last_pos = pos = a.row_pos[row];
     q_at = (row * a.n_heads + kvh * group + h0 + min(c, columns - 1)) * D;
+    if (slot < 0 && SPLIT && blockIdx.z > 0) return;
     if (slot < 0) {                                        // a row that sits out: zeros
       const int64_t at = (row * a.n_heads + kvh * group + h0) * D;
       for (int i = threadIdx.x; i < columns * D; i += blockDim.x) a.out[at + i] = 0.f;
@@ -88,6 +104,10 @@ __global__ __launch_bounds__(WAVES * WAVE) void attn_f32_kernel(AttnF32 a) {
   const int lo_col = a.window > 0 ? max(0, pos - a.window + 1) : 0;
   const int lo_all = a.window > 0 ? max(0, first_pos - a.window + 1) : 0;
   const int* table = a.page_table + (int64_t)slot * a.max_pages;
+  // half pages in turn over the waves of all splits; a split whose first wave has none has nothing to say
+  const int stride = SPLIT ? WAVES * a.n_splits : WAVES, first_unit = lo_all / 32 + (SPLIT ? WAVES * blockIdx.z : 0);
+  if (SPLIT && 32 * first_unit > last_pos) return;
+  const int live = SPLIT ? min(a.n_splits, (last_pos / 32 - lo_all / 32 + WAVES) / WAVES) : 1;
   f32x4 qv[DT];
 #pragma unroll
   for (int t = 0; t < DT; ++t) qv[t] = *(const f32x4*)(a.q + q_at + 16 * t + 4 * g);
@@ -96,11 +116,11 @@ __global__ __launch_bounds__(WAVES * WAVE) void attn_f32_kernel(AttnF32 a) {
   for (int t = 0; t < DT; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;                            // l: over the keys of this lane alone
   constexpr bool V_EARLY = DT <= 8;                        // wider heads have no registers for the values that soon
-  int u = lo_all / 32 + wave;
+  int u = first_unit + wave;
   int page = 32 * u <= last_pos ? table[u / 2] : -1;
-  for (; 32 * u <= last_pos; u += WAVES) {
+  for (; 32 * u <= last_pos; u += stride) {
     const int here = page;
-    page = 32 * (u + WAVES) <= last_pos ? table[(u + WAVES) / 2] : -1;
+    page = 32 * (u + stride) <= last_pos ? table[(u + stride) / 2] : -1;
     if (here < 0) continue;
     const int64_t base = ((int64_t)here * a.n_kv + kvh) * PAGE_TOKENS * D;
     const float* kp = a.k_pages + base + (int64_t)(32 * (u & 1) + c) * D + 4 * g;
@@ -200,16 +220,73 @@ __global__ __launch_bounds__(WAVES * WAVE) void attn_f32_kernel(AttnF32 a) {
       total += wgt * merge_l[v * 16 + col];
       sum += wgt * merge_o[(v * 16 + col) * OS + d];
     }
+    if (SPLIT && live > 1) {
+      const int64_t at = (out_at / D + col) * a.n_splits + blockIdx.z;
+      store_far(a.part_o + at * D + d, sum);
+      if (d == 0) {
+        store_far(a.part_ml + 2 * at, top);
+        store_far(a.part_ml + 2 * at + 1, total);
+      }
+      continue;
+    }
     // whatever the total is: a score of NaN or +inf, or none but -inf (0 / 0), leaves no number, as in the softmax
+    a.out[out_at + col * out_step + d] = sum / total;
+  }
+  if (!SPLIT || live == 1) return;
+  // The workgroup that comes last of a row's splits adds them up, in their order, so that results do not depend on timing. Nobody
+  // waits: the others are gone by then. What they wrote is counted only once it has arrived.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __shared__ int came_last;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int* count = a.arrivals + (int64_t)blockIdx.x * gridDim.y + blockIdx.y;
+    const int before = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    came_last = before == live - 1;
+    if (came_last) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next launch
+  }
+  __syncthreads();
+  if (!came_last) return;
+  auto ask = [&](float (&o8)[8], int idx, int v0) {        // eight partial results on their way at a time
+    const float* po = a.part_o + (out_at / D + idx / D) * a.n_splits * D + idx % D;
+#pragma unroll
+    for (int v = 0; v < 8; ++v)
+      if (v0 + v < live) o8[v] = load_far(po + (int64_t)(v0 + v) * D);
+  };
+  float o8[8];
+  if (threadIdx.x < columns * D) ask(o8, threadIdx.x, 0);  // the first of them along with the weights
+  float* ml = attn_f32_lds;                                // [16][F32_MAX_SPLITS][2], where the waves' results were
+  for (int i = threadIdx.x; i < columns * live; i += blockDim.x) {
+    const int64_t at = (out_at / D + i / live) * a.n_splits + i % live;
+    ml[2 * (i / live * F32_MAX_SPLITS + i % live)] = load_far(a.part_ml + 2 * at);
+    ml[2 * (i / live * F32_MAX_SPLITS + i % live) + 1] = load_far(a.part_ml + 2 * at + 1);
+  }
+  __syncthreads();
+  for (int idx = threadIdx.x; idx < columns * D; idx += blockDim.x) {
+    const int col = idx / D, d = idx % D;
+    const float* mine = ml + 2 * F32_MAX_SPLITS * col;
+    float top = -INFINITY;
+    for (int v = 0; v < live; ++v) top = fmaxf(top, mine[2 * v]);
+    float sum = 0.f, total = 0.f;
+    for (int v0 = 0; v0 < live; v0 += 8) {
+      if (v0 > 0 || idx != (int)threadIdx.x) ask(o8, idx, v0);
+#pragma unroll
+      for (int v = 0; v < 8; ++v) {
+        if (v0 + v >= live) continue;
+        const float mv = mine[2 * (v0 + v)], wgt = mv == -INFINITY ? 0.f : expf(mv - top);
+        total += wgt * mine[2 * (v0 + v) + 1];
+        sum += wgt * o8[v];
+      }
+    }
     a.out[out_at + col * out_step + d] = sum / total;
   }
 }
 
-template <int DT, int WAVES, bool TILES>
+template <int DT, int WAVES, bool TILES, bool SPLIT = false>
 static int launch_attn_f32(const AttnF32& a, dim3 grid, hipStream_t stream) {
-  constexpr int lds = WAVES * 16 * (16 * DT + 1 + 2) * 4;
+  constexpr int merge = WAVES * 16 * (16 * DT + 1 + 2) * 4, weights = SPLIT ? 16 * F32_MAX_SPLITS * 2 * 4 : 0;
+  constexpr int lds = merge > weights ? merge : weights;
   static_assert(lds <= 160 * 1024, "the merge must fit a compute unit's LDS");
-  auto kernel = attn_f32_kernel<DT, WAVES, TILES>;
+  auto kernel = attn_f32_kernel<DT, WAVES, TILES, SPLIT>;
   static bool raised = false;                              // more dynamic LDS than the default limit allows
   if (lds > 64 * 1024 && !raised) {
     if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return -2;
@@ -224,7 +301,10 @@ static int dispatch_attn_f32(const AttnF32& a, dim3 grid, hipStream_t stream) {
   if (a.n_kv <= 0 || a.n_heads % a.n_kv || a.head_dim <= 0 || a.head_dim % 16 || a.head_dim > 256 || grid.y > 65535 ||
       (((uintptr_t)a.q | (uintptr_t)a.k_pages | (uintptr_t)a.v_pages) & 15))
     return -1;
-#define ATTN_F32(DTV, WV) case DTV: return launch_attn_f32<DTV, WV, TILES>(a, grid, stream)
+#define ATTN_F32(DTV, WV)                                                                                      \
+  case DTV:                                                                                                      \
+    if (!TILES && a.n_splits > 1) return launch_attn_f32<DTV, F32_SPLIT_WAVES(DTV), false, true>(a, grid, stream);    \
+    return launch_attn_f32<DTV, WV, TILES>(a, grid, stream)
   switch (a.head_dim / 16) {                               // eight waves where the merge of a decoding row fits twice a unit
     ATTN_F32(1, 4); ATTN_F32(2, 4); ATTN_F32(3, 4); ATTN_F32(4, 4);
     ATTN_F32(5, 4); ATTN_F32(6, 4); ATTN_F32(7, 4); ATTN_F32(8, (TILES ? 4 : 8));
@@ -235,16 +315,19 @@ static int dispatch_attn_f32(const AttnF32& a, dim3 grid, hipStream_t stream) {
   return -1;
 }
 
-// One row per sequence or any rows: each on its own, by its slot and position.
+// One row per sequence or any rows: each on its own, by its slot and position. With n_splits > 1 a row's keys go over so many
+// workgroups (partial results and counters as in AttnF32).
 DRYFT_API int dryft_attn_f32_rows(const void* q, const void* k_pages, const void* v_pages, const int* page_table,
                                   int max_pages, const int* row_slot, const int* row_pos, void* out, int n_rows, int n_heads,
-                                  int n_kv, int head_dim, float scale, int window, hipStream_t stream) {
+                                  int n_kv, int head_dim, float scale, int window, int n_splits, float* part_o, float* part_ml,
+                                  int* arrivals, hipStream_t stream) {
   if (n_rows <= 0) return 0;
-  if (n_kv <= 0) return -1;
+  if (n_kv <= 0 || n_splits < 1 || n_splits > F32_MAX_SPLITS || (n_splits > 1 && !(part_o && part_ml && arrivals))) return -1;
   AttnF32 a = {(const float*)q, (const float*)k_pages, (const float*)v_pages, page_table, max_pages, row_slot, row_pos,
-               nullptr, nullptr, nullptr, nullptr, 0, (float*)out, n_heads, n_kv, head_dim, scale, window};
+               nullptr, nullptr, nullptr, nullptr, 0, (float*)out, n_heads, n_kv, head_dim, scale, window, n_splits, part_o, part_ml,
+               arrivals};
   const int blocks = (n_heads / n_kv + 15) / 16;
-  return dispatch_attn_f32<false>(a, dim3(n_rows, n_kv * blocks), stream);
+  return dispatch_attn_f32<false>(a, dim3(n_rows, n_kv * blocks, n_splits), stream);
 }
 
 // Rows in tiles of 16 of one sequence (tile_cu: their prefix sums over the sequences; max_tiles bounds their number).
@@ -255,6 +338,6 @@ DRYFT_API int dryft_attn_f32_tiles(const void* q, const void* k_pages, const voi
                                    int head_dim, float scale, int window, hipStream_t stream) {
   if (n_seqs <= 0 || max_tiles <= 0) return 0;
   AttnF32 a = {(const float*)q, (const float*)k_pages, (const float*)v_pages, page_table, max_pages, nullptr, nullptr,
-               seq_slot, cu_rows, tile_cu, seq_start, n_seqs, (float*)out, n_heads, n_kv, head_dim, scale, window};
+               seq_slot, cu_rows, tile_cu, seq_start, n_seqs, (float*)out, n_heads, n_kv, head_dim, scale, window, 1, nullptr, nullptr, nullptr};
   return dispatch_attn_f32<true>(a, dim3(max_tiles, n_heads), stream);
 }

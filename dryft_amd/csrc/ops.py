@@ -79,7 +79,7 @@ _SIGNATURES = {
                                             _F, _P, _I, _P, _I, _P],
                   "dryft_attn_decode_fused_bf16": [_P, _L, _I, _L, _P, _P, _I, _I, _F, _P, _P, _I, _I, _P, _P, _P, _I, _P, _P,
                                                    _P, _I, _P, _P, _I, _P, _P, _I, _I, _I, _F, _I, _P]},
-    "attn_f32": {"dryft_attn_f32_rows": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _F, _I, _P],
+    "attn_f32": {"dryft_attn_f32_rows": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _F, _I, _I, _P, _P, _P, _P],
                  "dryft_attn_f32_tiles": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _P, _I, _I, _I, _F, _I, _P]},
     "gemm_f32": {"dryft_gemm_stream_f32": [_P, _L, _P, _P, _I, _I, _I, _P],
                  "dryft_gemm_rows_f32": [_P, _L, _P, _P, _I, _I, _I, _I, _P],
@@ -665,6 +665,7 @@ def attn_rows(q, k_pages, v_pages, page_table, row_slot, row_pos, out, n_heads: 
         _stream()), "attn_rows")
 
 
+ATTN_F32_SPLITS = 32
 ATTN_F32_TILE = 16       # rows of a sequence that a workgroup of attn_f32 takes in steps of many rows
 
 
@@ -676,11 +677,12 @@ def attn_f32_takes(q, k_pages, v_pages, head_dim: int) -> bool:
 
 
 def attn_f32(q, k_pages, v_pages, page_table, out, n_heads: int, n_kv: int, head_dim: int, scale: float, window: int, *,
-             row_slot=None, row_pos=None, tiles=None) -> None:
+             row_slot=None, row_pos=None, tiles=None, splits: int = 1, arrivals=None) -> None:
     """Causal attention of float32 rows on the matrix cores' full-precision instruction. Either every row on its own
     (``row_slot``, ``row_pos``: int32, one per row; rows with slot -1 become zeros), or in tiles of ``ATTN_F32_TILE`` rows of
     a sequence: ``tiles = (seq_slot, cu_rows, tile_cu, seq_start, n_seqs, max_tiles)``, where the rows of sequences that sit
-    out are not written."""
+    out are not written. ``splits``: over how many workgroups the keys of each of the rows go (at most ``ATTN_F32_SPLITS``;
+    ``arrivals`` as in ``attn_split_bf16``)."""
     _gpu(q, "q", torch.float32)
     _gpu(out, "out", torch.float32)
     rows = q.numel() // (n_heads * head_dim)
@@ -696,9 +698,17 @@ def attn_f32(q, k_pages, v_pages, page_table, out, n_heads: int, n_kv: int, head
             _gpu(t, name, torch.int32)
             if not (t.numel() >= rows):
                 raise KernelError(f"{name}: needs {rows} entries")
+        if not 1 <= splits <= ATTN_F32_SPLITS:
+            raise KernelError(f"attn_f32: 1 to {ATTN_F32_SPLITS} splits, got {splits}")
+        part_o = part_ml = None
+        if splits > 1:
+            part_o = torch.empty((rows, n_heads, splits, head_dim), dtype=torch.float32, device=q.device)
+            part_ml = torch.empty((rows, n_heads, splits, 2), dtype=torch.float32, device=q.device)
+            arrivals = _arrivals(arrivals, rows, n_heads, n_kv, True, q)
         _check(_fn("attn_f32", "dryft_attn_f32_rows")(
             _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(page_table), page_table.shape[1], _ptr(row_slot), _ptr(row_pos),
-            _ptr(out), rows, n_heads, n_kv, head_dim, float(scale), int(window), _stream()), "attn_f32_rows")
+            _ptr(out), rows, n_heads, n_kv, head_dim, float(scale), int(window), splits, _ptr(part_o), _ptr(part_ml),
+            _ptr(arrivals) if splits > 1 else 0, _stream()), "attn_f32_rows")
         return
     seq_slot, cu_rows, tile_cu, seq_start, n_seqs, max_tiles = tiles
     for name, t, n in (("seq_slot", seq_slot, n_seqs), ("cu_rows", cu_rows, n_seqs + 1), ("tile_cu", tile_cu, n_seqs + 1),

@@ -71,7 +71,8 @@ def float32_form(rows: int, n_heads: int, n_kv: int, head_dim: int, longest: int
     units, and cost a sixteenth of the chip where they do not. Microseconds between launches that stream 32 MB, plain / rows /
     tiles, 16 heads on 8 of 128: 16 rows at 200 keys 12.3 / 12.3 / 16.2, at 1,024 44 / 40 / 49, at 4,096 163 / 131 / 177; 33 rows
     at 200 keys 21 / 22 / 16, at 4,096 369 / 247 / 177. One row, plain / rows, 20 keys 8.1 / 6.9, 280 20.5 / 15.8, 1,024 51 / 39;
-    without the launches between, 4,096 164 / 126, 16,384 642 / 478.
+    without the launches between, 4,096 164 / 126, 16,384 642 / 478 (rows by one workgroup a kv head; few decoding rows go over
+    several, ``float32_splits``).
     The plain kernel is ahead in short contexts where a row's work on the matrix cores is long (heads of more than 128: no
     registers to ask for the values with the keys) or its columns fill two workgroups (groups of more than 16): 8 heads on 1 of
     256, one row, 20 / 150 / 280 / 512 keys 11.2 / 17.7 / 29.6 / 39.6 against 11.8 / 21.3 / 28.6 / 40.1; 16 on 4 of 192 at 150 /
@@ -81,6 +82,14 @@ def float32_form(rows: int, n_heads: int, n_kv: int, head_dim: int, longest: int
     if few and (group > 16 or head_dim > 128 and group >= 4) and keys <= (512 if group > 16 else 256):
         return "plain"
     return "rows" if longest == 1 or few else "tiles"
+
+
+def float32_splits(rows: int, n_heads: int, n_kv: int, keys: int) -> int:
+    """Over how many workgroups the keys of a float32 decoding row go: as many as make one for each compute unit, none where that is
+    fewer than four (16 heads on 8 of 128, 16 rows, two: 150 keys 11.3 -> 11.9 us, of 256 19.4 -> 22.2), nor more than half pages go
+    round two waves each. More than one a unit is no better: four rows of 4,096 keys, 8 / 16 / 32 splits 35 / 39 / 45 us."""
+    splits = min(_UNITS // (rows * n_kv * ((n_heads // n_kv + 15) // 16)), ops.ATTN_F32_SPLITS)
+    return max(1, min(splits, -(-keys // 64))) if splits >= 4 else 1
 
 
 def add_bias(delta, bias: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
@@ -505,8 +514,11 @@ class GQAAttention(Mixer):
                                  self.head_dim, self.scale, window)
         elif ops.attn_f32_takes(q, line.k, line.v, self.head_dim) and form != "plain":
             if form == "rows":
+                splits = float32_splits(rows, self.n_heads, self.n_kv, min(window or ctx.max_kv_len, ctx.max_kv_len)) \
+                    if ctx.max_q_len == 1 and rows == ctx.n_seqs else 1
                 ops.attn_f32(q, line.k, line.v, line.page_table, out, self.n_heads, self.n_kv, self.head_dim, self.scale,
-                             window, row_slot=ctx.row_slot, row_pos=ctx.row_pos)
+                             window, row_slot=ctx.row_slot, row_pos=ctx.row_pos, splits=splits,
+                             arrivals=split_counters(ctx, self.n_heads, self.n_kv) if splits > 1 else None)
             else:
                 tile_cu, max_tiles = ctx.tiles(ops.ATTN_F32_TILE)
                 ops.attn_f32(q, line.k, line.v, line.page_table, out, self.n_heads, self.n_kv, self.head_dim, self.scale,

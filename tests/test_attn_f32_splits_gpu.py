@@ -1,0 +1,80 @@
+"""Float32 decoding attention whose keys go over several workgroups: against 64 bits, against one workgroup a row, where scores are no
+numbers, and with the counters of one launch used again by the next."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+LENS = (1, 33, 700, 96, 129, 260)
+SLOTS = (2, 0, 7, -1, 5, 1)
+
+
+def pages_of(G, D, seed):
+    g = torch.Generator().manual_seed(seed)
+    per = -(-max(LENS) // 64)
+    k, v = torch.randn(len(LENS) * per, G, 64, D, generator=g), torch.randn(len(LENS) * per, G, D, 64, generator=g)
+    order, table = torch.randperm(len(LENS) * per, generator=g), torch.full((9, per), -1, dtype=torch.int32)
+    for i, (slot, n) in enumerate(zip(SLOTS, LENS)):
+        if slot >= 0:
+            table[slot, :-(-n // 64)] = order[i * per:i * per + -(-n // 64)].int()
+    return g, k, v, table
+
+
+@pytest.mark.parametrize("splits", [2, 5, 32])
+@pytest.mark.parametrize("window", [0, 40])
+@pytest.mark.parametrize("H,G,D", [(16, 8, 128), (4, 1, 64), (20, 1, 32), (4, 4, 256), (6, 2, 144), (2, 1, 16)])
+def test_keys_over_workgroups(H, G, D, window, splits):
+    from dryft_amd.csrc import ops
+    g, k, v, table = pages_of(G, D, H + D)
+    n = len(LENS)
+    q = torch.randn(n, H, D, generator=g).to(DEV)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    kd, vd, td = k.to(DEV), v.to(DEV), table.to(DEV)
+    facts = dict(row_slot=i32(SLOTS), row_pos=i32([x - 1 for x in LENS]))
+    one, counters = torch.full_like(q, 7.0), torch.zeros(ops.split_arrivals(n, H, G), dtype=torch.int32, device=DEV)
+    ops.attn_f32(q, kd, vd, td, one, H, G, D, D ** -0.5, window, **facts)
+    for _ in range(3):
+        got = torch.full_like(q, 7.0)
+        ops.attn_f32(q, kd, vd, td, got, H, G, D, D ** -0.5, window, splits=splits, arrivals=counters, **facts)
+        # sums of the same products in another order: 700 keys, a few 2^-24 each, of values near 1
+        assert float((got - one).abs().max()) <= 32 * 2.0 ** -24 and not counters.any()
+    assert not got[SLOTS.index(-1)].any()
+    pos_of = torch.empty(64, dtype=torch.long)                       # the column of a page of values in which a position lies
+    for p in range(64):
+        b, r = p // 32 * 32, p % 32
+        pos_of[p] = b + 8 * (r % 16 // 4) + 4 * (r // 16) + r % 4
+    for i, (slot, length) in enumerate(zip(SLOTS, LENS)):
+        if slot < 0:
+            continue
+        held = table[slot, :-(-length // 64)].long()
+        keys = k[held].permute(0, 2, 1, 3).reshape(-1, G, D)[:length].double()
+        values = v[held][..., pos_of].permute(0, 3, 1, 2).reshape(-1, G, D)[:length].double()
+        lo = max(0, length - window) if window else 0
+        for h in range(H):
+            s = (keys[lo:, h // (H // G)] @ q[i, h].double().cpu()) * D ** -0.5
+            want = torch.softmax(s, 0) @ values[lo:, h // (H // G)]
+            assert float((got[i, h].double().cpu() - want).abs().max()) <= 64 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
+def test_scores_without_a_number(bad):
+    """A key that is no number shows in the row whichever workgroup meets it, as with one workgroup a row."""
+    from dryft_amd.csrc import ops
+    H, G, D = 4, 2, 64
+    g, k, v, table = pages_of(G, D, 3)
+    q = torch.rand(len(LENS), H, D, generator=g).to(DEV) + 0.1
+    k[table[7, 4].long(), :, 9] = bad
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    facts = dict(row_slot=i32(SLOTS), row_pos=i32([x - 1 for x in LENS]))
+    one, got = torch.full_like(q, 7.0), torch.full_like(q, 7.0)
+    at = (q, k.to(DEV), v.to(DEV), table.to(DEV))
+    ops.attn_f32(*at, one, H, G, D, D ** -0.5, 0, **facts)
+    ops.attn_f32(*at, got, H, G, D, D ** -0.5, 0, splits=8, **facts)
+    assert torch.equal(got.isfinite(), one.isfinite()) and got[3].eq(0).all() and got[0].isfinite().all()
+    assert float((got.nan_to_num(0.0, 0.0, 0.0) - one.nan_to_num(0.0, 0.0, 0.0)).abs().max()) <= 32 * 2.0 ** -24
+
+
+def test_where_keys_are_split():
+    from dryft_amd.parts.attention import float32_splits
+    assert float32_splits(1, 16, 8, 4096) == 32 and float32_splits(4, 16, 8, 512) == 8 and float32_splits(8, 16, 8, 4096) == 4
+    assert float32_splits(4, 16, 8, 40) == 1 and float32_splits(16, 16, 8, 4096) == 1 and float32_splits(1, 40, 1, 4096) == 32
