@@ -217,7 +217,10 @@ def _mid_plan(tiles: int, n: int, k: int, may_split: bool) -> tuple[int, int]:
     17 to 128 rows, where partial sums count 0.3; its choice is there within 3 % of the best pair on average (worst 12 %), and
     14 % ahead of what served these sizes before. The kernel that adds them up on its way in counts for the rest: steps of 64
     / 96 sequences through Qwen3-0.6B 1,587 / 2,032 us with 0.3, 1,558 / 1,982 with 0.6, 1,555 / 1,972 with 0.8, of 128 through
-    Qwen3-4B (12 layers) 1,732, 1,707 and 1,716. Against ``gemm_wide`` at 17 to 32 rows, 64 rows a workgroup and three stages at 33 to
+    Qwen3-4B (12 layers) 1,732, 1,707 and 1,716. Four waves leave no unit without a workgroup (2,048 x 2,048 at 96 rows, 8 splits 5.9 us, the modelled 4 6.7;
+    4,096 x 12,288, 8 waves 27.2, 4 with 4 splits 31.0) but for outputs so few that sixteen splits are needed for that: 1,024 x 3,072 at
+    64 rows, 16 / 12 splits 4.53 / 4.55, 5 waves 5.09; steps of 48 / 64 / 96 sequences through Qwen3-0.6B 3 % less than with wider
+    workgroups there. Against ``gemm_wide`` at 17 to 32 rows, 64 rows a workgroup and three stages at 33 to
     64, and ``gemm_tall`` beyond, us: 6,144 x 2,560 at 17 / 32 / 64 / 96 rows 8.2 / 8.7 / 10.0 / 11.5 (10.2 / 10.9 / 11.7 / 13.2),
     2,560 x 9,728 10.5 / 11.1 / 12.8 / 14.7 (13.1 / 12.9 / 14.5 / 15.7), 4,096 x 1,024 4.0 / 4.2 / 5.0 / 5.7 (5.3 / 5.8 / 5.0 / 7.0),
     10,240 x 5,120 19.7 / 21.0 / 23.8 / 26.2 (36.6 / 35.5 / 42.2 / 27.5)."""
@@ -225,7 +228,8 @@ def _mid_plan(tiles: int, n: int, k: int, may_split: bool) -> tuple[int, int]:
     best, best_cost = (4, 1), float("inf")
     for waves in ops.MID_WAVES:
         blocks = -(-n // (16 * waves))
-        wants = (1,) if not may_split else (small_mid_plan(n, k),) if waves == 4 else range(1, min(groups, 16) + 1)
+        fills = waves == 4 and blocks * 16 > _COMPUTE_UNITS      # one workgroup for each unit and no fewer: see above
+        wants = (1,) if not may_split else (small_mid_plan(n, k),) if fills else range(1, min(groups, 16) + 1)
         for splits in {ops.gemm_mid_splits(k, want) for want in wants}:
             rounds = -(-(blocks * splits) // _COMPUTE_UNITS)
             if splits > 1 and rounds > 1:
