@@ -28,8 +28,8 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 struct AttnF32 {
   const float* q;                 // [rows, n_heads, D]
-  const float* k_pages;
-  const float* v_pages;
+  float* k_pages;                 // written where the row's own key and value are appended
+  float* v_pages;
   const int* page_table;
   int max_pages;
   const int* row_slot;            // decoding
@@ -47,6 +47,13 @@ struct AttnF32 {
   float* part_o;                  // [rows, n_heads, n_splits, D]
   float* part_ml;                 // [rows, n_heads, n_splits, 2]
   int* arrivals;                  // [rows, kv heads * blocks of 16 heads]
+  // decoding with the work of the norm / rotation / append kernel: a row's q heads | k heads | v heads as the projection left them
+  const float* qkv;
+  int64_t stride;
+  const float *q_w, *k_w;         // per-head norms, or null
+  float eps;
+  const float *cos_t, *sin_t;     // [positions, head_dim / 2]
+  int write_kv;
 };
 
 // Values that workgroups of one launch hand to one another: past the caches that the chip's compute dies keep for themselves.
@@ -56,7 +63,7 @@ __device__ __forceinline__ float load_far(const float* p) { return __hip_atomic_
 #define F32_SPLIT_WAVES(DT) ((DT) <= 4 ? 8 : (DT) <= 8 ? 4 : 2)
 #define F32_MAX_SPLITS 32
 
-template <int DT, int WAVES, bool TILES, bool SPLIT = false>
+template <int DT, int WAVES, bool TILES, bool SPLIT = false, bool FUSED = false>
 __global__ __launch_bounds__(WAVES * WAVE) void attn_f32_kernel(AttnF32 a) {
   extern __shared__ __align__(16) float attn_f32_lds[];
   constexpr int D = 16 * DT, OS = D + 1;
@@ -109,8 +116,61 @@ __global__ __launch_bounds__(WAVES * WAVE) void attn_f32_kernel(AttnF32 a) {
   if (SPLIT && 32 * first_unit > last_pos) return;
   const int live = SPLIT ? min(a.n_splits, (last_pos / 32 - lo_all / 32 + WAVES) / WAVES) : 1;
   f32x4 qv[DT];
+  f32x4 own_k[FUSED ? DT : 1];                             // the row's own key, as the lanes of its column hold it, and value
+  float own_v[FUSED ? DT : 1];
+  const bool owner = FUSED && a.write_kv && last_pos / 32 >= first_unit + wave && (last_pos / 32 - first_unit - wave) % stride == 0;
+  if constexpr (FUSED) {
+    // Heads are normed and turned as they lie: a lane's features 16 t + 4g .. + 3 turn with those of t + DT / 2. The wave that reads the
+    // half page of the row's own position also makes the new key and value, puts them into its operands and appends them.
+    const float* src = a.qkv + (int64_t)blockIdx.x * a.stride;
+    const float* qp = src + (int64_t)(kvh * group + min(c, columns - 1)) * D + 4 * g;
+    f32x4 wq[DT], wk[DT], cs[DT / 2], sn[DT / 2];
 #pragma unroll
-  for (int t = 0; t < DT; ++t) qv[t] = *(const f32x4*)(a.q + q_at + 16 * t + 4 * g);
+    for (int t = 0; t < DT; ++t) {
+      qv[t] = *(const f32x4*)(qp + 16 * t);
+      if (a.q_w != nullptr) wq[t] = *(const f32x4*)(a.q_w + 16 * t + 4 * g);
+    }
+#pragma unroll
+    for (int t = 0; t < DT / 2; ++t) {
+      cs[t] = *(const f32x4*)(a.cos_t + (int64_t)pos * (D / 2) + 16 * t + 4 * g);
+      sn[t] = *(const f32x4*)(a.sin_t + (int64_t)pos * (D / 2) + 16 * t + 4 * g);
+    }
+    if (owner) {
+      const float* kq = src + (int64_t)(a.n_heads + kvh) * D + 4 * g;
+      const float* vq = src + (int64_t)(a.n_heads + a.n_kv + kvh) * D + c;
+#pragma unroll
+      for (int t = 0; t < DT; ++t) {
+        own_k[t] = *(const f32x4*)(kq + 16 * t);
+        own_v[t] = vq[16 * t];
+        if (a.k_w != nullptr) wk[t] = *(const f32x4*)(a.k_w + 16 * t + 4 * g);
+      }
+    }
+    auto turn = [&](f32x4 (&x)[DT], const f32x4 (&w)[DT], bool normed) {
+      if (normed) {
+        float ss = 0.f;
+#pragma unroll
+        for (int t = 0; t < DT; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) ss += x[t][i] * x[t][i];
+        ss += __shfl_xor(ss, 16, WAVE);
+        ss += __shfl_xor(ss, 32, WAVE);
+        const float inv = rsqrtf(ss / (float)D + a.eps);
+#pragma unroll
+        for (int t = 0; t < DT; ++t) x[t] = x[t] * inv * w[t];
+      }
+#pragma unroll
+      for (int t = 0; t < DT / 2; ++t) {
+        const f32x4 one = x[t], two = x[t + DT / 2];
+        x[t] = one * cs[t] - two * sn[t];
+        x[t + DT / 2] = two * cs[t] + one * sn[t];
+      }
+    };
+    turn(qv, wq, a.q_w != nullptr);
+    if (owner) turn(own_k, wk, a.k_w != nullptr);
+  } else {
+#pragma unroll
+    for (int t = 0; t < DT; ++t) qv[t] = *(const f32x4*)(a.q + q_at + 16 * t + 4 * g);
+  }
   f32x4 o[DT];
 #pragma unroll
   for (int t = 0; t < DT; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -136,6 +196,24 @@ __global__ __launch_bounds__(WAVES * WAVE) void attn_f32_kernel(AttnF32 a) {
       for (int t = 0; t < DT; ++t)
 #pragma unroll
         for (int half = 0; half < 2; ++half) vv[t][half] = *(const f32x4*)(vp + (int64_t)16 * t * PAGE_TOKENS + 4 * half);
+    }
+    if constexpr (FUSED) {
+      static_assert(V_EARLY, "the own value goes into what has been asked for");
+      if (owner && u == last_pos / 32) {
+        const int in_page = last_pos % PAGE_TOKENS, place = value_column(in_page) % 32;
+#pragma unroll
+        for (int t = 0; t < DT; ++t) {
+#pragma unroll
+          for (int half = 0; half < 2; ++half) {
+            if (c == in_page % 16 && half == in_page % 32 / 16) kv[half][t] = own_k[t];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (g == place / 8 && 4 * half + i == place % 8) vv[t][half][i] = own_v[t];
+          }
+          if (c == 0) *(f32x4*)(a.k_pages + base + (int64_t)in_page * D + 16 * t + 4 * g) = own_k[t];
+          if (g == 0) a.v_pages[base + (int64_t)(16 * t + c) * PAGE_TOKENS + value_column(in_page)] = own_v[t];
+        }
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
     // four sums side by side: an instruction need not wait for the one before it
@@ -281,12 +359,12 @@ __global__ __launch_bounds__(WAVES * WAVE) void attn_f32_kernel(AttnF32 a) {
   }
 }
 
-template <int DT, int WAVES, bool TILES, bool SPLIT = false>
+template <int DT, int WAVES, bool TILES, bool SPLIT = false, bool FUSED = false>
 static int launch_attn_f32(const AttnF32& a, dim3 grid, hipStream_t stream) {
   constexpr int merge = WAVES * 16 * (16 * DT + 1 + 2) * 4, weights = SPLIT ? 16 * F32_MAX_SPLITS * 2 * 4 : 0;
   constexpr int lds = merge > weights ? merge : weights;
   static_assert(lds <= 160 * 1024, "the merge must fit a compute unit's LDS");
-  auto kernel = attn_f32_kernel<DT, WAVES, TILES, SPLIT>;
+  auto kernel = attn_f32_kernel<DT, WAVES, TILES, SPLIT, FUSED>;
   static bool raised = false;                              // more dynamic LDS than the default limit allows
   if (lds > 64 * 1024 && !raised) {
     if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return -2;
@@ -315,6 +393,41 @@ static int dispatch_attn_f32(const AttnF32& a, dim3 grid, hipStream_t stream) {
   return -1;
 }
 
+// One row per sequence with the work of dryft_qk_norm_rope_kv: heads of 32, 64, 96 or (split) 128 features that turn as a whole, at most
+// 16 query heads a kv head. Splits and their scratch as below. Two launches / one, us: 16 heads on 8 of 128, four sequences of 150 / 1,024
+// keys 14.6 / 11.7 and 18.8 / 16.1; 8 on 1 of 64 10.2 / 8.8 and 13.6 / 12.5; 64 sequences of 150, 12 heads of 96, 38.5 / 34.1. -2: sizes or addresses that the kernel does not take.
+DRYFT_API int dryft_attn_f32_fused(const void* qkv, int64_t stride, const float* q_w, const float* k_w, float eps, const float* cos_t,
+                                   const float* sin_t, int write_kv, void* k_pages, void* v_pages, const int* page_table,
+                                   int max_pages, const int* row_slot, const int* row_pos, void* out, int n_rows, int n_heads,
+                                   int n_kv, int head_dim, float scale, int window, int n_splits, float* part_o, float* part_ml,
+                                   int* arrivals, hipStream_t stream) {
+  if (n_rows <= 0) return 0;
+  if (n_kv <= 0 || n_heads % n_kv || n_splits < 1 || n_splits > F32_MAX_SPLITS || (n_splits > 1 && !(part_o && part_ml && arrivals)))
+    return -1;
+  if (head_dim <= 0 || head_dim % 32 || head_dim > 128 || n_heads > 16 * n_kv || n_kv > 65535 || stride % 4 || !cos_t || !sin_t ||
+      (q_w == nullptr) != (k_w == nullptr) ||
+      (((uintptr_t)qkv | (uintptr_t)q_w | (uintptr_t)k_w | (uintptr_t)cos_t | (uintptr_t)sin_t | (uintptr_t)k_pages | (uintptr_t)v_pages) & 15))
+    return -2;
+  AttnF32 a = {nullptr, (float*)k_pages, (float*)v_pages, page_table, max_pages, row_slot, row_pos, nullptr, nullptr, nullptr, nullptr, 0,
+               (float*)out, n_heads, n_kv, head_dim, scale, window, n_splits, part_o, part_ml, arrivals, (const float*)qkv, stride, q_w,
+               k_w, eps, cos_t, sin_t, write_kv};
+  const dim3 grid(n_rows, n_kv, n_splits);
+  if (n_splits > 1) {
+    switch (head_dim / 16) {
+      case 2: return launch_attn_f32<2, F32_SPLIT_WAVES(2), false, true, true>(a, grid, stream);
+      case 4: return launch_attn_f32<4, F32_SPLIT_WAVES(4), false, true, true>(a, grid, stream);
+      case 6: return launch_attn_f32<6, F32_SPLIT_WAVES(6), false, true, true>(a, grid, stream);
+      case 8: return launch_attn_f32<8, F32_SPLIT_WAVES(8), false, true, true>(a, grid, stream);
+    }
+  }
+  switch (head_dim / 16) {
+    case 2: return launch_attn_f32<2, 4, false, false, true>(a, grid, stream);
+    case 4: return launch_attn_f32<4, 4, false, false, true>(a, grid, stream);
+    case 6: return launch_attn_f32<6, 4, false, false, true>(a, grid, stream);
+  }
+  return -2;                                               // 128 features in eight waves: no registers for the new key
+}
+
 // One row per sequence or any rows: each on its own, by its slot and position. With n_splits > 1 a row's keys go over so many
 // workgroups (partial results and counters as in AttnF32).
 DRYFT_API int dryft_attn_f32_rows(const void* q, const void* k_pages, const void* v_pages, const int* page_table,
@@ -323,7 +436,7 @@ DRYFT_API int dryft_attn_f32_rows(const void* q, const void* k_pages, const void
                                   int* arrivals, hipStream_t stream) {
   if (n_rows <= 0) return 0;
   if (n_kv <= 0 || n_splits < 1 || n_splits > F32_MAX_SPLITS || (n_splits > 1 && !(part_o && part_ml && arrivals))) return -1;
-  AttnF32 a = {(const float*)q, (const float*)k_pages, (const float*)v_pages, page_table, max_pages, row_slot, row_pos,
+  AttnF32 a = {(const float*)q, (float*)k_pages, (float*)v_pages, page_table, max_pages, row_slot, row_pos,
                nullptr, nullptr, nullptr, nullptr, 0, (float*)out, n_heads, n_kv, head_dim, scale, window, n_splits, part_o, part_ml,
                arrivals};
   const int blocks = (n_heads / n_kv + 15) / 16;
@@ -337,7 +450,7 @@ DRYFT_API int dryft_attn_f32_tiles(const void* q, const void* k_pages, const voi
                                    const int* seq_start, int n_seqs, int max_tiles, void* out, int n_heads, int n_kv,
                                    int head_dim, float scale, int window, hipStream_t stream) {
   if (n_seqs <= 0 || max_tiles <= 0) return 0;
-  AttnF32 a = {(const float*)q, (const float*)k_pages, (const float*)v_pages, page_table, max_pages, nullptr, nullptr,
+  AttnF32 a = {(const float*)q, (float*)k_pages, (float*)v_pages, page_table, max_pages, nullptr, nullptr,
                seq_slot, cu_rows, tile_cu, seq_start, n_seqs, (float*)out, n_heads, n_kv, head_dim, scale, window, 1, nullptr, nullptr, nullptr};
   return dispatch_attn_f32<true>(a, dim3(max_tiles, n_heads), stream);
 }

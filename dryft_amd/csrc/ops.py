@@ -79,7 +79,9 @@ _SIGNATURES = {
                                             _F, _P, _I, _P, _I, _P],
                   "dryft_attn_decode_fused_bf16": [_P, _L, _I, _L, _P, _P, _I, _I, _F, _P, _P, _I, _I, _P, _P, _P, _I, _P, _P,
                                                    _P, _I, _P, _P, _I, _P, _P, _I, _I, _I, _F, _I, _P]},
-    "attn_f32": {"dryft_attn_f32_rows": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _F, _I, _I, _P, _P, _P, _P],
+    "attn_f32": {"dryft_attn_f32_fused": [_P, _L, _P, _P, _F, _P, _P, _I, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _F, _I, _I, _P, _P, _P,
+                                          _P],
+                 "dryft_attn_f32_rows": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _F, _I, _I, _P, _P, _P, _P],
                  "dryft_attn_f32_tiles": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _P, _I, _I, _I, _F, _I, _P]},
     "gemm_f32": {"dryft_gemm_stream_f32": [_P, _L, _P, _P, _I, _I, _I, _P],
                  "dryft_gemm_rows_f32": [_P, _L, _P, _P, _I, _I, _I, _I, _P],
@@ -720,6 +722,51 @@ def attn_f32(q, k_pages, v_pages, page_table, out, n_heads: int, n_kv: int, head
         _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(page_table), page_table.shape[1], _ptr(seq_slot), _ptr(cu_rows),
         _ptr(tile_cu), _ptr(seq_start), n_seqs, int(max_tiles), _ptr(out), n_heads, n_kv, head_dim, float(scale), int(window),
         _stream()), "attn_f32_tiles")
+
+
+def attn_f32_fused_takes(qkv, q_weight, k_weight, cos, sin, rot: int, k_pages, v_pages, n_heads: int, n_kv: int, head_dim: int,
+                         splits: int) -> bool:
+    """Does ``attn_f32_fused`` take these heads (32, 64, 96 or 128 features that turn as a whole, at most 16 query heads a kv head,
+    float32 weights) at these addresses? Heads of 128 only with their keys split: eight waves a workgroup leave no registers for the
+    new key (16 rows of 1,024 keys 57.6 us against 48.9 in two launches)."""
+    weights = [] if q_weight is None and k_weight is None else [q_weight, k_weight]
+    return qkv.dtype == torch.float32 and head_dim in ((32, 64, 96, 128) if splits > 1 else (32, 64, 96)) and rot == head_dim and cos is not None and \
+        n_heads <= 16 * n_kv and qkv.stride(0) % 4 == 0 and all(w is not None and w.dtype == torch.float32 for w in weights) and \
+        all(t.data_ptr() % 16 == 0 for t in (qkv, cos, sin, k_pages, v_pages, *weights))
+
+
+def attn_f32_fused(qkv, q_weight, k_weight, eps: float, cos, sin, write_kv: bool, k_pages, v_pages, page_table, row_slot, row_pos, out,
+                   n_heads: int, n_kv: int, head_dim: int, scale: float, window: int, splits: int = 1, arrivals=None) -> None:
+    """One float32 row per sequence: ``qk_norm_rope_kv`` and ``attn_f32`` by rows in one launch (``attn_f32_fused_takes``)."""
+    _gpu(qkv, "qkv", torch.float32)
+    rows = qkv.shape[0]
+    if not (qkv.dim() == 2 and qkv.stride(1) == 1 and qkv.shape[1] >= (n_heads + 2 * n_kv) * head_dim):
+        raise KernelError(f"attn_f32_fused: qkv needs {(n_heads + 2 * n_kv) * head_dim} columns, has {tuple(qkv.shape)}")
+    _gpu(cos, "cos", torch.float32)
+    _gpu(sin, "sin", torch.float32)
+    if not (cos.dim() == 2 and cos.shape == sin.shape and cos.shape[1] == head_dim // 2 and cos.is_contiguous() and sin.is_contiguous()):
+        raise KernelError(f"cos, sin: must be contiguous float32 [positions, {head_dim // 2}]")
+    for name, w in (("q_weight", q_weight), ("k_weight", k_weight)):
+        if w is not None:
+            _f32_vector(w, name, head_dim)
+    if not attn_f32_fused_takes(qkv, q_weight, k_weight, cos, sin, head_dim, k_pages, v_pages, n_heads, n_kv, head_dim, splits):
+        raise KernelError(f"attn_f32_fused: {n_heads} heads on {n_kv} of {head_dim}, {splits} splits, or addresses that it does not take")
+    _check_pages(k_pages, v_pages, page_table, n_kv, head_dim, torch.float32)
+    _row_facts(rows, row_slot=row_slot, row_pos=row_pos)
+    _gpu(out, "out", torch.float32)
+    if not (out.is_contiguous() and out.numel() == rows * n_heads * head_dim):
+        raise KernelError("attn_f32_fused: out must be [rows, heads, head_dim]")
+    if not 1 <= splits <= ATTN_F32_SPLITS:
+        raise KernelError(f"attn_f32_fused: 1 to {ATTN_F32_SPLITS} splits, got {splits}")
+    part_o = part_ml = None
+    if splits > 1:
+        part_o = torch.empty((rows, n_heads, splits, head_dim), dtype=torch.float32, device=qkv.device)
+        part_ml = torch.empty((rows, n_heads, splits, 2), dtype=torch.float32, device=qkv.device)
+        arrivals = _arrivals(arrivals, rows, n_heads, n_kv, True, qkv)
+    _check(_fn("attn_f32", "dryft_attn_f32_fused")(
+        _ptr(qkv), qkv.stride(0), _ptr(q_weight), _ptr(k_weight), float(eps), _ptr(cos), _ptr(sin), int(bool(write_kv)), _ptr(k_pages),
+        _ptr(v_pages), _ptr(page_table), page_table.shape[1], _ptr(row_slot), _ptr(row_pos), _ptr(out), rows, n_heads, n_kv, head_dim,
+        float(scale), int(window), splits, _ptr(part_o), _ptr(part_ml), _ptr(arrivals) if splits > 1 else 0, _stream()), "attn_f32_fused")
 
 
 def _check_rel(rel, n_heads: int) -> None:

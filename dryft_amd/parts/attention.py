@@ -497,12 +497,22 @@ class GQAAttention(Mixer):
                                            ctx.n_seqs, max_tiles, out, self.n_heads, self.n_kv, self.head_dim,
                                            self.scale, window)
             return self._projected(out, rows, leave_product)
+        form = float32_form(rows, self.n_heads, self.n_kv, self.head_dim, ctx.max_q_len,
+                            min(window or ctx.max_kv_len, ctx.max_kv_len)) if h.dtype == torch.float32 else None
+        one_each = form == "rows" and ctx.max_q_len == 1 and rows == ctx.n_seqs
+        f32_splits = float32_splits(rows, self.n_heads, self.n_kv, min(window or ctx.max_kv_len, ctx.max_kv_len)) if one_each else 1
+        counters = split_counters(ctx, self.n_heads, self.n_kv) if f32_splits > 1 else None
+        if one_each and ops.attn_f32_fused_takes(qkv, self.q_norm, self.k_norm, cos, sin, self.rotary_dim, line.k, line.v, self.n_heads,
+                                                 self.n_kv, self.head_dim, f32_splits):
+            # one row a sequence: norm, turn, append and attention in one launch
+            ops.attn_f32_fused(qkv, self.q_norm, self.k_norm, self.qk_norm_eps or 0.0, cos, sin, writes_cache, line.k, line.v,
+                               line.page_table, ctx.row_slot, ctx.row_pos, out, self.n_heads, self.n_kv, self.head_dim, self.scale,
+                               window, splits=f32_splits, arrivals=counters)
+            return self._projected(out, rows, leave_product)
         q = torch.empty((rows, self.n_heads, self.head_dim), dtype=h.dtype, device=h.device)
         ops.qk_norm_rope_kv(qkv, self.q_norm, self.k_norm, self.qk_norm_eps or 0.0, cos, sin, self.rotary_dim,
                             ctx.row_slot, ctx.row_pos, q, line.k, line.v, line.page_table, writes_cache,
                             self.n_heads, self.n_kv, self.head_dim)
-        form = float32_form(rows, self.n_heads, self.n_kv, self.head_dim, ctx.max_q_len,
-                            min(window or ctx.max_kv_len, ctx.max_kv_len)) if h.dtype == torch.float32 else None
         if decoding:
             ops.attn_split_bf16(q, line.k, line.v, line.page_table, ctx.seq_slot, ctx.cu_rows, ctx.kv_len,
                                 ctx.n_seqs, part_o, part_ml, splits, out, self.n_heads, self.n_kv, self.head_dim,
@@ -514,11 +524,8 @@ class GQAAttention(Mixer):
                                  self.head_dim, self.scale, window)
         elif ops.attn_f32_takes(q, line.k, line.v, self.head_dim) and form != "plain":
             if form == "rows":
-                splits = float32_splits(rows, self.n_heads, self.n_kv, min(window or ctx.max_kv_len, ctx.max_kv_len)) \
-                    if ctx.max_q_len == 1 and rows == ctx.n_seqs else 1
                 ops.attn_f32(q, line.k, line.v, line.page_table, out, self.n_heads, self.n_kv, self.head_dim, self.scale,
-                             window, row_slot=ctx.row_slot, row_pos=ctx.row_pos, splits=splits,
-                             arrivals=split_counters(ctx, self.n_heads, self.n_kv) if splits > 1 else None)
+                             window, row_slot=ctx.row_slot, row_pos=ctx.row_pos, splits=f32_splits, arrivals=counters)
             else:
                 tile_cu, max_tiles = ctx.tiles(ops.ATTN_F32_TILE)
                 ops.attn_f32(q, line.k, line.v, line.page_table, out, self.n_heads, self.n_kv, self.head_dim, self.scale,

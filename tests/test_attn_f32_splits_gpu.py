@@ -78,3 +78,32 @@ def test_where_keys_are_split():
     from dryft_amd.parts.attention import float32_splits
     assert float32_splits(1, 16, 8, 4096) == 32 and float32_splits(4, 16, 8, 512) == 8 and float32_splits(8, 16, 8, 4096) == 4
     assert float32_splits(4, 16, 8, 40) == 1 and float32_splits(16, 16, 8, 4096) == 1 and float32_splits(1, 40, 1, 4096) == 32
+
+
+@pytest.mark.parametrize("write", [True, False])
+@pytest.mark.parametrize("splits", [1, 4, 32])
+@pytest.mark.parametrize("H,G,D,normed,window", [(16, 8, 128, True, 0), (16, 1, 64, False, 0), (6, 3, 96, True, 40), (4, 4, 32, True, 0), (20, 4, 128, False, 33)])
+def test_turn_and_attention_in_one(H, G, D, normed, window, splits, write):
+    """Against the launch of its own for norm, turn and append and then one workgroup a row: float32 throughout, the same formulas."""
+    from dryft_amd.csrc import ops
+    if D == 128:
+        splits = max(splits, 2)                    # unsplit, heads of 128 keep the two launches
+    g, k, v, table = pages_of(G, D, H + D)
+    n = len(LENS)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    qkv = torch.randn(n, (H + 2 * G) * D + 4, generator=g).to(DEV)
+    ang = torch.randn(max(LENS), D // 2, generator=g)
+    cos, sin, td = ang.cos().to(DEV), ang.sin().to(DEV), table.to(DEV)
+    qw, kw = (torch.randn(D, generator=g).to(DEV) for _ in range(2)) if normed else (None, None)
+    facts = dict(row_slot=i32(SLOTS), row_pos=i32([x - 1 for x in LENS]))
+    k1, v1, k2, v2 = (t.to(DEV).clone() for t in (k, v, k, v))
+    q, want, got = (torch.full((n, H, D), 7.0, device=DEV) for _ in range(3))
+    assert ops.attn_f32_fused_takes(qkv, qw, kw, cos, sin, D, k2, v2, H, G, D, splits)
+    ops.qk_norm_rope_kv(qkv, qw, kw, 1e-6, cos, sin, D, facts["row_slot"], facts["row_pos"], q, k1, v1, td, write, H, G, D)
+    ops.attn_f32(q, k1, v1, td, want, H, G, D, D ** -0.5, window, **facts)
+    ops.attn_f32_fused(qkv, qw, kw, 1e-6, cos, sin, write, k2, v2, td, facts["row_slot"], facts["row_pos"], got, H, G, D, D ** -0.5, window,
+                       splits=splits)
+    # keys: products of two values of a few units, rounded once or twice more; scores of 128 of those, softmax weights of at most 1
+    assert torch.equal(v1, v2) and float((k1 - k2).abs().max()) <= 16 * 2.0 ** -24 * float(k1.abs().max())
+    assert int((k2 != k.to(DEV)).any(-1).sum()) == (sum(s >= 0 for s in SLOTS) * G if write else 0)
+    assert float((got - want).abs().max()) <= 256 * 2.0 ** -24 * float(want.abs().max()) and not got[SLOTS.index(-1)].any()
