@@ -41,21 +41,15 @@ __global__ __launch_bounds__(256) void causal_conv_kernel(const T* __restrict__ 
   store_from_float(out + row * C + c, acc);
 }
 
-// The same for eight neighbouring channels a thread, read and written 16 bytes at a time, with the weights tap by tap
-// (`w_t [taps, C]`): for inputs, outputs and tails whose rows start at multiples of 8 channels.
+// One row of eight neighbouring channels, read and written 16 bytes at a time, with the weights tap by tap (`w_t [taps, C]`):
+// for inputs, outputs and tails whose rows start at multiples of 8 channels.
 template <typename T>
-__global__ __launch_bounds__(256) void causal_conv_vec_kernel(const T* __restrict__ u, int64_t u_stride, int col,
-                                                              const float* __restrict__ in_bias,
-                                                              const float* __restrict__ w_t,
-                                                              const float* __restrict__ out_bias, int taps, int act,
-                                                              const int* __restrict__ row_slot,
-                                                              const int* __restrict__ row_seq,
-                                                              const int* __restrict__ row_pos,
-                                                              const int* __restrict__ seq_start,
-                                                              const float* __restrict__ tail, T* __restrict__ out, int C) {
-  const int64_t row = blockIdx.x;
-  const int c = (blockIdx.y * blockDim.x + threadIdx.x) * 8;
-  if (c >= C) return;
+__device__ __forceinline__ void conv_row_of_eight(int64_t row, int c, const T* __restrict__ u, int64_t u_stride, int col,
+                                                  const float* __restrict__ in_bias, const float* __restrict__ w_t,
+                                                  const float* __restrict__ out_bias, int taps, int act,
+                                                  const int* __restrict__ row_slot, const int* __restrict__ row_seq,
+                                                  const int* __restrict__ row_pos, const int* __restrict__ seq_start,
+                                                  const float* __restrict__ tail, T* __restrict__ out, int C) {
   const int slot = row_slot[row];
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (slot < 0) {
@@ -87,6 +81,81 @@ __global__ __launch_bounds__(256) void causal_conv_vec_kernel(const T* __restric
     for (int i = 0; i < 8; ++i) acc[i] = acc[i] / (1.f + expf(-acc[i]));
   }
   store8_from_float(out + row * C + c, acc);
+}
+
+// A thread a row of eight channels.
+template <typename T>
+__global__ __launch_bounds__(256) void causal_conv_vec_kernel(const T* __restrict__ u, int64_t u_stride, int col,
+                                                              const float* __restrict__ in_bias,
+                                                              const float* __restrict__ w_t,
+                                                              const float* __restrict__ out_bias, int taps, int act,
+                                                              const int* __restrict__ row_slot,
+                                                              const int* __restrict__ row_seq,
+                                                              const int* __restrict__ row_pos,
+                                                              const int* __restrict__ seq_start,
+                                                              const float* __restrict__ tail, T* __restrict__ out, int C) {
+  const int64_t row = blockIdx.x;
+  const int c = (blockIdx.y * blockDim.x + threadIdx.x) * 8;
+  if (c >= C) return;
+  conv_row_of_eight(row, c, u, u_stride, col, in_bias, w_t, out_bias, taps, act, row_slot, row_seq, row_pos, seq_start, tail, out, C);
+}
+
+// R rows of eight channels a thread: where they are neighbours of one sequence with all the inputs they need among this step's rows,
+// R + TAPS - 1 loads go out together instead of R x TAPS, and the weights are read once; other runs of rows go one by one. Sums in the
+// same order, so the same bits.
+// Bound by bytes, of which a row a thread asks TAPS times over, behind a chain of facts and taps. us a row a thread / four rows, bfloat16,
+// 4 taps, one sequence: 2,048 x 2,048 11.2 / 9.2, 2,048 x 4,096 19.6 / 14.5, 5,099 x 4,096 38.4 / 27.2, x 8,192 70.7 / 47.3 (3.5 TB/s);
+// float32 5,099 x 8,192 136 / 79. Eight rows: 9.2 to 15.6, 14.5 to 19.2, 27.2 to 28.1, 47.3 to 46.1: too few waves but for the largest.
+template <typename T, int TAPS, int R>
+__global__ __launch_bounds__(256) void causal_conv_rows_kernel(const T* __restrict__ u, int64_t u_stride, int col,
+                                                               const float* __restrict__ in_bias,
+                                                               const float* __restrict__ w_t,
+                                                               const float* __restrict__ out_bias, int act,
+                                                               const int* __restrict__ row_slot,
+                                                               const int* __restrict__ row_seq,
+                                                               const int* __restrict__ row_pos,
+                                                               const int* __restrict__ seq_start,
+                                                               const float* __restrict__ tail, T* __restrict__ out, int n_rows, int C) {
+  const int64_t r0 = (int64_t)blockIdx.x * R;
+  const int c = (blockIdx.y * blockDim.x + threadIdx.x) * 8;
+  if (c >= C) return;
+  bool together = r0 + R <= n_rows;
+  if (together) {
+    const int seq = row_seq[r0], pos = row_pos[r0];
+    bool same = true;
+#pragma unroll
+    for (int i = 0; i < R; ++i) same &= row_slot[r0 + i] >= 0 && row_seq[r0 + i] == seq && row_pos[r0 + i] == pos + i;
+    together = same && pos - (TAPS - 1) >= seq_start[seq];
+  }
+  if (!together) {
+    for (int64_t row = r0; row < r0 + R && row < n_rows; ++row)
+      conv_row_of_eight(row, c, u, u_stride, col, in_bias, w_t, out_bias, TAPS, act, row_slot, row_seq, row_pos, seq_start, tail, out, C);
+    return;
+  }
+  float wj[TAPS][8], ib[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, ob[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  float v[R + TAPS - 1][8];
+#pragma unroll
+  for (int i = 0; i < R + TAPS - 1; ++i) load8_as_float(u + (r0 + i - (TAPS - 1)) * u_stride + col + c, v[i]);
+#pragma unroll
+  for (int j = 0; j < TAPS; ++j) load8_as_float(w_t + (int64_t)j * C + c, wj[j]);
+  if (in_bias) load8_as_float(in_bias + c, ib);
+  if (out_bias) load8_as_float(out_bias + c, ob);
+#pragma unroll
+  for (int i = 0; i < R + TAPS - 1; ++i)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[i][e] += ib[e];
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    float acc[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      acc[e] = ob[e];
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j) acc[e] += wj[j][e] * v[i + j][e];
+      if (act == 1) acc[e] = acc[e] / (1.f + expf(-acc[e]));
+    }
+    store8_from_float(out + (r0 + i) * C + c, acc);
+  }
 }
 
 // The tail after the step: the last taps - 1 inputs of each sequence, from this step's rows and, where the step
@@ -162,14 +231,34 @@ DRYFT_API int dryft_conv_max_taps() { return CONV_MAX_TAPS; }
 DRYFT_API int dryft_causal_conv(const void* u, int64_t u_stride, int col, const float* in_bias, const float* w,
                                 const float* w_t, const float* out_bias, int taps, int act, const int* row_slot,
                                 const int* row_seq, const int* row_pos, const int* seq_start, const float* tail, void* out,
-                                int n_rows, int C, int is_f32, hipStream_t stream) {
+                                int n_rows, int n_seqs, int C, int is_f32, hipStream_t stream) {
   if (n_rows <= 0) return 0;
   if (taps < 1 || taps > CONV_MAX_TAPS || C <= 0 || (taps > 1 && tail == nullptr)) return -1;
   auto aligned = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
   // steps of few rows keep the kernel of a channel a thread: eight times the threads for the same few loads each
   if (n_rows >= 32 && w_t != nullptr && C % 8 == 0 && col % 8 == 0 && u_stride % 8 == 0 && aligned(u) && aligned(out) && aligned(w_t) &&
       aligned(tail) && aligned(in_bias) && aligned(out_bias)) {
-    dim3 grid(n_rows, (C / 8 + 255) / 256), block(256);
+    const int across = (C / 8 + 255) / 256;
+    // Four rows a thread where that leaves enough waves, in loads of a row a thread: 16 Mi values. Below, us a row a thread / four: 616 x 4,096
+    // of 4 taps 7.7 / 9.8, 700 x 8,192 of 2 taps 10.8 / 11.4; on the line 2,048 x 2,048 of 4 taps 11.2 / 9.2, 616 x 8,192 13.6 / 12.6. And 16 rows
+    // a sequence or more, since runs across a sequence's start go row by row: 5,100 x 4,096 in sequences of 17 36.1 / 32.2, of 5 32.4 / 37.3.
+    if (taps >= 2 && taps <= 4 && (int64_t)n_rows * C * taps >= (16 << 20) && n_rows / 16 >= n_seqs) {
+#define CONV_ROWS(TT, TAPS)                                                                                                \
+  hipLaunchKernelGGL((causal_conv_rows_kernel<TT, TAPS, 4>), dim3((n_rows + 3) / 4, across), dim3(256), 0, stream, (const TT*)u, \
+                     u_stride, col, in_bias, w_t, out_bias, act, row_slot, row_seq, row_pos, seq_start, tail, (TT*)out, n_rows, C)
+      if (is_f32) {
+        if (taps == 2) CONV_ROWS(float, 2);
+        else if (taps == 3) CONV_ROWS(float, 3);
+        else CONV_ROWS(float, 4);
+      } else {
+        if (taps == 2) CONV_ROWS(bf16_t, 2);
+        else if (taps == 3) CONV_ROWS(bf16_t, 3);
+        else CONV_ROWS(bf16_t, 4);
+      }
+#undef CONV_ROWS
+      return DRYFT_LAUNCH_CHECK();
+    }
+    dim3 grid(n_rows, across), block(256);
     if (is_f32)
       hipLaunchKernelGGL(causal_conv_vec_kernel<float>, grid, block, 0, stream, (const float*)u, u_stride, col, in_bias,
                          w_t, out_bias, taps, act, row_slot, row_seq, row_pos, seq_start, tail, (float*)out, C);

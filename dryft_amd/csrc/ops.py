@@ -129,7 +129,7 @@ _SIGNATURES = {
             "dryft_moe_table_route": [_P, _P, _P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P],
             "dryft_moe_combine": [_P, _P, _P, _P, _P, _L, _I, _P, _I, _I, _I, _I, _P]},
     "conv": {"dryft_conv_max_taps": [],
-             "dryft_causal_conv": [_P, _L, _I, _P, _P, _P, _P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _P],
+             "dryft_causal_conv": [_P, _L, _I, _P, _P, _P, _P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P],
              "dryft_conv_step": [_P, _L, _I, _P, _P, _P, _P, _I, _I, _P, _P, _P, _P, _I, _I, _I, _P],
              "dryft_conv_tail": [_P, _L, _I, _P, _I, _P, _P, _P, _P, _I, _I, _I, _P]},
     "ssm": {"dryft_ssm_max_state": [],
@@ -2765,14 +2765,15 @@ def _row_facts(rows: int, **tensors) -> None:
 
 
 def causal_conv(u, col: int, channels: int, in_bias, weight, out_bias, silu: bool, row_slot, row_seq, row_pos, seq_start,
-                tail, out, weight_t=None, moves_tail: bool = False) -> torch.Tensor:
+                tail, out, weight_t=None, moves_tail: bool = False, n_seqs: int | None = None) -> torch.Tensor:
     """``out[t, c] = act(sum_j weight[c, j] * v[t - taps + 1 + j, c] + out_bias[c])`` with ``v = u[:, col + c] + in_bias[c]``
     over each sequence's own rows, the ``taps - 1`` inputs before the step's first row from ``tail [slots, taps - 1,
     channels]`` (float32), zeros before the sequence's start. ``act`` is the identity or (``silu``) ``z sigmoid(z)``.
     Rows of sequences that sit out give zeros. The tail is not touched (``conv_tail`` moves it on). With ``weight_t``
     (the same weights as contiguous float32 ``[taps, channels]``) and rows that start at multiples of 8 channels a thread
     takes 8 channels at a time. ``moves_tail``: for steps that bring every sequence at most one row, with two taps or more;
-    the tail moves on in the same launch."""
+    the tail moves on in the same launch. ``n_seqs``: how many sequences the rows are of, by which the kernel is chosen (as
+    many as ``seq_start`` holds unless said)."""
     _gpu(u, "u")
     rows = u.shape[0]
     if not (u.dim() == 2 and u.stride(1) == 1 and 0 <= col and col + channels <= u.shape[1]):
@@ -2809,7 +2810,8 @@ def causal_conv(u, col: int, channels: int, in_bias, weight, out_bias, silu: boo
     _check(_fn("conv", "dryft_causal_conv")(_ptr(u), u.stride(0), col, _ptr(in_bias), _ptr(weight), _ptr(weight_t),
                                             _ptr(out_bias), taps,
                                             1 if silu else 0, _ptr(row_slot), _ptr(row_seq), _ptr(row_pos),
-                                            _ptr(seq_start), _ptr(tail) if taps > 1 else 0, _ptr(out), rows, channels,
+                                            _ptr(seq_start), _ptr(tail) if taps > 1 else 0, _ptr(out), rows,
+                                            seq_start.numel() if n_seqs is None else n_seqs, channels,
                                             _float_flag(u, "u"), _stream()), "causal_conv")
     return out
 

@@ -31,7 +31,7 @@ def short_conv(u: torch.Tensor, col: int, channels: int, weight: torch.Tensor, c
     # a step of one row a sequence reads every earlier input from the tail, which then moves on in the same launch
     one_row = writes_cache and taps > 1 and ctx.max_q_len == 1
     ops.causal_conv(u, col, channels, in_bias, weight, out_bias, silu, ctx.row_slot, ctx.row_seq, ctx.row_pos,
-                    ctx.seq_start, tail, out, weight_t=weight_t, moves_tail=one_row)
+                    ctx.seq_start, tail, out, weight_t=weight_t, moves_tail=one_row, n_seqs=ctx.n_seqs)
     if writes_cache and taps > 1 and not one_row:
         ops.conv_tail(u, col, channels, in_bias, taps, ctx.seq_slot, ctx.cu_rows, ctx.q_len, ctx.n_seqs, tail)
     return out
