@@ -583,8 +583,93 @@ __global__ __launch_bounds__(256) void moe_product_mfma_kernel(const bf16_t* __r
   }
 }
 
-// For steps of few rows (decoding), where no expert has more than 16 places. A workgroup takes 16 rows of an expert's weights (for the
-// gated unit 8 gate rows and their 8 up rows). Operands as in gemm_lines.hip: a load brings four weight rows, 256 contiguous bytes of
+// For steps of few rows (decoding), where no expert has more than 16 places: two kernels, chosen in ops.py (`moe_lines_pay`, with
+// both sides' figures).
+//
+// The first has a workgroup take 16 outputs of a tile (for the gated unit 16 gate rows and their 16 up rows); its WAVES waves split K
+// in runs of whole blocks of 64, with the operand rows straight from memory (they are few and stay in the vector cache) and four blocks
+// in flight; the waves' sums meet in LDS and are added in the order 0, 1, .... What bounds it is the trip to memory, not the 2 to 17 MB
+// that a step reads: with one wave walking all of K the same product is eight trips one after the other in a quarter as many
+// workgroups (in a decoding step, 4 places of 16 experts of 2 x 512 x 2048: 24.3 us, so 8.3; 16 places 26.0 and 16.6; the
+// products back to the width, 2048 x 512: 6.1 and 4.9, 9.3 and 9.1). Eight waves where that leaves a wave two blocks
+// or more, else four. It takes all 16 places in one pass over the weights.
+template <typename O, bool GLU, int WAVES>
+__global__ __launch_bounds__(WAVES * WAVE) void moe_product_few_kernel(const bf16_t* __restrict__ a, int64_t a_stride,
+                                                              const bf16_t* __restrict__ w,
+                                                              const int* __restrict__ sorted_pair,
+                                                              const int* __restrict__ tile_expert,
+                                                              const int* __restrict__ tile_start,
+                                                              const int* __restrict__ tile_rows,
+                                                              const int* __restrict__ n_tiles, O* __restrict__ out,
+                                                              int top, int n_out, int k_dim, float limit, float alpha, float offset, int act) {
+  __shared__ f32x4 sums[WAVES][GLU ? 2 : 1][WAVE];
+  const int tile = blockIdx.x;
+  if (tile >= *n_tiles) return;
+  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, c = lane % 16, g = lane / 16;
+  const int n0 = blockIdx.y * 16;                             // the grid has no workgroup without outputs
+  const int expert = tile_expert[tile], start = tile_start[tile], count = tile_rows[tile];
+  const int w_rows = GLU ? 2 * n_out : n_out;
+  const bf16_t* we = w + (int64_t)expert * w_rows * k_dim;
+  const int n_mine = min(n0 + c, n_out - 1);
+  const bf16_t* w_gate = we + (int64_t)n_mine * k_dim + 16 * g;
+  const bf16_t* w_up = we + ((int64_t)n_out + n_mine) * k_dim + 16 * g;
+  const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  const int per = ((k_dim + 63) / 64 + WAVES - 1) / WAVES * 64;          // a wave's run of K, whole blocks
+  const int k_begin = min(wave * per, k_dim), k_end = min(k_begin + per, k_dim);
+  for (int m0 = 0; m0 < count; m0 += 16) {
+    const int place = start + min(m0 + c, count - 1);
+    const bf16_t* x = a + (int64_t)(top > 0 ? sorted_pair[place] / top : place) * a_stride + 16 * g;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f}, acc_up = {0.f, 0.f, 0.f, 0.f};
+    for (int k0 = k_begin; k0 < k_end; k0 += 256) {
+      bf16x8 wg[8], wu[8], xv[8];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int k = k0 + 64 * u;
+        const bool in0 = k + 16 * g < k_end, in1 = k + 16 * g + 8 < k_end;     // K is a multiple of 8
+        wg[2 * u] = in0 ? *(const bf16x8*)(w_gate + k) : zero;
+        wg[2 * u + 1] = in1 ? *(const bf16x8*)(w_gate + k + 8) : zero;
+        wu[2 * u] = (GLU && in0) ? *(const bf16x8*)(w_up + k) : zero;
+        wu[2 * u + 1] = (GLU && in1) ? *(const bf16x8*)(w_up + k + 8) : zero;
+        xv[2 * u] = in0 ? *(const bf16x8*)(x + k) : zero;
+        xv[2 * u + 1] = in1 ? *(const bf16x8*)(x + k + 8) : zero;
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wg[u], xv[u], acc, 0, 0, 0);
+        if (GLU) acc_up = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wu[u], xv[u], acc_up, 0, 0, 0);
+      }
+    }
+    sums[wave][0][lane] = acc;
+    if (GLU) sums[wave][GLU ? 1 : 0][lane] = acc_up;
+    __syncthreads();
+    // wave 0 holds the sums: entry i of lane (c, g) is output 4 g + i of place c
+    if (wave == 0 && m0 + c < count) {
+#pragma unroll
+      for (int v = 1; v < WAVES; ++v) {
+        acc += sums[v][0][lane];
+        if (GLU) acc_up += sums[v][GLU ? 1 : 0][lane];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int n = n0 + 4 * g + i;
+        if (n >= n_out) continue;
+        float v = acc[i];
+        if (GLU) {
+          const float gv = fminf(rounded_as<bf16_t>(v), limit);
+          const float uv = fminf(fmaxf(rounded_as<bf16_t>(acc_up[i]), -limit), limit);
+          v = gv / (1.f + expf(-alpha * gv)) * (uv + offset);
+        } else if (act == 1) {
+          const float r = fmaxf(rounded_as<bf16_t>(v), 0.f);
+          v = r * r;
+        }
+        store_from_float(out + (int64_t)(start + m0 + c) * n_out + n, v);
+      }
+    }
+    __syncthreads();                                          // the sums have been read
+  }
+}
+
+// The second has a workgroup take 16 rows of an expert's weights (for the gated unit 8 gate rows and their 8 up rows). Operands as in gemm_lines.hip: a load brings four weight rows, 256 contiguous bytes of
 // each, which are a matrix-core operand as they are ("row" c of it is piece c % 4 of weight row c / 4), the places' rows are cut
 // the same way, and of the 16 x 16 products those of equal pieces count. K is split over the waves in blocks of 128 values
 // in turn; their sums meet in LDS and are added in the order 0, 1, ....
@@ -592,6 +677,8 @@ __global__ __launch_bounds__(256) void moe_product_mfma_kernel(const bf16_t* __r
 // What bounds it is the weights (4.2 to 67 MB) and the trips to memory ahead of them (the tile, its rows, their operands).
 // A pass takes up to four places of an expert (eight where a step has more than four rows); more are walked pass by pass: with
 // sixteen a pass the registers leave half as many workgroups (the product back to the width at 12 rows 14.1 us, with eight 10.5).
+// ONCE: the caches give the weights' lines up first. Not where passes follow one another, which find them there: gated products at more
+// than four places an expert on average, time against the first kernel's with / without, K of 1,024 to 2,047 1.02 / 0.97, 2,048 and more 0.89 / 0.86.
 // In a captured chain on rotating weights of 16 experts, four of them a row (2 x 512 and 512 of 2,048, the shared one 1,024), us
 // at 1 / 2 / 4 / 8 / 16 rows against a kernel that took the operands' rows 32 bytes at a time: gate and up 6.6 / 7.9 / 11.2 / 13.3 / 14.1
 // (8.9 / 9.9 / 17.6 / 19.6 / 25.9), down 4.9 / 5.9 / 8.3 / 9.8 / 10.5 (5.5 / 6.6 / 9.1 / 10.1 / 10.8), both with the shared expert, whose
@@ -608,7 +695,7 @@ struct SharedExpert {
 #define MOE_LINE_WAVES 4                                       // eight: 20.8 / 22.7 us of a layer at 4 rows, 25 / 37 at 8
 #define MOE_LINE_AHEAD 4                                       // blocks of K of a wave on their way
 
-template <typename O, bool GLU, int X>
+template <typename O, bool GLU, int X, bool ONCE>
 __global__ __launch_bounds__(MOE_LINE_WAVES * WAVE) void moe_lines_kernel(const bf16_t* __restrict__ a, int64_t a_stride,
                                                                  const bf16_t* __restrict__ w, const int* __restrict__ sorted_pair,
                                                                  const int* __restrict__ tile_expert, const int* __restrict__ tile_start,
@@ -661,7 +748,10 @@ __global__ __launch_bounds__(MOE_LINE_WAVES * WAVE) void moe_lines_kernel(const 
         int k = (wave + (i0 + d) * WAVES) * 128 + at;
         k = k < k_dim ? k : 0;                                // beyond K (a multiple of 8): any values, zeros below
 #pragma unroll
-        for (int t = 0; t < T; ++t) wv[d][t] = __builtin_nontemporal_load((const bf16x8*)(wp[t] + k));
+        for (int t = 0; t < T; ++t) {
+          if constexpr (ONCE) wv[d][t] = __builtin_nontemporal_load((const bf16x8*)(wp[t] + k));
+          else wv[d][t] = *(const bf16x8*)(wp[t] + k);
+        }
 #pragma unroll
         for (int i = 0; i < X; ++i) xv[d][i] = *(const bf16x8*)(xp[i] + k);
       }
@@ -725,11 +815,13 @@ __global__ __launch_bounds__(MOE_LINE_WAVES * WAVE) void moe_lines_kernel(const 
 
 // shared_w: a shared expert's weights of the same product, for all shared_rows rows of shared_a ([shared_n, shared_k], with glu [2
 // shared_n, shared_k], its unit by shared_limit and shared_alpha as in GateAct); shared_out in bfloat16. Only where no expert
-// has more than 16 places, in bfloat16, shared_k a multiple of 8.
+// has more than 16 places, in bfloat16, shared_k a multiple of 8, by the kernel of whole lines.
+// lines: which kernel takes bfloat16 steps of at most 16 places an expert: the first (0), that of whole lines with weights that the
+// caches give up first (1) or keep (2).
 DRYFT_API int dryft_moe_product(const void* a, int64_t a_stride, const void* w, const int* sorted_pair,
                                 const int* tile_expert, const int* tile_start, const int* tile_rows, const int* n_tiles,
                                 int max_tiles, void* out, int out_is_f32, int top, int n_out, int k_dim, int glu,
-                                float limit, float alpha, float offset, int act, int most_places, int is_f32, const void* shared_a,
+                                float limit, float alpha, float offset, int act, int most_places, int lines, int is_f32, const void* shared_a,
                                 int64_t shared_stride, const void* shared_w, void* shared_out, int shared_rows, int shared_n,
                                 int shared_k, float shared_limit, float shared_alpha, hipStream_t stream) {
   if (max_tiles <= 0) return 0;
@@ -753,16 +845,17 @@ DRYFT_API int dryft_moe_product(const void* a, int64_t a_stride, const void* w, 
   }
   if (lined) {
     const int outs = glu ? MOE_LINE_ROWS / 2 : MOE_LINE_ROWS;
-    const int64_t few = (int64_t)max_tiles * ((n_out + outs - 1) / outs) + (shared_w != nullptr ? (shared_n + outs - 1) / outs : 0);
-    if (most_places <= 16 && few <= 1 << 24) {           // no expert can get more places than that
-#define MOE_LINES_X(O, G, XV)                                                                                        \
-  hipLaunchKernelGGL((moe_lines_kernel<O, G, XV>), dim3((unsigned)few), dim3(MOE_LINE_WAVES * WAVE), 0, stream,       \
+    const int64_t workgroups = (int64_t)max_tiles * ((n_out + outs - 1) / outs) + (shared_w != nullptr ? (shared_n + outs - 1) / outs : 0);
+    if (most_places <= 16 && lines && workgroups <= 1 << 24) {
+#define MOE_LINES_X(O, G, XV, ONCE)                                                                                   \
+  hipLaunchKernelGGL((moe_lines_kernel<O, G, XV, ONCE>), dim3((unsigned)workgroups), dim3(MOE_LINE_WAVES * WAVE), 0, stream, \
                      (const bf16_t*)a, a_stride, (const bf16_t*)w, sorted_pair, tile_expert, tile_start, tile_rows, n_tiles, \
                      max_tiles, (O*)out, top, n_out, k_dim, limit, alpha, offset, act, both)
 #define MOE_LINES(O, G)                                                                                              \
   do {                                                                                                               \
-    if (most_places <= 4) MOE_LINES_X(O, G, 1);                                                                       \
-    else MOE_LINES_X(O, G, 2);                                                                                        \
+    if (most_places <= 4) MOE_LINES_X(O, G, 1, true);                                                                 \
+    else if (lines == 1) MOE_LINES_X(O, G, 2, true);                                                                  \
+    else MOE_LINES_X(O, G, 2, false);                                                                                 \
   } while (0)
       if (glu) MOE_LINES(bf16_t, true);
       else if (out_is_f32) MOE_LINES(float, false);
@@ -772,6 +865,24 @@ DRYFT_API int dryft_moe_product(const void* a, int64_t a_stride, const void* w, 
       return DRYFT_LAUNCH_CHECK();
     }
     if (shared_w != nullptr) return -1;
+    const dim3 few(max_tiles, (n_out + 15) / 16);
+    if (most_places <= 16 && few.y <= 65535) {           // no expert can get more places than that
+#define MOE_FEW_WAVES(O, G, W)                                                                                    \
+  hipLaunchKernelGGL((moe_product_few_kernel<O, G, W>), few, dim3(W * WAVE), 0, stream, (const bf16_t*)a, a_stride, \
+                     (const bf16_t*)w, sorted_pair, tile_expert, tile_start, tile_rows, n_tiles, (O*)out, top, n_out, \
+                     k_dim, limit, alpha, offset, act)
+#define MOE_FEW(O, G)                                                                                             \
+  do {                                                                                                            \
+    if (k_dim >= 1024) MOE_FEW_WAVES(O, G, 8);                                                                     \
+    else MOE_FEW_WAVES(O, G, 4);                                                                                   \
+  } while (0)
+      if (glu) MOE_FEW(bf16_t, true);
+      else if (out_is_f32) MOE_FEW(float, false);
+      else MOE_FEW(bf16_t, false);
+#undef MOE_FEW_WAVES
+#undef MOE_FEW
+      return DRYFT_LAUNCH_CHECK();
+    }
 #define MOE_MFMA(O, G)                                                                                            \
   hipLaunchKernelGGL((moe_product_mfma_kernel<O, G>), grid, block, 0, stream, (const bf16_t*)a, a_stride,          \
                      (const bf16_t*)w, sorted_pair, tile_expert, tile_start, tile_rows, n_tiles, (O*)out, top, n_out, \

@@ -124,7 +124,7 @@ _SIGNATURES = {
                "dryft_head_gate": [_P, _P, _L, _I, _P, _I, _I, _I, _I, _I, _I, _P]},
     "moe": {"dryft_moe_route": [_P, _L, _P, _I, _I, _I, _I, _F, _P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P],
             "dryft_moe_plan": [_P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _P],
-            "dryft_moe_product": [_P, _L, _P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _F, _F, _F, _I, _I, _I, _P, _L, _P, _P, _I,
+            "dryft_moe_product": [_P, _L, _P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _F, _F, _F, _I, _I, _I, _I, _P, _L, _P, _P, _I,
                                   _I, _I, _F, _F, _P],
             "dryft_moe_table_route": [_P, _P, _P, _P, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P],
             "dryft_moe_combine": [_P, _P, _P, _P, _P, _L, _I, _P, _I, _I, _I, _I, _P]},
@@ -2608,6 +2608,28 @@ def moe_takes_shared(a, w, plan: MoePlan, shared_w) -> bool:
         a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and shared_w.data_ptr() % 16 == 0
 
 
+def moe_lines_pay(plan: MoePlan, n_experts: int, k: int, gated: bool) -> int:
+    """Which kernel of few rows a product of K = ``k`` goes to: 0 the one that splits K over a workgroup's waves in runs, 1 the one
+    that reads whole lines, 2 that one with its weights kept in the caches. The second has more of K on its way at once but a shorter
+    walk does not fill that, and it goes over the weights again for every eight places of an expert, the first for sixteen. Time of
+    the second against the first over 1,700 sizes (2 to 128 experts, 64 to 5,120 outputs, K of 64 to 5,120, weights from memory):
+    gated products at up to four rows from K = 256 on 0.88, from 512 on 0.85, beyond 0.65 to 0.75 (below 256 not tried); at five to
+    sixteen rows K of 256 to 511 1.01 (up to 1.26), 512 to 1,023 0.92, beyond 0.7; products without a gate at up to four rows K below 256
+    1.16, of 256 to 511 1.05, of 512 to 1,023 0.95, at more rows there 1.01 (up to 1.18), from 1,024 on 0.83 to 0.89 at any. Rows that do
+    not start at whole lines (K % 64) lose it some of that: without a gate 0.97 to 1.15 from K = 1,024 on, gated up to 1.33 below.
+    More than eight rows of more than four places an expert on average: gated 1.2 below K = 1,024, then 0.86 to 0.97
+    with the weights kept, without a gate 1.05 to 1.45 (16 rows that all go to 4 experts, 4,976 x 136, 3.7 us and 8.7).
+    Where a shared expert rides along it is the second whatever the sizes, which saves the launches: whole layers of experts at up to
+    eight rows 0.75 to 0.87 of the time with the shared expert by itself (560 sizes, none above 0.98), at 9 to 16, the weights kept,
+    0.83 to 0.98 (up to 1.14)."""
+    rows, whole = plan.most_places, k % 64 == 0
+    if rows > 8 and plan.n_pairs > 4 * n_experts:
+        return 2 if gated and whole and k >= 1024 else 0
+    if gated:
+        return int(k >= (1024 if not whole else 256 if rows <= 4 else 512))
+    return int(whole and k >= (512 if rows <= 4 else 1024))
+
+
 def moe_products(a, w, plan: MoePlan, out, top: int, glu: tuple | None = None, act: str | None = None,
                  shared: tuple | None = None) -> None:
     """``out[place] = W_e a_row`` for every place of the plan, ``e`` the place's expert. ``top`` > 0: ``a`` is
@@ -2657,6 +2679,7 @@ def moe_products(a, w, plan: MoePlan, out, top: int, glu: tuple | None = None, a
         _ptr(a), a.stride(0), _ptr(w), _ptr(plan.sorted_pair), _ptr(plan.tiles[0]), _ptr(plan.tiles[1]),
         _ptr(plan.tiles[2]), _ptr(plan.n_tiles), plan.max_tiles, _ptr(out), 1 if out.dtype == torch.float32 else 0,
         int(top), n_out, k, 1 if glu else 0, float(limit), float(alpha), float(offset), 1 if act else 0, plan.most_places,
+        moe_lines_pay(plan, w.shape[0], k, bool(glu)) if shared is None else 1 if plan.most_places <= 8 else 2,
         _float_flag(a, "a"), *ride, _stream()),
         "moe_products")
 

@@ -39,6 +39,13 @@ from .linear import lines_pay, linear
 from .mlp import ClampedGLU, SquaredReLU, SwiGLU
 
 
+# Beyond eight rows the shared expert rides only while the products back to the width are fewer outputs than this, experts in use times
+# width: 6,000 workgroups of the kernel that reads whole lines, of which each goes over its weights twice there. Whole layers against the
+# shared expert by itself, experts of less than 512 inner: 1.04 on average beyond (up to 1.14), 0.95 from half as many on, 0.83 to 0.91 below;
+# of 240 and 1,224 inner, rows that do not start at whole lines, 1.08.
+_RIDES_BELOW = 96_000
+
+
 class RoutedExperts(FeedForward):
     def __init__(self, hidden_size: int, experts: int, top: int, intermediate_size: int, limit: float | None = None,
                  route_scale: float = 1.0, groups: tuple[int, int] | None = None,
@@ -177,6 +184,8 @@ class RoutedExperts(FeedForward):
         if shared is None or type(shared) not in (ClampedGLU, SwiGLU, SquaredReLU) or "forward" in vars(shared):
             return False
         rows, w_in = h.shape[0], self._shared_unit()[0]
+        if rows > 8 and (self.inter % 64 or min(rows * self.top, self.n_experts) * self.hidden >= _RIDES_BELOW):
+            return False
         return ops.moe_takes_shared(h, self.w_gate_up, plan, w_in) and self.inter % 8 == 0 and shared.inter % 8 == 0 and \
             self.w_down.data_ptr() % 16 == 0 and shared.w_down.data_ptr() % 16 == 0 and \
             (ops.few_glu_pays(rows, shared.inter, self.hidden) if self.gated else lines_pay(rows, shared.inter, self.hidden)) and \

@@ -58,6 +58,33 @@ def test_experts_and_the_shared_one(rows, experts, top, k, inter, shared_inter, 
     close(y_s, act_s.cpu().double() @ down_s.double().T, torch.bfloat16, what="shared, back")
 
 
+@pytest.mark.parametrize("rows,experts,top", [(1, 4, 4), (4, 16, 2), (6, 3, 3), (9, 2, 2), (16, 1, 1), (16, 16, 4)])
+@pytest.mark.parametrize("k,inter", [(64, 24), (248, 1024), (256, 520), (512, 72), (1032, 512), (1024, 1080)])
+@pytest.mark.parametrize("kind", ["silu", "clamped", "relu2"])
+def test_experts_alone(rows, experts, top, k, inter, kind):
+    """Without a shared expert the kernel follows from rows, places and K: every one it may be, on both sides of the lines."""
+    from dryft_amd.csrc import ops
+    torch.manual_seed(rows * 1000 + k + inter)
+    halves = 1 if kind == "relu2" else 2
+    x = torch.randn(rows, k).to(torch.bfloat16)
+    w = (torch.randn(experts, halves * inter, k) * 2 / math.sqrt(k)).to(torch.bfloat16)
+    down = (torch.randn(experts, k, inter) / math.sqrt(inter)).to(torch.bfloat16)
+    chosen = torch.stack([torch.randperm(experts)[:top] for _ in range(rows)]).to(torch.int32)
+    plan = ops.moe_plan(chosen.to(DEV), experts)
+    act, y = torch.full((rows * top, inter), float("nan"), dtype=torch.bfloat16, device=DEV), torch.full((rows * top, k), float("nan"), device=DEV)
+    how = dict(act="relu2") if kind == "relu2" else dict(glu=(float("inf"), 1.0, 0.0) if kind == "silu" else (1.5, 1.702))
+    ops.moe_products(x.to(DEV), w.to(DEV), plan, act, top, **how)
+    ops.moe_products(act, down.to(DEV), plan, y, 0)
+    place = plan.place_of.cpu().view(rows, top)
+    a = act.cpu().double()
+    for e in range(experts):
+        at = [(r, int(place[r, t])) for r in range(rows) for t in range(top) if int(chosen[r, t]) == e]
+        if at:
+            r, p = [i for i, _ in at], [j for _, j in at]
+            close(act[p], unit_of(x[r].double() @ w[e].double().T, kind), torch.bfloat16, ulps=4.0, what=f"expert {e}")
+            close(y[p], a[p] @ down[e].double().T, torch.float32, what=f"expert {e}, back")
+
+
 def test_a_replaced_shared_expert_is_called():
     """A shared expert whose ``forward`` was replaced on the object runs as it says, ahead of everything that rides along."""
     from dryft_amd.csrc import ops
