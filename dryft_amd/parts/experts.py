@@ -46,6 +46,10 @@ from .mlp import ClampedGLU, SquaredReLU, SwiGLU
 _RIDES_BELOW = 96_000
 
 
+# By the experts' unit, the class of their shared expert and its call as this library has it: what the grouped products stand for.
+_SHARED_AS_MADE = {unit: (made, made.forward) for unit, made in (("clamped", ClampedGLU), ("silu", SwiGLU), ("relu2", SquaredReLU))}
+
+
 class RoutedExperts(FeedForward):
     def __init__(self, hidden_size: int, experts: int, top: int, intermediate_size: int, limit: float | None = None,
                  route_scale: float = 1.0, groups: tuple[int, int] | None = None,
@@ -81,8 +85,8 @@ class RoutedExperts(FeedForward):
             raise ValueError(f"{experts} experts in {count} groups of which {keep} are kept cannot give {top}")
         self.shared = None
         if shared:
-            self.shared = ClampedGLU(hidden_size, shared[0], shared[1], alpha) if unit == "clamped" else \
-                SwiGLU(hidden_size, shared[0]) if unit == "silu" else SquaredReLU(hidden_size, shared[0])
+            made = _SHARED_AS_MADE[unit][0]
+            self.shared = made(hidden_size, shared[0], shared[1], alpha) if unit == "clamped" else made(hidden_size, shared[0])
         self.w_router = self.correction = self.router_bias = self.w_gate_up = self.w_down = self.table = None
 
     def tensor_specs(self):
@@ -181,7 +185,8 @@ class RoutedExperts(FeedForward):
         """Are the shared expert's products made in the launches of the routed ones? Steps of few rows whose own products would
         go to the same kind of kernel (``few_glu_pays``, ``lines_pay``), and only where the shared expert is as it was made."""
         shared = self.shared
-        if shared is None or type(shared) not in (ClampedGLU, SwiGLU, SquaredReLU) or "forward" in vars(shared):
+        made, call = _SHARED_AS_MADE[self.unit]
+        if type(shared) is not made or made.forward is not call or "forward" in vars(shared) or getattr(shared, "relu", False):
             return False
         rows, w_in = h.shape[0], self._shared_unit()[0]
         if rows > 8 and (self.inter % 64 or min(rows * self.top, self.n_experts) * self.hidden >= _RIDES_BELOW):

@@ -85,20 +85,29 @@ def test_experts_alone(rows, experts, top, k, inter, kind):
             close(y[p], a[p] @ down[e].double().T, torch.float32, what=f"expert {e}, back")
 
 
-def test_a_replaced_shared_expert_is_called():
-    """A shared expert whose ``forward`` was replaced on the object runs as it says, ahead of everything that rides along."""
+@pytest.mark.parametrize("unit", ["silu", "clamped", "relu2"])
+@pytest.mark.parametrize("how", ["object", "class", "exchanged"])
+def test_a_replaced_shared_expert_is_called(monkeypatch, unit, how):
+    """A shared expert whose ``forward`` was replaced, or that is another part, adds what it says to what the routed ones give without one."""
     from dryft_amd.csrc import ops
+    from dryft_amd.parts.base import FeedForward
     from dryft_amd.parts.experts import RoutedExperts
-    part = RoutedExperts(64, 4, 2, 16, unit="silu", shared=(24,), correction=False)
-    part.compute_dtype = torch.bfloat16
     torch.manual_seed(0)
-    part.load({name: torch.randn(*spec[0]).to(torch.bfloat16).to(DEV) * 0.1 for name, spec in part.tensor_specs().items()})
-    h, ctx = torch.randn(3, 64).to(torch.bfloat16).to(DEV), None
-    plain = part.forward(h, ctx)
-    plan = ops.MoePlan(6, 4, DEV, most_places=3)
+    make = lambda shared: RoutedExperts(64, 4, 2, 64, limit=1.5 if unit == "clamped" else None, unit=unit, shared=shared, correction=False, shared_gate=False)
+    part, alone = make((24, 1.5)), make(None)
+    part.compute_dtype = alone.compute_dtype = torch.bfloat16
+    tensors = {name: torch.randn(*spec[0]).to(torch.bfloat16).to(DEV) * 0.1 for name, spec in part.tensor_specs().items()}
+    part.load(tensors)
+    alone.load(tensors)
+    h, plan = torch.randn(3, 64).to(torch.bfloat16).to(DEV), ops.MoePlan(6, 4, DEV, most_places=3)
     assert part._shared_rides(h, plan)
-    made = part.shared.forward
-    part.shared.forward = lambda rows, step: 0 * made(rows, step).summed(torch.bfloat16) if hasattr(made(rows, step), "summed") else 0 * made(rows, step)
-    assert not part._shared_rides(h, plan)
-    without = part.forward(h, ctx)
-    assert not torch.equal(plain, without)
+    half = lambda *a, **k: torch.full((3, 64), 0.5, dtype=torch.bfloat16, device=DEV)
+    if how == "object":
+        part.shared.forward = half
+    elif how == "class":
+        monkeypatch.setattr(type(part.shared), "forward", half)
+    else:
+        part.shared = type("Half", (FeedForward,), {"forward": half})()
+    # both sides round the routed sum once to bfloat16, one of them with 0.5 added
+    got, want = part.forward(h, None).double(), alone.forward(h, None).double() + 0.5
+    assert bool(((got - want).abs() <= 2.0 ** -8 * (got.abs() + (want - 0.5).abs())).all())

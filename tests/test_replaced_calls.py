@@ -165,3 +165,38 @@ def test_mixers_side_by_side_with_a_replaced_call_begin_alone(monkeypatch, name)
         both.mixers["left"].forward_split = lambda h, ctx, line, writes_cache: (3 * h, None)
     assert both._first_products(h, STEP) == {}
     assert torch.equal(both.mixers["left"].forward_split(h, STEP, None, True)[0], 3 * h)
+
+
+def routed(unit):
+    from dryft_amd.parts.experts import RoutedExperts
+    part = RoutedExperts(64, 4, 2, 64, limit=2.0 if unit == "clamped" else None, unit=unit, shared=(128, 2.0), correction=False)
+    part.load({name: torch.zeros(*spec[0], dtype=torch.bfloat16) for name, spec in part.tensor_specs().items()})
+    return part
+
+
+@pytest.mark.parametrize("unit", ["silu", "clamped", "relu2"])
+def test_only_the_shared_expert_that_was_made_rides_along(monkeypatch, unit):
+    """A shared expert whose call is replaced, on the object or on its class, or that is exchanged for one of another unit, runs as it
+    says and not in the routed ones' launches, which know the unit of the routed ones alone."""
+    from dryft_amd.csrc import ops
+    from dryft_amd.parts.mlp import ClampedGLU, ReGLU, SquaredReLU, SwiGLU
+    part, h, plan = routed(unit), torch.zeros(3, 64, dtype=torch.bfloat16), ops.MoePlan(6, 4, "cpu", most_places=3)
+    made, own = part.shared, type(part.shared)
+    assert part._shared_rides(h, plan)
+    made.forward = lambda h, ctx: h
+    assert not part._shared_rides(h, plan)
+    del made.forward
+    with monkeypatch.context() as m:
+        m.setattr(own, "forward", lambda self, h, ctx, leave_product=False: h)
+        assert not part._shared_rides(h, plan)
+    assert part._shared_rides(h, plan)
+    for other in (ClampedGLU(64, 128, 2.0), SwiGLU(64, 128), ReGLU(64, 128), SquaredReLU(64, 128)):
+        if type(other) is own:
+            continue
+        other.load({name: torch.zeros(*spec[0], dtype=torch.bfloat16) for name, spec in other.tensor_specs().items()})
+        part.shared = other
+        assert not part._shared_rides(h, plan), type(other)
+    part.shared = made
+    if unit == "silu":
+        made.relu = True                                     # the gated unit's own switch
+        assert not part._shared_rides(h, plan)
