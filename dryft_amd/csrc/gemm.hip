@@ -551,11 +551,13 @@ DRYFT_API int dryft_gemm_wide_swiglu_bf16(const void* x, int64_t x_stride, const
 // with depths of their own (26 at best). The plain product of the same form was no faster than what serves it now.
 // Walking K from a different starting group in every workgroup took Qwen3-8B's gate/up (rows 8,192 bytes apart)
 // from 44 to 38 us at 8 to 40 rows; at Qwen3-4B's 5,120 bytes it changes nothing.
-// The caches are told that the weights are read once (panel_load16_once): in a captured chain on rotating cold weights, us at 17 /
-// 33 / 64 rows, 9,728 outputs of K 2,560 19.5 / 20.7 / 23.4 (without 20.9 / 21.5 / 23.6), 12,288 of 4,096 35.9 / 36.6 / 38.2 (39.2 /
-// 39.3 / 40.9), 8,192 of 2,048 12.9 / 13.3 / 15.4 (13.9 / 13.7 / 15.2). At 65 to 96 rows it loads 80 or 96 rows of x where the tall form below
-// loads 128: at 65 / 80 / 96 rows the first 23.7 / 24.4 / 26.3 (26.0 / 27.2 / 28.3), the second 39.2 / 39.0 / 40.5 (44.5 / 47.8 / 45.3),
-// 3,072 of 1,024 8.5 / 8.8 / 9.7 (9.9 / 10.0 / 10.2); at 112 it is behind (31.8 / 29.8, 52 / 45, 11.3 / 10.4).
+// Matrices of 48 MiB on are read as lines that the caches give up first (panel_load16_once): with 0.89 to 0.96 of the time in a captured
+// chain on weights from memory (us at 17 / 33 / 64 rows, 9,728 outputs of K 2,560 19.5 / 20.7 / 23.4, without 20.9 / 21.5 / 23.6, 12,288 of
+// 4,096 35.9 / 36.6 / 38.2 and 39.2 / 39.3 / 40.9), and models of three layers of such do not stay in the last-level cache between steps.
+// Smaller ones may: 0.95 to 0.98 from memory, but weights of 150 MB in all, which stay, take 1.05 to 1.48 of the time with the
+// hint (2 x 1,376 of 5,120 at 32 rows 14.9 and 22.1, 2 x 4,928 of 1,280 7.1 and 9.1; the hint as a branch in the kernel 1.01 to 1.08).
+// At 65 to 96 rows it loads 80 or 96 rows of x where the tall form below loads 128: at 65 / 80 / 96 rows 9,728 of 2,560 23.7 / 24.4 / 26.3 (26.0 / 27.2 / 28.3), 12,288 of 4,096 39.2 / 39.0 / 40.5 (44.5 / 47.8 / 45.3),
+// 3,072 of 1,024 8.6 / 8.9 / 9.6 (9.7 / 9.9 / 10.2); at 112 it is behind (31.8 / 29.8, 52 / 45, 11.3 / 10.4).
 __device__ __forceinline__ void panel_load16(const void* base, uint32_t offset, uint32_t lds_base) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(offset), "s"(base) : "memory", "m0");
 }
@@ -602,13 +604,14 @@ __device__ __forceinline__ void swiglu_store4(bf16_t* __restrict__ y_row, int fi
 
 #define PANEL_GROUP 128                      // values of K in a group; K must be a multiple of it
 #define PANEL_ROWS 96
+#define PANEL_ONCE_BYTES (48 << 20)          // gate/up matrices from here on are read as lines not kept
 // Groups of K in LDS: three, or two where a third does not fit (96 rows of x and 128 of W).
 constexpr int panel_stages(int mt, int waves) { return 3 * (16 * waves + 16 * mt) * 2 * PANEL_GROUP <= 160 * 1024 ? 3 : 2; }
 
 // WAVES waves, 8 outputs each: a wave's 16 weight rows are the gate rows of its 8 outputs and then their up rows, so
 // that gate and up of an output meet in lanes 32 apart and no LDS pass is needed at the end. The launcher picks
 // WAVES so that the workgroups are about as many as the compute units and all run at once.
-template <int MT, int WAVES>
+template <int MT, int WAVES, bool ONCE>
 __global__ __launch_bounds__(64 * WAVES) void gemm_panel_swiglu_kernel(const bf16_t* __restrict__ x, int64_t x_stride,
                                                                        const bf16_t* __restrict__ w,
                                                                        bf16_t* __restrict__ y, int M, int N, int K,
@@ -650,7 +653,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_panel_swiglu_kernel(const bf1
     const unsigned char* xb = (const unsigned char*)x + (int64_t)gk * RB;
     const uint32_t at = lds0 + stage * STAGE_BYTES;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) panel_load16_once<true>(wb, w_from[i], at + (16 * wave + 4 * i) * RB);
+    for (int i = 0; i < 4; ++i) panel_load16_once<ONCE>(wb, w_from[i], at + (16 * wave + 4 * i) * RB);
 #pragma unroll
     for (int i = 0; i < X_LOADS; ++i) panel_load16(xb, x_from[i], at + W_BYTES + x_piece[i] * 1024);
   };
@@ -711,13 +714,13 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_panel_swiglu_kernel(const bf1
   }
 }
 
-template <int MT, int WAVES>
-static int launch_panel_swiglu(const void* x, int64_t x_stride, const void* w, void* y, int M, int N, int K,
+template <int MT, int WAVES, bool ONCE>
+static int launch_panel(const void* x, int64_t x_stride, const void* w, void* y, int M, int N, int K,
                                hipStream_t stream, GateAct act) {
   constexpr int lds = panel_stages(MT, WAVES) * (16 * WAVES + 16 * MT) * 2 * PANEL_GROUP;
   static_assert(lds <= 160 * 1024, "the stages must fit a compute unit's LDS");
   static bool raised = false;                              // more dynamic LDS than the default limit allows
-  auto kernel = gemm_panel_swiglu_kernel<MT, WAVES>;
+  auto kernel = gemm_panel_swiglu_kernel<MT, WAVES, ONCE>;
   if (lds > 64 * 1024 && !raised) {
     if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return -2;
     raised = true;
@@ -726,6 +729,13 @@ static int launch_panel_swiglu(const void* x, int64_t x_stride, const void* w, v
   hipLaunchKernelGGL(kernel, grid, block, lds, stream, (const bf16_t*)x, x_stride, (const bf16_t*)w, (bf16_t*)y, M, N, K,
                      act);
   return DRYFT_LAUNCH_CHECK();
+}
+
+template <int MT, int WAVES>
+static int launch_panel_swiglu(const void* x, int64_t x_stride, const void* w, void* y, int M, int N, int K,
+                               hipStream_t stream, GateAct act) {
+  if ((int64_t)4 * N * K >= PANEL_ONCE_BYTES) return launch_panel<MT, WAVES, true>(x, x_stride, w, y, M, N, K, stream, act);
+  return launch_panel<MT, WAVES, false>(x, x_stride, w, y, M, N, K, stream, act);
 }
 
 template <int MT>

@@ -11,11 +11,12 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-@pytest.mark.parametrize("m", [65, 80, 81, 96])
-@pytest.mark.parametrize("inter,k,waves", [(47, 128, 0), (100, 640, 5), (136, 256, 8), (1024, 2560, 4)])
+@pytest.mark.parametrize("m", [5, 17, 64, 65, 80, 81, 96])
+@pytest.mark.parametrize("inter,k,waves", [(47, 128, 0), (100, 640, 5), (136, 256, 8), (1024, 2560, 4), (6152, 2048, 0)])
 @pytest.mark.parametrize("unit", ["silu", "relu", "clamped"])
 def test_panel_of_up_to_96_rows(m, inter, k, waves, unit):
-    """Five and six tiles of rows, three stages in LDS and (eight waves at 96 rows) two; rows of x wider apart than K."""
+    """One to six tiles of rows, three stages in LDS and (eight waves at 96 rows) two; weights kept and, from 48 MiB on, read once; rows of
+    x wider apart than K."""
     from dryft_amd.csrc import ops
     torch.manual_seed(m + inter + k)
     x = torch.randn(m, k + 8).to(torch.bfloat16)
