@@ -2121,12 +2121,17 @@ def rglru_scan(coef, proj, x_col: int, y_col: int, x_bias, y_bias, taps: int, se
 RGLRU_TOKEN_BLOCK = 256
 
 
-def rglru_token_takes(proj, state, gate_a, gate_i, vectors, blocks: int) -> bool:
+def rglru_token_takes(proj, state, gate_a, gate_i, vectors, blocks: int, taps: int = 1) -> bool:
     """Does ``rglru_token`` take these tensors, and gain by it: bfloat16, blocks of a multiple of 32 channels up to ``RGLRU_TOKEN_BLOCK``, the state, the
     gates and the ``vectors`` (gate biases, lam, y_bias) at 16-byte addresses; up to 16 rows only blocks of at most 128 channels (4 rows of
-    blocks of 256: 18.4 us against 13.9 for gates and walk, 64 rows 25 against 121; 4 rows of blocks of 128 8.1 against 12.1)."""
-    size = state.shape[1] // blocks if blocks > 0 else 0
-    return proj.dtype == torch.bfloat16 and size % 32 == 0 and 0 < size <= (RGLRU_TOKEN_BLOCK if proj.shape[0] > 16 else 128) and \
+    blocks of 256: 18.4 us against 13.9 for gates and walk, 64 rows 25 against 121; 4 rows of blocks of 128 8.1 against 12.1). A workgroup's
+    waves, one for 16 channels, form the convolution of its rows one after another, which ``taps`` beyond four make long for the two or four
+    waves of small blocks: 8 taps, blocks of 32 channels, 2 / 6 / 16 / 32 / 128 rows 10.1 / 12.8 / 26.8 / 26.8 / 31.0 against 12.9 / 10.2 / 10.7 /
+    18.3 / 22.2, of 64, 8 / 16 / 24 rows 12.7 / 17.4 / 18.1 against 13.6 / 13.0 / 30.1."""
+    rows, size = proj.shape[0], state.shape[1] // blocks if blocks > 0 else 0
+    if taps > 4 and ((size == 32 and rows > 2) or (size == 64 and 8 < rows <= 16)):
+        return False
+    return proj.dtype == torch.bfloat16 and size % 32 == 0 and 0 < size <= (RGLRU_TOKEN_BLOCK if rows > 16 else 128) and \
         all(t.data_ptr() % 16 == 0 for t in (state, gate_a, gate_i, *vectors))
 
 

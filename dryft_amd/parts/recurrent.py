@@ -161,7 +161,8 @@ class GatedLinearRecurrence(Mixer):
         proj = linear(h, self.w_in)
         tail = line["tail"].state if self.taps > 1 else None
         if ctx.max_q_len == 1 and ops.rglru_token_takes(proj, line["state"].state, self.gate_a, self.gate_i,
-                                                        (self.gate_a_bias, self.gate_i_bias, self.lam, self.y_bias), self.blocks):
+                                                        (self.gate_a_bias, self.gate_i_bias, self.lam, self.y_bias), self.blocks,
+                                                        self.taps):
             # one row a sequence: gates, walk and the convolution's memory in one launch
             out = torch.empty((rows, W), dtype=h.dtype, device=h.device)
             ops.rglru_token(proj, W, 0, self.x_bias, self.y_bias, self.conv, self.conv_bias, self.taps, self.gate_a, self.gate_a_bias,

@@ -149,3 +149,16 @@ def test_experts_of_few_rows_go_where_they_were_measured_ahead(rows, experts, to
     from dryft_amd.csrc import ops
     plan = ops.MoePlan(rows * top, experts, "cpu", most_places=rows)
     assert ops.moe_lines_pay(plan, experts, k, gated) == kernel
+
+
+@pytest.mark.parametrize("rows,size,taps,takes", [
+    (16, 128, 4, True), (16, 256, 4, False), (16, 160, 4, False), (17, 256, 4, True), (17, 288, 4, False), (4, 48, 4, False), (16, 32, 4, True),
+    (2, 32, 8, True), (3, 32, 8, False), (128, 32, 5, False), (8, 64, 8, True), (9, 64, 8, False), (17, 64, 8, True), (16, 96, 16, True)])
+def test_one_row_of_a_gated_recurrence_goes_where_it_was_measured_ahead(rows, size, taps, takes):
+    from dryft_amd.csrc import ops
+    blocks = 3
+    aligned = lambda *shape, dtype: torch.empty(shape, dtype=dtype)
+    proj, state = aligned(rows, 2 * blocks * size, dtype=torch.bfloat16), aligned(rows, blocks * size, dtype=torch.float32)
+    gate, vector = aligned(blocks, size, size, dtype=torch.bfloat16), aligned(blocks * size, dtype=torch.float32)
+    assert ops.rglru_token_takes(proj, state, gate, gate, (vector,) * 4, blocks, taps) == takes
+    assert not ops.rglru_token_takes(proj.float(), state, gate, gate, (vector,) * 4, blocks, taps)
