@@ -84,12 +84,24 @@ def float32_form(rows: int, n_heads: int, n_kv: int, head_dim: int, longest: int
     return "rows" if longest == 1 or few else "tiles"
 
 
-def float32_splits(rows: int, n_heads: int, n_kv: int, keys: int) -> int:
+def float32_splits(rows: int, n_heads: int, n_kv: int, keys: int, head_dim: int = 128) -> int:
     """Over how many workgroups the keys of a float32 decoding row go: as many as make one for each compute unit, none where that is
     fewer than four (16 heads on 8 of 128, 16 rows, two: 150 keys 11.3 -> 11.9 us, of 256 19.4 -> 22.2), nor more than half pages go
-    round two waves each. More than one a unit is no better: four rows of 4,096 keys, 8 / 16 / 32 splits 35 / 39 / 45 us."""
+    round two waves each. More than one a unit is no better: four rows of 4,096 keys, 8 / 16 / 32 splits 35 / 39 / 45 us.
+    And only where the rounds of half pages that are saved outweigh the last workgroup's adding up, a load for every query head, feature and
+    split on as few as two waves. Up to 64 features (eight waves) that is from 129 keys on (2 splits of 66 to 128 keys 5 to 8 % behind); beyond, a
+    model in us, a half page's round ~ features, fitted to 980 times of 30 to 3,000 keys: what it splits is ahead or within 5 % but for 4 of
+    780 (1.10 at most), what it leaves whole would take 1.2 times as long split on average. 16 heads on one of 256, four rows of 304
+    keys, whole / split 33 / 51 us, of 192, 1,033 keys in a window of 512 38 / 48; 64 on 4 of 80, eight of 158 12.7 / 15.4."""
+    columns = min(16, n_heads // n_kv)
     splits = min(_UNITS // (rows * n_kv * ((n_heads // n_kv + 15) // 16)), ops.ATTN_F32_SPLITS)
-    return max(1, min(splits, -(-keys // 64))) if splits >= 4 else 1
+    splits = max(1, min(splits, -(-keys // 64))) if splits >= 4 else 1
+    if splits == 1 or head_dim <= 64:
+        return splits if keys > 128 else 1
+    waves, alone, halves = (4 if head_dim <= 128 else 2), (8 if head_dim == 128 else 4), -(-keys // 32)
+    size, parts = head_dim / 512, min(splits, -(-halves // waves))
+    saved = 3.9 * size * alone * -(-halves // alone) - (5.0 if waves == 4 else 6.6) * size * waves * -(-halves // (waves * splits))
+    return splits if saved > 0.15 * columns * head_dim * parts / (64 * waves) + (1.0 if waves == 4 else 5.0) else 1
 
 
 def add_bias(delta, bias: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
@@ -500,7 +512,7 @@ class GQAAttention(Mixer):
         form = float32_form(rows, self.n_heads, self.n_kv, self.head_dim, ctx.max_q_len,
                             min(window or ctx.max_kv_len, ctx.max_kv_len)) if h.dtype == torch.float32 else None
         one_each = form == "rows" and ctx.max_q_len == 1 and rows == ctx.n_seqs
-        f32_splits = float32_splits(rows, self.n_heads, self.n_kv, min(window or ctx.max_kv_len, ctx.max_kv_len)) if one_each else 1
+        f32_splits = float32_splits(rows, self.n_heads, self.n_kv, min(window or ctx.max_kv_len, ctx.max_kv_len), self.head_dim) if one_each else 1
         counters = split_counters(ctx, self.n_heads, self.n_kv) if f32_splits > 1 else None
         if one_each and ops.attn_f32_fused_takes(qkv, self.q_norm, self.k_norm, cos, sin, self.rotary_dim, line.k, line.v, self.n_heads,
                                                  self.n_kv, self.head_dim, f32_splits):

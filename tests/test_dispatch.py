@@ -162,3 +162,12 @@ def test_one_row_of_a_gated_recurrence_goes_where_it_was_measured_ahead(rows, si
     gate, vector = aligned(blocks, size, size, dtype=torch.bfloat16), aligned(blocks * size, dtype=torch.float32)
     assert ops.rglru_token_takes(proj, state, gate, gate, (vector,) * 4, blocks, taps) == takes
     assert not ops.rglru_token_takes(proj.float(), state, gate, gate, (vector,) * 4, blocks, taps)
+
+
+@pytest.mark.parametrize("rows,heads,kv,keys,width,splits", [
+    (4, 16, 8, 512, 128, 8), (4, 16, 8, 128, 64, 1), (4, 16, 8, 192, 64, 3), (4, 16, 1, 304, 256, 1), (4, 64, 4, 334, 256, 1),
+    (4, 16, 1, 4096, 256, 32), (8, 64, 4, 158, 80, 1), (1, 6, 2, 114, 256, 1), (1, 4, 1, 1024, 192, 16), (1, 16, 1, 256, 80, 1)])
+def test_float32_keys_are_split_where_that_was_measured_ahead(rows, heads, kv, keys, width, splits):
+    """What was up to twice as slow split, since the last workgroup adds up many wide parts, stays with one workgroup."""
+    from dryft_amd.parts.attention import float32_splits
+    assert float32_splits(rows, heads, kv, keys, width) == splits
