@@ -1743,12 +1743,23 @@ def map_difference(a, out, v_dim: int, lam: float, post: float, eps: float) -> t
 ROWS_A_KV_HEAD = 16         # rows of queries of a kv head that ``attn_turned_bf16`` takes (two maps are two rows)
 
 
-def turns_in_attention(n_seqs: int, rows_a_kv_head: int, page_dim: int) -> bool:
-    """Does ``attn_turned_bf16`` take a step of so many sequences, and gain by it? A wave turns every fourth row of queries, one or two
-    at a time: 16 rows of 128 features for 8 sequences of 1,000 keys 16.1 us against 15.2 for the turn in a launch of its own, 8 rows
-    of 64 (two maps) 10.8 against 12.5. Heads beyond 192 features leave it no registers: 8 x 1,000 keys 30 against 25. From 32
-    sequences on the other launch's rows cost more than either: 16 rows of 224 29 against 41, of 128 for 64 sequences 24 against 34."""
-    return rows_a_kv_head <= ROWS_A_KV_HEAD and (n_seqs >= 32 or (rows_a_kv_head <= 8 and page_dim <= 192))
+def turns_in_attention(n_seqs: int, rows_a_kv_head: int, page_dim: int, kv_keys: int = 0, spares: bool = False) -> bool:
+    """Does ``attn_turned_bf16`` take a step of so many sequences, and gain by it? ``kv_keys``: kv heads times the keys a sequence has at
+    most; ``spares``: two maps a head, or a gate whose launch it spares too.
+
+    A wave turns every fourth row of queries, one or two at a time, in every workgroup of a kv head. Time of the one launch against the
+    two or three, 1,300 steps of 8 to 16,000 keys: up to six rows a kv head 0.72 to 0.98 up to 160 features (129 to 159, which
+    leave the registers no room for whole tiles, 0.97 to 1.01 at five and six), seven 0.83 to 0.97, eight 0.87 to 0.88 up to 64 features, beyond
+    0.93 to 0.98 without maps or gate (up to 1.10) and 0.9 with, at 160 1.01 (up to 1.13); heads of 192 1.03 to 1.18 (up to 1.32) and wider
+    ones spill. From 32 sequences on the other launch's rows cost more: 0.66 to 0.77 at up to 16 rows of any width; only heads of 161
+    to 192 features lose that where the keys are many (32 to 64 sequences, kv heads times keys 0.5 to 1 up to 150,000, beyond up to 1.33)."""
+    if rows_a_kv_head > ROWS_A_KV_HEAD:
+        return False
+    six = 160 < page_dim <= 192
+    if n_seqs >= 32:
+        return not six or n_seqs * kv_keys < 150_000
+    most = 8 if page_dim <= 64 or (spares and page_dim <= 128) else 7 if page_dim <= 128 or page_dim == 160 else 4 if page_dim < 160 else 0
+    return rows_a_kv_head <= most
 
 
 class Turned(NamedTuple):

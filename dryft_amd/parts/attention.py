@@ -341,10 +341,12 @@ class GQAAttention(Mixer):
         matrix_cores = h.dtype == torch.bfloat16 and (wide or (D == Dv and D % MATRIX_CORE_HEAD_STEP == 0))
         window = self.window or 0
         g_col = self.q_dim + self.kv_dim + self.v_dim
-        if matrix_cores and ctx.max_q_len == 1 and ops.turns_in_attention(ctx.n_seqs, H // G, wide or D):
+        gates_there = self.output_gate and not self.head_gate and not wide
+        if matrix_cores and ctx.max_q_len == 1 and ops.turns_in_attention(
+                ctx.n_seqs, H // G, wide or D, G * min(self.window or self.chunk or ctx.max_kv_len, ctx.max_kv_len), gates_there):
             # one row a sequence: turn, append, attention and a gate of every feature in one launch
             P = wide or D
-            gate = proj[:, g_col:g_col + self.o_dim] if self.output_gate and not self.head_gate and not wide else None
+            gate = proj[:, g_col:g_col + self.o_dim] if gates_there else None
             turned = ops.Turned(src, 0, self.q_dim, self.q_dim + self.kv_dim, D, Dv, cos, sin, rot, by_pairs,
                                 q_weight=self.q_norm if self.qk_norm_eps is not None else None,
                                 k_weight=self.k_norm if self.qk_norm_eps is not None else None,

@@ -111,7 +111,7 @@ class DifferentialAttention(Mixer):
         wide, step = self.page_dim(), self.map_width()
         decoding = bool(wide) and ctx.max_q_len == 1
         window, post = self.window or 0, 1.0 - self.diff
-        if decoding and ops.turns_in_attention(ctx.n_seqs, 2 * H // G, wide):
+        if decoding and ops.turns_in_attention(ctx.n_seqs, 2 * H // G, wide, G * min(self.window or ctx.max_kv_len, ctx.max_kv_len), True):
             # one row a sequence: turn, append and attention in one launch
             out = torch.empty((rows, H, Dv), dtype=h.dtype, device=h.device)
             splits = key_splits(ctx.n_seqs, G, self.window or ctx.max_kv_len)

@@ -164,6 +164,18 @@ def test_one_row_of_a_gated_recurrence_goes_where_it_was_measured_ahead(rows, si
     assert not ops.rglru_token_takes(proj.float(), state, gate, gate, (vector,) * 4, blocks, taps)
 
 
+@pytest.mark.parametrize("seqs,rows,width,kv_keys,spares,takes", [
+    (4, 8, 64, 4000, False, True), (4, 9, 64, 4000, False, False), (4, 8, 128, 4000, True, True), (4, 8, 128, 4000, False, False),
+    (4, 7, 128, 4000, False, True), (31, 7, 160, 4000, True, True), (4, 8, 160, 4000, True, False), (4, 4, 144, 4000, False, True),
+    (4, 5, 144, 4000, True, False), (4, 1, 176, 100, True, False), (1, 1, 192, 100, False, False), (8, 2, 256, 100, True, False),
+    (32, 16, 128, 1 << 20, False, True), (32, 16, 256, 1 << 20, False, True), (32, 16, 192, 4687, False, True),
+    (32, 16, 192, 4688, True, False), (64, 17, 64, 100, True, False)])
+def test_the_turn_goes_into_attention_where_it_was_measured_ahead(seqs, rows, width, kv_keys, spares, takes):
+    """Heads of 192 features and 5 to 8 rows a kv head of odd widths were up to a third slower in one launch."""
+    from dryft_amd.csrc import ops
+    assert ops.turns_in_attention(seqs, rows, width, kv_keys, spares) == takes
+
+
 @pytest.mark.parametrize("rows,heads,kv,keys,width,splits", [
     (4, 16, 8, 512, 128, 8), (4, 16, 8, 128, 64, 1), (4, 16, 8, 192, 64, 3), (4, 16, 1, 304, 256, 1), (4, 64, 4, 334, 256, 1),
     (4, 16, 1, 4096, 256, 32), (8, 64, 4, 158, 80, 1), (1, 6, 2, 114, 256, 1), (1, 4, 1, 1024, 192, 16), (1, 16, 1, 256, 80, 1)])
