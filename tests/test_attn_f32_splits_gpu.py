@@ -2,6 +2,7 @@
 numbers, and with the counters of one launch used again by the next."""
 import pytest
 import torch
+from test_attn_turned_gpu import exact_rows, turned_exactly
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -84,7 +85,7 @@ def test_where_keys_are_split():
 @pytest.mark.parametrize("splits", [1, 4, 32])
 @pytest.mark.parametrize("H,G,D,normed,window", [(16, 8, 128, True, 0), (16, 1, 64, False, 0), (6, 3, 96, True, 40), (4, 4, 32, True, 0), (20, 4, 128, False, 33)])
 def test_turn_and_attention_in_one(H, G, D, normed, window, splits, write):
-    """Against the launch of its own for norm, turn and append and then one workgroup a row: float32 throughout, the same formulas."""
+    """Against 64 bits, and against the launch of its own for norm, turn and append and then one workgroup a row: float32 throughout."""
     from dryft_amd.csrc import ops
     if D == 128:
         splits = max(splits, 2)                    # unsplit, heads of 128 keep the two launches
@@ -107,3 +108,13 @@ def test_turn_and_attention_in_one(H, G, D, normed, window, splits, write):
     assert torch.equal(v1, v2) and float((k1 - k2).abs().max()) <= 16 * 2.0 ** -24 * float(k1.abs().max())
     assert int((k2 != k.to(DEV)).any(-1).sum()) == (sum(s >= 0 for s in SLOTS) * G if write else 0)
     assert float((got - want).abs().max()) <= 256 * 2.0 ** -24 * float(want.abs().max()) and not got[SLOTS.index(-1)].any()
+    x, new, cpu = qkv.double().cpu(), {}, lambda t: None if t is None else t.double().cpu()
+    for i, length in enumerate(LENS):
+        at = (cpu(cos)[length - 1], cpu(sin)[length - 1], D, False, 1e-6)
+        q, key = (turned_exactly(x[i, a:a + m * D].view(m, D), cpu(w), *at) for a, m, w in ((0, H, qw), (H * D, G, kw)))
+        new[i] = (q, key, x[i, (H + G) * D:(H + 2 * G) * D].view(G, D)) if write else (q, None, None)
+    for i, o, spread, product in exact_rows(table, k, v, SLOTS, LENS, new, G, D ** -0.5, window):
+        # a score is a sum of D products of values with some 16 roundings of 2^-24 each behind them (sum of squares, norm, turn), as large as the
+        # largest times D^1/2 where they fall either way, times the scale D^-1/2; that counts twice in the quotient, and its sums add theirs
+        tol = 2.0 ** -24 * (4 * 16 * product + 64) * spread
+        assert bool(((got[i].double().cpu() - o).abs() <= tol).all()), (i, float(((got[i].double().cpu() - o).abs() / tol).max()))

@@ -1,6 +1,8 @@
-"""Decoding attention whose queries, key and value come straight from the projection, against the kernels it stands for: the turn and
-the append to the cache in one launch, attention in another, the gate in a third. The same roundings in the same places, so pages
-and outputs differ by the roundings of a differently contracted product at most."""
+"""Decoding attention whose queries, key and value come straight from the projection: against 64 bits, and against the kernels it stands
+for, the turn and the append to the cache in one launch, attention in another, the gate in a third. The same roundings in the same
+places, so pages and outputs differ by the roundings of a differently contracted product at most."""
+import math
+
 import pytest
 import torch
 
@@ -32,6 +34,51 @@ def close(a, b):
     a, b = a.double().cpu(), b.double().cpu()
     assert bool(torch.isfinite(b).all())
     return float((a - b).abs().max()) <= 2.0 ** -6 * float(b.abs().max()) and float((a - b).pow(2).mean().sqrt()) <= 2.0 ** -10 * float(b.abs().max())
+
+
+def turned_exactly(x, w, cos, sin, rot, pairs, eps, unit=False):
+    """Heads ``x [heads, D]`` normed by ``w`` (None: not), the first ``rot`` features turned, made unit behind that (``unit``), in 64 bits."""
+    if w is not None:
+        x = x * (x.pow(2).mean(-1, keepdim=True) + eps).rsqrt() * w
+    if rot:
+        one, two = (x[:, 0:rot:2], x[:, 1:rot:2]) if pairs else (x[:, :rot // 2], x[:, rot // 2:rot])
+        first, second = one * cos - two * sin, two * cos + one * sin
+        x = torch.cat([torch.stack([first, second], -1).flatten(1) if pairs else torch.cat([first, second], -1), x[:, rot:]], -1)
+    return x * (x.pow(2).mean(-1, keepdim=True) + eps).rsqrt() if unit else x
+
+
+def exact_rows(table, k, v, slots, lens, new, G, scale, window=0, chunk=0, cap=0.0, sink=None, rel=None):
+    """Attention of each live sequence's row in 64 bits over pages ``k [pages, G, 64, .]`` and ``v [pages, G, ., 64]``. ``new[i]``: the row's
+    queries ``[H, D]``, and its keys and values ``[G, .]`` where they are appended (else None: the pages hold them). Yields the sequence, the
+    outputs and, for their error, the sums of ``p |v|`` and the largest product of a feature of q and one of a key that it sees."""
+    column = torch.tensor([p // 32 * 32 + 8 * (p % 16 // 4) + 4 * (p % 32 // 16) + p % 4 for p in range(64)])
+    for i, (slot, length) in enumerate(zip(slots, lens)):
+        if slot < 0:
+            continue
+        q, own_k, own_v = new[i]
+        H, D = q.shape
+        held = table[slot, :-(-length // 64)].long()
+        keys = k[held][..., :D].permute(0, 2, 1, 3).flatten(0, 1)[:length].double().clone()
+        values = v[held][..., column].permute(0, 3, 1, 2).flatten(0, 1)[:length].double().clone()
+        if own_k is not None:
+            keys[-1], values[-1, :, :own_v.shape[-1]] = own_k, own_v
+        pos = length - 1
+        lo = pos - pos % chunk if chunk else max(0, length - window) if window else 0
+        kh, vh = (t[lo:].repeat_interleave(H // G, 1).permute(1, 0, 2).contiguous() for t in (keys, values))
+        sc = (kh * q[:, None]).sum(-1) * scale
+        if cap:
+            sc = cap * torch.tanh(sc / cap)
+        if rel is not None:
+            sc = sc + rel.double()[(pos - torch.arange(lo, length)).clamp(max=rel.shape[0] - 1)].T
+        p = torch.softmax(sc if sink is None else torch.cat([sc, sink.double()[:, None]], 1), 1)[:, :length - lo, None]
+        yield i, (p * vh).sum(1), (p * vh.abs()).sum(1), float((q[:, None] * kh).abs().max())
+
+
+def room(want, spread, product, scale):
+    """How far bfloat16 results may be off: probabilities rounded (2^-9 of each, in sum and total), the result's own rounding, and a feature
+    of q or of the new key that lies next to the middle of two bfloat16 numbers rounded the other way (2^-8 of its product in a
+    score, which counts twice in the quotient; two of them)."""
+    return 2.0 ** -8 * want.abs() + (2.0 ** -8 + 4 * 2.0 ** -8 * product * scale) * spread + 1e-6
 
 
 @pytest.mark.parametrize("splits", [1, 3])
@@ -75,6 +122,18 @@ def test_turn_and_attention(splits, write, form, H, G, D, Dv, P, rot):
     ops.attn_turned_bf16(t, write, k2, v2, *at, *parts(), splits, got, H, G, P, scale, window, cap, sink, chunk, rel)
     assert torch.equal(v1, v2) and close(k2, k1) and int((k1 != k2).sum()) <= 2 + n * G * D // 50
     assert close(got, want) and not got[SLOTS.index(-1)].any()
+    x, cpu = src.double().cpu(), lambda t: None if t is None else t.double().cpu()
+    new, rounded = {}, lambda t: t.bfloat16().double()
+    for i, length in enumerate(LENS):
+        tables = (cpu(cos)[length - 1], cpu(sin)[length - 1]) if rot else (None, None)
+        heads = [turned_exactly(x[i, a:a + m * D].view(m, D), cpu(w), *tables, rot, what[0] == "pairs", eps, unit)
+                 for a, m, w in ((0, H, qw), (H * D, G, kw))]
+        new[i] = (rounded(heads[0]), rounded(heads[1]) if write else None, x[i, (H + G) * D:cols].view(G, Dv) if write else None)
+    for i, o, spread, product in exact_rows(f["table"].cpu(), k.cpu(), v.cpu(), SLOTS, LENS, new, G, scale, window, chunk, cap,
+                                            *(None if t is None else t.cpu() for t in (sink, rel))):
+        by = torch.sigmoid(x[i, cols:cols + H * Dv].view(H, P)) if gate is not None else 1.0
+        tol = room(o, spread, product, scale) * by + (2.0 ** -8 * (o * by).abs() if gate is not None else 0.0)
+        assert bool(((got[i].double().cpu() - o * by).abs() <= tol).all()), i
 
 
 @pytest.mark.parametrize("splits", [1, 3])
@@ -105,3 +164,22 @@ def test_turn_and_difference(splits, write, H, G, D, Dv, rot, bias, sums):
     ops.attn_turned_bf16(t, write, k2, v2, *at, *parts(), splits, got, H, G, P, scale, 0, maps=(step_w, lam, post, eps))
     assert torch.equal(v1, v2) and close(k2, k1) and int((k1 != k2).sum()) <= 2 + n * G * D // 50
     assert close(got, want) and not got[SLOTS.index(-1)].any()
+    x = (src.cpu().sum(0).bfloat16() if sums else src.cpu()).double() + (b.double().cpu() if bias else 0.0)
+    new, rounded = {}, lambda t: t.bfloat16().double()
+    for i, length in enumerate(LENS):
+        tables = (cos.double().cpu()[length - 1], sin.double().cpu()[length - 1]) if rot else (None, None)
+        q, key = (turned_exactly(x[i, a:a + 2 * m * D].view(2 * m, D), None, *tables, rot, True, eps) for a, m in ((0, H), (2 * H * D, G)))
+        new[i] = q, key, rounded(x[i, 2 * (H + G) * D:].view(G, Dv))
+    maps = []
+    for m in range(2):                              # the maps are attentions of their own on their features of the keys
+        km = k[..., m * step_w:m * step_w + D].cpu()
+        mine = {i: (rounded(q[m::2]), rounded(key[m::2]) if write else None, val if write else None) for i, (q, key, val) in new.items()}
+        maps.append({i: rest for i, *rest in exact_rows(f["table"].cpu(), km, v[:, :, :Dv].cpu(), SLOTS, LENS, mine, G, scale)})
+    for i in maps[0]:
+        (o1, s1, p1), (o2, s2, p2) = maps[0][i], maps[1][i]
+        d = o1 - lam * o2
+        by = (d.pow(2).mean(-1, keepdim=True) + eps).rsqrt() * post
+        # the difference of the maps' errors, through the norm: its own and that of the root mean square
+        tol = (room(o1, s1, p1, scale) + lam * room(o2, s2, p2, scale)) * by
+        tol = tol + (d * by).abs() * (tol / post).pow(2).mean(-1, keepdim=True).sqrt() + 2.0 ** -8 * (d * by).abs()
+        assert bool(((got[i].double().cpu() - d * by).abs() <= tol).all()), i

@@ -183,3 +183,32 @@ def test_float32_keys_are_split_where_that_was_measured_ahead(rows, heads, kv, k
     """What was up to twice as slow split, since the last workgroup adds up many wide parts, stays with one workgroup."""
     from dryft_amd.parts.attention import float32_splits
     assert float32_splits(rows, heads, kv, keys, width) == splits
+
+
+@pytest.mark.parametrize("rows,n,k,split,pays", [
+    (17, 5120, 25600, True, True), (64, 5120, 25600, True, True), (65, 5120, 25600, True, False), (128, 5120, 17408, True, True),
+    (65, 10240, 9856, True, False), (65, 10240, 9792, True, True), (96, 1024, 2048, True, True), (97, 1024, 2048, True, False),
+    (97, 4096, 2048, True, True), (97, 4096, 1984, True, False), (128, 151936, 2560, False, True)])
+def test_products_of_17_to_128_rows_by_size(rows, n, k, split, pays):
+    """Split products leave for the kernel whose waves own rows of x beyond 64 rows and 192 MiB, and beyond 96 rows below 16 MiB."""
+    from dryft_amd.parts.linear import mid_pays
+    assert mid_pays(rows, n, k, split) == pays
+
+
+@pytest.mark.parametrize("rows,outputs,k,kernel", [
+    (64, 9728, 2560, "panel"), (65, 9728, 2560, "panel"), (96, 9728, 2560, "panel"), (97, 9728, 2560, "tall"), (256, 9728, 2560, "tall"),
+    (257, 9728, 2560, "library"), (64, 25600, 5120, "panel"), (96, 17408, 5120, "panel"), (65, 25600, 5120, "library"),
+    (97, 17408, 5120, "library"), (65, 19661, 5120, "library"), (65, 19660, 5120, "panel"), (65, 512, 2624, "tall"), (64, 512, 2624, "library")])
+def test_gate_up_by_rows_size_and_depth(monkeypatch, rows, outputs, k, kernel):
+    """In the order in which the feed-forward asks: what it calls."""
+    from dryft_amd.csrc import ops
+    from dryft_amd.parts import mlp
+    called = []
+    for name, what in (("gemm_few_glu_bf16", "few"), ("gemm_panel_swiglu_bf16", "panel"), ("gemm_tall_swiglu_bf16", "tall"),
+                       ("gemm_many_glu_bf16", "many"), ("silu_mul", "library")):
+        monkeypatch.setattr(ops, name, lambda *a, what=what, **b: called.append(what))
+    monkeypatch.setattr(mlp, "linear", lambda x, w, **kw: x)
+    part = mlp.SwiGLU(k, outputs)
+    part.w_gate_up, part.w_down = fake(2 * outputs, k), fake(k, outputs)
+    part.forward(fake(rows, k), None, leave_product=True)
+    assert called == [kernel]

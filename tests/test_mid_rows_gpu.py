@@ -37,10 +37,13 @@ def test_panel_of_up_to_96_rows(m, inter, k, waves, unit):
 
 @pytest.mark.parametrize("m", [17, 33, 64, 65, 81, 97, 128])
 @pytest.mark.parametrize("n,k,waves,splits", [(77, 64, 5, 1), (97, 320, 6, 5), (100, 192, 8, 3), (2560, 1664, 5, 7),
-                                              (33000, 128, 8, 1), (20500, 192, 4, 1), (4200, 1024, 4, 4), (2056, 2048, 8, 16)])
+                                              (33000, 128, 8, 1), (20500, 192, 4, 1), (4200, 1024, 4, 4), (2056, 2048, 8, 16),
+                                              (2560, 9728, 5, 8), (6144, 2560, 6, 4), (33000, 1024, 8, 1), (1531, 2560, 8, 2),
+                                              (1200, 1280, 5, 1), (1000, 1600, 6, 1), (25000, 832, 6, 1), (7000, 3072, 8, 4)])
 def test_products_of_17_to_128_rows(m, n, k, waves, splits):
     """Every width of a workgroup, runs of K of one group and of unequal length, weights kept and read once, launches of more
-    workgroups than compute units (two stages in LDS); a row of x wider than K."""
+    workgroups than compute units (two stages in LDS); a row of x wider than K. And runs several times as long as the ring of two to four
+    stages, in each of these: what a wrong wait or stage would show in."""
     from dryft_amd.csrc import ops
     torch.manual_seed(m + n + k)
     x, w = torch.randn(m, k + 8).to(torch.bfloat16).to(DEV)[:, :k], (torch.randn(n, k) / math.sqrt(k)).to(torch.bfloat16).to(DEV)
