@@ -556,7 +556,8 @@ DRYFT_API int dryft_gemm_wide_swiglu_bf16(const void* x, int64_t x_stride, const
 // 4,096 35.9 / 36.6 / 38.2 and 39.2 / 39.3 / 40.9), and models of three layers of such do not stay in the last-level cache between steps.
 // Smaller ones may: 0.95 to 0.98 from memory, but weights of 150 MB in all, which stay, take 1.05 to 1.48 of the time with the
 // hint (2 x 1,376 of 5,120 at 32 rows 14.9 and 22.1, 2 x 4,928 of 1,280 7.1 and 9.1; the hint as a branch in the kernel 1.01 to 1.08).
-// At 65 to 96 rows it loads 80 or 96 rows of x where the tall form below loads 128: at 65 / 80 / 96 rows 9,728 of 2,560 23.7 / 24.4 / 26.3 (26.0 / 27.2 / 28.3), 12,288 of 4,096 39.2 / 39.0 / 40.5 (44.5 / 47.8 / 45.3),
+// At 65 to 96 rows it loads 80 or 96 rows of x where the tall form below loads 128: at 65 / 80 / 96 rows 9,728 of 2,560 23.7 / 24.4 /
+// 26.3 (26.0 / 27.2 / 28.3), 12,288 of 4,096 39.2 / 39.0 / 40.5 (44.5 / 47.8 / 45.3),
 // 3,072 of 1,024 8.6 / 8.9 / 9.6 (9.7 / 9.9 / 10.2); at 112 it is behind (31.8 / 29.8, 52 / 45, 11.3 / 10.4).
 __device__ __forceinline__ void panel_load16(const void* base, uint32_t offset, uint32_t lds_base) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(offset), "s"(base) : "memory", "m0");
@@ -969,7 +970,8 @@ static int mid_waves(const void* x, int64_t x_stride, const void* w, float* part
   }
 }
 
-// M <= 256 (beyond 128 four waves only). partials[splits, M, N] = float partial sums of x . W^T over `splits` equal runs of groups
+// M <= 256 (beyond 128 four waves only, for callers of this entry point: `linear` sends such rows to the tall form, which takes in fewer
+// bytes of x for a row of W). partials[splits, M, N] = float partial sums of x . W^T over `splits` equal runs of groups
 // of 64 values of K (the last run may be shorter, none may be empty); a workgroup owns 16 `waves` outputs (4, 5, 6 or 8 waves); K a
 // multiple of 64; x and W within reach of 32-bit byte offsets.
 DRYFT_API int dryft_gemm_mid_bf16(const void* x, int64_t x_stride, const void* w, float* partials, int M, int N, int K,

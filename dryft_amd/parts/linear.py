@@ -199,7 +199,9 @@ def mid_pays(m: int, n: int, k: int, may_split: bool) -> bool:
     the first, but for split products of large matrices (5,120 x 25,600, 250 MiB, at 77 / 96 / 128 rows 59 / 69 / 80 us against
     54 / 58 / 63; 5,120 x 17,408, 170 MiB, 36 / 38 / 42 against 38 / 40 / 43) and beyond 96 rows of small ones, whose partial sums
     weigh more than they (steps of 128 sequences through Qwen3-0.6B, 4 to 8 MiB, 2,295 against 2,284 us; Qwen3-4B's, 12 layers,
-    20 MiB on, 1,707 against 1,812)."""
+    20 MiB on, 1,707 against 1,812). Whole float32 results of any size: 200 of 65 to 4,096 outputs (routers) take 0.62 of the time that
+    ``gemm_wide`` and ``gemm_block`` took, 0.86 at most, 55 heads of up to 160,000 outputs 0.74. Split products with the norm behind, 800
+    sizes: 0.97 on average; 19, of less than 8 MiB but for one, are 3 to 8 % slower than before."""
     size = n * k * 2
     return m <= WIDE_ROWS or not may_split or (size <= 192 << 20 and (m <= 96 or size >= 16 << 20))
 
@@ -260,11 +262,12 @@ def panel_swiglu_ok(x: torch.Tensor, w_gate_up: torch.Tensor) -> bool:
 
 
 _PANEL_BYTES = 384 << 20        # gate/up matrices up to here go there at 65 to 96 rows too
-_TALL_SWIGLU_BYTES = 256 << 20  # gate/up matrices up to here go to the kernel whose waves own rows of x at 65 to 256 rows
+_TALL_SWIGLU_BYTES = 256 << 20  # gate/up matrices up to here go to the kernel whose waves own rows of x beyond that, up to 256 rows
 
 
 def tall_swiglu_ok(x: torch.Tensor, w_gate_up: torch.Tensor) -> bool:
-    """Does the fused gate/up product with its activation go, at 65 to 256 rows, to the kernel whose waves each own
+    """Does the fused gate/up product with its activation go, at 97 to 256 rows, and at 65 to 96 where ``panel_swiglu_ok``, which is
+    asked first, leaves it (K a multiple of 64 alone), to the kernel whose waves each own
     rows of x? In-graph times on rotating cold weights, us, against the vendor library plus the activation kernel:
     Qwen3-4B's sizes 30.0 against 35.6 at 128 rows, 36.3 against 51.0 at 256; Qwen3-8B's 46.8 against 55.5 and 57.9
     against 66.1; Qwen3-14B's (356 MB) 102 against 100 and 129 against 111, so matrices beyond 256 MiB stay with the
