@@ -105,7 +105,8 @@ class DifferentialAttention(Mixer):
             cos, sin, rot = table.cos, table.sin, table.dims
             if rot > D:
                 raise ValueError(f"the position encoding rotates {rot} features, a map has {D}")
-        proj = linear(h, self.w_qkv, allow_partials=True, partial_rows=_PARTIAL_ROWS)
+        # float32 rows want their sums whole: the kernel behind adds up parts for bfloat16 queries alone
+        proj = linear(h, self.w_qkv, allow_partials=h.dtype == torch.bfloat16, partial_rows=_PARTIAL_ROWS)
         if isinstance(proj, Partials):
             proj = (proj.data, proj.count)
         wide, step = self.page_dim(), self.map_width()

@@ -261,6 +261,18 @@ def test_attention_alone(dtype, shape):
             assert mixer_error(got, ref, dtype) <= MIXER_TOL[dtype], (shape, cuts[:3])
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows", [5, 8, 16])
+def test_attention_alone_at_a_width_whose_products_split(dtype, rows):
+    """Steps of 5 to 16 rows at width 1,024, where float32 products split K over workgroups too."""
+    layer = SHAPES["cores-128"]
+    t, plan = mixer_case(layer, 1024, seed=rows)
+    part, cache, positions = load_mixer(plan, t, dtype)
+    seqs = [torch.randn(rows, 1024, generator=torch.Generator().manual_seed(rows)).to(TORCH[dtype]).float()]
+    want = P.attention(seqs[0].double(), double(P.part(t, "l0.mix.")), layer["mixer"], EPS)[0]
+    assert mixer_error(run_mixer(part, cache, positions, dtype, seqs, [])[0], want, dtype) <= MIXER_TOL[dtype]
+
+
 SHOW_CUTS = ([], list(range(120, 200)), [64, 128], [2, 63, 65, 127, 129], [19, 20, 21])
 
 
