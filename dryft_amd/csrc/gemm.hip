@@ -832,6 +832,7 @@ static int panel_entry(const void* x, int64_t x_stride, const void* w, void* y, 
 // times as long (a compute unit looks up a line, or half of one, every 8 cycles or so); K over the waves too, with one
 // sum at the end: the same.
 #define MID_GROUP 64
+#define MID_ROWS 128
 
 template <int MT, int WAVES, int STAGES, bool ONCE>
 __global__ __launch_bounds__(64 * WAVES) void gemm_mid_kernel(const bf16_t* __restrict__ x, int64_t x_stride,
@@ -970,14 +971,13 @@ static int mid_waves(const void* x, int64_t x_stride, const void* w, float* part
   }
 }
 
-// M <= 256 (beyond 128 four waves only, for callers of this entry point: `linear` sends such rows to the tall form, which takes in fewer
-// bytes of x for a row of W). partials[splits, M, N] = float partial sums of x . W^T over `splits` equal runs of groups
+// M <= 128. partials[splits, M, N] = float partial sums of x . W^T over `splits` equal runs of groups
 // of 64 values of K (the last run may be shorter, none may be empty); a workgroup owns 16 `waves` outputs (4, 5, 6 or 8 waves); K a
 // multiple of 64; x and W within reach of 32-bit byte offsets.
 DRYFT_API int dryft_gemm_mid_bf16(const void* x, int64_t x_stride, const void* w, float* partials, int M, int N, int K,
                                   int splits, int waves, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (M > 256 || K <= 0 || K % MID_GROUP || splits < 1 || x_stride % 8 || (((uintptr_t)x | (uintptr_t)w) & 15) ||
+  if (M > MID_ROWS || K <= 0 || K % MID_GROUP || splits < 1 || x_stride % 8 || (((uintptr_t)x | (uintptr_t)w) & 15) ||
       ((uintptr_t)partials & 15) || (int64_t)N * K * 2 >= (int64_t)4 << 30 || (int64_t)M * x_stride * 2 >= (int64_t)4 << 30)
     return -1;
   const int groups = K / MID_GROUP, per = (groups + splits - 1) / splits;
@@ -987,10 +987,7 @@ DRYFT_API int dryft_gemm_mid_bf16(const void* x, int64_t x_stride, const void* w
   if (M <= 64) return mid_waves<4>(x, x_stride, w, partials, M, N, K, splits, waves, stream);
   if (M <= 80) return mid_waves<5>(x, x_stride, w, partials, M, N, K, splits, waves, stream);
   if (M <= 96) return mid_waves<6>(x, x_stride, w, partials, M, N, K, splits, waves, stream);
-  if (M <= 128) return mid_waves<8>(x, x_stride, w, partials, M, N, K, splits, waves, stream);
-  if (waves != 4) return -1;
-  if (M <= 192) return launch_mid<12, 4, 3, false>(x, x_stride, w, partials, M, N, K, splits, stream);
-  return launch_mid<16, 4, 3, false>(x, x_stride, w, partials, M, N, K, splits, stream);
+  return mid_waves<8>(x, x_stride, w, partials, M, N, K, splits, waves, stream);
 }
 
 // -------------------------------------------------------------------------------------------- tall

@@ -1351,8 +1351,7 @@ def gemm_tall_bf16(x, w, partials, splits: int, tiles: int) -> torch.Tensor:
     return partials
 
 
-MID_ROWS = 256      # the most rows gemm_mid takes
-MID_MOST = 128      # the most it takes with other than 4 waves
+MID_ROWS = 128      # the most rows the kernel takes
 MID_WAVES = (4, 5, 6, 8)
 MID_GROUP = 64      # values of K it walks at a time; K must be a multiple, and the splits are runs of such groups
 
@@ -1369,7 +1368,8 @@ def gemm_mid_splits(k: int, splits: int) -> int:
 def gemm_mid_bf16(x, w, partials, splits: int, waves: int = 4) -> torch.Tensor:
     """Float partial sums ``partials[splits, M, N]`` of ``x @ w.T`` over ``splits`` runs of K, for 1 to 256 rows, by the
     kernel whose operands go from memory straight into LDS. K must be a multiple of 64 and ``splits`` one that
-    ``gemm_mid_splits`` returns; a workgroup owns ``16 * waves`` outputs (4, 5, 6 or 8 waves; beyond 128 rows 4)."""
+    ``gemm_mid_splits`` returns; a workgroup owns ``16 * waves`` outputs (4, 5, 6 or 8 waves). Beyond ``MID_ROWS`` rows, with 4
+    waves, the runs are ``gemm_tall_bf16``'s, which is ahead there."""
     _gpu(x, "x", torch.bfloat16)
     _gpu(w, "w", torch.bfloat16)
     _gpu(partials, "partials", torch.float32)
@@ -1377,16 +1377,18 @@ def gemm_mid_bf16(x, w, partials, splits: int, waves: int = 4) -> torch.Tensor:
     n = w.shape[0]
     if not (w.shape == (n, k) and w.is_contiguous() and x.stride(1) == 1):
         raise KernelError("gemm_mid: x [M,K] row-major, w [N,K] contiguous")
-    if not (m <= MID_ROWS and k % MID_GROUP == 0 and x.stride(0) % 8 == 0):
-        raise KernelError(f"gemm_mid: needs M <= {MID_ROWS} and K % {MID_GROUP} == 0, got M={m} K={k}")
+    if not (m <= TALL_ROWS and k % MID_GROUP == 0 and x.stride(0) % 8 == 0):
+        raise KernelError(f"gemm_mid: needs M <= {TALL_ROWS} and K % {MID_GROUP} == 0, got M={m} K={k}")
     if not (x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and partials.data_ptr() % 16 == 0):
         raise KernelError("gemm_mid: operands must be 16-byte aligned")
     if not (splits >= 1 and gemm_mid_splits(k, splits) == splits):
         raise KernelError(f"gemm_mid: {splits} splits would leave a run of K = {k} empty")
     if not (partials.shape == (splits, m, n) and partials.is_contiguous()):
         raise KernelError(f"gemm_mid: partials must be [{splits},{m},{n}]")
-    if not (waves in MID_WAVES and (m <= MID_MOST or waves == 4)):
-        raise KernelError(f"gemm_mid: waves 4, 5, 6 or 8, beyond {MID_MOST} rows 4")
+    if not (waves in MID_WAVES and (m <= MID_ROWS or waves == 4)):
+        raise KernelError(f"gemm_mid: waves 4, 5, 6 or 8, beyond {MID_ROWS} rows 4")
+    if m > MID_ROWS:
+        return gemm_tall_bf16(x, w, partials, splits, 4)
     _check(_fn("gemm", "dryft_gemm_mid_bf16")(_ptr(x), x.stride(0), _ptr(w), _ptr(partials), m, n, k, int(splits),
                                               int(waves), _stream()), "gemm_mid_bf16")
     return partials

@@ -365,7 +365,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, *, out_dtype: torch.dtype | None = 
         out = torch.empty((m, n), dtype=out_dtype, device=x.device)
         ops.gemm_stream_bf16(x, w, out, None, group, 1, depth)
         return out
-    if m <= ops.MID_MOST and (allow_partials or out_dtype == torch.float32) and few_ok and k % ops.MID_GROUP == 0 and \
+    if m <= ops.MID_ROWS and (allow_partials or out_dtype == torch.float32) and few_ok and k % ops.MID_GROUP == 0 and \
             within_direct_reach(x, w) and mid_pays(m, n, k, allow_partials):
         waves, splits = mid_plan(m, n, k, allow_partials)
         partials = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)

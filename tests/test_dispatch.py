@@ -218,7 +218,7 @@ def test_gate_up_by_rows_size_and_depth(monkeypatch, rows, outputs, k, kernel):
     ("token_step.h", "TOKEN_MAX_DIM", "TOKEN_MAX_DIM", 0), ("rglru.hip", "RG_TOKEN_BLOCK", "RGLRU_TOKEN_BLOCK", 0),
     ("rglru.hip", "RG_MAX_TAPS", "RGLRU_MAX_TAPS", 0), ("attn_f32.hip", "F32_MAX_SPLITS", "ATTN_F32_SPLITS", 0),
     ("gemm_lines.hip", "LINES_BESIDE", "LINES_TOGETHER", 1), ("gemm.hip", "PANEL_ROWS", "PANEL_ROWS", 0),
-    ("gemm.hip", "PANEL_GROUP", "PANEL_GROUP", 0), ("gemm.hip", "MID_GROUP", "MID_GROUP", 0), ("mlstm.hip", "MLSTM_COLS", "MLSTM_COLUMNS", 0),
+    ("gemm.hip", "PANEL_GROUP", "PANEL_GROUP", 0), ("gemm.hip", "MID_GROUP", "MID_GROUP", 0), ("gemm.hip", "MID_ROWS", "MID_ROWS", 0), ("mlstm.hip", "MLSTM_COLS", "MLSTM_COLUMNS", 0),
     ("conv.hip", "CONV_MAX_TAPS", "CONV_MAX_TAPS", 0), ("ssm.hip", "SSM_MAX_STATE", "SSM_MAX_STATE", 0),
     ("moe.hip", "MOE_MAX_EXPERTS", "MOE_MAX_EXPERTS", 0)])
 def test_limits_that_both_sides_hold_are_the_same(file, define, constant, more):
